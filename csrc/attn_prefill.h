@@ -1,0 +1,17 @@
+// attn_prefill.h — arguments of the prompt attention kernels.
+#pragma once
+#include "common.h"
+
+struct ApArgs {
+  const u16* q;          // [M, ldq], heads of head_dim values, rotated
+  const void* kc;        // [kvh, S, head_dim] bf16, or e4m3 with kS / vS
+  const void* vc;
+  u16* out;              // [M, nh * head_dim]
+  const int* len_ptr;    // position of row 0
+  const float* kS;       // [kvh, S]
+  const float* vS;
+  float* part;           // split keys: [split, kvh, rows, head_dim + 4]
+  int M, nh, kvh, ldq, S, fold;
+  float scale, softcap;
+  int window;
+};

@@ -1,0 +1,448 @@
+// attn_prefill.hip — flash attention of prompt rows over the KV pool.
+//
+// One wave holds 32 query rows and walks the keys in tiles of 32; a block
+// of four waves shares the tiles through LDS.  The rows of a block are
+// (position, head) pairs of ONE kv head, so a K/V tile is read once for
+// all heads of its group and a check of five proposed tokens fills half a
+// tile instead of five heads' own.
+//
+// S^T = K Q^T puts a query in a lane (column lane&31 of
+// mfma_f32_32x32x16), so maximum, sum and rescaling never leave the lane
+// pair (l, l+32).  The 16 scores a lane then holds are, in register order,
+// the k elements of the second product's B operand for keys
+// {0-3,8-11} + 4*half of a 16-key slab, so P goes from accumulator to
+// operand without moving between lanes; V^T comes out of LDS in that same
+// key order with ds_read_b64_tr_b16, which turns a 4-key x 16-dim tile so
+// that a lane holds one dim's four keys.
+//
+// What bounds it: head_dim 128 spends 512 MFMA cycles and about 450 VALU
+// cycles on 32 keys x 32 rows; two blocks of 64 KB LDS on a CU overlap them.
+// Measured (32/8 heads of 128, 2048 rows behind 6139 keys): 314 us,
+// 765 TFLOP/s; a wave per head and 16 queries took 1422 us.  5 rows of 24/8
+// heads over 906 keys, split: 19 us, unsplit per-head waves 74 us.  Head
+// dim 256 spills some 20 registers at two waves a SIMD and is still faster
+// than one wave without (2048 rows behind 2048 keys: 163 to 219 us, before
+// 507 us).
+#include "common.h"
+#include "attn_prefill.h"
+
+typedef short ap_s4 __attribute__((ext_vector_type(4)));
+typedef __bf16 ap_b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 ap_b2 __attribute__((ext_vector_type(2)));
+typedef float ap_f16 __attribute__((ext_vector_type(16)));
+
+#define LOG2E 1.4426950408889634f
+
+// tanh by exp2: |error| below 2e-7, exact limits at +-inf
+DEVINL float ap_tanh(float x) {
+  const float e = __builtin_amdgcn_exp2f(x * (2.f * LOG2E));
+  return 1.f - 2.f * __builtin_amdgcn_rcpf(e + 1.f);
+}
+
+// LDS rows are `HD` bf16.  K: 16-byte slots swizzled by the row (a b128
+// fragment read takes one slot of 32 rows); V: 64-byte chunks swizzled (a
+// transposed read takes one chunk of 8 rows).
+template <int HD> DEVINL int k_slot(int row, int slot) {
+  return slot ^ (row & (HD / 8 < 16 ? 7 : 15));
+}
+template <int HD> DEVINL int v_slot(int row, int slot) {
+  const int x = HD == 64 ? (row >> 1) & 1 : row & 3;
+  return slot ^ (x << 2);
+}
+
+template <int HD, int BKV, int NW, bool KV8, bool CAP>
+__global__ void __launch_bounds__(64 * NW, 2)
+k_attn_rows(ApArgs a) {
+  constexpr int RB = HD * 2;                 // LDS bytes of a row
+  constexpr int TILE = BKV * RB;
+  constexpr int SLOTS = HD / 8;              // 16-byte slots of a row
+  constexpr int NS = BKV / 32;               // 32-key parts of a tile
+  constexpr int NT = 64 * NW;
+  __shared__ __attribute__((aligned(16))) char Ks[2][TILE];
+  __shared__ __attribute__((aligned(16))) char Vs[2][TILE];
+  __shared__ __attribute__((aligned(16))) float Sc[2][2][KV8 ? BKV : 4];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hh = lane >> 5, col = lane & 31;
+  const int grp = a.nh / a.kvh;
+  // heads vary fastest, so that with a multiple of eight of them the
+  // blocks of a kv head land on one XCD and share its L2
+  const int kvhead = blockIdx.x;
+  const int nq = gridDim.y;
+  // longest rows first; where two blocks a CU hold the whole grid, a long
+  // one shares its CU with a short one
+  int qt = nq - 1 - (int)blockIdx.y;
+  if (a.fold && (int)blockIdx.y >= nq / 2) qt = (int)blockIdx.y - nq / 2;
+
+  const int pos0 = *a.len_ptr;
+  const int nrows = a.M * grp;
+  const int row0 = (qt * NW + wave) * 32;
+  const int row = row0 + col;
+  const int rowc = min(row, nrows - 1);
+  const int my_m = rowc / grp, my_g = rowc % grp;
+  const int qpos = pos0 + my_m;
+  // positions of the wave's first and last row, and of the block's last
+  const int q_lo = pos0 + min(row0, nrows - 1) / grp;
+  const int q_hi = pos0 + min(row0 + 31, nrows - 1) / grp;
+  const int b_lo = pos0 + min(qt * NW * 32, nrows - 1) / grp;
+  const int b_hi = pos0 + min(qt * NW * 32 + NW * 32 - 1, nrows - 1) / grp;
+  const bool live = row0 < nrows;
+
+  // keys [k_lo, k_hi) of this block
+  int k_lo = 0, k_hi = b_hi + 1;
+  if (a.window > 0) k_lo = max(0, b_lo + 1 - a.window);
+  if (gridDim.z > 1) {
+    const int tiles = (k_hi - k_lo + BKV - 1) / BKV;
+    const int per = (tiles + gridDim.z - 1) / gridDim.z;
+    const int lo = k_lo + (int)blockIdx.z * per * BKV;
+    k_hi = min(k_hi, lo + per * BKV);
+    k_lo = lo;
+  }
+  const int t_last = b_hi;                   // last key that may be read
+
+  // Q: B operand, column = row of the tile, 8 dims at 16*c + 8*hh
+  ap_b8 qf[HD / 16];
+  {
+    const u16* qp = a.q + (size_t)my_m * a.ldq +
+                    (size_t)(kvhead * grp + my_g) * HD + hh * 8;
+#pragma unroll
+    for (int c = 0; c < HD / 16; c++) qf[c] = *(const ap_b8*)(qp + c * 16);
+  }
+
+  const char* Kg = (const char*)a.kc + (size_t)kvhead * a.S * HD * (KV8 ? 1 : 2);
+  const char* Vg = (const char*)a.vc + (size_t)kvhead * a.S * HD * (KV8 ? 1 : 2);
+  const float* kS = KV8 ? a.kS + (size_t)kvhead * a.S : nullptr;
+  const float* vS = KV8 ? a.vS + (size_t)kvhead * a.S : nullptr;
+
+  // bf16 pool: straight into LDS.  A wave's instruction fills 1 KB, lane by
+  // lane; the swizzle sits in the address that the lane reads.
+  constexpr int RPI = 1024 / RB;             // rows an instruction fills
+  auto stage16 = [&](int buf, int t0) {
+#pragma unroll
+    for (int i = 0; i < BKV / RPI / NW; i++) {
+      const int r0 = (i * NW + wave) * RPI;
+      const int r = r0 + lane / SLOTS, s = lane % SLOTS;
+      const size_t t = min(t0 + r, t_last);
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) uint32_t*)(
+              Kg + t * RB + k_slot<HD>(r, s) * 16),
+          (__attribute__((address_space(3))) uint32_t*)(&Ks[buf][r0 * RB]),
+          16, 0, 0);
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) uint32_t*)(
+              Vg + t * RB + v_slot<HD>(r, s) * 16),
+          (__attribute__((address_space(3))) uint32_t*)(&Vs[buf][r0 * RB]),
+          16, 0, 0);
+    }
+  };
+  // fp8 pool: through registers, widened to bf16 (exact) on the way in;
+  // the scale of a key stays out of the rounding: it multiplies the fp32
+  // score, the one of a value the fp32 probability.
+  constexpr int L8 = KV8 ? BKV * HD / 16 / NT : 1;   // 16-byte loads a thread
+  u4v_ kr[L8], vr[L8];
+  constexpr int NSC = (2 * BKV + NT - 1) / NT;
+  float scr[NSC];
+  auto load8 = [&](int t0) {
+    if constexpr (KV8) {
+#pragma unroll
+      for (int i = 0; i < L8; i++) {
+        const int e = i * NT + tid, r = e / (HD / 16), s = e % (HD / 16);
+        const size_t t = min(t0 + r, t_last);
+        kr[i] = *(const u4v_*)(Kg + t * HD + s * 16);
+        vr[i] = *(const u4v_*)(Vg + t * HD + s * 16);
+      }
+#pragma unroll
+      for (int i = 0; i < NSC; i++) {
+        const int e = i * NT + tid;
+        if (e < 2 * BKV)
+          scr[i] = (e < BKV ? kS : vS)[min(t0 + e % BKV, t_last)];
+      }
+    }
+  };
+  auto store8 = [&](int buf) {
+    if constexpr (KV8) {
+#pragma unroll
+      for (int i = 0; i < L8; i++) {
+        const int e = i * NT + tid, r = e / (HD / 16), s = e % (HD / 16);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          union { ap_b2 b[4]; s8v v; } ko, vo;
+#pragma unroll
+          for (int d = 0; d < 2; d++) {
+            ko.b[d * 2] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                kr[i][h * 2 + d], 1.0f, false);
+            ko.b[d * 2 + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                kr[i][h * 2 + d], 1.0f, true);
+            vo.b[d * 2] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                vr[i][h * 2 + d], 1.0f, false);
+            vo.b[d * 2 + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                vr[i][h * 2 + d], 1.0f, true);
+          }
+          const int sl = s * 2 + h;
+          *(s8v*)(&Ks[buf][r * RB + k_slot<HD>(r, sl) * 16]) = ko.v;
+          *(s8v*)(&Vs[buf][r * RB + v_slot<HD>(r, sl) * 16]) = vo.v;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < NSC; i++) {
+        const int e = i * NT + tid;
+        if (e < 2 * BKV) Sc[buf][e / BKV][e % BKV] = scr[i];
+      }
+    }
+  };
+
+  float m = -INFINITY, l = 0.f;     // m in units of log2
+  ap_f16 o[HD / 32];
+#pragma unroll
+  for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) o[d][r] = 0.f;
+  const float c1 = CAP ? a.scale / a.softcap : a.scale * LOG2E;
+  const float c2 = CAP ? a.softcap * LOG2E : 1.f;
+
+  if (k_lo < k_hi) {
+    if constexpr (KV8) { load8(k_lo); store8(0); }
+    else stage16(0, k_lo);
+  }
+  __syncthreads();
+  int cur = 0;
+  for (int t0 = k_lo; t0 < k_hi; t0 += BKV) {
+    const bool more = t0 + BKV < k_hi;
+    if (more) {
+      if constexpr (KV8) load8(t0 + BKV);
+      else stage16(cur ^ 1, t0 + BKV);
+    }
+    const bool some = live && t0 <= q_hi &&
+                      (a.window <= 0 || t0 + BKV > q_lo - a.window);
+    if (some) {
+      ap_f16 s[NS];
+#pragma unroll
+      for (int n = 0; n < NS; n++) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[n][r] = 0.f;
+        const int kr_ = n * 32 + col;
+#pragma unroll
+        for (int c = 0; c < HD / 16; c++) {
+          const ap_b8 kf = *(const ap_b8*)(
+              &Ks[cur][kr_ * RB + k_slot<HD>(kr_, c * 2 + hh) * 16]);
+          s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[c], s[n], 0,
+                                                         0, 0);
+        }
+      }
+      // keys t0 + 32n + 8(r/4) + 4hh + r%4
+      const bool edge = t0 + BKV - 1 > q_lo || t0 + BKV > k_hi ||
+                        (a.window > 0 && t0 <= q_hi - a.window);
+      float mx = -INFINITY;
+#pragma unroll
+      for (int n = 0; n < NS; n++) {
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++) {
+          f4v ks = {1.f, 1.f, 1.f, 1.f};
+          if constexpr (KV8)
+            ks = *(const f4v*)(&Sc[cur][0][n * 32 + q4 * 8 + hh * 4]);
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            float v = s[n][q4 * 4 + j] * c1;
+            if constexpr (KV8) v *= ks[j];
+            if constexpr (CAP) v = c2 * ap_tanh(v);
+            if (edge) {
+              const int t = t0 + n * 32 + q4 * 8 + hh * 4 + j;
+              if (t > qpos || t >= k_hi ||
+                  (a.window > 0 && t <= qpos - a.window))
+                v = -INFINITY;
+            }
+            s[n][q4 * 4 + j] = v;
+            mx = fmaxf(mx, v);
+          }
+        }
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float mn = fmaxf(m, mx);
+      const float mu = mn == -INFINITY ? 0.f : mn;
+      if (__any(mn > m)) {
+        const float al = __builtin_amdgcn_exp2f(m - mu);
+        l *= al;
+#pragma unroll
+        for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) o[d][r] *= al;
+        m = mn;
+      }
+#pragma unroll
+      for (int n = 0; n < NS; n++) {
+#pragma unroll
+        for (int sl = 0; sl < 2; sl++) {
+          float p[8];
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            p[j] = __builtin_amdgcn_exp2f(s[n][sl * 8 + j] - mu);
+            l += p[j];
+          }
+          if constexpr (KV8) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+              const f4v vs = *(const f4v*)(
+                  &Sc[cur][1][n * 32 + sl * 16 + h * 8 + hh * 4]);
+#pragma unroll
+              for (int j = 0; j < 4; j++) p[h * 4 + j] *= vs[j];
+            }
+          }
+          union { ap_b2 b[4]; ap_b8 v; } pf;
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            pf.b[j][0] = (__bf16)p[j * 2];
+            pf.b[j][1] = (__bf16)p[j * 2 + 1];
+          }
+          // V^T: dims 32d + col, keys as above; a lane of the read points
+          // at 4 dims of key (lane/4)%4 of its 16-lane group's tile
+          const int vrow = n * 32 + sl * 16 + hh * 4 + ((lane & 15) >> 2);
+          const int vcol = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+#pragma unroll
+          for (int d = 0; d < HD / 32; d++) {
+            const int dim = d * 32 + vcol;
+            union { ap_s4 h[2]; ap_b8 v; } vf;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+              const int r = vrow + h * 8;
+              vf.h[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                  (__attribute__((address_space(3))) ap_s4*)(
+                      &Vs[cur][r * RB + v_slot<HD>(r, dim >> 3) * 16 +
+                               (dim & 7) * 2]));
+            }
+            o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf.v, o[d],
+                                                           0, 0, 0);
+          }
+        }
+      }
+    }
+    if constexpr (KV8) { if (more) store8(cur ^ 1); }
+    __syncthreads();
+    cur ^= 1;
+  }
+
+  l += __shfl_xor(l, 32);
+  if (row >= nrows) return;
+  if (gridDim.z == 1) {
+    const float inv = 1.f / l;
+    u16* op = a.out + ((size_t)my_m * a.nh + kvhead * grp + my_g) * HD;
+#pragma unroll
+    for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4++) {
+        union { ap_b2 b[2]; unsigned long long u; } w;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          w.b[j / 2][j % 2] = (__bf16)(o[d][q4 * 4 + j] * inv);
+        *(unsigned long long*)(op + d * 32 + q4 * 8 + hh * 4) = w.u;
+      }
+  } else {
+    // unnormalised part of this key range: HD values, maximum, sum
+    float* pp = a.part + (((size_t)blockIdx.z * a.kvh + kvhead) * nrows +
+                          row) * (HD + 4);
+#pragma unroll
+    for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4++)
+        *(f4v*)(pp + d * 32 + q4 * 8 + hh * 4) =
+            f4v{o[d][q4 * 4], o[d][q4 * 4 + 1], o[d][q4 * 4 + 2],
+                o[d][q4 * 4 + 3]};
+    if (hh == 0) { pp[HD] = m; pp[HD + 1] = l; }
+  }
+}
+
+// the parts of a row, one wave a row
+template <int HD>
+__global__ void __launch_bounds__(256) k_attn_rows_merge(ApArgs a, int split) {
+  const int lane = threadIdx.x & 63, grp = a.nh / a.kvh;
+  const int nrows = a.M * grp;
+  const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= nrows * a.kvh) return;
+  const int kvhead = w / nrows, row = w % nrows;
+  const size_t stride = (size_t)a.kvh * nrows * (HD + 4);
+  const float* p = a.part + ((size_t)kvhead * nrows + row) * (HD + 4);
+  float m = -INFINITY;
+  for (int z = 0; z < split; z++) m = fmaxf(m, p[z * stride + HD]);
+  float l = 0.f, v[HD / 64];
+#pragma unroll
+  for (int i = 0; i < HD / 64; i++) v[i] = 0.f;
+  for (int z = 0; z < split; z++) {
+    const float mz = p[z * stride + HD];
+    if (mz == -INFINITY) continue;
+    const float al = __builtin_amdgcn_exp2f(mz - m);
+    l += p[z * stride + HD + 1] * al;
+#pragma unroll
+    for (int i = 0; i < HD / 64; i++)
+      v[i] += p[z * stride + i * 64 + lane] * al;
+  }
+  u16* op = a.out + ((size_t)(row / grp) * a.nh + kvhead * grp + row % grp) * HD;
+#pragma unroll
+  for (int i = 0; i < HD / 64; i++) op[i * 64 + lane] = f2b(v[i] / l);
+}
+
+template <int HD, int BKV, int NW, bool KV8>
+static void ap_go(const ApArgs& a, dim3 grid, hipStream_t s) {
+  if (a.softcap > 0.f)
+    hipLaunchKernelGGL((k_attn_rows<HD, BKV, NW, KV8, true>), grid,
+                       dim3(64 * NW), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_attn_rows<HD, BKV, NW, KV8, false>), grid,
+                       dim3(64 * NW), 0, s, a);
+}
+
+template <int HD, int BKV>
+static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
+                         hipStream_t s) {
+  const int rows = a.M * (a.nh / a.kvh);
+  // up to 32 rows are one wave's; more share their tiles among four
+  const int nw = rows <= 32 ? 1 : 4;
+  const int tiles = (rows + nw * 32 - 1) / (nw * 32);
+  // Too few blocks for 256 CUs of two each: the keys are split too, down
+  // to four tiles a block.
+  int split = 1;
+  const int want = nw == 1 ? 1024 : 512;
+  if (tiles * a.kvh * 2 <= want && a.part) {
+    split = want / (tiles * a.kvh);
+    const int span = a.window > 0 ? (keys < a.window + a.M ? keys
+                                                           : a.window + a.M)
+                                  : keys;
+    const int most = span / (4 * BKV);
+    if (split > most) split = most;
+    if (split > 64) split = 64;
+    const long each = (long)a.kvh * rows * (HD + 4);
+    if (split > part_floats / each) split = (int)(part_floats / each);
+    if (split < 1) split = 1;
+  }
+  a.fold = split == 1 && tiles % 2 == 0 && tiles * a.kvh <= 512;
+  dim3 grid(a.kvh, tiles, split);
+  if (nw == 1) {
+    if (kv8) ap_go<HD, BKV, 1, true>(a, grid, s);
+    else ap_go<HD, BKV, 1, false>(a, grid, s);
+  } else {
+    if (kv8) ap_go<HD, BKV, 4, true>(a, grid, s);
+    else ap_go<HD, BKV, 4, false>(a, grid, s);
+  }
+  if (split > 1)
+    hipLaunchKernelGGL((k_attn_rows_merge<HD>), dim3((rows * a.kvh + 3) / 4),
+                       dim3(256), 0, s, a, split);
+  return hipGetLastError();
+}
+
+// keys: number of keys that the last row sees, as far as the host knows
+// (a hint for the split; the kernel goes by *len_ptr)
+extern "C" hipError_t launch_attn_prefill_mfma(
+    const void* q, const void* kc, const void* vc, void* out,
+    const void* len_ptr, const void* kS, const void* vS, void* part,
+    long part_floats, int kv8, int M, int nh, int kvh, int hd, int ldq,
+    int S, int keys, float scale, float softcap, int window,
+    hipStream_t stream) {
+  if (M < 1 || kvh < 1 || nh % kvh || ldq < nh * hd || ldq % 8)
+    return hipErrorInvalidValue;
+  ApArgs a = {(const u16*)q, kc, vc, (u16*)out, (const int*)len_ptr,
+              (const float*)kS, (const float*)vS, (float*)part, M, nh, kvh,
+              ldq, S, 0, scale, softcap, window};
+  if (hd == 64) return ap_run<64, 64>(a, kv8, keys, part_floats, stream);
+  if (hd == 128) return ap_run<128, 64>(a, kv8, keys, part_floats, stream);
+  if (hd == 256) return ap_run<256, 32>(a, kv8, keys, part_floats, stream);
+  return hipErrorInvalidValue;
+}

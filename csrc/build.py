@@ -30,7 +30,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "csrc")
 PKG = os.path.join(ROOT, "llm_np_cp_amd")
 LIBS = {
-    "llmops": ["llm_ops.hip", "xgmi_comm.hip"],
+    "llmops": ["llm_ops.hip", "attn_prefill.hip", "xgmi_comm.hip"],
     "linear": ["linear.hip"],
     "latent": ["latent_attn.hip"],
     "gqa": ["gqa_attn.hip"],
@@ -41,7 +41,7 @@ LIBS = {
     "lightning": ["lightning.hip"],
     "moe": ["moe.hip"],
 }
-HEADERS = ["attn_split.h", "common.h", "gemm_tile.h", "hybrid.h", "mingru.h",
+HEADERS = ["attn_prefill.h", "attn_split.h", "common.h", "gemm_tile.h", "hybrid.h", "mingru.h",
            "moe.h"]
 # Packed fp32 VALU forms are kept out of all device code: some of them
 # have returned wrong results on this hardware.  (The host pass warns that

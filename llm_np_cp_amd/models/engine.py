@@ -540,8 +540,9 @@ class GPUModel(DecodeLoop):
         return s if (s is None or self.max_batch == 1) else s[self._pb]
 
     def _layers_forward(self, M: int, layer_hook=None,
-                        batch_attn: bool = False):
-        """Layer stack over rows [0, M).  ``batch_attn``: rows are M
+                        batch_attn: bool = False, keys: int = 0):
+        """Layer stack over rows [0, M), the last of which sees ``keys``
+        keys.  ``batch_attn``: rows are M
         INDEPENDENT sequences at the same position (lockstep batched
         decode) — the fused decode-attention kernel runs per row over
         per-sequence KV pools instead of the prefill attention."""
@@ -582,7 +583,8 @@ class GPUModel(DecodeLoop):
                         self.len_buf, M, self.nh_l, self.kvh_l, self.hd,
                         self.scale, softcap=self.attn_softcap,
                         window=window or 0,
-                        kS=self._ks(i), vS=self._vs(i))
+                        kS=self._ks(i), vS=self._vs(i),
+                        part=self.b_gemm_acc, keys=keys)
                 else:
                     # per-query VALU kernel: every production head_dim is
                     # 64/128/256 (MFMA above); kept as the documented
@@ -718,7 +720,7 @@ class GPUModel(DecodeLoop):
                 torch.cuda.synchronize()
                 hidden[i + 1][d0:d0 + h.shape[0]] = \
                     h.float().cpu().numpy()
-            self._layers_forward(M, layer_hook=hook)
+            self._layers_forward(M, layer_hook=hook, keys=done + M)
             ho.rmsnorm(self.b_h[:M], self.g_final, self.b_xn[:M],
                        eps=self.config.rms_norm_eps)
             if self.wq4:
@@ -781,7 +783,7 @@ class GPUModel(DecodeLoop):
             ho.i32_set(self.len_buf, pos0 + done)
             ho.embed(self.embed, self.ids_buf, self.b_h, M,
                      self.config.embed_scale)
-            self._layers_forward(M)
+            self._layers_forward(M, keys=pos0 + done + M)
             ho.rmsnorm(self.b_h[:M], self.g_final, self.b_xn[:M],
                        eps=self.config.rms_norm_eps)
             if self.wq4:
@@ -848,7 +850,7 @@ class GPUModel(DecodeLoop):
             ho.i32_set(self.len_buf, pos0 + done)
             ho.embed(self.embed, self.ids_buf, self.b_h, M,
                      self.config.embed_scale)
-            self._layers_forward(M)
+            self._layers_forward(M, keys=pos0 + done + M)
             done += M
         ho.i32_set(self.len_buf, pos0 + n)
         self._host_len = pos0 + n
@@ -1272,7 +1274,7 @@ class GPUModel(DecodeLoop):
                 ho.i32_set(self.len_buf, done)
                 ho.embed(self.embed, self.ids_buf, self.b_h, M,
                          self.config.embed_scale)
-                self._layers_forward(M)
+                self._layers_forward(M, keys=done + M)
                 done += M
             self._lm_head_last(M)
             self.bt_logits32[b].copy_(self.b_logits)
@@ -1303,7 +1305,7 @@ class GPUModel(DecodeLoop):
             ho.i32_set(self.len_buf, done)
             ho.embed(self.embed, self.ids_buf, self.b_h, M,
                      self.config.embed_scale)
-            self._layers_forward(M)
+            self._layers_forward(M, keys=done + M)
             done += M
         self._lm_head_last(M)
         self._pb = 0

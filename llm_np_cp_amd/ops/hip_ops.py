@@ -42,7 +42,8 @@ _SIGS = {
     "launch_attn": [ctypes.c_void_p] * 7 + [ctypes.c_int] * 6 +
                    [ctypes.c_float, ctypes.c_float, ctypes.c_int,
                     ctypes.c_void_p],
-    "launch_attn_prefill_mfma": [ctypes.c_void_p] * 7 + [ctypes.c_int] * 6 +
+    "launch_attn_prefill_mfma": [ctypes.c_void_p] * 8 + [ctypes.c_long] +
+                                [ctypes.c_int] * 8 +
                                 [ctypes.c_float, ctypes.c_float,
                                  ctypes.c_int, ctypes.c_void_p],
     "launch_attn_dec": [ctypes.c_void_p] * 9 + [ctypes.c_int] +
@@ -252,15 +253,20 @@ def attn_prefill_mfma(q: torch.Tensor, k_cache: torch.Tensor,
                       len_ptr: torch.Tensor, M: int, nh: int, kvh: int,
                       hd: int, scale: float, softcap: float = 0.0,
                       window: int = 0, kS: torch.Tensor | None = None,
-                      vS: torch.Tensor | None = None):
+                      vS: torch.Tensor | None = None,
+                      part: torch.Tensor | None = None, keys: int = 0):
     """Flash prefill attention (MFMA, online softmax); q already roped,
-    caches already written for [0, pos0+M)."""
+    caches already written for [0, pos0+M).  With part (fp32 scratch) few
+    rows split their keys over more blocks; keys (pos0+M, as far as the
+    host knows) sizes that split."""
     S = k_cache.shape[1]
     _check(lib().launch_attn_prefill_mfma(
         _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(len_ptr),
-        _ptr(kS), _ptr(vS), 1 if kS is not None else 0,
-        M, nh, kvh, hd, S, ctypes.c_float(scale), ctypes.c_float(softcap),
-        window, _stream()), "attn_prefill_mfma")
+        _ptr(kS), _ptr(vS), _ptr(part),
+        ctypes.c_long(0 if part is None else part.numel()),
+        1 if kS is not None else 0,
+        M, nh, kvh, hd, nh * hd, S, max(keys, M), ctypes.c_float(scale),
+        ctypes.c_float(softcap), window, _stream()), "attn_prefill_mfma")
 
 
 def attn_dec(qkv: torch.Tensor, k_cache: torch.Tensor,
