@@ -904,239 +904,6 @@ extern "C" hipError_t launch_gemv_fp8_mx(
 }
 
 // ====================================================================
-// Skinny fp8 MFMA GEMM pair (batched decode, B = 3..16): matrix cores
-// own the MACs — the multi-x GEMV above is VALU-ISSUE-bound beyond B=2
-// (128 irreducible FMAs per 16 weight bytes at B=8).
-//   1. k_stage_quant_mx: per sequence row, apply the staging op
-//      (RAW/NORM/GLU/NORM2/NORM_EMBED) and quantize to e4m3 + scale
-//      (one block per row; row stats need full-K visibility).
-//   2. k_gemm_fp8_skinny: Y[B,N] = (sx_b*sw_n) * Xq[B,K] @ Wq[N,K]^T
-//      with ONE 16-row mfma_f32_16x16x32_fp8_fp8 tile per wave — W is
-//      nt-streamed exactly once; Xq re-reads stay L2-hot (~N*K/4 B).
-// ====================================================================
-
-extern "C" __global__ void k_zero_f32(float* p, long total);
-
-extern "C" __global__ void __launch_bounds__(256)
-k_stage_quant_mx(const u16* __restrict__ x, long xstride,
-                 const u16* __restrict__ x2, long x2stride,
-                 const float* __restrict__ g, const float* __restrict__ g2,
-                 uint8_t* __restrict__ xq, float* __restrict__ sx,
-                 u16* __restrict__ hout, long hstride, int K, int B,
-                 int stage, int act, float eps, float escale) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* red = (float*)(smem + (size_t)K * 4);
-  const int b = blockIdx.x;
-  const u16* xb = x + (size_t)b * xstride;
-  if (stage == STAGE_NORM_EMBED)
-    xb = x + (size_t)((const int*)x2)[b] * (size_t)K;
-  const u16* x2b = (stage == STAGE_NORM_EMBED || x2 == nullptr)
-                       ? nullptr : x2 + (size_t)b * x2stride;
-  u16* houtb = hout ? hout + (size_t)b * hstride : nullptr;
-  // stage into f32 LDS (row stats via the shared per-row helper)
-  gemv_stage_mx_row<true>(smem, 0, xb, x2b, g, g2, houtb, K, 1, stage,
-                          act, eps, escale, red, true);
-  __syncthreads();
-  // absmax -> scale -> quantize to global
-  const float* xf = (const float*)smem;
-  float am = 0.f;
-  for (int i = threadIdx.x; i < K; i += 256) am = fmaxf(am, fabsf(xf[i]));
-#pragma unroll
-  for (int w = 1; w < 64; w <<= 1) am = fmaxf(am, __shfl_xor(am, w));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = am;
-  __syncthreads();
-  am = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  float sc = fmaxf(am, 1e-8f) / 448.0f;
-  if (threadIdx.x == 0) sx[b] = sc;
-  const float rs = 1.0f / sc;
-  uint8_t* q = xq + (size_t)b * K;
-  for (int i = threadIdx.x * 8; i < K; i += 2048) {
-    uint32_t lo = 0, hi = 0;
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(xf[i] * rs, xf[i + 1] * rs, lo,
-                                         false);
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(xf[i + 2] * rs, xf[i + 3] * rs,
-                                         lo, true);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(xf[i + 4] * rs, xf[i + 5] * rs,
-                                         hi, false);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(xf[i + 6] * rs, xf[i + 7] * rs,
-                                         hi, true);
-    *(uint32_t*)(q + i) = lo;
-    *(uint32_t*)(q + i + 4) = hi;
-  }
-}
-
-extern "C" hipError_t launch_stage_quant_mx(
-    const void* x, long xstride, const void* x2, long x2stride,
-    const void* g, const void* g2, void* xq, void* sx, void* hout,
-    long hstride, int K, int B, int stage, int act, float eps,
-    float escale, hipStream_t stream) {
-  size_t lds = (size_t)K * 4 + 64;
-  if (lds > 160 * 1024 || K % 16 != 0) return hipErrorInvalidValue;
-  static bool raised = false;
-  if (lds > 65536 && !raised) {
-    hipFuncSetAttribute((const void*)&k_stage_quant_mx,
-                        hipFuncAttributeMaxDynamicSharedMemorySize,
-                        160 * 1024);
-    raised = true;
-  }
-  hipLaunchKernelGGL(k_stage_quant_mx, dim3(B), dim3(256), lds, stream,
-                     (const u16*)x, xstride, (const u16*)x2, x2stride,
-                     (const float*)g, (const float*)g2, (uint8_t*)xq,
-                     (float*)sx, (u16*)hout, hstride, K, B, stage, act,
-                     eps, escale);
-  return hipGetLastError();
-}
-
-// one 16x16 output tile per wave; acc row = X row (B dim), col = W row.
-// TWO interleaved 64-byte K-chains per wave (independent mfma
-// accumulators — the dependent-chain latency was the v1 bound) and a
-// K-split grid.y for small-N occupancy (atomicAdd into an fp32 accbuf,
-// scales/epilogue applied by k_skinny_fin).
-extern "C" __global__ void __launch_bounds__(256)
-k_gemm_fp8_skinny(const uint8_t* __restrict__ Xq,
-                  const float* __restrict__ sx,
-                  const uint8_t* __restrict__ Wq,
-                  const float* __restrict__ sw, void* __restrict__ y,
-                  long ystride, const u16* __restrict__ res, long rstride,
-                  const u16* __restrict__ bias, float* __restrict__ accbuf,
-                  int out_f32, float softcap, int B, int N, int K) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int fr = lane & 15, fk8 = (lane >> 4) * 8;
-  const int asrc = fr < B ? fr : 0;  // padded A rows read row 0
-  const uint8_t* Xr = Xq + (size_t)asrc * K + fk8;
-  const int SK = gridDim.y;
-  const int kchunks = (K / 32 + SK - 1) / SK;
-  const int k_lo = blockIdx.y * kchunks * 32;
-  int k_hi = k_lo + kchunks * 32;
-  if (k_hi > K) k_hi = K;
-  if (k_hi <= k_lo) return;
-  for (int n0 = (blockIdx.x * 4 + wave) * 16; n0 < N;
-       n0 += gridDim.x * 4 * 16) {
-    int wr = n0 + fr;
-    if (wr >= N) wr = N - 1;
-    const uint8_t* Wr = Wq + (size_t)wr * K + fk8;
-    f4v acc_a = {0.f, 0.f, 0.f, 0.f};
-    f4v acc_b = {0.f, 0.f, 0.f, 0.f};
-    f4v acc_c = {0.f, 0.f, 0.f, 0.f};
-    f4v acc_d = {0.f, 0.f, 0.f, 0.f};
-    int k = k_lo;
-    // 4 independent chains x 256 B: PMC showed waves PARKED on memory
-    // 69% of cycles with only 2 chains in flight
-    for (; k + 256 <= k_hi; k += 256) {
-      long a0 = *(const long*)(Xr + k);
-      long b0 = __builtin_nontemporal_load((const long*)(Wr + k));
-      long a1 = *(const long*)(Xr + k + 32);
-      long b1 = __builtin_nontemporal_load((const long*)(Wr + k + 32));
-      long a2 = *(const long*)(Xr + k + 64);
-      long b2 = __builtin_nontemporal_load((const long*)(Wr + k + 64));
-      long a3 = *(const long*)(Xr + k + 96);
-      long b3 = __builtin_nontemporal_load((const long*)(Wr + k + 96));
-      long a4 = *(const long*)(Xr + k + 128);
-      long b4 = __builtin_nontemporal_load((const long*)(Wr + k + 128));
-      long a5 = *(const long*)(Xr + k + 160);
-      long b5 = __builtin_nontemporal_load((const long*)(Wr + k + 160));
-      long a6 = *(const long*)(Xr + k + 192);
-      long b6 = __builtin_nontemporal_load((const long*)(Wr + k + 192));
-      long a7 = *(const long*)(Xr + k + 224);
-      long b7 = __builtin_nontemporal_load((const long*)(Wr + k + 224));
-      acc_a = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a0, b0, acc_a,
-                                                         0, 0, 0);
-      acc_b = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a1, b1, acc_b,
-                                                         0, 0, 0);
-      acc_c = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a2, b2, acc_c,
-                                                         0, 0, 0);
-      acc_d = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a3, b3, acc_d,
-                                                         0, 0, 0);
-      acc_a = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a4, b4, acc_a,
-                                                         0, 0, 0);
-      acc_b = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a5, b5, acc_b,
-                                                         0, 0, 0);
-      acc_c = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a6, b6, acc_c,
-                                                         0, 0, 0);
-      acc_d = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a7, b7, acc_d,
-                                                         0, 0, 0);
-    }
-    for (; k < k_hi; k += 32) {
-      long a0 = *(const long*)(Xr + k);
-      long b0 = __builtin_nontemporal_load((const long*)(Wr + k));
-      acc_a = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(a0, b0, acc_a,
-                                                         0, 0, 0);
-    }
-    const int col = n0 + fr;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int b = (lane >> 4) * 4 + r;
-      if (b < B && col < N) {
-        float v = (acc_a[r] + acc_b[r]) + (acc_c[r] + acc_d[r]);
-        if (SK > 1) {
-          atomicAdd(accbuf + (size_t)b * N + col, v);
-        } else {
-          v *= sx[b] * sw[col];
-          if (softcap > 0.f) v = softcap * tanhf(v / softcap);
-          if (bias) v += b2f(bias[col]);
-          if (res) v += b2f(res[(size_t)b * rstride + col]);
-          if (out_f32) ((float*)y)[(size_t)b * ystride + col] = v;
-          else ((u16*)y)[(size_t)b * ystride + col] = f2b(v);
-        }
-      }
-    }
-  }
-}
-
-// SK>1 epilogue: raw sums -> scales/softcap/bias/res -> y
-extern "C" __global__ void __launch_bounds__(256)
-k_skinny_fin(const float* __restrict__ accbuf, const float* __restrict__ sx,
-             const float* __restrict__ sw, void* __restrict__ y,
-             long ystride, const u16* __restrict__ res, long rstride,
-             const u16* __restrict__ bias, int out_f32, float softcap,
-             int B, int N) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long)B * N) return;
-  const int b = (int)(i / N), col = (int)(i % N);
-  float v = accbuf[(size_t)b * N + col] * sx[b] * sw[col];
-  if (softcap > 0.f) v = softcap * tanhf(v / softcap);
-  if (bias) v += b2f(bias[col]);
-  if (res) v += b2f(res[(size_t)b * rstride + col]);
-  if (out_f32) ((float*)y)[(size_t)b * ystride + col] = v;
-  else ((u16*)y)[(size_t)b * ystride + col] = f2b(v);
-}
-
-extern "C" hipError_t launch_gemm_fp8_skinny(
-    const void* Xq, const void* sx, const void* Wq, const void* sw,
-    void* y, long ystride, const void* res, long rstride, const void* bias,
-    void* accbuf, int out_f32, float softcap, int B, int N, int K,
-    hipStream_t stream) {
-  if (B < 1 || B > 16 || K % 32 != 0) return hipErrorInvalidValue;
-  int blocks = (N + 63) / 64;
-  if (blocks > 1024) blocks = 1024;
-  int sk = 1;
-  if (accbuf && blocks < 512) {
-    sk = 512 / blocks;
-    if (sk > 8) sk = 8;
-    while (sk > 1 && K / 32 < sk) sk--;
-  }
-  if (sk > 1) {
-    long total = (long)B * N;
-    hipLaunchKernelGGL(k_zero_f32, dim3((uint32_t)((total + 1023) / 1024)),
-                       dim3(256), 0, stream, (float*)accbuf, total);
-  }
-  hipLaunchKernelGGL(k_gemm_fp8_skinny, dim3(blocks, sk), dim3(256), 0,
-                     stream, (const uint8_t*)Xq, (const float*)sx,
-                     (const uint8_t*)Wq, (const float*)sw, y, ystride,
-                     (const u16*)res, rstride, (const u16*)bias,
-                     (float*)accbuf, out_f32, softcap, B, N, K);
-  if (sk > 1) {
-    long total = (long)B * N;
-    hipLaunchKernelGGL(k_skinny_fin, dim3((uint32_t)((total + 255) / 256)),
-                       dim3(256), 0, stream, (const float*)accbuf,
-                       (const float*)sx, (const float*)sw, y, ystride,
-                       (const u16*)res, rstride, (const u16*)bias, out_f32,
-                       softcap, B, N);
-  }
-  return hipGetLastError();
-}
-
-// ====================================================================
 // MXFP4 GEMV: y[N] = W4[N,K] @ stage(x)[K] (+res); 2 fp4/byte with one
 // e8m0 scale per 32 elements.  Same packed structure as the fp8 GEMV
 // (fp32 x staging or XDIR direct reads feeding fp32 FMAs) — the
@@ -1414,7 +1181,7 @@ k_rope_cache(u16* __restrict__ q, const u16* __restrict__ kin,
              const u16* __restrict__ vin, u16* __restrict__ kc,
              u16* __restrict__ vc, const float* __restrict__ cost,
              const float* __restrict__ sint, const int* __restrict__ pos_ptr,
-             int nh, int kvh, int hd, int S) {
+             int nh, int kvh, int hd, int S, int ldq, int ldkv) {
   const int m = blockIdx.x;
   const int pos = *pos_ptr + m;
   const int hd2 = hd / 2;
@@ -1422,7 +1189,7 @@ k_rope_cache(u16* __restrict__ q, const u16* __restrict__ kin,
   const float* sp = sint + (size_t)pos * hd2;
 
   // q rotation in place
-  u16* qr = q + (size_t)m * nh * hd;
+  u16* qr = q + (size_t)m * ldq;
   for (int idx = threadIdx.x; idx < nh * hd2; idx += 256) {
     int h = idx / hd2, i = idx % hd2;
     float x1 = b2f(qr[h * hd + i]);
@@ -1432,8 +1199,8 @@ k_rope_cache(u16* __restrict__ q, const u16* __restrict__ kin,
     qr[h * hd + i + hd2] = f2b(x2 * c + x1 * s);
   }
   // k rotation -> cache; v copy -> cache
-  const u16* kr = kin + (size_t)m * kvh * hd;
-  const u16* vr = vin + (size_t)m * kvh * hd;
+  const u16* kr = kin + (size_t)m * ldkv;
+  const u16* vr = vin + (size_t)m * ldkv;
   for (int idx = threadIdx.x; idx < kvh * hd2; idx += 256) {
     int h = idx / hd2, i = idx % hd2;
     float x1 = b2f(kr[h * hd + i]);
@@ -1460,7 +1227,7 @@ k_rope_cache_fp8(u16* __restrict__ q, const u16* __restrict__ kin,
                  float* __restrict__ vS, const float* __restrict__ cost,
                  const float* __restrict__ sint,
                  const int* __restrict__ pos_ptr,
-                 int nh, int kvh, int hd, int S) {
+                 int nh, int kvh, int hd, int S, int ldq, int ldkv) {
   __shared__ float row[256];
   __shared__ float red[4];
   const int m = blockIdx.x;
@@ -1471,7 +1238,7 @@ k_rope_cache_fp8(u16* __restrict__ q, const u16* __restrict__ kin,
   const int tid = threadIdx.x;
 
   // q rotation in place (q stays bf16)
-  u16* qr = q + (size_t)m * nh * hd;
+  u16* qr = q + (size_t)m * ldq;
   for (int idx = tid; idx < nh * hd2; idx += 256) {
     int h = idx / hd2, i = idx % hd2;
     float x1 = b2f(qr[h * hd + i]);
@@ -1481,8 +1248,8 @@ k_rope_cache_fp8(u16* __restrict__ q, const u16* __restrict__ kin,
     qr[h * hd + i + hd2] = f2b(x2 * c + x1 * s);
   }
 
-  const u16* kr = kin + (size_t)m * kvh * hd;
-  const u16* vr = vin + (size_t)m * kvh * hd;
+  const u16* kr = kin + (size_t)m * ldkv;
+  const u16* vr = vin + (size_t)m * ldkv;
   for (int h = 0; h < kvh; h++) {
     // rotated k row -> LDS floats
     __syncthreads();
@@ -1530,19 +1297,19 @@ extern "C" hipError_t launch_rope_cache(void* q, const void* kin,
                                         void* kS, void* vS, int kv8,
                                         const void* cost, const void* sint,
                                         const void* pos_ptr, int M, int nh,
-                                        int kvh, int hd, int S,
-                                        hipStream_t stream) {
+                                        int kvh, int hd, int S, int ldq,
+                                        int ldkv, hipStream_t stream) {
   if (kv8) {
     hipLaunchKernelGGL(k_rope_cache_fp8, dim3(M), dim3(256), 0, stream,
                        (u16*)q, (const u16*)kin, (const u16*)vin,
                        (uint8_t*)kc, (uint8_t*)vc, (float*)kS, (float*)vS,
                        (const float*)cost, (const float*)sint,
-                       (const int*)pos_ptr, nh, kvh, hd, S);
+                       (const int*)pos_ptr, nh, kvh, hd, S, ldq, ldkv);
   } else {
     hipLaunchKernelGGL(k_rope_cache, dim3(M), dim3(256), 0, stream, (u16*)q,
                        (const u16*)kin, (const u16*)vin, (u16*)kc, (u16*)vc,
                        (const float*)cost, (const float*)sint,
-                       (const int*)pos_ptr, nh, kvh, hd, S);
+                       (const int*)pos_ptr, nh, kvh, hd, S, ldq, ldkv);
   }
   return hipGetLastError();
 }
@@ -1566,7 +1333,7 @@ __global__ void __launch_bounds__(256)
 k_attn_t(const u16* __restrict__ q, const void* __restrict__ kc,
          const void* __restrict__ vc, u16* __restrict__ out,
          const int* __restrict__ len_ptr, const float* __restrict__ kS,
-         const float* __restrict__ vS, int nh, int kvh, int hd, int S,
+         const float* __restrict__ vS, int nh, int kvh, int hd, int ldq, int S,
          float scale, float softcap, int window) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float* red = (float*)smem;  // [4][hd] acc + [4][2] m,l
@@ -1586,7 +1353,7 @@ k_attn_t(const u16* __restrict__ q, const void* __restrict__ kc,
   // q fragment for this head (8 dims), fp32
   float qf[8];
   {
-    s8v v = *(const s8v*)(q + ((size_t)m * nh + h) * hd + d0);
+    s8v v = *(const s8v*)(q + (size_t)m * ldq + h * hd + d0);
 #pragma unroll
     for (int j = 0; j < 8; j++) qf[j] = b2f(((u16*)&v)[j]);
   }
@@ -2103,7 +1870,7 @@ extern "C" hipError_t launch_attn(const void* q, const void* kc,
                                   const void* vc, void* out,
                                   const void* len_ptr, const void* kS,
                                   const void* vS, int kv8, int M, int nh,
-                                  int kvh, int hd, int S, float scale,
+                                  int kvh, int hd, int ldq, int S, float scale,
                                   float softcap, int window,
                                   hipStream_t stream) {
   size_t lds = (4 * hd + 8) * sizeof(float);
@@ -2111,7 +1878,7 @@ extern "C" hipError_t launch_attn(const void* q, const void* kc,
   hipLaunchKernelGGL((k_attn_t<KV8V>), dim3(nh, M), dim3(256), lds, stream, \
                      (const u16*)q, kc, vc, (u16*)out,                      \
                      (const int*)len_ptr, (const float*)kS,                 \
-                     (const float*)vS, nh, kvh, hd, S, scale, softcap,      \
+                     (const float*)vS, nh, kvh, hd, ldq, S, scale, softcap, \
                      window)
   if (kv8) ATTN_CASE(true);
   else ATTN_CASE(false);
@@ -2556,49 +2323,78 @@ extern "C" hipError_t launch_quant_fp4(const void* X, void* Q, void* E,
 // HW convert: v_cvt_pk_fp8_f32 (OCP e4m3fn on gfx950, saturating).
 // ====================================================================
 
-extern "C" __global__ void __launch_bounds__(256)
-k_quant_fp8_rows(const u16* __restrict__ X, uint8_t* __restrict__ Q,
+// Few rows take 1024 threads each (a row is then read once, into registers;
+// 16 rows of 14336: 2.7 us, by 256 threads 4.4), many rows 256.
+DEVINL void load8(const u16* p, float* f) {
+  const s8v v = *(const s8v*)p;
+#pragma unroll
+  for (int j = 0; j < 8; j++) f[j] = b2f(((u16*)&v)[j]);
+}
+DEVINL void load8(const float* p, float* f) {
+  *(f4v*)f = *(const f4v*)p;
+  *(f4v*)(f + 4) = *(const f4v*)(p + 4);
+}
+
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT)
+k_quant_fp8_rows(const T* __restrict__ X, uint8_t* __restrict__ Q,
                  float* __restrict__ S, int K) {
-  __shared__ float wmax[4];
+  constexpr int KEEP = 3;                    // chunks that stay in registers
+  __shared__ float wmax[NT / 64];
   const int row = blockIdx.x;
-  const u16* xr = X + (size_t)row * K;
+  const T* xr = X + (size_t)row * K;
   uint8_t* qr = Q + (size_t)row * K;
 
-  float amax = 0.f;
-  for (int i = threadIdx.x * 8; i < K; i += 2048) {
-    s8v v = *(const s8v*)(xr + i);
+  float amax = 0.f, kept[KEEP][8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(b2f(((u16*)&v)[j])));
+  for (int c = 0; c < KEEP; c++) {
+    const int i = (c * NT + threadIdx.x) * 8;
+    if (i < K) {
+      load8(xr + i, kept[c]);
+#pragma unroll
+      for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(kept[c][j]));
+    }
+  }
+  for (int i = (KEEP * NT + threadIdx.x) * 8; i < K; i += NT * 8) {
+    float f[8];
+    load8(xr + i, f);
+#pragma unroll
+    for (int j = 0; j < 8; j++) amax = fmaxf(amax, fabsf(f[j]));
   }
 #pragma unroll
   for (int m = 1; m < 64; m <<= 1) amax = fmaxf(amax, __shfl_xor(amax, m));
   if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = amax;
   __syncthreads();
-  amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+#pragma unroll
+  for (int w = 0; w < NT / 64; w++) amax = fmaxf(amax, wmax[w]);
   const float s = fmaxf(amax, 1e-8f) / 448.0f;
   const float rs = 1.0f / s;
   if (threadIdx.x == 0) S[row] = s;
 
-  for (int i = threadIdx.x * 8; i < K; i += 2048) {
-    s8v v = *(const s8v*)(xr + i);
-    float f[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) f[j] = b2f(((u16*)&v)[j]) * rs;
-    uint32_t lo = 0, hi = 0;
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], lo, false);
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], hi, false);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], hi, true);
-    *(uint32_t*)(qr + i) = lo;
-    *(uint32_t*)(qr + i + 4) = hi;
+  for (int c = 0; c < KEEP; c++) {
+    const int i = (c * NT + threadIdx.x) * 8;
+    if (i < K)
+      *(unsigned long long*)(qr + i) = f32x8_to_fp8(kept[c], rs);
+  }
+  for (int i = (KEEP * NT + threadIdx.x) * 8; i < K; i += NT * 8) {
+    float f[8];
+    load8(xr + i, f);
+    *(unsigned long long*)(qr + i) = f32x8_to_fp8(f, rs);
   }
 }
 
 extern "C" hipError_t launch_quant_fp8(const void* X, void* Q, void* S,
-                                       int M, int K, hipStream_t stream) {
+                                       int f32, int M, int K,
+                                       hipStream_t stream) {
   if (K % 8 != 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_quant_fp8_rows, dim3(M), dim3(256), 0, stream,
-                     (const u16*)X, (uint8_t*)Q, (float*)S, K);
+#define QUANT_CASE(T, NT)                                                    \
+  hipLaunchKernelGGL((k_quant_fp8_rows<T, NT>), dim3(M), dim3(NT), 0, stream, \
+                     (const T*)X, (uint8_t*)Q, (float*)S, K)
+  const bool few = M <= 64 && K > 2048;
+  if (f32) { if (few) QUANT_CASE(float, 1024); else QUANT_CASE(float, 256); }
+  else { if (few) QUANT_CASE(u16, 1024); else QUANT_CASE(u16, 256); }
+#undef QUANT_CASE
   return hipGetLastError();
 }
 

@@ -58,7 +58,7 @@ class GPUModel(DecodeLoop):
         # copy (the fp8 machinery flag covers both quantized modes)
         self.fp8 = dtype in ("fp8", "fp4")
         self.wq4 = dtype == "fp4"
-        # fp4 + batch pools: the skinny MFMA GEMM consumes fp8, so keep
+        # fp4 + batch pools: a group's decode steps run on fp8, so keep
         # the fp8 copy only then; max_batch=1 fp4 engines are SINGLE-COPY
         self.keep_fp8 = (dtype == "fp8") or (self.wq4 and max_batch > 1)
         if kv_dtype not in ("bf16", "fp8"):
@@ -364,9 +364,9 @@ class GPUModel(DecodeLoop):
         self.b_h = torch.zeros(PC, H, **bf)
         self.b_xn = torch.zeros(PC, H, **bf)
         self.b_t1 = torch.zeros(PC, H, **bf)
-        self.b_q = torch.zeros(PC, self.nh_l * hd, **bf)
-        self.b_k = torch.zeros(PC, self.kvh_l * hd, **bf)
-        self.b_v = torch.zeros(PC, self.kvh_l * hd, **bf)
+        # q | k | v of a row, from one projection
+        self.b_rqkv = torch.zeros(PC, (self.nh_l + 2 * self.kvh_l) * hd,
+                                  **bf)
         self.b_att = torch.zeros(PC, self.nh_l * hd, **bf)
         self.b_gate = torch.zeros(PC, I, **bf)
         self.b_up = torch.zeros(PC, I, **bf)
@@ -377,6 +377,12 @@ class GPUModel(DecodeLoop):
             kmax = max(H, I, self.nh_l * hd)
             self.b_xq = torch.zeros(PC * kmax, dtype=torch.uint8, device=dev)
             self.b_sx = torch.zeros(PC, dtype=torch.float32, device=dev)
+            # act(gate) * up of few rows, to be rounded to e4m3 next
+            self.b_act32 = torch.zeros(ho.FEW_ROWS, I, dtype=torch.float32,
+                                       device=dev)
+        # few-row products that split K: blocks that are done, by column
+        # group (the parts go to b_gemm_acc)
+        self.row_cnt = torch.zeros(256, dtype=torch.int32, device=dev)
         self.b_logits_l = torch.zeros(self.vocab_l, dtype=torch.float32,
                                       device=dev)
         self.b_logits = (self.b_logits_l if not self.tp_branch else
@@ -419,8 +425,7 @@ class GPUModel(DecodeLoop):
         if self.max_batch > 1:
             B, nhh = self.max_batch, self.nh_l * hd
             i64 = dict(dtype=torch.int64, device=dev)
-            self.bt_qkv = torch.zeros(B, (self.nh_l + 2 * self.kvh_l) * hd,
-                                      **bf)
+            self.bt_qkv = self.b_rqkv[:B]
             self.bt_logits = torch.zeros(B, self.vocab_l, **bf)
             self.bt_logits32 = torch.zeros(B, cfg.vocab_size,
                                            dtype=torch.float32, device=dev)
@@ -462,20 +467,52 @@ class GPUModel(DecodeLoop):
     # ------------------------------------------------------------------
     # layer stack over rows [0, M) of the scratch buffers
     # ------------------------------------------------------------------
+    def _rows(self, lw, name, x, y, M: int, g=None, res=None, bias=None,
+              act: int = -1, softcap: float = 0.0, batch: bool = False):
+        """Projection of up to FEW_ROWS rows in one launch, W streamed
+        once: norm of x (g), activation of gate and up rows (act), softcap,
+        bias and residual on the way.  Rows beside e4m3 weights are rounded
+        to e4m3, a row alone is not (GEMV).  ``batch``: a decode step of a
+        group, which runs on the e4m3 copy where the engine holds MXFP4
+        too."""
+        eps = self.config.rms_norm_eps
+        e4m3 = self.fp8 and (batch or not self.wq4)
+        if e4m3 and M == 1:
+            if g is not None:
+                ho.rmsnorm(x[:1], g, self.b_xn[:1], eps=eps)
+                x = self.b_xn
+            w, s = lw[name + "_q"], lw[name + "_s"]
+            if act < 0:
+                ho.gemv_fp8(w, s, x, y, res=res if bias is None else bias,
+                            softcap=softcap)
+                return
+            n = w.shape[0] // 2
+            ho.gemv_fp8(w, s, x, self.b_gu)
+            ho.glu(self.b_gu[:n], self.b_gu[n:], y[:1], act)
+            return
+        if g is not None and x.shape[-1] > ho.ROW_NORM_K:
+            ho.rmsnorm(x[:M], g, self.b_xn[:M], eps=eps)
+            x, g = self.b_xn, None
+        kw = dict(g=g, eps=eps, res=res, bias=bias, act=act, softcap=softcap,
+                  part=self.b_gemm_acc, cnt=self.row_cnt)
+        if e4m3:
+            if g is None:
+                K = x.shape[-1]
+                ho.quant_fp8(x[:M], self.b_xq, self.b_sx)
+                x, kw["sx"] = self.b_xq[:M * K].view(M, K), self.b_sx
+            ho.row_gemm(x, lw[name + "_q"], y, M, ws=lw[name + "_s"], **kw)
+        elif self.wq4:
+            ho.row_gemm(x, lw[name + "_q4"], y, M, we=lw[name + "_e4"], **kw)
+        else:
+            ho.row_gemm(x, lw[name], y, M, **kw)
+
     def _linear(self, lw, name, x, y, res=None, M: int = 1,
-                softcap: float = 0.0):
+                batch: bool = False):
         """Projection by weight NAME so dtype routing stays in one
-        place: bf16 GEMV/MFMA-GEMM, or (fp8) GEMV / fp8-MFMA GEMM with
+        place: few rows, bf16 MFMA GEMM, or (fp8) fp8-MFMA GEMM with
         on-the-fly activation row quantization."""
-        if M == 1:
-            if self.wq4:
-                ho.gemv_fp4(lw[name + "_q4"], lw[name + "_e4"], x, y,
-                            res=res, softcap=softcap)
-            elif self.fp8:
-                ho.gemv_fp8(lw[name + "_q"], lw[name + "_s"], x, y,
-                            res=res, softcap=softcap)
-            else:
-                ho.gemv(lw[name], x, y, res=res, softcap=softcap)
+        if M <= ho.FEW_ROWS:
+            self._rows(lw, name, x, y, M, res=res, batch=batch)
         elif self.wq4:
             ho.gemm_fp4w(x[:M], lw[name + "_q4"], lw[name + "_e4"], y[:M],
                          res=res[:M] if res is not None else None,
@@ -491,14 +528,14 @@ class GPUModel(DecodeLoop):
             ho.gemm(x[:M], lw[name], y, res=res[:M] if res is not None else None,
                     accbuf=self.b_gemm_acc)
 
-    def _rowpar_ar(self, lw, name, x, y, M: int):
+    def _rowpar_ar(self, lw, name, x, y, M: int, batch: bool = False):
         """Row-parallel projection followed by all-reduce over TP ranks.
         For prefill-sized M the rows are split in two: the all-reduce of
         chunk A runs on RCCL's comm stream while chunk B's GEMM occupies
         the compute stream (SURVEY §2.3 'overlap comm on 2nd stream' —
         the reference has no distributed code at all)."""
         if not (self._async_ar and M >= 512):
-            self._linear(lw, name, x, y, M=M)
+            self._linear(lw, name, x, y, M=M, batch=batch)
             tpu.all_reduce(y[:M])
             return
         import torch.distributed as dist
@@ -549,16 +586,37 @@ class GPUModel(DecodeLoop):
         cfg = self.config
         eps = cfg.rms_norm_eps
         h, xn, t1 = self.b_h, self.b_xn, self.b_t1
+        few = M <= ho.FEW_ROWS
+        qkv = self.b_rqkv[:M]
+        nq, nkv = self.nh_l * self.hd, self.kvh_l * self.hd
+        q, k, v = qkv.split([nq, nkv, nkv], dim=1)
+
+        def into_h(name, x):
+            """h += x W^T (over all ranks), Gemma's through its post norm."""
+            post = {"wo": "g_post", "wdown": "g_postffn"}[name]
+            if self.gemma:
+                self._rowpar_ar(lw, name, x, t1, M, batch_attn)
+                ho.rmsnorm(t1[:M], lw[post], h[:M], res=h[:M], eps=eps)
+            elif self.tp_branch:
+                self._rowpar_ar(lw, name, x, t1, M, batch_attn)
+                ho.addinto(h[:M], t1[:M])
+            else:
+                self._linear(lw, name, x, h, res=h, M=M, batch=batch_attn)
+
         if layer_hook is not None:
             layer_hook(-1, h[:M])  # embedding output
         for i, lw in enumerate(self.layers):
             window = cfg.sliding_window if cfg.is_sliding(i) else 0
-            ho.rmsnorm(h[:M], lw["g_in"], xn[:M], eps=eps)
-            if batch_attn:
-                self._linear(lw, "wqkv", xn, self.bt_qkv, M=M)
+            if few:
+                self._rows(lw, "wqkv", h, qkv, M, g=lw["g_in"],
+                           bias=lw.get("bqkv"), batch=batch_attn)
+            else:
+                ho.rmsnorm(h[:M], lw["g_in"], xn[:M], eps=eps)
+                self._linear(lw, "wqkv", xn, qkv, M=M)
                 if "bqkv" in lw:
-                    ho.bias_add(self.bt_qkv, lw["bqkv"], M)
-                ho.attn_dec(self.bt_qkv, self.k_cache[i], self.v_cache[i],
+                    ho.bias_add(qkv, lw["bqkv"], M)
+            if batch_attn:
+                ho.attn_dec(qkv, self.k_cache[i], self.v_cache[i],
                             self.b_att[0], self.bt_lens, self.cos_t,
                             self.sin_t, self.bt_scratch, self.bt_attn_cnt,
                             self.nh_l, self.kvh_l, self.hd, self.scale,
@@ -566,20 +624,13 @@ class GPUModel(DecodeLoop):
                             split=self.attn_split, kS=self.k_scale[i],
                             vS=self.v_scale[i], batch=M)
             else:
-                self._linear(lw, "wq", xn, self.b_q, M=M)
-                self._linear(lw, "wk", xn, self.b_k, M=M)
-                self._linear(lw, "wv", xn, self.b_v, M=M)
-                if "bqkv" in lw:
-                    ho.bias_add(self.b_q, lw["bias_q"], M)
-                    ho.bias_add(self.b_k, lw["bias_k"], M)
-                    ho.bias_add(self.b_v, lw["bias_v"], M)
-                ho.rope_cache(self.b_q, self.b_k, self.b_v, self._kc(i),
+                ho.rope_cache(q, k, v, self._kc(i),
                               self._vc(i), self.cos_t, self.sin_t,
                               self.len_buf, M, self.nh_l, self.kvh_l,
                               self.hd, kS=self._ks(i), vS=self._vs(i))
                 if self.hd in (64, 128, 256):
                     ho.attn_prefill_mfma(
-                        self.b_q, self._kc(i), self._vc(i), self.b_att,
+                        q, self._kc(i), self._vc(i), self.b_att,
                         self.len_buf, M, self.nh_l, self.kvh_l, self.hd,
                         self.scale, softcap=self.attn_softcap,
                         window=window or 0,
@@ -589,40 +640,31 @@ class GPUModel(DecodeLoop):
                     # per-query VALU kernel: every production head_dim is
                     # 64/128/256 (MFMA above); kept as the documented
                     # debugging/odd-shape fallback
-                    ho.attn(self.b_q, self._kc(i), self._vc(i),
+                    ho.attn(q, self._kc(i), self._vc(i),
                             self.b_att, self.len_buf, M, self.nh_l,
                             self.kvh_l, self.hd, self.scale,
                             softcap=self.attn_softcap,
                             window=window or 0,
                             kS=self._ks(i), vS=self._vs(i))
-            if self.gemma:
-                self._rowpar_ar(lw, "wo", self.b_att, t1, M)
-                ho.rmsnorm(t1[:M], lw["g_post"], h[:M], res=h[:M], eps=eps)
-                ho.rmsnorm(h[:M], lw["g_preffn"], xn[:M], eps=eps)
-            else:
-                if self.tp_branch:
-                    self._rowpar_ar(lw, "wo", self.b_att, t1, M)
-                    ho.addinto(h[:M], t1[:M])
-                else:
-                    self._linear(lw, "wo", self.b_att, h, res=h, M=M)
-                ho.rmsnorm(h[:M], lw["g_post"], xn[:M], eps=eps)
+            into_h("wo", self.b_att)
+            g_mlp = lw["g_preffn"] if self.gemma else lw["g_post"]
             if self.moe:
+                ho.rmsnorm(h[:M], g_mlp, xn[:M], eps=eps)
                 self._moe_mlp_rows(lw, M)
-                if layer_hook is not None:
-                    layer_hook(i, h[:M])
-                continue
-            self._linear(lw, "wgate", xn, self.b_gate, M=M)
-            self._linear(lw, "wup", xn, self.b_up, M=M)
-            ho.glu(self.b_gate[:M], self.b_up[:M], self.b_gate[:M], self.act)
-            if self.gemma:
-                self._rowpar_ar(lw, "wdown", self.b_gate, t1, M)
-                ho.rmsnorm(t1[:M], lw["g_postffn"], h[:M], res=h[:M], eps=eps)
             else:
-                if self.tp_branch:
-                    self._rowpar_ar(lw, "wdown", self.b_gate, t1, M)
-                    ho.addinto(h[:M], t1[:M])
+                a = self.b_gate
+                if few:
+                    if 1 < M and self.fp8 and (batch_attn or not self.wq4):
+                        a = self.b_act32
+                    self._rows(lw, "wgu", h, a, M, g=g_mlp, act=self.act,
+                               batch=batch_attn)
                 else:
-                    self._linear(lw, "wdown", self.b_gate, h, res=h, M=M)
+                    ho.rmsnorm(h[:M], g_mlp, xn[:M], eps=eps)
+                    self._linear(lw, "wgate", xn, self.b_gate, M=M)
+                    self._linear(lw, "wup", xn, self.b_up, M=M)
+                    ho.glu(self.b_gate[:M], self.b_up[:M], self.b_gate[:M],
+                           self.act)
+                into_h("wdown", a)
             if layer_hook is not None:
                 layer_hook(i, h[:M])
 
@@ -669,6 +711,38 @@ class GPUModel(DecodeLoop):
                 ho.gemm(gate[:M], lw["wdown_all"][d_lo:d_hi], t1[:M],
                         accbuf=self.b_gemm_acc)
             ho.moe_scale_add(self.b_h, t1, self.moe_dense[e:], E, M, H)
+
+    @property
+    def _head(self):
+        """lm_head under the weight names that _rows expects."""
+        if self.fp8:
+            h = {"_q4": self.lm_head_q4, "_e4": self.lm_head_e4} \
+                if self.wq4 else {}
+            if self.keep_fp8:
+                h.update({"_q": self.lm_head_q, "_s": self.lm_head_s})
+            return h
+        return {"": self.lm_head}
+
+    def _head_rows(self, M: int, out: torch.Tensor):
+        """out[:M] = logits (bf16, this rank's vocabulary) of rows of h."""
+        if M <= ho.FEW_ROWS:
+            self._rows(self._head, "", self.b_h, out, M, g=self.g_final,
+                       softcap=self.final_softcap)
+            return
+        ho.rmsnorm(self.b_h[:M], self.g_final, self.b_xn[:M],
+                   eps=self.config.rms_norm_eps)
+        if self.wq4:
+            ho.gemm_fp4w(self.b_xn[:M], self.lm_head_q4, self.lm_head_e4,
+                         out[:M], accbuf=self.b_gemm_acc)
+        elif self.fp8:
+            ho.quant_fp8(self.b_xn[:M], self.b_xq, self.b_sx)
+            ho.gemm_fp8(self.b_xq, self.b_sx, self.lm_head_q, self.lm_head_s,
+                        out[:M], M, self.H, accbuf=self.b_gemm_acc)
+        else:
+            ho.gemm(self.b_xn[:M], self.lm_head, out[:M],
+                    accbuf=self.b_gemm_acc)
+        if self.final_softcap:
+            ho.softcap(out[:M], self.final_softcap)
 
     def _lm_head_last(self, M: int):
         """Final norm + lm_head on the last row -> self.b_logits (f32, V);
@@ -721,22 +795,7 @@ class GPUModel(DecodeLoop):
                 hidden[i + 1][d0:d0 + h.shape[0]] = \
                     h.float().cpu().numpy()
             self._layers_forward(M, layer_hook=hook, keys=done + M)
-            ho.rmsnorm(self.b_h[:M], self.g_final, self.b_xn[:M],
-                       eps=self.config.rms_norm_eps)
-            if self.wq4:
-                ho.gemm_fp4w(self.b_xn[:M], self.lm_head_q4,
-                             self.lm_head_e4, logits_buf[:M],
-                             accbuf=self.b_gemm_acc)
-            elif self.fp8:
-                ho.quant_fp8(self.b_xn[:M], self.b_xq, self.b_sx)
-                ho.gemm_fp8(self.b_xq, self.b_sx, self.lm_head_q,
-                            self.lm_head_s, logits_buf[:M], M, self.H,
-                            accbuf=self.b_gemm_acc)
-            else:
-                ho.gemm(self.b_xn[:M], self.lm_head, logits_buf[:M],
-                        accbuf=self.b_gemm_acc)
-            if self.final_softcap:
-                ho.softcap(logits_buf[:M], self.final_softcap)
+            self._head_rows(M, logits_buf)
             if self.world > 1:
                 # gather vocab shards on-device (each rank holds the
                 # columns [r*vocab_l, (r+1)*vocab_l) of rows [0, M))
@@ -784,22 +843,7 @@ class GPUModel(DecodeLoop):
             ho.embed(self.embed, self.ids_buf, self.b_h, M,
                      self.config.embed_scale)
             self._layers_forward(M, keys=pos0 + done + M)
-            ho.rmsnorm(self.b_h[:M], self.g_final, self.b_xn[:M],
-                       eps=self.config.rms_norm_eps)
-            if self.wq4:
-                ho.gemm_fp4w(self.b_xn[:M], self.lm_head_q4,
-                             self.lm_head_e4, logits_buf[:M],
-                             accbuf=self.b_gemm_acc)
-            elif self.fp8:
-                ho.quant_fp8(self.b_xn[:M], self.b_xq, self.b_sx)
-                ho.gemm_fp8(self.b_xq, self.b_sx, self.lm_head_q,
-                            self.lm_head_s, logits_buf[:M], M, self.H,
-                            accbuf=self.b_gemm_acc)
-            else:
-                ho.gemm(self.b_xn[:M], self.lm_head, logits_buf[:M],
-                        accbuf=self.b_gemm_acc)
-            if self.final_softcap:
-                ho.softcap(logits_buf[:M], self.final_softcap)
+            self._head_rows(M, logits_buf)
             if self.world > 1:
                 # gather vocab shards on-device (each rank holds the
                 # columns [r*vocab_l, (r+1)*vocab_l) of rows [0, M))
@@ -1041,39 +1085,36 @@ class GPUModel(DecodeLoop):
     # ------------------------------------------------------------------
     def _decode_batch_step(self, B: int, greedy: bool, min_p: float,
                            temperature: float = 1.0):
-        """One decode step for B lockstep sequences.  fp8 weights with
-        B<=8 take the fused MULTI-X GEMV path (one weight stream feeds
-        B accumulators — near single-sequence step time); otherwise the
-        layer stack runs as M=B-row MFMA GEMMs.  Graph-replayable
-        (all state device-side)."""
+        """One decode step for B lockstep sequences: the layer stack over
+        B rows, up to FEW_ROWS of them with W streamed once a projection.
+        Graph-replayable (all state device-side).  The multi-x GEMV path
+        (fp8, B<=8, VALU-bound) is there for comparison, by
+        LLM_BATCH_MX_MAX."""
         cfg = self.config
-        # measured (profiles/decode_kernels_r02.md): the SKINNY fp8 MFMA
-        # GEMM wins at every B (even B=2: 1.34 vs the multi-x GEMV's
-        # 1.44 ms — the GEMV is VALU-ISSUE-bound, 128 irreducible
-        # FMAs per 16 weight bytes at B=8).  The multi-x path stays
-        # available via LLM_BATCH_MX_MAX for comparison.
         import os as _os  # noqa: delayed so env changes apply per call
         mx_max = int(_os.environ.get("LLM_BATCH_MX_MAX", "0"))
         if (self.fp8 and B <= mx_max and not cfg.attention_bias
                 and not self.moe):
             return self._decode_batch_step_mx(B, greedy, min_p, temperature)
-        if self.fp8 and B <= 16 and not self.moe:
-            return self._decode_batch_step_skinny(B, greedy, min_p,
-                                                  temperature)
         ho.embed(self.embed, self.bt_next, self.b_h, B, cfg.embed_scale)
         self._layers_forward(B, batch_attn=True)
-        ho.rmsnorm(self.b_h[:B], self.g_final, self.b_xn[:B],
-                   eps=cfg.rms_norm_eps)
-        if self.fp8:
-            ho.quant_fp8(self.b_xn[:B], self.b_xq, self.b_sx)
-            ho.gemm_fp8(self.b_xq, self.b_sx, self.lm_head_q,
-                        self.lm_head_s, self.bt_logits[:B], B, self.H,
-                        accbuf=self.b_gemm_acc)
+        if B <= ho.FEW_ROWS:
+            self._rows(self._head, "", self.b_h, self.bt_logits, B,
+                       g=self.g_final, softcap=self.final_softcap,
+                       batch=True)
         else:
-            ho.gemm(self.b_xn[:B], self.lm_head, self.bt_logits[:B],
-                    accbuf=self.b_gemm_acc)
-        if self.final_softcap:
-            ho.softcap(self.bt_logits[:B], self.final_softcap)
+            ho.rmsnorm(self.b_h[:B], self.g_final, self.b_xn[:B],
+                       eps=cfg.rms_norm_eps)
+            if self.fp8:
+                ho.quant_fp8(self.b_xn[:B], self.b_xq, self.b_sx)
+                ho.gemm_fp8(self.b_xq, self.b_sx, self.lm_head_q,
+                            self.lm_head_s, self.bt_logits[:B], B, self.H,
+                            accbuf=self.b_gemm_acc)
+            else:
+                ho.gemm(self.b_xn[:B], self.lm_head, self.bt_logits[:B],
+                        accbuf=self.b_gemm_acc)
+            if self.final_softcap:
+                ho.softcap(self.bt_logits[:B], self.final_softcap)
         ho.sample(self.bt_logits[:B], min_p, greedy, self.seed,
                   self.rng_ctr, self.bt_gmax, self.bt_pick, self.bt_next,
                   self.bt_ring, self.bt_nout, self.bt_lens, bump_len=True,
@@ -1153,95 +1194,6 @@ class GPUModel(DecodeLoop):
                            self.bt_logits, B, H, self.vocab_l,
                            stage=ho.STAGE_NORM, g=self.g_final, eps=eps,
                            softcap=self.final_softcap)
-        ho.sample(self.bt_logits[:B], min_p, greedy, self.seed,
-                  self.rng_ctr, self.bt_gmax, self.bt_pick, self.bt_next,
-                  self.bt_ring, self.bt_nout, self.bt_lens, bump_len=True,
-                  temperature=temperature, cnt=self.bt_cnt, batch=B)
-
-    def _decode_batch_step_skinny(self, B: int, greedy: bool,
-                                  min_p: float, temperature: float = 1.0):
-        """Batched decode via (stage+quant, skinny fp8 MFMA GEMM) pairs:
-        B = 3..16 lockstep rows, W streamed once per projection."""
-        cfg = self.config
-        eps = cfg.rms_norm_eps
-        H, I = self.H, self.inter_l
-        h = self.b_h
-        hb = self.bt_hb
-        t1, t2, gu = self.bt_t1, self.bt_t2, self.bt_gu
-        qkvw = (self.nh_l + 2 * self.kvh_l) * self.hd
-        nhh = self.nh_l * self.hd
-        xq, sx = self.b_xq, self.b_sx
-        prev = None
-        for i, lw in enumerate(self.layers):
-            window = cfg.sliding_window if cfg.is_sliding(i) else 0
-            if self.gemma and prev is not None:
-                ho.stage_quant_mx(t2, H, xq, sx, B, H, stage=ho.STAGE_NORM2,
-                                  x2=h, x2stride=H, g=prev["g_postffn"],
-                                  g2=lw["g_in"], hout=hb, hstride=H,
-                                  eps=eps)
-                h, hb = hb, h
-            elif i == 0:
-                ho.stage_quant_mx(self.embed, 0, xq, sx, B, H,
-                                  stage=ho.STAGE_NORM_EMBED,
-                                  x2=self.bt_next, g=lw["g_in"], hout=h,
-                                  hstride=H, eps=eps,
-                                  escale=cfg.embed_scale)
-            else:
-                ho.stage_quant_mx(h, H, xq, sx, B, H, stage=ho.STAGE_NORM,
-                                  g=lw["g_in"], eps=eps)
-            ho.gemm_fp8_skinny(xq, sx, lw["wqkv_q"], lw["wqkv_s"],
-                               self.bt_qkv, B, qkvw, bias=lw.get("bqkv"),
-                               accbuf=self.b_gemm_acc)
-            prev = lw
-            ho.attn_dec(self.bt_qkv, self.k_cache[i], self.v_cache[i],
-                        self.b_att[0], self.bt_lens, self.cos_t, self.sin_t,
-                        self.bt_scratch, self.bt_attn_cnt,
-                        self.nh_l, self.kvh_l, self.hd, self.scale,
-                        softcap=self.attn_softcap, window=window or 0,
-                        split=self.attn_split, kS=self.k_scale[i],
-                        vS=self.v_scale[i], batch=B)
-            ho.stage_quant_mx(self.b_att, nhh, xq, sx, B, nhh)
-            if self.gemma:
-                ho.gemm_fp8_skinny(xq, sx, lw["wo_q"], lw["wo_s"], t1, B, H,
-                                   accbuf=self.b_gemm_acc)
-                ho.stage_quant_mx(t1, H, xq, sx, B, H,
-                                  stage=ho.STAGE_NORM2, x2=h, x2stride=H,
-                                  g=lw["g_post"], g2=lw["g_preffn"],
-                                  hout=hb, hstride=H, eps=eps)
-                h, hb = hb, h
-                ho.gemm_fp8_skinny(xq, sx, lw["wgu_q"], lw["wgu_s"], gu, B,
-                                   2 * I, accbuf=self.b_gemm_acc)
-                ho.stage_quant_mx(gu, 2 * I, xq, sx, B, I,
-                                  stage=ho.STAGE_GLU, x2=gu[:, I:],
-                                  x2stride=2 * I, act=self.act)
-                ho.gemm_fp8_skinny(xq, sx, lw["wdown_q"], lw["wdown_s"],
-                                   t2, B, H, accbuf=self.b_gemm_acc)
-            else:
-                ho.gemm_fp8_skinny(xq, sx, lw["wo_q"], lw["wo_s"], h, B, H,
-                                   res=h, rstride=H,
-                                   accbuf=self.b_gemm_acc)
-                ho.stage_quant_mx(h, H, xq, sx, B, H, stage=ho.STAGE_NORM,
-                                  g=lw["g_post"], eps=eps)
-                ho.gemm_fp8_skinny(xq, sx, lw["wgu_q"], lw["wgu_s"], gu, B,
-                                   2 * I, accbuf=self.b_gemm_acc)
-                ho.stage_quant_mx(gu, 2 * I, xq, sx, B, I,
-                                  stage=ho.STAGE_GLU, x2=gu[:, I:],
-                                  x2stride=2 * I, act=self.act)
-                ho.gemm_fp8_skinny(xq, sx, lw["wdown_q"], lw["wdown_s"], h,
-                                   B, H, res=h, rstride=H,
-                                   accbuf=self.b_gemm_acc)
-        if self.gemma:
-            ho.stage_quant_mx(t2, H, xq, sx, B, H, stage=ho.STAGE_NORM2,
-                              x2=h, x2stride=H,
-                              g=self.layers[-1]["g_postffn"],
-                              g2=self.g_final, hout=hb, hstride=H, eps=eps)
-        else:
-            ho.stage_quant_mx(h, H, xq, sx, B, H, stage=ho.STAGE_NORM,
-                              g=self.g_final, eps=eps)
-        ho.gemm_fp8_skinny(xq, sx, self.lm_head_q, self.lm_head_s,
-                           self.bt_logits, B, self.vocab_l,
-                           softcap=self.final_softcap,
-                           accbuf=self.b_gemm_acc)
         ho.sample(self.bt_logits[:B], min_p, greedy, self.seed,
                   self.rng_ctr, self.bt_gmax, self.bt_pick, self.bt_next,
                   self.bt_ring, self.bt_nout, self.bt_lens, bump_len=True,

@@ -37,9 +37,9 @@ _SIGS = {
     "launch_rmsnorm": [ctypes.c_void_p] * 4 + [ctypes.c_int] * 2 +
                       [ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
     "launch_rope_cache": [ctypes.c_void_p] * 7 + [ctypes.c_int] +
-                         [ctypes.c_void_p] * 3 + [ctypes.c_int] * 5 +
+                         [ctypes.c_void_p] * 3 + [ctypes.c_int] * 7 +
                          [ctypes.c_void_p],
-    "launch_attn": [ctypes.c_void_p] * 7 + [ctypes.c_int] * 6 +
+    "launch_attn": [ctypes.c_void_p] * 7 + [ctypes.c_int] * 7 +
                    [ctypes.c_float, ctypes.c_float, ctypes.c_int,
                     ctypes.c_void_p],
     "launch_attn_prefill_mfma": [ctypes.c_void_p] * 8 + [ctypes.c_long] +
@@ -61,6 +61,9 @@ _SIGS = {
                      [ctypes.c_int, ctypes.c_void_p],
     "launch_gemm_bf16": [ctypes.c_void_p] * 5 + [ctypes.c_int] * 3 +
                         [ctypes.c_void_p],
+    "launch_row_gemm": [ctypes.c_void_p] * 11 + [ctypes.c_long] +
+                       [ctypes.c_int] * 10 +
+                       [ctypes.c_float, ctypes.c_float, ctypes.c_void_p],
     "launch_prefetch": [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p,
                         ctypes.c_void_p],
     "launch_softcap": [ctypes.c_void_p, ctypes.c_long, ctypes.c_float,
@@ -70,7 +73,7 @@ _SIGS = {
     "launch_bias_add": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                         ctypes.c_int, ctypes.c_void_p],
     "launch_i32_set": [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
-    "launch_quant_fp8": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 2 +
+    "launch_quant_fp8": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 +
                         [ctypes.c_void_p],
     "launch_quant_fp4": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 2 +
                         [ctypes.c_void_p],
@@ -78,19 +81,6 @@ _SIGS = {
                        [ctypes.c_float, ctypes.c_int, ctypes.c_float,
                         ctypes.c_int, ctypes.c_int, ctypes.c_int,
                         ctypes.c_float, ctypes.c_void_p],
-    "launch_stage_quant_mx": [ctypes.c_void_p, ctypes.c_long,
-                              ctypes.c_void_p, ctypes.c_long] +
-                             [ctypes.c_void_p] * 4 +
-                             [ctypes.c_void_p, ctypes.c_long] +
-                             [ctypes.c_int] * 4 +
-                             [ctypes.c_float, ctypes.c_float,
-                              ctypes.c_void_p],
-    "launch_gemm_fp8_skinny": [ctypes.c_void_p] * 5 + [ctypes.c_long] +
-                              [ctypes.c_void_p, ctypes.c_long] +
-                              [ctypes.c_void_p, ctypes.c_void_p,
-                               ctypes.c_int,
-                               ctypes.c_float] + [ctypes.c_int] * 3 +
-                              [ctypes.c_void_p],
     "launch_gemv_fp8_mx": [ctypes.c_void_p] * 3 + [ctypes.c_long] +
                           [ctypes.c_void_p, ctypes.c_long] +
                           [ctypes.c_void_p] * 3 + [ctypes.c_long] +
@@ -150,6 +140,11 @@ def _check(err: int, name: str):
 
 def _ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
+
+
+def _ld(t, width: int) -> int:
+    """Elements from row to row (rows of one buffer may lie in another's)."""
+    return t.stride(0) if t.dim() > 1 else width
 
 
 # ----------------------------------------------------------------------
@@ -226,13 +221,16 @@ def rope_cache(q: torch.Tensor, k_in: torch.Tensor, v_in: torch.Tensor,
                pos_ptr: torch.Tensor, M: int, nh: int, kvh: int, hd: int,
                kS: torch.Tensor | None = None,
                vS: torch.Tensor | None = None):
-    """kS/vS given => fp8 (e4m3) KV pool with per-(head,pos) scales."""
+    """kS/vS given => fp8 (e4m3) KV pool with per-(head,pos) scales.
+    q, k_in, v_in: M rows, which may lie in one fused buffer (k_in and v_in
+    equally far apart)."""
     S = k_cache.shape[1]
+    assert _ld(v_in, kvh * hd) == _ld(k_in, kvh * hd)
     _check(lib().launch_rope_cache(
         _ptr(q), _ptr(k_in), _ptr(v_in), _ptr(k_cache), _ptr(v_cache),
         _ptr(kS), _ptr(vS), 1 if kS is not None else 0,
         _ptr(cos_t), _ptr(sin_t), _ptr(pos_ptr), M, nh, kvh, hd, S,
-        _stream()), "rope_cache")
+        _ld(q, nh * hd), _ld(k_in, kvh * hd), _stream()), "rope_cache")
 
 
 def attn(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -244,8 +242,8 @@ def attn(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     _check(lib().launch_attn(
         _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(len_ptr),
         _ptr(kS), _ptr(vS), 1 if kS is not None else 0,
-        M, nh, kvh, hd, S, ctypes.c_float(scale), ctypes.c_float(softcap),
-        window, _stream()), "attn")
+        M, nh, kvh, hd, _ld(q, nh * hd), S, ctypes.c_float(scale),
+        ctypes.c_float(softcap), window, _stream()), "attn")
 
 
 def attn_prefill_mfma(q: torch.Tensor, k_cache: torch.Tensor,
@@ -265,7 +263,8 @@ def attn_prefill_mfma(q: torch.Tensor, k_cache: torch.Tensor,
         _ptr(kS), _ptr(vS), _ptr(part),
         ctypes.c_long(0 if part is None else part.numel()),
         1 if kS is not None else 0,
-        M, nh, kvh, hd, nh * hd, S, max(keys, M), ctypes.c_float(scale),
+        M, nh, kvh, hd, _ld(q, nh * hd), S, max(keys, M),
+        ctypes.c_float(scale),
         ctypes.c_float(softcap), window, _stream()), "attn_prefill_mfma")
 
 
@@ -362,14 +361,52 @@ def gemm(X: torch.Tensor, W: torch.Tensor, Y: torch.Tensor,
                                   _ptr(accbuf), M, N, K, _stream()), "gemm")
 
 
+FEW_ROWS = 16        # rows that row_gemm takes
+ROW_NORM_K = 4096    # the longest row that it norms
+
+
+def row_gemm(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, M: int,
+             ws: torch.Tensor | None = None,
+             we: torch.Tensor | None = None,
+             g: torch.Tensor | None = None, eps: float = 1e-5,
+             bias: torch.Tensor | None = None,
+             res: torch.Tensor | None = None, act: int = -1,
+             softcap: float = 0.0, part: torch.Tensor | None = None,
+             cnt: torch.Tensor | None = None,
+             sx: torch.Tensor | None = None):
+    """Y[M<=16, N] = X W^T for few rows of x (2-D, rows may be apart), W
+    streamed once: bf16, e4m3 (ws: row scales) or MXFP4 (we: exponents).
+    x is bf16; beside e4m3 weights its rows are rounded to e4m3: by the
+    caller (x bytes, sx scales), or after the norm that is taken here.
+    g: RMSNorm of x on the way (K <= ROW_NORM_K).  act 0/1: w holds gate
+    rows, then up rows, and Y = act(gate) * up.  Then softcap, bias, res.
+    part (fp32) and cnt (int32, zero; left zero) let K be split."""
+    wt = 1 if ws is not None else 2 if we is not None else 0
+    K = x.shape[-1]
+    N = w.shape[0] // (2 if act >= 0 else 1)
+    assert w.shape[1] * (2 if wt == 2 else 1) == K and w.is_contiguous()
+    assert x.stride(-1) == 1 and y.stride(-1) == 1
+    assert x.dtype == (torch.uint8 if wt == 1 and g is None
+                       else torch.bfloat16)
+    _check(lib().launch_row_gemm(
+        _ptr(x), _ptr(sx), _ptr(w), _ptr(ws), _ptr(we), _ptr(g), _ptr(bias),
+        _ptr(res), _ptr(y), _ptr(part), _ptr(cnt),
+        ctypes.c_long(0 if part is None else part.numel()),
+        0 if cnt is None else cnt.numel(), wt, M, N, K, x.stride(0),
+        res.stride(0) if res is not None else 0, y.stride(0), act,
+        1 if y.dtype == torch.float32 else 0, ctypes.c_float(eps), ctypes.c_float(softcap), _stream()),
+        "row_gemm")
+
+
 def quant_fp8(x: torch.Tensor, q: torch.Tensor, s: torch.Tensor):
     """Per-row e4m3fn quantization on device: q = fp8(x / s_row),
-    s_row = absmax/448.  x: (M,K) bf16 contiguous; q: >= M*K uint8;
+    s_row = absmax/448.  x: (M,K) bf16 or fp32, contiguous; q: >= M*K uint8;
     s: >= M fp32.  Used for weights at load and activations per GEMM."""
     M = 1 if x.dim() == 1 else x.shape[0]
     K = x.shape[-1]
     assert q.numel() >= M * K and s.numel() >= M
-    _check(lib().launch_quant_fp8(_ptr(x), _ptr(q), _ptr(s), M, K,
+    _check(lib().launch_quant_fp8(_ptr(x), _ptr(q), _ptr(s),
+                                  1 if x.dtype == torch.float32 else 0, M, K,
                                   _stream()), "quant_fp8")
 
 
@@ -439,42 +476,6 @@ def gemv_fp8_mx(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
         _ptr(hout), ctypes.c_long(hstride), N, K, B, stage, act,
         ctypes.c_float(eps), out_f32, ctypes.c_float(softcap),
         ctypes.c_float(escale), _stream()), "gemv_fp8_mx")
-
-
-def stage_quant_mx(x: torch.Tensor, xstride: int, xq: torch.Tensor,
-                   sx: torch.Tensor, B: int, K: int, stage: int = 0,
-                   x2: torch.Tensor | None = None, x2stride: int = 0,
-                   g: torch.Tensor | None = None,
-                   g2: torch.Tensor | None = None,
-                   hout: torch.Tensor | None = None, hstride: int = 0,
-                   act: int = 0, eps: float = 1e-5, escale: float = 1.0):
-    """Per-sequence-row staging op + e4m3 quantization -> xq[B,K], sx[B]
-    (feeds the skinny fp8 MFMA GEMM).  Strides in elements."""
-    _check(lib().launch_stage_quant_mx(
-        _ptr(x), ctypes.c_long(xstride), _ptr(x2), ctypes.c_long(x2stride),
-        _ptr(g), _ptr(g2), _ptr(xq), _ptr(sx), _ptr(hout),
-        ctypes.c_long(hstride), K, B, stage, act, ctypes.c_float(eps),
-        ctypes.c_float(escale), _stream()), "stage_quant_mx")
-
-
-def gemm_fp8_skinny(xq: torch.Tensor, sx: torch.Tensor, Wq: torch.Tensor,
-                    sw: torch.Tensor, y: torch.Tensor, B: int,
-                    ystride: int, res: torch.Tensor | None = None,
-                    rstride: int = 0, bias: torch.Tensor | None = None,
-                    softcap: float = 0.0,
-                    accbuf: torch.Tensor | None = None):
-    """Y[B<=16, N] = (sx_b*sw_n) * Xq @ Wq^T: one 16-row fp8 MFMA tile
-    per wave, W nt-streamed once (batched decode B=3..16).  accbuf
-    (fp32, >= B*N) enables the K-split path for small-N occupancy."""
-    N, K = Wq.shape
-    out_f32 = 1 if y.dtype == torch.float32 else 0
-    if accbuf is not None and accbuf.numel() < B * N:
-        accbuf = None
-    _check(lib().launch_gemm_fp8_skinny(
-        _ptr(xq), _ptr(sx), _ptr(Wq), _ptr(sw), _ptr(y),
-        ctypes.c_long(ystride), _ptr(res), ctypes.c_long(rstride),
-        _ptr(bias), _ptr(accbuf), out_f32, ctypes.c_float(softcap),
-        B, N, K, _stream()), "gemm_fp8_skinny")
 
 
 def gemm_fp4w(X: torch.Tensor, Wq4: torch.Tensor, We4: torch.Tensor,

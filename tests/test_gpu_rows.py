@@ -63,3 +63,64 @@ def test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8):
     # bf16 probabilities and results: 2^-9 at most each
     assert off(out[:M], ref.view(M, -1)) < 2.0 ** -8
     assert (out[M] == 7.0).all()
+
+
+def mxfp4_values(q, e):
+    """MXFP4 bytes and exponents as 64-bit values."""
+    grid = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0],
+                        dtype=torch.float64, device=q.device)
+    c = torch.stack([q & 15, q >> 4], -1).reshape(q.shape[0], -1).long()
+    v = grid[c & 7] * torch.where(c > 7, -1.0, 1.0)
+    return v * torch.exp2(e.double() - 127).repeat_interleave(32, 1)
+
+
+# outputs: less than half a tile, a tile and a rest, more tiles than blocks;
+# K: one slab of 64, slabs that eight waves share unevenly, split over blocks
+@pytest.mark.parametrize("N,K", [(5, 64), (24, 192), (200, 320), (520, 8192),
+                                 (4616, 1088)])
+@pytest.mark.parametrize("M", [1, 7, 16])
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "fp4"])
+@pytest.mark.parametrize("norm,act", [(False, -1), (True, -1), (False, 1),
+                                      (True, 0)])
+def test_few_rows(N, K, M, kind, norm, act):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    if norm and K > ho.ROW_NORM_K:
+        pytest.skip("normed by a kernel of its own")
+    W = normal(N * (2 if act >= 0 else 1), K, seed=4, scale=K ** -0.5)
+    X = normal(M, K + 16, seed=5)[:, :K]            # rows apart
+    g = torch.rand(K, device="cuda") + 0.5 if norm else None
+    bias, res = (normal(M, N, seed=6) for _ in range(2))
+    kw, Wd, x = {}, W.double(), X.double()
+    if norm:
+        x = x / torch.sqrt((x * x).mean(1, keepdim=True) + 1e-5) * g.double()
+    if kind == "fp8":
+        W, kw["ws"], Wd = e4m3(W)
+        q, s, x = e4m3(x)
+        if not norm:
+            X, kw["sx"] = q, s
+    elif kind == "fp4":
+        q = torch.empty(W.shape[0], K // 2, dtype=torch.uint8, device="cuda")
+        e = torch.empty(W.shape[0], K // 32, dtype=torch.uint8, device="cuda")
+        ho.quant_fp4(W, q, e)
+        W, kw["we"], Wd = q, e, mxfp4_values(q, e)
+    part = torch.zeros(1 << 22, device="cuda")
+    cnt = torch.zeros(256, dtype=torch.int32, device="cuda")
+    Y = torch.full((M + 1, N), 7.0, device="cuda").bfloat16()
+    for _ in range(2):                              # counters are left zero
+        ho.row_gemm(X, W, Y, M, g=g, bias=bias[0].contiguous(), res=res,
+                    act=act, softcap=30.0, part=part, cnt=cnt, **kw)
+    z = x @ Wd.T
+    if kind == "fp8" and act >= 0:
+        z = z.bfloat16().double()
+    if act >= 0:
+        f = (torch.nn.functional.silu if act == 0 else lambda t:
+             torch.nn.functional.gelu(t, approximate="tanh"))
+        z = f(z[:, :N]) * z[:, N:]
+    z = 30.0 * torch.tanh(z / 30.0) + bias[0].double() + res.double()
+    # bf16 normed rows and results: 2^-9 at most each, twice through a gate;
+    # a normed value that lies on the edge of two e4m3 ones may take the
+    # other: 2^-4 of it, and one in some hundred does
+    assert off(Y[:M], z) < (2.0 ** -6 if norm and kind == "fp8"
+                            else 2.0 ** -7)
+    assert (Y[M] == 7.0).all() and not cnt.any()
