@@ -31,7 +31,7 @@ CSRC = os.path.join(ROOT, "csrc")
 PKG = os.path.join(ROOT, "llm_np_cp_amd")
 LIBS = {
     "llmops": ["llm_ops.hip", "attn_prefill.hip", "row_gemm.hip",
-               "xgmi_comm.hip"],
+               "gemm_prompt.hip", "xgmi_comm.hip"],
     "linear": ["linear.hip"],
     "latent": ["latent_attn.hip"],
     "gqa": ["gqa_attn.hip"],

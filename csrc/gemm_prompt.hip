@@ -1,0 +1,445 @@
+// gemm_prompt.hip — linears of many rows: Y[M,N] = X[M,K] W[N,K]^T, bf16 or
+// e4m3 with row scales, fp32 sums, bf16 out.
+//
+// Slabs of 128 bytes a row (64 bf16, 128 e4m3) go straight into LDS, two or
+// three buffers, one barrier a slab that waits for the next slab only and
+// leaves the DMA behind it in flight.  That wait is what bounds these
+// products (a slab is back from L2 or memory after one to two microseconds,
+// the matrix cores want one a microsecond): with every DMA drained at each
+// barrier 2048x4096x14336 ran at 1030 TFLOP/s in bf16 and 870 in e4m3, with
+// 128x256 tiles and three buffers it runs at 1160 and 2180.
+//
+// Rows are XOR-swizzled by 16-byte slots; the DMA writes lane-linear, so the
+// swizzle sits in the address that a lane reads and in the fragment reads.  The order of k inside a slab is free as
+// long as X and W agree: a lane's two slots are two bf16 operands or one
+// e4m3 operand of the 128-deep MFMA.  W is the first operand, so a lane
+// ends with four neighbouring outputs of one row and stores them at once.
+//
+// Blocks of one XCD take neighbouring tiles, rows fastest, so that its L2
+// holds the few panels of W they share.  Gate and up rows of W alternate by
+// 16 in a tile (GLU): a lane has both halves of its outputs and stores
+// act(gate) * up, half the bytes and one launch instead of three.
+//
+// With few tiles K is split over blocks; the last block of a tile to arrive
+// adds the parts in their order (the result does not depend on timing).
+#include "common.h"
+
+typedef short gp_s8 __attribute__((ext_vector_type(8)));
+typedef int gp_i8 __attribute__((ext_vector_type(8)));
+typedef __bf16 gp_b2 __attribute__((ext_vector_type(2)));
+
+struct GpArgs {
+  const void* x;       // [M, K]
+  const void* w;       // [N, K], GLU: [2N, K] gate then up
+  const float* sx;     // e4m3: row scales
+  const float* sw;
+  const u16* res;      // [M, N]
+  const u16* bias;     // [N]
+  u16* y;              // [M, N]
+  float* part;         // split K: [tile, split, BM*BN]
+  int* cnt;            // split K: blocks of a tile that are done
+  int M, N, K, act, tm, tn;
+};
+
+DEVINL float gp_act(float x, int act) {
+  if (act == 0) return x / (1.f + __expf(-x));
+  const float c = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+  // tanh by exp: exact limits at +-inf
+  return x * (1.f - 1.f / (__expf(2.f * c) + 1.f));
+}
+
+// Barrier after the wave's LDS reads and all but its last N DMA loads.  The
+// builtin tells the compiler which of them are over; it would wait for all
+// of them before the next read otherwise.
+template <int N> DEVINL void gp_meet() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | 7 << 4);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <bool F8, int BM, int BN, int WM, int WN, int NS, bool GLU>
+__global__ void __launch_bounds__(64 * WM * WN)
+k_gemm_prompt(GpArgs a) {
+  constexpr int NW = WM * WN;
+  constexpr int FM = BM / WM / 16, FN = BN / WN / 16;   // fragments of a wave
+  constexpr int AI = BM / 8 / NW, BI = BN / 8 / NW;     // DMA of a wave
+  static_assert(AI > 0 && BI > 0 && FM > 0 && FN % (GLU ? 2 : 1) == 0);
+  constexpr int PS = AI + BI;
+  // An array a buffer, and the loop unrolled over them: the compiler sees
+  // that a DMA into one does not touch what is read from another, and puts
+  // no wait for it before the reads.
+  constexpr int ZA = BM * 128, ZB = BN * 128;
+  __shared__ __attribute__((aligned(16))) char A0[ZA], A1[ZA];
+  __shared__ __attribute__((aligned(16))) char B0[ZB], B1[ZB];
+  __shared__ __attribute__((aligned(16))) char A2[NS > 2 ? ZA : 16],
+      B2[NS > 2 ? ZB : 16];
+  __shared__ int last_flag;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  // tiles of an XCD (block id modulo 8) are neighbours
+  const int tiles = a.tm * a.tn, chunk = (tiles + 7) / 8;
+  const int tile = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= chunk || tile >= tiles) return;
+  const int bm = tile % a.tm * BM, bn = tile / a.tm * (GLU ? BN / 2 : BN);
+
+  const size_t rowb = (size_t)a.K * (F8 ? 1 : 2);       // bytes of a row
+  const int slabs = (int)((rowb + 127) / 128);
+  const int SK = gridDim.y, per = (slabs + SK - 1) / SK;
+  const int s_lo = blockIdx.y * per, s_hi = min(s_lo + per, slabs);
+  // e4m3 rows of 64 * odd: the last slab is half a slab
+  const bool half = F8 && (rowb & 127) && s_hi == slabs;
+
+  const int g_r = lane >> 3, g_s = lane & 7;
+  const char* pa[AI];
+  const char* pb[BI];
+#pragma unroll
+  for (int i = 0; i < AI; i++) {
+    const int r = (wave * AI + i) * 8 + g_r;
+    pa[i] = (const char*)a.x + (size_t)min(bm + r, a.M - 1) * rowb;
+  }
+#pragma unroll
+  for (int i = 0; i < BI; i++) {
+    const int r = (wave * BI + i) * 8 + g_r;
+    size_t row;
+    if (GLU) {
+      const int n = min(bn + (r >> 5) * 16 + (r & 15), a.N - 1);
+      row = ((r >> 4) & 1) ? (size_t)a.N + n : (size_t)n;
+    } else {
+      row = min(bn + r, a.N - 1);
+    }
+    pb[i] = (const char*)a.w + row * rowb;
+  }
+  // row r of a tile keeps slot q at q ^ ((r >> 1) & 7)
+  const int src0 = (g_s ^ (g_r >> 1)) * 16, src1 = src0 ^ 64;
+  auto stage = [&](char* A, char* B, int s) {
+    int o0 = src0, o1 = src1;
+    if (F8 && half && s == slabs - 1) o0 &= 63, o1 &= 63;   // stay in the row
+    const size_t k0 = (size_t)s * 128 + o0, k1 = (size_t)s * 128 + o1;
+#pragma unroll
+    for (int i = 0; i < AI; i++)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) uint32_t*)(
+              pa[i] + (((wave * AI + i) & 1) ? k1 : k0)),
+          (__attribute__((address_space(3))) uint32_t*)(
+              A + (wave * AI + i) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < BI; i++)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) uint32_t*)(
+              pb[i] + (((wave * BI + i) & 1) ? k1 : k0)),
+          (__attribute__((address_space(3))) uint32_t*)(
+              B + (wave * BI + i) * 1024), 16, 0, 0);
+  };
+
+  f4v acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; i++)
+#pragma unroll
+    for (int j = 0; j < FN; j++) acc[i][j] = {0.f, 0.f, 0.f, 0.f};
+
+  const int fr = lane & 15, fk = lane >> 4;
+  const int x0 = (fk ^ (fr >> 1)) * 16, x1 = x0 ^ 64;
+  const int la = (wm * FM * 16 + fr) * 128, lb = (wn * FN * 16 + fr) * 128;
+
+  // A slab ends with a meeting that hands over the next one: its DMA is
+  // over, that of the NS - 2 behind it stays in flight.  The loop is free of
+  // conditions while there are slabs to ask for; the last few wait for all.
+  int s = s_lo;
+  if (s_lo < s_hi) {
+    stage(A0, B0, s_lo);
+    if (s_lo + 1 < s_hi) stage(A1, B1, s_lo + 1);
+    if (NS > 2 && s_lo + 2 < s_hi) stage(A2, B2, s_lo + 2);
+    // all but the first may still be in flight
+    if (s_lo + NS <= s_hi) gp_meet<PS * (NS - 1)>();
+    else gp_meet<0>();
+    if constexpr (F8) {
+      auto slab = [&](char* A, char* B, int s, bool steady) {
+        const char *ca = A + la, *cb = B + lb;
+        if (steady || !(half && s == slabs - 1)) {
+          union { u4v_ q[2]; gp_i8 v; } wb[FN];
+#pragma unroll
+          for (int j = 0; j < FN; j++) {
+            wb[j].q[0] = *(const u4v_*)(cb + j * 2048 + x0);
+            wb[j].q[1] = *(const u4v_*)(cb + j * 2048 + x1);
+          }
+          // block scales of one (e8m0 127): the row scales come at the end
+#pragma unroll
+          for (int i = 0; i < FM; i++) {
+            union { u4v_ q[2]; gp_i8 v; } xa;
+            xa.q[0] = *(const u4v_*)(ca + i * 2048 + x0);
+            xa.q[1] = *(const u4v_*)(ca + i * 2048 + x1);
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+              acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                  wb[j].v, xa.v, acc[i][j], 0, 0, 0, 0x7f7f7f7f, 0,
+                  0x7f7f7f7f);
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < FM; i++) {
+            union { u4v_ q; long l[2]; } xa, wb;
+            xa.q = *(const u4v_*)(ca + i * 2048 + x0);
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+              wb.q = *(const u4v_*)(cb + j * 2048 + x0);
+#pragma unroll
+              for (int h = 0; h < 2; h++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                    wb.l[h], xa.l[h], acc[i][j], 0, 0, 0);
+            }
+          }
+        }
+        if (steady) {
+          gp_meet<PS * (NS - 2)>();
+          stage(A, B, s + NS);
+        } else if (s + 1 < s_hi) {
+          gp_meet<0>();
+          if (s + NS < s_hi) stage(A, B, s + NS);
+        }
+      };
+      for (; s + 2 * NS <= s_hi; s += NS) {
+        slab(A0, B0, s, true);
+        slab(A1, B1, s + 1, true);
+        if (NS > 2) slab(A2, B2, s + 2, true);
+      }
+      for (; s < s_hi; s += NS) {
+        slab(A0, B0, s, false);
+        if (s + 1 < s_hi) slab(A1, B1, s + 1, false);
+        if (NS > 2 && s + 2 < s_hi) slab(A2, B2, s + 2, false);
+      }
+    } else {
+      // Half a slab of fragments ahead: the hand-over stands between two
+      // halves' products, when the second half is in registers already.
+      union Frag { u4v_ q; gp_s8 v; };
+      Frag xa[2][FM], wb[2][FN];
+      auto fetch = [&](int h, const char* A, const char* B) {
+        const char *ca = A + la + (h ? x1 : x0), *cb = B + lb + (h ? x1 : x0);
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+          wb[h][j].q = *(const u4v_*)(cb + j * 2048);
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+          xa[h][i].q = *(const u4v_*)(ca + i * 2048);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto mma = [&](int h) {
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+          for (int j = 0; j < FN; j++)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                wb[h][j].v, xa[h][i].v, acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto slab = [&](char* A, char* B, const char* An, const char* Bn,
+                      int s, bool steady) {
+        fetch(1, A, B);
+        mma(0);
+        if (steady) {
+          gp_meet<PS * (NS - 2)>();
+          stage(A, B, s + NS);
+          fetch(0, An, Bn);
+        } else if (s + 1 < s_hi) {
+          gp_meet<0>();
+          if (s + NS < s_hi) stage(A, B, s + NS);
+          fetch(0, An, Bn);
+        }
+        mma(1);
+      };
+      fetch(0, A0, B0);
+      for (; s + 2 * NS <= s_hi; s += NS) {
+        slab(A0, B0, A1, B1, s, true);
+        slab(A1, B1, NS > 2 ? A2 : A0, NS > 2 ? B2 : B0, s + 1, true);
+        if (NS > 2) slab(A2, B2, A0, B0, s + 2, true);
+      }
+      for (; s < s_hi; s += NS) {
+        slab(A0, B0, A1, B1, s, false);
+        if (s + 1 < s_hi)
+          slab(A1, B1, NS > 2 ? A2 : A0, NS > 2 ? B2 : B0, s + 1, false);
+        if (NS > 2 && s + 2 < s_hi) slab(A2, B2, A0, B0, s + 2, false);
+      }
+    }
+  }
+
+  if (SK > 1) {
+    // fragments as they lie in registers: the last block reads them alike
+    float* pp = a.part + (size_t)tile * SK * (BM * BN) + tid * 4;
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++)
+        *(f4v*)(pp + (size_t)blockIdx.y * (BM * BN) +
+                (i * FN + j) * (NW * 256)) = acc[i][j];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const int t = __hip_atomic_fetch_add(&a.cnt[tile], 1, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+      last_flag = t == SK - 1;
+    }
+    __syncthreads();
+    if (!last_flag) return;
+    if (tid == 0) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      a.cnt[tile] = 0;                                  // for the next launch
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++) {
+        f4v v = {0.f, 0.f, 0.f, 0.f};
+        for (int q = 0; q < SK; q++)
+          v += *(const f4v*)(pp + (size_t)q * (BM * BN) +
+                             (i * FN + j) * (NW * 256));
+        acc[i][j] = v;
+      }
+  }
+
+  // fragment (i, j): row i*16 + fr, outputs j*16 + fk*4 + 0..3
+  constexpr int P = GLU ? 2 : 1;
+  const bool wide = a.N % 4 == 0;
+#pragma unroll
+  for (int i = 0; i < FM; i++) {
+    const int row = bm + (wm * FM + i) * 16 + fr;
+    if (row >= a.M) continue;
+    const float sx = F8 ? a.sx[row] : 1.f;
+#pragma unroll
+    for (int j = 0; j < FN; j += P) {
+      const int n = bn + (wn * FN + j) / P * 16 + fk * 4;
+      if (n >= a.N) continue;
+      f4v v = acc[i][j];
+      if (F8) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] *= sx * a.sw[min(n + r, a.N - 1)];
+      }
+      if constexpr (GLU) {
+        f4v u = acc[i][j + 1];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          if (F8) u[r] *= sx * a.sw[a.N + min(n + r, a.N - 1)];
+          v[r] = gp_act(v[r], a.act) * u[r];
+        }
+      }
+      const size_t at = (size_t)row * a.N + n;
+      if (wide) {
+        union { gp_b2 b[2]; u16 h[4]; unsigned long long q; } o;
+        if (a.bias) {
+          o.q = *(const unsigned long long*)(a.bias + n);
+#pragma unroll
+          for (int r = 0; r < 4; r++) v[r] += b2f(o.h[r]);
+        }
+        if (a.res) {
+          o.q = *(const unsigned long long*)(a.res + at);
+#pragma unroll
+          for (int r = 0; r < 4; r++) v[r] += b2f(o.h[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) o.b[r / 2][r % 2] = (__bf16)v[r];
+        *(unsigned long long*)(a.y + at) = o.q;
+      } else {
+        for (int r = 0; r < 4 && n + r < a.N; r++) {
+          float f = v[r];
+          if (a.bias) f += b2f(a.bias[n + r]);
+          if (a.res) f += b2f(a.res[at + r]);
+          a.y[at + r] = f2b(f);
+        }
+      }
+    }
+  }
+}
+
+template <bool F8, int BM, int BN, int WM, int WN, int NS>
+static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
+  const bool glu = a.act >= 0;
+  const int wide = glu ? BN / 2 : BN;
+  a.tm = (a.M + BM - 1) / BM;
+  a.tn = (a.N + wide - 1) / wide;
+  const dim3 grid((a.tm * a.tn + 7) / 8 * 8, sk);
+  if (glu)
+    hipLaunchKernelGGL((k_gemm_prompt<F8, BM, BN, WM, WN, NS, true>), grid,
+                       dim3(64 * WM * WN), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_gemm_prompt<F8, BM, BN, WM, WN, NS, false>), grid,
+                       dim3(64 * WM * WN), 0, s, a);
+  return hipGetLastError();
+}
+
+// Tile sizes, and microseconds that a slab takes on a CU that runs one block
+// of them or as many as fit (measured, bf16; e4m3 slabs move the same bytes
+// and differ by a tenth).  The big tiles win where there are rounds of them,
+// the small ones where a part-filled last round would cost more.
+struct GpTile { int bm, bn, occ; float one, full; };
+static const GpTile gp_tiles[] = {
+    {256, 256, 1, 1.80f, 1.80f},    // bf16 only: e4m3 fragments would spill
+    {128, 256, 1, 1.00f, 1.00f}, {128, 128, 2, 0.645f, 1.10f},
+    {64, 128, 2, 0.42f, 0.70f},  {128, 64, 2, 0.41f, 0.70f},
+    {64, 64, 3, 0.32f, 0.55f},   {32, 64, 4, 0.20f, 0.50f},
+};
+
+template <bool F8>
+static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
+                         hipStream_t s) {
+  const int width = a.act >= 0 ? 2 * a.N : a.N;
+  const int slabs = (int)(((long)a.K * (F8 ? 1 : 2) + 127) / 128);
+  int best = -1, best_sk = 1;
+  float best_t = 0.f;
+  for (int c = F8 ? 1 : 0; c < (int)(sizeof(gp_tiles) / sizeof(GpTile)); c++) {
+    const GpTile& g = gp_tiles[c];
+    const long tiles = (long)((a.M + g.bm - 1) / g.bm) *
+                       ((width + g.bn - 1) / g.bn);
+    for (int sk = 1; sk <= 8; sk *= 2) {
+      const double parts = (double)tiles * sk * g.bm * g.bn;
+      if (sk > 1 && (tiles > ncnt || parts > part_floats || slabs / sk < 4))
+        break;
+      const int per = (int)((tiles * sk + 255) / 256);   // blocks of a CU
+      float t = per / g.occ * g.full;
+      if (per % g.occ)
+        t += g.one + (g.full - g.one) * (per % g.occ - 1) /
+                         (g.occ > 1 ? g.occ - 1 : 1);
+      t *= (slabs + sk - 1) / sk;
+      if (sk > 1) t += 3.f + (float)(parts * 8e-6 / 4.0);  // write and read
+      if (best < 0 || t < best_t) {
+        best = c;
+        best_sk = sk;
+        best_t = t;
+      }
+    }
+  }
+  switch (best) {
+    case 0:
+      if constexpr (!F8) return gp_go<F8, 256, 256, 2, 4, 2>(a, best_sk, s);
+      break;
+    case 1: return gp_go<F8, 128, 256, 2, 4, 3>(a, best_sk, s);
+    case 2: return gp_go<F8, 128, 128, 2, 2, 2>(a, best_sk, s);
+    case 3: return gp_go<F8, 64, 128, 2, 2, 3>(a, best_sk, s);
+    case 4: return gp_go<F8, 128, 64, 2, 2, 3>(a, best_sk, s);
+    case 5: return gp_go<F8, 64, 64, 2, 2, 3>(a, best_sk, s);
+    case 6: return gp_go<F8, 32, 64, 2, 2, 3>(a, best_sk, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+// sx, sw: row scales of e4m3 x and w.  act < 0: no gate.  part and cnt (zero,
+// left zero) let K be split.
+extern "C" hipError_t launch_gemm_prompt(
+    const void* x, const void* w, const void* sx, const void* sw,
+    const void* res, const void* bias, void* y, void* part, void* cnt,
+    long part_floats, int ncnt, int M, int N, int K, int act,
+    hipStream_t stream) {
+  if (M < 1 || N < 1 || K < 64 || K % 64 || (!sx != !sw))
+    return hipErrorInvalidValue;
+  GpArgs a = {x, w, (const float*)sx, (const float*)sw, (const u16*)res,
+              (const u16*)bias, (u16*)y, (float*)part, (int*)cnt, M, N, K,
+              act, 0, 0};
+  if (!part || !cnt) part_floats = 0;
+  return sx ? gp_run<true>(a, part_floats, ncnt, stream)
+            : gp_run<false>(a, part_floats, ncnt, stream);
+}

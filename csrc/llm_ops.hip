@@ -18,7 +18,7 @@
 //  K1 softmax RawKernel      -> online softmax in k_attn_dec /
 //                               k_attn_rows / k_attn
 //  K2 cuBLAS GEMM/GEMV       -> k_gemv_{bf16,fp8}_t (decode),
-//                               k_gemm_bf16 MFMA (prefill)
+//                               k_gemm_prompt MFMA (prefill)
 //  K3 elementwise ufuncs     -> fused GEMV staging (NORM/GLU/NORM2),
 //                               k_rmsnorm, k_glu, k_softcap, k_addinto
 //  K4 KV concat              -> in-place pool writes
@@ -31,7 +31,6 @@
 #include <cstdlib>
 
 #include "common.h"
-#include "gemm_tile.h"
 
 // ====================================================================
 // GEMV: y[N] = W[N,K] @ stage(x)[K]  (+ res)  (optional softcap, f32 out)
@@ -2127,64 +2126,11 @@ extern "C" hipError_t launch_sample(const void* logits, int V, int lbf16,
   return hipGetLastError();
 }
 
-// ====================================================================
-// Prefill GEMM: Y[M,N] = X[M,K] @ W[N,K]^T (+res), bf16 in/out, fp32 acc.
-// MFMA v_mfma_f32_16x16x32_bf16; prefill only — decode uses k_gemv_bf16.
-// ====================================================================
-
 typedef short bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define BM 128
 #define BN 128
 #define BK 64
-
-// TS=BM=BN tile (128 or 64) over the shared MFMA main loop (gemm_tile.h).
-// The 64-tile variant exists because M=N=2048-class prefill GEMMs give
-// the 128-tile only ~256 blocks = 1 block/CU — no occupancy to hide the
-// DMA/barrier latency (measured 250 TF; see profiles/prefill_gemm_r02.md).
-template <int TS>
-__global__ void __launch_bounds__(256)
-k_gemm_bf16_t(const u16* __restrict__ X, const u16* __restrict__ W,
-              u16* __restrict__ Y, const u16* __restrict__ res,
-              float* __restrict__ accbuf, int M, int N, int K) {
-  __shared__ __attribute__((aligned(16))) char lds[gemm_lds_bytes<TS, TS>()];
-  const int bm = blockIdx.x * TS, bn = blockIdx.y * TS;
-  const int SK = gridDim.z;
-  const int kslices = (K / BK + SK - 1) / SK;
-  const int k_lo = blockIdx.z * kslices * BK;
-  int k_hi = k_lo + kslices * BK;
-  if (k_hi > K) k_hi = K;
-  const int nt = (k_hi - k_lo) / BK;
-  if (nt <= 0) return;
-
-  f4v acc[TS / 32][TS / 32];
-  gemm_mainloop<TS, TS, u16>(
-      acc, lds,
-      [&](int r) { return X + (size_t)min(bm + r, M - 1) * K; },
-      [&](int r) { return W + (size_t)min(bn + r, N - 1) * K; }, k_lo, nt);
-
-#pragma unroll
-  for (int i = 0; i < TS / 32; i++) {
-#pragma unroll
-    for (int j = 0; j < TS / 32; j++) {
-      const int col = bn + gemm_col<TS>(j);
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = bm + gemm_row0<TS>(i) + r;
-        if (row < M && col < N) {
-          float v = acc[i][j][r];
-          if (SK > 1) {
-            atomicAdd(accbuf + (size_t)row * N + col, v);
-          } else {
-            if (res) v += b2f(res[(size_t)row * N + col]);
-            Y[(size_t)row * N + col] = f2b(v);
-          }
-        }
-      }
-    }
-  }
-}
 
 // convert split-K fp32 accumulator to bf16 (+res); also used to zero it
 extern "C" __global__ void __launch_bounds__(256)
@@ -2205,48 +2151,6 @@ k_zero_f32(float* __restrict__ p, long total) {
   } else {
     for (; i < total; i++) p[i] = 0.f;  // tail: no over-write past total
   }
-}
-
-extern "C" hipError_t launch_gemm_bf16(const void* X, const void* W, void* Y,
-                                       const void* res, void* accbuf, int M,
-                                       int N, int K, hipStream_t stream) {
-  int gm = (M + BM - 1) / BM, gn = (N + BN - 1) / BN;
-  int ts = 128;
-  // small grids underfill 256 CUs at 1 block/CU with the 128-tile;
-  // the 64-tile doubles DMA traffic per output, so only when K is
-  // shallow enough that occupancy dominates (A/B: llama-1b 2k TTFT
-  // 11.8->10.4 ms; deep-K gemma shapes prefer the 128-tile)
-  if (gm * gn < 300 && K <= 2048 && K % 64 == 0) {
-    ts = 64;
-    gm = (M + 63) / 64;
-    gn = (N + 63) / 64;
-  }
-  int sk = 1;
-  if (accbuf && gm * gn < 160) {  // split K while the grid underfills
-    while (sk < 8 && gm * gn * sk * 2 <= 512 && (K / BK) % (sk * 2) == 0)
-      sk *= 2;
-  }
-  if (sk > 1) {
-    long total = (long)M * N;
-    hipLaunchKernelGGL(k_zero_f32, dim3((uint32_t)((total + 1023) / 1024)),
-                       dim3(256), 0, stream, (float*)accbuf, total);
-  }
-  dim3 grid(gm, gn, sk);
-  if (ts == 64)
-    hipLaunchKernelGGL((k_gemm_bf16_t<64>), grid, dim3(256), 0, stream,
-                       (const u16*)X, (const u16*)W, (u16*)Y, (const u16*)res,
-                       (float*)accbuf, M, N, K);
-  else
-    hipLaunchKernelGGL((k_gemm_bf16_t<128>), grid, dim3(256), 0, stream,
-                       (const u16*)X, (const u16*)W, (u16*)Y, (const u16*)res,
-                       (float*)accbuf, M, N, K);
-  if (sk > 1) {
-    long total = (long)M * N;
-    hipLaunchKernelGGL(k_gemm_fin, dim3((uint32_t)((total + 255) / 256)),
-                       dim3(256), 0, stream, (const float*)accbuf,
-                       (const u16*)res, (u16*)Y, total);
-  }
-  return hipGetLastError();
 }
 
 // ====================================================================
@@ -2395,144 +2299,6 @@ extern "C" hipError_t launch_quant_fp8(const void* X, void* Q, void* S,
   if (f32) { if (few) QUANT_CASE(float, 1024); else QUANT_CASE(float, 256); }
   else { if (few) QUANT_CASE(u16, 1024); else QUANT_CASE(u16, 256); }
 #undef QUANT_CASE
-  return hipGetLastError();
-}
-
-// ====================================================================
-// fp8 MFMA prefill GEMM: Y[M,N] = (sx_m * sy_n) * Xq[M,K] @ Wq[N,K]^T,
-// both operands OCP e4m3 with per-row scales (north star "CDNA4 fp8
-// MFMA").  v_mfma_f32_16x16x32_fp8_fp8; BM=BN=128, BK=64 (two K=32
-// slices), 4 waves (2x2), 64x64 per wave; LDS rows padded to 80 B so
-// 16-B stores stay aligned and b64 fragment reads spread banks.
-// Same split-K scheme as the bf16 GEMM (scales folded before the
-// atomicAdd so k_gemm_fin stays shared).
-// ====================================================================
-
-typedef long i64frag;
-
-extern "C" __global__ void __launch_bounds__(256)
-k_gemm_fp8(const uint8_t* __restrict__ X, const float* __restrict__ sx,
-           const uint8_t* __restrict__ W, const float* __restrict__ sw,
-           u16* __restrict__ Y, const u16* __restrict__ res,
-           float* __restrict__ accbuf, int M, int N, int K) {
-  constexpr int LDR = 80;  // padded LDS row stride (bytes)
-  __shared__ uint8_t As[2][128 * LDR];
-  __shared__ uint8_t Bs[2][128 * LDR];
-
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int wrow = wave >> 1, wcol = wave & 1;
-  const int bm = blockIdx.x * 128, bn = blockIdx.y * 128;
-
-  const int SK = gridDim.z;
-  const int kslices = (K / 64 + SK - 1) / SK;
-  const int k_lo = blockIdx.z * kslices * 64;
-  int k_hi = k_lo + kslices * 64;
-  if (k_hi > K) k_hi = K;
-  const int nt = (k_hi - k_lo) / 64;
-  if (nt <= 0) return;
-
-  f4v acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc[i][j] = {0.f, 0.f, 0.f, 0.f};
-
-  // stage: 128 rows x 64 B per operand; 256 threads x 2 iters x 16 B
-  auto stage = [&](int buf, int kt) {
-    const int k0 = k_lo + kt * 64;
-    for (int i = tid; i < 128 * 4; i += 256) {
-      int r = i >> 2, seg = i & 3;
-      int gr = bm + r;
-      int grc = gr < M ? gr : (M > 0 ? M - 1 : 0);
-      *(u4v_*)(&As[buf][r * LDR + seg * 16]) =
-          *(const u4v_*)(X + (size_t)grc * K + k0 + seg * 16);
-      int gb = bn + r;
-      int gbc = gb < N ? gb : N - 1;
-      *(u4v_*)(&Bs[buf][r * LDR + seg * 16]) =
-          *(const u4v_*)(W + (size_t)gbc * K + k0 + seg * 16);
-    }
-  };
-
-  stage(0, 0);
-  __syncthreads();
-
-  const int fr = lane & 15, fk8 = (lane >> 4) * 8;  // frag row / k-offset
-  int cur = 0;
-  for (int t = 0; t < nt; t++) {
-    if (t + 1 < nt) stage(cur ^ 1, t + 1);  // fill other buf during MFMA
-#pragma unroll
-    for (int sl = 0; sl < 2; sl++) {  // two K=32 slices per 64-B tile
-      i64frag a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        int ra = wrow * 64 + i * 16 + fr;
-        a[i] = *(const i64frag*)(&As[cur][ra * LDR + sl * 32 + fk8]);
-        int rb = wcol * 64 + i * 16 + fr;
-        b[i] = *(const i64frag*)(&Bs[cur][rb * LDR + sl * 32 + fk8]);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
-              a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();  // next iter writes cur / reads cur^1
-    cur ^= 1;
-  }
-
-  // epilogue: C col = lane&15, row = (lane>>4)*4 + reg (same map as bf16)
-  const int cc = lane & 15, cr = (lane >> 4) * 4;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        int row = bm + wrow * 64 + i * 16 + cr + r;
-        int col = bn + wcol * 64 + j * 16 + cc;
-        if (row < M && col < N) {
-          float v = acc[i][j][r] * sx[row] * sw[col];
-          if (SK > 1) {
-            atomicAdd(accbuf + (size_t)row * N + col, v);
-          } else {
-            if (res) v += b2f(res[(size_t)row * N + col]);
-            Y[(size_t)row * N + col] = f2b(v);
-          }
-        }
-      }
-    }
-  }
-}
-
-extern "C" hipError_t launch_gemm_fp8(const void* X, const void* sx,
-                                      const void* W, const void* sw, void* Y,
-                                      const void* res, void* accbuf, int M,
-                                      int N, int K, hipStream_t stream) {
-  if (K % 64 != 0) return hipErrorInvalidValue;
-  int gm = (M + 127) / 128, gn = (N + 127) / 128;
-  int sk = 1;
-  if (accbuf && gm * gn < 160) {
-    while (sk < 8 && gm * gn * sk * 2 <= 512 && (K / 64) % (sk * 2) == 0)
-      sk *= 2;
-  }
-  if (sk > 1) {
-    long total = (long)M * N;
-    hipLaunchKernelGGL(k_zero_f32, dim3((uint32_t)((total + 1023) / 1024)),
-                       dim3(256), 0, stream, (float*)accbuf, total);
-  }
-  dim3 grid(gm, gn, sk);
-  hipLaunchKernelGGL(k_gemm_fp8, grid, dim3(256), 0, stream,
-                     (const uint8_t*)X, (const float*)sx, (const uint8_t*)W,
-                     (const float*)sw, (u16*)Y, (const u16*)res,
-                     (float*)accbuf, M, N, K);
-  if (sk > 1) {
-    long total = (long)M * N;
-    hipLaunchKernelGGL(k_gemm_fin, dim3((uint32_t)((total + 255) / 256)),
-                       dim3(256), 0, stream, (const float*)accbuf,
-                       (const u16*)res, (u16*)Y, total);
-  }
   return hipGetLastError();
 }
 

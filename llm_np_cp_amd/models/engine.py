@@ -240,9 +240,6 @@ class GPUModel(DecodeLoop):
                     hrows(w[f"{p}.mlp.up_proj.weight"])], axis=0)
                 down_np = hcols(w[f"{p}.mlp.down_proj.weight"])
             o_np = hcols(w[f"{a}.o_proj.weight"])
-            nq = self.nh_l * hd
-            nkv = self.kvh_l * hd
-            I = self.inter_l
             lw = {
                 "g_in": gamma(w[f"{p}.input_layernorm.weight"]),
                 "g_post": gamma(w[f"{p}.post_attention_layernorm.weight"]),
@@ -256,43 +253,9 @@ class GPUModel(DecodeLoop):
                         lw[name + "_q"], lw[name + "_s"] = quant8(arr)
                     if self.wq4:
                         lw[name + "_q4"], lw[name + "_e4"] = quant4(arr)
-                if self.keep_fp8:
-                    lw.update({
-                        "wq_q": lw["wqkv_q"][:nq],
-                        "wq_s": lw["wqkv_s"][:nq],
-                        "wk_q": lw["wqkv_q"][nq:nq + nkv],
-                        "wk_s": lw["wqkv_s"][nq:nq + nkv],
-                        "wv_q": lw["wqkv_q"][nq + nkv:],
-                        "wv_s": lw["wqkv_s"][nq + nkv:],
-                        "wgate_q": lw["wgu_q"][:I],
-                        "wgate_s": lw["wgu_s"][:I],
-                        "wup_q": lw["wgu_q"][I:], "wup_s": lw["wgu_s"][I:],
-                    })
-                if self.wq4:
-                    lw.update({
-                        "wq_q4": lw["wqkv_q4"][:nq],
-                        "wq_e4": lw["wqkv_e4"][:nq],
-                        "wk_q4": lw["wqkv_q4"][nq:nq + nkv],
-                        "wk_e4": lw["wqkv_e4"][nq:nq + nkv],
-                        "wv_q4": lw["wqkv_q4"][nq + nkv:],
-                        "wv_e4": lw["wqkv_e4"][nq + nkv:],
-                        "wgate_q4": lw["wgu_q4"][:I],
-                        "wgate_e4": lw["wgu_e4"][:I],
-                        "wup_q4": lw["wgu_q4"][I:],
-                        "wup_e4": lw["wgu_e4"][I:],
-                    })
             else:
-                wqkv = bf16(qkv_np)
-                wgu = bf16(gu_np)
-                lw.update({
-                    # fused tensors (decode path) + contiguous row views
-                    "wqkv": wqkv,
-                    "wq": wqkv[:nq], "wk": wqkv[nq:nq + nkv],
-                    "wv": wqkv[nq + nkv:],
-                    "wgu": wgu, "wgate": wgu[:I], "wup": wgu[I:],
-                    "wo": bf16(o_np),
-                    "wdown": bf16(down_np),
-                })
+                lw.update({"wqkv": bf16(qkv_np), "wgu": bf16(gu_np),
+                           "wo": bf16(o_np), "wdown": bf16(down_np)})
             if self.moe:
                 # router weights + decode-shaped views: the GEMV sees the
                 # FIRST expert's rows (N=2I / N=H) and offsets the base
@@ -318,16 +281,12 @@ class GPUModel(DecodeLoop):
                 lw["g_postffn"] = gamma(w[f"{p}.post_feedforward_layernorm.weight"])
             if cfg.attention_bias:
                 # Qwen-2 family: fused qkv bias (decode GEMV adds it via
-                # the res slot; prefill adds it after the GEMM)
+                # the res slot, the products of more rows as they store)
                 bias_np = _np.concatenate([
                     hrows(w[f"{a}.q_proj.bias"]),
                     hrows(w[f"{a}.k_proj.bias"]),
                     hrows(w[f"{a}.v_proj.bias"])], axis=0)
-                bqkv = bf16(bias_np.reshape(1, -1))[0]
-                lw["bqkv"] = bqkv
-                lw["bias_q"] = bqkv[:nq]
-                lw["bias_k"] = bqkv[nq:nq + nkv]
-                lw["bias_v"] = bqkv[nq + nkv:]
+                lw["bqkv"] = bf16(bias_np.reshape(1, -1))[0]
             self.layers.append(lw)
 
     def _alloc_state(self, prefill_chunk: int):
@@ -369,7 +328,8 @@ class GPUModel(DecodeLoop):
                                   **bf)
         self.b_att = torch.zeros(PC, self.nh_l * hd, **bf)
         self.b_gate = torch.zeros(PC, I, **bf)
-        self.b_up = torch.zeros(PC, I, **bf)
+        if self.wq4:          # its prompts have gate and up apart
+            self.b_up = torch.zeros(PC, I, **bf)
         self.b_gemm_acc = torch.zeros(PC * max(I, H), dtype=torch.float32,
                                       device=dev)
         if self.fp8:
@@ -377,12 +337,17 @@ class GPUModel(DecodeLoop):
             kmax = max(H, I, self.nh_l * hd)
             self.b_xq = torch.zeros(PC * kmax, dtype=torch.uint8, device=dev)
             self.b_sx = torch.zeros(PC, dtype=torch.float32, device=dev)
+            if self.moe:
+                self.b_aq = torch.zeros(PC * I, dtype=torch.uint8, device=dev)
+                self.b_sa = torch.zeros(PC, dtype=torch.float32, device=dev)
             # act(gate) * up of few rows, to be rounded to e4m3 next
             self.b_act32 = torch.zeros(ho.FEW_ROWS, I, dtype=torch.float32,
                                        device=dev)
         # few-row products that split K: blocks that are done, by column
         # group (the parts go to b_gemm_acc)
         self.row_cnt = torch.zeros(256, dtype=torch.int32, device=dev)
+        # the same of many-row products, by tile
+        self.tile_cnt = torch.zeros(1024, dtype=torch.int32, device=dev)
         self.b_logits_l = torch.zeros(self.vocab_l, dtype=torch.float32,
                                       device=dev)
         self.b_logits = (self.b_logits_l if not self.tp_branch else
@@ -507,26 +472,35 @@ class GPUModel(DecodeLoop):
             ho.row_gemm(x, lw[name], y, M, **kw)
 
     def _linear(self, lw, name, x, y, res=None, M: int = 1,
-                batch: bool = False):
+                batch: bool = False, bias=None, act: int = -1):
         """Projection by weight NAME so dtype routing stays in one
         place: few rows, bf16 MFMA GEMM, or (fp8) fp8-MFMA GEMM with
-        on-the-fly activation row quantization."""
+        on-the-fly activation row quantization.  ``act``: gate and up rows,
+        y = act(gate) * up."""
         if M <= ho.FEW_ROWS:
             self._rows(lw, name, x, y, M, res=res, batch=batch)
-        elif self.wq4:
-            ho.gemm_fp4w(x[:M], lw[name + "_q4"], lw[name + "_e4"], y[:M],
-                         res=res[:M] if res is not None else None,
-                         accbuf=self.b_gemm_acc)
-        elif self.fp8:
-            K = x.shape[-1]
+            return
+        res = res[:M] if res is not None else None
+        kw = dict(res=res, accbuf=self.b_gemm_acc)
+        if self.wq4:
+            q, e = lw[name + "_q4"], lw[name + "_e4"]
+            if act >= 0:
+                n = q.shape[0] // 2
+                ho.gemm_fp4w(x[:M], q[:n], e[:n], y[:M], **kw)
+                ho.gemm_fp4w(x[:M], q[n:], e[n:], self.b_up[:M], **kw)
+                ho.glu(y[:M], self.b_up[:M], y[:M], act)
+            else:
+                ho.gemm_fp4w(x[:M], q, e, y[:M], **kw)
+            if bias is not None:
+                ho.bias_add(y[:M], bias, M)
+            return
+        kw.update(bias=bias, act=act, cnt=self.tile_cnt)
+        if self.fp8:
             ho.quant_fp8(x[:M], self.b_xq, self.b_sx)
             ho.gemm_fp8(self.b_xq, self.b_sx, lw[name + "_q"],
-                        lw[name + "_s"], y[:M], M, K,
-                        res=res[:M] if res is not None else None,
-                        accbuf=self.b_gemm_acc)
+                        lw[name + "_s"], y[:M], M, x.shape[-1], **kw)
         else:
-            ho.gemm(x[:M], lw[name], y, res=res[:M] if res is not None else None,
-                    accbuf=self.b_gemm_acc)
+            ho.gemm(x[:M], lw[name], y, **kw)
 
     def _rowpar_ar(self, lw, name, x, y, M: int, batch: bool = False):
         """Row-parallel projection followed by all-reduce over TP ranks.
@@ -551,9 +525,11 @@ class GPUModel(DecodeLoop):
             elif self.fp8:
                 ho.gemm_fp8(self.b_xq[a * K:], self.b_sx[a:],
                             lw[name + "_q"], lw[name + "_s"], y[a:b],
-                            b - a, K, accbuf=self.b_gemm_acc)
+                            b - a, K, accbuf=self.b_gemm_acc,
+                            cnt=self.tile_cnt)
             else:
-                ho.gemm(x[a:b], lw[name], y[a:b], accbuf=self.b_gemm_acc)
+                ho.gemm(x[a:b], lw[name], y[a:b], accbuf=self.b_gemm_acc,
+                        cnt=self.tile_cnt)
             # async -> lands on the RCCL stream after the chunk's GEMM;
             # the compute stream proceeds to the next chunk immediately
             works.append(dist.all_reduce(y[a:b], async_op=True))
@@ -612,9 +588,7 @@ class GPUModel(DecodeLoop):
                            bias=lw.get("bqkv"), batch=batch_attn)
             else:
                 ho.rmsnorm(h[:M], lw["g_in"], xn[:M], eps=eps)
-                self._linear(lw, "wqkv", xn, qkv, M=M)
-                if "bqkv" in lw:
-                    ho.bias_add(qkv, lw["bqkv"], M)
+                self._linear(lw, "wqkv", xn, qkv, M=M, bias=lw.get("bqkv"))
             if batch_attn:
                 ho.attn_dec(qkv, self.k_cache[i], self.v_cache[i],
                             self.b_att[0], self.bt_lens, self.cos_t,
@@ -660,10 +634,7 @@ class GPUModel(DecodeLoop):
                                batch=batch_attn)
                 else:
                     ho.rmsnorm(h[:M], g_mlp, xn[:M], eps=eps)
-                    self._linear(lw, "wgate", xn, self.b_gate, M=M)
-                    self._linear(lw, "wup", xn, self.b_up, M=M)
-                    ho.glu(self.b_gate[:M], self.b_up[:M], self.b_gate[:M],
-                           self.act)
+                    self._linear(lw, "wgu", xn, a, M=M, act=self.act)
                 into_h("wdown", a)
             if layer_hook is not None:
                 layer_hook(i, h[:M])
@@ -678,38 +649,27 @@ class GPUModel(DecodeLoop):
         cfg = self.config
         E, I, H = cfg.num_local_experts, self.inter_l, self.H
         eps = cfg.rms_norm_eps
-        xn, gate, up, t1 = self.b_xn, self.b_gate, self.b_up, self.b_t1
+        xn, gate, t1 = self.b_xn, self.b_gate, self.b_t1
         ho.moe_route(self.b_h, lw["g_post"], lw["wg"], M, self.topk,
                      self.moe_idx, self.moe_w, dense=self.moe_dense,
                      eps=eps)
+        kw = dict(accbuf=self.b_gemm_acc, cnt=self.tile_cnt)
+        if self.fp8:
+            ho.quant_fp8(xn[:M], self.b_xq, self.b_sx)
         for e in range(E):
-            g_lo, g_hi = e * 2 * I, e * 2 * I + I
-            u_hi = (e + 1) * 2 * I
-            d_lo, d_hi = e * H, (e + 1) * H
+            gu, dn = slice(e * 2 * I, (e + 1) * 2 * I), \
+                slice(e * H, (e + 1) * H)
             if self.fp8:
-                ho.quant_fp8(xn[:M], self.b_xq, self.b_sx)
-                ho.gemm_fp8(self.b_xq, self.b_sx,
-                            lw["wgu_q_all"][g_lo:g_hi],
-                            lw["wgu_s_all"][g_lo:g_hi], gate[:M], M, H,
-                            accbuf=self.b_gemm_acc)
-                ho.gemm_fp8(self.b_xq, self.b_sx,
-                            lw["wgu_q_all"][g_hi:u_hi],
-                            lw["wgu_s_all"][g_hi:u_hi], up[:M], M, H,
-                            accbuf=self.b_gemm_acc)
-                ho.glu(gate[:M], up[:M], gate[:M], self.act)
-                ho.quant_fp8(gate[:M], self.b_xq, self.b_sx)
-                ho.gemm_fp8(self.b_xq, self.b_sx,
-                            lw["wdown_q_all"][d_lo:d_hi],
-                            lw["wdown_s_all"][d_lo:d_hi], t1[:M], M, I,
-                            accbuf=self.b_gemm_acc)
+                ho.gemm_fp8(self.b_xq, self.b_sx, lw["wgu_q_all"][gu],
+                            lw["wgu_s_all"][gu], gate[:M], M, H,
+                            act=self.act, **kw)
+                ho.quant_fp8(gate[:M], self.b_aq, self.b_sa)
+                ho.gemm_fp8(self.b_aq, self.b_sa, lw["wdown_q_all"][dn],
+                            lw["wdown_s_all"][dn], t1[:M], M, I, **kw)
             else:
-                ho.gemm(xn[:M], lw["wgu_all"][g_lo:g_hi], gate[:M],
-                        accbuf=self.b_gemm_acc)
-                ho.gemm(xn[:M], lw["wgu_all"][g_hi:u_hi], up[:M],
-                        accbuf=self.b_gemm_acc)
-                ho.glu(gate[:M], up[:M], gate[:M], self.act)
-                ho.gemm(gate[:M], lw["wdown_all"][d_lo:d_hi], t1[:M],
-                        accbuf=self.b_gemm_acc)
+                ho.gemm(xn[:M], lw["wgu_all"][gu], gate[:M], act=self.act,
+                        **kw)
+                ho.gemm(gate[:M], lw["wdown_all"][dn], t1[:M], **kw)
             ho.moe_scale_add(self.b_h, t1, self.moe_dense[e:], E, M, H)
 
     @property
@@ -723,24 +683,25 @@ class GPUModel(DecodeLoop):
             return h
         return {"": self.lm_head}
 
-    def _head_rows(self, M: int, out: torch.Tensor):
+    def _head_rows(self, M: int, out: torch.Tensor, batch: bool = False):
         """out[:M] = logits (bf16, this rank's vocabulary) of rows of h."""
         if M <= ho.FEW_ROWS:
             self._rows(self._head, "", self.b_h, out, M, g=self.g_final,
-                       softcap=self.final_softcap)
+                       softcap=self.final_softcap, batch=batch)
             return
         ho.rmsnorm(self.b_h[:M], self.g_final, self.b_xn[:M],
                    eps=self.config.rms_norm_eps)
-        if self.wq4:
+        if self.wq4 and not batch:
             ho.gemm_fp4w(self.b_xn[:M], self.lm_head_q4, self.lm_head_e4,
                          out[:M], accbuf=self.b_gemm_acc)
         elif self.fp8:
             ho.quant_fp8(self.b_xn[:M], self.b_xq, self.b_sx)
             ho.gemm_fp8(self.b_xq, self.b_sx, self.lm_head_q, self.lm_head_s,
-                        out[:M], M, self.H, accbuf=self.b_gemm_acc)
+                        out[:M], M, self.H, accbuf=self.b_gemm_acc,
+                        cnt=self.tile_cnt)
         else:
             ho.gemm(self.b_xn[:M], self.lm_head, out[:M],
-                    accbuf=self.b_gemm_acc)
+                    accbuf=self.b_gemm_acc, cnt=self.tile_cnt)
         if self.final_softcap:
             ho.softcap(out[:M], self.final_softcap)
 
@@ -1098,23 +1059,7 @@ class GPUModel(DecodeLoop):
             return self._decode_batch_step_mx(B, greedy, min_p, temperature)
         ho.embed(self.embed, self.bt_next, self.b_h, B, cfg.embed_scale)
         self._layers_forward(B, batch_attn=True)
-        if B <= ho.FEW_ROWS:
-            self._rows(self._head, "", self.b_h, self.bt_logits, B,
-                       g=self.g_final, softcap=self.final_softcap,
-                       batch=True)
-        else:
-            ho.rmsnorm(self.b_h[:B], self.g_final, self.b_xn[:B],
-                       eps=cfg.rms_norm_eps)
-            if self.fp8:
-                ho.quant_fp8(self.b_xn[:B], self.b_xq, self.b_sx)
-                ho.gemm_fp8(self.b_xq, self.b_sx, self.lm_head_q,
-                            self.lm_head_s, self.bt_logits[:B], B, self.H,
-                            accbuf=self.b_gemm_acc)
-            else:
-                ho.gemm(self.b_xn[:B], self.lm_head, self.bt_logits[:B],
-                        accbuf=self.b_gemm_acc)
-            if self.final_softcap:
-                ho.softcap(self.bt_logits[:B], self.final_softcap)
+        self._head_rows(B, self.bt_logits, batch=True)
         ho.sample(self.bt_logits[:B], min_p, greedy, self.seed,
                   self.rng_ctr, self.bt_gmax, self.bt_pick, self.bt_next,
                   self.bt_ring, self.bt_nout, self.bt_lens, bump_len=True,

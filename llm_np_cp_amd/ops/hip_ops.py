@@ -59,8 +59,8 @@ _SIGS = {
                       ctypes.c_int, ctypes.c_uint64, ctypes.c_float] +
                      [ctypes.c_void_p] * 8 +
                      [ctypes.c_int, ctypes.c_void_p],
-    "launch_gemm_bf16": [ctypes.c_void_p] * 5 + [ctypes.c_int] * 3 +
-                        [ctypes.c_void_p],
+    "launch_gemm_prompt": [ctypes.c_void_p] * 9 + [ctypes.c_long] +
+                          [ctypes.c_int] * 5 + [ctypes.c_void_p],
     "launch_row_gemm": [ctypes.c_void_p] * 11 + [ctypes.c_long] +
                        [ctypes.c_int] * 10 +
                        [ctypes.c_float, ctypes.c_float, ctypes.c_void_p],
@@ -89,8 +89,6 @@ _SIGS = {
                           [ctypes.c_int] * 5 +
                           [ctypes.c_float, ctypes.c_int, ctypes.c_float,
                            ctypes.c_float, ctypes.c_void_p],
-    "launch_gemm_fp8": [ctypes.c_void_p] * 7 + [ctypes.c_int] * 3 +
-                       [ctypes.c_void_p],
     "launch_gemm_fp4w": [ctypes.c_void_p] * 6 + [ctypes.c_int] * 3 +
                         [ctypes.c_void_p],
     "launch_moe_route": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4 +
@@ -346,19 +344,28 @@ def sample(logits: torch.Tensor, min_p: float, greedy: bool, seed: int,
         1 if bump_len else 0, _stream()), "sample")
 
 
+def _gemm_prompt(name, x, w, sx, sw, y, M, K, res, bias, act, accbuf, cnt):
+    N = w.shape[0] // (2 if act >= 0 else 1)
+    assert w.shape[1] == K and K % 64 == 0
+    _check(lib().launch_gemm_prompt(
+        _ptr(x), _ptr(w), _ptr(sx), _ptr(sw), _ptr(res), _ptr(bias), _ptr(y),
+        _ptr(accbuf), _ptr(cnt),
+        ctypes.c_long(0 if accbuf is None else accbuf.numel()),
+        0 if cnt is None else cnt.numel(), M, N, K, act, _stream()), name)
+
+
 def gemm(X: torch.Tensor, W: torch.Tensor, Y: torch.Tensor,
          res: torch.Tensor | None = None,
-         accbuf: torch.Tensor | None = None):
-    """Y[M,N] = X[M,K] @ W[N,K]^T (+res), bf16, MFMA prefill path.
-    With accbuf (fp32 scratch >= M*N) small-M launches split K over
-    grid.z for chip fill."""
+         accbuf: torch.Tensor | None = None,
+         bias: torch.Tensor | None = None, act: int = -1,
+         cnt: torch.Tensor | None = None):
+    """Y[M,N] = X[M,K] @ W[N,K]^T (+bias, +res), bf16, MFMA prefill path.
+    act 0/1: W holds gate rows, then up rows, and Y = act(gate) * up.
+    accbuf (fp32) and cnt (int32, zero; left zero) let K be split over
+    blocks where there are few tiles."""
     M, K = X.shape
-    N = W.shape[0]
-    assert W.shape[1] == K and K % 64 == 0
-    if accbuf is not None and accbuf.numel() < M * N:
-        accbuf = None
-    _check(lib().launch_gemm_bf16(_ptr(X), _ptr(W), _ptr(Y), _ptr(res),
-                                  _ptr(accbuf), M, N, K, _stream()), "gemm")
+    _gemm_prompt("gemm", X, W, None, None, Y, M, K, res, bias, act, accbuf,
+                 cnt)
 
 
 FEW_ROWS = 16        # rows that row_gemm takes
@@ -443,16 +450,14 @@ def gemv_fp4(Wq: torch.Tensor, We: torch.Tensor, x: torch.Tensor,
 def gemm_fp8(xq: torch.Tensor, sx: torch.Tensor, Wq: torch.Tensor,
              sw: torch.Tensor, y: torch.Tensor, M: int, K: int,
              res: torch.Tensor | None = None,
-             accbuf: torch.Tensor | None = None):
-    """Y[M,N] = (sx_m * sw_n) * Xq[M,K] @ Wq[N,K]^T (+res): fp8 MFMA
-    prefill path (both operands e4m3 with per-row scales)."""
-    N = Wq.shape[0]
-    assert Wq.shape[-1] == K and K % 64 == 0
-    if accbuf is not None and accbuf.numel() < M * N:
-        accbuf = None
-    _check(lib().launch_gemm_fp8(
-        _ptr(xq), _ptr(sx), _ptr(Wq), _ptr(sw), _ptr(y), _ptr(res),
-        _ptr(accbuf), M, N, K, _stream()), "gemm_fp8")
+             accbuf: torch.Tensor | None = None,
+             bias: torch.Tensor | None = None, act: int = -1,
+             cnt: torch.Tensor | None = None):
+    """Y[M,N] = (sx_m * sw_n) * Xq[M,K] @ Wq[N,K]^T (+bias, +res): fp8 MFMA
+    prefill path (both operands e4m3 with per-row scales); the rest as in
+    gemm."""
+    _gemm_prompt("gemm_fp8", xq, Wq, sx, sw, y, M, K, res, bias, act, accbuf,
+                 cnt)
 
 
 def gemv_fp8_mx(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,

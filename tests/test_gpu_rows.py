@@ -124,3 +124,41 @@ def test_few_rows(N, K, M, kind, norm, act):
     assert off(Y[:M], z) < (2.0 ** -6 if norm and kind == "fp8"
                             else 2.0 ** -7)
     assert (Y[M] == 7.0).all() and not cnt.any()
+
+
+# tiles of 32 to 256 rows and 64 to 256 outputs, by what the sizes call for:
+# a rest of a tile both ways, outputs that are no multiple of four, K of one
+# slab, of one more than the buffers, split over blocks, half a slab (e4m3)
+@pytest.mark.parametrize("M,N,K", [
+    (17, 70, 64), (37, 258, 192), (33, 200, 8192), (130, 1000, 320),
+    (300, 3000, 448), (513, 4100, 256), (1030, 2050, 64), (2050, 6200, 128),
+    (2049, 16500, 64)])
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+@pytest.mark.parametrize("act", [-1, 0, 1])
+def test_many_rows(M, N, K, kind, act):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    W = normal(N * (2 if act >= 0 else 1), K, seed=7, scale=K ** -0.5)
+    X = normal(M, K, seed=8)
+    bias, res = normal(N, seed=9), normal(M, N, seed=10)
+    part = torch.zeros(1 << 24, device="cuda")
+    cnt = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    Y = torch.full((M + 1, N), 7.0, device="cuda").bfloat16()
+    kw = dict(res=res, bias=bias, act=act, accbuf=part, cnt=cnt)
+    Wd, x = W.double(), X.double()
+    if kind == "fp8":
+        (W, sw, Wd), (X, sx, x) = e4m3(W), e4m3(X)
+    for _ in range(2):                              # counters are left zero
+        if kind == "fp8":
+            ho.gemm_fp8(X, sx, W, sw, Y[:M], M, K, **kw)
+        else:
+            ho.gemm(X, W, Y[:M], **kw)
+    z = x @ Wd.T
+    if act >= 0:
+        f = (torch.nn.functional.silu if act == 0 else lambda t:
+             torch.nn.functional.gelu(t, approximate="tanh"))
+        z = f(z[:, :N]) * z[:, N:]
+    z = z + bias.double() + res.double()
+    # exact products, fp32 sums, bf16 results: 2^-9 at most
+    assert off(Y[:M], z) < 2.0 ** -9
+    assert (Y[M] == 7.0).all() and not cnt.any()
