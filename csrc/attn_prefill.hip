@@ -17,12 +17,13 @@
 //
 // What bounds it: head_dim 128 spends 512 MFMA cycles and about 450 VALU
 // cycles on 32 keys x 32 rows; two blocks of 64 KB LDS on a CU overlap them.
-// Measured (32/8 heads of 128, 2048 rows behind 6139 keys): 314 us,
-// 765 TFLOP/s; a wave per head and 16 queries took 1422 us.  5 rows of 24/8
-// heads over 906 keys, split: 19 us, unsplit per-head waves 74 us.  Head
-// dim 256 spills some 20 registers at two waves a SIMD and is still faster
-// than one wave without (2048 rows behind 2048 keys: 163 to 219 us, before
-// 507 us).
+// Measured (32/8 heads of 128, 2048 rows behind 6139 keys): 291 us,
+// 827 TFLOP/s; a wave per head and 16 queries took 1422 us.  (With both
+// buffers in one array the DMA drained ahead of every tile's reads: 314 us.)
+// 5 rows of 24/8 heads over 906 keys, split: 18 us, unsplit per-head waves
+// 74 us.  Head dim 256 at two waves a SIMD just fits the registers, an fp8
+// pool spills some 40; one wave a SIMD without spills was slower (2048 rows
+// behind 2048 keys: 219 us to 163 when it still spilled 20, now 118).
 #include "common.h"
 #include "attn_prefill.h"
 
@@ -58,9 +59,14 @@ k_attn_rows(ApArgs a) {
   constexpr int SLOTS = HD / 8;              // 16-byte slots of a row
   constexpr int NS = BKV / 32;               // 32-key parts of a tile
   constexpr int NT = 64 * NW;
-  __shared__ __attribute__((aligned(16))) char Ks[2][TILE];
-  __shared__ __attribute__((aligned(16))) char Vs[2][TILE];
-  __shared__ __attribute__((aligned(16))) float Sc[2][2][KV8 ? BKV : 4];
+  constexpr bool RAW = !CAP && !KV8;
+  // an array a buffer, and the loop unrolled over the two: the compiler sees
+  // that the DMA into one does not touch what is read from the other, and
+  // does not wait for it before the reads
+  __shared__ __attribute__((aligned(16))) char K0[TILE], K1[TILE];
+  __shared__ __attribute__((aligned(16))) char V0[TILE], V1[TILE];
+  __shared__ __attribute__((aligned(16))) float S0[2][KV8 ? BKV : 4],
+      S1[2][KV8 ? BKV : 4];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -118,7 +124,7 @@ k_attn_rows(ApArgs a) {
   // bf16 pool: straight into LDS.  A wave's instruction fills 1 KB, lane by
   // lane; the swizzle sits in the address that the lane reads.
   constexpr int RPI = 1024 / RB;             // rows an instruction fills
-  auto stage16 = [&](int buf, int t0) {
+  auto stage16 = [&](char* Ks, char* Vs, int t0) {
 #pragma unroll
     for (int i = 0; i < BKV / RPI / NW; i++) {
       const int r0 = (i * NW + wave) * RPI;
@@ -127,12 +133,12 @@ k_attn_rows(ApArgs a) {
       __builtin_amdgcn_global_load_lds(
           (const __attribute__((address_space(1))) uint32_t*)(
               Kg + t * RB + k_slot<HD>(r, s) * 16),
-          (__attribute__((address_space(3))) uint32_t*)(&Ks[buf][r0 * RB]),
+          (__attribute__((address_space(3))) uint32_t*)(Ks + r0 * RB),
           16, 0, 0);
       __builtin_amdgcn_global_load_lds(
           (const __attribute__((address_space(1))) uint32_t*)(
               Vg + t * RB + v_slot<HD>(r, s) * 16),
-          (__attribute__((address_space(3))) uint32_t*)(&Vs[buf][r0 * RB]),
+          (__attribute__((address_space(3))) uint32_t*)(Vs + r0 * RB),
           16, 0, 0);
     }
   };
@@ -160,7 +166,7 @@ k_attn_rows(ApArgs a) {
       }
     }
   };
-  auto store8 = [&](int buf) {
+  auto store8 = [&](char* Ks, char* Vs, float (*Sc)[KV8 ? BKV : 4]) {
     if constexpr (KV8) {
 #pragma unroll
       for (int i = 0; i < L8; i++) {
@@ -180,17 +186,31 @@ k_attn_rows(ApArgs a) {
                 vr[i][h * 2 + d], 1.0f, true);
           }
           const int sl = s * 2 + h;
-          *(s8v*)(&Ks[buf][r * RB + k_slot<HD>(r, sl) * 16]) = ko.v;
-          *(s8v*)(&Vs[buf][r * RB + v_slot<HD>(r, sl) * 16]) = vo.v;
+          *(s8v*)(Ks + r * RB + k_slot<HD>(r, sl) * 16) = ko.v;
+          *(s8v*)(Vs + r * RB + v_slot<HD>(r, sl) * 16) = vo.v;
         }
       }
 #pragma unroll
       for (int i = 0; i < NSC; i++) {
         const int e = i * NT + tid;
-        if (e < 2 * BKV) Sc[buf][e / BKV][e % BKV] = scr[i];
+        if (e < 2 * BKV) Sc[e / BKV][e % BKV] = scr[i];
       }
     }
   };
+
+  // LDS offsets of fragments that the swizzle makes differ by more than a
+  // constant: 8 of K (16-byte slots of a row), 4 of V (64-byte chunks)
+  constexpr int KC = HD / 16 < 8 ? HD / 16 : 8, VD = HD / 32 < 4 ? HD / 32 : 4;
+  const int vrow = hh * 4 + ((lane & 15) >> 2);
+  const int vcol = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+  int kb[KC], vb[VD];
+#pragma unroll
+  for (int c = 0; c < KC; c++)
+    kb[c] = col * RB + k_slot<HD>(col, c * 2 + hh) * 16;
+#pragma unroll
+  for (int d = 0; d < VD; d++)
+    vb[d] = vrow * RB + v_slot<HD>(vrow, d * 4 + (vcol >> 3)) * 16 +
+            (vcol & 7) * 2;
 
   float m = -INFINITY, l = 0.f;     // m in units of log2
   ap_f16 o[HD / 32];
@@ -201,17 +221,12 @@ k_attn_rows(ApArgs a) {
   const float c1 = CAP ? a.scale / a.softcap : a.scale * LOG2E;
   const float c2 = CAP ? a.softcap * LOG2E : 1.f;
 
-  if (k_lo < k_hi) {
-    if constexpr (KV8) { load8(k_lo); store8(0); }
-    else stage16(0, k_lo);
-  }
-  __syncthreads();
-  int cur = 0;
-  for (int t0 = k_lo; t0 < k_hi; t0 += BKV) {
+  auto tile = [&](char* Ks, char* Vs, float (*Sc)[KV8 ? BKV : 4], char* Kn,
+                  char* Vn, float (*Sn)[KV8 ? BKV : 4], int t0) {
     const bool more = t0 + BKV < k_hi;
     if (more) {
       if constexpr (KV8) load8(t0 + BKV);
-      else stage16(cur ^ 1, t0 + BKV);
+      else stage16(Kn, Vn, t0 + BKV);
     }
     const bool some = live && t0 <= q_hi &&
                       (a.window <= 0 || t0 + BKV > q_lo - a.window);
@@ -221,11 +236,10 @@ k_attn_rows(ApArgs a) {
       for (int n = 0; n < NS; n++) {
 #pragma unroll
         for (int r = 0; r < 16; r++) s[n][r] = 0.f;
-        const int kr_ = n * 32 + col;
 #pragma unroll
         for (int c = 0; c < HD / 16; c++) {
           const ap_b8 kf = *(const ap_b8*)(
-              &Ks[cur][kr_ * RB + k_slot<HD>(kr_, c * 2 + hh) * 16]);
+              Ks + kb[c % KC] + c / KC * 256 + n * 32 * RB);
           s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[c], s[n], 0,
                                                          0, 0);
         }
@@ -233,30 +247,41 @@ k_attn_rows(ApArgs a) {
       // keys t0 + 32n + 8(r/4) + 4hh + r%4
       const bool edge = t0 + BKV - 1 > q_lo || t0 + BKV > k_hi ||
                         (a.window > 0 && t0 <= q_hi - a.window);
+      // Plain scores stay as they are: their scale rides in the exponent.
+      if constexpr (!RAW) {
+#pragma unroll
+        for (int n = 0; n < NS; n++)
+#pragma unroll
+          for (int q4 = 0; q4 < 4; q4++) {
+            f4v ks = {1.f, 1.f, 1.f, 1.f};
+            if constexpr (KV8)
+              ks = *(const f4v*)(&Sc[0][n * 32 + q4 * 8 + hh * 4]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+              float v = s[n][q4 * 4 + j] * c1;
+              if constexpr (KV8) v *= ks[j];
+              if constexpr (CAP) v = c2 * ap_tanh(v);
+              s[n][q4 * 4 + j] = v;
+            }
+          }
+      }
+      if (edge) {
+#pragma unroll
+        for (int n = 0; n < NS; n++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            const int t = t0 + n * 32 + (r >> 2) * 8 + hh * 4 + (r & 3);
+            const bool bad = (t > qpos) | (t >= k_hi) |
+                             ((a.window > 0) & (t <= qpos - a.window));
+            s[n][r] = bad ? -INFINITY : s[n][r];
+          }
+      }
       float mx = -INFINITY;
 #pragma unroll
-      for (int n = 0; n < NS; n++) {
+      for (int n = 0; n < NS; n++)
 #pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-          f4v ks = {1.f, 1.f, 1.f, 1.f};
-          if constexpr (KV8)
-            ks = *(const f4v*)(&Sc[cur][0][n * 32 + q4 * 8 + hh * 4]);
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            float v = s[n][q4 * 4 + j] * c1;
-            if constexpr (KV8) v *= ks[j];
-            if constexpr (CAP) v = c2 * ap_tanh(v);
-            if (edge) {
-              const int t = t0 + n * 32 + q4 * 8 + hh * 4 + j;
-              if (t > qpos || t >= k_hi ||
-                  (a.window > 0 && t <= qpos - a.window))
-                v = -INFINITY;
-            }
-            s[n][q4 * 4 + j] = v;
-            mx = fmaxf(mx, v);
-          }
-        }
-      }
+        for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[n][r]);
+      if constexpr (RAW) mx *= c1;
       mx = fmaxf(mx, __shfl_xor(mx, 32));
       const float mn = fmaxf(m, mx);
       const float mu = mn == -INFINITY ? 0.f : mn;
@@ -276,14 +301,15 @@ k_attn_rows(ApArgs a) {
           float p[8];
 #pragma unroll
           for (int j = 0; j < 8; j++) {
-            p[j] = __builtin_amdgcn_exp2f(s[n][sl * 8 + j] - mu);
+            p[j] = __builtin_amdgcn_exp2f(
+                RAW ? fmaf(s[n][sl * 8 + j], c1, -mu) : s[n][sl * 8 + j] - mu);
             l += p[j];
           }
           if constexpr (KV8) {
 #pragma unroll
             for (int h = 0; h < 2; h++) {
               const f4v vs = *(const f4v*)(
-                  &Sc[cur][1][n * 32 + sl * 16 + h * 8 + hh * 4]);
+                  &Sc[1][n * 32 + sl * 16 + h * 8 + hh * 4]);
 #pragma unroll
               for (int j = 0; j < 4; j++) p[h * 4 + j] *= vs[j];
             }
@@ -296,29 +322,32 @@ k_attn_rows(ApArgs a) {
           }
           // V^T: dims 32d + col, keys as above; a lane of the read points
           // at 4 dims of key (lane/4)%4 of its 16-lane group's tile
-          const int vrow = n * 32 + sl * 16 + hh * 4 + ((lane & 15) >> 2);
-          const int vcol = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
 #pragma unroll
           for (int d = 0; d < HD / 32; d++) {
-            const int dim = d * 32 + vcol;
             union { ap_s4 h[2]; ap_b8 v; } vf;
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-              const int r = vrow + h * 8;
+            for (int h = 0; h < 2; h++)
               vf.h[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                   (__attribute__((address_space(3))) ap_s4*)(
-                      &Vs[cur][r * RB + v_slot<HD>(r, dim >> 3) * 16 +
-                               (dim & 7) * 2]));
-            }
+                      Vs + vb[d % VD] + d / VD * 256 +
+                      (n * 32 + sl * 16 + h * 8) * RB));
             o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf.v, o[d],
                                                            0, 0, 0);
           }
         }
       }
     }
-    if constexpr (KV8) { if (more) store8(cur ^ 1); }
+    if constexpr (KV8) { if (more) store8(Kn, Vn, Sn); }
     __syncthreads();
-    cur ^= 1;
+  };
+  if (k_lo < k_hi) {
+    if constexpr (KV8) { load8(k_lo); store8(K0, V0, S0); }
+    else stage16(K0, V0, k_lo);
+  }
+  __syncthreads();
+  for (int t0 = k_lo; t0 < k_hi; t0 += 2 * BKV) {
+    tile(K0, V0, S0, K1, V1, S1, t0);
+    if (t0 + BKV < k_hi) tile(K1, V1, S1, K0, V0, S0, t0 + BKV);
   }
 
   l += __shfl_xor(l, 32);
