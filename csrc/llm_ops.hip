@@ -1500,371 +1500,6 @@ k_attn_t(const u16* __restrict__ q, const void* __restrict__ kc,
   }
 }
 
-// ====================================================================
-// Fused decode attention (M=1): RoPE(q,k) + KV-pool write + online-
-// softmax GQA, split over the KV range.  grid = (nh, SPLIT): each block
-// scans one chunk of history; partial (m, l, acc) results are combined
-// by the LAST-arriving block of each head via the agent-scope
-// release/acquire + ticket recipe (guide §6 G16) — placement-independent
-// and graph-replay-safe (the merger resets its head's counter).
-// The SPLIT-1 chunk also handles the current token from registers and
-// one block per kv-head persists the new k/v to the pool.
-// Gemma-2 semantics included: sliding window + attn-logit softcap.
-// ====================================================================
-
-template <bool KV8>
-__global__ void __launch_bounds__(256)
-k_attn_dec_t(const u16* __restrict__ qkv, void* __restrict__ kc,
-             void* __restrict__ vc, u16* __restrict__ out,
-             const int* __restrict__ len_ptr, const float* __restrict__ cost,
-             const float* __restrict__ sint, float* __restrict__ kS,
-             float* __restrict__ vS, float* __restrict__ scratch,
-             int* __restrict__ cnt, int nh, int kvh, int hd, int S,
-             float scale, float softcap, int window) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  float* red = (float*)smem;              // [4][hd] + [4][2] + flag
-  int* lastflag = (int*)(red + 4 * hd + 8);
-
-  const int h = blockIdx.x;
-  const int chunk = blockIdx.y, SPLIT = gridDim.y;
-  // batch axis (lockstep sequences): per-b qkv/out rows, KV pool,
-  // scales, merge scratch and tickets; the position is shared
-  const int b = blockIdx.z;
-  qkv += (size_t)b * (nh + 2 * kvh) * hd;
-  out += (size_t)b * nh * hd;
-  kc = (char*)kc + (size_t)b * kvh * S * hd * (KV8 ? 1 : 2);
-  vc = (char*)vc + (size_t)b * kvh * S * hd * (KV8 ? 1 : 2);
-  if (KV8) { kS += (size_t)b * kvh * S; vS += (size_t)b * kvh * S; }
-  scratch += (size_t)b * nh * SPLIT * (hd + 2);
-  cnt += b * nh;
-  const int grp = nh / kvh;
-  const int kvhead = h / grp;
-  // RAGGED batch: each sequence row sits at its own position
-  // (len_ptr is a per-row array; the single-sequence path passes its
-  // scalar length buffer and reads index 0)
-  const int pos = len_ptr[b];
-  int start = 0;
-  if (window > 0 && pos + 1 - window > 0) start = pos + 1 - window;
-  // history chunk [c0, c1) of [start, pos)
-  const int hist = pos - start;
-  const int clen = (hist + SPLIT - 1) / SPLIT;
-  const int c0 = start + chunk * clen;
-  const int c1 = min(c0 + clen, pos);
-  const bool last_chunk = (chunk == SPLIT - 1);
-
-  const int LP = hd / 8;
-  const int PP = 64 / LP;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int p = lane / LP, d0 = (lane % LP) * 8;
-  const int hd2 = hd / 2;
-  const float* cp = cost + (size_t)pos * hd2;
-  const float* sp = sint + (size_t)pos * hd2;
-
-  const u16* qh = qkv + (size_t)h * hd;
-  const u16* kh = qkv + (size_t)(nh + kvhead) * hd;
-  const u16* vh = qkv + (size_t)(nh + kvh + kvhead) * hd;
-  float qf[8], kn[8], vn[8];
-  {
-    const bool lo = d0 < hd2;
-    const int dp = lo ? d0 + hd2 : d0 - hd2;
-    const int ci = lo ? d0 : d0 - hd2;
-    s8v qa = *(const s8v*)(qh + d0);
-    s8v qb = *(const s8v*)(qh + dp);
-    s8v ka = *(const s8v*)(kh + d0);
-    s8v kb = *(const s8v*)(kh + dp);
-    s8v va = *(const s8v*)(vh + d0);
-    f4v c0v = *(const f4v*)(cp + ci);
-    f4v c1v = *(const f4v*)(cp + ci + 4);
-    f4v s0v = *(const f4v*)(sp + ci);
-    f4v s1v = *(const f4v*)(sp + ci + 4);
-    const float sgn = lo ? -1.f : 1.f;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      float c = j < 4 ? c0v[j] : c1v[j - 4];
-      float s = j < 4 ? s0v[j] : s1v[j - 4];
-      qf[j] = b2f(((u16*)&qa)[j]) * c + sgn * b2f(((u16*)&qb)[j]) * s;
-      kn[j] = b2f(((u16*)&ka)[j]) * c + sgn * b2f(((u16*)&kb)[j]) * s;
-      vn[j] = b2f(((u16*)&va)[j]);
-    }
-  }
-  const u16* K0 = (const u16*)kc + (size_t)kvhead * S * hd;
-  const u16* V0 = (const u16*)vc + (size_t)kvhead * S * hd;
-  const uint8_t* K08 = (const uint8_t*)kc + (size_t)kvhead * S * hd;
-  const uint8_t* V08 = (const uint8_t*)vc + (size_t)kvhead * S * hd;
-  const float* kS0 = KV8 ? kS + (size_t)kvhead * S : nullptr;
-  const float* vS0 = KV8 ? vS + (size_t)kvhead * S : nullptr;
-
-  if (last_chunk && h == kvhead * grp && wave == 0 && p == 0) {
-    if (KV8) {
-      // per-(head,pos) absmax across the LP lanes (each holds 8 dims)
-      float kam = 0.f, vam = 0.f;
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        kam = fmaxf(kam, fabsf(kn[j]));
-        vam = fmaxf(vam, fabsf(vn[j]));
-      }
-      for (int w = 1; w < LP; w <<= 1) {
-        kam = fmaxf(kam, __shfl_xor(kam, w));
-        vam = fmaxf(vam, __shfl_xor(vam, w));
-      }
-      float ksc = fmaxf(kam, 1e-8f) / 448.0f;
-      float vsc = fmaxf(vam, 1e-8f) / 448.0f;
-      *(unsigned long long*)((uint8_t*)kc +
-          ((size_t)kvhead * S + pos) * hd + d0) = f32x8_to_fp8(kn, 1.f / ksc);
-      *(unsigned long long*)((uint8_t*)vc +
-          ((size_t)kvhead * S + pos) * hd + d0) = f32x8_to_fp8(vn, 1.f / vsc);
-      if (lane == 0) {
-        kS[(size_t)kvhead * S + pos] = ksc;
-        vS[(size_t)kvhead * S + pos] = vsc;
-      }
-    } else {
-      u16 ko[8], vo[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++) { ko[j] = f2b(kn[j]); vo[j] = f2b(vn[j]); }
-      *(s8v*)((u16*)kc + ((size_t)kvhead * S + pos) * hd + d0) = *(s8v*)ko;
-      *(s8v*)((u16*)vc + ((size_t)kvhead * S + pos) * hd + d0) = *(s8v*)vo;
-    }
-  }
-
-  float mrun = -INFINITY, lrun = 0.f, acc[8];
-#pragma unroll
-  for (int j = 0; j < 8; j++) acc[j] = 0.f;
-
-  // software-pipelined history scan: K[i+1]/V[i+1] issue while the
-  // score/online-update of iteration i computes (the serial
-  // K->dot->softmax->V chain was the latency bottleneck at small T)
-  {
-    int t0 = c0 + wave * PP;
-    if (t0 < c1) {
-      // 2-AHEAD software pipeline: K/V for iterations i+1 and i+2 are
-      // in flight while iteration i computes (the serial
-      // K->dot->softmax->V chain is the latency bound at small T)
-      auto ldkv = [&](int tt, bool& vld, s8v& ko, s8v& vo,
-                      unsigned long long& kro, unsigned long long& vro,
-                      float& kso, float& vso) {
-        vld = false;
-        if (tt < c1) {
-          int t_ = tt + p;
-          vld = t_ < c1;
-          int tl_ = vld ? t_ : c0;
-          if (KV8) {
-            kro = *(const unsigned long long*)(K08 + (size_t)tl_ * hd + d0);
-            vro = *(const unsigned long long*)(V08 + (size_t)tl_ * hd + d0);
-            kso = kS0[tl_]; vso = vS0[tl_];
-          } else {
-            ko = *(const s8v*)(K0 + (size_t)tl_ * hd + d0);
-            vo = *(const s8v*)(V0 + (size_t)tl_ * hd + d0);
-          }
-        }
-      };
-      s8v kv{}, vv{}, kvn{}, vvn{};
-      unsigned long long kraw = 0, vraw = 0, krawn = 0, vrawn = 0;
-      float ksc = 1.f, vsc = 1.f, kscn = 1.f, vscn = 1.f;
-      bool valid, validn;
-      ldkv(t0, valid, kv, vv, kraw, vraw, ksc, vsc);
-      ldkv(t0 + 4 * PP, validn, kvn, vvn, krawn, vrawn, kscn, vscn);
-      for (; t0 < c1; t0 += 4 * PP) {
-        s8v kv2{}, vv2{};
-        unsigned long long kraw2 = 0, vraw2 = 0;
-        float ksc2 = 1.f, vsc2 = 1.f;
-        bool valid2;
-        ldkv(t0 + 8 * PP, valid2, kv2, vv2, kraw2, vraw2, ksc2, vsc2);
-        float partial = 0.f;
-        if (KV8) {
-          // dequant straight to f32 in the dot (4 cvt + 8 fma per 8
-          // elems — cheaper than the bf16 path's 8 shifts + 8 fma)
-          f2v c0_ = __builtin_amdgcn_cvt_pk_f32_fp8((uint32_t)kraw, false);
-          f2v c1_ = __builtin_amdgcn_cvt_pk_f32_fp8((uint32_t)kraw, true);
-          f2v c2_ = __builtin_amdgcn_cvt_pk_f32_fp8((uint32_t)(kraw >> 32),
-                                                    false);
-          f2v c3_ = __builtin_amdgcn_cvt_pk_f32_fp8((uint32_t)(kraw >> 32),
-                                                    true);
-          partial = qf[0] * c0_[0] + qf[1] * c0_[1] + qf[2] * c1_[0] +
-                    qf[3] * c1_[1] + qf[4] * c2_[0] + qf[5] * c2_[1] +
-                    qf[6] * c3_[0] + qf[7] * c3_[1];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; j++) partial += qf[j] * b2f(((u16*)&kv)[j]);
-        }
-        for (int w = 1; w < LP; w <<= 1) partial += __shfl_xor(partial, w);
-        float score = partial * (KV8 ? ksc : 1.f) * scale;
-        if (softcap > 0.f) score = softcap * tanhf(score / softcap);
-        if (!valid) score = -INFINITY;
-        float mnew = fmaxf(mrun, score);
-        float alpha = (mnew == -INFINITY) ? 0.f : __expf(mrun - mnew);
-        float pv = (mnew == -INFINITY) ? 0.f : __expf(score - mnew);
-        lrun = lrun * alpha + pv;
-        if (KV8) {
-          float pvv = pv * vsc;
-          f2v d0_ = __builtin_amdgcn_cvt_pk_f32_fp8((uint32_t)vraw, false);
-          f2v d1_ = __builtin_amdgcn_cvt_pk_f32_fp8((uint32_t)vraw, true);
-          f2v d2_ = __builtin_amdgcn_cvt_pk_f32_fp8((uint32_t)(vraw >> 32),
-                                                    false);
-          f2v d3_ = __builtin_amdgcn_cvt_pk_f32_fp8((uint32_t)(vraw >> 32),
-                                                    true);
-          float vf[8] = {d0_[0], d0_[1], d1_[0], d1_[1],
-                         d2_[0], d2_[1], d3_[0], d3_[1]};
-#pragma unroll
-          for (int j = 0; j < 8; j++)
-            acc[j] = acc[j] * alpha + pvv * vf[j];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; j++)
-            acc[j] = acc[j] * alpha + pv * b2f(((u16*)&vv)[j]);
-        }
-        if (mnew != -INFINITY) mrun = mnew;
-        kv = kvn; vv = vvn; kraw = krawn; vraw = vrawn;
-        valid = validn; ksc = kscn; vsc = vscn;
-        kvn = kv2; vvn = vv2; krawn = kraw2; vrawn = vraw2;
-        validn = valid2; kscn = ksc2; vscn = vsc2;
-      }
-    }
-  }
-
-  // current position from registers (last chunk, p == 0 lanes of wave 0)
-  if (last_chunk && wave == 0 && p == 0) {
-    float partial = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; j++) partial += qf[j] * kn[j];
-    for (int w = 1; w < LP; w <<= 1) partial += __shfl_xor(partial, w);
-    float score = partial * scale;
-    if (softcap > 0.f) score = softcap * tanhf(score / softcap);
-    float mnew = fmaxf(mrun, score);
-    float alpha = __expf(mrun - mnew);
-    float pv = __expf(score - mnew);
-    lrun = lrun * alpha + pv;
-#pragma unroll
-    for (int j = 0; j < 8; j++) acc[j] = acc[j] * alpha + pv * vn[j];
-    mrun = mnew;
-  }
-
-  // merge position-groups within the wave
-  for (int w = LP; w < 64; w <<= 1) {
-    float mo = __shfl_xor(mrun, w);
-    float lo2 = __shfl_xor(lrun, w);
-    float mn = fmaxf(mrun, mo);
-    float sa = (mrun == -INFINITY && mo == -INFINITY) ? 0.f : __expf(mrun - mn);
-    float sb = (mrun == -INFINITY && mo == -INFINITY) ? 0.f : __expf(mo - mn);
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      float ao = __shfl_xor(acc[j], w);
-      acc[j] = acc[j] * sa + ao * sb;
-    }
-    lrun = lrun * sa + lo2 * sb;
-    mrun = mn;
-  }
-
-  // merge the 4 waves via LDS -> block partial in red[0..hd)+m,l
-  float* accs = red;
-  float* mls = red + 4 * hd;
-  if (lane < LP) {
-#pragma unroll
-    for (int j = 0; j < 8; j++) accs[wave * hd + d0 + j] = acc[j];
-  }
-  if (lane == 0) {
-    mls[wave * 2] = mrun;
-    mls[wave * 2 + 1] = lrun;
-  }
-  __syncthreads();
-
-  float* part = scratch + ((size_t)h * SPLIT + chunk) * (hd + 2);
-  if (wave == 0) {
-    float mt = fmaxf(fmaxf(mls[0], mls[2]), fmaxf(mls[4], mls[6]));
-    float lt = 0.f, sc[4];
-#pragma unroll
-    for (int w = 0; w < 4; w++) {
-      sc[w] = (mls[w * 2] == -INFINITY) ? 0.f : __expf(mls[w * 2] - mt);
-      lt += mls[w * 2 + 1] * sc[w];
-    }
-    if (SPLIT == 1) {
-      // single chunk: normalize in registers and write out directly
-      float inv = 1.f / lt;
-      for (int d = lane; d < hd; d += 64) {
-        float v = 0.f;
-#pragma unroll
-        for (int w = 0; w < 4; w++) v += accs[w * hd + d] * sc[w];
-        out[(size_t)h * hd + d] = f2b(v * inv);
-      }
-    } else {
-      for (int d = lane; d < hd; d += 64) {
-        float v = 0.f;
-#pragma unroll
-        for (int w = 0; w < 4; w++) v += accs[w * hd + d] * sc[w];
-        part[2 + d] = v;  // UNnormalized chunk acc at max mt, sum lt
-      }
-      if (lane == 0) { part[0] = mt; part[1] = lt; }
-    }
-  }
-  if (SPLIT == 1) return;
-
-  // publish + ticket (G16 R1: plain stores -> per-wave drain -> barrier
-  // -> one-lane agent release -> asm drain -> relaxed ticket)
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    int t = __hip_atomic_fetch_add(&cnt[h], 1, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-    *lastflag = (t == SPLIT - 1);
-  }
-  __syncthreads();
-  if (!*lastflag) return;
-
-  // last arriver of this head: acquire, merge all chunk partials
-  if (threadIdx.x == 0)
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  __syncthreads();
-  if (wave == 0) {
-    const float* base = scratch + (size_t)h * SPLIT * (hd + 2);
-    float mt = -INFINITY;
-    for (int c = 0; c < SPLIT; c++)
-      mt = fmaxf(mt, base[(size_t)c * (hd + 2)]);
-    float lt = 0.f;
-    for (int c = 0; c < SPLIT; c++) {
-      float mc = base[(size_t)c * (hd + 2)];
-      if (mc != -INFINITY)
-        lt += base[(size_t)c * (hd + 2) + 1] * __expf(mc - mt);
-    }
-    float inv = 1.f / lt;
-    for (int d = lane; d < hd; d += 64) {
-      float v = 0.f;
-      for (int c = 0; c < SPLIT; c++) {
-        float mc = base[(size_t)c * (hd + 2)];
-        if (mc != -INFINITY)
-          v += base[(size_t)c * (hd + 2) + 2 + d] * __expf(mc - mt);
-      }
-      out[(size_t)h * hd + d] = f2b(v * inv);
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) cnt[h] = 0;  // re-arm for the next graph replay
-}
-
-extern "C" hipError_t launch_attn_dec(const void* qkv, void* kc, void* vc,
-                                      void* out, const void* len_ptr,
-                                      const void* cost, const void* sint,
-                                      void* kS, void* vS, int kv8,
-                                      void* scratch, void* cnt, int split,
-                                      int batch,
-                                      int nh, int kvh, int hd, int S,
-                                      float scale, float softcap, int window,
-                                      hipStream_t stream) {
-  size_t lds = (4 * hd + 8) * sizeof(float) + 16;
-#define ATTN_DEC_CASE(KV8V)                                                  \
-  hipLaunchKernelGGL((k_attn_dec_t<KV8V>), dim3(nh, split, batch),          \
-                     dim3(256), lds,                                        \
-                     stream, (const u16*)qkv, kc, vc, (u16*)out,            \
-                     (const int*)len_ptr, (const float*)cost,               \
-                     (const float*)sint, (float*)kS, (float*)vS,            \
-                     (float*)scratch, (int*)cnt, nh, kvh, hd, S, scale,     \
-                     softcap, window)
-  if (kv8) ATTN_DEC_CASE(true);
-  else ATTN_DEC_CASE(false);
-#undef ATTN_DEC_CASE
-  return hipGetLastError();
-}
-
 extern "C" hipError_t launch_attn(const void* q, const void* kc,
                                   const void* vc, void* out,
                                   const void* len_ptr, const void* kS,

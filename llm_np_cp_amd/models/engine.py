@@ -368,10 +368,10 @@ class GPUModel(DecodeLoop):
         # split-T decode attention scratch (partials + per-head tickets)
         import os as _os
         _sp = _os.environ.get("LLM_ATTN_SPLIT")
-        # measured (fp8 llama-1b): T~100 split2 1493 > split4 1483;
-        # T~4k split8 1108 > split16 1050; T~8k split16 963 > split32
+        # ranges of the history that a step may take: the kernel takes one
+        # for some 256 keys, up to so many
         self.attn_split = (int(_sp) if _sp else
-                           min(16, max(2, self.max_seq // 512)))
+                           min(64, max(1, -(-self.max_seq // 256))))
         self.attn_scratch = torch.zeros(
             self.nh_l * self.attn_split * (hd + 2), dtype=torch.float32,
             device=dev)
@@ -401,8 +401,11 @@ class GPUModel(DecodeLoop):
             self.bt_gmax = torch.zeros(B, **i64)
             self.bt_pick = torch.zeros(B, **i64)
             self.bt_cnt = torch.zeros(B, **i32)
+            # a group fills the chip with fewer
+            self.bt_split = min(self.attn_split,
+                                max(1, 2048 // (B * self.kvh_l)))
             self.bt_scratch = torch.zeros(
-                B * self.nh_l * self.attn_split * (hd + 2),
+                B * self.nh_l * self.bt_split * (hd + 2),
                 dtype=torch.float32, device=dev)
             self.bt_attn_cnt = torch.zeros(B * self.nh_l, **i32)
             # fused multi-x path scratch (fp8, B<=8)
@@ -595,7 +598,7 @@ class GPUModel(DecodeLoop):
                             self.sin_t, self.bt_scratch, self.bt_attn_cnt,
                             self.nh_l, self.kvh_l, self.hd, self.scale,
                             softcap=self.attn_softcap, window=window or 0,
-                            split=self.attn_split, kS=self.k_scale[i],
+                            split=self.bt_split, kS=self.k_scale[i],
                             vS=self.v_scale[i], batch=M)
             else:
                 ho.rope_cache(q, k, v, self._kc(i),
@@ -1103,7 +1106,7 @@ class GPUModel(DecodeLoop):
                         self.bt_scratch, self.bt_attn_cnt,
                         self.nh_l, self.kvh_l, self.hd, self.scale,
                         softcap=self.attn_softcap, window=window or 0,
-                        split=self.attn_split, kS=self.k_scale[i],
+                        split=self.bt_split, kS=self.k_scale[i],
                         vS=self.v_scale[i], batch=B)
             if self.gemma:
                 ho.gemv_fp8_mx(lw["wo_q"], lw["wo_s"], self.b_att, t1, B,

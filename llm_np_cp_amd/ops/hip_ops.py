@@ -274,11 +274,11 @@ def attn_dec(qkv: torch.Tensor, k_cache: torch.Tensor,
              scale: float, softcap: float = 0.0, window: int = 0,
              split: int = 1, kS: torch.Tensor | None = None,
              vS: torch.Tensor | None = None, batch: int = 1):
-    """Fused decode attention: RoPE(q,k) + KV write + online softmax,
-    KV range split over `split` blocks/head (last-arriver merge).
-    kS/vS given => fp8 KV pool (quantized write + dequant scan).
-    batch>1: grid.z = lockstep sequence rows (per-b qkv/out rows, KV
-    pools, scratch and tickets; shared device position)."""
+    """Fused decode attention: RoPE(q,k) + KV write + online softmax, the
+    history in up to `split` ranges (as many as the device finds worth it;
+    last-arriver merge).  kS/vS given => fp8 KV pool (quantized write +
+    dequant scan).  batch>1: lockstep sequence rows, each with its own
+    position, KV pool, scratch and tickets."""
     S = k_cache.shape[-2]
     _check(lib().launch_attn_dec(
         _ptr(qkv), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(len_ptr),

@@ -162,3 +162,62 @@ def test_many_rows(M, N, K, kind, act):
     # exact products, fp32 sums, bf16 results: 2^-9 at most
     assert off(Y[:M], z) < 2.0 ** -9
     assert (Y[M] == 7.0).all() and not cnt.any()
+
+
+# histories of nothing, one key, a part of a tile, a block's range and one
+# key more, ranges of several tiles; heads that fill no group of four; a
+# window; head dims of both kernels
+@pytest.mark.parametrize("hd,nh,kvh", [(16, 4, 2), (64, 3, 3), (64, 10, 2),
+                                       (128, 8, 1), (256, 4, 2), (512, 2, 1)])
+@pytest.mark.parametrize("pos", [0, 1, 33, 257, 1500])
+@pytest.mark.parametrize("kv8", [False, True])
+def test_new_tokens(hd, nh, kvh, pos, kv8):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    B, S = 2, pos + 9
+    at = [pos, pos // 2]
+    qkv = normal(B, (nh + 2 * kvh) * hd, seed=1)
+    pools = [normal(B, kvh, S, hd, seed=2 + i) for i in range(2)]
+    true, sc = [x.double() for x in pools], [None, None]
+    if kv8:
+        for i, x in enumerate(pools):
+            q, s, t = e4m3(x.reshape(-1, hd))
+            pools[i] = q.view(torch.uint8).view(x.shape).contiguous()
+            sc[i], true[i] = s.view(B, kvh, S).contiguous(), t.view(x.shape)
+    t = torch.arange(S, device="cuda").double()[:, None] * (
+        1e4 ** -(torch.arange(hd // 2, device="cuda") * 2.0 / hd).double())
+    cos, sin = t.cos().float(), t.sin().float()
+    ln = torch.tensor(at, dtype=torch.int32, device="cuda")
+    for split, win, cap in ((1, 0, 0.0), (5, 0, 30.0), (80, 40, 0.0)):
+        part = torch.zeros(B * nh * split * (hd + 2), device="cuda")
+        cnt = torch.zeros(B * nh, dtype=torch.int32, device="cuda")
+        out = torch.full((B + 1, nh * hd), 7.0, device="cuda").bfloat16()
+        for _ in range(2):                          # counters are left zero
+            ho.attn_dec(qkv, pools[0], pools[1], out, ln, cos, sin, part, cnt,
+                        nh, kvh, hd, hd ** -0.5, softcap=cap, window=win,
+                        split=split, kS=sc[0], vS=sc[1], batch=B)
+        for b, p in enumerate(at):
+            x = qkv[b].double().view(-1, hd)
+            c, s, h = cos[p].double(), sin[p].double(), hd // 2
+            x[:nh + kvh] = torch.cat(
+                [x[:nh + kvh, :h] * c - x[:nh + kvh, h:] * s,
+                 x[:nh + kvh, h:] * c + x[:nh + kvh, :h] * s], -1)
+            lo = max(0, p + 1 - win) if win else 0
+            k, v = (torch.cat([true[i][b, :, lo:p],
+                               x[nh + i * kvh:nh + (i + 1) * kvh, None]], 1)
+                    .repeat_interleave(nh // kvh, 0) for i in range(2))
+            z = (k * x[:nh, None]).sum(-1) * hd ** -0.5
+            if cap:
+                z = cap * torch.tanh(z / cap)
+            y = (torch.softmax(z, -1)[..., None] * v).sum(1).reshape(-1)
+            # fp32 all the way; the bf16 result has 8 bits: half a unit of
+            # the last is at most 2^-8 of each value (2^-9 over many of them,
+            # but there are as few as 64)
+            assert off(out[b], y) < 2.0 ** -8
+            for i in range(2):                      # the pool's new row
+                row, want = pools[i][b, :, p], x[nh + i * kvh:][:kvh]
+                if kv8:
+                    row = row.view(torch.float8_e4m3fn).double() \
+                        * sc[i][b, :, p, None].double()
+                assert off(row, want) < (2.0 ** -4 if kv8 else 2.0 ** -8)
+        assert (out[B] == 7.0).all() and not cnt.any()
