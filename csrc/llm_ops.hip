@@ -31,33 +31,8 @@
 #include <cstdlib>
 
 #include "common.h"
+#include "gemv.h"
 
-// ====================================================================
-// GEMV: y[N] = W[N,K] @ stage(x)[K]  (+ res)  (optional softcap, f32 out)
-// W bf16 row-major; one wave per output row; the input vector is staged
-// once into LDS with an optional fused pre-op (this is where the decode
-// path's RMSNorm and GLU live — they cost an LDS pass, not a kernel):
-//   stage 0 (RAW):  xs = x1
-//   stage 1 (NORM): xs = rmsnorm(x1) * g     (g fp32, Gemma +1 prefolded)
-//   stage 2 (GLU):  xs = act(x1) * x2        (act 0 = SiLU, 1 = tanh-GELU)
-// Decode is bound by streaming W once: target ~HBM roofline.
-// ====================================================================
-
-#define GEMV_ROWS_PER_BLOCK 4
-#define STAGE_RAW 0
-#define STAGE_NORM 1
-#define STAGE_GLU 2
-// NORM2 (Gemma sandwich fusion): h' = h + rmsnorm(x)*g  (post-norm +
-// residual), block 0 persists h' to global, then xs = rmsnorm(h')*g2
-// (pre-norm of the projection this GEMV computes).  Removes the two
-// standalone k_rmsnorm launches per Gemma layer.
-#define STAGE_NORM2 3
-// NORM_EMBED: like NORM but x = embedding TABLE base; the row is
-// gathered at *tok (device token id) and scaled by escale first —
-// fuses the k_embed launch into the first QKV GEMV of the decode step.
-#define STAGE_NORM_EMBED 4
-
-// staging helper shared by bf16/fp8 GEMV (RMSNorm / GLU fused pre-ops)
 DEVINL float stage_red_sum(float* red) {
   const int nw = blockDim.x >> 6;
   float t = 0.f;
@@ -65,252 +40,11 @@ DEVINL float stage_red_sum(float* red) {
   return t;
 }
 
-DEVINL const u16* gemv_stage(char* smem, const u16* x, const u16* x2,
-                             const float* g, const float* g2, u16* hout,
-                             int K, int stage, int act, float eps,
-                             float escale) {
-  u16* xs = (u16*)smem;
-  const int STRIDE = blockDim.x * 8;
-  if (stage == STAGE_NORM2) {
-    // x2 = h_in (read-only here); block 0 persists h' into hout — a
-    // DIFFERENT buffer (ping-pong), since other blocks still read h_in
-    const u16* h = x2;
-    float* red = (float*)(smem + (size_t)K * 2);
-    // pass 1: sumsq of x (the un-normed projection output t)
-    float ss = 0.f;
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v v = *(const s8v*)(x + i);
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        float f = b2f(((u16*)&v)[j]);
-        ss += f * f;
-      }
-    }
-    ss = wave_reduce_sum(ss);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    float rnorm_a = rsqrtf(stage_red_sum(red) / (float)K + eps);
-    __syncthreads();
-    // pass 2: h' = h + norm_a(x)*g (bf16-rounded, matching the
-    // standalone k_rmsnorm mode 1), stash h' in LDS, sumsq of h'
-    float ss2 = 0.f;
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v v = *(const s8v*)(x + i);
-      s8v hv = *(const s8v*)(h + i);
-      f4v ga = *(const f4v*)(g + i);
-      f4v gb = *(const f4v*)(g + i + 4);
-      u16 o[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        float f = b2f(((u16*)&v)[j]) * rnorm_a * (j < 4 ? ga[j] : gb[j - 4])
-                  + b2f(((u16*)&hv)[j]);
-        o[j] = f2b(f);
-        float fr = b2f(o[j]);
-        ss2 += fr * fr;
-      }
-      *(s8v*)(xs + i) = *(s8v*)o;
-      if (blockIdx.x == 0) *(s8v*)(hout + i) = *(s8v*)o;  // persist h'
-    }
-    ss2 = wave_reduce_sum(ss2);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss2;
-    __syncthreads();
-    float rnorm_b = rsqrtf(stage_red_sum(red) / (float)K + eps);
-    // pass 3: xs = norm_b(h')*g2
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v v = *(s8v*)(xs + i);
-      f4v ga = *(const f4v*)(g2 + i);
-      f4v gb = *(const f4v*)(g2 + i + 4);
-      u16 o[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        o[j] = f2b(b2f(((u16*)&v)[j]) * rnorm_b *
-                   (j < 4 ? ga[j] : gb[j - 4]));
-      *(s8v*)(xs + i) = *(s8v*)o;
-    }
-    __syncthreads();
-    return xs;
-  }
-  if (stage == STAGE_NORM || stage == STAGE_NORM_EMBED) {
-    // NORM_EMBED: x is the embedding TABLE; gather row *x2 (token id),
-    // scale by escale (bf16-rounded, matching the standalone k_embed),
-    // and have block 0 persist it as the residual-stream h
-    const u16* xsrc = x;
-    if (stage == STAGE_NORM_EMBED)
-      xsrc = x + (size_t)(*(const int*)x2) * (size_t)K;
-    float ss = 0.f;
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v v = *(const s8v*)(xsrc + i);
-      if (stage == STAGE_NORM_EMBED) {
-        u16 o[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-          o[j] = f2b(b2f(((u16*)&v)[j]) * escale);
-        v = *(s8v*)o;
-        if (blockIdx.x == 0) *(s8v*)(hout + i) = v;
-      }
-      *(s8v*)(xs + i) = v;
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        float f = b2f(((u16*)&v)[j]);
-        ss += f * f;
-      }
-    }
-    float* red = (float*)(smem + (size_t)K * 2);
-    ss = wave_reduce_sum(ss);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    float rnorm = rsqrtf(stage_red_sum(red) / (float)K + eps);
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v v = *(s8v*)(xs + i);
-      u16 o[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        o[j] = f2b(b2f(((u16*)&v)[j]) * rnorm * g[i + j]);
-      *(s8v*)(xs + i) = *(s8v*)o;
-    }
-  } else if (stage == STAGE_GLU) {
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v gv = *(const s8v*)(x + i);
-      s8v uv = *(const s8v*)(x2 + i);
-      u16 o[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        float xx = b2f(((u16*)&gv)[j]);
-        float a;
-        if (act == 0) {
-          a = xx / (1.f + __expf(-xx));
-        } else {
-          float c = 0.7978845608028654f * (xx + 0.044715f * xx * xx * xx);
-          a = 0.5f * xx * (1.f + tanhf(c));
-        }
-        o[j] = f2b(a * b2f(((u16*)&uv)[j]));
-      }
-      *(s8v*)(xs + i) = *(s8v*)o;
-    }
-  }
-  if (stage != STAGE_RAW) __syncthreads();
-  return (stage == STAGE_RAW) ? x : xs;  // RAW: L2-hot, no barrier
-}
-
-// f32 variant of the staging pass, used by the fp8 GEMV: x lands in LDS
-// as fp32 PAIRS so the inner loop can feed its FMAs directly from
-// the v_cvt_pk_f32_fp8 outputs (the round-1 fp8 stream was
-// conversion-VALU-bound at 4.3 TB/s — this halves the VALU work per
-// weight byte).  Semantics match gemv_stage: the NORM2-persisted h' is
-// still bf16-rounded (it feeds the residual stream), only the staged
-// vector skips the final bf16 round-trip (within GEMV tolerance).
-DEVINL const float* gemv_stage_f32(char* smem, const u16* x, const u16* x2,
-                                   const float* g, const float* g2,
-                                   u16* hout, int K, int stage, int act,
-                                   float eps, float escale) {
-  float* xs = (float*)smem;
-  const int STRIDE = blockDim.x * 8;
-  if (stage == STAGE_RAW) {
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v v = *(const s8v*)(x + i);
-#pragma unroll
-      for (int j = 0; j < 8; j++) xs[i + j] = b2f(((u16*)&v)[j]);
-    }
-    __syncthreads();
-    return xs;
-  }
-  float* red = (float*)(smem + (size_t)K * 4);
-  if (stage == STAGE_NORM2) {
-    const u16* h = x2;
-    float ss = 0.f;
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v v = *(const s8v*)(x + i);
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        float f = b2f(((u16*)&v)[j]);
-        ss += f * f;
-      }
-    }
-    ss = wave_reduce_sum(ss);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    float rnorm_a = rsqrtf(stage_red_sum(red) / (float)K + eps);
-    __syncthreads();
-    float ss2 = 0.f;
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v v = *(const s8v*)(x + i);
-      s8v hv = *(const s8v*)(h + i);
-      f4v ga = *(const f4v*)(g + i);
-      f4v gb = *(const f4v*)(g + i + 4);
-      u16 o[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        float f = b2f(((u16*)&v)[j]) * rnorm_a * (j < 4 ? ga[j] : gb[j - 4])
-                  + b2f(((u16*)&hv)[j]);
-        o[j] = f2b(f);           // bf16-rounded h' (residual stream)
-        float fr = b2f(o[j]);
-        xs[i + j] = fr;
-        ss2 += fr * fr;
-      }
-      if (blockIdx.x == 0) *(s8v*)(hout + i) = *(s8v*)o;
-    }
-    ss2 = wave_reduce_sum(ss2);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss2;
-    __syncthreads();
-    float rnorm_b = rsqrtf(stage_red_sum(red) / (float)K + eps);
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        xs[i + j] = xs[i + j] * rnorm_b * g2[i + j];
-    }
-    __syncthreads();
-    return xs;
-  }
-  if (stage == STAGE_NORM || stage == STAGE_NORM_EMBED) {
-    const u16* xsrc = x;
-    if (stage == STAGE_NORM_EMBED)
-      xsrc = x + (size_t)(*(const int*)x2) * (size_t)K;
-    float ss = 0.f;
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v v = *(const s8v*)(xsrc + i);
-      if (stage == STAGE_NORM_EMBED) {
-        u16 o[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-          o[j] = f2b(b2f(((u16*)&v)[j]) * escale);
-        v = *(s8v*)o;
-        if (blockIdx.x == 0) *(s8v*)(hout + i) = v;
-      }
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        float f = b2f(((u16*)&v)[j]);
-        xs[i + j] = f;
-        ss += f * f;
-      }
-    }
-    ss = wave_reduce_sum(ss);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    float rnorm = rsqrtf(stage_red_sum(red) / (float)K + eps);
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-#pragma unroll
-      for (int j = 0; j < 8; j++) xs[i + j] *= rnorm * g[i + j];
-    }
-  } else if (stage == STAGE_GLU) {
-    for (int i = threadIdx.x * 8; i < K; i += STRIDE) {
-      s8v gv = *(const s8v*)(x + i);
-      s8v uv = *(const s8v*)(x2 + i);
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        float xx = b2f(((u16*)&gv)[j]);
-        float a;
-        if (act == 0) {
-          a = xx / (1.f + __expf(-xx));
-        } else {
-          float c = 0.7978845608028654f * (xx + 0.044715f * xx * xx * xx);
-          a = 0.5f * xx * (1.f + tanhf(c));
-        }
-        xs[i + j] = a * b2f(((u16*)&uv)[j]);
-      }
-    }
-  }
-  __syncthreads();
-  return xs;
+DEVINL void fp4x8_to_f32p(uint32_t dw, float sc, f2v* o) {
+  o[0] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(dw, sc, 0);
+  o[1] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(dw, sc, 1);
+  o[2] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(dw, sc, 2);
+  o[3] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(dw, sc, 3);
 }
 
 DEVINL void gemv_epilogue(float acc, int row, void* y, const u16* res,
@@ -321,349 +55,7 @@ DEVINL void gemv_epilogue(float acc, int row, void* y, const u16* res,
   else ((u16*)y)[row] = f2b(acc);
 }
 
-// NT: non-temporal weight loads (read-once stream, keep L2 for x/KV —
-// MI355X_MICROARCH "nt-weights").  RPW: rows per wave (ILP: RPW x 4
-// weight loads in flight).
-template <bool NT, int RPW>
-__global__ void __launch_bounds__(512)
-k_gemv_bf16_t(const u16* __restrict__ W, const u16* __restrict__ x,
-              const u16* __restrict__ x2, const float* __restrict__ g,
-              const float* __restrict__ g2, void* __restrict__ y,
-              const u16* __restrict__ res, int N, int K, int stage, int act,
-              float eps, int out_f32, float softcap, float escale,
-              const int* __restrict__ eidx, long wstride,
-              const float* __restrict__ oscale) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const u16* xv = gemv_stage(smem, x, x2, g, g2, (u16*)res, K, stage, act,
-                             eps, escale);
-  // MoE: expert-indexed weight base + device output scale (router
-  // prob); scalar loads, uniform branch — free on the dense path
-  if (eidx) W += (size_t)(*eidx) * wstride;
-  const float osc = oscale ? *oscale : 1.0f;
-  // NORM2 / NORM_EMBED borrow `res` as the persisted-h output
-  const u16* eres = (stage == STAGE_NORM2 || stage == STAGE_NORM_EMBED)
-                        ? nullptr : res;
-
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wpb = blockDim.x >> 6;
-  const int rstride = gridDim.x * wpb * RPW;  // grid-stride rows
-  for (int row0 = (blockIdx.x * wpb + wave) * RPW; row0 < N;
-       row0 += rstride) {                    // wave setup over many rows
-  const u16* Wr[RPW];
-  float a0[RPW], a1[RPW], a2[RPW], a3[RPW];
-#pragma unroll
-  for (int r = 0; r < RPW; r++) {
-    int rr = row0 + r < N ? row0 + r : N - 1;
-    Wr[r] = W + (size_t)rr * K;
-    a0[r] = a1[r] = a2[r] = a3[r] = 0.f;
-  }
-  int k = lane * 8;
-  for (; k + 1536 < K; k += 2048) {
-    s8v x0 = *(const s8v*)(xv + k);
-    s8v x1 = *(const s8v*)(xv + k + 512);
-    s8v x2v = *(const s8v*)(xv + k + 1024);
-    s8v x3 = *(const s8v*)(xv + k + 1536);
-#pragma unroll
-    for (int r = 0; r < RPW; r++) {
-      s8v w0, w1, w2, w3;
-      if (NT) {
-        w0 = __builtin_nontemporal_load((const s8v*)(Wr[r] + k));
-        w1 = __builtin_nontemporal_load((const s8v*)(Wr[r] + k + 512));
-        w2 = __builtin_nontemporal_load((const s8v*)(Wr[r] + k + 1024));
-        w3 = __builtin_nontemporal_load((const s8v*)(Wr[r] + k + 1536));
-      } else {
-        w0 = *(const s8v*)(Wr[r] + k);
-        w1 = *(const s8v*)(Wr[r] + k + 512);
-        w2 = *(const s8v*)(Wr[r] + k + 1024);
-        w3 = *(const s8v*)(Wr[r] + k + 1536);
-      }
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        a0[r] += b2f(((u16*)&w0)[j]) * b2f(((u16*)&x0)[j]);
-        a1[r] += b2f(((u16*)&w1)[j]) * b2f(((u16*)&x1)[j]);
-        a2[r] += b2f(((u16*)&w2)[j]) * b2f(((u16*)&x2v)[j]);
-        a3[r] += b2f(((u16*)&w3)[j]) * b2f(((u16*)&x3)[j]);
-      }
-    }
-  }
-  for (; k < K; k += 512) {
-    s8v x0 = *(const s8v*)(xv + k);
-#pragma unroll
-    for (int r = 0; r < RPW; r++) {
-      s8v w0 = NT ? __builtin_nontemporal_load((const s8v*)(Wr[r] + k))
-                  : *(const s8v*)(Wr[r] + k);
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        a0[r] += b2f(((u16*)&w0)[j]) * b2f(((u16*)&x0)[j]);
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < RPW; r++) {
-    float acc = osc * wave_reduce_sum((a0[r] + a1[r]) + (a2[r] + a3[r]));
-    if (lane == 0 && row0 + r < N)
-      gemv_epilogue(acc, row0 + r, y, eres, out_f32, softcap);
-  }
-  }  // row0 grid-stride loop
-}
-
-extern "C" hipError_t launch_gemv_bf16(const void* W, const void* x,
-                                       const void* x2, const void* g,
-                                       const void* g2, void* y,
-                                       const void* res, int N, int K,
-                                       int stage, int act, float eps,
-                                       int out_f32, float softcap,
-                                       int nt, int rpw, int maxblocks,
-                                       float escale, const void* eidx,
-                                       long wstride, const void* oscale,
-                                       hipStream_t stream) {
-  size_t lds = (stage == STAGE_RAW) ? 0 : ((size_t)K * 2 + 32);
-  static int rpw_env_b = -1;
-  if (rpw_env_b < 0) {
-    const char* p = getenv("LLM_GEMV_RPW");
-    rpw_env_b = p ? atoi(p) : 0;
-  }
-  if (rpw_env_b > 0) rpw = rpw_env_b;
-  else if (rpw <= 1)
-    // deep-K only: the fp8 GEMV's large-N rpw rule measured NEGATIVE
-    // for bf16 (1b 1234->1218, gemma-2b 536->526)
-    rpw = (K >= 3584 && N >= 3072) ? 2 : 1;
-  int threads = 256;  // 512 measured slower (fp8 1391->1328)
-  int wpb = threads / 64;
-  int blocks = (N + wpb * rpw - 1) / (wpb * rpw);
-  int cap = maxblocks > 0 ? maxblocks : 1024;
-  if (blocks > cap) blocks = cap;  // grid-stride the rest (Guideline 11)
-#define GEMV_CASE(NTV, RPWV)                                                 \
-  hipLaunchKernelGGL((k_gemv_bf16_t<NTV, RPWV>), dim3(blocks), dim3(threads),\
-                     lds, stream, (const u16*)W, (const u16*)x,              \
-                     (const u16*)x2, (const float*)g, (const float*)g2, y,   \
-                     (const u16*)res, N, K, stage, act, eps, out_f32,        \
-                     softcap, escale, (const int*)eidx, wstride,             \
-                     (const float*)oscale)
-  if (nt && rpw == 2) GEMV_CASE(true, 2);
-  else if (nt) GEMV_CASE(true, 1);
-  else if (rpw == 2) GEMV_CASE(false, 2);
-  else GEMV_CASE(false, 1);
-#undef GEMV_CASE
-  return hipGetLastError();
-}
-
-// ====================================================================
-// fp8 GEMV: y[N] = scale[n] * (W8[N,K] @ stage(x)[K]) (+res) (softcap)
-// W8 = OCP e4m3fn, per-output-row scales (absmax/448 quantization at
-// load).  Halves decode weight traffic vs bf16 -> ~2x decode ceiling.
-// Same fused staging modes as the bf16 GEMV; x stays bf16.
-// HW dequant: v_cvt_pk_f32_fp8 (gfx950, OCP not fnuz).
-// ====================================================================
-
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));  // = u4v_ alias
-
-// Inner loop is PACKED: x is staged as fp32 in LDS (gemv_stage_f32),
-// each v_cvt_pk_f32_fp8 output pair feeds two FMAs against an
-// LDS fp32 pair — ~16 VALU per 16 weight bytes vs ~40 for the round-1
-// scalar form (the fp8 stream was conversion-bound at 4.3 TB/s while
-// bf16 hit 6.4; see profiles/decode_kernels_r01.md).
-template <bool NT, int RPW, bool XDIR>
-__global__ void __launch_bounds__(512)
-k_gemv_fp8_t(const uint8_t* __restrict__ W, const float* __restrict__ scales,
-             const u16* __restrict__ x, const u16* __restrict__ x2,
-             const float* __restrict__ g, const float* __restrict__ g2,
-             void* __restrict__ y, const u16* __restrict__ res, int N, int K,
-             int stage, int act, float eps, int out_f32, float softcap,
-             float escale, const int* __restrict__ eidx, long wstride,
-             long sstride, const float* __restrict__ oscale) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  // XDIR (RAW stage only): x read from global per row iteration — the
-  // f32 LDS staging pass costs ~2K B of LDS+global traffic per BLOCK,
-  // which rivals the weight bytes when a block covers only a few rows
-  // (N~3.5k o/down projections; see profiles/decode_kernels_r02.md)
-  const float* xv = XDIR ? nullptr
-                         : gemv_stage_f32(smem, x, x2, g, g2, (u16*)res, K,
-                                          stage, act, eps, escale);
-  const u16* eres = (stage == STAGE_NORM2 || stage == STAGE_NORM_EMBED)
-                        ? nullptr : res;
-  // MoE: expert-indexed weight/scale base + device output scale
-  if (eidx) {
-    W += (size_t)(*eidx) * wstride;
-    scales += (size_t)(*eidx) * sstride;
-  }
-  const float osc = oscale ? *oscale : 1.0f;
-
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wpb = blockDim.x >> 6;
-  const int rstride = gridDim.x * wpb * RPW;
-  for (int row0 = (blockIdx.x * wpb + wave) * RPW; row0 < N;
-       row0 += rstride) {
-  const uint8_t* Wr[RPW];
-  f2v a0[RPW], a1[RPW];
-#pragma unroll
-  for (int r = 0; r < RPW; r++) {
-    int rr = row0 + r < N ? row0 + r : N - 1;
-    Wr[r] = W + (size_t)rr * K;
-    a0[r] = (f2v){0.f, 0.f};
-    a1[r] = (f2v){0.f, 0.f};
-  }
-  int k = lane * 16;
-  for (; k + 1024 + 16 <= K; k += 2048) {
-    s8v xda, xdb, xdc, xdd;
-    if (XDIR) {
-      xda = *(const s8v*)(x + k); xdb = *(const s8v*)(x + k + 8);
-      xdc = *(const s8v*)(x + k + 1024); xdd = *(const s8v*)(x + k + 1032);
-    }
-#pragma unroll
-    for (int r = 0; r < RPW; r++) {
-      u4v w0 = NT ? __builtin_nontemporal_load((const u4v*)(Wr[r] + k))
-                  : *(const u4v*)(Wr[r] + k);
-      u4v w1 = NT ? __builtin_nontemporal_load((const u4v*)(Wr[r] + k + 1024))
-                  : *(const u4v*)(Wr[r] + k + 1024);
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        f2v ca = __builtin_amdgcn_cvt_pk_f32_fp8(w0[q], false);
-        f2v cb = __builtin_amdgcn_cvt_pk_f32_fp8(w0[q], true);
-        f2v xa, xb, xc, xd;
-        if (XDIR) {
-          const u16* p0 = (q < 2) ? (const u16*)&xda : (const u16*)&xdb;
-          const int o0 = (q & 1) * 4;
-          xa = (f2v){b2f(p0[o0]), b2f(p0[o0 + 1])};
-          xb = (f2v){b2f(p0[o0 + 2]), b2f(p0[o0 + 3])};
-          const u16* p1 = (q < 2) ? (const u16*)&xdc : (const u16*)&xdd;
-          xc = (f2v){b2f(p1[o0]), b2f(p1[o0 + 1])};
-          xd = (f2v){b2f(p1[o0 + 2]), b2f(p1[o0 + 3])};
-        } else {
-          xa = *(const f2v*)(xv + k + q * 4);
-          xb = *(const f2v*)(xv + k + q * 4 + 2);
-          xc = *(const f2v*)(xv + k + 1024 + q * 4);
-          xd = *(const f2v*)(xv + k + 1024 + q * 4 + 2);
-        }
-        a0[r] += ca * xa;
-        a1[r] += cb * xb;
-        f2v da = __builtin_amdgcn_cvt_pk_f32_fp8(w1[q], false);
-        f2v db = __builtin_amdgcn_cvt_pk_f32_fp8(w1[q], true);
-        a0[r] += da * xc;
-        a1[r] += db * xd;
-      }
-    }
-  }
-  for (; k < K; k += 1024) {
-    s8v xda, xdb;
-    if (XDIR) {
-      xda = *(const s8v*)(x + k); xdb = *(const s8v*)(x + k + 8);
-    }
-#pragma unroll
-    for (int r = 0; r < RPW; r++) {
-      u4v w0 = NT ? __builtin_nontemporal_load((const u4v*)(Wr[r] + k))
-                  : *(const u4v*)(Wr[r] + k);
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        f2v ca = __builtin_amdgcn_cvt_pk_f32_fp8(w0[q], false);
-        f2v cb = __builtin_amdgcn_cvt_pk_f32_fp8(w0[q], true);
-        f2v xa, xb;
-        if (XDIR) {
-          const u16* p0 = (q < 2) ? (const u16*)&xda : (const u16*)&xdb;
-          const int o0 = (q & 1) * 4;
-          xa = (f2v){b2f(p0[o0]), b2f(p0[o0 + 1])};
-          xb = (f2v){b2f(p0[o0 + 2]), b2f(p0[o0 + 3])};
-        } else {
-          xa = *(const f2v*)(xv + k + q * 4);
-          xb = *(const f2v*)(xv + k + q * 4 + 2);
-        }
-        a0[r] += ca * xa;
-        a1[r] += cb * xb;
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < RPW; r++) {
-    int rr = row0 + r < N ? row0 + r : N - 1;
-    f2v s = a0[r] + a1[r];
-    float acc = osc * wave_reduce_sum(s[0] + s[1]) * scales[rr];
-    if (lane == 0 && row0 + r < N)
-      gemv_epilogue(acc, row0 + r, y, eres, out_f32, softcap);
-  }
-  }  // row0 grid-stride loop
-}
-
-extern "C" hipError_t launch_gemv_fp8(const void* W, const void* scales,
-                                      const void* x, const void* x2,
-                                      const void* g, const void* g2, void* y,
-                                      const void* res, int N, int K,
-                                      int stage, int act, float eps,
-                                      int out_f32, float softcap, int nt,
-                                      int rpw, int maxblocks, float escale,
-                                      const void* eidx, long wstride,
-                                      long sstride, const void* oscale,
-                                      hipStream_t stream) {
-  static int xdir_raw = -1, rows_min = -1, rpw_env = -1;
-  if (xdir_raw < 0) {
-    const char* e = getenv("LLM_GEMV_XDIR");
-    xdir_raw = e ? atoi(e) : 1;          // default ON for RAW stage
-    const char* r = getenv("LLM_GEMV_ROWSMIN");
-    rows_min = r ? atoi(r) : 1;
-    const char* p = getenv("LLM_GEMV_RPW");
-    rpw_env = p ? atoi(p) : 0;
-  }
-  if (rpw_env > 0) rpw = rpw_env;
-  else if (rpw <= 1)
-    // deep-K rows: 2x loads in flight (gemma-9b 240->300, llama-8b
-    // 393->442, qwen-7b 352->442); N floor keeps small-N shapes (1B
-    // down-proj) at full block count.  Very large N (gate+up, lm_head)
-    // also gains: waves already grid-stride many rows, RPW doubles the
-    // in-flight rows per iteration.
-    rpw = ((K >= 3584 && N >= 3072) || N >= 12288) ? 2 : 1;
-  const int xdir = (stage == STAGE_RAW) && xdir_raw;
-  // fp32 staging for packed math (all non-RAW stages; RAW reads direct)
-  size_t lds = xdir ? 0 : ((size_t)K * 4 + 32);
-  if (lds > 65536) {
-    // gfx950 allows up to 160 KB dynamic LDS with an explicit opt-in
-    // (e.g. Gemma-27B down-proj K=36864)
-    static bool raised = false;
-    if (!raised) {
-#define GEMV8_RAISE(NTV, RPWV)                                              \
-      hipFuncSetAttribute((const void*)&k_gemv_fp8_t<NTV, RPWV, false>,     \
-                          hipFuncAttributeMaxDynamicSharedMemorySize,       \
-                          160 * 1024)
-      GEMV8_RAISE(true, 1); GEMV8_RAISE(true, 2);
-      GEMV8_RAISE(false, 1); GEMV8_RAISE(false, 2);
-#undef GEMV8_RAISE
-      raised = true;
-    }
-  }
-  int threads = 256;  // 512 measured slower (fp8 1391->1328)
-  int wpb = threads / 64;
-  int blocks = (N + wpb * rpw - 1) / (wpb * rpw);
-  int cap = maxblocks > 0 ? maxblocks : 1024;
-  if (rows_min > 1 && !xdir) {
-    // amortize the staging pass over >= rows_min rows per wave
-    int cap2 = N / (wpb * rpw * rows_min);
-    if (cap2 < 64) cap2 = 64;
-    if (cap > cap2) cap = cap2;
-  }
-  if (blocks > cap) blocks = cap;
-#define GEMV8_CASE(NTV, RPWV, XD)                                           \
-  hipLaunchKernelGGL((k_gemv_fp8_t<NTV, RPWV, XD>), dim3(blocks),           \
-                     dim3(threads),                                         \
-                     lds, stream, (const uint8_t*)W, (const float*)scales,  \
-                     (const u16*)x, (const u16*)x2, (const float*)g,        \
-                     (const float*)g2, y, (const u16*)res, N, K, stage,     \
-                     act, eps, out_f32, softcap, escale, (const int*)eidx,  \
-                     wstride, sstride, (const float*)oscale)
-  if (xdir) {
-    if (nt && rpw == 4) GEMV8_CASE(true, 4, true);
-    else if (nt && rpw == 2) GEMV8_CASE(true, 2, true);
-    else if (nt) GEMV8_CASE(true, 1, true);
-    else if (rpw == 4) GEMV8_CASE(false, 4, true);
-    else if (rpw == 2) GEMV8_CASE(false, 2, true);
-    else GEMV8_CASE(false, 1, true);
-  } else {
-    if (nt && rpw == 4) GEMV8_CASE(true, 4, false);
-    else if (nt && rpw == 2) GEMV8_CASE(true, 2, false);
-    else if (nt) GEMV8_CASE(true, 1, false);
-    else if (rpw == 4) GEMV8_CASE(false, 4, false);
-    else if (rpw == 2) GEMV8_CASE(false, 2, false);
-    else GEMV8_CASE(false, 1, false);
-  }
-#undef GEMV8_CASE
-  return hipGetLastError();
-}
 
 // ====================================================================
 // Multi-x fp8 GEMV (batched decode, B = 2..8 lockstep sequences):
@@ -899,206 +291,6 @@ extern "C" hipError_t launch_gemv_fp8_mx(
   else if (BT == 4) { if (xf32) MX_CASE(4, true); else MX_CASE(4, false); }
   else { if (xf32) MX_CASE(8, true); else MX_CASE(8, false); }
 #undef MX_CASE
-  return hipGetLastError();
-}
-
-// ====================================================================
-// MXFP4 GEMV: y[N] = W4[N,K] @ stage(x)[K] (+res); 2 fp4/byte with one
-// e8m0 scale per 32 elements.  Same packed structure as the fp8 GEMV
-// (fp32 x staging or XDIR direct reads feeding fp32 FMAs) — the
-// block scale rides inside v_cvt_scalef32_pk_f32_fp4, so per-ELEMENT
-// VALU matches fp8 at HALF the weight bytes.
-// ====================================================================
-
-typedef uint32_t u2v_ __attribute__((ext_vector_type(2)));
-
-DEVINL void fp4x8_to_f32p(uint32_t dw, float sc, f2v* o) {
-  o[0] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(dw, sc, 0);
-  o[1] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(dw, sc, 1);
-  o[2] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(dw, sc, 2);
-  o[3] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(dw, sc, 3);
-}
-
-template <bool NT, int RPW, bool XDIR>
-__global__ void __launch_bounds__(512)
-k_gemv_fp4_t(const uint8_t* __restrict__ W, const uint8_t* __restrict__ E,
-             const u16* __restrict__ x, const u16* __restrict__ x2,
-             const float* __restrict__ g, const float* __restrict__ g2,
-             void* __restrict__ y, const u16* __restrict__ res, int N, int K,
-             int stage, int act, float eps, int out_f32, float softcap,
-             float escale) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const float* xv = XDIR ? nullptr
-                         : gemv_stage_f32(smem, x, x2, g, g2, (u16*)res, K,
-                                          stage, act, eps, escale);
-  const u16* eres = (stage == STAGE_NORM2 || stage == STAGE_NORM_EMBED)
-                        ? nullptr : res;
-
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wpb = blockDim.x >> 6;
-  const int rstride = gridDim.x * wpb * RPW;
-  const int K2 = K / 2, K32 = K / 32;
-  for (int row0 = (blockIdx.x * wpb + wave) * RPW; row0 < N;
-       row0 += rstride) {
-  const uint8_t* Wr[RPW];
-  const uint8_t* Er[RPW];
-  f2v a0[RPW], a1[RPW];
-#pragma unroll
-  for (int r = 0; r < RPW; r++) {
-    int rr = row0 + r < N ? row0 + r : N - 1;
-    Wr[r] = W + (size_t)rr * K2;
-    Er[r] = E + (size_t)rr * K32;
-    a0[r] = (f2v){0.f, 0.f};
-    a1[r] = (f2v){0.f, 0.f};
-  }
-  int k = lane * 16;
-  for (; k + 1024 + 16 <= K; k += 2048) {
-    s8v xda, xdb, xdc, xdd;
-    if (XDIR) {
-      xda = *(const s8v*)(x + k); xdb = *(const s8v*)(x + k + 8);
-      xdc = *(const s8v*)(x + k + 1024); xdd = *(const s8v*)(x + k + 1032);
-    }
-#pragma unroll
-    for (int r = 0; r < RPW; r++) {
-      u2v_ w0 = NT ? __builtin_nontemporal_load((const u2v_*)(Wr[r] + k / 2))
-                    : *(const u2v_*)(Wr[r] + k / 2);
-      u2v_ w1 = NT ? __builtin_nontemporal_load(
-                          (const u2v_*)(Wr[r] + (k + 1024) / 2))
-                    : *(const u2v_*)(Wr[r] + (k + 1024) / 2);
-      union { float f; uint32_t u; } s0, s1;
-      s0.u = (uint32_t)Er[r][k / 32] << 23;
-      s1.u = (uint32_t)Er[r][(k + 1024) / 32] << 23;
-      f2v c0[8], c1[8];
-      fp4x8_to_f32p(w0[0], s0.f, c0);
-      fp4x8_to_f32p(w0[1], s0.f, c0 + 4);
-      fp4x8_to_f32p(w1[0], s1.f, c1);
-      fp4x8_to_f32p(w1[1], s1.f, c1 + 4);
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        f2v ca = c0[q * 2];
-        f2v cb = c0[q * 2 + 1];
-        f2v xa, xb, xc, xd;
-        if (XDIR) {
-          const u16* p0 = (q < 2) ? (const u16*)&xda : (const u16*)&xdb;
-          const int o0 = (q & 1) * 4;
-          xa = (f2v){b2f(p0[o0]), b2f(p0[o0 + 1])};
-          xb = (f2v){b2f(p0[o0 + 2]), b2f(p0[o0 + 3])};
-          const u16* p1 = (q < 2) ? (const u16*)&xdc : (const u16*)&xdd;
-          xc = (f2v){b2f(p1[o0]), b2f(p1[o0 + 1])};
-          xd = (f2v){b2f(p1[o0 + 2]), b2f(p1[o0 + 3])};
-        } else {
-          xa = *(const f2v*)(xv + k + q * 4);
-          xb = *(const f2v*)(xv + k + q * 4 + 2);
-          xc = *(const f2v*)(xv + k + 1024 + q * 4);
-          xd = *(const f2v*)(xv + k + 1024 + q * 4 + 2);
-        }
-        a0[r] += ca * xa;
-        a1[r] += cb * xb;
-        a0[r] += c1[q * 2] * xc;
-        a1[r] += c1[q * 2 + 1] * xd;
-      }
-    }
-  }
-  for (; k < K; k += 1024) {
-    s8v xda, xdb;
-    if (XDIR) {
-      xda = *(const s8v*)(x + k); xdb = *(const s8v*)(x + k + 8);
-    }
-#pragma unroll
-    for (int r = 0; r < RPW; r++) {
-      u2v_ w0 = NT ? __builtin_nontemporal_load((const u2v_*)(Wr[r] + k / 2))
-                    : *(const u2v_*)(Wr[r] + k / 2);
-      union { float f; uint32_t u; } s0;
-      s0.u = (uint32_t)Er[r][k / 32] << 23;
-      f2v c0[8];
-      fp4x8_to_f32p(w0[0], s0.f, c0);
-      fp4x8_to_f32p(w0[1], s0.f, c0 + 4);
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        f2v ca = c0[q * 2];
-        f2v cb = c0[q * 2 + 1];
-        f2v xa, xb;
-        if (XDIR) {
-          const u16* p0 = (q < 2) ? (const u16*)&xda : (const u16*)&xdb;
-          const int o0 = (q & 1) * 4;
-          xa = (f2v){b2f(p0[o0]), b2f(p0[o0 + 1])};
-          xb = (f2v){b2f(p0[o0 + 2]), b2f(p0[o0 + 3])};
-        } else {
-          xa = *(const f2v*)(xv + k + q * 4);
-          xb = *(const f2v*)(xv + k + q * 4 + 2);
-        }
-        a0[r] += ca * xa;
-        a1[r] += cb * xb;
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < RPW; r++) {
-    f2v s = a0[r] + a1[r];
-    float acc = wave_reduce_sum(s[0] + s[1]);
-    if (lane == 0 && row0 + r < N)
-      gemv_epilogue(acc, row0 + r, y, eres, out_f32, softcap);
-  }
-  }  // row0 grid-stride loop
-}
-
-extern "C" hipError_t launch_gemv_fp4(const void* W, const void* E,
-                                      const void* x, const void* x2,
-                                      const void* g, const void* g2, void* y,
-                                      const void* res, int N, int K,
-                                      int stage, int act, float eps,
-                                      int out_f32, float softcap, int nt,
-                                      int rpw, int maxblocks, float escale,
-                                      hipStream_t stream) {
-  if (K % 32 != 0) return hipErrorInvalidValue;
-  static int xdir_raw4 = -1, rpw_env4 = -1;
-  if (xdir_raw4 < 0) {
-    const char* e = getenv("LLM_GEMV_XDIR");
-    xdir_raw4 = e ? atoi(e) : 1;
-    const char* p = getenv("LLM_GEMV_RPW");
-    rpw_env4 = p ? atoi(p) : 0;
-  }
-  if (rpw_env4 > 0) rpw = rpw_env4;
-  else if (rpw <= 1)
-    rpw = (K >= 3584 && N >= 3072) ? 2 : 1;  // same policy as fp8
-  const int xdir = (stage == STAGE_RAW) && xdir_raw4;
-  size_t lds = xdir ? 0 : ((size_t)K * 4 + 32);
-  if (lds > 65536) {
-    static bool raised4 = false;
-    if (!raised4) {
-#define GEMV4_RAISE(NTV, RPWV, XDV)                                         \
-      hipFuncSetAttribute((const void*)&k_gemv_fp4_t<NTV, RPWV, XDV>,       \
-                          hipFuncAttributeMaxDynamicSharedMemorySize,       \
-                          160 * 1024)
-      GEMV4_RAISE(true, 1, false); GEMV4_RAISE(true, 2, false);
-      GEMV4_RAISE(false, 1, false); GEMV4_RAISE(false, 2, false);
-#undef GEMV4_RAISE
-      raised4 = true;
-    }
-  }
-  int threads = 256;
-  int wpb = threads / 64;
-  int blocks = (N + wpb * rpw - 1) / (wpb * rpw);
-  int cap = maxblocks > 0 ? maxblocks : 1024;
-  if (blocks > cap) blocks = cap;
-#define GEMV4_CASE(NTV, RPWV, XD)                                           \
-  hipLaunchKernelGGL((k_gemv_fp4_t<NTV, RPWV, XD>), dim3(blocks),           \
-                     dim3(threads), lds, stream, (const uint8_t*)W,         \
-                     (const uint8_t*)E, (const u16*)x, (const u16*)x2,      \
-                     (const float*)g, (const float*)g2, y, (const u16*)res, \
-                     N, K, stage, act, eps, out_f32, softcap, escale)
-  if (xdir) {
-    if (nt && rpw == 2) GEMV4_CASE(true, 2, true);
-    else if (nt) GEMV4_CASE(true, 1, true);
-    else if (rpw == 2) GEMV4_CASE(false, 2, true);
-    else GEMV4_CASE(false, 1, true);
-  } else {
-    if (nt && rpw == 2) GEMV4_CASE(true, 2, false);
-    else if (nt) GEMV4_CASE(true, 1, false);
-    else if (rpw == 2) GEMV4_CASE(false, 2, false);
-    else GEMV4_CASE(false, 1, false);
-  }
-#undef GEMV4_CASE
   return hipGetLastError();
 }
 

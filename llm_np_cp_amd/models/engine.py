@@ -364,7 +364,11 @@ class GPUModel(DecodeLoop):
                                          device=dev)
         self.b_hb = torch.zeros(H, **bf)   # gemma residual ping-pong
         self.b_t2 = torch.zeros(H, **bf)   # gemma ffn-out delta
-        self.b_gu = torch.zeros(2 * I, **bf)
+        # act(gate) * up of a decode step (of each expert): fp32 beside
+        # weights that are multiplied in fp32
+        self.b_act = torch.zeros(
+            self.topk if self.moe else 1, I, device=dev,
+            dtype=torch.float32 if self.fp8 else torch.bfloat16)
         # split-T decode attention scratch (partials + per-head tickets)
         import os as _os
         _sp = _os.environ.get("LLM_ATTN_SPLIT")
@@ -454,9 +458,7 @@ class GPUModel(DecodeLoop):
                 ho.gemv_fp8(w, s, x, y, res=res if bias is None else bias,
                             softcap=softcap)
                 return
-            n = w.shape[0] // 2
-            ho.gemv_fp8(w, s, x, self.b_gu)
-            ho.glu(self.b_gu[:n], self.b_gu[n:], y[:1], act)
+            ho.gemv_fp8(w, s, x, y[0], act=act, glu=True)
             return
         if g is not None and x.shape[-1] > ho.ROW_NORM_K:
             ho.rmsnorm(x[:M], g, self.b_xn[:M], eps=eps)
@@ -946,13 +948,11 @@ class GPUModel(DecodeLoop):
                 tpu.all_reduce(t1)
                 # NORM2: h' = h + norm(t1)*g_post (persisted to hnext),
                 # stage = norm(h')*g_preffn — both sandwich norms fused
-                self._dgemv(lw, "wgu", t1, self.b_gu, stage=ho.STAGE_NORM2,
+                self._dgemv(lw, "wgu", t1, self.b_act, stage=ho.STAGE_NORM2,
                             x2=h, g=lw["g_post"], g2=lw["g_preffn"],
-                            res=hnext, eps=eps)
+                            res=hnext, eps=eps, glu=True, act=self.act)
                 h, hnext = hnext, h
-                self._dgemv(lw, "wdown", self.b_gu[:self.inter_l], t2,
-                            stage=ho.STAGE_GLU, x2=self.b_gu[self.inter_l:],
-                            act=self.act)
+                self._dgemv(lw, "wdown", self.b_act, t2)
                 tpu.all_reduce(t2)
             else:
                 if self.tp_branch:
@@ -962,49 +962,35 @@ class GPUModel(DecodeLoop):
                 else:
                     self._dgemv(lw, "wo", self.b_att[0], h, res=h)
                 if self.moe:
-                    # router -> topk expert-indexed GEMV pairs: W base
-                    # offset by the device idx, output scaled by the
-                    # device router prob, accumulated into h via res.
-                    # xn is staged ONCE: expert 0's down-proj already
-                    # updates h, so expert 1 must not re-norm it
+                    # router -> both products of all topk experts at once:
+                    # W by the device's idx, the second one's results
+                    # weighted by the device's router probs into h
                     ho.moe_route(h, lw["g_post"], lw["wg"], 1, self.topk,
                                  self.moe_idx, self.moe_w, eps=eps)
-                    xn0 = self.b_xn[0]
-                    ho.rmsnorm(h, lw["g_post"], xn0, eps=eps)
                     I, H = self.inter_l, self.H
-                    for j in range(self.topk):
-                        ei = self.moe_idx[j:j + 1]
-                        osc = self.moe_w[j:j + 1]
-                        if self.fp8:
-                            ho.gemv_fp8(lw["wgu_q"], lw["wgu_s"], xn0,
-                                        self.b_gu, eidx=ei,
-                                        wstride=2 * I * H, sstride=2 * I)
-                            ho.gemv_fp8(lw["wdown_q"], lw["wdown_s"],
-                                        self.b_gu[:I], h, res=h,
-                                        stage=ho.STAGE_GLU,
-                                        x2=self.b_gu[I:], act=self.act,
-                                        eidx=ei, wstride=H * I,
-                                        sstride=H, oscale=osc)
-                        else:
-                            ho.gemv(lw["wgu"], xn0, self.b_gu, eidx=ei,
-                                    wstride=2 * I * H)
-                            ho.gemv(lw["wdown"], self.b_gu[:I], h, res=h,
-                                    stage=ho.STAGE_GLU, x2=self.b_gu[I:],
-                                    act=self.act, eidx=ei,
-                                    wstride=H * I, oscale=osc)
+                    ei = self.moe_idx[:self.topk]
+                    up = dict(stage=ho.STAGE_NORM, g=lw["g_post"], eps=eps,
+                              glu=True, act=self.act, eidx=ei,
+                              wstride=2 * I * H)
+                    dn = dict(res=h, eidx=ei, wstride=H * I,
+                              oscale=self.moe_w)
+                    if self.fp8:
+                        ho.gemv_fp8(lw["wgu_q"], lw["wgu_s"], h, self.b_act,
+                                    sstride=2 * I, **up)
+                        ho.gemv_fp8(lw["wdown_q"], lw["wdown_s"], self.b_act,
+                                    h, sstride=H, **dn)
+                    else:
+                        ho.gemv(lw["wgu"], h, self.b_act, **up)
+                        ho.gemv(lw["wdown"], self.b_act, h, **dn)
                     continue
-                self._dgemv(lw, "wgu", h, self.b_gu, stage=ho.STAGE_NORM,
-                            g=lw["g_post"], eps=eps)
+                self._dgemv(lw, "wgu", h, self.b_act, stage=ho.STAGE_NORM,
+                            g=lw["g_post"], eps=eps, glu=True, act=self.act)
                 if self.tp_branch:
-                    self._dgemv(lw, "wdown", self.b_gu[:self.inter_l], t1,
-                                stage=ho.STAGE_GLU,
-                                x2=self.b_gu[self.inter_l:], act=self.act)
+                    self._dgemv(lw, "wdown", self.b_act, t1)
                     tpu.all_reduce(t1)
                     ho.addinto(h, t1)
                 else:
-                    self._dgemv(lw, "wdown", self.b_gu[:self.inter_l], h,
-                                res=h, stage=ho.STAGE_GLU,
-                                x2=self.b_gu[self.inter_l:], act=self.act)
+                    self._dgemv(lw, "wdown", self.b_act, h, res=h)
         if pf:
             ev = torch.cuda.Event()
             ev.record(self._pf_stream)

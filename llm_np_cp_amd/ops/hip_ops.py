@@ -24,16 +24,10 @@ _LIB_PATH = os.path.join(os.path.dirname(os.path.dirname(
     os.path.abspath(__file__))), "_libllmops.so")
 
 _SIGS = {
-    "launch_gemv_bf16": [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 +
-                        [ctypes.c_float, ctypes.c_int, ctypes.c_float,
-                         ctypes.c_int, ctypes.c_int, ctypes.c_int,
-                         ctypes.c_float, ctypes.c_void_p, ctypes.c_long,
-                         ctypes.c_void_p, ctypes.c_void_p],
-    "launch_gemv_fp8": [ctypes.c_void_p] * 8 + [ctypes.c_int] * 4 +
-                       [ctypes.c_float, ctypes.c_int, ctypes.c_float,
-                        ctypes.c_int, ctypes.c_int, ctypes.c_int,
-                        ctypes.c_float, ctypes.c_void_p, ctypes.c_long,
-                        ctypes.c_long, ctypes.c_void_p, ctypes.c_void_p],
+    "launch_gemv": [ctypes.c_void_p] * 9 + [ctypes.c_int] * 8 +
+                   [ctypes.c_float] * 3 +
+                   [ctypes.c_int, ctypes.c_void_p, ctypes.c_int] +
+                   [ctypes.c_long] * 2 + [ctypes.c_void_p] * 2,
     "launch_rmsnorm": [ctypes.c_void_p] * 4 + [ctypes.c_int] * 2 +
                       [ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
     "launch_rope_cache": [ctypes.c_void_p] * 7 + [ctypes.c_int] +
@@ -77,10 +71,6 @@ _SIGS = {
                         [ctypes.c_void_p],
     "launch_quant_fp4": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 2 +
                         [ctypes.c_void_p],
-    "launch_gemv_fp4": [ctypes.c_void_p] * 8 + [ctypes.c_int] * 4 +
-                       [ctypes.c_float, ctypes.c_int, ctypes.c_float,
-                        ctypes.c_int, ctypes.c_int, ctypes.c_int,
-                        ctypes.c_float, ctypes.c_void_p],
     "launch_gemv_fp8_mx": [ctypes.c_void_p] * 3 + [ctypes.c_long] +
                           [ctypes.c_void_p, ctypes.c_long] +
                           [ctypes.c_void_p] * 3 + [ctypes.c_long] +
@@ -157,6 +147,19 @@ STAGE_RAW, STAGE_NORM, STAGE_GLU, STAGE_NORM2 = 0, 1, 2, 3
 STAGE_NORM_EMBED = 4
 
 
+def _gemv(wt, W, ws, we, K, x, y, res, softcap, stage, x2, g, act, eps,
+          maxblocks, g2, escale, eidx, wstride, sstride, oscale, glu):
+    _check(lib().launch_gemv(
+        _ptr(W), _ptr(ws), _ptr(we), _ptr(x), _ptr(x2), _ptr(g), _ptr(g2),
+        _ptr(y), _ptr(res), wt, W.shape[0] // (2 if glu else 1), K, stage,
+        act, int(glu), int(x.dtype == torch.float32),
+        int(y.dtype == torch.float32), ctypes.c_float(eps),
+        ctypes.c_float(softcap), ctypes.c_float(escale), maxblocks,
+        _ptr(eidx), 1 if eidx is None else eidx.numel(),
+        ctypes.c_long(wstride), ctypes.c_long(sstride), _ptr(oscale),
+        _stream()), "gemv")
+
+
 def gemv(W: torch.Tensor, x: torch.Tensor, y: torch.Tensor,
          res: torch.Tensor | None = None, softcap: float = 0.0,
          stage: int = 0, x2: torch.Tensor | None = None,
@@ -164,20 +167,18 @@ def gemv(W: torch.Tensor, x: torch.Tensor, y: torch.Tensor,
          nt: int = 1, rpw: int = 1, maxblocks: int = 0,
          g2: torch.Tensor | None = None, escale: float = 1.0,
          eidx: torch.Tensor | None = None, wstride: int = 0,
-         oscale: torch.Tensor | None = None):
-    """y[N] = W[N,K] @ stage(x)[K] (+res); stage fuses RMSNorm / GLU /
+         oscale: torch.Tensor | None = None, glu: bool = False):
+    """y[N] = W[N,K] @ stage(x)[K] (+res); stage takes RMSNorm / GLU /
     the Gemma sandwich (NORM2: x2 = h_in, g/g2 = post/pre gammas, res =
     h_out ping-pong) / the embed gather (NORM_EMBED: x = embed table,
-    x2 = token-id i32, res = persisted h) into the LDS staging pass;
-    nt = non-temporal W."""
-    N, K = W.shape
-    out_f32 = 1 if y.dtype == torch.float32 else 0
-    _check(lib().launch_gemv_bf16(
-        _ptr(W), _ptr(x), _ptr(x2), _ptr(g), _ptr(g2), _ptr(y), _ptr(res),
-        N, K, stage, act, ctypes.c_float(eps), out_f32,
-        ctypes.c_float(softcap), nt, rpw, maxblocks,
-        ctypes.c_float(escale), _ptr(eidx), ctypes.c_long(wstride),
-        _ptr(oscale), _stream()), "gemv")
+    x2 = token-id i32, res = persisted h) on the way.  x is bf16, or fp32
+    (RAW).  glu: W holds gate rows, then up rows: y[N/2] = act(gate) * up.
+    eidx/wstride/oscale: W of expert *eidx, its result times *oscale; of
+    several experts the results are added up (x [n, K]), with glu they stand
+    one after the other.  nt and rpw are kept for callers: the kernel streams
+    W past the caches and picks its rows by itself."""
+    _gemv(0, W, None, None, W.shape[1], x, y, res, softcap, stage, x2, g,
+          act, eps, maxblocks, g2, escale, eidx, wstride, 0, oscale, glu)
 
 
 def gemv_fp8(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
@@ -188,18 +189,12 @@ def gemv_fp8(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
              maxblocks: int = 0, g2: torch.Tensor | None = None,
              escale: float = 1.0, eidx: torch.Tensor | None = None,
              wstride: int = 0, sstride: int = 0,
-             oscale: torch.Tensor | None = None):
-    """y[N] = scales * (Wq[N,K] @ stage(x)); Wq = e4m3fn bytes.
-    eidx/wstride/sstride/oscale: MoE expert indexing — W and scales
-    offset by the device int32 *eidx, output scaled by *oscale."""
-    N, K = Wq.shape
-    out_f32 = 1 if y.dtype == torch.float32 else 0
-    _check(lib().launch_gemv_fp8(
-        _ptr(Wq), _ptr(scales), _ptr(x), _ptr(x2), _ptr(g), _ptr(g2),
-        _ptr(y), _ptr(res), N, K, stage, act, ctypes.c_float(eps), out_f32,
-        ctypes.c_float(softcap), nt, rpw, maxblocks,
-        ctypes.c_float(escale), _ptr(eidx), ctypes.c_long(wstride),
-        ctypes.c_long(sstride), _ptr(oscale), _stream()), "gemv_fp8")
+             oscale: torch.Tensor | None = None, glu: bool = False):
+    """y[N] = scales * (Wq[N,K] @ stage(x)); Wq = e4m3fn bytes; the rest
+    as for gemv (sstride: scales of an expert)."""
+    _gemv(1, Wq, scales, None, Wq.shape[1], x, y, res, softcap, stage, x2, g,
+          act, eps, maxblocks, g2, escale, eidx, wstride, sstride, oscale,
+          glu)
 
 
 def rmsnorm(x: torch.Tensor, g: torch.Tensor, y: torch.Tensor,
@@ -434,17 +429,12 @@ def gemv_fp4(Wq: torch.Tensor, We: torch.Tensor, x: torch.Tensor,
              x2: torch.Tensor | None = None, g: torch.Tensor | None = None,
              act: int = 0, eps: float = 1e-5, nt: int = 1, rpw: int = 1,
              maxblocks: int = 0, g2: torch.Tensor | None = None,
-             escale: float = 1.0):
+             escale: float = 1.0, glu: bool = False):
     """y[N] = W4[N,K] @ stage(x): MXFP4 weights (Wq: N x K/2 packed
-    bytes, We: N x K/32 e8m0 scale bytes) — half the fp8 stream."""
-    N = Wq.shape[0]
-    K = Wq.shape[1] * 2
-    out_f32 = 1 if y.dtype == torch.float32 else 0
-    _check(lib().launch_gemv_fp4(
-        _ptr(Wq), _ptr(We), _ptr(x), _ptr(x2), _ptr(g), _ptr(g2),
-        _ptr(y), _ptr(res), N, K, stage, act, ctypes.c_float(eps), out_f32,
-        ctypes.c_float(softcap), nt, rpw, maxblocks,
-        ctypes.c_float(escale), _stream()), "gemv_fp4")
+    bytes, We: N x K/32 e8m0 scale bytes) — half the fp8 stream; the rest
+    as for gemv."""
+    _gemv(2, Wq, None, We, Wq.shape[1] * 2, x, y, res, softcap, stage, x2, g,
+          act, eps, maxblocks, g2, escale, None, 0, 0, None, glu)
 
 
 def gemm_fp8(xq: torch.Tensor, sx: torch.Tensor, Wq: torch.Tensor,

@@ -221,3 +221,106 @@ def test_new_tokens(hd, nh, kvh, pos, kv8):
                         * sc[i][b, :, p, None].double()
                 assert off(row, want) < (2.0 ** -4 if kv8 else 2.0 ** -8)
         assert (out[B] == 7.0).all() and not cnt.any()
+
+
+# K: less than a load of the lanes, one and a rest, several waves with a rest,
+# more loads than a wave takes, more than one pass; rows: fewer than waves,
+# odd, more than a block's threads; what x may be on the way
+@pytest.mark.parametrize("N,K", [(5, 64), (300, 544), (517, 3584),
+                                 (33, 11008), (40, 41984), (140000, 96)])
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "fp4"])
+@pytest.mark.parametrize("glu", [False, True])
+def test_one_row(N, K, kind, glu):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    W = normal(N * (2 if glu else 1), K, seed=4, scale=K ** -0.5)
+    x, u = normal(K, seed=5), normal(K, seed=6)
+    g, g2 = (normal(K, seed=s).float() for s in (7, 8))
+    res, table = normal(N, seed=9), normal(3, K, seed=10)
+    tok = torch.tensor([2], dtype=torch.int32, device="cuda")
+    w, f, Wd = [W], ho.gemv, W.double()
+    if kind == "fp8":
+        q, s, Wd = e4m3(W)
+        w, f = [q, s], ho.gemv_fp8
+    if kind == "fp4":
+        q = torch.empty(W.shape[0], K // 2, dtype=torch.uint8, device="cuda")
+        e = torch.empty(W.shape[0], K // 32, dtype=torch.uint8, device="cuda")
+        ho.quant_fp4(W, q, e)
+        w, f, Wd = [q, e], ho.gemv_fp4, mxfp4_values(q, e)
+
+    def rms(t):
+        return t * torch.rsqrt(t.pow(2).mean() + 1e-5)
+
+    xd, ud, hd = x.double(), u.double(), (table[2].double() * 1.5)
+    h2 = (ud + rms(xd) * g.double()).bfloat16()
+    hd = hd.bfloat16()
+    keep = torch.full((K + 1,), 7.0, device="cuda").bfloat16()
+    ways = [(dict(x=x, res=res), xd, None)]
+    if kind != "bf16":
+        ways.append((dict(x=x.float() * 1.001, res=res),
+                     (x.float() * 1.001).double(), None))
+    if K < 32768:
+        ways += [
+            (dict(x=x, stage=ho.STAGE_NORM, g=g, res=res),
+             rms(xd) * g.double(), None),
+            (dict(x=x, stage=ho.STAGE_GLU, x2=u, act=1, res=res),
+             torch.nn.functional.gelu(xd, approximate="tanh") * ud, None),
+            (dict(x=x, stage=ho.STAGE_NORM2, x2=u, g=g, g2=g2, res=keep),
+             rms(h2.double()) * g2.double(), h2),
+            (dict(x=table, stage=ho.STAGE_NORM_EMBED, x2=tok, g=g,
+                  escale=1.5, res=keep), rms(hd.double()) * g.double(), hd)]
+    for kw, ref, kept in ways:
+        y = torch.full((N + 1,), 7.0, device="cuda")
+        if glu:
+            kw["act"] = 1
+        f(*w, kw.pop("x"), y[:N], glu=glu, softcap=20.0, **kw)
+        z = Wd @ ref
+        if glu:
+            z = torch.nn.functional.gelu(z[:N], approximate="tanh") * z[N:]
+        z = 20.0 * torch.tanh(z / 20.0)
+        if kept is None:
+            z = z + res.double()
+        else:       # the residual stream, rounded after fp32 sums
+            assert off(keep[:K], kept.double()) < 2.0 ** -9
+            assert keep[K] == 7.0
+        # fp32 all the way; bf16 weights meet x rounded to bf16 (2^-8 of each
+        # at most, twice through a gate), a kept row may round the other way
+        assert off(y[:N], z) < (2.0 ** -7 if kind == "bf16" or kept is not None
+                                else 2.0 ** -18)
+        assert y[N] == 7.0
+
+
+# experts of a step at once: apart through the gate, added up after it
+@pytest.mark.parametrize("n", [1, 2, 3, 8])
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+def test_experts_of_one_row(n, kind):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    E, I, H = 9, 208, 144
+    up, dn = (normal(E * r, k, seed=s, scale=k ** -0.5)
+              for r, k, s in ((2 * I, H, 1), (H, I, 2)))
+    x, res, g = normal(H, seed=3), normal(H, seed=4), normal(H, seed=5).float()
+    idx = torch.randperm(E, generator=torch.Generator().manual_seed(n))[:n]
+    idx = idx.int().cuda()
+    p = torch.rand(n, generator=torch.Generator().manual_seed(6)).cuda()
+    f, ups, dns, U, D = ho.gemv, [up], [dn], up.double(), dn.double()
+    if kind == "fp8":
+        (a, b, U), (c, d, D), f = e4m3(up), e4m3(dn), ho.gemv_fp8
+        ups, dns = [a, b], [c, d]
+    ups, dns = ([t[:r] for t in ts] for ts, r in ((ups, 2 * I), (dns, H)))
+    kw, kd = (dict(sstride=s) if kind == "fp8" else {} for s in (2 * I, H))
+    a = torch.full((n + 1, I), 7.0, device="cuda")
+    if kind == "bf16":
+        a = a.bfloat16()
+    f(*ups, x, a[:n], stage=ho.STAGE_NORM, g=g, glu=True, eidx=idx,
+      wstride=2 * I * H, **kw)
+    y = res.clone()
+    f(*dns, a[:n], y, res=y, eidx=idx, wstride=H * I, oscale=p, **kd)
+    xn = x.double() * torch.rsqrt(x.double().pow(2).mean() + 1e-5) * g.double()
+    z = res.double()
+    for j, e in enumerate(idx.tolist()):
+        t = U[e * 2 * I:(e + 1) * 2 * I] @ xn
+        t = torch.nn.functional.silu(t[:I]) * t[I:]
+        assert off(a[j], t) < (2.0 ** -7 if kind == "bf16" else 2.0 ** -18)
+        z = z + p[j].double() * (D[e * H:(e + 1) * H] @ t)
+    assert off(y, z) < 2.0 ** -7 and (a[n] == 7.0).all()
