@@ -22,7 +22,8 @@
 //          152064x3584 82.7 -> 54 (5.4 TB/s)
 // Of the small ones 2 us are the launch, 1 the first loads, 0.7 to 2 the work
 // on x and on the last rows; MXFP4 is bound by widening (13 us of 37888x3584
-// without its loads).#include "common.h"
+// without its loads).
+#include "common.h"
 #include "gemv.h"
 
 typedef float gv_f4 __attribute__((ext_vector_type(4), aligned(4)));
