@@ -1,8 +1,8 @@
 // gemm_prompt.hip — linears of many rows: Y[M,N] = X[M,K] W[N,K]^T, bf16 or
 // e4m3 with row scales, fp32 sums, bf16 out.
 //
-// Slabs of 128 bytes a row (64 bf16, 128 e4m3) go straight into LDS, two or
-// three buffers, one barrier a slab that waits for the next slab only and
+// Slabs of 128 bytes a row (64 bf16, 128 e4m3) go straight into LDS, two to
+// six buffers, one barrier a slab that waits for the next slab only and
 // leaves the DMA behind it in flight.  That wait is what bounds these
 // products (a slab is back from L2 or memory after one to two microseconds,
 // the matrix cores want one a microsecond): with every DMA drained at each
@@ -10,8 +10,8 @@
 // 128x256 tiles and three buffers it runs at 1160 and 2180.
 //
 // Rows are XOR-swizzled by 16-byte slots; the DMA writes lane-linear, so the
-// swizzle sits in the address that a lane reads and in the fragment reads.  The order of k inside a slab is free as
-// long as X and W agree: a lane's two slots are two bf16 operands or one
+// swizzle sits in the address that a lane reads and in the fragment reads.
+// The order of k inside a slab is free as long as X and W agree: a lane's two slots are two bf16 operands or one
 // e4m3 operand of the 128-deep MFMA.  W is the first operand, so a lane
 // ends with four neighbouring outputs of one row and stores them at once.
 //
@@ -70,10 +70,13 @@ k_gemm_prompt(GpArgs a) {
   // that a DMA into one does not touch what is read from another, and puts
   // no wait for it before the reads.
   constexpr int ZA = BM * 128, ZB = BN * 128;
-  __shared__ __attribute__((aligned(16))) char A0[ZA], A1[ZA];
-  __shared__ __attribute__((aligned(16))) char B0[ZB], B1[ZB];
-  __shared__ __attribute__((aligned(16))) char A2[NS > 2 ? ZA : 16],
-      B2[NS > 2 ? ZB : 16];
+#define GP_BUF(i)                                                            \
+  __shared__ __attribute__((aligned(16))) char A##i[NS > i ? ZA : 16],       \
+      B##i[NS > i ? ZB : 16];
+  GP_BUF(0) GP_BUF(1) GP_BUF(2) GP_BUF(3) GP_BUF(4) GP_BUF(5)
+#undef GP_BUF
+  char* const A[6] = {A0, A1, A2, A3, A4, A5};
+  char* const B[6] = {B0, B1, B2, B3, B4, B5};
   __shared__ int last_flag;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -149,9 +152,9 @@ k_gemm_prompt(GpArgs a) {
   // conditions while there are slabs to ask for; the last few wait for all.
   int s = s_lo;
   if (s_lo < s_hi) {
-    stage(A0, B0, s_lo);
-    if (s_lo + 1 < s_hi) stage(A1, B1, s_lo + 1);
-    if (NS > 2 && s_lo + 2 < s_hi) stage(A2, B2, s_lo + 2);
+#pragma unroll
+    for (int u = 0; u < NS; u++)
+      if (s_lo + u < s_hi) stage(A[u], B[u], s_lo + u);
     // all but the first may still be in flight
     if (s_lo + NS <= s_hi) gp_meet<PS * (NS - 1)>();
     else gp_meet<0>();
@@ -201,14 +204,13 @@ k_gemm_prompt(GpArgs a) {
         }
       };
       for (; s + 2 * NS <= s_hi; s += NS) {
-        slab(A0, B0, s, true);
-        slab(A1, B1, s + 1, true);
-        if (NS > 2) slab(A2, B2, s + 2, true);
+#pragma unroll
+        for (int u = 0; u < NS; u++) slab(A[u], B[u], s + u, true);
       }
       for (; s < s_hi; s += NS) {
-        slab(A0, B0, s, false);
-        if (s + 1 < s_hi) slab(A1, B1, s + 1, false);
-        if (NS > 2 && s + 2 < s_hi) slab(A2, B2, s + 2, false);
+#pragma unroll
+        for (int u = 0; u < NS; u++)
+          if (s + u < s_hi) slab(A[u], B[u], s + u, false);
       }
     } else {
       // Half a slab of fragments ahead: the hand-over stands between two
@@ -251,17 +253,17 @@ k_gemm_prompt(GpArgs a) {
         }
         mma(1);
       };
-      fetch(0, A0, B0);
+      fetch(0, A[0], B[0]);
       for (; s + 2 * NS <= s_hi; s += NS) {
-        slab(A0, B0, A1, B1, s, true);
-        slab(A1, B1, NS > 2 ? A2 : A0, NS > 2 ? B2 : B0, s + 1, true);
-        if (NS > 2) slab(A2, B2, A0, B0, s + 2, true);
+#pragma unroll
+        for (int u = 0; u < NS; u++)
+          slab(A[u], B[u], A[(u + 1) % NS], B[(u + 1) % NS], s + u, true);
       }
       for (; s < s_hi; s += NS) {
-        slab(A0, B0, A1, B1, s, false);
-        if (s + 1 < s_hi)
-          slab(A1, B1, NS > 2 ? A2 : A0, NS > 2 ? B2 : B0, s + 1, false);
-        if (NS > 2 && s + 2 < s_hi) slab(A2, B2, A0, B0, s + 2, false);
+#pragma unroll
+        for (int u = 0; u < NS; u++)
+          if (s + u < s_hi)
+            slab(A[u], B[u], A[(u + 1) % NS], B[(u + 1) % NS], s + u, false);
       }
     }
   }
@@ -291,16 +293,29 @@ k_gemm_prompt(GpArgs a) {
       a.cnt[tile] = 0;                                  // for the next launch
     }
     __syncthreads();
+    // up to 16 fragments of a part on the way at a time: a part a trip, not
+    // a fragment of one
+    constexpr int G = FM * FN > 16 ? 16 / FN : FM;
 #pragma unroll
-    for (int i = 0; i < FM; i++)
+    for (int i0 = 0; i0 < FM; i0 += G) {
 #pragma unroll
-      for (int j = 0; j < FN; j++) {
-        f4v v = {0.f, 0.f, 0.f, 0.f};
-        for (int q = 0; q < SK; q++)
-          v += *(const f4v*)(pp + (size_t)q * (BM * BN) +
-                             (i * FN + j) * (NW * 256));
-        acc[i][j] = v;
+      for (int i = 0; i < G; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) acc[i0 + i][j] = {0.f, 0.f, 0.f, 0.f};
+      for (int q = 0; q < SK; q++) {
+        f4v t[G][FN];
+#pragma unroll
+        for (int i = 0; i < G; i++)
+#pragma unroll
+          for (int j = 0; j < FN; j++)
+            t[i][j] = *(const f4v*)(pp + (size_t)q * (BM * BN) +
+                                    ((i0 + i) * FN + j) * (NW * 256));
+#pragma unroll
+        for (int i = 0; i < G; i++)
+#pragma unroll
+          for (int j = 0; j < FN; j++) acc[i0 + i][j] += t[i][j];
       }
+    }
   }
 
   // fragment (i, j): row i*16 + fr, outputs j*16 + fk*4 + 0..3
@@ -373,17 +388,24 @@ static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
 }
 
 // Tile sizes, and microseconds that a slab takes on a CU that runs one block
-// of them or as many as fit (measured, bf16; e4m3 slabs move the same bytes
-// and differ by a tenth).  The big tiles win where there are rounds of them,
-// the small ones where a part-filled last round would cost more.
+// of them or as many as fit (measured with a full chip, bf16; e4m3 slabs move
+// the same bytes and differ by a tenth).  Large tiles ask L2 for the fewest
+// bytes a product: 128x128 by four waves wants 64 bytes a clock, all that a
+// CU gets.  They win where there are rounds of them; where tiles are fewer
+// than the chip has CUs a smaller one that is deep in flight does.
 struct GpTile { int bm, bn, occ; float one, full; };
 static const GpTile gp_tiles[] = {
-    {256, 256, 1, 1.80f, 1.80f},    // bf16 only: e4m3 fragments would spill
-    {128, 256, 1, 1.00f, 1.00f}, {128, 128, 2, 0.645f, 1.10f},
-    {64, 128, 2, 0.42f, 0.70f},  {128, 64, 2, 0.41f, 0.70f},
-    {64, 64, 3, 0.32f, 0.55f},   {32, 64, 4, 0.20f, 0.50f},
+    {256, 256, 1, 1.60f, 1.60f},    // bf16 only: e4m3 fragments would spill
+    {128, 256, 1, 0.94f, 0.94f}, {128, 128, 2, 0.82f, 1.10f},
+    {128, 128, 1, 0.56f, 0.56f},    // eight waves, four buffers
+    {64, 128, 2, 0.41f, 0.665f}, {128, 64, 2, 0.41f, 0.665f},
+    {64, 64, 2, 0.26f, 0.47f},   {32, 64, 2, 0.17f, 0.40f},
 };
 
+// us, chosen by rates of one block on an otherwise idle chip -> by these:
+//   1999x2048x8192 110 -> 72, 2048x6144x4096 132 -> 101, 2048x2304x9216 194 ->
+//   125, 907x2304x9216 92 -> 69, 300x3584x18944 189 -> 84, 60x4608x3584 35 ->
+//   18, 37x2048x8192 25 -> 18
 template <bool F8>
 static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
                          hipStream_t s) {
@@ -399,13 +421,17 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
       const double parts = (double)tiles * sk * g.bm * g.bn;
       if (sk > 1 && (tiles > ncnt || parts > part_floats || slabs / sk < 4))
         break;
-      const int per = (int)((tiles * sk + 255) / 256);   // blocks of a CU
-      float t = per / g.occ * g.full;
-      if (per % g.occ)
-        t += g.one + (g.full - g.one) * (per % g.occ - 1) /
-                         (g.occ > 1 ? g.occ - 1 : 1);
+      // Full rounds and a rest.  Blocks alone on their CU share L2 and
+      // memory with fewer others where not all CUs have one; a few CUs with
+      // two set the time for all.
+      const float x = (float)(tiles * sk) / 256.f;       // blocks of a CU
+      const float rest = x - (int)(x / g.occ) * g.occ;
+      float t = (int)(x / g.occ) * g.full;
+      if (rest > 1.f) t += g.one + (g.full - g.one) * (0.35f + 0.65f * (rest - 1.f));
+      else if (rest > 0.f) t += g.one * (0.8f + 0.2f * rest);
       t *= (slabs + sk - 1) / sk;
-      if (sk > 1) t += 3.f + (float)(parts * 8e-6 / 4.0);  // write and read
+      // parts written and read (2.6 TB/s), a trip for each
+      if (sk > 1) t += 3.f + 0.7f * sk + (float)(parts * 1.54e-6);
       if (best < 0 || t < best_t) {
         best = c;
         best_sk = sk;
@@ -419,10 +445,11 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
       break;
     case 1: return gp_go<F8, 128, 256, 2, 4, 3>(a, best_sk, s);
     case 2: return gp_go<F8, 128, 128, 2, 2, 2>(a, best_sk, s);
-    case 3: return gp_go<F8, 64, 128, 2, 2, 3>(a, best_sk, s);
-    case 4: return gp_go<F8, 128, 64, 2, 2, 3>(a, best_sk, s);
-    case 5: return gp_go<F8, 64, 64, 2, 2, 3>(a, best_sk, s);
-    case 6: return gp_go<F8, 32, 64, 2, 2, 3>(a, best_sk, s);
+    case 3: return gp_go<F8, 128, 128, 2, 4, 4>(a, best_sk, s);
+    case 4: return gp_go<F8, 64, 128, 2, 2, 3>(a, best_sk, s);
+    case 5: return gp_go<F8, 128, 64, 2, 2, 3>(a, best_sk, s);
+    case 6: return gp_go<F8, 64, 64, 2, 2, 4>(a, best_sk, s);
+    case 7: return gp_go<F8, 32, 64, 2, 2, 6>(a, best_sk, s);
   }
   return hipErrorInvalidValue;
 }

@@ -131,7 +131,7 @@ def test_few_rows(N, K, M, kind, norm, act):
 # slab, of one more than the buffers, split over blocks, half a slab (e4m3)
 @pytest.mark.parametrize("M,N,K", [
     (17, 70, 64), (37, 258, 192), (33, 200, 8192), (130, 1000, 320),
-    (300, 3000, 448), (513, 4100, 256), (1030, 2050, 64), (2050, 6200, 128),
+    (300, 3000, 448), (310, 2500, 1216), (513, 4100, 256), (1030, 2050, 64), (2050, 6200, 128),
     (2049, 16500, 64)])
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
 @pytest.mark.parametrize("act", [-1, 0, 1])
