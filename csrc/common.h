@@ -25,10 +25,25 @@ DEVINL u16 f2b(float f) {
   return (u16)(u >> 16);
 }
 
+// Sum over a wave, alike in all lanes.  Lanes 1, 2, 4 and 8 away are operands
+// of the add itself (where four lanes agree, the mirror image in eight is the
+// lane four away), rows of 16 and halves are swapped in registers: 40 cycles,
+// by ds_bpermute 400.
+template <int C> DEVINL float dpp_from(float v) {
+  return __uint_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_uint(v), C, 0xf, 0xf, true));
+}
 DEVINL float wave_reduce_sum(float v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m);
-  return v;
+  v += dpp_from<0xB1>(v);
+  v += dpp_from<0x4E>(v);
+  v += dpp_from<0x141>(v);
+  v += dpp_from<0x128>(v);
+  uint32_t u = __float_as_uint(v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  u = __float_as_uint(v);
+  const auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
 
 typedef float f2v __attribute__((ext_vector_type(2)));

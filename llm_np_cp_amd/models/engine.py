@@ -572,12 +572,14 @@ class GPUModel(DecodeLoop):
         nq, nkv = self.nh_l * self.hd, self.kvh_l * self.hd
         q, k, v = qkv.split([nq, nkv, nkv], dim=1)
 
-        def into_h(name, x):
-            """h += x W^T (over all ranks), Gemma's through its post norm."""
+        def into_h(name, x, g=None):
+            """h += x W^T (over all ranks), Gemma's through its post norm
+            and, with g, on to the norm that follows."""
             post = {"wo": "g_post", "wdown": "g_postffn"}[name]
             if self.gemma:
                 self._rowpar_ar(lw, name, x, t1, M, batch_attn)
-                ho.rmsnorm(t1[:M], lw[post], h[:M], res=h[:M], eps=eps)
+                ho.rmsnorm(t1[:M], lw[post], h[:M], res=h[:M], eps=eps, g2=g,
+                           y2=None if g is None else xn[:M])
             elif self.tp_branch:
                 self._rowpar_ar(lw, name, x, t1, M, batch_attn)
                 ho.addinto(h[:M], t1[:M])
@@ -592,7 +594,8 @@ class GPUModel(DecodeLoop):
                 self._rows(lw, "wqkv", h, qkv, M, g=lw["g_in"],
                            bias=lw.get("bqkv"), batch=batch_attn)
             else:
-                ho.rmsnorm(h[:M], lw["g_in"], xn[:M], eps=eps)
+                if not self.gemma or i == 0:    # else by the layer before
+                    ho.rmsnorm(h[:M], lw["g_in"], xn[:M], eps=eps)
                 self._linear(lw, "wqkv", xn, qkv, M=M, bias=lw.get("bqkv"))
             if batch_attn:
                 ho.attn_dec(qkv, self.k_cache[i], self.v_cache[i],
@@ -625,8 +628,8 @@ class GPUModel(DecodeLoop):
                             softcap=self.attn_softcap,
                             window=window or 0,
                             kS=self._ks(i), vS=self._vs(i))
-            into_h("wo", self.b_att)
             g_mlp = lw["g_preffn"] if self.gemma else lw["g_post"]
+            into_h("wo", self.b_att, None if few else g_mlp)
             if self.moe:
                 ho.rmsnorm(h[:M], g_mlp, xn[:M], eps=eps)
                 self._moe_mlp_rows(lw, M)
@@ -638,9 +641,12 @@ class GPUModel(DecodeLoop):
                     self._rows(lw, "wgu", h, a, M, g=g_mlp, act=self.act,
                                batch=batch_attn)
                 else:
-                    ho.rmsnorm(h[:M], g_mlp, xn[:M], eps=eps)
+                    if not self.gemma:
+                        ho.rmsnorm(h[:M], g_mlp, xn[:M], eps=eps)
                     self._linear(lw, "wgu", xn, a, M=M, act=self.act)
-                into_h("wdown", a)
+                last = few or i + 1 == len(self.layers)
+                into_h("wdown", a,
+                       None if last else self.layers[i + 1]["g_in"])
             if layer_hook is not None:
                 layer_hook(i, h[:M])
 

@@ -28,8 +28,8 @@ _SIGS = {
                    [ctypes.c_float] * 3 +
                    [ctypes.c_int, ctypes.c_void_p, ctypes.c_int] +
                    [ctypes.c_long] * 2 + [ctypes.c_void_p] * 2,
-    "launch_rmsnorm": [ctypes.c_void_p] * 4 + [ctypes.c_int] * 2 +
-                      [ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
+    "launch_rmsnorm": [ctypes.c_void_p] * 6 + [ctypes.c_int] * 2 +
+                      [ctypes.c_float, ctypes.c_void_p],
     "launch_rope_cache": [ctypes.c_void_p] * 7 + [ctypes.c_int] +
                          [ctypes.c_void_p] * 3 + [ctypes.c_int] * 7 +
                          [ctypes.c_void_p],
@@ -198,14 +198,15 @@ def gemv_fp8(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
 
 
 def rmsnorm(x: torch.Tensor, g: torch.Tensor, y: torch.Tensor,
-            res: torch.Tensor | None = None, eps: float = 1e-5):
-    """mode 0: y = norm(x)*g ; with res: y = res + norm(x)*g (Gemma post)."""
+            res: torch.Tensor | None = None, eps: float = 1e-5,
+            g2: torch.Tensor | None = None, y2: torch.Tensor | None = None):
+    """y = norm(x)*g ; with res: y = res + norm(x)*g (Gemma post).  With g2
+    also y2 = norm(y)*g2, the norm behind the residual."""
     M = 1 if x.dim() == 1 else x.shape[0]
     H = x.shape[-1]
-    mode = 0 if res is None else 1
     _check(lib().launch_rmsnorm(
-        _ptr(x), _ptr(g), _ptr(res), _ptr(y), M, H,
-        ctypes.c_float(eps), mode, _stream()), "rmsnorm")
+        _ptr(x), _ptr(g), _ptr(res), _ptr(y), _ptr(g2), _ptr(y2), M, H,
+        ctypes.c_float(eps), _stream()), "rmsnorm")
 
 
 def rope_cache(q: torch.Tensor, k_in: torch.Tensor, v_in: torch.Tensor,

@@ -131,8 +131,8 @@ def test_few_rows(N, K, M, kind, norm, act):
 # slab, of one more than the buffers, split over blocks, half a slab (e4m3)
 @pytest.mark.parametrize("M,N,K", [
     (17, 70, 64), (37, 258, 192), (33, 200, 8192), (130, 1000, 320),
-    (300, 3000, 448), (310, 2500, 1216), (513, 4100, 256), (1030, 2050, 64), (2050, 6200, 128),
-    (2049, 16500, 64)])
+    (300, 3000, 448), (310, 2500, 1216), (513, 4100, 256), (1030, 2050, 64),
+    (2050, 6200, 128), (2049, 16500, 64)])
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
 @pytest.mark.parametrize("act", [-1, 0, 1])
 def test_many_rows(M, N, K, kind, act):
@@ -324,3 +324,26 @@ def test_experts_of_one_row(n, kind):
         assert off(a[j], t) < (2.0 ** -7 if kind == "bf16" else 2.0 ** -18)
         z = z + p[j].double() * (D[e * H:(e + 1) * H] @ t)
     assert off(y, z) < 2.0 ** -7 and (a[n] == 7.0).all()
+
+
+# widths: one load of a few lanes, a thread each, a rest in each number of
+# loads, the widest
+@pytest.mark.parametrize("H", [8, 2048, 2304, 4104, 9000, 16384])
+@pytest.mark.parametrize("M", [1, 5])
+def test_two_norms(M, H):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    x, h = normal(M, H, seed=1), normal(M, H, seed=2)
+    g, g2 = normal(H, seed=3).float(), normal(H, seed=4).float()
+    y = torch.full((M + 1, H), 7.0, device="cuda").bfloat16()
+    z = y.clone()
+    y[:M] = h                                  # in place
+    ho.rmsnorm(x, g, y[:M], res=y[:M], eps=1e-5, g2=g2, y2=z[:M])
+
+    def rms(t):
+        return t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + 1e-5)
+
+    # bf16 results: 2^-8 of each value, the second from the first as it is
+    assert off(y[:M], rms(x.double()) * g.double() + h.double()) < 2.0 ** -8
+    assert off(z[:M], rms(y[:M].double()) * g2.double()) < 2.0 ** -8
+    assert (y[M] == 7.0).all() and (z[M] == 7.0).all()
