@@ -79,6 +79,18 @@ DEVINL float block_sum(float v, float* red) {
   return t;
 }
 
+// the same over NT threads, red 16-byte aligned, NT / 64 floats that nobody
+// reads or writes any more: one barrier
+template <int NT> DEVINL float block_sum_once(float v, float* red) {
+  v = wave_reduce_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float t = 0.f;
+#pragma unroll
+  for (int w = 0; w < NT / 64; w++) t += red[w];
+  return t;
+}
+
 DEVINL float sigmoid_f(float z) { return 1.f / (1.f + expf(-z)); }
 DEVINL float logsigmoid_f(float z) {
   return fminf(z, 0.f) - log1pf(expf(-fabsf(z)));

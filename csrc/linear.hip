@@ -88,13 +88,16 @@ DEVINL void stage_row(const RowStage& s, size_t row, bool keep, float* red,
                       Put put) {
   const int tid = threadIdx.x, W = s.W;
   const size_t o = row * W;
-  float xv[U], gv[U], yv[U];
+  float xv[U], gv[U], yv[U], av[U], tv[U];
+  const float* gt = s.gate ? s.gate + row * s.ldg : nullptr;
 #pragma unroll
-  for (int u = 0; u < U; u++) {
+  for (int u = 0; u < U; u++) {              // all on the way together
     const int i = tid + u * NT;
     xv[u] = i < W ? s.x[o + i] : 0.f;
     gv[u] = s.g && i < W ? s.g[i] : 0.f;
     if (s.y) yv[u] = i < W ? s.y[o + i] : 0.f;
+    if (s.xadd) av[u] = i < W ? s.xadd[o + i] : 0.f;
+    tv[u] = gt && i < W ? gt[i] : 0.f;
   }
   [[maybe_unused]] int pos = 0;
   [[maybe_unused]] float* ring = nullptr;
@@ -147,16 +150,13 @@ DEVINL void stage_row(const RowStage& s, size_t row, bool keep, float* red,
       ss += yv[u] * yv[u];
     }
     for (int i = tid + U * NT; i < W; i += NT) ss += s.y[o + i] * s.y[o + i];
-    rb = 1.f / sqrtf(block_sum(ss, red) / (float)W + s.eps);
+    rb = 1.f / sqrtf(block_sum_once<NT>(ss, red) / (float)W + s.eps);
 #pragma unroll
     for (int u = 0; u < U; u++) xv[u] += yv[u] * rb * gb[u];
   }
   if (s.xadd)
 #pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int i = tid + u * NT;
-      if (i < W) xv[u] += s.xadd[o + i];
-    }
+    for (int u = 0; u < U; u++) xv[u] += av[u];
   auto late = [&](int i) {              // elements beyond the registers
     float v = s.x[o + i];
     if (s.y) v += s.y[o + i] * rb * s.gb[i];
@@ -172,12 +172,11 @@ DEVINL void stage_row(const RowStage& s, size_t row, bool keep, float* red,
       const float v = late(i);
       ss += v * v;
     }
-    rn = 1.f / sqrtf(block_sum(ss, red) / (float)W + s.eps);
+    rn = 1.f / sqrtf(block_sum_once<NT>(ss, red + NT / 64) / (float)W + s.eps);
   }
-  const float* gt = s.gate ? s.gate + row * s.ldg : nullptr;
-  auto finish = [&](int i, float v, float g) {
+  auto finish = [&](int i, float v, float g, float t) {
     if (s.g && i < s.Kp)
-      put(i, i < W ? v * rn * g * (gt ? sigmoid_f(gt[i]) : 1.f) : 0.f);
+      put(i, i < W ? v * rn * g * (gt ? sigmoid_f(t) : 1.f) : 0.f);
     // xout may be x: its reads are done
     if (keep && s.xout && i < W) s.xout[o + i] = v;
   };
@@ -203,9 +202,10 @@ DEVINL void stage_row(const RowStage& s, size_t row, bool keep, float* red,
     return;
   }
 #pragma unroll
-  for (int u = 0; u < U; u++) finish(tid + u * NT, xv[u], gv[u]);
+  for (int u = 0; u < U; u++) finish(tid + u * NT, xv[u], gv[u], tv[u]);
   for (int i = tid + U * NT; i < max(W, s.Kp); i += NT)
-    finish(i, i < W ? late(i) : 0.f, s.g && i < W ? s.g[i] : 0.f);
+    finish(i, i < W ? late(i) : 0.f, s.g && i < W ? s.g[i] : 0.f,
+           gt && i < W ? gt[i] : 0.f);
 }
 
 // ---- staging a row of several residual streams ----------------------------
@@ -380,7 +380,7 @@ k_group_rows(RowStage s, int groups, T* __restrict__ out) {
 template <typename T, int U>
 __global__ void __launch_bounds__(256)
 k_norm_rows(RowStage s, const int* __restrict__ rows, T* __restrict__ out) {
-  __shared__ float red[4];
+  __shared__ float red[8];
   T* o = out + (size_t)blockIdx.x * s.Kp;
   stage_row<256, U>(s, rows ? rows[blockIdx.x] : blockIdx.x, true, red,
                [&](int i, float v) { o[i] = El<T>::st(v); });
@@ -747,7 +747,7 @@ DEVINL float gelu_f(float v) {
 template <typename T, int MODE, int U, int NR, int HS = 0>
 __global__ void __launch_bounds__(LIN_NT) k_lin_row(LinRowArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  __shared__ float red[LIN_NT / 64 * (MODE == ROW_POLY ? 3 : 1)];
+  __shared__ float red[LIN_NT / 64 * (MODE == ROW_POLY ? 3 : 2)];
   constexpr int V = El<T>::V, S = 64 * V, NK = 8 / NR;
   T* xs = (T*)smem;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -977,42 +977,75 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs a) {
 
 // up to 16*MF rows: a tile of NB (16, or 8 to have more blocks) outputs per
 // block, K over NW waves, both operands straight from memory (the weights are
-// read once)
+// read once).  A load of W takes 8 rows x 128 bytes, whole lines, and an
+// exchange with lane ^ 8 makes operands of two of them (row_gemm.hip); in 16
+// rows x 64 bytes, and half of the lanes idle for eight outputs, 4 rows of
+// 32000x2048 took 28.6 us, now 24.3, 8192x2048 9.8 -> 8.9, 2048x8192 (in two
+// trips of loads, now one) 11.0 -> 9.6.
 template <typename T, int MF, int NW, int NB = 16>
 __global__ void __launch_bounds__(64 * NW) k_gemm_skinny(GemmArgs a) {
   __shared__ float red[NW * MF * 256];
-  constexpr int U = MF == 1 ? 8 : 4;
+  constexpr int R = NB / 8;                  // loads of a slab of W
+  constexpr int U = MF == 1 ? 8 / R : MF == 2 ? 4 : 2;
   const int tid = threadIdx.x, wave = wave_index(), lane = tid & 63;
   const int lr = lane & 15, gq = lane >> 4, z = blockIdx.z;
+  const bool low = lr < 8;
   const int K = z ? a.K2 : a.K, ldw = z ? a.K2 : a.ldw;
-  const int n0 = blockIdx.x * NB, nch = K * (int)sizeof(T) / 64;
-  const char* wr = (const char*)((const T*)a.W + (size_t)z * a.wz +
-                                 (size_t)min(n0 + lr, a.N - 1) * ldw) +
-                   gq * 16;
+  const int n0 = blockIdx.x * NB, nsl = K * (int)sizeof(T) / 128;
+  const char* wr[R];
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    wr[r] = (const char*)((const T*)a.W + (size_t)z * a.wz +
+                          (size_t)min(n0 + r * 8 + (lane & 7), a.N - 1) * ldw) +
+            (lane >> 3) * 16;
   const char* xr[MF];
 #pragma unroll
   for (int i = 0; i < MF; i++)
     xr[i] = (const char*)((const T*)a.X + (size_t)z * a.xz +
-                          (size_t)min(i * 16 + lr, a.M - 1) * a.ldx) + gq * 16;
+                          (size_t)min(i * 16 + lr, a.M - 1) * a.ldx) + gq * 32;
   f4v acc[MF];
 #pragma unroll
   for (int i = 0; i < MF; i++) acc[i] = {0.f, 0.f, 0.f, 0.f};
-  for (int c = wave; c < nch; c += U * NW) {
-    f4v w[U], xv[U][MF];
+  auto turn = [](float v) {                  // the value of lane ^ 8
+    return dpp_from<0x128>(v);
+  };
+  for (int s = wave; s < nsl; s += U * NW) {
+    f4v w[U][R], xv[U][MF][2];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int cu = c + u * NW;
-      const bool in = cu < nch;
-      w[u] = in && lr < NB ? ld16nt(wr + (size_t)cu * 64) : f4v{0.f, 0.f, 0.f, 0.f};
+      const int su = s + u * NW;
+      const bool in = su < nsl;
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        w[u][r] = in ? ld16nt(wr[r] + (size_t)su * 128)
+                     : f4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < MF; i++)
-        xv[u][i] = in ? ld16(xr[i] + cu * 64) : f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+          xv[u][i][q] = in ? ld16(xr[i] + (size_t)su * 128 + q * 16)
+                           : f4v{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
-    for (int u = 0; u < U; u++)
+    for (int u = 0; u < U; u++) {
+      f4v c[2];                              // row lr, chunks 2gq and 2gq + 1
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        if constexpr (R == 1) {
+          c[0][d] = w[u][0][d];              // rows 8-15 are not there
+          c[1][d] = turn(w[u][0][d]);
+        } else {
+          const float got = turn(low ? w[u][1][d] : w[u][0][d]);
+          c[0][d] = low ? w[u][0][d] : got;
+          c[1][d] = low ? got : w[u][1][d];
+        }
+      }
 #pragma unroll
       for (int i = 0; i < MF; i++)
-        acc[i] = GemmMma<T>::mma(xv[u][i], w[u], acc[i]);
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+          acc[i] = GemmMma<T>::mma(xv[u][i][q], c[q], acc[i]);
+    }
   }
 #pragma unroll
   for (int i = 0; i < MF; i++)
