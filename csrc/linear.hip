@@ -945,14 +945,13 @@ template <class Body> DEVINL void with_epilogue(int epi, Body body) {
 
 template <typename T, int BM, int BN>
 __global__ void __launch_bounds__(256) k_gemm(GemmArgs a) {
-  __shared__ __attribute__((aligned(16))) char lds[gemm_lds_bytes<BM, BN>()];
   const int bm = blockIdx.y * BM, bn = blockIdx.x * BN, z = blockIdx.z;
   const T* X = (const T*)a.X + (size_t)z * a.xz;
   const T* W = (const T*)a.W + (size_t)z * a.wz;
   const int K = z ? a.K2 : a.K, ldw = z ? a.K2 : a.ldw;
   f4v acc[BM / 32][BN / 32];
   gemm_mainloop<BM, BN, T>(
-      acc, lds,
+      acc,
       [&](int r) { return X + (size_t)min(bm + r, a.M - 1) * a.ldx; },
       [&](int r) { return W + (size_t)min(bn + r, a.N - 1) * ldw; }, 0,
       K / GemmMma<T>::BK);

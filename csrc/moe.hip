@@ -133,7 +133,6 @@ __global__ void __launch_bounds__(1024) k_moe_sort(const int* __restrict__ idx,
 // gate/up of gathered rows; act rows are in expert order
 template <typename T, int BM, int BN>
 __global__ void __launch_bounds__(256) k_moe_gu(MoeArgs m, MoeSort s) {
-  __shared__ __attribute__((aligned(16))) char lds[gemm_lds_bytes<BM, BN>()];
   const int t = blockIdx.y, nr = s.tile_n[t];
   if (nr == 0) return;
   const int e = s.tile_e[t], p0 = s.tile_row0[t];
@@ -143,7 +142,7 @@ __global__ void __launch_bounds__(256) k_moe_gu(MoeArgs m, MoeSort s) {
   const T* W = moe_gu_base<T>(m, e);
   f4v acc[BM / 32][BN / 32];
   gemm_mainloop<BM, BN, T>(
-      acc, lds,
+      acc,
       [&](int r) {
         return (const T*)m.h +
                (size_t)(s.perm[p0 + min(r, nr - 1)] / m.K1) * m.ldh;
@@ -178,7 +177,6 @@ __global__ void __launch_bounds__(256) k_moe_gu(MoeArgs m, MoeSort s) {
 template <typename T, int BM, int BN>
 __global__ void __launch_bounds__(256) k_moe_down(MoeArgs m, MoeSort s,
                                                   T* __restrict__ y) {
-  __shared__ __attribute__((aligned(16))) char lds[gemm_lds_bytes<BM, BN>()];
   const int t = blockIdx.y, nr = s.tile_n[t];
   if (nr == 0) return;
   const int e = s.tile_e[t], p0 = s.tile_row0[t], bn = blockIdx.x * BN;
@@ -186,7 +184,7 @@ __global__ void __launch_bounds__(256) k_moe_down(MoeArgs m, MoeSort s,
   const T* W = moe_down_base<T>(m, e);
   f4v acc[BM / 32][BN / 32];
   gemm_mainloop<BM, BN, T>(
-      acc, lds,
+      acc,
       [&](int r) {
         return (const T*)m.act + (size_t)(p0 + min(r, nr - 1)) * m.ldact;
       },
