@@ -1,13 +1,27 @@
 // row_gemm.hip — linears of few rows: Y[M,N] = X[M,K] W[N,K]^T, up to 16 rows.
 //
 // Bound by streaming W once.  X (its RMSNorm taken on the way) waits in LDS
-// while a block walks tiles of 16 outputs; its eight waves share out K, so
-// W goes from memory to the MFMA operand with no LDS and no barrier between,
-// the next slabs already in flight, and the partial sums meet in LDS once a
-// tile.  Deep or narrow products split K over blocks as well; the last block
-// of a column group to arrive adds the parts in their order.  What used to
-// be a launch of its own rides along: norm, gate activation (gate and up
-// rows of W belong to the same tile), bias, soft cap, residual.
+// while a block takes its share of the outputs, alike for all blocks, in tiles
+// of 16 (of 8 where a share is small); W goes from memory to the MFMA operand
+// with no LDS and no barrier between.  The slabs of all its tiles are one list
+// that the eight waves share out evenly, the next group always in flight:
+// every load is taken, at a place that stays at the list's end, for the
+// compiler counts those behind a load that it waits for only where no branch
+// and no use of a value stands between.  What a wave has of a tile goes to
+// LDS, and the waves meet once.
+// us, by tiles dealt out whole, a meeting each, and a choice of value or zero
+// right behind each e4m3 and MXFP4 load -> here:
+//   16 rows e4m3  2x14336x3584 34.4 -> 22.6 (4.5 TB/s), with the norm 40.5 ->
+//                 27.5; 3584x14336 25.7 -> 19.1; 32768x3584 43.8 -> 29.9
+//   4 rows e4m3   8192x3584 14.7 -> 9.6, 3584x14336 19.0 -> 14.0
+//   3 rows bf16   4608x3584 14.8 -> 11.6, 2x18944x3584 55.4 -> 51.0 (5.3 TB/s)
+//   4 rows MXFP4  2x8192x3072 14.1 -> 11.8
+// Left: two us of launch, the norm of 16 rows in each block (5 us), and the
+// meeting of parts where K is split.
+// Deep or narrow products split K over blocks as well; the last block of a
+// column group to arrive adds the parts in their order.  What used to be a
+// launch of its own rides along: norm, gate activation (gate and up rows of W
+// belong to the same tile), bias, soft cap, residual.
 //
 // A wave's load takes 8 rows x 128 bytes of W (whole lines: 6.9 TB/s; 16
 // rows x 64 bytes reach 5.7), which leaves lane l with row l&7 and 16-byte
@@ -20,6 +34,7 @@
 
 typedef __bf16 rg_b8 __attribute__((ext_vector_type(8)));
 typedef __bf16 rg_b2 __attribute__((ext_vector_type(2)));
+typedef float rg_f4 __attribute__((ext_vector_type(4), aligned(4)));
 
 struct RgArgs {
   const void* x;       // [M, ldx] bf16; e4m3 beside e4m3 weights and no norm
@@ -34,6 +49,7 @@ struct RgArgs {
   float* part;         // split K: sums of a tile, [tile, split, ...]
   int* cnt;            // split K: blocks of a column group that are done
   int M, N, K, ldx, ldr, ldy, act, out_f32, kr;
+  int rpb;             // outputs of a block
   float eps, softcap;
 };
 
@@ -90,9 +106,10 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
   constexpr int P = GLU ? 2 : 1;             // weight rows of an output
   constexpr int R = NB / 8;                  // loads of a slab and matrix
   constexpr int U = 8 / (P * R);             // slabs of a group: 8 loads
-  __shared__ __attribute__((aligned(16))) float red[RG_NW][P][256];
   __shared__ float sx[16];
   __shared__ int last_flag;
+  // X, then what the waves have of the tiles: of tile t wave w's is w + t,
+  // since a wave starts where the one before ends
   extern __shared__ __attribute__((aligned(16))) char xs[];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -104,63 +121,100 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
   const int k0 = blockIdx.y * a.kr;
   const int kn = min(a.kr, a.K - k0);        // elements of this block
   const int nslab = (kn + SE - 1) / SE;
-  const int spw = (nslab + RG_NW - 1) / RG_NW;
-  const int s_lo = min(wave * spw, nslab), s_hi = min(s_lo + spw, nslab);
-  const int ngrp = (spw + U - 1) / U;        // alike in all waves
-  const int ntile = (a.N + NB - 1) / NB;
+  const int n0 = blockIdx.x * a.rpb, n1 = min(n0 + a.rpb, a.N);
+  const int ntile = (n1 - n0 + NB - 1) / NB;
   const int xstride = nslab * SE * XB + 16;  // bytes: rows on other banks
 
-  u4v_ wc[U][P * R], wn[U][P * R];
-  uint32_t ec[U][P], en[U][P];
-  auto load = [&](u4v_ (&w)[U][P * R], uint32_t (&ex)[U][P], int tile,
-                  int grp) {
+  // a wave's place in the list: slabs still to come, the next one's tile, slab
+  struct Place { int left, t, s; };
+  const int steps = ntile * nslab, per = (steps + RG_NW - 1) / RG_NW;
+  float* red = (float*)(xs + a.M * xstride);
+  Place at;                                  // a wave without slabs: left 0
+  {
+    const int lo = min(wave * per, steps), l = min(lo, steps - 1);
+    at.left = min(per, steps - lo);
+    at.t = l / nslab;
+    at.s = l % nslab;
+  }
+  auto step = [&](Place& p, int by) {        // by 1 or 0, without a branch
+    p.left -= by;
+    p.s += by;
+    const int over = p.s == nslab;
+    p.s -= over ? nslab : 0;
+    p.t += over;
+  };
+
+  u4v_ wa[U][P * R], wb[U][P * R];
+  uint32_t ea[U][P], eb[U][P];
+  Place ahead = at;
+  auto load = [&](u4v_ (&w)[U][P * R], uint32_t (&ex)[U][P]) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int s = s_lo + grp * U + u;
-      if (s < s_hi) {
-        const int ke = k0 + s * SE + c8 * E;
-        const bool in = SE == 64 || ke < a.K;   // K is a multiple of 64
+      // behind K (e4m3, MXFP4: half a slab) X is zero, whatever W is
+      const int ke = k0 + ahead.s * SE + c8 * E;
+      const size_t kb = (size_t)(SE == 64 || ke < a.K ? ke : 0) * 16 / E;
 #pragma unroll
-        for (int p = 0; p < P; p++) {
+      for (int m = 0; m < P; m++) {
 #pragma unroll
-          for (int r = 0; r < R; r++) {
-            const size_t row = (size_t)p * a.N +
-                               min(tile * NB + r * 8 + r8, a.N - 1);
-            const char* q = (const char*)a.w + row * ((size_t)a.K * 16 / E) +
-                            (size_t)(in ? ke : 0) * 16 / E;
-            w[u][p * R + r] = __builtin_nontemporal_load((const u4v_*)q);
-            if (!in) w[u][p * R + r] = u4v_{};
-          }
-          if constexpr (WT == RG_FP4) {
-            // exponents of this lane's two chunks after the exchange
-            const size_t row = (size_t)p * a.N +
-                               min(tile * NB + (lr & (NB - 1)), a.N - 1);
-            const int kb = (k0 + s * SE) / 32 + gq * 2;
-            ex[u][p] = kb < a.K / 32
-                           ? *(const u16*)(a.we + row * (a.K / 32) + kb)
-                           : 0;
-          }
+        for (int r = 0; r < R; r++) {
+          const size_t row = (size_t)m * a.N +
+                             min(n0 + ahead.t * NB + r * 8 + r8, n1 - 1);
+          w[u][m * R + r] = __builtin_nontemporal_load(
+              (const u4v_*)((const char*)a.w +
+                            row * ((size_t)a.K * 16 / E) + kb));
+        }
+        if constexpr (WT == RG_FP4) {
+          // exponents of this lane's two chunks after the exchange
+          const size_t row = (size_t)m * a.N +
+                             min(n0 + ahead.t * NB + (lr & (NB - 1)), n1 - 1);
+          const int k2 = min((k0 + ahead.s * SE) / 32 + gq * 2, a.K / 32 - 2);
+          ex[u][m] = *(const u16*)(a.we + row * (a.K / 32) + k2);
         }
       }
+      step(ahead, ahead.left > 1);
     }
   };
 
-  int tile = blockIdx.x;
+  // what an output needs besides its sum: of a thread's first ones ahead of
+  // all else
+  struct Rest { float s, s2, add; };
+  auto rest = [&](int e) {
+    const int row = (e >> 4) & 15, cl = e & 15, n = n0 + (e >> 8) * NB + cl;
+    Rest o = {1.f, 1.f, 0.f};
+    if (row >= a.M || n >= n1 || cl >= NB) return o;
+    if (WT == RG_FP8) {
+      o.s = a.ws[n];
+      if (GLU) o.s2 = a.ws[a.N + n];
+    }
+    if (a.bias) o.add = b2f(a.bias[n]);
+    if (a.res) o.add += b2f(a.res[(size_t)row * a.ldr + n]);
+    return o;
+  };
+  constexpr int NT = 64 * RG_NW, J = 2;
+  Rest o[J];
+#pragma unroll
+  for (int j = 0; j < J; j++)
+    if (KS == 1) o[j] = rest(tid + j * NT);
 
   // X into LDS, zeros behind K.  Its loads go out ahead of W's: they come
   // from L2 and return first, and loads return in order.
   if constexpr (NORM) {
     s8v v[2][RG_NORM_K / 512];
+    rg_f4 g[RG_NORM_K / 512][2];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int j = 0; j < RG_NORM_K / 512; j++)
+      if (j * 512 < kn) {
+        const int k = min(j * 512 + lane * 8, kn - 8);
+        g[j][0] = *(const rg_f4*)(a.g + k);
+        g[j][1] = *(const rg_f4*)(a.g + k + 4);
 #pragma unroll
-      for (int j = 0; j < RG_NORM_K / 512; j++) {
-        const int row = i * RG_NW + wave, k = j * 512 + lane * 8;
-        v[i][j] = s8v{};
-        if (row < a.M && k < kn)
-          v[i][j] = *(const s8v*)((const u16*)a.x + (size_t)row * a.ldx + k);
+        for (int i = 0; i < 2; i++) {
+          const int row = i * RG_NW + wave;
+          if (row < a.M)
+            v[i][j] = *(const s8v*)((const u16*)a.x + (size_t)row * a.ldx + k);
+        }
       }
-    load(wc, ec, tile, 0);
+    load(wa, ea);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
       const int row = i * RG_NW + wave;
@@ -168,14 +222,15 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
       float ss = 0.f;
 #pragma unroll
       for (int j = 0; j < RG_NORM_K / 512; j++)
+        if (j * 512 + lane * 8 < kn)
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-          const float f = b2f(((u16*)&v[i][j])[q]);
-          ss += f * f;
-        }
+          for (int q = 0; q < 8; q++) {
+            const float f = b2f(((u16*)&v[i][j])[q]);
+            ss += f * f;
+          }
       const float rn = rsqrtf(wave_reduce_sum(ss) / (float)a.K + a.eps);
       auto normed = [&](int j, int q) {
-        return b2f(((u16*)&v[i][j])[q]) * rn * a.g[j * 512 + lane * 8 + q];
+        return b2f(((u16*)&v[i][j])[q]) * rn * g[j][q / 4][q % 4];
       };
       float am = 1.f;
       if constexpr (WT == RG_FP8) {          // rows rounded to e4m3
@@ -214,9 +269,10 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
   } else {
     constexpr int NV = 12, VE = 16 / XB;     // 16-byte loads a thread
     const int per = nslab * SE / VE, all = a.M * per;
+    const float rper = 1.f / per;            // e / per: exact below 2^20
     u4v_ v[NV];
     auto get = [&](int e) {
-      const int row = e / per, k = (e - row * per) * VE;
+      const int row = (int)((e + 0.5f) * rper), k = (e - row * per) * VE;
       u4v_ r{};
       if (e < all && k < kn)
         r = *(const u4v_*)((const char*)a.x +
@@ -224,43 +280,31 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
       return r;
     };
     auto put = [&](int e, u4v_ r) {
-      const int row = e / per, k = (e - row * per) * VE;
+      const int row = (int)((e + 0.5f) * rper), k = (e - row * per) * VE;
       if (e < all) *(u4v_*)(xs + row * xstride + k * XB) = r;
     };
 #pragma unroll
-    for (int j = 0; j < NV; j++) v[j] = get(j * 64 * RG_NW + tid);
-    load(wc, ec, tile, 0);
-    if (WT == RG_FP8 && tid < a.M) sx[tid] = a.sx[tid];
+    for (int j = 0; j < NV; j++)
+      if (j * NT < all) v[j] = get(j * NT + tid);
+    const float sr = WT == RG_FP8 ? a.sx[min(tid, a.M - 1)] : 0.f;
+    load(wa, ea);
+    if (WT == RG_FP8 && tid < a.M) sx[tid] = sr;
 #pragma unroll
-    for (int j = 0; j < NV; j++) put(j * 64 * RG_NW + tid, v[j]);
-    for (int e0 = NV * 64 * RG_NW; e0 < all; e0 += NV * 64 * RG_NW) {
+    for (int j = 0; j < NV; j++)
+      if (j * NT < all) put(j * NT + tid, v[j]);
+    for (int e0 = NV * NT; e0 < all; e0 += NV * NT) {
 #pragma unroll
-      for (int j = 0; j < NV; j++) v[j] = get(e0 + j * 64 * RG_NW + tid);
+      for (int j = 0; j < NV; j++) v[j] = get(e0 + j * NT + tid);
 #pragma unroll
-      for (int j = 0; j < NV; j++) put(e0 + j * 64 * RG_NW + tid, v[j]);
+      for (int j = 0; j < NV; j++) put(e0 + j * NT + tid, v[j]);
     }
   }
   const char* xr = xs + min(lr, a.M - 1) * xstride + gq * 2 * E * XB;
   __syncthreads();
 
-  // what an output needs besides its sum: loaded ahead of the next tile's W,
-  // since loads return in order
-  struct Rest { float s, s2, add; };
-  auto rest = [&](int t) {
-    const int row = (tid >> 4) & 15, cl = tid & 15, n = t * NB + cl;
-    Rest o = {1.f, 1.f, 0.f};
-    if (row >= a.M || n >= a.N || cl >= NB) return o;
-    if (WT == RG_FP8) {
-      o.s = a.ws[n];
-      if (GLU) o.s2 = a.ws[a.N + n];
-    }
-    if (a.bias) o.add = b2f(a.bias[n]);
-    if (a.res) o.add += b2f(a.res[(size_t)row * a.ldr + n]);
-    return o;
-  };
-  auto finish = [&](int t, float v, float up, const Rest& o) {
-    const int row = tid >> 4, cl = tid & 15, n = t * NB + cl;
-    if (row >= a.M || n >= a.N || cl >= NB) return;
+  auto finish = [&](int e, float v, float up, const Rest& o) {
+    const int row = (e >> 4) & 15, cl = e & 15, n = n0 + (e >> 8) * NB + cl;
+    if (row >= a.M || n >= n1 || cl >= NB) return;
     if (WT == RG_FP8) {
       v *= sx[row] * o.s;
       up *= sx[row] * o.s2;
@@ -279,92 +323,107 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
     else ((u16*)a.y)[(size_t)row * a.ldy + n] = f2b(v);
   };
 
-  for (; tile < ntile; tile += gridDim.x) {
-    f4v acc[P];
+  f4v acc[P];
 #pragma unroll
-    for (int p = 0; p < P; p++) acc[p] = {0.f, 0.f, 0.f, 0.f};
-    Rest ahead = {1.f, 1.f, 0.f};
-    if (KS == 1 && tid < 256) ahead = rest(tile);
-
-    for (int grp = 0; grp < ngrp; grp++) {
-      const bool next = grp + 1 < ngrp;
-      const int tn = next ? tile : tile + (int)gridDim.x;
-      if (tn < ntile) load(wn, en, tn, next ? grp + 1 : 0);
+  for (int p = 0; p < P; p++) acc[p] = {0.f, 0.f, 0.f, 0.f};
+  auto group = [&](u4v_ (&w)[U][P * R], uint32_t (&ex)[U][P]) {
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int s = s_lo + grp * U + u;
-        if (s < s_hi) {
-          // row lr, chunks 2gq and 2gq+1 of either matrix
-          u4v_ ch[P][2];
+    for (int u = 0; u < U; u++) {
+      // row lr, chunks 2gq and 2gq+1 of either matrix
+      u4v_ ch[P][2];
 #pragma unroll
-          for (int p = 0; p < P; p++) {
-            if constexpr (R == 1) {
-              // rows 8-15 are not there: their outputs are dropped
-              ch[p][0] = wc[u][p];
+      for (int p = 0; p < P; p++) {
+        if constexpr (R == 1) {
+          // rows 8-15 are not there: their outputs are dropped
+          ch[p][0] = w[u][p];
 #pragma unroll
-              for (int d = 0; d < 4; d++) ch[p][1][d] = swap8(wc[u][p][d]);
-            } else {
+          for (int d = 0; d < 4; d++) ch[p][1][d] = swap8(w[u][p][d]);
+        } else {
 #pragma unroll
-              for (int d = 0; d < 4; d++) {
-                const uint32_t a0 = wc[u][p * R][d], a1 = wc[u][p * R + 1][d];
-                const uint32_t got = swap8(low ? a1 : a0);
-                ch[p][0][d] = low ? a0 : got;
-                ch[p][1][d] = low ? got : a1;
-              }
-            }
+          for (int d = 0; d < 4; d++) {
+            const uint32_t a0 = w[u][p * R][d], a1 = w[u][p * R + 1][d];
+            const uint32_t got = swap8(low ? a1 : a0);
+            ch[p][0][d] = low ? a0 : got;
+            ch[p][1][d] = low ? got : a1;
           }
-#pragma unroll
-          for (int q = 0; q < 2; q++)
-#pragma unroll
-            for (int f = 0; f < XF; f++) {
-              // 8 elements of X: 16 bytes of bf16, half as much of e4m3
-              const u4v_ xf = *(const u4v_*)(
-                  xr + s * SE * XB + (q * XF + f) / (3 - XB) * 16);
-#pragma unroll
-              for (int p = 0; p < P; p++)
-                acc[p] = rg_mma<WT>(xf, ch[p][q], f,
-                                    WT == RG_FP4 ? (ec[u][p] >> (8 * q)) & 255
-                                                 : 0, acc[p]);
-            }
         }
       }
 #pragma unroll
-      for (int u = 0; u < U; u++) {
+      for (int q = 0; q < 2; q++)
 #pragma unroll
-        for (int j = 0; j < P * R; j++) wc[u][j] = wn[u][j];
+        for (int f = 0; f < XF; f++) {
+          // 8 elements of X: 16 bytes of bf16, half as much of e4m3
+          const u4v_ xf = *(const u4v_*)(
+              xr + at.s * SE * XB + (q * XF + f) / (3 - XB) * 16);
 #pragma unroll
-        for (int p = 0; p < P; p++) ec[u][p] = en[u][p];
+          for (int p = 0; p < P; p++)
+            acc[p] = rg_mma<WT>(xf, ch[p][q], f,
+                                WT == RG_FP4 ? (ex[u][p] >> (8 * q)) & 255
+                                             : 0, acc[p]);
+        }
+      // sums behind the list's end are not put anywhere
+      const int t = at.t;
+      step(at, 1);
+      if (at.left >= 0 && (at.s == 0 || at.left == 0)) {
+        // element r of acc: row gq*4 + r, output lr
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            red[((wave + t) * P + p) * 256 + (gq * 4 + r) * 16 + lr] =
+                acc[p][r];
+          acc[p] = {0.f, 0.f, 0.f, 0.f};
+        }
       }
     }
+  };
+  // the last group by itself: no loads behind it
+  for (int todo = at.left - U;;) {
+    if (todo <= 0) {
+      group(wa, ea);
+      break;
+    }
+    load(wb, eb);
+    todo -= U;
+    group(wa, ea);
+    if (todo <= 0) {
+      group(wb, eb);
+      break;
+    }
+    load(wa, ea);
+    todo -= U;
+    group(wb, eb);
+  }
 
-    // element r of acc: row gq*4 + r, output lr.  The barriers wait for LDS
-    // only: the next tile's loads stay in flight.
-    auto meet = [&] {
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    };
+  // outputs of four tiles at a time, two a thread
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  const int tiles = (a.rpb + NB - 1) / NB;   // of a full block
+  float* parts = a.part + (size_t)blockIdx.x * tiles * KS * (P * 256);
+  const float rper = 1.f / per;
+  for (int e0 = tid; e0 < ntile * 256; e0 += NT * J) {
+    if (KS == 1 && e0 != tid)
 #pragma unroll
-    for (int p = 0; p < P; p++)
+      for (int j = 0; j < J; j++) o[j] = rest(e0 + j * NT);
 #pragma unroll
-      for (int r = 0; r < 4; r++)
-        red[wave][p][(gq * 4 + r) * 16 + lr] = acc[p][r];
-    meet();
-    if (tid < 256) {
+    for (int j = 0; j < J; j++) {
+      const int e = e0 + j * NT, t = e >> 8;
+      if (t >= ntile || ((e >> 4) & 15) >= a.M) continue;
+      // waves that have slabs of it; exact for less than 2^20 slabs
+      const int lo = (int)((t * nslab + 0.5f) * rper);
+      const int hi = (int)((t * nslab + nslab - 0.5f) * rper);
       float v = 0.f, up = 0.f;
-#pragma unroll
-      for (int q = 0; q < RG_NW; q++) {
-        v += red[q][0][tid];
-        if (GLU) up += red[q][P - 1][tid];
+      for (int q = lo; q <= hi; q++) {
+        v += red[(q + t) * P * 256 + (e & 255)];
+        if (GLU) up += red[((q + t) * P + P - 1) * 256 + (e & 255)];
       }
       if (KS == 1) {
-        finish(tile, v, up, ahead);
+        finish(e, v, up, o[j]);
       } else {
-        float* pp =
-            a.part + ((size_t)tile * KS + blockIdx.y) * (P * 256) + tid;
+        float* pp = parts + ((size_t)t * KS + blockIdx.y) * (P * 256) + (e & 255);
         pp[0] = v;
         if (GLU) pp[256] = up;
       }
     }
-    meet();
   }
   if (KS == 1) return;
 
@@ -386,28 +445,36 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
     a.cnt[blockIdx.x] = 0;                   // for the next launch
   }
   __syncthreads();
-  if (tid >= 256) return;
-  for (tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
-    const float* pp = a.part + (size_t)tile * KS * (P * 256) + tid;
+  for (int e = tid; e < ntile * 256; e += 64 * RG_NW) {
+    if (((e >> 4) & 15) >= a.M) continue;
+    const float* pp = parts + (size_t)(e >> 8) * KS * (P * 256) + (e & 255);
+    const Rest o = rest(e);
     float v = 0.f, up = 0.f;
-    for (int q = 0; q < KS; q++) {
-      v += pp[(size_t)q * (P * 256)];
-      if (GLU) up += pp[(size_t)q * (P * 256) + 256];
+    for (int q0 = 0; q0 < KS; q0 += 8) {     // eight parts a trip
+      float x[8], y[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        x[q] = pp[(size_t)min(q0 + q, KS - 1) * (P * 256)];
+        if (GLU) y[q] = pp[(size_t)min(q0 + q, KS - 1) * (P * 256) + 256];
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+        if (q0 + q < KS) {
+          v += x[q];
+          if (GLU) up += y[q];
+        }
     }
-    finish(tile, v, up, rest(tile));
+    finish(e, v, up, o);
   }
 }
 
-// LDS that X may take: all but the sums
-template <bool GLU> constexpr int rg_room() {
-  return (160 - RG_NW * (GLU ? 2 : 1) - 1) * 1024;
-}
+#define RG_ROOM (159 * 1024)     // LDS of a block: X and the sums
 
 template <int WT, int NB, bool GLU, bool NORM>
 static void rg_go(const RgArgs& a, dim3 grid, size_t lds, hipStream_t s) {
   static const hipError_t raised = hipFuncSetAttribute(
       (const void*)&k_row_gemm<WT, NB, GLU, NORM>,
-      hipFuncAttributeMaxDynamicSharedMemorySize, rg_room<GLU>());
+      hipFuncAttributeMaxDynamicSharedMemorySize, RG_ROOM);
   (void)raised;
   hipLaunchKernelGGL((k_row_gemm<WT, NB, GLU, NORM>), grid, dim3(64 * RG_NW),
                      lds, s, a);
@@ -424,34 +491,40 @@ static hipError_t rg_run(RgArgs a, long part_floats, int ncnt,
   auto lds_of = [&](int ks) {
     return (long)a.M * (part_k(ks) * (WT == RG_FP8 ? 1 : 2) + 16);
   };
-  auto fits = [&](int ks, int nb) {
-    const long nt = (a.N + nb - 1) / nb;
-    return lds_of(ks) <= rg_room<GLU>() &&
-           (ks == 1 || (!a.g && nt * ks * P * 256 <= part_floats &&
-                        (nt < 256 ? nt : 256) <= ncnt));
+  // A block a CU, with X in place for all its outputs: two a CU read X twice
+  // and run no faster (5 rows, 2x8192x2048: 16.9 us, 512 blocks 21.1;
+  // 32768x3072 38.9 and 43.9).  Less than eight outputs a block gain nothing;
+  // more than LDS has room for the sums of are left to blocks of a next round.
+  auto tile_of = [&](int r) { return r <= 24 && (r - 1) % 16 < 8 ? 8 : 16; };
+  auto share = [&](int ks) {
+    const int ng = 256 / ks > 1 ? 256 / ks : 1, r = (a.N + ng - 1) / ng;
+    const long most = (RG_ROOM - lds_of(ks)) / (P * 1024) - (RG_NW - 1);
+    return most < 1 ? 0 : (int)(r < 8 ? 8 : r < most * 16 ? r : most * 16);
+  };
+  auto fits = [&](int ks) {
+    const int r = share(ks);
+    if (r < 1) return false;
+    const int nb = tile_of(r);
+    const long ng = (a.N + r - 1) / r, nt = ng * ((r + nb - 1) / nb);
+    return ks == 1 ||
+           (!a.g && nt * ks * P * 256 <= part_floats && ng <= ncnt);
   };
   // as many parts of K as it takes for X to fit
-  int ks = 1, nb = 16;
-  while (ks < 64 && !fits(ks, nb)) ks++;
-  // Narrow products: half tiles and more parts until the 256 CUs have a
-  // block each, or a part is down to 512.  (5 rows, 2048x8192: 128 blocks
-  // 12.0 us, 256 of half tiles 10.1.)
-  if ((a.N + 15) / 16 * ks < 192) {
-    nb = 8;
-    while (ks < 16 && (a.N + 7) / 8 * ks < 192 && a.K / (ks + 1) >= 512 &&
-           fits(ks + 1, nb)) ks++;
-  }
-  if (!fits(ks, nb)) return hipErrorInvalidValue;
+  int ks = 1;
+  while (ks < 64 && !fits(ks)) ks++;
+  // Narrow products: more parts until the 256 CUs have a block each, or a
+  // part is down to 512.  (5 rows, 2048x8192: 128 blocks 12.0 us, 256 of half
+  // tiles 10.1.)
+  while (ks < 16 && (a.N + share(ks) - 1) / share(ks) * ks < 192 &&
+         a.K / (ks + 1) >= 512 && fits(ks + 1))
+    ks++;
+  if (!fits(ks)) return hipErrorInvalidValue;
   a.kr = part_k(ks);
   ks = (a.K + a.kr - 1) / a.kr;
-  // A block a CU, walking tiles with X in place: two a CU read X twice and
-  // run no faster (5 rows, 2x8192x2048: 16.9 us, 512 blocks 21.1; 32768x3072
-  // 38.9 and 43.9).
-  const int nt = (a.N + nb - 1) / nb;
-  int ng = 256 / ks > 1 ? 256 / ks : 1;
-  if (ng > nt) ng = nt;
-  dim3 grid(ng, ks);
-  const size_t lds = lds_of(ks);
+  a.rpb = share(ks);
+  const int nb = tile_of(a.rpb), tiles = (a.rpb + nb - 1) / nb;
+  const dim3 grid((a.N + a.rpb - 1) / a.rpb, ks);
+  const size_t lds = lds_of(ks) + (size_t)(tiles + RG_NW - 1) * P * 1024;
   if (a.g) {
     if (nb == 8) rg_go<WT, 8, GLU, true>(a, grid, lds, s);
     else rg_go<WT, 16, GLU, true>(a, grid, lds, s);
@@ -476,7 +549,7 @@ extern "C" hipError_t launch_row_gemm(
   RgArgs a = {x, (const float*)sx, w, (const float*)ws, (const uint8_t*)we,
               (const float*)g, (const u16*)bias, (const u16*)res, y,
               (float*)part, (int*)cnt, M, N, K, ldx, ldr, ldy, act, out_f32,
-              0, eps, softcap};
+              0, 0, eps, softcap};
   if (!part || !cnt) part_floats = 0;
 #define RG_CASE(WTV)                                                         \
   return act >= 0 ? rg_run<WTV, true>(a, part_floats, ncnt, stream)          \

@@ -75,9 +75,10 @@ def mxfp4_values(q, e):
 
 
 # outputs: less than half a tile, a tile and a rest, more tiles than blocks;
-# K: one slab of 64, slabs that eight waves share unevenly, split over blocks
+# K: one slab of 64, slabs that eight waves share unevenly, split over blocks;
+# more outputs than LDS has room for the sums of beside 16 long rows
 @pytest.mark.parametrize("N,K", [(5, 64), (24, 192), (200, 320), (520, 8192),
-                                 (4616, 1088)])
+                                 (4616, 1088), (30000, 4608)])
 @pytest.mark.parametrize("M", [1, 7, 16])
 @pytest.mark.parametrize("kind", ["bf16", "fp8", "fp4"])
 @pytest.mark.parametrize("norm,act", [(False, -1), (True, -1), (False, 1),
