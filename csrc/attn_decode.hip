@@ -28,8 +28,7 @@
 // ranges (as before) -> here:
 //   32/8 heads of 64, 90 keys 7.6 -> 4.6; 4000 keys 22.2 -> 10.0
 //   32/8 of 128, 6040 e4m3 keys 39.2 -> 15.5; 160 keys 9.8 -> 6.4
-//   16/8 of 256, 16 sequences of 620 keys, softcap 52.3 -> 34.5 (two blocks of four waves a
-//     CU by registers, 384 blocks: a nearly empty last wave)
+//   16/8 of 256, 16 sequences of 620 keys, softcap 52.3 -> 25.4 (two ranges)
 //   64/8 of 128, 4 sequences of 2000 keys 97 -> 23
 //   16/4 of 128, 32000 keys 131 -> 38 (0.85 TB/s: few blocks, long ranges)
 //
@@ -454,9 +453,12 @@ k_attn_dec(AdArgs a) {
   const int pos = a.len[b];
   const int start = a.window > 0 ? max(0, pos + 1 - a.window) : 0;
   const int hist = pos - start;
-  // a tile for every wave of a block, more where the grid ends
+  // A tile for every wave of a block, more where the grid ends; one range as
+  // long as two rounds will do (345 keys of 128, 6 sequences: 8.9 us, two
+  // ranges and their merge 10.0).
   const int tiles = (hist + TK - 1) / TK;
-  const int eff = min(max(1, (tiles + NW - 1) / NW), (int)gridDim.y);
+  const int eff = tiles <= 2 * NW ? 1
+                                  : min((tiles + NW - 1) / NW, (int)gridDim.y);
   if (chunk >= eff) return;
   const int per = (tiles + eff - 1) / eff;
   const int c0 = start + chunk * per * TK, c1 = min(c0 + per * TK, pos);
