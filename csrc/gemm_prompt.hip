@@ -39,6 +39,11 @@ struct GpArgs {
   float* part;         // split K: [tile, split, BM*BN]
   int* cnt;            // split K: blocks of a tile that are done
   int M, N, K, act, tm, tn;
+  // Routed experts: a row tile has n[t] rows of expert e[t]; row r of it is
+  // pair perm[row0[t] + r].  x by token (a pair / top) and y in that order
+  // (gather), or x in that order and y by pair.
+  const int *perm, *tile_e, *tile_row0, *tile_n;
+  int top, gather;
 };
 
 DEVINL float gp_act(float x, int act) {
@@ -58,7 +63,8 @@ template <int N> DEVINL void gp_meet() {
   asm volatile("" ::: "memory");
 }
 
-template <bool F8, int BM, int BN, int WM, int WN, int NS, bool GLU>
+template <bool F8, int BM, int BN, int WM, int WN, int NS, bool GLU,
+          bool MOE = false>
 __global__ void __launch_bounds__(64 * WM * WN)
 k_gemm_prompt(GpArgs a) {
   constexpr int NW = WM * WN;
@@ -86,7 +92,19 @@ k_gemm_prompt(GpArgs a) {
   const int tiles = a.tm * a.tn, chunk = (tiles + 7) / 8;
   const int tile = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= chunk || tile >= tiles) return;
-  const int bm = tile % a.tm * BM, bn = tile / a.tm * (GLU ? BN / 2 : BN);
+  const int bm = MOE ? 0 : tile % a.tm * BM;
+  const int bn = tile / a.tm * (GLU ? BN / 2 : BN);
+  // the rows of a tile that are there
+  const int rows = MOE ? a.tile_n[tile % a.tm] : a.M;
+  if (MOE && rows == 0) return;
+  const int* perm = MOE ? a.perm + a.tile_row0[tile % a.tm] : nullptr;
+  const int first = MOE ? a.tile_row0[tile % a.tm] : 0;
+  const size_t w0 = MOE ? (size_t)a.tile_e[tile % a.tm] * (GLU ? 2 : 1) * a.N
+                        : 0;                 // first row of the expert's W
+  auto x_row = [&](int r) {
+    if (!MOE) return r;
+    return a.gather ? perm[r] / a.top : first + r;
+  };
 
   const size_t rowb = (size_t)a.K * (F8 ? 1 : 2);       // bytes of a row
   const int slabs = (int)((rowb + 127) / 128);
@@ -101,7 +119,7 @@ k_gemm_prompt(GpArgs a) {
 #pragma unroll
   for (int i = 0; i < AI; i++) {
     const int r = (wave * AI + i) * 8 + g_r;
-    pa[i] = (const char*)a.x + (size_t)min(bm + r, a.M - 1) * rowb;
+    pa[i] = (const char*)a.x + (size_t)x_row(min(bm + r, rows - 1)) * rowb;
   }
 #pragma unroll
   for (int i = 0; i < BI; i++) {
@@ -113,7 +131,7 @@ k_gemm_prompt(GpArgs a) {
     } else {
       row = min(bn + r, a.N - 1);
     }
-    pb[i] = (const char*)a.w + row * rowb;
+    pb[i] = (const char*)a.w + (w0 + row) * rowb;
   }
   // row r of a tile keeps slot q at q ^ ((r >> 1) & 7)
   const int src0 = (g_s ^ (g_r >> 1)) * 16, src1 = src0 ^ 64;
@@ -323,9 +341,10 @@ k_gemm_prompt(GpArgs a) {
   const bool wide = a.N % 4 == 0;
 #pragma unroll
   for (int i = 0; i < FM; i++) {
-    const int row = bm + (wm * FM + i) * 16 + fr;
-    if (row >= a.M) continue;
-    const float sx = F8 ? a.sx[row] : 1.f;
+    const int r_in = bm + (wm * FM + i) * 16 + fr;
+    if (r_in >= rows) continue;
+    const float sx = F8 ? a.sx[x_row(r_in)] : 1.f;
+    const int row = !MOE ? r_in : a.gather ? first + r_in : perm[r_in];
 #pragma unroll
     for (int j = 0; j < FN; j += P) {
       const int n = bn + (wn * FN + j) / P * 16 + fk * 4;
@@ -333,13 +352,18 @@ k_gemm_prompt(GpArgs a) {
       f4v v = acc[i][j];
       if (F8) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) v[r] *= sx * a.sw[min(n + r, a.N - 1)];
+        for (int r = 0; r < 4; r++) v[r] *= sx * a.sw[w0 + min(n + r, a.N - 1)];
       }
       if constexpr (GLU) {
         f4v u = acc[i][j + 1];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-          if (F8) u[r] *= sx * a.sw[a.N + min(n + r, a.N - 1)];
+          if (F8) {
+            // to be rounded to e4m3 next, where a value's last bits decide
+            // which of two it takes: from bf16 halves, as by single launches
+            u[r] = b2f(f2b(u[r] * sx * a.sw[w0 + a.N + min(n + r, a.N - 1)]));
+            v[r] = b2f(f2b(v[r]));
+          }
           v[r] = gp_act(v[r], a.act) * u[r];
         }
       }
@@ -465,8 +489,155 @@ extern "C" hipError_t launch_gemm_prompt(
     return hipErrorInvalidValue;
   GpArgs a = {x, w, (const float*)sx, (const float*)sw, (const u16*)res,
               (const u16*)bias, (u16*)y, (float*)part, (int*)cnt, M, N, K,
-              act, 0, 0};
+              act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
   if (!part || !cnt) part_floats = 0;
   return sx ? gp_run<true>(a, part_floats, ncnt, stream)
             : gp_run<false>(a, part_floats, ncnt, stream);
+}
+
+// ---- routed experts --------------------------------------------------------
+// Every expert used to take all rows, E/top times the work, with a launch a
+// product and one to add: 16 products and 8 sums a layer for eight experts.
+// Here the pairs of a row and a choice are sorted by expert on the device, a
+// row tile belongs to one expert, and each product is one launch (a tile more
+// than there may be an expert is launched and leaves).  1100 rows, eight
+// experts of 2x4096x2048, two a row, and 24 steps: 5.17 -> 4.00 ms.
+//
+// One block: pairs (token, choice) by expert, and the row tiles of each.
+// Pairs of an expert may come in any order: a row's result does not depend on
+// its place.
+__global__ void __launch_bounds__(1024)
+k_expert_sort(const int* __restrict__ idx, int* __restrict__ perm,
+              int* __restrict__ tile_e, int* __restrict__ tile_row0,
+              int* __restrict__ tile_n, int pairs, int E, int bm,
+              int maxtiles) {
+  __shared__ int cnt[64], start[65], tile0[65];
+  const int tid = threadIdx.x;
+  if (tid < E) cnt[tid] = 0;
+  __syncthreads();
+  for (int p = tid; p < pairs; p += 1024) atomicAdd(&cnt[idx[p]], 1);
+  __syncthreads();
+  if (tid == 0) {
+    int s = 0, t = 0;
+    for (int e = 0; e < E; e++) {
+      start[e] = s;
+      tile0[e] = t;
+      s += cnt[e];
+      t += (cnt[e] + bm - 1) / bm;
+    }
+    start[E] = s;
+    tile0[E] = t;
+  }
+  __syncthreads();
+  for (int t = tid; t < maxtiles; t += 1024) {
+    int e = 0, n = 0, r0 = 0;
+    if (t < tile0[E]) {
+      while (t >= tile0[e + 1]) e++;
+      r0 = start[e] + (t - tile0[e]) * bm;
+      n = min(bm, start[e + 1] - r0);
+    }
+    tile_e[t] = e;
+    tile_row0[t] = r0;
+    tile_n[t] = n;
+  }
+  __syncthreads();
+  if (tid < E) cnt[tid] = 0;
+  __syncthreads();
+  for (int p = tid; p < pairs; p += 1024) {
+    const int e = idx[p];
+    perm[start[e] + atomicAdd(&cnt[e], 1)] = p;
+  }
+}
+
+// h[t] += w[t, j] y[t, j], 8 elements a thread: one expert after the other, h
+// bf16 between them, as when each expert's result was a launch of its own
+__global__ void __launch_bounds__(256)
+k_expert_sum(const u16* __restrict__ y, const float* __restrict__ w,
+             const int* __restrict__ idx, u16* __restrict__ h, int top,
+             int H) {
+  const int t = blockIdx.y, i = (blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= H) return;
+  const size_t p0 = (size_t)t * top;
+  s8v hv = *(const s8v*)(h + (size_t)t * H + i);
+  for (int n = 0, last = -1; n < top; n++) {
+    int j = -1;                              // the next expert
+    for (int q = 0; q < top; q++)
+      if (idx[p0 + q] > last && (j < 0 || idx[p0 + q] < idx[p0 + j])) j = q;
+    if (j < 0) break;
+    last = idx[p0 + j];
+    const s8v v = *(const s8v*)(y + (p0 + j) * H + i);
+    const float s = w[p0 + j];
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+      ((u16*)&hv)[k] = f2b(b2f(((u16*)&hv)[k]) + s * b2f(((u16*)&v)[k]));
+  }
+  *(s8v*)(h + (size_t)t * H + i) = hv;
+}
+
+// rows of a tile: what an expert gets on average, or more (278 rows each:
+// 128; with 64 W is read twice as often)
+static int expert_bm(int pairs, int E) {
+  const int mean = pairs / E;
+  return mean >= 96 ? 128 : mean >= 24 ? 64 : 32;
+}
+
+extern "C" hipError_t launch_expert_sort(const void* idx, void* sorted,
+                                         int pairs, int E, long room,
+                                         hipStream_t stream) {
+  const int bm = expert_bm(pairs, E), tiles = pairs / bm + E;
+  if (pairs < 1 || E < 1 || E > 64 || room < pairs + 3L * tiles)
+    return hipErrorInvalidValue;
+  int* p = (int*)sorted;
+  hipLaunchKernelGGL(k_expert_sort, dim3(1), dim3(1024), 0, stream,
+                     (const int*)idx, p, p + pairs, p + pairs + tiles,
+                     p + pairs + 2 * tiles, pairs, E, bm, tiles);
+  return hipGetLastError();
+}
+
+template <bool F8, int BM, int BN, int WM, int WN, int NS>
+static hipError_t gp_experts(GpArgs a, hipStream_t s) {
+  const int wide = a.act >= 0 ? BN / 2 : BN;
+  a.tn = (a.N + wide - 1) / wide;
+  const dim3 grid((a.tm * a.tn + 7) / 8 * 8), nt(64 * WM * WN);
+  if (a.act >= 0)
+    hipLaunchKernelGGL((k_gemm_prompt<F8, BM, BN, WM, WN, NS, true, true>),
+                       grid, nt, 0, s, a);
+  else
+    hipLaunchKernelGGL((k_gemm_prompt<F8, BM, BN, WM, WN, NS, false, true>),
+                       grid, nt, 0, s, a);
+  return hipGetLastError();
+}
+
+// y = x W^T of each pair's expert.  sorted: of launch_expert_sort.  gather: x
+// by token, y in the sorted order; else x in that order, y by pair.
+extern "C" hipError_t launch_expert_gemm(
+    const void* x, const void* w, const void* sx, const void* sw, void* y,
+    const void* sorted, int pairs, int E, int top, int gather, int N, int K,
+    int act, hipStream_t stream) {
+  if (pairs < 1 || E < 1 || E > 64 || top < 1 || pairs % top || N < 1 ||
+      K < 64 || K % 64 || (!sx != !sw))
+    return hipErrorInvalidValue;
+  const int bm = expert_bm(pairs, E), tiles = pairs / bm + E;
+  const int* p = (const int*)sorted;
+  GpArgs a = {x, w, (const float*)sx, (const float*)sw, nullptr, nullptr,
+              (u16*)y, nullptr, nullptr, pairs, N, K, act, tiles, 0, p,
+              p + pairs, p + pairs + tiles, p + pairs + 2 * tiles, top,
+              gather};
+#define EXPERTS(F8)                                                          \
+  return bm == 128  ? gp_experts<F8, 128, 128, 2, 4, 4>(a, stream)           \
+         : bm == 64 ? gp_experts<F8, 64, 64, 2, 2, 4>(a, stream)             \
+                    : gp_experts<F8, 32, 64, 2, 2, 6>(a, stream)
+  if (sx) EXPERTS(true);
+  EXPERTS(false);
+#undef EXPERTS
+}
+
+extern "C" hipError_t launch_expert_sum(const void* y, const void* w,
+                                        const void* idx, void* h, int M,
+                                        int top, int H, hipStream_t stream) {
+  if (M < 1 || top < 1 || H < 8 || H % 8) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_expert_sum, dim3((H / 8 + 255) / 256, M), dim3(256), 0,
+                     stream, (const u16*)y, (const float*)w, (const int*)idx, (u16*)h, top,
+                     H);
+  return hipGetLastError();
 }

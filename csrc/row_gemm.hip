@@ -30,6 +30,8 @@
 // the MFMA operand, since the order of k is free as long as X agrees.
 // MXFP4 weights are widened to bf16 in registers (exact) beside a bf16 X;
 // e4m3 weights meet rows of X rounded to e4m3, as in the prompt's products.
+#include <type_traits>
+
 #include "common.h"
 
 typedef __bf16 rg_b8 __attribute__((ext_vector_type(8)));
@@ -50,6 +52,7 @@ struct RgArgs {
   int* cnt;            // split K: blocks of a column group that are done
   int M, N, K, ldx, ldr, ldy, act, out_f32, kr;
   int rpb;             // outputs of a block
+  int n16;             // NORM 2
   float eps, softcap;
 };
 
@@ -97,8 +100,9 @@ DEVINL float rg_act(float x, int act) {
 #define RG_NW 8
 #define RG_NORM_K 4096     // the longest row that is normed on the way
 
-// NB: outputs of a tile (8: half of an MFMA tile).
-template <int WT, int NB, bool GLU, bool NORM>
+// NB: outputs of a tile (8: half of an MFMA tile).  NORM 2: to bf16 before
+// e4m3, like a prompt's rows (a choice in the loop cost 16 rows 2 us).
+template <int WT, int NB, bool GLU, int NORM>
 __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
   constexpr int E = RgT<WT>::E, SE = 8 * E;  // elements of a chunk, a slab
   constexpr int XF = E / 8;                  // fragments of a chunk
@@ -198,7 +202,7 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
 
   // X into LDS, zeros behind K.  Its loads go out ahead of W's: they come
   // from L2 and return first, and loads return in order.
-  if constexpr (NORM) {
+  if constexpr (NORM > 0) {
     s8v v[2][RG_NORM_K / 512];
     rg_f4 g[RG_NORM_K / 512][2];
 #pragma unroll
@@ -230,7 +234,8 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
           }
       const float rn = rsqrtf(wave_reduce_sum(ss) / (float)a.K + a.eps);
       auto normed = [&](int j, int q) {
-        return b2f(((u16*)&v[i][j])[q]) * rn * g[j][q / 4][q % 4];
+        const float f = b2f(((u16*)&v[i][j])[q]) * rn * g[j][q / 4][q % 4];
+        return NORM == 2 ? b2f(f2b(f)) : f;
       };
       float am = 1.f;
       if constexpr (WT == RG_FP8) {          // rows rounded to e4m3
@@ -470,7 +475,7 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
 
 #define RG_ROOM (159 * 1024)     // LDS of a block: X and the sums
 
-template <int WT, int NB, bool GLU, bool NORM>
+template <int WT, int NB, bool GLU, int NORM>
 static void rg_go(const RgArgs& a, dim3 grid, size_t lds, hipStream_t s) {
   static const hipError_t raised = hipFuncSetAttribute(
       (const void*)&k_row_gemm<WT, NB, GLU, NORM>,
@@ -525,13 +530,13 @@ static hipError_t rg_run(RgArgs a, long part_floats, int ncnt,
   const int nb = tile_of(a.rpb), tiles = (a.rpb + nb - 1) / nb;
   const dim3 grid((a.N + a.rpb - 1) / a.rpb, ks);
   const size_t lds = lds_of(ks) + (size_t)(tiles + RG_NW - 1) * P * 1024;
-  if (a.g) {
-    if (nb == 8) rg_go<WT, 8, GLU, true>(a, grid, lds, s);
-    else rg_go<WT, 16, GLU, true>(a, grid, lds, s);
-  } else {
-    if (nb == 8) rg_go<WT, 8, GLU, false>(a, grid, lds, s);
-    else rg_go<WT, 16, GLU, false>(a, grid, lds, s);
-  }
+  auto go = [&](auto norm) {
+    if (nb == 8) rg_go<WT, 8, GLU, decltype(norm)::value>(a, grid, lds, s);
+    else rg_go<WT, 16, GLU, decltype(norm)::value>(a, grid, lds, s);
+  };
+  if (!a.g) go(std::integral_constant<int, 0>());
+  else if (WT != RG_FP8 || !a.n16) go(std::integral_constant<int, 1>());
+  else go(std::integral_constant<int, WT == RG_FP8 ? 2 : 1>());
   return hipGetLastError();
 }
 
@@ -540,7 +545,7 @@ extern "C" hipError_t launch_row_gemm(
     const void* x, const void* sx, const void* w, const void* ws,
     const void* we, const void* g, const void* bias, const void* res, void* y, void* part,
     void* cnt, long part_floats, int ncnt, int wt, int M, int N, int K,
-    int ldx, int ldr, int ldy, int act, int out_f32, float eps,
+    int ldx, int ldr, int ldy, int act, int out_f32, int n16, float eps,
     float softcap, hipStream_t stream) {
   if (M < 1 || M > 16 || N < 1 || K < 64 || K % 64 || ldx < K || ldx % (wt == RG_FP8 && !g ? 16 : 8) ||
       ldy < N || (res && ldr < N) || (g && K > RG_NORM_K) ||
@@ -549,7 +554,7 @@ extern "C" hipError_t launch_row_gemm(
   RgArgs a = {x, (const float*)sx, w, (const float*)ws, (const uint8_t*)we,
               (const float*)g, (const u16*)bias, (const u16*)res, y,
               (float*)part, (int*)cnt, M, N, K, ldx, ldr, ldy, act, out_f32,
-              0, 0, eps, softcap};
+              0, 0, n16, eps, softcap};
   if (!part || !cnt) part_floats = 0;
 #define RG_CASE(WTV)                                                         \
   return act >= 0 ? rg_run<WTV, true>(a, part_floats, ncnt, stream)          \

@@ -327,7 +327,9 @@ class GPUModel(DecodeLoop):
         self.b_rqkv = torch.zeros(PC, (self.nh_l + 2 * self.kvh_l) * hd,
                                   **bf)
         self.b_att = torch.zeros(PC, self.nh_l * hd, **bf)
-        self.b_gate = torch.zeros(PC, I, **bf)
+        # act(gate) * up; of each of a row's experts
+        pairs = PC * (self.topk if self.moe else 1)
+        self.b_gate = torch.zeros(pairs, I, **bf)
         if self.wq4:          # its prompts have gate and up apart
             self.b_up = torch.zeros(PC, I, **bf)
         self.b_gemm_acc = torch.zeros(PC * max(I, H), dtype=torch.float32,
@@ -338,8 +340,10 @@ class GPUModel(DecodeLoop):
             self.b_xq = torch.zeros(PC * kmax, dtype=torch.uint8, device=dev)
             self.b_sx = torch.zeros(PC, dtype=torch.float32, device=dev)
             if self.moe:
-                self.b_aq = torch.zeros(PC * I, dtype=torch.uint8, device=dev)
-                self.b_sa = torch.zeros(PC, dtype=torch.float32, device=dev)
+                self.b_aq = torch.zeros(pairs * I, dtype=torch.uint8,
+                                        device=dev)
+                self.b_sa = torch.zeros(pairs, dtype=torch.float32,
+                                        device=dev)
             # act(gate) * up of few rows, to be rounded to e4m3 next
             self.b_act32 = torch.zeros(ho.FEW_ROWS, I, dtype=torch.float32,
                                        device=dev)
@@ -360,8 +364,9 @@ class GPUModel(DecodeLoop):
                                        device=dev)
             self.moe_w = torch.zeros(PC * self.topk, dtype=torch.float32,
                                      device=dev)
-            self.moe_dense = torch.zeros(PC * E, dtype=torch.float32,
-                                         device=dev)
+            self.moe_order = torch.zeros(pairs + 3 * (pairs // 32 + E),
+                                         dtype=torch.int32, device=dev)
+            self.b_pairs = torch.zeros(pairs, H, **bf)
         self.b_hb = torch.zeros(H, **bf)   # gemma residual ping-pong
         self.b_t2 = torch.zeros(H, **bf)   # gemma ffn-out delta
         # act(gate) * up of a decode step (of each expert): fp32 beside
@@ -471,7 +476,9 @@ class GPUModel(DecodeLoop):
                 K = x.shape[-1]
                 ho.quant_fp8(x[:M], self.b_xq, self.b_sx)
                 x, kw["sx"] = self.b_xq[:M * K].view(M, K), self.b_sx
-            ho.row_gemm(x, lw[name + "_q"], y, M, ws=lw[name + "_s"], **kw)
+            # a prompt's rows are bf16 on their way to e4m3, a step's fp32
+            ho.row_gemm(x, lw[name + "_q"], y, M, ws=lw[name + "_s"],
+                        norm16=not batch, **kw)
         elif self.wq4:
             ho.row_gemm(x, lw[name + "_q4"], y, M, we=lw[name + "_e4"], **kw)
         else:
@@ -637,7 +644,7 @@ class GPUModel(DecodeLoop):
             else:
                 a = self.b_gate
                 if few:
-                    if 1 < M and self.fp8 and (batch_attn or not self.wq4):
+                    if 1 < M and self.fp8 and batch_attn:
                         a = self.b_act32
                     self._rows(lw, "wgu", h, a, M, g=g_mlp, act=self.act,
                                batch=batch_attn)
@@ -652,37 +659,34 @@ class GPUModel(DecodeLoop):
                 layer_hook(i, h[:M])
 
     def _moe_mlp_rows(self, lw, M: int):
-        """Prefill/batch MoE MLP over rows [0, M): router weights per
-        row (dense M x E grid), then ONE GEMM pass per expert with the
-        output folded into h weighted by that row's prob (0 if
-        unrouted).  Work is E/topk x the routed minimum — prefill is
-        compute-rich and this keeps the MFMA GEMM path; decode uses the
-        expert-indexed GEMVs instead (`_decode_step`)."""
+        """Prefill/batch MoE MLP over rows [0, M): the router's choices,
+        sorted by expert on the device, then both products over each
+        expert's own rows, and a row's results weighted into h; decode
+        multiplies by the chosen experts directly (`_decode_step`)."""
         cfg = self.config
-        E, I, H = cfg.num_local_experts, self.inter_l, self.H
-        eps = cfg.rms_norm_eps
-        xn, gate, t1 = self.b_xn, self.b_gate, self.b_t1
-        ho.moe_route(self.b_h, lw["g_post"], lw["wg"], M, self.topk,
-                     self.moe_idx, self.moe_w, dense=self.moe_dense,
-                     eps=eps)
-        kw = dict(accbuf=self.b_gemm_acc, cnt=self.tile_cnt)
+        E, I, H, top = (cfg.num_local_experts, self.inter_l, self.H,
+                        self.topk)
+        pairs = M * top
+        a, order = self.b_gate[:pairs], self.moe_order
+        ho.moe_route(self.b_h, lw["g_post"], lw["wg"], M, top,
+                     self.moe_idx, self.moe_w, eps=cfg.rms_norm_eps)
+        ho.expert_sort(self.moe_idx, order, pairs, E)
         if self.fp8:
-            ho.quant_fp8(xn[:M], self.b_xq, self.b_sx)
-        for e in range(E):
-            gu, dn = slice(e * 2 * I, (e + 1) * 2 * I), \
-                slice(e * H, (e + 1) * H)
-            if self.fp8:
-                ho.gemm_fp8(self.b_xq, self.b_sx, lw["wgu_q_all"][gu],
-                            lw["wgu_s_all"][gu], gate[:M], M, H,
-                            act=self.act, **kw)
-                ho.quant_fp8(gate[:M], self.b_aq, self.b_sa)
-                ho.gemm_fp8(self.b_aq, self.b_sa, lw["wdown_q_all"][dn],
-                            lw["wdown_s_all"][dn], t1[:M], M, I, **kw)
-            else:
-                ho.gemm(xn[:M], lw["wgu_all"][gu], gate[:M], act=self.act,
-                        **kw)
-                ho.gemm(gate[:M], lw["wdown_all"][dn], t1[:M], **kw)
-            ho.moe_scale_add(self.b_h, t1, self.moe_dense[e:], E, M, H)
+            ho.quant_fp8(self.b_xn[:M], self.b_xq, self.b_sx)
+            ho.expert_gemm(self.b_xq, lw["wgu_q_all"], a, order, pairs, E,
+                           top, H, True, act=self.act, sx=self.b_sx,
+                           sw=lw["wgu_s_all"])
+            ho.quant_fp8(a, self.b_aq, self.b_sa)
+            ho.expert_gemm(self.b_aq, lw["wdown_q_all"], self.b_pairs, order,
+                           pairs, E, top, I, False, sx=self.b_sa,
+                           sw=lw["wdown_s_all"])
+        else:
+            ho.expert_gemm(self.b_xn, lw["wgu_all"], a, order, pairs, E, top,
+                           H, True, act=self.act)
+            ho.expert_gemm(a, lw["wdown_all"], self.b_pairs, order, pairs, E,
+                           top, I, False)
+        ho.expert_sum(self.b_pairs, self.moe_w, self.moe_idx, self.b_h, M,
+                      top)
 
     @property
     def _head(self):

@@ -56,7 +56,7 @@ _SIGS = {
     "launch_gemm_prompt": [ctypes.c_void_p] * 9 + [ctypes.c_long] +
                           [ctypes.c_int] * 5 + [ctypes.c_void_p],
     "launch_row_gemm": [ctypes.c_void_p] * 11 + [ctypes.c_long] +
-                       [ctypes.c_int] * 10 +
+                       [ctypes.c_int] * 11 +
                        [ctypes.c_float, ctypes.c_float, ctypes.c_void_p],
     "launch_prefetch": [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p,
                         ctypes.c_void_p],
@@ -83,6 +83,12 @@ _SIGS = {
                         [ctypes.c_void_p],
     "launch_moe_route": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4 +
                         [ctypes.c_float] + [ctypes.c_void_p] * 4,
+    "launch_expert_sort": [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2 +
+                          [ctypes.c_long, ctypes.c_void_p],
+    "launch_expert_gemm": [ctypes.c_void_p] * 6 + [ctypes.c_int] * 7 +
+                          [ctypes.c_void_p],
+    "launch_expert_sum": [ctypes.c_void_p] * 4 + [ctypes.c_int] * 3 +
+                         [ctypes.c_void_p],
     "launch_moe_scale_add": [ctypes.c_void_p] * 3 +
                             [ctypes.c_long, ctypes.c_int, ctypes.c_int,
                              ctypes.c_void_p],
@@ -376,12 +382,13 @@ def row_gemm(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, M: int,
              res: torch.Tensor | None = None, act: int = -1,
              softcap: float = 0.0, part: torch.Tensor | None = None,
              cnt: torch.Tensor | None = None,
-             sx: torch.Tensor | None = None):
+             sx: torch.Tensor | None = None, norm16: bool = False):
     """Y[M<=16, N] = X W^T for few rows of x (2-D, rows may be apart), W
     streamed once: bf16, e4m3 (ws: row scales) or MXFP4 (we: exponents).
     x is bf16; beside e4m3 weights its rows are rounded to e4m3: by the
     caller (x bytes, sx scales), or after the norm that is taken here.
-    g: RMSNorm of x on the way (K <= ROW_NORM_K).  act 0/1: w holds gate
+    g: RMSNorm of x on the way (K <= ROW_NORM_K; norm16: rounded to bf16
+    before e4m3).  act 0/1: w holds gate
     rows, then up rows, and Y = act(gate) * up.  Then softcap, bias, res.
     part (fp32) and cnt (int32, zero; left zero) let K be split."""
     wt = 1 if ws is not None else 2 if we is not None else 0
@@ -397,8 +404,8 @@ def row_gemm(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, M: int,
         ctypes.c_long(0 if part is None else part.numel()),
         0 if cnt is None else cnt.numel(), wt, M, N, K, x.stride(0),
         res.stride(0) if res is not None else 0, y.stride(0), act,
-        1 if y.dtype == torch.float32 else 0, ctypes.c_float(eps), ctypes.c_float(softcap), _stream()),
-        "row_gemm")
+        1 if y.dtype == torch.float32 else 0, int(norm16),
+        ctypes.c_float(eps), ctypes.c_float(softcap), _stream()), "row_gemm")
 
 
 def quant_fp8(x: torch.Tensor, q: torch.Tensor, s: torch.Tensor):
@@ -606,6 +613,35 @@ def moe_route(h: torch.Tensor, g: torch.Tensor, wg: torch.Tensor, M: int,
     _check(lib().launch_moe_route(
         _ptr(h), _ptr(g), _ptr(wg), M, H, E, topk, ctypes.c_float(eps),
         _ptr(idx), _ptr(w), _ptr(dense), _stream()), "moe_route")
+
+
+def expert_sort(idx: torch.Tensor, out: torch.Tensor, pairs: int, E: int):
+    """Pairs (token, choice) by expert and the row tiles of each, for
+    expert_gemm; out: int32, pairs * 1.2 + 4 E + 64 will do."""
+    _check(lib().launch_expert_sort(
+        _ptr(idx), _ptr(out), pairs, E, ctypes.c_long(out.numel()),
+        _stream()), "expert_sort")
+
+
+def expert_gemm(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor,
+                order: torch.Tensor, pairs: int, E: int, top: int, K: int,
+                gather: bool, act: int = -1, sx: torch.Tensor | None = None,
+                sw: torch.Tensor | None = None):
+    """Each pair's row times its expert's W (w: experts one after the
+    other; act: gate and up rows).  gather: x by token, y in ``order``; else
+    x in ``order``, y by pair.  sx/sw: e4m3 rows and weights."""
+    N = w.shape[0] // E // (2 if act >= 0 else 1)
+    _check(lib().launch_expert_gemm(
+        _ptr(x), _ptr(w), _ptr(sx), _ptr(sw), _ptr(y), _ptr(order), pairs, E,
+        top, int(gather), N, K, act, _stream()), "expert_gemm")
+
+
+def expert_sum(y: torch.Tensor, w: torch.Tensor, idx: torch.Tensor,
+               h: torch.Tensor, M: int, top: int):
+    """h[t] += w[t, j] * y[t, j] over a token's choices, by expert."""
+    _check(lib().launch_expert_sum(
+        _ptr(y), _ptr(w), _ptr(idx), _ptr(h), M, top, h.shape[-1], _stream()),
+        "expert_sum")
 
 
 def moe_scale_add(y: torch.Tensor, x: torch.Tensor, w: torch.Tensor,

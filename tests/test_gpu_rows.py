@@ -156,6 +156,8 @@ def test_many_rows(M, N, K, kind, act):
             ho.gemm(X, W, Y[:M], **kw)
     z = x @ Wd.T
     if act >= 0:
+        if kind == "fp8":               # bf16 halves on their way to e4m3
+            z = z.bfloat16().double()
         f = (torch.nn.functional.silu if act == 0 else lambda t:
              torch.nn.functional.gelu(t, approximate="tanh"))
         z = f(z[:, :N]) * z[:, N:]
@@ -348,3 +350,60 @@ def test_two_norms(M, H):
     assert off(y[:M], rms(x.double()) * g.double() + h.double()) < 2.0 ** -8
     assert off(z[:M], rms(y[:M].double()) * g2.double()) < 2.0 ** -8
     assert (y[M] == 7.0).all() and (z[M] == 7.0).all()
+
+
+# rows of an expert: none, one, less and more than a tile of 32, 64 and 128
+@pytest.mark.parametrize("M,E,top", [(1, 8, 2), (40, 8, 3), (200, 9, 2),
+                                     (330, 4, 2), (70, 64, 8)])
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+def test_experts_of_many_rows(M, E, top, kind):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    H, I = 192, 320
+    up, dn = (normal(E * r, k, seed=s, scale=k ** -0.5)
+              for r, k, s in ((2 * I, H, 1), (H, I, 2)))
+    x, h = normal(M, H, seed=3), normal(M, H, seed=4)
+    r = torch.rand(M, E, generator=torch.Generator().manual_seed(5))
+    r[:, E - 1] *= 0.01                             # hardly ever taken
+    idx = r.topk(top, 1).indices.int().cuda().contiguous()
+    p = torch.rand(M, top, generator=torch.Generator().manual_seed(6)).cuda()
+    pairs = M * top
+    order = torch.full((pairs + 3 * (pairs // 32 + E),), -1,
+                       dtype=torch.int32, device="cuda")
+    a = torch.full((pairs + 1, I), 7.0, device="cuda").bfloat16()
+    y = torch.full((pairs + 1, H), 7.0, device="cuda").bfloat16()
+    ho.expert_sort(idx, order, pairs, E)
+    perm = order[:pairs].long()
+    who = idx.reshape(-1).long()
+    assert (perm.sort().values == torch.arange(pairs, device="cuda")).all()
+    assert (who[perm].diff() >= 0).all()
+    if kind == "fp8":
+        (uq, us, U), (dq, ds, D), (xq, xs, X) = e4m3(up), e4m3(dn), e4m3(x)
+        ho.expert_gemm(xq, uq, a[:pairs], order, pairs, E, top, H, True,
+                       act=0, sx=xs, sw=us)
+        aq, sa, ad = e4m3(a[:pairs])
+        ho.expert_gemm(aq, dq, y[:pairs], order, pairs, E, top, I, False,
+                       sx=sa, sw=ds)
+    else:
+        U, D, X = up.double(), dn.double(), x.double()
+        ho.expert_gemm(x, up, a[:pairs], order, pairs, E, top, H, True, act=0)
+        ho.expert_gemm(a[:pairs], dn, y[:pairs], order, pairs, E, top, I,
+                       False)
+        ad = a[:pairs].double()
+    out = h.clone()
+    ho.expert_sum(y, p, idx, out, M, top)
+    U, D = U.view(E, 2 * I, H), D.view(E, H, I)
+    za, zy = torch.zeros_like(ad), torch.zeros(pairs, H, device="cuda").double()
+    for e in range(E):
+        at = (who[perm] == e).nonzero()[:, 0]       # places in the order
+        t = X[perm[at] // top] @ U[e].T
+        if kind == "fp8":
+            t = t.bfloat16().double()
+        za[at] = torch.nn.functional.silu(t[:, :I]) * t[:, I:]
+        zy[perm[at]] = ad[at] @ D[e].T
+    # exact products, fp32 sums, bf16 results: 2^-8 of each value at most
+    assert off(a[:pairs], za) < 2.0 ** -8 and off(y[:pairs], zy) < 2.0 ** -8
+    z = h.double() + (y[:pairs].double().view(M, top, H)
+                      * p.double()[..., None]).sum(1)
+    assert off(out, z) < 2.0 ** -8 * top            # bf16 after each expert
+    assert (a[pairs] == 7.0).all() and (y[pairs] == 7.0).all()
