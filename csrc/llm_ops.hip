@@ -844,7 +844,10 @@ DEVINL int unpack_idx(uint64_t p) { return 0x7fffffff - (int)(uint32_t)p; }
 // pass 1 (min-p only): global max logit -> gmax[b] (packed).
 // Batched: grid.y = sequence row b (lbf16: logits stored bf16 — the
 // batched lm_head GEMM path emits bf16 rows).
-extern "C" __global__ void __launch_bounds__(256)
+#define SMP_NT 512      // threads of a block
+#define SMP_U 4         // logits of a thread at a time
+
+extern "C" __global__ void __launch_bounds__(SMP_NT)
 k_logit_max(const void* __restrict__ logits, int V, int lbf16,
             unsigned long long* __restrict__ gmax,
             uint64_t* __restrict__ ctr) {
@@ -858,9 +861,19 @@ k_logit_max(const void* __restrict__ logits, int V, int lbf16,
   const u16* lh = (const u16*)logits + (size_t)b * V;
   float mv = -INFINITY;
   int mi = 0;
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < V; i += gridDim.x * 256) {
-    float v = lbf16 ? b2f(lh[i]) : lf[i];
-    if (v > mv || (v == mv && i < mi)) { mv = v; mi = i; }
+  for (int i0 = blockIdx.x * SMP_NT * SMP_U + threadIdx.x; i0 < V;
+       i0 += gridDim.x * SMP_NT * SMP_U) {
+    float v[SMP_U];
+#pragma unroll
+    for (int u = 0; u < SMP_U; u++) {
+      const int i = min(i0 + u * SMP_NT, V - 1);
+      v[u] = lbf16 ? b2f(lh[i]) : lf[i];
+    }
+#pragma unroll
+    for (int u = 0; u < SMP_U; u++) {
+      const int i = min(i0 + u * SMP_NT, V - 1);
+      if (v[u] > mv || (v[u] == mv && i < mi)) { mv = v[u]; mi = i; }
+    }
   }
   uint64_t pk = pack_ki(fkey(mv), mi);
 #pragma unroll
@@ -868,12 +881,12 @@ k_logit_max(const void* __restrict__ logits, int V, int lbf16,
     uint64_t o = __shfl_xor((unsigned long long)pk, w);
     if (o > pk) pk = o;
   }
-  __shared__ unsigned long long ws[4];
+  __shared__ unsigned long long ws[SMP_NT / 64];
   if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = pk;
   __syncthreads();
   if (threadIdx.x == 0) {
     uint64_t b = ws[0];
-    for (int w = 1; w < 4; w++) if (ws[w] > b) b = ws[w];
+    for (int w = 1; w < SMP_NT / 64; w++) if (ws[w] > b) b = ws[w];
     atomicMax(gmax, (unsigned long long)b);
   }
 }
@@ -885,7 +898,7 @@ k_logit_max(const void* __restrict__ logits, int V, int lbf16,
 // Temperature folds into both the min-p keep-set and the Gumbel score:
 //   p_i(T) >= min_p * p_max(T)  <=>  l_i >= l_max + T*ln(min_p)
 //   Gumbel-argmax over p(T)     <=>  argmax of l_i/T + G_i
-extern "C" __global__ void __launch_bounds__(256)
+extern "C" __global__ void __launch_bounds__(SMP_NT)
 k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
               long ring_stride, float min_p,
               int greedy, uint64_t seed, float inv_temp,
@@ -906,17 +919,28 @@ k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
   const uint32_t c = (uint32_t)(*ctr) ^ ((uint32_t)b * 0x85ebca6bu);
   float bv = -INFINITY;
   int bi = 0x7fffffff;
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < V; i += gridDim.x * 256) {
-    float v = lbf16 ? b2f(lh[i]) : lf[i];
-    if (v < thresh) continue;
-    float sc = v;
-    if (!greedy) {
-      uint32_t r = hash32(hash32((uint32_t)i ^ (c * 0x9e3779b9u)) ^
-                          (uint32_t)seed);
-      float u = (r + 1.0f) * 2.3283064e-10f;  // (0,1]
-      sc = v * inv_temp - __logf(-__logf(u));
+  for (int i0 = blockIdx.x * SMP_NT * SMP_U + threadIdx.x; i0 < V;
+       i0 += gridDim.x * SMP_NT * SMP_U) {
+    float vs[SMP_U];
+#pragma unroll
+    for (int u = 0; u < SMP_U; u++) {
+      const int i = min(i0 + u * SMP_NT, V - 1);
+      vs[u] = lbf16 ? b2f(lh[i]) : lf[i];
     }
-    if (sc > bv || (sc == bv && i < bi)) { bv = sc; bi = i; }
+#pragma unroll
+    for (int u = 0; u < SMP_U; u++) {
+      const int i = min(i0 + u * SMP_NT, V - 1);
+      const float v = vs[u];
+      if (v < thresh) continue;
+      float sc = v;
+      if (!greedy) {
+        uint32_t r = hash32(hash32((uint32_t)i ^ (c * 0x9e3779b9u)) ^
+                            (uint32_t)seed);
+        float u1 = (r + 1.0f) * 2.3283064e-10f;  // (0,1]
+        sc = v * inv_temp - __logf(-__logf(u1));
+      }
+      if (sc > bv || (sc == bv && i < bi)) { bv = sc; bi = i; }
+    }
   }
   uint64_t pk = pack_ki(fkey(bv), bi);
 #pragma unroll
@@ -924,13 +948,13 @@ k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
     uint64_t o = __shfl_xor((unsigned long long)pk, w);
     if (o > pk) pk = o;
   }
-  __shared__ unsigned long long ws[4];
+  __shared__ unsigned long long ws[SMP_NT / 64];
   __shared__ int lastflag;
   if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = pk;
   __syncthreads();
   if (threadIdx.x == 0) {
     uint64_t b = ws[0];
-    for (int w = 1; w < 4; w++) if (ws[w] > b) b = ws[w];
+    for (int w = 1; w < SMP_NT / 64; w++) if (ws[w] > b) b = ws[w];
     atomicMax(pick, (unsigned long long)b);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     int t = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_ACQ_REL,
@@ -964,19 +988,17 @@ extern "C" hipError_t launch_sample(const void* logits, int V, int lbf16,
                                     void* out_ring, void* nout,
                                     void* len_ptr, int bump_len,
                                     hipStream_t stream) {
-  int blocks = (V + 255) / 256;
-  if (blocks > 512) blocks = 512;
-  // batched rows: keep TOTAL thread count constant (the B=8 sampler
-  // measured 102 us with a full grid per row)
-  if (batch > 1) {
-    blocks = blocks / batch + 1;
-    if (blocks < 16) blocks = 16;
-  }
+  // Blocks queue up at one address, twice in the pick: both launches took
+  // 23.3 us for a vocabulary of 128256 in 501 blocks of 256 logits, in 63 of
+  // 2048 9.2 (32768: 11.1 and 9.0).  The rows of a group queue up apart.
+  int blocks = (V + SMP_NT * SMP_U - 1) / (SMP_NT * SMP_U);
+  const int most = batch > 4 ? 16 : 64 / (batch > 0 ? batch : 1);
+  if (blocks > most) blocks = most;
   if (!greedy)
-    hipLaunchKernelGGL(k_logit_max, dim3(blocks, batch), dim3(256), 0,
+    hipLaunchKernelGGL(k_logit_max, dim3(blocks, batch), dim3(SMP_NT), 0,
                        stream, logits, V, lbf16, (unsigned long long*)gmax,
                        (uint64_t*)ctr);
-  hipLaunchKernelGGL(k_sample_pick, dim3(blocks, batch), dim3(256), 0,
+  hipLaunchKernelGGL(k_sample_pick, dim3(blocks, batch), dim3(SMP_NT), 0,
                      stream, logits, V, lbf16, ring_stride, min_p, greedy,
                      seed, inv_temp,
                      (unsigned long long*)gmax, (uint64_t*)ctr,
