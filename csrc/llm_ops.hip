@@ -1,12 +1,11 @@
 // llm_ops.hip — hand-written CDNA4 (gfx950 / MI355X) kernels for the
 // Llama-3.2 / Gemma-2 decode + prefill forward pass.
 //
-// Design notes (MI355X-first, per /opt/skills/guides/cdna_hip_programming.md):
+// Design notes (MI355X-first):
 //  - wave64 everywhere; block sizes are multiples of 64
 //  - bf16 I/O, fp32 accumulation; all bf16 traffic vectorized 16 B/lane
-//  - decode is weight-bandwidth-bound: the GEMV kernel streams W rows with
-//    deep unrolled dwordx4 loads straight to VGPRs (no LDS round trip for
-//    the streamed operand — guide §5 "GEMV / M<=16 decode weights")
+//  - products of one row, of few and of many are in gemv.hip, row_gemm.hip
+//    and gemm_prompt.hip, attention in attn_decode.hip and attn_prefill.hip
 //  - attention never materializes QK^T: online softmax in registers
 //  - KV cache is a preallocated pool, written in place (decode: inside
 //    the fused attention kernel; prefill: k_rope_cache) — replaces the
@@ -14,11 +13,11 @@
 //  - every kernel is hipGraph-capture-safe (no mallocs/syncs; sequence
 //    position and sampled token ids live in device memory)
 //
-// Replaces (reference parity):
+// What stands here for the reference's GPU pieces:
 //  K1 softmax RawKernel      -> online softmax in k_attn_dec /
 //                               k_attn_rows / k_attn
-//  K2 cuBLAS GEMM/GEMV       -> k_gemv_{bf16,fp8}_t (decode),
-//                               k_gemm_prompt MFMA (prefill)
+//  K2 cuBLAS GEMM/GEMV       -> k_gemv (decode), k_row_gemm (few rows),
+//                               k_gemm_prompt (prefill)
 //  K3 elementwise ufuncs     -> fused GEMV staging (NORM/GLU/NORM2),
 //                               k_rmsnorm, k_glu, k_softcap, k_addinto
 //  K4 KV concat              -> in-place pool writes
