@@ -296,7 +296,8 @@ extern "C" hipError_t launch_gemv_fp8_mx(
 // ====================================================================
 // RMSNorm of bf16 rows: y = [res +] norm(x) * g (g fp32, Gemma's +1 folded
 // in); with g2 also y2 = norm(y) * g2, the norm that follows a sandwich's
-// residual.
+// residual, or the same as e4m3 rows (16 rows ahead of a product: each of its
+// 256 blocks took 5 us for the norm and the rounding).
 //
 // A block of four waves a row, which stays in their registers; g and the
 // residual are on the way before anything is summed.  Bound by the launch and
@@ -311,8 +312,9 @@ template <int NC>
 __global__ void __launch_bounds__(256)
 k_rmsnorm(const u16* __restrict__ x, const float* __restrict__ g,
           const u16* res, u16* y, const float* __restrict__ g2,
-          u16* __restrict__ y2, int H, float eps) {
-  __shared__ float red[2][4];
+          u16* __restrict__ y2, uint8_t* __restrict__ q2,
+          float* __restrict__ s2, int H, float eps) {
+  __shared__ float red[3][4];
   const size_t at = (size_t)blockIdx.x * H;
   s8v v[NC], r[NC];
   f4v gg[NC][2], hh[NC][2];
@@ -361,28 +363,57 @@ k_rmsnorm(const u16* __restrict__ x, const float* __restrict__ g,
   }
   if (!g2) return;
   const float rm = norm(red[1]);
+  if (!q2) {
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      u16 o[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        o[j] = f2b(b2f(((u16*)&v[c])[j]) * rm * hh[c][j / 4][j % 4]);
+      if (k[c] < H) *(s8v*)(y2 + at + k[c]) = *(s8v*)o;
+    }
+    return;
+  }
+  // rows for an e4m3 product: what it would do to them in each of its blocks
+  float am = 0.f;
+#pragma unroll
+  for (int c = 0; c < NC; c++)
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      hh[c][j / 4][j % 4] *= b2f(((u16*)&v[c])[j]) * rm;
+      am = fmaxf(am, k[c] < H ? fabsf(hh[c][j / 4][j % 4]) : 0.f);
+    }
+#pragma unroll
+  for (int w = 1; w < 64; w <<= 1) am = fmaxf(am, __shfl_xor(am, w));
+  if ((threadIdx.x & 63) == 0) red[2][threadIdx.x >> 6] = am;
+  __syncthreads();
+  am = fmaxf(fmaxf(red[2][0], red[2][1]), fmaxf(red[2][2], red[2][3]));
+  am = fmaxf(am, 1e-8f) / 448.0f;
+  if (threadIdx.x == 0) s2[blockIdx.x] = am;
 #pragma unroll
   for (int c = 0; c < NC; c++) {
-    u16 o[8];
+    float f[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++)
-      o[j] = f2b(b2f(((u16*)&v[c])[j]) * rm * hh[c][j / 4][j % 4]);
-    if (k[c] < H) *(s8v*)(y2 + at + k[c]) = *(s8v*)o;
+    for (int j = 0; j < 8; j++) f[j] = hh[c][j / 4][j % 4];
+    if (k[c] < H)
+      *(unsigned long long*)(q2 + at + k[c]) = f32x8_to_fp8(f, 1.0f / am);
   }
 }
 
 extern "C" hipError_t launch_rmsnorm(const void* x, const void* g,
                                      const void* res, void* y, const void* g2,
-                                     void* y2, int M, int H, float eps,
-                                     hipStream_t stream) {
+                                     void* y2, void* q2, void* s2, int M,
+                                     int H, float eps, hipStream_t stream) {
   // a row stays in the registers of four waves
-  if (M < 0 || H < 8 || H > 16384 || H % 8 != 0 || !g2 != !y2)
+  if (M < 0 || H < 8 || H > 16384 || H % 8 != 0 || !g2 != (!y2 && !q2) ||
+      !q2 != !s2 || (y2 && q2))
     return hipErrorInvalidValue;
   if (M == 0) return hipSuccess;
 #define RMS_GO(NC)                                                           \
   hipLaunchKernelGGL(k_rmsnorm<NC>, dim3(M), dim3(256), 0, stream,           \
                      (const u16*)x, (const float*)g, (const u16*)res,        \
-                     (u16*)y, (const float*)g2, (u16*)y2, H, eps)
+                     (u16*)y, (const float*)g2, (u16*)y2, (uint8_t*)q2,      \
+                     (float*)s2, H, eps)
   if (H <= 2048) RMS_GO(1);
   else if (H <= 4096) RMS_GO(2);
   else if (H <= 8192) RMS_GO(4);

@@ -446,9 +446,10 @@ class GPUModel(DecodeLoop):
     # layer stack over rows [0, M) of the scratch buffers
     # ------------------------------------------------------------------
     def _rows(self, lw, name, x, y, M: int, g=None, res=None, bias=None,
-              act: int = -1, softcap: float = 0.0, batch: bool = False):
+              act: int = -1, softcap: float = 0.0, batch: bool = False,
+              ready: bool = False):
         """Projection of up to FEW_ROWS rows in one launch, W streamed
-        once: norm of x (g), activation of gate and up rows (act), softcap,
+        once: norm of x (g; ``ready``: b_xq holds the normed e4m3 rows), activation of gate and up rows (act), softcap,
         bias and residual on the way.  Rows beside e4m3 weights are rounded
         to e4m3, a row alone is not (GEMV).  ``batch``: a decode step of a
         group, which runs on the e4m3 copy where the engine holds MXFP4
@@ -472,9 +473,10 @@ class GPUModel(DecodeLoop):
         kw = dict(g=g, eps=eps, res=res, bias=bias, act=act, softcap=softcap,
                   part=self.b_gemm_acc, cnt=self.row_cnt)
         if e4m3:
-            if g is None:
-                K = x.shape[-1]
-                ho.quant_fp8(x[:M], self.b_xq, self.b_sx)
+            if g is None or ready:
+                K, kw["g"] = x.shape[-1], None
+                if not ready:
+                    ho.quant_fp8(x[:M], self.b_xq, self.b_sx)
                 x, kw["sx"] = self.b_xq[:M * K].view(M, K), self.b_sx
             # a prompt's rows are bf16 on their way to e4m3, a step's fp32
             ho.row_gemm(x, lw[name + "_q"], y, M, ws=lw[name + "_s"],
@@ -576,6 +578,8 @@ class GPUModel(DecodeLoop):
         eps = cfg.rms_norm_eps
         h, xn, t1 = self.b_h, self.b_xn, self.b_t1
         few = M <= ho.FEW_ROWS
+        # a step's rows go from one norm to the next as e4m3 (Gemma)
+        step8 = self.gemma and few and batch_attn and self.fp8 and M > 1
         qkv = self.b_rqkv[:M]
         nq, nkv = self.nh_l * self.hd, self.kvh_l * self.hd
         q, k, v = qkv.split([nq, nkv, nkv], dim=1)
@@ -586,8 +590,10 @@ class GPUModel(DecodeLoop):
             post = {"wo": "g_post", "wdown": "g_postffn"}[name]
             if self.gemma:
                 self._rowpar_ar(lw, name, x, t1, M, batch_attn)
-                ho.rmsnorm(t1[:M], lw[post], h[:M], res=h[:M], eps=eps, g2=g,
-                           y2=None if g is None else xn[:M])
+                to = {} if g is None else \
+                    dict(g2=g, q2=self.b_xq, s2=self.b_sx) if step8 else \
+                    dict(g2=g, y2=xn[:M])
+                ho.rmsnorm(t1[:M], lw[post], h[:M], res=h[:M], eps=eps, **to)
             elif self.tp_branch:
                 self._rowpar_ar(lw, name, x, t1, M, batch_attn)
                 ho.addinto(h[:M], t1[:M])
@@ -600,7 +606,8 @@ class GPUModel(DecodeLoop):
             window = cfg.sliding_window if cfg.is_sliding(i) else 0
             if few:
                 self._rows(lw, "wqkv", h, qkv, M, g=lw["g_in"],
-                           bias=lw.get("bqkv"), batch=batch_attn)
+                           bias=lw.get("bqkv"), batch=batch_attn,
+                           ready=step8 and i > 0)
             else:
                 if not self.gemma or i == 0:    # else by the layer before
                     ho.rmsnorm(h[:M], lw["g_in"], xn[:M], eps=eps)
@@ -637,7 +644,7 @@ class GPUModel(DecodeLoop):
                             window=window or 0,
                             kS=self._ks(i), vS=self._vs(i))
             g_mlp = lw["g_preffn"] if self.gemma else lw["g_post"]
-            into_h("wo", self.b_att, None if few else g_mlp)
+            into_h("wo", self.b_att, g_mlp if step8 or not few else None)
             if self.moe:
                 ho.rmsnorm(h[:M], g_mlp, xn[:M], eps=eps)
                 self._moe_mlp_rows(lw, M)
@@ -647,12 +654,12 @@ class GPUModel(DecodeLoop):
                     if 1 < M and self.fp8 and batch_attn:
                         a = self.b_act32
                     self._rows(lw, "wgu", h, a, M, g=g_mlp, act=self.act,
-                               batch=batch_attn)
+                               batch=batch_attn, ready=step8)
                 else:
                     if not self.gemma:
                         ho.rmsnorm(h[:M], g_mlp, xn[:M], eps=eps)
                     self._linear(lw, "wgu", xn, a, M=M, act=self.act)
-                last = few or i + 1 == len(self.layers)
+                last = few and not step8 or i + 1 == len(self.layers)
                 into_h("wdown", a,
                        None if last else self.layers[i + 1]["g_in"])
             if layer_hook is not None:

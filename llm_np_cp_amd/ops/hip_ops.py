@@ -28,7 +28,7 @@ _SIGS = {
                    [ctypes.c_float] * 3 +
                    [ctypes.c_int, ctypes.c_void_p, ctypes.c_int] +
                    [ctypes.c_long] * 2 + [ctypes.c_void_p] * 2,
-    "launch_rmsnorm": [ctypes.c_void_p] * 6 + [ctypes.c_int] * 2 +
+    "launch_rmsnorm": [ctypes.c_void_p] * 8 + [ctypes.c_int] * 2 +
                       [ctypes.c_float, ctypes.c_void_p],
     "launch_rope_cache": [ctypes.c_void_p] * 7 + [ctypes.c_int] +
                          [ctypes.c_void_p] * 3 + [ctypes.c_int] * 7 +
@@ -205,13 +205,16 @@ def gemv_fp8(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
 
 def rmsnorm(x: torch.Tensor, g: torch.Tensor, y: torch.Tensor,
             res: torch.Tensor | None = None, eps: float = 1e-5,
-            g2: torch.Tensor | None = None, y2: torch.Tensor | None = None):
+            g2: torch.Tensor | None = None, y2: torch.Tensor | None = None,
+            q2: torch.Tensor | None = None, s2: torch.Tensor | None = None):
     """y = norm(x)*g ; with res: y = res + norm(x)*g (Gemma post).  With g2
-    also y2 = norm(y)*g2, the norm behind the residual."""
+    also y2 = norm(y)*g2, the norm behind the residual, or the same as e4m3
+    rows q2 with scales s2."""
     M = 1 if x.dim() == 1 else x.shape[0]
     H = x.shape[-1]
     _check(lib().launch_rmsnorm(
-        _ptr(x), _ptr(g), _ptr(res), _ptr(y), _ptr(g2), _ptr(y2), M, H,
+        _ptr(x), _ptr(g), _ptr(res), _ptr(y), _ptr(g2), _ptr(y2), _ptr(q2),
+        _ptr(s2), M, H,
         ctypes.c_float(eps), _stream()), "rmsnorm")
 
 

@@ -348,8 +348,18 @@ def test_two_norms(M, H):
 
     # bf16 results: 2^-8 of each value, the second from the first as it is
     assert off(y[:M], rms(x.double()) * g.double() + h.double()) < 2.0 ** -8
-    assert off(z[:M], rms(y[:M].double()) * g2.double()) < 2.0 ** -8
+    ref = rms(y[:M].double()) * g2.double()
+    assert off(z[:M], ref) < 2.0 ** -8
     assert (y[M] == 7.0).all() and (z[M] == 7.0).all()
+    q = torch.full((M + 1, H), 5, dtype=torch.uint8, device="cuda")
+    s = torch.zeros(M + 1, device="cuda")
+    y[:M] = h
+    ho.rmsnorm(x, g, y[:M], res=y[:M], eps=1e-5, g2=g2, q2=q, s2=s)
+    got = q.view(torch.float8_e4m3fn).double() * s[:, None].double()
+    # four bits: 2^-4 of each value; the scale is the largest one's
+    assert off(got[:M], ref) < 2.0 ** -4
+    assert torch.allclose(s[:M].double(), ref.abs().amax(1) / 448, rtol=1e-5)
+    assert (q[M] == 5).all() and s[M] == 0
 
 
 # rows of an expert: none, one, less and more than a tile of 32, 64 and 128
