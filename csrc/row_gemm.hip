@@ -485,59 +485,112 @@ static void rg_go(const RgArgs& a, dim3 grid, size_t lds, hipStream_t s) {
                      lds, s, a);
 }
 
-template <int WT, bool GLU>
-static hipError_t rg_run(RgArgs a, long part_floats, int ncnt,
-                         hipStream_t s) {
-  constexpr int SE = 8 * RgT<WT>::E, P = GLU ? 2 : 1;
-  // K per block for a split, whole slabs
-  auto part_k = [&](int ks) {
-    return ((a.K + ks - 1) / ks + SE - 1) / SE * SE;
-  };
-  auto lds_of = [&](int ks) {
-    return (long)a.M * (part_k(ks) * (WT == RG_FP8 ? 1 : 2) + 16);
-  };
+// How a product goes: m rows a launch, K in ks parts of kr, rpb outputs a
+// block in tiles of nb, ng blocks a part; LDS of a block, floats of `part`.
+struct RgPlan { int m, ks, kr, rpb, nb, ng; long lds, floats; };
+
+static int rg_up(int a, int b) { return (a + b - 1) / b; }
+
+static bool rg_plan_rows(RgPlan& p, int wt, bool glu, bool norm, int M, int N,
+                         int K, long part_floats, int ncnt) {
+  const int P = glu ? 2 : 1, XB = wt == RG_FP8 ? 1 : 2;
+  const int SE = wt == RG_BF16 ? 64 : wt == RG_FP8 ? 128 : 256;
   // A block a CU, with X in place for all its outputs: two a CU read X twice
   // and run no faster (5 rows, 2x8192x2048: 16.9 us, 512 blocks 21.1;
   // 32768x3072 38.9 and 43.9).  Less than eight outputs a block gain nothing;
   // more than LDS has room for the sums of are left to blocks of a next round.
-  auto tile_of = [&](int r) { return r <= 24 && (r - 1) % 16 < 8 ? 8 : 16; };
-  auto share = [&](int ks) {
-    const int ng = 256 / ks > 1 ? 256 / ks : 1, r = (a.N + ng - 1) / ng;
-    const long most = (RG_ROOM - lds_of(ks)) / (P * 1024) - (RG_NW - 1);
-    return most < 1 ? 0 : (int)(r < 8 ? 8 : r < most * 16 ? r : most * 16);
+  auto plan = [&](int ks) {
+    RgPlan q = {M, ks, rg_up(rg_up(K, ks), SE) * SE, 0, 16, 0, 0, 0};
+    q.lds = (long)M * (q.kr * XB + 16);
+    const int r = rg_up(N, 256 / ks > 1 ? 256 / ks : 1);
+    const long most = (RG_ROOM - q.lds) / (P * 1024) - (RG_NW - 1);
+    if (most < 1) return q;                  // ng 0: X does not fit
+    q.rpb = r < 8 ? 8 : r < most * 16 ? r : (int)most * 16;
+    if (q.rpb <= 24 && (q.rpb - 1) % 16 < 8 && rg_up(q.rpb, 8) <= most)
+      q.nb = 8;
+    q.ng = rg_up(N, q.rpb);
+    const int tiles = rg_up(q.rpb, q.nb);
+    q.lds += (long)(tiles + RG_NW - 1) * P * 1024;
+    if (ks > 1) q.floats = (long)q.ng * tiles * ks * P * 256;
+    return q;
   };
-  auto fits = [&](int ks) {
-    const int r = share(ks);
-    if (r < 1) return false;
-    const int nb = tile_of(r);
-    const long ng = (a.N + r - 1) / r, nt = ng * ((r + nb - 1) / nb);
-    return ks == 1 ||
-           (!a.g && nt * ks * P * 256 <= part_floats && ng <= ncnt);
+  auto fits = [&](const RgPlan& q) {
+    return q.ng && (q.ks == 1 || (!norm && q.floats <= part_floats &&
+                                  q.ng <= ncnt));
+  };
+  // the next number of parts that has slabs for all of them
+  auto after = [&](int ks) {
+    do ks++;
+    while (ks < 64 && rg_up(K, rg_up(rg_up(K, ks), SE) * SE) != ks);
+    return ks;
   };
   // as many parts of K as it takes for X to fit
-  int ks = 1;
-  while (ks < 64 && !fits(ks)) ks++;
+  p = plan(1);
+  for (int ks = after(1); ks < 64 && !fits(p); ks = after(ks)) p = plan(ks);
+  if (!fits(p)) return false;
   // Narrow products: more parts until the 256 CUs have a block each, or a
   // part is down to 512.  (5 rows, 2048x8192: 128 blocks 12.0 us, 256 of half
   // tiles 10.1.)
-  while (ks < 16 && (a.N + share(ks) - 1) / share(ks) * ks < 192 &&
-         a.K / (ks + 1) >= 512 && fits(ks + 1))
-    ks++;
-  if (!fits(ks)) return hipErrorInvalidValue;
-  a.kr = part_k(ks);
-  ks = (a.K + a.kr - 1) / a.kr;
-  a.rpb = share(ks);
-  const int nb = tile_of(a.rpb), tiles = (a.rpb + nb - 1) / nb;
-  const dim3 grid((a.N + a.rpb - 1) / a.rpb, ks);
-  const size_t lds = lds_of(ks) + (size_t)(tiles + RG_NW - 1) * P * 1024;
+  while (p.ng * p.ks < 192) {
+    const int ks = after(p.ks);
+    if (ks > 16 || K / ks < 512) break;
+    const RgPlan q = plan(ks);
+    if (!fits(q)) break;
+    p = q;
+  }
+  return true;
+}
+
+// Where the room for parts is too small for the rows' X, fewer rows a launch.
+static bool rg_plan(RgPlan& p, int wt, bool glu, bool norm, int M, int N,
+                    int K, long part_floats, int ncnt) {
+  for (int m = M; m > 0; m = m > 1 ? (m + 1) / 2 : 0)
+    if (rg_plan_rows(p, wt, glu, norm, m, N, K, part_floats, ncnt))
+      return true;
+  return false;
+}
+
+template <int WT, bool GLU>
+static hipError_t rg_run(RgArgs a, long part_floats, int ncnt,
+                         hipStream_t s) {
+  RgPlan p;
+  if (!rg_plan(p, WT, GLU, a.g, a.M, a.N, a.K, part_floats, ncnt))
+    return hipErrorInvalidValue;
+  a.kr = p.kr;
+  a.rpb = p.rpb;
+  const dim3 grid(p.ng, p.ks);
   auto go = [&](auto norm) {
-    if (nb == 8) rg_go<WT, 8, GLU, decltype(norm)::value>(a, grid, lds, s);
-    else rg_go<WT, 16, GLU, decltype(norm)::value>(a, grid, lds, s);
+    if (p.nb == 8) rg_go<WT, 8, GLU, decltype(norm)::value>(a, grid, p.lds, s);
+    else rg_go<WT, 16, GLU, decltype(norm)::value>(a, grid, p.lds, s);
   };
-  if (!a.g) go(std::integral_constant<int, 0>());
-  else if (WT != RG_FP8 || !a.n16) go(std::integral_constant<int, 1>());
-  else go(std::integral_constant<int, WT == RG_FP8 ? 2 : 1>());
+  const RgArgs all = a;
+  for (int r = 0; r < all.M; r += p.m) {
+    a.M = all.M - r < p.m ? all.M - r : p.m;
+    a.x = (const char*)all.x +
+          (size_t)r * a.ldx * (WT == RG_FP8 && !a.g ? 1 : 2);
+    if (a.sx) a.sx = all.sx + r;
+    if (a.res) a.res = all.res + (size_t)r * a.ldr;
+    a.y = (char*)all.y + (size_t)r * a.ldy * (a.out_f32 ? 4 : 2);
+    if (!a.g) go(std::integral_constant<int, 0>());
+    else if (WT != RG_FP8 || !a.n16) go(std::integral_constant<int, 1>());
+    else go(std::integral_constant<int, WT == RG_FP8 ? 2 : 1>());
+  }
   return hipGetLastError();
+}
+
+// The plan of a product as numbers (m, ks, kr, rpb, nb, ng), its LDS and the
+// floats of `part` that it takes; what it would take where there is room
+// enough says how much to allocate.
+extern "C" hipError_t row_gemm_plan(int wt, int glu, int norm, int M, int N,
+                                    int K, long part_floats, int ncnt,
+                                    long* out) {
+  RgPlan p;
+  if (wt < 0 || wt > RG_FP4 || M < 1 || M > 16 || N < 1 || K < 64 || K % 64 ||
+      !rg_plan(p, wt, glu, norm, M, N, K, part_floats, ncnt))
+    return hipErrorInvalidValue;
+  const long v[8] = {p.m, p.ks, p.kr, p.rpb, p.nb, p.ng, p.lds, p.floats};
+  for (int i = 0; i < 8; i++) out[i] = v[i];
+  return hipSuccess;
 }
 
 // wt: 0 bf16, 1 e4m3 with ws, 2 MXFP4 with we.  act < 0: no gate.

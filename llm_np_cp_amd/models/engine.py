@@ -324,16 +324,26 @@ class GPUModel(DecodeLoop):
         self.b_xn = torch.zeros(PC, H, **bf)
         self.b_t1 = torch.zeros(PC, H, **bf)
         # q | k | v of a row, from one projection
-        self.b_rqkv = torch.zeros(PC, (self.nh_l + 2 * self.kvh_l) * hd,
-                                  **bf)
+        nqkv = (self.nh_l + 2 * self.kvh_l) * hd
+        self.b_rqkv = torch.zeros(PC, nqkv, **bf)
         self.b_att = torch.zeros(PC, self.nh_l * hd, **bf)
         # act(gate) * up; of each of a row's experts
         pairs = PC * (self.topk if self.moe else 1)
         self.b_gate = torch.zeros(pairs, I, **bf)
         if self.wq4:          # its prompts have gate and up apart
             self.b_up = torch.zeros(PC, I, **bf)
-        self.b_gemm_acc = torch.zeros(PC * max(I, H), dtype=torch.float32,
-                                      device=dev)
+        # fp32 parts of products that split K, and of attention that splits
+        # its keys.  A few long rows beside many outputs can take more than a
+        # short chunk of a prompt does.
+        few = [(nqkv, H), (H, self.nh_l * hd), (self.vocab_l, H)]
+        if not self.moe:
+            few += [(I, H, True), (H, I)]
+        kinds = ["fp4"] * self.wq4 + ["fp8"] * self.keep_fp8 \
+            if self.fp8 else ["bf16"]
+        self.b_gemm_acc = torch.zeros(
+            max([PC * max(I, H)] +
+                [ho.row_gemm_room(k, *p) for k in kinds for p in few]),
+            dtype=torch.float32, device=dev)
         if self.fp8:
             # activation-quant scratch for the fp8 MFMA prefill GEMMs
             kmax = max(H, I, self.nh_l * hd)

@@ -58,6 +58,8 @@ _SIGS = {
     "launch_row_gemm": [ctypes.c_void_p] * 11 + [ctypes.c_long] +
                        [ctypes.c_int] * 11 +
                        [ctypes.c_float, ctypes.c_float, ctypes.c_void_p],
+    "row_gemm_plan": [ctypes.c_int] * 6 + [ctypes.c_long, ctypes.c_int,
+                                           ctypes.c_void_p],
     "launch_prefetch": [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p,
                         ctypes.c_void_p],
     "launch_softcap": [ctypes.c_void_p, ctypes.c_long, ctypes.c_float,
@@ -393,7 +395,8 @@ def row_gemm(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, M: int,
     g: RMSNorm of x on the way (K <= ROW_NORM_K; norm16: rounded to bf16
     before e4m3).  act 0/1: w holds gate
     rows, then up rows, and Y = act(gate) * up.  Then softcap, bias, res.
-    part (fp32) and cnt (int32, zero; left zero) let K be split."""
+    part (fp32) and cnt (int32, zero; left zero) let K be split; where long
+    rows need that and part is too small, fewer rows go at a time."""
     wt = 1 if ws is not None else 2 if we is not None else 0
     K = x.shape[-1]
     N = w.shape[0] // (2 if act >= 0 else 1)
@@ -409,6 +412,26 @@ def row_gemm(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, M: int,
         res.stride(0) if res is not None else 0, y.stride(0), act,
         1 if y.dtype == torch.float32 else 0, int(norm16),
         ctypes.c_float(eps), ctypes.c_float(softcap), _stream()), "row_gemm")
+
+
+def row_gemm_plan(kind: str, M: int, N: int, K: int, glu: bool = False,
+                  norm: bool = False, part: int = 1 << 62,
+                  cnt: int = 256) -> dict | None:
+    """How row_gemm goes about a product with so many floats of part and
+    counters (None: it does not take it).  Host arithmetic only."""
+    out = (ctypes.c_long * 8)()
+    if lib().row_gemm_plan(("bf16", "fp8", "fp4").index(kind), int(glu),
+                           int(norm), M, N, K, ctypes.c_long(part), cnt,
+                           ctypes.cast(out, ctypes.c_void_p)):
+        return None
+    return dict(zip(("rows", "splits", "k", "outputs", "tile", "blocks",
+                     "lds", "floats"), out))
+
+
+def row_gemm_room(kind: str, N: int, K: int, glu: bool = False) -> int:
+    """Floats of part with which any number of rows goes in one launch."""
+    plans = [row_gemm_plan(kind, M, N, K, glu) for M in range(1, FEW_ROWS + 1)]
+    return max(p["floats"] if p else 0 for p in plans)
 
 
 def quant_fp8(x: torch.Tensor, q: torch.Tensor, s: torch.Tensor):

@@ -127,6 +127,46 @@ def test_few_rows(N, K, M, kind, norm, act):
     assert (Y[M] == 7.0).all() and not cnt.any()
 
 
+# long rows beside room for parts of all, of fewer rows and of none; a tile of
+# sums that just does not fit (8 rows of 9536)
+@pytest.mark.parametrize("kind,M,N,K", [
+    ("bf16", 16, 520, 8192), ("bf16", 8, 4608, 9536), ("fp8", 13, 300, 19008),
+    ("fp4", 16, 70, 12288)])
+@pytest.mark.parametrize("act", [-1, 0])
+@pytest.mark.parametrize("room", [0, 100000, 1 << 22])
+def test_few_rows_of_little_room(kind, M, N, K, act, room):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    W = normal(N * (2 if act >= 0 else 1), K, seed=4, scale=K ** -0.5)
+    X = normal(M, K + 16, seed=5)[:, :K]
+    bias, res = (normal(M, N, seed=6) for _ in range(2))
+    kw, Wd, x = {}, W.double(), X.double()
+    if kind == "fp8":
+        W, kw["ws"], Wd = e4m3(W)
+        X, kw["sx"], x = e4m3(X)
+    elif kind == "fp4":
+        q = torch.empty(W.shape[0], K // 2, dtype=torch.uint8, device="cuda")
+        e = torch.empty(W.shape[0], K // 32, dtype=torch.uint8, device="cuda")
+        ho.quant_fp4(W, q, e)
+        W, kw["we"], Wd = q, e, mxfp4_values(q, e)
+    part = torch.full((room + 64,), 7.0, device="cuda")
+    cnt = torch.zeros(256, dtype=torch.int32, device="cuda")
+    Y = torch.full((M + 1, N), 7.0, device="cuda").bfloat16()
+    Y[:M] = res                                     # in place
+    ho.row_gemm(X, W, Y, M, bias=bias[0].contiguous(), res=Y, act=act,
+                part=part[:room], cnt=cnt, **kw)
+    z = x @ Wd.T
+    if act >= 0:
+        if kind == "fp8":
+            z = z.bfloat16().double()
+        z = torch.nn.functional.silu(z[:, :N]) * z[:, N:]
+    z = z + bias[0].double() + res.double()
+    # exact products, fp32 sums, bf16 results: 2^-9 at most, and the halves
+    # of an e4m3 gate
+    assert off(Y[:M], z) < 2.0 ** -8
+    assert (Y[M] == 7.0).all() and not cnt.any() and (part[room:] == 7.0).all()
+
+
 # tiles of 32 to 256 rows and 64 to 256 outputs, by what the sizes call for:
 # a rest of a tile both ways, outputs that are no multiple of four, K of one
 # slab, of one more than the buffers, split over blocks, half a slab (e4m3)
