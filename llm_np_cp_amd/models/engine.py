@@ -459,8 +459,9 @@ class GPUModel(DecodeLoop):
               act: int = -1, softcap: float = 0.0, batch: bool = False,
               ready: bool = False):
         """Projection of up to FEW_ROWS rows in one launch, W streamed
-        once: norm of x (g; ``ready``: b_xq holds the normed e4m3 rows), activation of gate and up rows (act), softcap,
-        bias and residual on the way.  Rows beside e4m3 weights are rounded
+        once: norm of x (g; ``ready``: b_xq and b_sx hold the normed rows as
+        e4m3), activation of gate and up rows (act), softcap, bias and
+        residual on the way.  Rows beside e4m3 weights are rounded
         to e4m3, a row alone is not (GEMV).  ``batch``: a decode step of a
         group, which runs on the e4m3 copy where the engine holds MXFP4
         too."""
@@ -477,7 +478,7 @@ class GPUModel(DecodeLoop):
                 return
             ho.gemv_fp8(w, s, x, y[0], act=act, glu=True)
             return
-        if g is not None and x.shape[-1] > ho.ROW_NORM_K:
+        if g is not None and not ready and x.shape[-1] > ho.ROW_NORM_K:
             ho.rmsnorm(x[:M], g, self.b_xn[:M], eps=eps)
             x, g = self.b_xn, None
         kw = dict(g=g, eps=eps, res=res, bias=bias, act=act, softcap=softcap,
