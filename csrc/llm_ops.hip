@@ -297,7 +297,9 @@ extern "C" hipError_t launch_gemv_fp8_mx(
 // RMSNorm of bf16 rows: y = [res +] norm(x) * g (g fp32, Gemma's +1 folded
 // in); with g2 also y2 = norm(y) * g2, the norm that follows a sandwich's
 // residual, or the same as e4m3 rows (16 rows ahead of a product: each of its
-// 256 blocks took 5 us for the norm and the rounding).
+// 256 blocks took 5 us for the norm and the rounding).  Without g2 norm(x) * g
+// itself may go to e4m3, from fp32: of rows that are too long for the product
+// to norm.
 //
 // A block of four waves a row, which stays in their registers; g and the
 // residual are on the way before anything is summed.  Bound by the launch and
@@ -348,21 +350,28 @@ k_rmsnorm(const u16* __restrict__ x, const float* __restrict__ g,
     ss = (sums[0] + sums[1]) + (sums[2] + sums[3]);
     return rsqrtf(ss / (float)H + eps);
   };
-  const float rn = norm(red[0]);
+  float rm = norm(red[0]);
+  if (y) {
 #pragma unroll
-  for (int c = 0; c < NC; c++) {
-    u16 o[8];
+    for (int c = 0; c < NC; c++) {
+      u16 o[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      float f = b2f(((u16*)&v[c])[j]) * rn * gg[c][j / 4][j % 4];
-      if (res) f += b2f(((u16*)&r[c])[j]);
-      o[j] = f2b(f);
+      for (int j = 0; j < 8; j++) {
+        float f = b2f(((u16*)&v[c])[j]) * rm * gg[c][j / 4][j % 4];
+        if (res) f += b2f(((u16*)&r[c])[j]);
+        o[j] = f2b(f);
+      }
+      v[c] = *(s8v*)o;
+      if (k[c] < H) *(s8v*)(y + at + k[c]) = v[c];
     }
-    v[c] = *(s8v*)o;
-    if (k[c] < H) *(s8v*)(y + at + k[c]) = v[c];
+    if (!g2) return;
+    rm = norm(red[1]);
+  } else {
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) hh[c][i] = gg[c][i];
   }
-  if (!g2) return;
-  const float rm = norm(red[1]);
   if (!q2) {
 #pragma unroll
     for (int c = 0; c < NC; c++) {
@@ -405,8 +414,8 @@ extern "C" hipError_t launch_rmsnorm(const void* x, const void* g,
                                      void* y2, void* q2, void* s2, int M,
                                      int H, float eps, hipStream_t stream) {
   // a row stays in the registers of four waves
-  if (M < 0 || H < 8 || H > 16384 || H % 8 != 0 || !g2 != (!y2 && !q2) ||
-      !q2 != !s2 || (y2 && q2))
+  if (M < 0 || H < 8 || H > 16384 || H % 8 != 0 || !q2 != !s2 ||
+      (y ? !g2 != (!y2 && !q2) || (y2 && q2) : !q2 || g2 || y2 || res))
     return hipErrorInvalidValue;
   if (M == 0) return hipSuccess;
 #define RMS_GO(NC)                                                           \

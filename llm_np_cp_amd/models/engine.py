@@ -479,8 +479,13 @@ class GPUModel(DecodeLoop):
             ho.gemv_fp8(w, s, x, y[0], act=act, glu=True)
             return
         if g is not None and not ready and x.shape[-1] > ho.ROW_NORM_K:
-            ho.rmsnorm(x[:M], g, self.b_xn[:M], eps=eps)
-            x, g = self.b_xn, None
+            if e4m3 and batch:
+                ho.rmsnorm(x[:M], g, None, eps=eps, q2=self.b_xq,
+                           s2=self.b_sx)
+                ready = True
+            else:
+                ho.rmsnorm(x[:M], g, self.b_xn[:M], eps=eps)
+                x, g = self.b_xn, None
         kw = dict(g=g, eps=eps, res=res, bias=bias, act=act, softcap=softcap,
                   part=self.b_gemm_acc, cnt=self.row_cnt)
         if e4m3:

@@ -205,13 +205,14 @@ def gemv_fp8(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
           glu)
 
 
-def rmsnorm(x: torch.Tensor, g: torch.Tensor, y: torch.Tensor,
+def rmsnorm(x: torch.Tensor, g: torch.Tensor, y: torch.Tensor | None,
             res: torch.Tensor | None = None, eps: float = 1e-5,
             g2: torch.Tensor | None = None, y2: torch.Tensor | None = None,
             q2: torch.Tensor | None = None, s2: torch.Tensor | None = None):
     """y = norm(x)*g ; with res: y = res + norm(x)*g (Gemma post).  With g2
     also y2 = norm(y)*g2, the norm behind the residual, or the same as e4m3
-    rows q2 with scales s2."""
+    rows q2 with scales s2.  y None: norm(x)*g itself as e4m3 rows, rounded
+    once."""
     M = 1 if x.dim() == 1 else x.shape[0]
     H = x.shape[-1]
     _check(lib().launch_rmsnorm(

@@ -48,3 +48,26 @@ def test_rows_that_are_ready_are_not_normed_again(monkeypatch):
     m._layers_forward(3, batch_attn=True)
     # ahead of the first product, then behind each branch
     assert len(calls) == 1 + 2 * 2
+
+
+# a step's rows go from fp32 to e4m3, however long they are; by way of bf16
+# one in fifty takes the other of two e4m3 values (and each scale moves)
+@pytest.mark.parametrize("dtype", ["fp8", "fp4"])
+@pytest.mark.parametrize("hidden", [4096, 4608])
+def test_long_rows_of_a_step_are_rounded_once(hidden, dtype):
+    m = engine(hidden=hidden, layers=1, dtype=dtype)
+    g = torch.rand(hidden, generator=torch.Generator().manual_seed(1)) + 0.5
+    lw = {"wqkv_q": torch.eye(hidden, device="cuda")[:512]
+          .to(torch.float8_e4m3fn).view(torch.uint8),
+          "wqkv_s": torch.ones(512, device="cuda")}
+    m.b_h.normal_(generator=torch.Generator("cuda").manual_seed(2))
+    y = torch.zeros(3, 512, dtype=torch.bfloat16, device="cuda")
+    # rows of a unit matrix: the product shows what its rows were
+    m._rows(lw, "wqkv", m.b_h, y, 3, g=g.cuda(), batch=True)
+    x = m.b_h[:3].double()
+    x = x * torch.rsqrt(x.pow(2).mean(1, keepdim=True) + 1e-5) \
+        * g.cuda().double()
+    s = (x.abs().amax(1, keepdim=True) / 448).float()
+    q = (x.float() / s).to(torch.float8_e4m3fn).float()[:, :512]
+    got = y.float() / s                     # bf16 of q * s: 2^-9 off
+    assert ((got - q).abs() > q.abs() * 2.0 ** -6).float().mean() < 0.002

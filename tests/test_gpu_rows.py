@@ -400,6 +400,13 @@ def test_two_norms(M, H):
     assert off(got[:M], ref) < 2.0 ** -4
     assert torch.allclose(s[:M].double(), ref.abs().amax(1) / 448, rtol=1e-5)
     assert (q[M] == 5).all() and s[M] == 0
+    ho.rmsnorm(x, g, None, q2=q, s2=s)         # the first norm, rounded once
+    ref = rms(x.double()) * g.double()
+    assert torch.allclose(s[:M].double(), ref.abs().amax(1) / 448, rtol=1e-6)
+    want = (ref / s[:M, None].double()).float().to(torch.float8_e4m3fn)
+    other = want.view(torch.uint8) != q[:M]    # fp32 sums: on the edge of two
+    assert other.float().mean() < 0.001
+    assert (q[M] == 5).all() and s[M] == 0
 
 
 # rows of an expert: none, one, less and more than a tile of 32, 64 and 128
