@@ -420,13 +420,10 @@ class GPUModel(DecodeLoop):
             self.bt_gmax = torch.zeros(B, **i64)
             self.bt_pick = torch.zeros(B, **i64)
             self.bt_cnt = torch.zeros(B, **i32)
-            # a group fills the chip with fewer (16 sequences of 620 keys, 8
-            # heads of 256: 2 ranges 25.4 us, 3 34.5, 5 38.5)
-            self.bt_split = min(self.attn_split,
-                                max(1, 256 // (B * self.kvh_l)))
+            # for any number of active rows
             self.bt_scratch = torch.zeros(
-                B * self.nh_l * self.bt_split * (hd + 2),
-                dtype=torch.float32, device=dev)
+                max(M * self._ranges(M) for M in range(1, B + 1)) *
+                self.nh_l * (hd + 2), dtype=torch.float32, device=dev)
             self.bt_attn_cnt = torch.zeros(B * self.nh_l, **i32)
             # fused multi-x path scratch (fp8, B<=8)
             self.bt_gu = torch.zeros(B, 2 * I, **bf)
@@ -583,6 +580,14 @@ class GPUModel(DecodeLoop):
         s = self.v_scale[i]
         return s if (s is None or self.max_batch == 1) else s[self._pb]
 
+    def _ranges(self, M: int) -> int:
+        """Ranges of the history that a step of M rows may take: the more
+        rows, the fewer fill the chip.  us, 8000 keys of 8 heads of 128, by
+        1, 2, 4, 8, 16 ranges: one row 76 44 27 18 15, four 81 49 31 28 35,
+        16 117 101 111 137 184; 16 rows of 620 keys, 8 heads of 256: 2 ranges
+        25, 3 35."""
+        return min(self.attn_split, max(1, 256 // (M * self.kvh_l)))
+
     def _layers_forward(self, M: int, layer_hook=None,
                         batch_attn: bool = False, keys: int = 0):
         """Layer stack over rows [0, M), the last of which sees ``keys``
@@ -634,7 +639,7 @@ class GPUModel(DecodeLoop):
                             self.sin_t, self.bt_scratch, self.bt_attn_cnt,
                             self.nh_l, self.kvh_l, self.hd, self.scale,
                             softcap=self.attn_softcap, window=window or 0,
-                            split=self.bt_split, kS=self.k_scale[i],
+                            split=self._ranges(M), kS=self.k_scale[i],
                             vS=self.v_scale[i], batch=M)
             else:
                 ho.rope_cache(q, k, v, self._kc(i),
@@ -1126,7 +1131,7 @@ class GPUModel(DecodeLoop):
                         self.bt_scratch, self.bt_attn_cnt,
                         self.nh_l, self.kvh_l, self.hd, self.scale,
                         softcap=self.attn_softcap, window=window or 0,
-                        split=self.bt_split, kS=self.k_scale[i],
+                        split=self._ranges(B), kS=self.k_scale[i],
                         vS=self.v_scale[i], batch=B)
             if self.gemma:
                 ho.gemv_fp8_mx(lw["wo_q"], lw["wo_s"], self.b_att, t1, B,

@@ -14,7 +14,8 @@ def _build():
     ensure_built()
 
 
-def engine(family="llama", hidden=4608, layers=2, **kw):
+def engine(family="llama", hidden=4608, layers=2, heads=(4, 2), max_seq=64,
+           max_batch=4, **kw):
     import llm_np_cp_amd as L
     from llm_np_cp_amd.io.loader import random_weights
     from llm_np_cp_amd.models.engine import GPUModel
@@ -22,12 +23,13 @@ def engine(family="llama", hidden=4608, layers=2, **kw):
     cfg = L.ModelConfig(
         model_type=family, vocab_size=512, hidden_size=hidden,
         intermediate_size=256, num_hidden_layers=layers,
-        num_attention_heads=4, num_key_value_heads=2, head_dim=64,
+        num_attention_heads=heads[0], num_key_value_heads=heads[1],
+        head_dim=64,
         hidden_act="gelu_pytorch_tanh" if family == "gemma2" else "silu",
         attn_logit_softcapping=50.0 if family == "gemma2" else None,
         final_logit_softcapping=30.0 if family == "gemma2" else None)
-    return GPUModel(cfg, random_weights(cfg, seed=3), max_seq=64,
-                    max_batch=4, **kw)
+    return GPUModel(cfg, random_weights(cfg, seed=3), max_seq=max_seq,
+                    max_batch=max_batch, **kw)
 
 
 def count(monkeypatch, name):
@@ -71,3 +73,23 @@ def test_long_rows_of_a_step_are_rounded_once(hidden, dtype):
     q = (x.float() / s).to(torch.float8_e4m3fn).float()[:, :512]
     got = y.float() / s                     # bf16 of q * s: 2^-9 off
     assert ((got - q).abs() > q.abs() * 2.0 ** -6).float().mean() < 0.002
+
+
+# the rows that are there set the ranges, not those there is room for
+@pytest.mark.parametrize("kv_dtype", ["bf16", "fp8"])
+def test_ranges_follow_the_active_rows(monkeypatch, kv_dtype):
+    m = engine(hidden=256, layers=1, heads=(8, 8), max_seq=2048,
+               max_batch=32, kv_dtype=kv_dtype)
+    lens = [1900 - 57 * b for b in range(32)]
+    for b, n in enumerate(lens):
+        m.prefill_row(b, (np.arange(n) * 7 + b) % 512)
+    x = torch.randn(32, 256, generator=torch.Generator().manual_seed(1))
+    calls, got = count(monkeypatch, "attn_dec"), {}
+    for M in (32, 1, 2, 5, 31):
+        m.b_h[:M].copy_(x[:M])
+        m._layers_forward(M, batch_attn=True)
+        got[M] = m.b_att[:M].float()
+        assert calls[-1][1]["split"] == min(8, max(1, 32 // M))
+        assert not m.bt_attn_cnt.any()
+        # sums in another order, bf16 results
+        assert (got[M] - got[32][:M]).norm() < 2.0 ** -8 * got[M].norm()
