@@ -468,12 +468,10 @@ class GPUModel(DecodeLoop):
             if g is not None:
                 ho.rmsnorm(x[:1], g, self.b_xn[:1], eps=eps)
                 x = self.b_xn
-            w, s = lw[name + "_q"], lw[name + "_s"]
-            if act < 0:
-                ho.gemv_fp8(w, s, x, y, res=res if bias is None else bias,
-                            softcap=softcap)
-                return
-            ho.gemv_fp8(w, s, x, y[0], act=act, glu=True)
+            assert bias is None or res is None, "one row adds one of them"
+            ho.gemv_fp8(lw[name + "_q"], lw[name + "_s"], x, y,
+                        res=res if bias is None else bias, softcap=softcap,
+                        act=max(act, 0), glu=act >= 0)
             return
         if g is not None and not ready and x.shape[-1] > ho.ROW_NORM_K:
             if e4m3 and batch:
@@ -506,13 +504,15 @@ class GPUModel(DecodeLoop):
         on-the-fly activation row quantization.  ``act``: gate and up rows,
         y = act(gate) * up."""
         if M <= ho.FEW_ROWS:
-            self._rows(lw, name, x, y, M, res=res, batch=batch)
+            self._rows(lw, name, x, y, M, res=res, bias=bias, act=act,
+                       batch=batch)
             return
         res = res[:M] if res is not None else None
         kw = dict(res=res, accbuf=self.b_gemm_acc)
         if self.wq4:
             q, e = lw[name + "_q4"], lw[name + "_e4"]
             if act >= 0:
+                assert res is None, "a gate beside MXFP4 adds nothing"
                 n = q.shape[0] // 2
                 ho.gemm_fp4w(x[:M], q[:n], e[:n], y[:M], **kw)
                 ho.gemm_fp4w(x[:M], q[n:], e[n:], self.b_up[:M], **kw)

@@ -1,0 +1,60 @@
+"""The engine's choices on the host, without a GPU: what goes to which
+kernel with which arguments."""
+
+import types
+
+import pytest
+import torch
+
+from llm_np_cp_amd.models import engine as eng
+
+
+class Calls(list):
+    def __getattr__(self, name):
+        def call(*a, **k):
+            self.append((name, a, k))
+        return call
+
+
+def fake(**kw):
+    """What _rows and _linear read of an engine."""
+    m = types.SimpleNamespace(
+        config=types.SimpleNamespace(rms_norm_eps=1e-5), fp8=False,
+        wq4=False, b_gemm_acc=None, row_cnt=None, tile_cnt=None,
+        b_xn=torch.zeros(32, 64), b_xq=torch.zeros(32 * 64),
+        b_sx=torch.zeros(32), b_up=torch.zeros(32, 64))
+    m.__dict__.update(kw)
+    m._rows = types.MethodType(eng.GPUModel._rows, m)
+    return m
+
+
+@pytest.mark.parametrize("M", [1, 3, 16, 17])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_linear_passes_bias_and_gate_on(monkeypatch, M, fp8):
+    calls = Calls()
+    calls.FEW_ROWS, calls.ROW_NORM_K = 16, 4096
+    monkeypatch.setattr(eng, "ho", calls)
+    x, y, b = torch.zeros(32, 64), torch.zeros(32, 64), torch.zeros(64)
+    w = torch.zeros(128, 64)
+    lw = {"w": w, "w_q": w, "w_s": torch.zeros(128)}
+    eng.GPUModel._linear(fake(fp8=fp8), lw, "w", x, y, M=M, bias=b, act=1)
+    name, _, kw = calls[-1]
+    assert name == ("gemm_fp8" if fp8 else "gemm") if M > 16 else \
+        ("gemv_fp8" if fp8 and M == 1 else "row_gemm")
+    assert (kw["res"] if name == "gemv_fp8" else kw["bias"]) is b
+    assert kw["act"] == 1 and kw.get("glu", True)
+
+
+def test_linear_refuses_what_a_path_cannot_add(monkeypatch):
+    calls = Calls()
+    calls.FEW_ROWS, calls.ROW_NORM_K = 16, 4096
+    monkeypatch.setattr(eng, "ho", calls)
+    x, w = torch.zeros(32, 64), torch.zeros(128, 64)
+    lw = {"w_q": w, "w_s": w, "w_q4": w, "w_e4": w}
+    with pytest.raises(AssertionError):         # one row: one of them
+        eng.GPUModel._linear(fake(fp8=True), lw, "w", x, x, M=1, res=x,
+                             bias=x[0])
+    with pytest.raises(AssertionError):         # gate and up apart
+        eng.GPUModel._linear(fake(fp8=True, wq4=True), lw, "w", x, x, M=20,
+                             res=x, act=0)
+    assert not calls
