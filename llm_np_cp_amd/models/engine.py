@@ -319,19 +319,20 @@ class GPUModel(DecodeLoop):
         self.sin_t = torch.from_numpy(np.sin(freqs).astype(np.float32)).to(dev)
 
         PC = self.PC = min(prefill_chunk, max(256, self.max_seq))
+        R = max(PC, self.max_batch)    # rows of a prompt's or a group's pass
         H, I = self.H, self.inter_l
-        self.b_h = torch.zeros(PC, H, **bf)
-        self.b_xn = torch.zeros(PC, H, **bf)
-        self.b_t1 = torch.zeros(PC, H, **bf)
+        self.b_h = torch.zeros(R, H, **bf)
+        self.b_xn = torch.zeros(R, H, **bf)
+        self.b_t1 = torch.zeros(R, H, **bf)
         # q | k | v of a row, from one projection
         nqkv = (self.nh_l + 2 * self.kvh_l) * hd
-        self.b_rqkv = torch.zeros(PC, nqkv, **bf)
-        self.b_att = torch.zeros(PC, self.nh_l * hd, **bf)
+        self.b_rqkv = torch.zeros(R, nqkv, **bf)
+        self.b_att = torch.zeros(R, self.nh_l * hd, **bf)
         # act(gate) * up; of each of a row's experts
-        pairs = PC * (self.topk if self.moe else 1)
+        pairs = R * (self.topk if self.moe else 1)
         self.b_gate = torch.zeros(pairs, I, **bf)
         if self.wq4:          # its prompts have gate and up apart
-            self.b_up = torch.zeros(PC, I, **bf)
+            self.b_up = torch.zeros(R, I, **bf)
         # fp32 parts of products that split K, and of attention that splits
         # its keys.  A few long rows beside many outputs can take more than a
         # short chunk of a prompt does.
@@ -341,14 +342,14 @@ class GPUModel(DecodeLoop):
         kinds = ["fp4"] * self.wq4 + ["fp8"] * self.keep_fp8 \
             if self.fp8 else ["bf16"]
         self.b_gemm_acc = torch.zeros(
-            max([PC * max(I, H)] +
+            max([R * max(I, H)] +
                 [ho.row_gemm_room(k, *p) for k in kinds for p in few]),
             dtype=torch.float32, device=dev)
         if self.fp8:
             # activation-quant scratch for the fp8 MFMA prefill GEMMs
             kmax = max(H, I, self.nh_l * hd)
-            self.b_xq = torch.zeros(PC * kmax, dtype=torch.uint8, device=dev)
-            self.b_sx = torch.zeros(PC, dtype=torch.float32, device=dev)
+            self.b_xq = torch.zeros(R * kmax, dtype=torch.uint8, device=dev)
+            self.b_sx = torch.zeros(R, dtype=torch.float32, device=dev)
             if self.moe:
                 self.b_aq = torch.zeros(pairs * I, dtype=torch.uint8,
                                         device=dev)
@@ -370,9 +371,9 @@ class GPUModel(DecodeLoop):
         self.b_qkv = torch.zeros((self.nh_l + 2 * self.kvh_l) * hd, **bf)
         if self.moe:
             E = cfg.num_local_experts
-            self.moe_idx = torch.zeros(PC * self.topk, dtype=torch.int32,
+            self.moe_idx = torch.zeros(R * self.topk, dtype=torch.int32,
                                        device=dev)
-            self.moe_w = torch.zeros(PC * self.topk, dtype=torch.float32,
+            self.moe_w = torch.zeros(R * self.topk, dtype=torch.float32,
                                      device=dev)
             self.moe_order = torch.zeros(pairs + 3 * (pairs // 32 + E),
                                          dtype=torch.int32, device=dev)
@@ -1100,7 +1101,7 @@ class GPUModel(DecodeLoop):
         cfg = self.config
         eps = cfg.rms_norm_eps
         H, I = self.H, self.inter_l
-        h = self.b_h            # (PC, H): rows 0..B = per-seq h
+        h = self.b_h            # rows 0..B = per-seq h
         hb = self.bt_hb         # gemma ping-pong
         t1, t2, gu = self.bt_t1, self.bt_t2, self.bt_gu
         qkvw = (self.nh_l + 2 * self.kvh_l) * self.hd

@@ -93,3 +93,17 @@ def test_ranges_follow_the_active_rows(monkeypatch, kv_dtype):
         assert not m.bt_attn_cnt.any()
         # sums in another order, bf16 results
         assert (got[M] - got[32][:M]).norm() < 2.0 ** -8 * got[M].norm()
+
+
+# buffers hold a group's rows where a prompt's chunk is shorter
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+def test_chunks_shorter_than_the_group(dtype):
+    prompts = [[5, 6, 7], [8, 9], [1], [2, 3, 4, 5, 6]] * 5
+    ids, h = [], []
+    for chunk in (2, 64):
+        m = engine(hidden=128, max_batch=20, dtype=dtype, prefill_chunk=chunk)
+        ids.append(m.generate_tokens_batch(prompts, 6))
+        h.append(m.b_h[:20].float())
+        assert m.b_att.shape[0] >= 20 and m.PC == chunk
+    assert (h[0] - h[1]).norm() < 0.05 * h[1].norm()
+    assert (ids[0] == ids[1]).mean() > 0.9          # ties of close logits
