@@ -43,8 +43,8 @@ LIBS = {
     "lightning": ["lightning.hip"],
     "moe": ["moe.hip"],
 }
-HEADERS = ["attn_prefill.h", "attn_split.h", "common.h", "gemm_tile.h", "hybrid.h", "mingru.h",
-           "moe.h"]
+HEADERS = ["attn_prefill.h", "attn_split.h", "common.h", "gemm_tile.h",
+           "gemv.h", "hybrid.h", "mingru.h", "moe.h"]
 # Packed fp32 VALU forms are kept out of all device code: some of them
 # have returned wrong results on this hardware.  (The host pass warns that
 # it does not know the feature.)

@@ -1,6 +1,8 @@
 """The engine's choices on the host, without a GPU: what goes to which
 kernel with which arguments."""
 
+import os
+import re
 import types
 
 import pytest
@@ -58,3 +60,13 @@ def test_linear_refuses_what_a_path_cannot_add(monkeypatch):
         eng.GPUModel._linear(fake(fp8=True, wq4=True), lw, "w", x, x, M=20,
                              res=x, act=0)
     assert not calls
+
+
+def test_every_header_is_known_to_the_build():
+    from csrc.build import CSRC, HEADERS, LIBS
+
+    there = [f for f in os.listdir(CSRC) if f.endswith((".h", ".hip"))]
+    names = {n for f in there for n in re.findall(
+        r'#include "(.+?)"', open(os.path.join(CSRC, f)).read())}
+    assert names <= set(HEADERS) <= set(there)
+    assert {s for src in LIBS.values() for s in src} <= set(there)
