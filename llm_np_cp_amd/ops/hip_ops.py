@@ -139,8 +139,9 @@ def _ptr(t) -> int:
 
 
 def _ld(t, width: int) -> int:
-    """Elements from row to row (rows of one buffer may lie in another's)."""
-    return t.stride(0) if t.dim() > 1 else width
+    """Elements from row to row: rows of one buffer may lie in another's;
+    what is in one piece may have any shape."""
+    return width if t.is_contiguous() else t.stride(0)
 
 
 # ----------------------------------------------------------------------

@@ -70,3 +70,19 @@ def test_every_header_is_known_to_the_build():
         r'#include "(.+?)"', open(os.path.join(CSRC, f)).read())}
     assert names <= set(HEADERS) <= set(there)
     assert {s for src in LIBS.values() for s in src} <= set(there)
+
+
+# one piece of any shape: rows follow one another; parts of a fused row: they
+# are as far apart as it is long (a single row may say anything)
+def test_distance_of_rows():
+    from llm_np_cp_amd.ops.hip_ops import _ld
+
+    M, nh, kvh, hd = 5, 4, 2, 16
+    q = torch.zeros(M, nh * hd)
+    for shape in ((M, nh * hd), (M * nh * hd,), (M, nh, hd), (1, M, nh, hd),
+                  (1, M * nh * hd), (M * nh, hd)):
+        assert _ld(q.view(shape), nh * hd) == nh * hd
+    fused = torch.zeros(M, (nh + 2 * kvh) * hd)
+    for t, w in zip(fused.split([nh * hd, kvh * hd, kvh * hd], 1),
+                    (nh * hd, kvh * hd, kvh * hd)):
+        assert _ld(t, w) == fused.shape[1]
