@@ -158,15 +158,18 @@ STAGE_NORM_EMBED = 4
 
 def _gemv(wt, W, ws, we, K, x, y, res, softcap, stage, x2, g, act, eps,
           maxblocks, g2, escale, eidx, wstride, sstride, oscale, glu):
+    N, ne = W.shape[0] // (2 if glu else 1), 1
+    if eidx is not None:        # experts that there are rows for
+        ne = min(eidx.numel(), y.numel() // N if glu else x.numel() // K)
+        assert oscale is None or oscale.numel() >= ne
     _check(lib().launch_gemv(
         _ptr(W), _ptr(ws), _ptr(we), _ptr(x), _ptr(x2), _ptr(g), _ptr(g2),
-        _ptr(y), _ptr(res), wt, W.shape[0] // (2 if glu else 1), K, stage,
-        act, int(glu), int(x.dtype == torch.float32),
+        _ptr(y), _ptr(res), wt, N, K, stage, act, int(glu),
+        int(x.dtype == torch.float32),
         int(y.dtype == torch.float32), ctypes.c_float(eps),
         ctypes.c_float(softcap), ctypes.c_float(escale), maxblocks,
-        _ptr(eidx), 1 if eidx is None else eidx.numel(),
-        ctypes.c_long(wstride), ctypes.c_long(sstride), _ptr(oscale),
-        _stream()), "gemv")
+        _ptr(eidx), ne, ctypes.c_long(wstride), ctypes.c_long(sstride),
+        _ptr(oscale), _stream()), "gemv")
 
 
 def gemv(W: torch.Tensor, x: torch.Tensor, y: torch.Tensor,
@@ -183,8 +186,8 @@ def gemv(W: torch.Tensor, x: torch.Tensor, y: torch.Tensor,
     x2 = token-id i32, res = persisted h) on the way.  x is bf16, or fp32
     (RAW).  glu: W holds gate rows, then up rows: y[N/2] = act(gate) * up.
     eidx/wstride/oscale: W of expert *eidx, its result times *oscale; of
-    several experts the results are added up (x [n, K]), with glu they stand
-    one after the other.  nt and rpw are kept for callers: the kernel streams
+    several experts (x [n, K]) the results are added up, with glu they stand
+    one after the other (y [n, N/2]).  nt and rpw are kept for callers: the kernel streams
     W past the caches and picks its rows by itself."""
     _gemv(0, W, None, None, W.shape[1], x, y, res, softcap, stage, x2, g,
           act, eps, maxblocks, g2, escale, eidx, wstride, 0, oscale, glu)

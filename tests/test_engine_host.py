@@ -86,3 +86,22 @@ def test_distance_of_rows():
     for t, w in zip(fused.split([nh * hd, kvh * hd, kvh * hd], 1),
                     (nh * hd, kvh * hd, kvh * hd)):
         assert _ld(t, w) == fused.shape[1]
+
+
+# the first of a longer list of experts, unless there are rows for more
+@pytest.mark.parametrize("listed,rows,glu,taken", [
+    (1, 1, False, 1), (3, 1, False, 1), (3, 3, False, 3), (9, 2, False, 2),
+    (3, 1, True, 1), (2, 2, True, 2), (2, 5, True, 2)])
+def test_experts_there_are_rows_for(monkeypatch, listed, rows, glu, taken):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    N, K, args = 32, 64, []
+    lib = types.SimpleNamespace(
+        launch_gemv=lambda *a: args.append(dict(zip(range(99), a))) or 0)
+    monkeypatch.setattr(ho, "lib", lambda: lib)
+    monkeypatch.setattr(ho, "_stream", lambda: 0)
+    x, y = torch.zeros(1 if glu else rows, K), torch.zeros(rows if glu else 1, N)
+    W = torch.zeros(N * (2 if glu else 1), K)
+    idx, p = torch.zeros(listed, dtype=torch.int32), torch.zeros(listed)
+    ho.gemv(W, x, y, eidx=idx, wstride=N * K, oscale=p, glu=glu)
+    assert args[0][22] == taken and args[0][10] == N and args[0][11] == K
