@@ -883,10 +883,10 @@ DEVINL int unpack_idx(uint64_t p) { return 0x7fffffff - (int)(uint32_t)p; }
 // pass 1 (min-p only): global max logit -> gmax[b] (packed).
 // Batched: grid.y = sequence row b (lbf16: logits stored bf16 — the
 // batched lm_head GEMM path emits bf16 rows).
-#define SMP_NT 512      // threads of a block
 #define SMP_U 4         // logits of a thread at a time
 
-extern "C" __global__ void __launch_bounds__(SMP_NT)
+template <int NT>       // threads of a block
+__global__ void __launch_bounds__(NT)
 k_logit_max(const void* __restrict__ logits, int V, int lbf16,
             unsigned long long* __restrict__ gmax,
             uint64_t* __restrict__ ctr) {
@@ -900,17 +900,17 @@ k_logit_max(const void* __restrict__ logits, int V, int lbf16,
   const u16* lh = (const u16*)logits + (size_t)b * V;
   float mv = -INFINITY;
   int mi = 0;
-  for (int i0 = blockIdx.x * SMP_NT * SMP_U + threadIdx.x; i0 < V;
-       i0 += gridDim.x * SMP_NT * SMP_U) {
+  for (int i0 = blockIdx.x * NT * SMP_U + threadIdx.x; i0 < V;
+       i0 += gridDim.x * NT * SMP_U) {
     float v[SMP_U];
 #pragma unroll
     for (int u = 0; u < SMP_U; u++) {
-      const int i = min(i0 + u * SMP_NT, V - 1);
+      const int i = min(i0 + u * NT, V - 1);
       v[u] = lbf16 ? b2f(lh[i]) : lf[i];
     }
 #pragma unroll
     for (int u = 0; u < SMP_U; u++) {
-      const int i = min(i0 + u * SMP_NT, V - 1);
+      const int i = min(i0 + u * NT, V - 1);
       if (v[u] > mv || (v[u] == mv && i < mi)) { mv = v[u]; mi = i; }
     }
   }
@@ -920,12 +920,12 @@ k_logit_max(const void* __restrict__ logits, int V, int lbf16,
     uint64_t o = __shfl_xor((unsigned long long)pk, w);
     if (o > pk) pk = o;
   }
-  __shared__ unsigned long long ws[SMP_NT / 64];
+  __shared__ unsigned long long ws[NT / 64];
   if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = pk;
   __syncthreads();
   if (threadIdx.x == 0) {
     uint64_t b = ws[0];
-    for (int w = 1; w < SMP_NT / 64; w++) if (ws[w] > b) b = ws[w];
+    for (int w = 1; w < NT / 64; w++) if (ws[w] > b) b = ws[w];
     atomicMax(gmax, (unsigned long long)b);
   }
 }
@@ -937,7 +937,8 @@ k_logit_max(const void* __restrict__ logits, int V, int lbf16,
 // Temperature folds into both the min-p keep-set and the Gumbel score:
 //   p_i(T) >= min_p * p_max(T)  <=>  l_i >= l_max + T*ln(min_p)
 //   Gumbel-argmax over p(T)     <=>  argmax of l_i/T + G_i
-extern "C" __global__ void __launch_bounds__(SMP_NT)
+template <int NT>
+__global__ void __launch_bounds__(NT)
 k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
               long ring_stride, float min_p,
               int greedy, uint64_t seed, float inv_temp,
@@ -958,17 +959,17 @@ k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
   const uint32_t c = (uint32_t)(*ctr) ^ ((uint32_t)b * 0x85ebca6bu);
   float bv = -INFINITY;
   int bi = 0x7fffffff;
-  for (int i0 = blockIdx.x * SMP_NT * SMP_U + threadIdx.x; i0 < V;
-       i0 += gridDim.x * SMP_NT * SMP_U) {
+  for (int i0 = blockIdx.x * NT * SMP_U + threadIdx.x; i0 < V;
+       i0 += gridDim.x * NT * SMP_U) {
     float vs[SMP_U];
 #pragma unroll
     for (int u = 0; u < SMP_U; u++) {
-      const int i = min(i0 + u * SMP_NT, V - 1);
+      const int i = min(i0 + u * NT, V - 1);
       vs[u] = lbf16 ? b2f(lh[i]) : lf[i];
     }
 #pragma unroll
     for (int u = 0; u < SMP_U; u++) {
-      const int i = min(i0 + u * SMP_NT, V - 1);
+      const int i = min(i0 + u * NT, V - 1);
       const float v = vs[u];
       if (v < thresh) continue;
       float sc = v;
@@ -987,13 +988,13 @@ k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
     uint64_t o = __shfl_xor((unsigned long long)pk, w);
     if (o > pk) pk = o;
   }
-  __shared__ unsigned long long ws[SMP_NT / 64];
+  __shared__ unsigned long long ws[NT / 64];
   __shared__ int lastflag;
   if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = pk;
   __syncthreads();
   if (threadIdx.x == 0) {
     uint64_t b = ws[0];
-    for (int w = 1; w < SMP_NT / 64; w++) if (ws[w] > b) b = ws[w];
+    for (int w = 1; w < NT / 64; w++) if (ws[w] > b) b = ws[w];
     atomicMax(pick, (unsigned long long)b);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     int t = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_ACQ_REL,
@@ -1027,22 +1028,40 @@ extern "C" hipError_t launch_sample(const void* logits, int V, int lbf16,
                                     void* out_ring, void* nout,
                                     void* len_ptr, int bump_len,
                                     hipStream_t stream) {
-  // Blocks queue up at one address, twice in the pick: both launches took
-  // 23.3 us for a vocabulary of 128256 in 501 blocks of 256 logits, in 63 of
-  // 2048 9.2 (32768: 11.1 and 9.0).  The rows of a group queue up apart.
-  int blocks = (V + SMP_NT * SMP_U - 1) / (SMP_NT * SMP_U);
-  const int most = batch > 4 ? 16 : 64 / (batch > 0 ? batch : 1);
+  // Every block queues up at a word of its row, twice in the pick, and the
+  // words of a group's rows share lines: some 25 ns a block, of whatever row.
+  // A trip of a block through its logits takes some 0.65 us.  One row: 63
+  // blocks of 2048 logits, 128256 of them greedy in 5.3 us (501 blocks of 256:
+  // 14.0).  A group takes larger blocks, and fewer of a row where there are
+  // many; us, greedy and min-p, in blocks of 256 threads, 16 of a row or more
+  // (as before) -> in 16 of 512 -> here:
+  //   16 rows of 32768   10.3, 16.5 ->  9.5, 14.4 ->  7.1, 11.8
+  //   16 rows of 256000  20.9, 33.4 -> 15.6, 25.3 -> 12.5, 20.6
+  //   64 rows of 128256  35.0, 48.6 -> 33.0, 48.8 -> 19.8, 34.2
+  //   64 rows of 256000  43.8, 65.8 -> 49.6, 71.6 -> 34.1, 52.6
+  const int nt = batch > 4 ? 1024 : 512;
+  int blocks = (V + nt * SMP_U - 1) / (nt * SMP_U);
+  const int most = batch > 32  ? 8
+                   : batch > 4 ? 16
+                               : 64 / (batch > 0 ? batch : 1);
   if (blocks > most) blocks = most;
-  if (!greedy)
-    hipLaunchKernelGGL(k_logit_max, dim3(blocks, batch), dim3(SMP_NT), 0,
-                       stream, logits, V, lbf16, (unsigned long long*)gmax,
-                       (uint64_t*)ctr);
-  hipLaunchKernelGGL(k_sample_pick, dim3(blocks, batch), dim3(SMP_NT), 0,
-                     stream, logits, V, lbf16, ring_stride, min_p, greedy,
-                     seed, inv_temp,
-                     (unsigned long long*)gmax, (uint64_t*)ctr,
-                     (unsigned long long*)pick, (int*)cnt, (int*)next_token,
-                     (int*)out_ring, (int*)nout, (int*)len_ptr, bump_len);
+#define SMP_GO(NT)                                                           \
+  if (!greedy)                                                               \
+    hipLaunchKernelGGL(k_logit_max<NT>, dim3(blocks, batch), dim3(NT), 0,    \
+                       stream, logits, V, lbf16, (unsigned long long*)gmax,  \
+                       (uint64_t*)ctr);                                      \
+  hipLaunchKernelGGL(k_sample_pick<NT>, dim3(blocks, batch), dim3(NT), 0,    \
+                     stream, logits, V, lbf16, ring_stride, min_p, greedy,   \
+                     seed, inv_temp, (unsigned long long*)gmax,              \
+                     (uint64_t*)ctr, (unsigned long long*)pick, (int*)cnt,   \
+                     (int*)next_token, (int*)out_ring, (int*)nout,           \
+                     (int*)len_ptr, bump_len)
+  if (nt == 1024) {
+    SMP_GO(1024);
+  } else {
+    SMP_GO(512);
+  }
+#undef SMP_GO
   return hipGetLastError();
 }
 

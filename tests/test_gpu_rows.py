@@ -464,3 +464,39 @@ def test_experts_of_many_rows(M, E, top, kind):
                       * p.double()[..., None]).sum(1)
     assert off(out, z) < 2.0 ** -8 * top            # bf16 after each expert
     assert (a[pairs] == 7.0).all() and (y[pairs] == 7.0).all()
+
+
+# a row, a few, a group in larger blocks, a large one in fewer; a vocabulary of
+# one, one short of a block's trip, one more, several trips
+@pytest.mark.parametrize("B", [1, 4, 5, 33])
+@pytest.mark.parametrize("V", [1, 63, 4095, 4097, 40001, 70000])
+def test_sampled_rows(B, V):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    logits = normal(33, V, seed=11, scale=2.0)
+    logits[:, V // 2] = logits[:, V // 3]           # ties: the first of them
+    logits[0, V - 1] = 60.0
+    i32 = dict(dtype=torch.int32, device="cuda")
+
+    def sample(rows, greedy):
+        n = len(rows)
+        i64 = dict(dtype=torch.int64, device="cuda")
+        ctr, gmax, pick = (torch.zeros(k, **i64) for k in (1, n, n))
+        cnt, tok, at, ln = (torch.zeros(n, **i32) for _ in range(4))
+        ring = torch.zeros(n, 4, **i32)
+        for _ in range(2):
+            ho.sample(rows, 0.05, greedy, 7, ctr, gmax, pick, tok, ring, at,
+                      ln, cnt=cnt, batch=n)
+        assert not gmax.any() and not pick.any() and not cnt.any()
+        assert (at == 2).all() and (ln == 2).all()
+        return ring[:, :2]
+
+    got = sample(logits[:B], True)
+    want = torch.from_numpy(logits[:B].float().cpu().numpy().argmax(1)).cuda()
+    assert (got == want[:, None]).all()
+    got = sample(logits[:B], False)
+    # noise is a row's and a token's, whoever looks at it
+    assert (got[:4] == sample(logits[:4], False)[:B]).all()
+    x = logits[:B].float()
+    kept = x.gather(1, got.long()) >= x.amax(1, keepdim=True) + math.log(0.05)
+    assert kept.all() and (V < 4000 or B < 5 or len(got.unique()) > 3)
