@@ -121,12 +121,16 @@ DEVINL void gv_meet() {
 }
 
 // J loads of 1 KB (64 lanes x 16 bytes) a wave and row; R rows in flight
-// while R others are multiplied
-template <int WT, int J, int R, bool RAW>
+// while R others are multiplied.  T: x as it is (GV_RAW), staged by all
+// threads of the block, 2048 elements at a time (T times), or by each group of
+// waves that covers K by itself (GV_OWN: rows too long for T).
+enum { GV_RAW = 0, GV_OWN = -1 };
+template <int WT, int J, int R, int T>
 __global__ void __launch_bounds__(512) k_gemv(GvArgs a) {
   constexpr int E = gv_e<WT>();
-  __shared__ float ssq[8];
-  // [kw][rows of the block], then a stretch of x for each wave to turn
+  constexpr bool RAW = T == GV_RAW, ALL = T > 0;
+  __shared__ float ssq[2][8];
+  // [kw][rows of the block], then x (or a stretch for each wave to turn)
   extern __shared__ __attribute__((aligned(16))) float red[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -190,121 +194,162 @@ __global__ void __launch_bounds__(512) k_gemv(GvArgs a) {
       in[j] = c < C;
       pc[j] = in[j] ? c : C - 1;
     }
-    // x, ahead of W: it comes from L2 and loads return in order.  Here lane l
-    // has elements 4l.. of every 256 of the wave's stretch: whole lines.
     constexpr int Q = E / 4;
-    gv_f4 v[J][Q], gg[RAW ? 1 : J][Q];
-    gv_u2 hr[RAW ? 1 : J][Q];
-    auto at = [&](int j, int i) {
-      return ((c0 + (j * kwe + (kw & (kwe - 1))) * 64) * Q + i * 64 + lane) * 4;
-    };
-    auto clip = [&](int e) { return min(e, a.K - 4); };
-    auto each = [&](auto f) {
-#pragma unroll
-      for (int j = 0; j < J; j++)
-#pragma unroll
-        for (int i = 0; i < Q; i++) f(j, i);
-    };
-    auto bf = [](gv_u2 u, int k) {
-      return __uint_as_float(k & 1 ? u[k >> 1] & 0xffff0000u : u[k >> 1] << 16);
-    };
+    f4v* const turn = (f4v*)(red + ((a.kw * rs + 3) & ~3));
     const u16* xs = (const u16*)a.x;
     if (stage == STAGE_NORM_EMBED)
       xs += (size_t)(*(const int*)a.x2) * a.K;
     if (a.ne > 1 && gridDim.y == 1) xs += (size_t)ex * a.K * (a.x_f32 ? 2 : 1);
-    if (RAW && a.x_f32) {
-      each([&](int j, int i) {
-        v[j][i] = *(const gv_f4*)((const float*)xs + clip(at(j, i)));
-      });
-      load(wa, xa, 0);
-    } else {
-      gv_u2 xr[J][Q];
-      each([&](int j, int i) {
-        xr[j][i] = *(const gv_u2*)(xs + clip(at(j, i)));
-      });
-      if constexpr (!RAW) {
-        if (stage == STAGE_GLU || stage == STAGE_NORM2)
-          each([&](int j, int i) {
-            hr[j][i] = *(const gv_u2*)(a.x2 + clip(at(j, i)));
-          });
-        if (stage != STAGE_GLU) {
-          const float* g = stage == STAGE_NORM2 ? a.g2 : a.g;
-          each([&](int j, int i) {
-            gg[j][i] = *(const gv_f4*)(g + clip(at(j, i)));
-          });
-        }
-      }
-      load(wa, xa, 0);
-      each([&](int j, int i) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) v[j][i][k] = bf(xr[j][i], k);
-      });
-    }
-    if constexpr (!RAW) {
+    auto clip = [&](int e) { return min(e, a.K - 4); };
+    auto bf = [](gv_u2 u, int k) {
+      return __uint_as_float(k & 1 ? u[k >> 1] & 0xffff0000u : u[k >> 1] << 16);
+    };
+    // What a stage does to NV pieces of four, at(i) the first element of the
+    // i-th: v from x, hr from x2, gg and g1 from the last and the first norm's
+    // g.  sums of n of the block's waves from w0 on; keeps: hout is written.
+    auto staged = [&](auto& v, auto& hr, auto& gg, auto& g1, auto at, int w0,
+                      int n, bool keeps) {
+      constexpr int NV = sizeof(v) / sizeof(v[0]);
       // 1 / root mean square over all of x
-      auto norm = [&] {
+      auto norm = [&](float* sq) {
         float ss = 0.f;
-        each([&](int j, int i) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
           float t = 0.f;
 #pragma unroll
-          for (int k = 0; k < 4; k++) t += v[j][i][k] * v[j][i][k];
-          ss += at(j, i) < a.K ? t : 0.f;
-        });
+          for (int k = 0; k < 4; k++) t += v[i][k] * v[i][k];
+          ss += at(i) < a.K ? t : 0.f;
+        }
         ss = gv_sum(ss);
-        gv_meet();                         // the last sums have been read
-        if (lane == 0) ssq[wave] = ss;
+        if (lane == 0) sq[wave] = ss;
         gv_meet();
         float t = 0.f;
-        for (int k = 0; k < a.kw; k++) t += ssq[(nw << a.kwl) + k];
+        for (int k = 0; k < n; k++) t += sq[w0 + k];
         return rsqrtf(t / (float)a.K + a.eps);
       };
       auto round = [](float f) { return WT == GV_BF16 ? b2f(f2b(f)) : f; };
       if (stage == STAGE_GLU) {
-        each([&](int j, int i) {
+#pragma unroll
+        for (int i = 0; i < NV; i++)
 #pragma unroll
           for (int k = 0; k < 4; k++)
-            v[j][i][k] = round(gv_act(v[j][i][k], a.act) * bf(hr[j][i], k));
-        });
-      } else {
-        if (stage != STAGE_NORM) {         // the residual stream is bf16
-          const bool keeps = blockIdx.x == 0 && nw == 0;
-          const float rn = stage == STAGE_NORM2 ? norm() : a.escale;
-          each([&](int j, int i) {
-            const int e = at(j, i);
-            u16 o[4];
+            v[i][k] = round(gv_act(v[i][k], a.act) * bf(hr[i], k));
+        return;
+      }
+      if (stage != STAGE_NORM) {           // the residual stream is bf16
+        const float rn = stage == STAGE_NORM2 ? norm(ssq[1]) : a.escale;
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-              float f = v[j][i][k] * rn;
-              if (stage == STAGE_NORM2)
-                f = f * a.g[clip(e) + k] + bf(hr[j][i], k);
-              o[k] = f2b(f);
-              v[j][i][k] = b2f(o[k]);
-            }
-            if (keeps && e < a.K) *(gv_u2*)(a.hout + e) = *(gv_u2*)o;
-          });
+        for (int i = 0; i < NV; i++) {
+          const int e = at(i);
+          u16 o[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++) {
+            float f = v[i][k] * rn;
+            if (stage == STAGE_NORM2) f = f * g1(i, k) + bf(hr[i], k);
+            o[k] = f2b(f);
+            v[i][k] = b2f(o[k]);
+          }
+          if (keeps && e < a.K) *(gv_u2*)(a.hout + e) = *(gv_u2*)o;
         }
-        const float rn = norm();
-        each([&](int j, int i) {
+      }
+      const float rn = norm(ssq[0]);
 #pragma unroll
-          for (int k = 0; k < 4; k++)
-            v[j][i][k] = round(v[j][i][k] * rn * gg[j][i][k]);
-        });
+      for (int i = 0; i < NV; i++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[i][k] = round(v[i][k] * rn * gg[i][k]);
+    };
+    // x, ahead of W: it comes from L2 and loads return in order.
+    if constexpr (ALL) {
+      auto at = [&](int i) { return (i * 512 + tid) * 4; };
+      gv_f4 v[T], gg[T], ga[T];
+      gv_u2 xr[T], hr[T];
+#pragma unroll
+      for (int i = 0; i < T; i++) xr[i] = *(const gv_u2*)(xs + clip(at(i)));
+      if (stage == STAGE_GLU || stage == STAGE_NORM2)
+#pragma unroll
+        for (int i = 0; i < T; i++)
+          hr[i] = *(const gv_u2*)(a.x2 + clip(at(i)));
+      if (stage != STAGE_GLU) {
+        const float* g = stage == STAGE_NORM2 ? a.g2 : a.g;
+#pragma unroll
+        for (int i = 0; i < T; i++) gg[i] = *(const gv_f4*)(g + clip(at(i)));
+        if (stage == STAGE_NORM2)
+#pragma unroll
+          for (int i = 0; i < T; i++)
+            ga[i] = *(const gv_f4*)(a.g + clip(at(i)));
+      }
+      load(wa, xa, 0);
+#pragma unroll
+      for (int i = 0; i < T; i++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[i][k] = bf(xr[i], k);
+      auto g1 = [&](int i, int k) { return ga[i][k]; };
+      staged(v, hr, gg, g1, at, 0, 8, blockIdx.x == 0);
+#pragma unroll
+      for (int i = 0; i < T; i++) {
+        const int n = i * 512 + tid;
+        if (n * 4 < a.K) turn[n ^ (n / Q & (Q - 1))] = v[i];
+      }
+      gv_meet();
+    }
+    // Here lane l has elements 4l.. of every 256 of the wave's stretch: whole
+    // lines.
+    constexpr int NV = ALL ? 1 : J * Q;
+    gv_f4 v[NV];
+    auto at = [&](int i) {
+      return ((c0 + (i / Q * kwe + (kw & (kwe - 1))) * 64) * Q + i % Q * 64 +
+              lane) * 4;
+    };
+    auto each = [&](auto f) {
+#pragma unroll
+      for (int i = 0; i < NV; i++) f(i);
+    };
+    if (RAW && a.x_f32) {
+      each([&](int i) {
+        v[i] = *(const gv_f4*)((const float*)xs + clip(at(i)));
+      });
+      load(wa, xa, 0);
+    } else if constexpr (!ALL) {
+      gv_f4 gg[NV];
+      gv_u2 xr[NV], hr[NV];
+      each([&](int i) { xr[i] = *(const gv_u2*)(xs + clip(at(i))); });
+      if constexpr (!RAW) {
+        if (stage == STAGE_GLU || stage == STAGE_NORM2)
+          each([&](int i) { hr[i] = *(const gv_u2*)(a.x2 + clip(at(i))); });
+        if (stage != STAGE_GLU) {
+          const float* g = stage == STAGE_NORM2 ? a.g2 : a.g;
+          each([&](int i) { gg[i] = *(const gv_f4*)(g + clip(at(i))); });
+        }
+      }
+      load(wa, xa, 0);
+      each([&](int i) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[i][k] = bf(xr[i], k);
+      });
+      if constexpr (!RAW) {
+        auto g1 = [&](int i, int k) { return a.g[clip(at(i)) + k]; };
+        staged(v, hr, gg, g1, at, nw << a.kwl, a.kw,
+               blockIdx.x == 0 && nw == 0);
       }
     }
     // each lane's E elements in a row, by way of LDS
-    f4v* turn = (f4v*)(red + ((a.kw * rs + 3) & ~3)) + wave * (64 * Q);
     float xv[J][E];
     gv_b2 xb2[J][4];                       // bf16 weights: x as it is
 #pragma unroll
     for (int j = 0; j < J; j++) {
+      f4v* to = turn + wave * (64 * Q);
+      if constexpr (ALL) {
+        to = turn + (j * kwe + (kw & (kwe - 1))) * (64 * Q);
+      } else {
 #pragma unroll
-      for (int i = 0; i < Q; i++) {
-        const int n = i * 64 + lane;
-        turn[n ^ (n / Q & (Q - 1))] = v[j][i];
+        for (int i = 0; i < Q; i++) {
+          const int n = i * 64 + lane;
+          to[n ^ (n / Q & (Q - 1))] = v[j * Q + i];
+        }
       }
 #pragma unroll
       for (int i = 0; i < Q; i++) {
-        const f4v t = turn[lane * Q + (i ^ (lane & (Q - 1)))];
+        const f4v t = to[lane * Q + (i ^ (lane & (Q - 1)))];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
           if constexpr (WT == GV_BF16) xb2[j][i * 2 + k / 2][k & 1] = (__bf16)t[k];
@@ -408,28 +453,59 @@ __global__ void __launch_bounds__(512) k_gemv(GvArgs a) {
 
 #define GV_ROOM (80 * 1024)                // LDS for the sums of a block
 
-template <int WT, int J, int R, bool RAW>
+template <int WT, int J, int R, int T>
 static hipError_t gv_launch(const GvArgs& a, dim3 grid, hipStream_t s) {
   static const hipError_t raised = hipFuncSetAttribute(
-      (const void*)&k_gemv<WT, J, R, RAW>,
+      (const void*)&k_gemv<WT, J, R, T>,
       hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
   (void)raised;
-  hipLaunchKernelGGL((k_gemv<WT, J, R, RAW>), grid, dim3(64 * a.kw * a.nw),
+  const int waves = T > 0 ? (1 << a.kwel) * J : a.kw * a.nw;
+  hipLaunchKernelGGL((k_gemv<WT, J, R, T>), grid, dim3(64 * a.kw * a.nw),
                      ((size_t)a.kw * (a.glu ? 2 : 1) * a.rpb + 3 +
-                      a.kw * a.nw * 64 * gv_e<WT>()) * 4, s, a);
+                      waves * 64 * gv_e<WT>()) * 4, s, a);
   return hipGetLastError();
+}
+
+// How x is staged: by all threads of a block, each element once, up to 8192 of
+// them (every model's rows).  By each group of waves that covers K for itself
+// two norms took longer than the 256 threads that staged into LDS before; us,
+// one norm and two, that -> by groups -> here:
+//   64x512 e4m3         3.6, 4.2 -> 4.3, 6.4 -> 3.6, 4.0
+//   2048x16384 e4m3     8.3, 9.4 -> 7.8, 13.0 -> 6.8, 7.2
+//   2304x4096 bf16      5.9, 7.6 -> 6.0, 8.5 -> 5.4, 6.3
+//   3584x4608 MXFP4     7.0, 8.5 -> 7.0, 12.0 -> 5.9, 6.7
+//   8192x10240 e4m3     16.9, 18.1 -> 14.6, 19.9 -> 14.2, 15.5
+// (weights of the small ones from L2).
+template <int WT, int J, int R>
+static hipError_t gv_stage(const GvArgs& a, dim3 grid, hipStream_t s) {
+  if (a.stage == STAGE_RAW) return gv_launch<WT, J, R, GV_RAW>(a, grid, s);
+  // up to 8192 elements are two loads at most, one of MXFP4
+  if constexpr (J <= (WT == GV_FP4 ? 1 : 2)) {
+    if (a.K <= 2048)
+      return gv_launch<WT, J, R, WT == GV_BF16 && J == 2 ? 2 : 1>(a, grid, s);
+    if constexpr (WT == GV_FP4 || J == 2) {
+      if (a.K <= 4096) return gv_launch<WT, J, R, 2>(a, grid, s);
+      if constexpr (WT != GV_FP4 || R <= 6)
+        if (a.K <= 8192) return gv_launch<WT, J, R, 4>(a, grid, s);
+    }
+  }
+  if constexpr (J > (WT == GV_BF16 ? 2 : WT == GV_FP8 ? 1 : 0))
+    return gv_launch<WT, J, R, GV_OWN>(a, grid, s);
+  return hipErrorInvalidValue;
 }
 
 template <int WT, int J>
 static hipError_t gv_go(const GvArgs& a, dim3 grid, int rows, hipStream_t s) {
   constexpr int RM = 8 / J > 1 ? 8 / J : 1;
   // rows in flight: the wave's, in equal turns of up to 8 KB
-  const int turns = (rows + RM - 1) / RM, r = (rows + turns - 1) / turns;
+  // (six of MXFP4 beside 8192 staged elements: registers)
+  const bool wide = WT == GV_FP4 && J == 1 && a.stage != STAGE_RAW &&
+                    a.K > 4096 && a.K <= 8192;
+  const int most = wide ? 6 : RM;
+  const int turns = (rows + most - 1) / most, r = (rows + turns - 1) / turns;
 #define GV_ROWS(RV)                                                          \
   if constexpr (RV <= RM)                                                    \
-    if (r <= RV)                                                             \
-      return a.stage == STAGE_RAW ? gv_launch<WT, J, RV, true>(a, grid, s)   \
-                                  : gv_launch<WT, J, RV, false>(a, grid, s);
+    if (r <= RV) return gv_stage<WT, J, RV>(a, grid, s);
   GV_ROWS(1)
   GV_ROWS(2)
   GV_ROWS(3)

@@ -333,6 +333,16 @@ def test_one_row(N, K, kind, glu):
         assert y[N] == 7.0
 
 
+# what all threads of a block stage: a part of a trip, one, a trip and a rest,
+# two, four, and one load more than that
+@pytest.mark.parametrize("K", [32, 2016, 2048, 2080, 4096, 4128, 6176, 8192,
+                               8224])
+@pytest.mark.parametrize("kind", ["bf16", "fp8", "fp4"])
+def test_one_row_of_every_staging(K, kind):
+    test_one_row(37, K, kind, True)
+    test_one_row(2600, K, kind, False)
+
+
 # experts of a step at once: apart through the gate, added up after it
 @pytest.mark.parametrize("n", [1, 2, 3, 8])
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
