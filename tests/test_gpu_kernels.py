@@ -311,11 +311,12 @@ def test_gemv_fused_glu_stage():
         assert_close(y, ref)
 
 
-def test_attn_dec_fused_matches_unfused():
+@pytest.mark.parametrize("pos0,S", [(11, 128), (700, 1024)])
+def test_attn_dec_fused_matches_unfused(pos0, S):
     """k_attn_dec (RoPE+cache+attn fused) vs rope_cache + attn chain."""
     from llm_np_cp_amd.ops import hip_ops as ho
 
-    nh, kvh, hd, S, pos0 = 4, 2, 64, 128, 11
+    nh, kvh, hd = 4, 2, 64
     qkv = randn_bf16((nh + 2 * kvh) * hd, seed=90)
     kc1 = torch.zeros(kvh, S, hd, dtype=torch.bfloat16, device=dev())
     vc1 = torch.zeros_like(kc1)
@@ -329,7 +330,8 @@ def test_attn_dec_fused_matches_unfused():
     sin_t = torch.from_numpy(np.sin(fr).astype(np.float32)).to(dev())
     pos = torch.tensor([pos0], dtype=torch.int32, device=dev())
 
-    # fused (exercise both the single-chunk and split-merge paths)
+    # fused: one range, and as many as the device takes of four (700 keys:
+    # three, which are merged)
     outs = []
     for split in (1, 4):
         kcx, vcx = kc1.clone(), vc1.clone()

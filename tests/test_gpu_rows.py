@@ -127,6 +127,61 @@ def test_few_rows(N, K, M, kind, norm, act):
     assert (Y[M] == 7.0).all() and not cnt.any()
 
 
+# the rows that an e4m3 product makes for itself: a prompt's by way of bf16, a
+# step's from fp32.  A unit matrix shows them: exact in an fp32 result.
+@pytest.mark.parametrize("K", [64, 512, 2304, 4096])
+@pytest.mark.parametrize("M", [2, 16])
+def test_rows_rounded_on_the_way(K, M):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    W = torch.eye(K, device="cuda").to(torch.float8_e4m3fn).view(torch.uint8)
+    X, one = normal(M, K, seed=12), torch.ones(K, device="cuda")
+    g = torch.rand(K, device="cuda") + 0.5
+    x = X.double()
+    x = (x * torch.rsqrt(x.pow(2).mean(1, keepdim=True) + 1e-5)
+         * g.double()).float()
+    got = {}
+    for norm16 in (False, True):
+        Y = torch.full((M + 1, K), 7.0, device="cuda")
+        ho.row_gemm(X, W, Y, M, ws=one, g=g, norm16=norm16)
+        want = x.bfloat16().float() if norm16 else x
+        s = want.abs().amax(1, keepdim=True) / 448
+        q = (want / s).to(torch.float8_e4m3fn).float()
+        # the norm's sums in fp32: a value on the edge takes the other one, a
+        # row's scale is off by a last bit of bf16 or fp32
+        far = (Y[:M] / s - q).abs() > q.abs() * 2.0 ** -6
+        assert far.float().mean() < 0.004
+        assert (Y[M] == 7.0).all()
+        got[norm16] = Y[:M]
+    if M * K > 8192:                    # and the two are told apart
+        d = (got[True] - got[False]).abs() > got[False].abs() * 2.0 ** -6
+        assert d.float().mean() > 0.008
+
+
+# what a step's gate hands to the rounding behind it: fp32, from bf16 halves
+@pytest.mark.parametrize("N,K", [(24, 192), (520, 8192)])
+@pytest.mark.parametrize("M", [3, 16])
+def test_gate_in_fp32(N, K, M):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    (W, ws, Wd) = e4m3(normal(2 * N, K, seed=4, scale=K ** -0.5))
+    X, sx, x = e4m3(normal(M, K, seed=5))
+    part = torch.zeros(1 << 20, device="cuda")
+    cnt = torch.zeros(256, dtype=torch.int32, device="cuda")
+    Y = torch.full((M + 1, N), 7.0, device="cuda")
+    for _ in range(2):
+        ho.row_gemm(X, W, Y, M, ws=ws, sx=sx, act=1, part=part, cnt=cnt)
+    z = (x @ Wd.T).bfloat16().double()
+    z = torch.nn.functional.gelu(z[:, :N], approximate="tanh") * z[:, N:]
+    # A half takes the other of two bf16 values where its sum, at most
+    # K 2^-24 off, crosses the middle of their distance of 2^-8: one in eight
+    # for 8192, some hundred times fewer by chance.  All others are fp32's; a
+    # result in bf16 would be off by 2^-9 nearly everywhere.
+    far = (Y[:M] - z).abs() > z.abs() * 2.0 ** -14
+    assert far.double().mean() < 1 / 16
+    assert (Y[M] == 7.0).all() and not cnt.any()
+
+
 # long rows beside room for parts of all, of fewer rows and of none; a tile of
 # sums that just does not fit (8 rows of 9536)
 @pytest.mark.parametrize("kind,M,N,K", [
@@ -215,10 +270,33 @@ def test_many_rows(M, N, K, kind, act):
 @pytest.mark.parametrize("pos", [0, 1, 33, 257, 1500])
 @pytest.mark.parametrize("kv8", [False, True])
 def test_new_tokens(hd, nh, kvh, pos, kv8):
+    check_new_tokens(hd, nh, kvh, [pos, pos // 2], kv8,
+                     ((1, 0, 0.0), (5, 0, 30.0), (80, 40, 0.0)))
+
+
+# ranges as the device chooses them (a tile of 32 keys for each wave): more
+# than the merge asks for at a time (16), as many as there may be (64 of 80),
+# behind a window, and so many that the last ones get no tile (410 tiles in 45
+# ranges of 10); the VALU's kernel alike
+@pytest.mark.parametrize("hd,nh,kvh,at,way", [
+    (64, 4, 1, [4400, 4353], (64, 0, 0.0)),
+    (64, 3, 3, [16500, 700], (80, 0, 30.0)),
+    (128, 8, 2, [13120, 13089], (45, 0, 0.0)),
+    (128, 5, 1, [16400, 3], (80, 5000, 0.0)),
+    (256, 4, 2, [2300, 8200], (64, 0, 50.0)),
+    (256, 2, 1, [3000, 2177], (20, 2176, 0.0)),
+    (512, 2, 1, [1500, 1088], (80, 0, 0.0)),
+    (512, 4, 2, [4500, 65], (80, 4000, 30.0)),
+    (16, 4, 2, [40000, 2049], (80, 0, 0.0))])
+@pytest.mark.parametrize("kv8", [False, True])
+def test_new_tokens_over_many_ranges(hd, nh, kvh, at, way, kv8):
+    check_new_tokens(hd, nh, kvh, at, kv8, (way,))
+
+
+def check_new_tokens(hd, nh, kvh, at, kv8, ways):
     from llm_np_cp_amd.ops import hip_ops as ho
 
-    B, S = 2, pos + 9
-    at = [pos, pos // 2]
+    B, S = len(at), max(at) + 9
     qkv = normal(B, (nh + 2 * kvh) * hd, seed=1)
     pools = [normal(B, kvh, S, hd, seed=2 + i) for i in range(2)]
     true, sc = [x.double() for x in pools], [None, None]
@@ -231,7 +309,7 @@ def test_new_tokens(hd, nh, kvh, pos, kv8):
         1e4 ** -(torch.arange(hd // 2, device="cuda") * 2.0 / hd).double())
     cos, sin = t.cos().float(), t.sin().float()
     ln = torch.tensor(at, dtype=torch.int32, device="cuda")
-    for split, win, cap in ((1, 0, 0.0), (5, 0, 30.0), (80, 40, 0.0)):
+    for split, win, cap in ways:
         part = torch.zeros(B * nh * split * (hd + 2), device="cuda")
         cnt = torch.zeros(B * nh, dtype=torch.int32, device="cuda")
         out = torch.full((B + 1, nh * hd), 7.0, device="cuda").bfloat16()
@@ -510,3 +588,27 @@ def test_sampled_rows(B, V):
     x = logits[:B].float()
     kept = x.gather(1, got.long()) >= x.amax(1, keepdim=True) + math.log(0.05)
     assert kept.all() and (V < 4000 or B < 5 or len(got.unique()) > 3)
+
+
+# rows that hold NaN or infinity: every choice is an expert's, others' rows are
+# theirs alone
+@pytest.mark.parametrize("E,top", [(4, 2), (8, 3), (64, 8)])
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+def test_router_of_rows_without_a_number(E, top, bad):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    M, H = 5, 192
+    h, g = normal(M, H, seed=1), torch.ones(H, device="cuda")
+    wg = normal(E, H, seed=2)
+    h[1, 7] = bad
+    idx = torch.full((M, top), -9, dtype=torch.int32, device="cuda")
+    w = torch.zeros(M, top, device="cuda")
+    ho.moe_route(h, g, wg, M, top, idx, w)
+    assert ((idx >= 0) & (idx < E)).all()
+    assert all(len(set(r)) == top for r in idx.tolist())
+    good = [0, 2, 3, 4]
+    x = h[good].double()
+    z = (x * torch.rsqrt(x.pow(2).mean(1, keepdim=True) + 1e-5)) @ wg.double().T
+    p, i = torch.softmax(z, 1).topk(top, 1)
+    assert (idx[good].long() == i).all()
+    assert off(w[good], p / p.sum(1, keepdim=True)) < 2.0 ** -16
