@@ -30,7 +30,7 @@
 //   32/8 of 128, 6040 e4m3 keys 39.2 -> 15.5; 160 keys 9.8 -> 6.4
 //   16/8 of 256, 16 sequences of 620 keys, softcap 52.3 -> 25.4 (two ranges)
 //   64/8 of 128, 4 sequences of 2000 keys 97 -> 23
-//   16/4 of 128, 32000 keys 131 -> 38 (0.85 TB/s: few blocks, long ranges)
+//   16/4 of 128, 32000 keys 131 -> 38 (1.7 TB/s: few blocks, long ranges)
 //
 // k_attn_dec_any serves the other head dims on the VALU.
 #include "common.h"

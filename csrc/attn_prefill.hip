@@ -21,8 +21,9 @@
 // 827 TFLOP/s; a wave per head and 16 queries took 1422 us.  (With both
 // buffers in one array the DMA drained ahead of every tile's reads: 314 us.)
 // 5 rows of 24/8 heads over 906 keys, split: 18 us, unsplit per-head waves
-// 74 us.  Head dim 256 at two waves a SIMD just fits the registers, an fp8
-// pool spills some 40; one wave a SIMD without spills was slower (2048 rows
+// 74 us.  Head dim 256 at two waves a SIMD just fits the registers without a
+// soft cap; with one it spills 7, beside an e4m3 pool 36 (12 to 14 where one
+// wave has all rows).  One wave a SIMD without spills was slower (2048 rows
 // behind 2048 keys: 219 us to 163 when it still spilled 20, now 118).
 #include "common.h"
 #include "attn_prefill.h"

@@ -46,6 +46,13 @@ DEVINL float wave_reduce_sum(float v) {
   return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
 
+// act 0: SiLU, 1: tanh-GELU
+DEVINL float gate_act(float x, int act) {
+  if (act == 0) return x / (1.f + __expf(-x));
+  const float c = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+  return 0.5f * x * (1.f + tanhf(c));
+}
+
 typedef float f2v __attribute__((ext_vector_type(2)));
 
 // 8 OCP-e4m3 bytes -> 8 bf16 (exact: e4m3's 3-bit mantissa fits bf16)

@@ -11,9 +11,10 @@
 //
 // Rows are XOR-swizzled by 16-byte slots; the DMA writes lane-linear, so the
 // swizzle sits in the address that a lane reads and in the fragment reads.
-// The order of k inside a slab is free as long as X and W agree: a lane's two slots are two bf16 operands or one
-// e4m3 operand of the 128-deep MFMA.  W is the first operand, so a lane
-// ends with four neighbouring outputs of one row and stores them at once.
+// The order of k inside a slab is free as long as X and W agree: a lane's two
+// slots are two bf16 operands or one e4m3 operand of the 128-deep MFMA.  W is
+// the first operand, so a lane ends with four neighbouring outputs of one row
+// and stores them at once.
 //
 // Blocks of one XCD take neighbouring tiles, rows fastest, so that its L2
 // holds the few panels of W they share.  Gate and up rows of W alternate by
@@ -46,10 +47,10 @@ struct GpArgs {
   int top, gather;
 };
 
+// gate_act with tanh by exp: an epilogue has some hundred of them a lane
 DEVINL float gp_act(float x, int act) {
   if (act == 0) return x / (1.f + __expf(-x));
   const float c = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-  // tanh by exp: exact limits at +-inf
   return x * (1.f - 1.f / (__expf(2.f * c) + 1.f));
 }
 
@@ -428,7 +429,7 @@ static const GpTile gp_tiles[] = {
 
 // us, chosen by rates of one block on an otherwise idle chip -> by these:
 //   1999x2048x8192 110 -> 72, 2048x6144x4096 132 -> 101, 2048x2304x9216 194 ->
-//   125, 907x2304x9216 92 -> 69, 300x3584x18944 189 -> 84, 60x4608x3584 35 ->
+//   125, 907x2304x9216 92 -> 83, 300x3584x18944 189 -> 84, 60x4608x3584 35 ->
 //   18, 37x2048x8192 25 -> 18
 template <bool F8>
 static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,

@@ -14,12 +14,12 @@
 // weight, and every block waited for x, its norm and the first weights in
 // turn.  us and TB/s, before -> here:
 //   bf16   2048x8192, gate before it  11.2 -> 8.8 (the gate is taken by the
-//          product before: 16384x2048 14.5 -> 14.5 with it), 3072x2048 5.7
+//          product before: 16384x2048 14.5 -> 14.4 with it), 3072x2048 5.7
 //          -> 5.5, 128256x2048 85 -> 83.5 (6.3 TB/s)
-//   e4m3   4096x14336, gate before it 17.6 -> 13.9, 28672x4096 23.7 -> 22.9,
-//          128256x4096 87 -> 86.5 (6.1 TB/s)
-//   MXFP4  3584x18944, gate before it 20.8 -> 13.8, 37888x3584 24.7 -> 20.1,
-//          152064x3584 82.7 -> 54 (5.4 TB/s)
+//   e4m3   4096x14336, gate before it 17.6 -> 13.9, 28672x4096 23.7 -> 22.2,
+//          128256x4096 87 -> 86 (6.1 TB/s)
+//   MXFP4  3584x18944, gate before it 20.8 -> 13.8, 37888x3584 24.7 -> 19.0,
+//          152064x3584 82.7 -> 53 (5.5 TB/s)
 // Of the small ones 2 us are the launch, 1 the first loads, 0.7 to 2 the work
 // on x and on the last rows; MXFP4 is bound by widening (13 us of 37888x3584
 // without its loads).
@@ -53,12 +53,6 @@ struct GvArgs {
 
 template <int WT> constexpr int gv_e() {   // weights of 16 bytes
   return WT == GV_BF16 ? 8 : WT == GV_FP8 ? 16 : 32;
-}
-
-DEVINL float gv_act(float x, int act) {
-  if (act == 0) return x / (1.f + __expf(-x));
-  const float c = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-  return 0.5f * x * (1.f + tanhf(c));
 }
 
 // the value of lane ^ W (W 7: mirrored in eight, W 8 and 12: turned in 16)
@@ -233,7 +227,7 @@ __global__ void __launch_bounds__(512) k_gemv(GvArgs a) {
         for (int i = 0; i < NV; i++)
 #pragma unroll
           for (int k = 0; k < 4; k++)
-            v[i][k] = round(gv_act(v[i][k], a.act) * bf(hr[i], k));
+            v[i][k] = round(gate_act(v[i][k], a.act) * bf(hr[i], k));
         return;
       }
       if (stage != STAGE_NORM) {           // the residual stream is bf16
@@ -442,7 +436,7 @@ __global__ void __launch_bounds__(512) k_gemv(GvArgs a) {
       if (a.glu) up += t * red[k * rs + nn + i];
     }
     v *= s1;
-    if (a.glu) v = gv_act(v, a.act) * (up * s2);
+    if (a.glu) v = gate_act(v, a.act) * (up * s2);
     if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
     v += add;
     const size_t at = (size_t)blockIdx.y * a.N + n;

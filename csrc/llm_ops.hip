@@ -46,14 +46,6 @@ DEVINL void fp4x8_to_f32p(uint32_t dw, float sc, f2v* o) {
   o[3] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(dw, sc, 3);
 }
 
-DEVINL void gemv_epilogue(float acc, int row, void* y, const u16* res,
-                          int out_f32, float softcap) {
-  if (softcap > 0.f) acc = softcap * tanhf(acc / softcap);
-  if (res) acc += b2f(res[row]);
-  if (out_f32) ((float*)y)[row] = acc;
-  else ((u16*)y)[row] = f2b(acc);
-}
-
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));  // = u4v_ alias
 
 // ====================================================================
@@ -113,14 +105,7 @@ DEVINL void gemv_stage_mx_row(char* smem, int b, const u16* xb,
       s8v uv = *(const s8v*)(x2b + i);
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        float xx = b2f(((u16*)&gv)[j]);
-        float a;
-        if (act == 0) {
-          a = xx / (1.f + __expf(-xx));
-        } else {
-          float c = 0.7978845608028654f * (xx + 0.044715f * xx * xx * xx);
-          a = 0.5f * xx * (1.f + tanhf(c));
-        }
+        const float a = gate_act(b2f(((u16*)&gv)[j]), act);
         MXSTORE(i + j, a * b2f(((u16*)&uv)[j]));
       }
     }
@@ -581,13 +566,12 @@ extern "C" hipError_t launch_rope_cache(void* q, const void* kin,
 // NOTE: with every shipped preset at head_dim in {64,128,256} the MFMA
 // prefill kernel below is taken instead; this per-query VALU kernel is
 // kept as the reachable fallback for odd head_dims and as the simple
-// DEBUGGING reference the fused kernels are compared against in tests
-// (SURVEY §2.2 K1).
+// DEBUGGING reference the fused kernels are compared against in tests.
 // grid (nh, M): block = head h, query row m (absolute pos = *len_ptr + m,
 // attends keys [start, pos+1)).  4 waves split the KV range; each lane
 // owns (sub-position, 8-dim chunk); merge within wave then across waves.
 // Sliding window + attention-logit softcap = real Gemma-2 semantics
-// (reference omitted both).
+// (the reference omitted both).
 // ====================================================================
 
 template <bool KV8>
@@ -797,15 +781,7 @@ k_glu(const u16* __restrict__ gate, const u16* __restrict__ up,
   u16 o[8];
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    float x = b2f(((u16*)&g)[j]);
-    float a;
-    if (act == 0) {
-      a = x / (1.f + __expf(-x));
-    } else {
-      float c = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-      a = 0.5f * x * (1.f + tanhf(c));
-    }
-    o[j] = f2b(a * b2f(((u16*)&u)[j]));
+    o[j] = f2b(gate_act(b2f(((u16*)&g)[j]), act) * b2f(((u16*)&u)[j]));
   }
   *(s8v*)(out + i) = *(s8v*)o;
 }
@@ -1160,8 +1136,8 @@ extern "C" hipError_t launch_quant_fp4(const void* X, void* Q, void* E,
 // ====================================================================
 // fp8 row quantization: Q[N,K] = e4m3(X / s_n), s_n = absmax_n / 448.
 // One block per row.  Used (a) at load time to quantize weights ON
-// DEVICE (drops the round-1 host-quant ~90 s for 9B and the duplicate
-// bf16 copy), (b) per prefill GEMM to quantize the
+// DEVICE (on the host a 9B model took ~90 s, and a duplicate bf16 copy
+// stayed), (b) per prefill GEMM to quantize the
 // activation rows so BOTH MFMA operands are fp8.
 // HW convert: v_cvt_pk_fp8_f32 (OCP e4m3fn on gfx950, saturating).
 // ====================================================================
@@ -1518,7 +1494,7 @@ extern "C" hipError_t launch_addinto(void* y, const void* a, long total,
 // Grid-wide barrier (device-side, graph-replay-safe).  Used by the
 // fused-layer decode path: phases of one layer run inside ONE kernel
 // with barriers instead of kernel boundaries (~4 us launch/ramp floor
-// each — profiles/decode_kernels_r01.md).
+// each).
 //
 // Protocol: `cnt` is a MONOTONIC u64 arrive counter (never reset — the
 // launch invariant is cnt % nblocks == 0, preserved because every
@@ -1599,13 +1575,13 @@ extern "C" hipError_t launch_i32_set(void* p, int v, hipStream_t stream) {
   return hipGetLastError();
 }
 // ====================================================================
-// Mixtral sparse-MoE helpers (beyond-parity: the reference has no MoE;
-// ROADMAP §5).  k_moe_route fuses the per-row RMSNorm, the router dots
+// Mixtral sparse-MoE helpers (the reference has no MoE).
+// k_moe_route fuses the per-row RMSNorm, the router dots
 // against Wg[E,H] (f32 accum — bf16 router logits would risk top-k
 // flips), the softmax over E, and the HF top-k renormalization
 // (modeling_mixtral MixtralTopKRouter), emitting compact (idx, w)
-// pairs for the expert-indexed decode GEMVs and optionally a dense
-// M x E weight grid for the prefill per-expert GEMM loop.
+// pairs for the expert-indexed products and optionally a dense M x E
+// weight grid.
 // One block per row; E <= 64, topk <= 8.  Bound by its chain of trips: the
 // row and gamma together, then all experts' weights at once (eight waves, an
 // expert each at a time), then one wave with an expert a lane.  Experts one
@@ -1708,9 +1684,9 @@ extern "C" hipError_t launch_moe_route(const void* h, const void* g,
   return hipGetLastError();
 }
 
-// y[m, :H] += w[m * wstride] * x[m, :H]  (bf16 I/O, f32 math) — the
-// prefill MoE combine: each expert's GEMM output is folded into the
-// residual stream weighted by that row's router prob (0 if unrouted).
+// y[m, :H] += w[m * wstride] * x[m, :H]  (bf16 I/O, f32 math): one expert's
+// results for all rows, weighted by a column of the dense grid (0 if
+// unrouted).
 extern "C" __global__ void __launch_bounds__(256)
 k_moe_scale_add(u16* __restrict__ y, const u16* __restrict__ xin,
                 const float* __restrict__ w, long wstride, int M, int H) {

@@ -91,12 +91,6 @@ DEVINL uint32_t swap8(uint32_t v) {        // the value of lane l^8
   return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true);
 }
 
-DEVINL float rg_act(float x, int act) {
-  if (act == 0) return x / (1.f + __expf(-x));
-  const float c = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-  return 0.5f * x * (1.f + tanhf(c));
-}
-
 #define RG_NW 8
 #define RG_NORM_K 4096     // the longest row that is normed on the way
 
@@ -320,7 +314,7 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
         up = b2f(f2b(up));
         v = b2f(f2b(v));
       }
-      v = rg_act(v, a.act) * up;
+      v = gate_act(v, a.act) * up;
     }
     if (a.softcap > 0.f) v = a.softcap * tanhf(v / a.softcap);
     v += o.add;

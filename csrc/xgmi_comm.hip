@@ -1,7 +1,7 @@
 // xgmi_comm.hip — one-shot peer-memory collectives for single-node TP
 // over xGMI (MI355X: 7 point-to-point links/GPU, ~153 GB/s each).
 //
-// Why not RCCL in the decode hot loop (SURVEY §5, VERDICT r1 items 1-2):
+// Why not RCCL in the decode hot loop:
 //  - decode TP payloads are hidden_size bf16 = 4-9 KB -> latency-bound;
 //    a ring all-reduce pays 2(world-1) link hops, ~10-20 us per call,
 //    and a TP=8 Gemma-9B step issues 84 of them.  One-shot over
