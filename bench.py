@@ -1,8 +1,8 @@
 #!/usr/bin/env python3
 """Flagship decode benchmark (driver contract).
 
-Measures the BASELINE.json metric: decode tokens/sec, batch 1, synthetic
-prompt, random-init weights, bf16.  Default model is Llama-3.2-1B at
+Measures decode tokens/sec, batch 1, synthetic prompt, random-init
+weights, bf16.  Default model is Llama-3.2-1B at
 EVERY N (TP=N) so the driver's 1/2/4/8-GPU curve compares like with
 like; the metric's second config (Gemma-2-9B TP=8, fp8) runs via
 ``--model gemma-2-9b --dtype fp8``.  A "step" is one decoded token; the
@@ -176,7 +176,7 @@ def main():
     ap.add_argument("--dtype", type=str, default="bf16",
                     choices=["bf16", "fp8", "fp4"],
                     help="weight dtype (constant across N for honest "
-                         "scaling; fp8 = BASELINE config 4)")
+                         "scaling)")
     ap.add_argument("--kv-dtype", type=str, default="bf16",
                     choices=["bf16", "fp8"],
                     help="KV-pool dtype (fp8 = e4m3 with per-head-pos "

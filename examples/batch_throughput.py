@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Throughput mode (GPU): B prompts decode in lockstep over
-per-sequence KV pools; the skinny fp8 MFMA GEMM streams each weight
-matrix ONCE per step for all rows.
+per-sequence KV pools; each weight matrix is streamed ONCE per step for
+all rows (up to 16).
 
     python examples/batch_throughput.py [preset] [batch] [tokens]
 """

@@ -195,7 +195,7 @@ class ModelConfig:
     # ------------------------------------------------------------------
     def rope_inv_freq(self):
         """Inverse frequencies, honoring llama3 rope_scaling (which the
-        reference ignored — SURVEY §2.4).  Returns a numpy fp64 array of
+        reference ignored).  Returns a numpy fp64 array of
         length head_dim//2."""
         import numpy as np
 

@@ -6,7 +6,7 @@ directory containing ``config.json`` plus either sharded safetensors with
 ``model.safetensors.index.json`` or a single ``model.safetensors``; applies
 the ``lm_head.weight -> model.embed_tokens.weight`` tying alias.
 
-Differences by design (SURVEY §5 checkpoint/resume):
+Differences by design:
 - no bare ``except:`` fallback (the reference swallowed all errors,
   ``llama3.2_model.py:1063``) — missing files raise;
 - this module reads LOCAL directories (hub repo ids are resolved one
@@ -132,7 +132,7 @@ class LazyCheckpointWeights:
 
 
 # ----------------------------------------------------------------------
-# Synthetic checkpoints (random init — no network, BASELINE.json terms)
+# Synthetic checkpoints (random init — no network)
 # ----------------------------------------------------------------------
 
 def hf_weight_shapes(cfg: ModelConfig) -> Dict[str, Tuple[int, ...]]:

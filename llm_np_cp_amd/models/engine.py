@@ -1,9 +1,10 @@
 """GPU inference engine: Llama-3.2 / Gemma-2 forward on hand-written
 CDNA4 HIP kernels, PyTorch tensors as memory containers only.
 
-MI355X-first design (SURVEY §7 stages 2-4):
-  - every compute op is a kernel from ``csrc/llm_ops.hip`` — no ATen math
-    in the forward pass, no eager fallback (ops fail loudly if the
+MI355X-first design:
+  - every compute op is a kernel of this repository (``csrc/``: products
+    of one row, of few and of many, attention of prompts and of new
+    tokens, norms, router, sampler) — no ATen math in the forward pass, no eager fallback (ops fail loudly if the
     extension is missing);
   - preallocated KV pool per layer (in-place writes, no concat);
   - decode state (seq length, sampled token, RNG counter, output ring)
@@ -16,7 +17,7 @@ MI355X-first design (SURVEY §7 stages 2-4):
 Reference parity: this replaces the CuPy model classes
 (``/root/reference/llama3.2_model.py:334-822``) — same capability
 (forward with KV cache, returns logits), built from the architectural
-spec in SURVEY §2.4 rather than translated.
+spec of the two families rather than translated.
 """
 
 from __future__ import annotations
@@ -39,7 +40,7 @@ class GPUModel(DecodeLoop):
                  seed: int = 0, force_tp_path: bool = False,
                  kv_dtype: str = "bf16", max_batch: int = 1):
         """``max_seq=None`` sizes the KV pool from FREE HBM after the
-        weights land (288 GB per MI355X — SURVEY §5 long-context), capped
+        weights land (288 GB per MI355X), capped
         at config.max_position_embeddings.  ``max_batch>1`` allocates
         per-sequence KV pools for lockstep batched decode
         (prefill_batch/decode_batch; beyond-parity serving capability)."""
@@ -53,9 +54,9 @@ class GPUModel(DecodeLoop):
         self.dtype = dtype
         if dtype not in ("bf16", "fp8", "fp4"):
             raise ValueError(f"unsupported dtype {dtype!r}")
-        # fp4 = MXFP4 weights on the single-sequence DECODE GEMVs (half
-        # the fp8 stream); prefill and batched decode run on the fp8
-        # copy (the fp8 machinery flag covers both quantized modes)
+        # fp4 = MXFP4 weights for decode steps of one sequence (half the
+        # fp8 stream) and for prompts; a group's decode steps run on an
+        # fp8 copy (the fp8 machinery flag covers both quantized modes)
         self.fp8 = dtype in ("fp8", "fp4")
         self.wq4 = dtype == "fp4"
         # fp4 + batch pools: a group's decode steps run on fp8, so keep
@@ -65,9 +66,9 @@ class GPUModel(DecodeLoop):
             raise ValueError(f"unsupported kv_dtype {kv_dtype!r}")
         self.kv_dtype = kv_dtype
         self.kv8 = kv_dtype == "fp8"  # e4m3 KV pool, per-(head,pos) scales
-        # Mixtral sparse MoE: per-token top-k routed experts (decode:
-        # expert-indexed GEMVs off device idx; prefill: dense per-expert
-        # GEMM loop weighted by router probs)
+        # Mixtral sparse MoE: per-token top-k routed experts (one row:
+        # products indexed by the device's choice; more: rows sorted by
+        # expert, each expert over its own)
         self.moe = config.is_moe
         self.topk = config.num_experts_per_tok
         if self.moe:
@@ -107,8 +108,7 @@ class GPUModel(DecodeLoop):
             slot_bytes = max(self.H * 2, self.vocab_l * 4, 1 << 16)
             tpu.init_xgmi(self.device, slot_bytes)
         # prefill-sized all-reduces: RCCL async on its own stream,
-        # overlapped with the next row-chunk's GEMM (north star: comm
-        # overlap on a second HIP stream).  Needs the nccl(=RCCL)
+        # overlapped with the next row-chunk's GEMM.  Needs the nccl(=RCCL)
         # backend; gloo (CPU CI) takes the inline path.
         import torch.distributed as dist
         self._async_ar = bool(
@@ -136,7 +136,7 @@ class GPUModel(DecodeLoop):
     # ------------------------------------------------------------------
     def _auto_max_seq(self) -> int:
         """KV pool length from free HBM (post-weights): fill the 288 GB
-        MI355X budget instead of a fixed 4k default (VERDICT r1 #10),
+        MI355X budget instead of a fixed 4k default,
         capped at the model's max_position_embeddings."""
         cfg = self.config
         free, _total = torch.cuda.mem_get_info(self.device)
@@ -181,7 +181,7 @@ class GPUModel(DecodeLoop):
             """Per-output-row e4m3fn quantization ON DEVICE (k_quant_
             fp8_rows): one bf16 upload, quantize, drop the bf16 copy —
             fp8 models hold a single weight copy in HBM and load in
-            seconds (round-1 host quant took ~90 s for 9B)."""
+            seconds (on the host 9B took ~90 s)."""
             t = bf16(a)
             N, K = t.shape
             q = torch.empty(N, K, dtype=torch.uint8, device=dev)
@@ -535,8 +535,8 @@ class GPUModel(DecodeLoop):
         """Row-parallel projection followed by all-reduce over TP ranks.
         For prefill-sized M the rows are split in two: the all-reduce of
         chunk A runs on RCCL's comm stream while chunk B's GEMM occupies
-        the compute stream (SURVEY §2.3 'overlap comm on 2nd stream' —
-        the reference has no distributed code at all)."""
+        the compute stream (the reference has no distributed code at
+        all)."""
         if not (self._async_ar and M >= 512):
             self._linear(lw, name, x, y, M=M, batch=batch)
             tpu.all_reduce(y[:M])
@@ -658,7 +658,7 @@ class GPUModel(DecodeLoop):
                 else:
                     # per-query VALU kernel: every production head_dim is
                     # 64/128/256 (MFMA above); kept as the documented
-                    # debugging/odd-shape fallback (SURVEY §2.2 K1)
+                    # debugging/odd-shape fallback
                     ho.attn(q, self._kc(i), self._vc(i),
                             self.b_att, self.len_buf, M, self.nh_l,
                             self.kvh_l, self.hd, self.scale,
@@ -770,7 +770,7 @@ class GPUModel(DecodeLoop):
     def forward_full(self, ids: np.ndarray,
                      return_hidden_states: bool = False):
         """All-positions logits (M, V) — reference-parity API (the HF
-        tuple shape, SURVEY §1 L3).  Prefill-style pass; vocab GEMM per
+        tuple shape).  Prefill-style pass; vocab GEMM per
         chunk.  Resets the cache.  With ``return_hidden_states`` also
         returns the L+1 per-layer hidden states (embedding output +
         each decoder layer, reference ``all_hidden_states``
@@ -817,7 +817,7 @@ class GPUModel(DecodeLoop):
             done += M
         ho.i32_set(self.len_buf, n)
         # mirror the device len so a following decode()'s overflow guard
-        # counts from the right base (KV-pool OOB otherwise)
+        # counts from the right base (it would run past the pool otherwise)
         self._host_len = n
         if return_hidden_states:
             return out, hidden
@@ -829,7 +829,7 @@ class GPUModel(DecodeLoop):
         be rolled back afterwards with ``rewind``).  This is the
         speculative-decoding VERIFY pass: the target model scores k
         draft tokens in one prefill-shaped pass instead of k decode
-        steps (ROADMAP §5; the reference has nothing comparable)."""
+        steps (the reference has nothing comparable)."""
         ids = np.asarray(ids, dtype=np.int32).ravel()
         n = len(ids)
         if n == 0:
@@ -931,9 +931,9 @@ class GPUModel(DecodeLoop):
 
     def _decode_step(self, greedy: bool, min_p: float,
                      temperature: float = 1.0):
-        """Fused decode path: 4 kernels/layer (llama) or 5 (gemma) —
-        RMSNorm and GLU live inside the GEMV staging pass, RoPE + KV
-        write inside the attention kernel; a side stream prefetches the
+        """Fused decode path: 5 kernels/layer — RMSNorm lives in the
+        staging of a product, GLU in the epilogue of gate and up, RoPE +
+        KV write inside the attention kernel; a side stream prefetches the
         next layer's weights through MALL, paced by per-layer events."""
         cfg = self.config
         eps = cfg.rms_norm_eps
@@ -1097,7 +1097,7 @@ class GPUModel(DecodeLoop):
     def _decode_batch_step_mx(self, B: int, greedy: bool, min_p: float,
                               temperature: float = 1.0):
         """Fused batched decode (fp8, B<=8): mirrors _decode_step's
-        4-5 kernels/layer with multi-x GEMVs over B rows."""
+        kernels with multi-x GEMVs over B rows."""
         cfg = self.config
         eps = cfg.rms_norm_eps
         H, I = self.H, self.inter_l

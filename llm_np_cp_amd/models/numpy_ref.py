@@ -2,9 +2,8 @@
 (Llama-3.2 / Gemma-2 / Qwen-2 / Mistral / Mixtral sparse-MoE).
 
 This is the in-repo oracle (the role HF ``transformers`` played for the
-reference) and BASELINE config 0 (the reference's NumPy path,
-``/root/reference/llama3.2_model_numpy.py``).  Deliberate fixes over the
-reference (SURVEY §7 stage 1):
+reference) and the counterpart of the reference's NumPy path
+(``llama3.2_model_numpy.py``).  Deliberate fixes over the reference:
 
 - numerically **stable** softmax everywhere (the reference's live NumPy
   softmax was unstabilized, ``llama3.2_model_numpy.py:915-919``);
@@ -12,7 +11,7 @@ reference (SURVEY §7 stage 1):
   ``llama3.2_model.py:471``);
 - llama3 ``rope_scaling`` honored (reference ignored it);
 - Gemma-2 sliding-window attention and attention-logit soft-capping
-  implemented (reference omitted both, SURVEY §2.4);
+  implemented (the reference omitted both);
 - decode feeds back token *ids*, not re-tokenized text (generate loop).
 
 All math is fp32 (weights are loaded/cast to fp32), accumulation in fp32.

@@ -636,7 +636,7 @@ def moe_route(h: torch.Tensor, g: torch.Tensor, wg: torch.Tensor, M: int,
     """Fused MoE router (Mixtral semantics): per row RMSNorm(h)*g ->
     E dots vs wg[E,H] (f32) -> softmax -> top-k renormalized.
     idx: (M*topk,) int32; w: (M*topk,) f32; dense: (M*E,) f32 per-expert
-    weights (0 if unrouted) for the prefill expert-GEMM loop."""
+    weights (0 if unrouted)."""
     E, H = wg.shape
     assert idx.numel() >= M * topk and w.numel() >= M * topk
     if dense is not None:

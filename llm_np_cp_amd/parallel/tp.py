@@ -3,9 +3,9 @@
 One process per GPU; ``torch.distributed`` backend "nccl" IS RCCL on
 ROCm.  World size 1 means every collective is a no-op, so the TP=1 path
 is the same code with collectives skipped (doubles as the CPU-CI "fake
-backend" — SURVEY §4 distributed test strategy).
+backend").
 
-Sharding scheme (SURVEY §7 stage 4):
+Sharding scheme:
   q/k/v projections  : head-sharded rows      (column-parallel)
   o_proj             : column-sharded         (row-parallel, all-reduce)
   gate/up            : row-sharded            (column-parallel)
@@ -118,8 +118,8 @@ def broadcast(t, src: int = 0):
 
 
 # ----------------------------------------------------------------------
-# Weight sharding (numpy, done at load time; SURVEY §5 checkpoint scope:
-# per-rank TP sharding happens on the host before the single H2D copy)
+# Weight sharding (numpy, done at load time: per-rank TP sharding happens
+# on the host before the single H2D copy)
 # ----------------------------------------------------------------------
 
 def shard_rows(w: np.ndarray, rank: int, world: int) -> np.ndarray:

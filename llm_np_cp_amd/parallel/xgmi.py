@@ -5,8 +5,7 @@ an RCCL ring pays 2(world-1) xGMI hops.  The one-shot scheme
 (``csrc/xgmi_comm.hip``: every rank pushes its vector to all peers, every
 rank reduces locally) is one hop and, crucially, a plain HIP kernel on
 the current stream — so the whole TP decode step captures into a
-hipGraph with no RCCL-in-graph dependency (resolves VERDICT r1 items
-1-2 by construction).
+hipGraph with no RCCL-in-graph dependency.
 
 Safety: ``create()`` runs a numerics self-check against
 ``torch.distributed.all_reduce`` on real hardware; any failure (IPC
@@ -15,9 +14,8 @@ so once.  The device kernel uses a bounded spin: a dead peer sets a
 sticky error flag instead of hanging the GPU, and ``check()`` raises on
 it at the next host sync point.
 
-Reference parity: the reference has no distributed code at all
-(SURVEY §2.3); this subsystem comes from BASELINE.json's north star
-("RCCL all-reduce over xGMI", TP=8 decode).
+The reference has no distributed code at all; this subsystem serves
+decode steps sharded over the GPUs of a node (TP=8).
 """
 
 from __future__ import annotations

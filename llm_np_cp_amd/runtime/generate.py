@@ -10,8 +10,7 @@ corrupts the stream for any token whose text does not round-trip.
 Works with both the NumPy oracle model and the GPU engine: a model here
 is anything with ``.forward(ids, cache, pos0) -> logits`` and
 ``.make_cache(max_seq)``.  Cache-less mode (``use_cache=False``) re-runs
-the full prefix each step — a correctness/debug mode, as in the reference
-(SURVEY §3.3).
+the full prefix each step — a correctness/debug mode, as in the reference.
 """
 
 from __future__ import annotations

@@ -1,6 +1,6 @@
 """HTTP serving layer with CONTINUOUS request batching.
 
-The reference has no server (no CLI, no server); this is the
+The reference has no server; this is the
 deployment-facing wrapper around the engine: OpenAI-style
 ``/v1/completions`` and ``/v1/chat/completions`` endpoints (both with
 ``"stream": true`` SSE token streaming) plus ``/health`` and ``/stats``.
@@ -255,7 +255,7 @@ def build_app(model_name: str = "llama-3.2-1b", backend: str = "auto",
     eos_set = (set() if eos is None else {int(eos)}
                if isinstance(eos, (int, float)) else {int(e) for e in eos})
 
-    # Prometheus metrics (SURVEY §5 observability); per-app registry so
+    # Prometheus metrics; per-app registry so
     # repeated build_app calls (tests) never collide on timeseries names
     try:
         from prometheus_client import (CollectorRegistry, Counter,

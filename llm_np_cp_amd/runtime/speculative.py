@@ -32,8 +32,8 @@ MFMA prefill GEMMs (``forward_positions``), so verifying k tokens
 streams the weights ONCE instead of k times — the same
 bandwidth argument that makes batched decode pay.
 
-The reference has no speculative decoding (SURVEY §2 — single-model
-greedy/min-p only); this is a beyond-parity capability (ROADMAP §5).
+The reference has no speculative decoding (single-model greedy/min-p
+only); this goes beyond it.
 """
 
 from __future__ import annotations

@@ -1,4 +1,4 @@
-"""Optional roctx range markers (SURVEY §5 tracing/profiling).
+"""Optional roctx range markers.
 
 When librocprofiler-sdk-roctx (or legacy libroctx64) is present, wrap
 engine phases in named ranges so `rocprofv3 --marker-trace` shows

@@ -7,9 +7,7 @@ The kernels are validated three ways without needing an 8-GPU node:
   2. two PROCESSES on one GPU exchange real hipIpc (dmabuf) handles and
      run XgmiComm.create()'s hardware self-check against gloo;
   3. a full TP=2 engine decode (two processes, one GPU) captures the
-     one-shot collectives inside a hipGraph and replays it — the
-     VERDICT r1 'graph capture x collectives' unknown, resolved on
-     hardware.
+     one-shot collectives inside a hipGraph and replays it.
 Cross-DEVICE coherence still needs a multi-GPU node (driver round-end);
 XgmiComm.create() re-runs the same self-check there at engine init.
 """

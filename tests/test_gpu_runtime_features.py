@@ -1,4 +1,4 @@
-"""Round-2 runtime-feature GPU tests (session KV reuse, LoRA,
+"""Runtime-feature GPU tests (session KV reuse, LoRA,
 stop strings on the device loop).  Kept in a file that sorts AFTER the
 core engine/kernel suites so an unexpected failure here cannot mask
 them under pytest -x."""

@@ -218,7 +218,7 @@ def test_mixtral_synthetic_checkpoint_roundtrip(tmp_path):
 
 
 def test_generate_greedy_matches_hf_generate():
-    """SURVEY §4 integration check: the full generate() loop (prefill +
+    """Integration check: the full generate() loop (prefill +
     cached feedback of sampled ids) reproduces transformers' own
     greedy `generate` token-for-token on a tiny random-init Llama."""
     import torch

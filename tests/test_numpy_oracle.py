@@ -1,6 +1,6 @@
 """NumPy reference model vs HF transformers on tiny random-init configs.
 
-This is the oracle-validation layer (SURVEY §4): the reference validated
+This is the oracle-validation layer: the reference validated
 itself interactively against ``transformers``; we make that comparison an
 automated test, then every later (HIP) component is tested against the
 NumPy model.

@@ -4,7 +4,7 @@ The GPU TP decode path uses exactly this arithmetic (engine._decode_step
 with world>1): head-sharded QKV, row-parallel o/down with all-reduce,
 vocab-sharded lm_head with all-gather.  Here the same sharding helpers
 are exercised with torch CPU tensors so CI without a GPU covers the
-distributed plumbing (SURVEY §4 distributed strategy)."""
+distributed plumbing."""
 
 import os
 

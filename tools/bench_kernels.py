@@ -3,8 +3,8 @@
 
 Times each decode-path kernel shape standalone: a hipGraph of REPS
 launches, timed with CUDA events, reported as us/launch and effective
-TB/s of weight traffic.  Used to pick GEMV variants (nt, rows-per-wave)
-— guide §5.4: within-probe comparison, same process, interleaved.
+TB/s of weight traffic (small shapes stay in the caches; --layersim
+times whole layers from memory).
 """
 
 import os
@@ -56,7 +56,7 @@ def main():
     ]
     print(f"{'shape':>9} {'N':>7} {'K':>6} | " +
           " | ".join(f"{v:>12}" for v in
-                     ["bf16", "bf16-nt", "bf16-nt-r2", "fp8-nt", "fp8-nt-r2"]))
+                     ["bf16", "bf16 norm", "fp8", "fp8 norm"]))
     for name, N, K in shapes:
         W = torch.randn(N, K, device=dev).to(torch.bfloat16) * 0.05
         s = W.float().abs().amax(dim=1).clamp_min(1e-8) / 448.0
@@ -64,13 +64,15 @@ def main():
         x = torch.randn(K, device=dev).to(torch.bfloat16)
         y = torch.empty(N, dtype=torch.bfloat16, device=dev)
         res = []
-        for kind, nt, rpw in [("bf16", 0, 1), ("bf16", 1, 1), ("bf16", 1, 2),
-                              ("fp8", 1, 1), ("fp8", 1, 2)]:
+        g = torch.rand(K, device=dev)
+        norm = dict(stage=ho.STAGE_NORM, g=g)
+        for kind, kw in (("bf16", {}), ("bf16", norm), ("fp8", {}),
+                         ("fp8", norm)):
             if kind == "bf16":
-                fn = lambda: ho.gemv(W, x, y, nt=nt, rpw=rpw)
+                fn = lambda: ho.gemv(W, x, y, **kw)
                 nbytes = N * K * 2
             else:
-                fn = lambda: ho.gemv_fp8(Wq, s, x, y, nt=nt, rpw=rpw)
+                fn = lambda: ho.gemv_fp8(Wq, s, x, y, **kw)
                 nbytes = N * K
             us = time_graph(fn)
             res.append(f"{us:6.2f}us {nbytes/us/1e6:5.2f}T")
@@ -128,8 +130,9 @@ if __name__ == "__main__" and "--layersim" not in sys.argv:
 
 def layersim():
     """In-context layer simulation: a graph over 16 DISTINCT layers'
-    GEMV weights (2.4 GB total > L3) — honest per-layer time without the
-    full engine; sweeps grid caps and nt."""
+    GEMV weights (2.4 GB total > L3), the products of a decode step as the
+    engine launches them — honest per-layer time without the full engine;
+    with all blocks and with half of them."""
     from csrc.build import ensure_built
     ensure_built()
     from llm_np_cp_amd.ops import hip_ops as ho
@@ -149,49 +152,24 @@ def layersim():
     h = torch.randn(H, device=dev).to(torch.bfloat16)
     qkv = torch.empty(H + NKV, dtype=torch.bfloat16, device=dev)
     att = torch.randn(H, device=dev).to(torch.bfloat16)
-    gu = torch.empty(2 * I, dtype=torch.bfloat16, device=dev)
+    act = torch.empty(I, dtype=torch.bfloat16, device=dev)
     g1 = torch.randn(H, device=dev)
 
-    def one_pass(nt, cap):
+    def one_pass(cap, **norm):
         for lw in layers:
-            ho.gemv(lw["wqkv"], h, qkv, stage=ho.STAGE_NORM, g=g1,
-                    nt=nt, maxblocks=cap)
-            ho.gemv(lw["wo"], att, h, res=h, nt=nt, maxblocks=cap)
-            ho.gemv(lw["wgu"], h, gu, stage=ho.STAGE_NORM, g=g1,
-                    nt=nt, maxblocks=cap)
-            ho.gemv(lw["wdown"], gu[:I], h, res=h, stage=ho.STAGE_GLU,
-                    x2=gu[I:], nt=nt, maxblocks=cap)
-
-    def raw_pass(nt, cap):
-        # same weight traffic, all stage=RAW (no staging barrier): isolates
-        # the cost of the fused-stage barrier vs pure streaming
-        for lw in layers:
-            ho.gemv(lw["wqkv"], h, qkv, nt=nt, maxblocks=cap)
-            ho.gemv(lw["wo"], att, h, res=h, nt=nt, maxblocks=cap)
-            ho.gemv(lw["wgu"], h, gu, nt=nt, maxblocks=cap)
-            ho.gemv(lw["wdown"], gu[:I], h, res=h, nt=nt, maxblocks=cap)
-
-    def fused_pass(nt, cap):
-        # single fused mega-GEMV per layer? approximate the ceiling with
-        # one N=(H+NKV+2I+H... ) not contiguous; instead: wgu+wdown merged
-        # is impossible -- emulate 2-kernel layer by doubling wgu only
-        for lw in layers:
-            ho.gemv(lw["wgu"], h, gu, stage=ho.STAGE_NORM, g=g1,
-                    nt=nt, maxblocks=cap)
-            ho.gemv(lw["wgu"], h, gu, nt=nt, maxblocks=cap)
+            ho.gemv(lw["wqkv"], h, qkv, maxblocks=cap, **norm)
+            ho.gemv(lw["wo"], att, h, res=h, maxblocks=cap)
+            ho.gemv(lw["wgu"], h, act, glu=True, maxblocks=cap, **norm)
+            ho.gemv(lw["wdown"], act, h, res=h, maxblocks=cap)
 
     print("layersim: 16 llama-1b layers of GEMVs (121.6 MB/layer bf16)")
-    for name, fn in (("staged", one_pass), ("all-raw", raw_pass)):
-        for nt in (1,):
-            for cap in (512, 1024):
-                us = time_graph(lambda: fn(nt, cap), reps=5, warmup=5)
-                print(f"  {name} nt={nt} cap={cap:5d}: {us/L:7.2f}us/layer "
-                      f"({121.6e6*L/us/1e6:4.2f} TB/s)")
-    # 2-kernel pass: 67MB x2 per layer
-    for cap in (512, 1024):
-        us = time_graph(lambda: fused_pass(1, cap), reps=5, warmup=5)
-        print(f"  two-wgu cap={cap:5d}: {us/L:7.2f}us/layer "
-              f"({134e6*L/us/1e6:4.2f} TB/s)")
+    # without the norms: what their staging costs beside the stream
+    for name, norm in (("staged", dict(stage=ho.STAGE_NORM, g=g1)),
+                       ("all-raw", {})):
+        for cap in (0, 128):
+            us = time_graph(lambda: one_pass(cap, **norm), reps=5, warmup=5)
+            print(f"  {name} cap={cap:5d}: {us/L:7.2f}us/layer "
+                  f"({121.6e6*L/us/1e6:4.2f} TB/s)")
 
 
 if __name__ == "__main__" and "--layersim" in sys.argv:

@@ -3,7 +3,7 @@
 
 With synthetic random weights the only honest pair is a QUANTIZED
 SELF-DRAFT (same weights, cheaper dtype) — independent random models
-never agree, so acceptance ~0 and speculation cannot win (BASELINE.md).
+never agree, so acceptance ~0 and speculation cannot win.
 Real speedups need a trained draft/target pair; this harness is the
 measurement tool for that day (and a correctness soak meanwhile: the
 speculative output must equal the greedy chain).
