@@ -69,6 +69,11 @@ __global__ void __launch_bounds__(256) k_last_tokens(PairEmbed a) {
 //   out = v + sum_j cw[taps-1-j] v(pos - j),    zero before position 0.
 // The last inputs v of a sequence are kept in a ring, ring[slot][pos % taps].
 // A row of up to NT*U elements stays in the registers of NT threads.
+// X says whether there may be an xadd or a gate: none; some, asked for with x;
+// some, read when they are due (rows that are longer than the registers).
+// Their registers cost where there is none (2048 rows of 4096, norm alone:
+// 11.8 us, with them 15.1).
+enum { ST_NONE, ST_AHEAD, ST_LATE };
 struct RowStage {
   const float* x;
   const float *y, *gb;      // nullable pair
@@ -83,21 +88,24 @@ struct RowStage {
   float eps;
 };
 
-template <int NT, int U, bool CONV = false, class Put>
+template <int NT, int U, int X, bool CONV = false, class Put>
 DEVINL void stage_row(const RowStage& s, size_t row, bool keep, float* red,
                       Put put) {
   const int tid = threadIdx.x, W = s.W;
   const size_t o = row * W;
   float xv[U], gv[U], yv[U], av[U], tv[U];
-  const float* gt = s.gate ? s.gate + row * s.ldg : nullptr;
+  const float* gt = X != ST_NONE && s.gate ? s.gate + row * s.ldg : nullptr;
+  const float* xadd = X != ST_NONE ? s.xadd : nullptr;
 #pragma unroll
   for (int u = 0; u < U; u++) {              // all on the way together
     const int i = tid + u * NT;
     xv[u] = i < W ? s.x[o + i] : 0.f;
-    gv[u] = s.g && i < W ? s.g[i] : 0.f;
+    if constexpr (!CONV) gv[u] = s.g && i < W ? s.g[i] : 0.f;
     if (s.y) yv[u] = i < W ? s.y[o + i] : 0.f;
-    if (s.xadd) av[u] = i < W ? s.xadd[o + i] : 0.f;
-    tv[u] = gt && i < W ? gt[i] : 0.f;
+    if constexpr (X == ST_AHEAD) {
+      if (xadd) av[u] = i < W ? xadd[o + i] : 0.f;
+      tv[u] = gt && i < W ? gt[i] : 0.f;
+    }
   }
   [[maybe_unused]] int pos = 0;
   [[maybe_unused]] float* ring = nullptr;
@@ -154,17 +162,21 @@ DEVINL void stage_row(const RowStage& s, size_t row, bool keep, float* red,
 #pragma unroll
     for (int u = 0; u < U; u++) xv[u] += yv[u] * rb * gb[u];
   }
-  if (s.xadd)
+  if (xadd)
 #pragma unroll
-    for (int u = 0; u < U; u++) xv[u] += av[u];
+    for (int u = 0; u < U; u++) {
+      const int i = tid + u * NT;
+      if constexpr (X == ST_AHEAD) xv[u] += av[u];
+      else if (i < W) xv[u] += xadd[o + i];
+    }
   auto late = [&](int i) {              // elements beyond the registers
     float v = s.x[o + i];
     if (s.y) v += s.y[o + i] * rb * s.gb[i];
-    if (s.xadd) v += s.xadd[o + i];
+    if (xadd) v += xadd[o + i];
     return v;
   };
   float rn = 0.f;
-  if (s.g) {
+  if (!CONV && s.g) {
     float ss = 0.f;
 #pragma unroll
     for (int u = 0; u < U; u++) ss += xv[u] * xv[u];
@@ -174,9 +186,9 @@ DEVINL void stage_row(const RowStage& s, size_t row, bool keep, float* red,
     }
     rn = 1.f / sqrtf(block_sum_once<NT>(ss, red + NT / 64) / (float)W + s.eps);
   }
-  auto finish = [&](int i, float v, float g, float t) {
+  auto finish = [&](int i, float v, float g, auto gate) {
     if (s.g && i < s.Kp)
-      put(i, i < W ? v * rn * g * (gt ? sigmoid_f(t) : 1.f) : 0.f);
+      put(i, i < W ? v * rn * g * (gt ? sigmoid_f(gate()) : 1.f) : 0.f);
     // xout may be x: its reads are done
     if (keep && s.xout && i < W) s.xout[o + i] = v;
   };
@@ -202,10 +214,13 @@ DEVINL void stage_row(const RowStage& s, size_t row, bool keep, float* red,
     return;
   }
 #pragma unroll
-  for (int u = 0; u < U; u++) finish(tid + u * NT, xv[u], gv[u], tv[u]);
+  for (int u = 0; u < U; u++) {
+    const int i = tid + u * NT;
+    finish(i, xv[u], gv[u], [&] { return X == ST_AHEAD ? tv[u] : gt[i]; });
+  }
   for (int i = tid + U * NT; i < max(W, s.Kp); i += NT)
     finish(i, i < W ? late(i) : 0.f, s.g && i < W ? s.g[i] : 0.f,
-           gt && i < W ? gt[i] : 0.f);
+           [&] { return gt[i]; });
 }
 
 // ---- staging a row of several residual streams ----------------------------
@@ -377,12 +392,12 @@ k_group_rows(RowStage s, int groups, T* __restrict__ out) {
 
 // one block per row; `rows` (nullable) picks the source row of each output
 // row.  out rows have Kp elements; the padding is written as zero.
-template <typename T, int U>
+template <typename T, int U, int X>
 __global__ void __launch_bounds__(256)
 k_norm_rows(RowStage s, const int* __restrict__ rows, T* __restrict__ out) {
   __shared__ float red[8];
   T* o = out + (size_t)blockIdx.x * s.Kp;
-  stage_row<256, U>(s, rows ? rows[blockIdx.x] : blockIdx.x, true, red,
+  stage_row<256, U, X>(s, rows ? rows[blockIdx.x] : blockIdx.x, true, red,
                [&](int i, float v) { o[i] = El<T>::st(v); });
 }
 
@@ -772,8 +787,10 @@ __global__ void __launch_bounds__(LIN_NT) k_lin_row(LinRowArgs a) {
   const size_t row = a.rows ? a.rows[0] : 0;
   const bool first = blockIdx.x == 0;
   if constexpr (MODE == ROW_NORM || MODE == ROW_CONV) {
-    stage_row<LIN_NT, U, MODE == ROW_CONV>(a.s, row, first, red,
-                                           [&](int i, float f) {
+    // a convolution has none (4096 wide: 19.7 us, with the registers 22.7,
+    // which leave no room for a second block on a CU)
+    stage_row<LIN_NT, U, MODE == ROW_NORM ? ST_AHEAD : ST_NONE,
+              MODE == ROW_CONV>(a.s, row, first, red, [&](int i, float f) {
       T v = El<T>::st(f);
       xs[i] = v;
       if (a.hout && first) ((T*)a.hout)[i] = v;
@@ -1157,12 +1174,21 @@ static bool bad_stage(const RowStage& s) {
 template <typename T>
 static void norm_rows(const RowStage& s, const void* rows, void* out, int M,
                       hipStream_t st) {
-  if (s.W <= 2048)
-    hipLaunchKernelGGL((k_norm_rows<T, 8>), dim3(M), dim3(256), 0, st, s,
-                       (const int*)rows, (T*)out);
-  else
-    hipLaunchKernelGGL((k_norm_rows<T, 16>), dim3(M), dim3(256), 0, st, s,
-                       (const int*)rows, (T*)out);
+#define NORM_ROWS(U, X)                                                      \
+  hipLaunchKernelGGL((k_norm_rows<T, U, X>), dim3(M), dim3(256), 0, st, s,   \
+                     (const int*)rows, (T*)out)
+  const bool some = s.gate || s.xadd;
+  if (s.W <= 2048) {
+    if (some) NORM_ROWS(8, ST_AHEAD);
+    else NORM_ROWS(8, ST_NONE);
+  } else if (!some) {
+    NORM_ROWS(16, ST_NONE);
+  } else if (s.W <= 4096) {
+    NORM_ROWS(16, ST_AHEAD);
+  } else {
+    NORM_ROWS(16, ST_LATE);
+  }
+#undef NORM_ROWS
 }
 
 extern "C" hipError_t launch_norm_rows(int f32, const RowStage* s,
