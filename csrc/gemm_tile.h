@@ -16,7 +16,12 @@
 // a loop unrolled over them let the compiler see that a DMA into one does not
 // touch what is read from another; it would wait for all of it before the
 // reads otherwise.  1664x2048 outputs of K 2048 and 8192, 128x64 tiles: 70 us
-// on average, now 51 (128x128 has room for two buffers only: as before).
+// on average, now 51.
+// Without DEEP two buffers, drained at each barrier, and the schedule is the
+// compiler's: for 128x128, which has no room for a third, for fp32, which is
+// bound by its products (2048x6144x1024: 202 us, in flight 273), and where
+// more than two blocks would share a CU, which they do with two buffers only
+// (513x8192x2048 in 640 blocks of 128x64: 30.7 us, in flight 33.5).
 // LDS rows are XOR-swizzled (slot ^= row & 7); the DMA writes lane-linear, so
 // the swizzle sits in the per-lane source address and in the fragment reads.
 //
@@ -58,14 +63,15 @@ template <int N> DEVINL void gemm_meet() {
   asm volatile("" ::: "memory");
 }
 
-template <int BM, int BN, typename T, class ARow, class BRow>
+template <int BM, int BN, typename T, bool DEEP = true, class ARow, class BRow>
 DEVINL void gemm_mainloop(f4v (&acc)[BM / 32][BN / 32], ARow arow, BRow brow,
                           int k_lo, int nt) {
   constexpr int FM = BM / 32, FN = BN / 32;
   constexpr int BK = GemmMma<T>::BK;
   constexpr int VE = 16 / sizeof(T);   // elements of a 16-byte slot
-  constexpr int NS = 73728 / ((BM + BN) * 128) > 4 ? 4
-                     : 73728 / ((BM + BN) * 128);       // buffers
+  constexpr int ROOM = 73728 / ((BM + BN) * 128);       // buffers
+  constexpr bool DRAIN = !DEEP || ROOM < 3;
+  constexpr int NS = DRAIN ? 2 : ROOM > 4 ? 4 : ROOM;
   constexpr int PS = FM + FN;                // DMA of a wave and slab
 #define GEMM_BUF(i)                                                          \
   __shared__ __attribute__((aligned(16))) char A##i[NS > i ? BM * 128 : 16], \
@@ -116,6 +122,36 @@ DEVINL void gemm_mainloop(f4v (&acc)[BM / 32][BN / 32], ARow arow, BRow brow,
   };
 
   const int fr = lane & 15, fk = lane >> 4;
+  if (nt < 1) return;
+  if constexpr (DRAIN) {
+    stage(A0, B0, 0);
+    __syncthreads();
+    for (int t = 0; t < nt; t++) {
+      const char *As = t & 1 ? A1 : A0, *Bs = t & 1 ? B1 : B0;
+      if (t + 1 < nt) stage(t & 1 ? A0 : A1, t & 1 ? B0 : B1, t + 1);
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        f4v a[FM], b[FN];
+#pragma unroll
+        for (int i = 0; i < FM; i++) {
+          const int ra = wrow * (BM / 2) + i * 16 + fr;
+          a[i] = *(const f4v*)(As + ra * 128 + ((h * 4 + fk) ^ (ra & 7)) * 16);
+        }
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+          const int rb = wcol * (BN / 2) + j * 16 + fr;
+          b[j] = *(const f4v*)(Bs + rb * 128 + ((h * 4 + fk) ^ (rb & 7)) * 16);
+        }
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+          for (int j = 0; j < FN; j++)
+            acc[i][j] = GemmMma<T>::mma(a[i], b[j], acc[i][j]);
+      }
+      __syncthreads();               // the DMA is over, the reads are done
+    }
+    return;
+  }
   // Half a slab of fragments ahead: the hand-over stands between two halves'
   // products, when the second half is in registers already.
   f4v a[2][FM], b[2][FN];
@@ -155,7 +191,6 @@ DEVINL void gemm_mainloop(f4v (&acc)[BM / 32][BN / 32], ARow arow, BRow brow,
     }
     mma(1);
   };
-  if (nt < 1) return;
 #pragma unroll
   for (int u = 0; u < NS; u++)
     if (u < nt) stage(A[u], B[u], u);

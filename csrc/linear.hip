@@ -960,14 +960,14 @@ template <class Body> DEVINL void with_epilogue(int epi, Body body) {
   }
 }
 
-template <typename T, int BM, int BN>
+template <typename T, int BM, int BN, bool DEEP>
 __global__ void __launch_bounds__(256) k_gemm(GemmArgs a) {
   const int bm = blockIdx.y * BM, bn = blockIdx.x * BN, z = blockIdx.z;
   const T* X = (const T*)a.X + (size_t)z * a.xz;
   const T* W = (const T*)a.W + (size_t)z * a.wz;
   const int K = z ? a.K2 : a.K, ldw = z ? a.K2 : a.ldw;
   f4v acc[BM / 32][BN / 32];
-  gemm_mainloop<BM, BN, T>(
+  gemm_mainloop<BM, BN, T, DEEP>(
       acc,
       [&](int r) { return X + (size_t)min(bm + r, a.M - 1) * a.ldx; },
       [&](int r) { return W + (size_t)min(bn + r, a.N - 1) * ldw; }, 0,
@@ -1380,19 +1380,28 @@ static void gemm_go(const GemmArgs& a, int Z, hipStream_t s) {
     hipLaunchKernelGGL((k_gemm_skinny<T, 2, 8>), sk, dim3(512), 0, s, a);
   } else if (a.M <= 64) {
     hipLaunchKernelGGL((k_gemm_skinny<T, 4, 8>), sk, dim3(512), 0, s, a);
-  } else if (b128 < 192) {
-    hipLaunchKernelGGL((k_gemm<T, 64, 64>),
-                       dim3((a.N + 63) / 64, (a.M + 63) / 64, Z), dim3(256), 0,
-                       s, a);
-  } else if (b128 < 300 || b128 < 0.7 * 512 * ((b128 + 511) / 512)) {
-    // two 128x128 tiles fit a CU; a part-filled last wave of them is worse
-    hipLaunchKernelGGL((k_gemm<T, 128, 64>),
-                       dim3((a.N + 63) / 64, (a.M + 127) / 128, Z), dim3(256),
-                       0, s, a);
   } else {
-    hipLaunchKernelGGL((k_gemm<T, 128, 128>),
-                       dim3((a.N + 127) / 128, (a.M + 127) / 128, Z),
-                       dim3(256), 0, s, a);
+    // DMA in flight while two blocks a CU hold the whole grid; fp32 only in
+    // small tiles with a CU each (2048x2048, 300 rows: 46 us, in flight 42)
+    auto tiles = [&](int bm, int bn) {
+      return dim3((a.N + bn - 1) / bn, (a.M + bm - 1) / bm, Z);
+    };
+    auto few = [&](dim3 g, long most) { return (long)g.x * g.y * Z <= most; };
+#define GEMM_GO(BM, BN, DEEP)                                                \
+  hipLaunchKernelGGL((k_gemm<T, BM, BN, DEEP>), tiles(BM, BN), dim3(256), 0, \
+                     s, a)
+    constexpr bool F32 = sizeof(T) == 4;
+    if (b128 < 192) {
+      if (few(tiles(64, 64), F32 ? 256 : 512)) GEMM_GO(64, 64, true);
+      else GEMM_GO(64, 64, false);
+    } else if (b128 < 300 || b128 < 0.7 * 512 * ((b128 + 511) / 512)) {
+      // two 128x128 tiles fit a CU; a part-filled last wave of them is worse
+      if (!F32 && few(tiles(128, 64), 512)) GEMM_GO(128, 64, !F32);
+      else GEMM_GO(128, 64, false);
+    } else {
+      GEMM_GO(128, 128, false);
+    }
+#undef GEMM_GO
   }
 }
 

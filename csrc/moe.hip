@@ -131,7 +131,7 @@ __global__ void __launch_bounds__(1024) k_moe_sort(const int* __restrict__ idx,
 }
 
 // gate/up of gathered rows; act rows are in expert order
-template <typename T, int BM, int BN>
+template <typename T, int BM, int BN, bool DEEP>
 __global__ void __launch_bounds__(256) k_moe_gu(MoeArgs m, MoeSort s) {
   const int t = blockIdx.y, nr = s.tile_n[t];
   if (nr == 0) return;
@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(256) k_moe_gu(MoeArgs m, MoeSort s) {
   const float lim = e == m.E ? m.lims : m.lim;
   const T* W = moe_gu_base<T>(m, e);
   f4v acc[BM / 32][BN / 32];
-  gemm_mainloop<BM, BN, T>(
+  gemm_mainloop<BM, BN, T, DEEP>(
       acc,
       [&](int r) {
         return (const T*)m.h +
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(256) k_moe_gu(MoeArgs m, MoeSort s) {
 }
 
 // down projection back to pair order, as T
-template <typename T, int BM, int BN>
+template <typename T, int BM, int BN, bool DEEP>
 __global__ void __launch_bounds__(256) k_moe_down(MoeArgs m, MoeSort s,
                                                   T* __restrict__ y) {
   const int t = blockIdx.y, nr = s.tile_n[t];
@@ -183,7 +183,7 @@ __global__ void __launch_bounds__(256) k_moe_down(MoeArgs m, MoeSort s,
   const int ff = e == m.E ? m.ffs : m.ff;
   const T* W = moe_down_base<T>(m, e);
   f4v acc[BM / 32][BN / 32];
-  gemm_mainloop<BM, BN, T>(
+  gemm_mainloop<BM, BN, T, DEEP>(
       acc,
       [&](int r) {
         return (const T*)m.act + (size_t)(p0 + min(r, nr - 1)) * m.ldact;
@@ -273,13 +273,29 @@ template <typename T, int BM>
 static void moe_go(const MoeArgs& m, const MoeSort& s, void* y,
                    hipStream_t st) {
   constexpr int BN = BM == 128 ? 128 : 64;
-  int ffm = m.ff > m.ffs ? m.ff : m.ffs;
-  hipLaunchKernelGGL((k_moe_gu<T, BM, BN>),
-                     dim3((2 * ffm + BN - 1) / BN, s.maxtiles), dim3(256), 0,
-                     st, m, s);
-  hipLaunchKernelGGL((k_moe_down<T, BM, BN>),
-                     dim3((m.W + BN - 1) / BN, s.maxtiles), dim3(256), 0, st,
-                     m, s, (T*)y);
+  const int ffm = m.ff > m.ffs ? m.ff : m.ffs;
+  const dim3 gu((2 * ffm + BN - 1) / BN, s.maxtiles);
+  const dim3 down((m.W + BN - 1) / BN, s.maxtiles);
+  // The main loop keeps DMA in flight in tiles of 32 rows (8 experts of
+  // 1024 x 2048, 64 tokens: 37 us drained at each barrier, 30 in flight) and
+  // in those of 64 while two blocks a CU hold the grid (256 tokens: 43 us,
+  // 35); of more, two buffers let more share a CU (16 experts of 2048 x 1024,
+  // 700 tokens: 63 us, in flight 71).  Of 128 rows it has no room to.
+  auto in_flight = [](dim3 g) {
+    return BM == 32 || (BM == 64 && (long)g.x * g.y <= 512);
+  };
+  if (in_flight(gu))
+    hipLaunchKernelGGL((k_moe_gu<T, BM, BN, BM <= 64>), gu, dim3(256), 0, st,
+                       m, s);
+  else
+    hipLaunchKernelGGL((k_moe_gu<T, BM, BN, BM == 32>), gu, dim3(256), 0, st,
+                       m, s);
+  if (in_flight(down))
+    hipLaunchKernelGGL((k_moe_down<T, BM, BN, BM <= 64>), down, dim3(256), 0,
+                       st, m, s, (T*)y);
+  else
+    hipLaunchKernelGGL((k_moe_down<T, BM, BN, BM == 32>), down, dim3(256), 0,
+                       st, m, s, (T*)y);
 }
 
 template <typename T>

@@ -1,4 +1,6 @@
-"""Staged rows of the layer-list kernels, within and beyond the registers."""
+"""Products and staged rows of the layer-list kernels at the sizes where their
+launches change: tiles and buffers of the row products, rows within and beyond
+the registers, experts by rows a tile."""
 
 import pytest
 import torch
@@ -19,6 +21,31 @@ def hy():
 def draw(seed, *shape, dtype=torch.float32):
     g = torch.Generator().manual_seed(seed)
     return torch.randn(*shape, generator=g).to(dtype).cuda()
+
+
+# A sum of K products in fp32 is off by at most K roundings of the sum of
+# their magnitudes (2^-24 each, twice that where a unit truncates).
+def product(X, W):
+    x, w = X.double(), W.double()
+    return x @ w.T, x.abs() @ w.abs().T * (X.shape[1] * 2.0 ** -23)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("M,N", [
+    (65, 70), (100, 2050),        # 64x64, few tiles
+    (1100, 1990), (1100, 2500),   # 64x64, more than two a CU
+    (1100, 2800),                 # 128x64
+    (1100, 4090),                 # 128x64, more than two a CU
+    (1100, 5100),                 # 128x128
+])
+@pytest.mark.parametrize("K", [64, 192, 576])
+def test_tiles_of_row_products(hy, dtype, M, N, K):
+    X, W = draw(M, M, K, dtype=DT[dtype]), draw(N, N, K, dtype=DT[dtype])
+    Y = torch.full((M + 1, N), 7.0, device="cuda")
+    hy.gemm_rows(X, W, Y, M, K, N, hy.EPI_F32)
+    want, far = product(X, W)
+    assert ((Y[:M].double() - want).abs() <= far).all()
+    assert (Y[M] == 7.0).all()
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
@@ -55,3 +82,54 @@ def test_staged_rows(hy, dtype, W, form):
     assert (out[:M, W:] == 0).all() and (out[M] == 7.0).all()
     if "xout" in kw:
         assert ((xout.double() - v).abs() <= far * size).all()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("T,bm", [
+    (5, 32), (90, 32), (150, 64),
+    (700, 64),                    # more blocks than two a CU
+    (700, 128)])
+def test_experts_by_rows_a_tile(hy, dtype, T, bm):
+    E, top, W, ff = 4, 2, 1088, 1024
+    dt = DT[dtype]
+    gu = draw(0, E, 2 * ff, W, dtype=dt) * W ** -0.5
+    down = draw(1, E, W, ff, dtype=dt) * ff ** -0.5
+    h = draw(2, T, W, dtype=dt)
+    gen = torch.Generator().manual_seed(T)
+    idx = torch.stack([torch.randperm(E, generator=gen)[:top]
+                       for _ in range(T)]).int().cuda()
+    wt = torch.rand(T, top, generator=gen).cuda()
+    pairs, tiles = T * top, T * top // bm + E
+    i32 = dict(device="cuda", dtype=torch.int32)
+    perm = torch.zeros(pairs, **i32)
+    at = [torch.zeros(tiles, **i32) for _ in range(3)]
+    act = torch.zeros(pairs, ff, device="cuda", dtype=dt)
+    y = torch.zeros(pairs, W, device="cuda", dtype=dt)
+    x = torch.full((T, W), 7.0, device="cuda")
+    m = hy.MoeArgs().put(h=h, gu=gu, down=down, idx=idx, wt=wt, act=act,
+                         ldh=W, ldact=ff, W=W, E=E, K1=top, ff=ff, ffs=0,
+                         glu=1, win=0, lim=0.0, lims=0.0)
+    s = hy.MoeSort().put(perm=perm, tile_e=at[0], tile_row0=at[1],
+                         tile_n=at[2], pairs=pairs, groups=E, bm=bm,
+                         maxtiles=tiles)
+    hy.moe_rows(int(dt == torch.float32), m, s, y, x, T, 1.0, True)
+    want = torch.zeros(T, W, device="cuda", dtype=torch.float64)
+    far = torch.zeros_like(want)
+    r = ROUND[dtype]
+    for e in range(E):
+        # 16 gate rows, then their 16 up rows
+        rows = gu[e].view(ff // 16, 2, 16, W)
+        g, dg = product(h, rows[:, 0].reshape(ff, W))
+        u, du = product(h, rows[:, 1].reshape(ff, W))
+        a = torch.nn.functional.silu(g) * u
+        # the slope of silu stays below 1.1; its own rounding is in 2^-20
+        da = (1.1 * dg * (u.abs() + du) + (g.abs() + dg) * du
+              + (r + 2.0 ** -20) * a.abs())
+        d = down[e].double()
+        o = a @ d.T
+        do = da @ d.abs().T + a.abs() @ d.abs().T * (ff * 2.0 ** -23)
+        do = do + r * (o.abs() + do)
+        by = ((idx == e) * wt).sum(1, keepdim=True).double()
+        want += by * o
+        far += by * (do + 2.0 ** -21 * o.abs())
+    assert ((x.double() - want).abs() <= far).all()
