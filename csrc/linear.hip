@@ -1044,6 +1044,7 @@ __global__ void __launch_bounds__(64 * NW) k_gemm_skinny(GemmArgs a) {
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
+      if (s + u * NW >= nsl) break;          // alike in a wave
       f4v c[2];                              // row lr, chunks 2gq and 2gq + 1
 #pragma unroll
       for (int d = 0; d < 4; d++) {

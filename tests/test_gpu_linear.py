@@ -1,6 +1,7 @@
 """Products and staged rows of the layer-list kernels at the sizes where their
-launches change: tiles and buffers of the row products, rows within and beyond
-the registers, experts by rows a tile."""
+launches change: tiles and buffers of the row products, few rows with fewer
+slabs than waves, rows within and beyond the registers, experts by rows a
+tile."""
 
 import pytest
 import torch
@@ -40,6 +41,18 @@ def product(X, W):
 ])
 @pytest.mark.parametrize("K", [64, 192, 576])
 def test_tiles_of_row_products(hy, dtype, M, N, K):
+    X, W = draw(M, M, K, dtype=DT[dtype]), draw(N, N, K, dtype=DT[dtype])
+    Y = torch.full((M + 1, N), 7.0, device="cuda")
+    hy.gemm_rows(X, W, Y, M, K, N, hy.EPI_F32)
+    want, far = product(X, W)
+    assert ((Y[:M].double() - want).abs() <= far).all()
+    assert (Y[M] == 7.0).all()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("M", [2, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,K", [(72, 64), (528, 512), (2056, 1088)])
+def test_few_rows_of_few_slabs(hy, dtype, M, N, K):
     X, W = draw(M, M, K, dtype=DT[dtype]), draw(N, N, K, dtype=DT[dtype])
     Y = torch.full((M + 1, N), 7.0, device="cuda")
     hy.gemm_rows(X, W, Y, M, K, N, hy.EPI_F32)
