@@ -136,21 +136,30 @@ def test_rows_rounded_on_the_way(K, M):
 
     W = torch.eye(K, device="cuda").to(torch.float8_e4m3fn).view(torch.uint8)
     X, one = normal(M, K, seed=12), torch.ones(K, device="cuda")
-    g = torch.rand(K, device="cuda") + 0.5
+    g = normal(1, K, seed=13)[0].float().abs() + 0.5
     x = X.double()
     x = (x * torch.rsqrt(x.pow(2).mean(1, keepdim=True) + 1e-5)
-         * g.double()).float()
+         * g.double()).abs()
     got = {}
     for norm16 in (False, True):
         Y = torch.full((M + 1, K), 7.0, device="cuda")
         ho.row_gemm(X, W, Y, M, ws=one, g=g, norm16=norm16)
-        want = x.bfloat16().float() if norm16 else x
-        s = want.abs().amax(1, keepdim=True) / 448
-        q = (want / s).to(torch.float8_e4m3fn).float()
-        # the norm's sums in fp32: a value on the edge takes the other one, a
-        # row's scale is off by a last bit of bf16 or fp32
-        far = (Y[:M] / s - q).abs() > q.abs() * 2.0 ** -6
-        assert far.float().mean() < 0.004
+        # The norm's sums and products in fp32, the scale and the division by
+        # it are off by less than 2^-18 (33 roundings of a sum of squares,
+        # halved by the root, and a dozen more): a value on an edge of bf16
+        # or e4m3 may take either side, no other may.
+        lo, hi = (x * (1 - 2.0 ** -18)).float(), (x * (1 + 2.0 ** -18)).float()
+        if norm16:
+            lo, hi = lo.bfloat16().float(), hi.bfloat16().float()
+        slo, shi = (v.amax(1, keepdim=True) / 448 for v in (lo, hi))
+        most = torch.full_like(hi, 448.0)       # of e4m3
+        lo = (lo / shi * (1 - 2.0 ** -18)).to(torch.float8_e4m3fn).float()
+        hi = torch.minimum(hi / slo * (1 + 2.0 ** -18), most)
+        hi = hi.to(torch.float8_e4m3fn).float()
+        y = Y[:M].abs()
+        assert (y >= lo * slo * (1 - 2.0 ** -18)).all()
+        assert (y <= hi * shi * (1 + 2.0 ** -18)).all()
+        assert ((Y[:M] >= 0) == (X >= 0))[y > 0].all()
         assert (Y[M] == 7.0).all()
         got[norm16] = Y[:M]
     if M * K > 8192:                    # and the two are told apart
