@@ -418,11 +418,94 @@ extern "C" hipError_t launch_rmsnorm(const void* x, const void* g,
 
 // ====================================================================
 // RoPE + KV-pool write.
-// q inout [M, nh*hd]; k_in/v_in [M, kvh*hd]; caches [kvh, S, hd].
+// q inout [M, nh*hd]; k_in/v_in [M, kvh*hd]; caches [kvh, S, hd] bf16, or
+// e4m3 with one fp32 scale per (kv_head, position): absmax/448 over the
+// head_dim values, the same scheme as the fp8 weights.
 // Position of row m is *pos_ptr + m (device scalar: graph-replay-safe).
 // cos/sin tables fp32 [max_seq, hd/2].
+//
+// Bound by memory where rows are many and by the trips of one thread where
+// they are few, so a thread has 16 values of one head, eight of either half,
+// and the hd/16 threads of a head meet for its e4m3 scale in registers.
+// us, by a block a row that took its heads in turn, two bytes at a time
+// (e4m3: a meeting of the block for every one) -> here:
+//   bf16  5 rows of 24/8 heads of 128 4.3 -> 2.9, 1999 of 32/8 of 64 8.4 ->
+//         6.2, 2048 of 32/8 of 128 13 -> 9.3 (37 of 32/8 of 64: 3.9 both)
+//   e4m3  120 rows of 8/4 heads of 256 8.8 -> 3.3, 2048 of 32/8 of 128
+//         27.4 -> 10.0
 // ====================================================================
 
+template <bool KV8>
+__global__ void __launch_bounds__(256)
+k_rope_rows(u16* __restrict__ q, const u16* __restrict__ kin,
+            const u16* __restrict__ vin, void* __restrict__ kc,
+            void* __restrict__ vc, float* __restrict__ kS,
+            float* __restrict__ vS, const float* __restrict__ cost,
+            const float* __restrict__ sint, const int* __restrict__ pos_ptr,
+            int M, int nh, int kvh, int hd, int S, int ldq, int ldkv) {
+  const int G = hd / 16, per = (nh + 2 * kvh) * G, hd2 = hd / 2;
+  const int at = blockIdx.x * 256 + threadIdx.x;
+  const bool there = at < M * per;
+  const int id = there ? at : M * per - 1;
+  const int m = id / per, u = id - m * per, h = u / G, t = u - h * G;
+  const int pos = *pos_ptr + m;
+  const u16* src = h < nh ? q + (size_t)m * ldq + h * hd
+                   : h < nh + kvh ? kin + (size_t)m * ldkv + (h - nh) * hd
+                   : vin + (size_t)m * ldkv + (h - nh - kvh) * hd;
+  const s8v lo = *(const s8v*)(src + t * 8);
+  const s8v hi = *(const s8v*)(src + hd2 + t * 8);
+  float a[8], b[8];
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    a[j] = b2f(((const u16*)&lo)[j]);
+    b[j] = b2f(((const u16*)&hi)[j]);
+  }
+  if (h < nh + kvh) {
+    const float* cp = cost + (size_t)pos * hd2 + t * 8;
+    const float* sp = sint + (size_t)pos * hd2 + t * 8;
+    const f4v c[2] = {*(const f4v*)cp, *(const f4v*)(cp + 4)};
+    const f4v s[2] = {*(const f4v*)sp, *(const f4v*)(sp + 4)};
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const float x1 = a[j], x2 = b[j], cj = c[j / 4][j % 4];
+      const float sj = s[j / 4][j % 4];
+      a[j] = x1 * cj - x2 * sj;
+      b[j] = x2 * cj + x1 * sj;
+    }
+  }
+  const int kh = h < nh + kvh ? h - nh : h - nh - kvh;   // of a key or value
+  const size_t row = (size_t)(h < nh ? 0 : kh) * S + pos;
+  if constexpr (KV8) {
+    // all lanes of the wave, also those that rotate queries
+    float am = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      am = fmaxf(am, fmaxf(fabsf(a[j]), fabsf(b[j])));
+    for (int w = 1; w < G; w <<= 1) am = fmaxf(am, __shfl_xor(am, w));
+    if (!there) return;
+    if (h >= nh) {
+      const float sc = fmaxf(am, 1e-8f) / 448.0f;
+      uint8_t* dst = (uint8_t*)(h < nh + kvh ? kc : vc) + row * hd + t * 8;
+      if (t == 0) (h < nh + kvh ? kS : vS)[row] = sc;
+      *(unsigned long long*)dst = f32x8_to_fp8(a, 1.0f / sc);
+      *(unsigned long long*)(dst + hd2) = f32x8_to_fp8(b, 1.0f / sc);
+      return;
+    }
+  }
+  if (!there) return;
+  u16* dst = h < nh ? q + (size_t)m * ldq + h * hd
+                    : (u16*)(h < nh + kvh ? kc : vc) + row * hd;
+  u16 o[8], p[8];
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    o[j] = f2b(a[j]);
+    p[j] = f2b(b[j]);
+  }
+  *(s8v*)(dst + t * 8) = *(s8v*)o;
+  *(s8v*)(dst + hd2 + t * 8) = *(s8v*)p;
+}
+
+// Any head size and alignment.
 extern "C" __global__ void __launch_bounds__(256)
 k_rope_cache(u16* __restrict__ q, const u16* __restrict__ kin,
              const u16* __restrict__ vin, u16* __restrict__ kc,
@@ -463,10 +546,6 @@ k_rope_cache(u16* __restrict__ q, const u16* __restrict__ kin,
   }
 }
 
-// fp8 (e4m3) KV-pool variant: K/V stored as bytes with one fp32 scale
-// per (kv_head, position) — absmax/448 over the head_dim values, the
-// same scheme as the fp8 weights.  Halves the attention read stream
-// (the long-context decode bound) at exact-representable dequant.
 extern "C" __global__ void __launch_bounds__(256)
 k_rope_cache_fp8(u16* __restrict__ q, const u16* __restrict__ kin,
                  const u16* __restrict__ vin, uint8_t* __restrict__ kc,
@@ -546,6 +625,24 @@ extern "C" hipError_t launch_rope_cache(void* q, const void* kin,
                                         const void* pos_ptr, int M, int nh,
                                         int kvh, int hd, int S, int ldq,
                                         int ldkv, hipStream_t stream) {
+  // 16 bytes at a time; e4m3: a head's threads are a power of two
+  const size_t low = (size_t)q | (size_t)kin | (size_t)vin | (size_t)kc |
+                     (size_t)vc | (size_t)cost | (size_t)sint;
+  const int G = hd / 16;
+  if (hd >= 16 && hd % 16 == 0 && ldq % 8 == 0 && ldkv % 8 == 0 &&
+      low % 16 == 0 && (!kv8 || (G <= 64 && (G & (G - 1)) == 0)) &&
+      (long)M * (nh + 2 * kvh) * G < 1L << 30) {
+    const dim3 grid((M * (nh + 2 * kvh) * G + 255) / 256);
+#define ROPE_GO(KV8)                                                         \
+  hipLaunchKernelGGL(k_rope_rows<KV8>, grid, dim3(256), 0, stream, (u16*)q,  \
+                     (const u16*)kin, (const u16*)vin, kc, vc, (float*)kS,   \
+                     (float*)vS, (const float*)cost, (const float*)sint,     \
+                     (const int*)pos_ptr, M, nh, kvh, hd, S, ldq, ldkv)
+    if (kv8) ROPE_GO(true);
+    else ROPE_GO(false);
+#undef ROPE_GO
+    return hipGetLastError();
+  }
   if (kv8) {
     hipLaunchKernelGGL(k_rope_cache_fp8, dim3(M), dim3(256), 0, stream,
                        (u16*)q, (const u16*)kin, (const u16*)vin,

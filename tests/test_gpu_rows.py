@@ -621,3 +621,48 @@ def test_router_of_rows_without_a_number(E, top, bad):
     p, i = torch.softmax(z, 1).topk(top, 1)
     assert (idx[good].long() == i).all()
     assert off(w[good], p / p.sum(1, keepdim=True)) < 2.0 ** -16
+
+
+# a thread has 16 values of a head (of 24: one at a time); rows that end
+# inside a block; a head's threads that are no power of two
+@pytest.mark.parametrize("hd,nh,kvh", [(16, 4, 2), (24, 2, 1), (48, 3, 1),
+                                       (64, 5, 1), (128, 6, 2), (256, 2, 2)])
+@pytest.mark.parametrize("M,pos0", [(1, 0), (5, 901), (37, 3)])
+@pytest.mark.parametrize("kv8", [False, True])
+def test_rotated_rows(hd, nh, kvh, M, pos0, kv8):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    S = pos0 + M + 1
+    rows = normal(M, (nh + 2 * kvh) * hd + 8, seed=1)[:, 8:]
+    x = rows.double()
+    a = torch.rand(S, hd // 2, device="cuda", dtype=torch.float64) * 6
+    cos, sin = torch.cos(a).float(), torch.sin(a).float()
+    kind = torch.uint8 if kv8 else torch.bfloat16
+    kc, vc = (torch.zeros(kvh, S, hd, device="cuda", dtype=kind)
+              for _ in "kv")
+    kS, vS = (torch.zeros(kvh, S, device="cuda") if kv8 else None
+              for _ in "kv")
+    q, k, v = rows.split([nh * hd, kvh * hd, kvh * hd], dim=1)
+    ho.rope_cache(q, k, v, kc, vc, cos, sin,
+                  torch.tensor([pos0], dtype=torch.int32, device="cuda"),
+                  M, nh, kvh, hd, kS=kS, vS=vS)
+    x = x.view(M, -1, hd)
+    c, s = (t[pos0:pos0 + M, None].double() for t in (cos, sin))
+    u, w = x[:, :nh + kvh].chunk(2, -1)
+    turned = torch.cat([u * c - w * s, w * c + u * s], -1)
+    # rounding off by half a last place: of 8 bits 2^-8 at most, e4m3's 4
+    # bits 2^-4
+    assert off(q.reshape(M, nh, hd), turned[:, :nh]) < 2 ** -8
+    for got, sc, ref in ((kc, kS, turned[:, nh:]), (vc, vS, x[:, nh + kvh:])):
+        new = got[:, pos0:pos0 + M].permute(1, 0, 2)
+        if kv8:
+            want = ref.abs().amax(-1) / 448
+            scale = sc[:, pos0:pos0 + M].T.double()
+            assert ((scale - want).abs() <= 1e-6 * want).all()
+            new = new.contiguous().view(torch.float8_e4m3fn).double() * \
+                scale[..., None]
+            assert off(new, ref) < 2 ** -4
+        else:
+            assert off(new, ref) < 2 ** -8
+        before = got[:, :pos0].float() if not kv8 else got[:, :pos0]
+        assert not before.any() and not got[:, pos0 + M:].any()
