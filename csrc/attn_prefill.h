@@ -8,6 +8,10 @@ struct ApArgs {
   const void* vc;
   u16* out;              // [M, nh * head_dim]
   const int* len_ptr;    // position of row 0
+  // Rows of several sequences, kc .. vS the pools of all: of each block's
+  // tile its number in the sequence, the sequence's first row, rows,
+  // position of the first and pool.
+  const int* tiles;
   const float* kS;       // [kvh, S]
   const float* vS;
   float* part;           // split keys: [split, kvh, rows, head_dim + 4]

@@ -25,6 +25,10 @@
 // soft cap; with one it spills 7, beside an e4m3 pool 36 (12 to 14 where one
 // wave has all rows).  One wave a SIMD without spills was slower (2048 rows
 // behind 2048 keys: 219 us to 163 when it still spilled 20, now 118).
+//
+// Rows of several sequences (a group's prompts in one batch) bring a table:
+// which rows, position and pool a block's tile belongs to, the ones with the
+// most keys first.  A scalar load a block; nothing else differs.
 #include "common.h"
 #include "attn_prefill.h"
 
@@ -82,8 +86,18 @@ k_attn_rows(ApArgs a) {
   int qt = nq - 1 - (int)blockIdx.y;
   if (a.fold && (int)blockIdx.y >= nq / 2) qt = (int)blockIdx.y - nq / 2;
 
-  const int pos0 = *a.len_ptr;
-  const int nrows = a.M * grp;
+  int base = 0, M = a.M, pool = 0, pos0;
+  if (a.tiles) {
+    const int* t = a.tiles + blockIdx.y * 5;
+    qt = t[0];
+    base = t[1];
+    M = t[2];
+    pos0 = t[3];
+    pool = t[4];
+  } else {
+    pos0 = *a.len_ptr;
+  }
+  const int nrows = M * grp;
   const int row0 = (qt * NW + wave) * 32;
   const int row = row0 + col;
   const int rowc = min(row, nrows - 1);
@@ -111,16 +125,17 @@ k_attn_rows(ApArgs a) {
   // Q: B operand, column = row of the tile, 8 dims at 16*c + 8*hh
   ap_b8 qf[HD / 16];
   {
-    const u16* qp = a.q + (size_t)my_m * a.ldq +
+    const u16* qp = a.q + (size_t)(base + my_m) * a.ldq +
                     (size_t)(kvhead * grp + my_g) * HD + hh * 8;
 #pragma unroll
     for (int c = 0; c < HD / 16; c++) qf[c] = *(const ap_b8*)(qp + c * 16);
   }
 
-  const char* Kg = (const char*)a.kc + (size_t)kvhead * a.S * HD * (KV8 ? 1 : 2);
-  const char* Vg = (const char*)a.vc + (size_t)kvhead * a.S * HD * (KV8 ? 1 : 2);
-  const float* kS = KV8 ? a.kS + (size_t)kvhead * a.S : nullptr;
-  const float* vS = KV8 ? a.vS + (size_t)kvhead * a.S : nullptr;
+  const size_t head = ((size_t)pool * a.kvh + kvhead) * a.S;   // first key's
+  const char* Kg = (const char*)a.kc + head * HD * (KV8 ? 1 : 2);
+  const char* Vg = (const char*)a.vc + head * HD * (KV8 ? 1 : 2);
+  const float* kS = KV8 ? a.kS + head : nullptr;
+  const float* vS = KV8 ? a.vS + head : nullptr;
 
   // bf16 pool: straight into LDS.  A wave's instruction fills 1 KB, lane by
   // lane; the swizzle sits in the address that the lane reads.
@@ -355,7 +370,8 @@ k_attn_rows(ApArgs a) {
   if (row >= nrows) return;
   if (gridDim.z == 1) {
     const float inv = 1.f / l;
-    u16* op = a.out + ((size_t)my_m * a.nh + kvhead * grp + my_g) * HD;
+    u16* op = a.out +
+              ((size_t)(base + my_m) * a.nh + kvhead * grp + my_g) * HD;
 #pragma unroll
     for (int d = 0; d < HD / 32; d++)
 #pragma unroll
@@ -368,8 +384,8 @@ k_attn_rows(ApArgs a) {
       }
   } else {
     // unnormalised part of this key range: HD values, maximum, sum
-    float* pp = a.part + (((size_t)blockIdx.z * a.kvh + kvhead) * nrows +
-                          row) * (HD + 4);
+    float* pp = a.part + (((size_t)blockIdx.z * a.kvh + kvhead) * a.M * grp +
+                          base * grp + row) * (HD + 4);
 #pragma unroll
     for (int d = 0; d < HD / 32; d++)
 #pragma unroll
@@ -420,30 +436,30 @@ static void ap_go(const ApArgs& a, dim3 grid, hipStream_t s) {
                        dim3(64 * NW), 0, s, a);
 }
 
+// most: rows of the longest sequence; ntiles: of several sequences
 template <int HD, int BKV>
 static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
-                         hipStream_t s) {
+                         int most, int ntiles, hipStream_t s) {
   const int rows = a.M * (a.nh / a.kvh);
   // up to 32 rows are one wave's; more share their tiles among four
-  const int nw = rows <= 32 ? 1 : 4;
-  const int tiles = (rows + nw * 32 - 1) / (nw * 32);
+  const int nw = most * (a.nh / a.kvh) <= 32 ? 1 : 4;
+  const int tiles = a.tiles ? ntiles : (rows + nw * 32 - 1) / (nw * 32);
   // Too few blocks for 256 CUs of two each: the keys are split too, down
   // to four tiles a block.
   int split = 1;
   const int want = nw == 1 ? 1024 : 512;
   if (tiles * a.kvh * 2 <= want && a.part) {
     split = want / (tiles * a.kvh);
-    const int span = a.window > 0 ? (keys < a.window + a.M ? keys
-                                                           : a.window + a.M)
-                                  : keys;
-    const int most = span / (4 * BKV);
-    if (split > most) split = most;
+    const int span = a.window > 0 && a.window + most < keys ? a.window + most
+                                                            : keys;
+    const int worth = span / (4 * BKV);
+    if (split > worth) split = worth;
     if (split > 64) split = 64;
     const long each = (long)a.kvh * rows * (HD + 4);
     if (split > part_floats / each) split = (int)(part_floats / each);
     if (split < 1) split = 1;
   }
-  a.fold = split == 1 && tiles % 2 == 0 && tiles * a.kvh <= 512;
+  a.fold = !a.tiles && split == 1 && tiles % 2 == 0 && tiles * a.kvh <= 512;
   dim3 grid(a.kvh, tiles, split);
   if (nw == 1) {
     if (kv8) ap_go<HD, BKV, 1, true>(a, grid, s);
@@ -459,20 +475,29 @@ static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
 }
 
 // keys: number of keys that the last row sees, as far as the host knows
-// (a hint for the split; the kernel goes by *len_ptr)
+// (a hint for the split; the kernel goes by *len_ptr).  tiles: M rows of
+// several sequences, the longest of `most` rows; a tile has 32 rows times
+// heads of a kv head where that is all of the longest, else 128.
 extern "C" hipError_t launch_attn_prefill_mfma(
     const void* q, const void* kc, const void* vc, void* out,
-    const void* len_ptr, const void* kS, const void* vS, void* part,
+    const void* len_ptr, const void* tiles, const void* kS, const void* vS,
+    void* part,
     long part_floats, int kv8, int M, int nh, int kvh, int hd, int ldq,
-    int S, int keys, float scale, float softcap, int window,
-    hipStream_t stream) {
-  if (M < 1 || kvh < 1 || nh % kvh || ldq < nh * hd || ldq % 8)
+    int S, int keys, int most, int ntiles, float scale, float softcap,
+    int window, hipStream_t stream) {
+  if (M < 1 || kvh < 1 || nh % kvh || ldq < nh * hd || ldq % 8 ||
+      (tiles && (ntiles < 1 || most < 1)))
     return hipErrorInvalidValue;
+  if (!tiles) most = M;
   ApArgs a = {(const u16*)q, kc, vc, (u16*)out, (const int*)len_ptr,
+              (const int*)tiles,
               (const float*)kS, (const float*)vS, (float*)part, M, nh, kvh,
               ldq, S, 0, scale, softcap, window};
-  if (hd == 64) return ap_run<64, 64>(a, kv8, keys, part_floats, stream);
-  if (hd == 128) return ap_run<128, 64>(a, kv8, keys, part_floats, stream);
-  if (hd == 256) return ap_run<256, 32>(a, kv8, keys, part_floats, stream);
+  if (hd == 64)
+    return ap_run<64, 64>(a, kv8, keys, part_floats, most, ntiles, stream);
+  if (hd == 128)
+    return ap_run<128, 64>(a, kv8, keys, part_floats, most, ntiles, stream);
+  if (hd == 256)
+    return ap_run<256, 32>(a, kv8, keys, part_floats, most, ntiles, stream);
   return hipErrorInvalidValue;
 }

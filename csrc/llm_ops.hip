@@ -421,7 +421,8 @@ extern "C" hipError_t launch_rmsnorm(const void* x, const void* g,
 // q inout [M, nh*hd]; k_in/v_in [M, kvh*hd]; caches [kvh, S, hd] bf16, or
 // e4m3 with one fp32 scale per (kv_head, position): absmax/448 over the
 // head_dim values, the same scheme as the fp8 weights.
-// Position of row m is *pos_ptr + m (device scalar: graph-replay-safe).
+// Position of row m is *pos_ptr + m (device scalar: graph-replay-safe), or
+// rows[m] in cache rows[M + m] of several.
 // cos/sin tables fp32 [max_seq, hd/2].
 //
 // Bound by memory where rows are many and by the trips of one thread where
@@ -442,13 +443,15 @@ k_rope_rows(u16* __restrict__ q, const u16* __restrict__ kin,
             void* __restrict__ vc, float* __restrict__ kS,
             float* __restrict__ vS, const float* __restrict__ cost,
             const float* __restrict__ sint, const int* __restrict__ pos_ptr,
-            int M, int nh, int kvh, int hd, int S, int ldq, int ldkv) {
+            const int* __restrict__ rows, int M, int nh, int kvh, int hd,
+            int S, int ldq, int ldkv) {
   const int G = hd / 16, per = (nh + 2 * kvh) * G, hd2 = hd / 2;
   const int at = blockIdx.x * 256 + threadIdx.x;
   const bool there = at < M * per;
   const int id = there ? at : M * per - 1;
   const int m = id / per, u = id - m * per, h = u / G, t = u - h * G;
-  const int pos = *pos_ptr + m;
+  const int pos = rows ? rows[m] : *pos_ptr + m;
+  const size_t pool = rows ? (size_t)rows[M + m] * kvh * S : 0;
   const u16* src = h < nh ? q + (size_t)m * ldq + h * hd
                    : h < nh + kvh ? kin + (size_t)m * ldkv + (h - nh) * hd
                    : vin + (size_t)m * ldkv + (h - nh - kvh) * hd;
@@ -474,7 +477,7 @@ k_rope_rows(u16* __restrict__ q, const u16* __restrict__ kin,
     }
   }
   const int kh = h < nh + kvh ? h - nh : h - nh - kvh;   // of a key or value
-  const size_t row = (size_t)(h < nh ? 0 : kh) * S + pos;
+  const size_t row = pool + (size_t)(h < nh ? 0 : kh) * S + pos;
   if constexpr (KV8) {
     // all lanes of the wave, also those that rotate queries
     float am = 0.f;
@@ -622,7 +625,8 @@ extern "C" hipError_t launch_rope_cache(void* q, const void* kin,
                                         const void* vin, void* kc, void* vc,
                                         void* kS, void* vS, int kv8,
                                         const void* cost, const void* sint,
-                                        const void* pos_ptr, int M, int nh,
+                                        const void* pos_ptr, const void* rows,
+                                        int M, int nh,
                                         int kvh, int hd, int S, int ldq,
                                         int ldkv, hipStream_t stream) {
   // 16 bytes at a time; e4m3: a head's threads are a power of two
@@ -637,12 +641,14 @@ extern "C" hipError_t launch_rope_cache(void* q, const void* kin,
   hipLaunchKernelGGL(k_rope_rows<KV8>, grid, dim3(256), 0, stream, (u16*)q,  \
                      (const u16*)kin, (const u16*)vin, kc, vc, (float*)kS,   \
                      (float*)vS, (const float*)cost, (const float*)sint,     \
-                     (const int*)pos_ptr, M, nh, kvh, hd, S, ldq, ldkv)
+                     (const int*)pos_ptr, (const int*)rows, M, nh, kvh, hd,  \
+                     S, ldq, ldkv)
     if (kv8) ROPE_GO(true);
     else ROPE_GO(false);
 #undef ROPE_GO
     return hipGetLastError();
   }
+  if (rows) return hipErrorInvalidValue;
   if (kv8) {
     hipLaunchKernelGGL(k_rope_cache_fp8, dim3(M), dim3(256), 0, stream,
                        (u16*)q, (const u16*)kin, (const u16*)vin,

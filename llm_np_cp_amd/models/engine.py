@@ -318,7 +318,8 @@ class GPUModel(DecodeLoop):
         self.cos_t = torch.from_numpy(np.cos(freqs).astype(np.float32)).to(dev)
         self.sin_t = torch.from_numpy(np.sin(freqs).astype(np.float32)).to(dev)
 
-        PC = self.PC = min(prefill_chunk, max(256, self.max_seq))
+        # a group's prompts are read together
+        PC = self.PC = min(prefill_chunk, max(256, self.max_seq * B))
         R = max(PC, self.max_batch)    # rows of a prompt's or a group's pass
         H, I = self.H, self.inter_l
         self.b_h = torch.zeros(R, H, **bf)
@@ -409,6 +410,11 @@ class GPUModel(DecodeLoop):
 
         if self.max_batch > 1:
             B, nhh = self.max_batch, self.nh_l * hd
+            # a chunk of several prompts: tokens, positions and pools of its
+            # rows, the attention's tiles, the prompts' last rows
+            pairs = PC * (self.nh_l // self.kvh_l)
+            self.pack_buf = torch.zeros(
+                3 * PC + 5 * (-(-pairs // 128) + B) + B, **i32)
             i64 = dict(dtype=torch.int64, device=dev)
             self.bt_qkv = self.b_rqkv[:B]
             self.bt_logits = torch.zeros(B, self.vocab_l, **bf)
@@ -590,9 +596,10 @@ class GPUModel(DecodeLoop):
         return min(self.attn_split, max(1, 256 // (M * self.kvh_l)))
 
     def _layers_forward(self, M: int, layer_hook=None,
-                        batch_attn: bool = False, keys: int = 0):
+                        batch_attn: bool = False, keys: int = 0, pack=None):
         """Layer stack over rows [0, M), the last of which sees ``keys``
-        keys.  ``batch_attn``: rows are M
+        keys.  ``pack``: rows of several prompts, (rows, tiles, longest) of
+        `_read_pack`.  ``batch_attn``: rows are M
         INDEPENDENT sequences at the same position (lockstep batched
         decode) — the fused decode-attention kernel runs per row over
         per-sequence KV pools instead of the prefill attention."""
@@ -642,6 +649,18 @@ class GPUModel(DecodeLoop):
                             softcap=self.attn_softcap, window=window or 0,
                             split=self._ranges(M), kS=self.k_scale[i],
                             vS=self.v_scale[i], batch=M)
+            elif pack is not None:
+                rows, tiles, most = pack
+                kv = dict(kS=self.k_scale[i], vS=self.v_scale[i])
+                ho.rope_cache(q, k, v, self.k_cache[i], self.v_cache[i],
+                              self.cos_t, self.sin_t, self.len_buf, M,
+                              self.nh_l, self.kvh_l, self.hd, rows=rows, **kv)
+                ho.attn_prefill_mfma(
+                    q, self.k_cache[i], self.v_cache[i], self.b_att,
+                    self.len_buf, M, self.nh_l, self.kvh_l, self.hd,
+                    self.scale, softcap=self.attn_softcap, window=window or 0,
+                    part=self.b_gemm_acc, keys=keys, tiles=tiles, most=most,
+                    **kv)
             else:
                 ho.rope_cache(q, k, v, self._kc(i),
                               self._vc(i), self.cos_t, self.sin_t,
@@ -751,9 +770,9 @@ class GPUModel(DecodeLoop):
             ho.softcap(out[:M], self.final_softcap)
 
     def _lm_head_last(self, M: int):
-        """Final norm + lm_head on the last row -> self.b_logits (f32, V);
+        """Final norm + lm_head on row M - 1 -> self.b_logits (f32, V);
         the norm rides in the GEMV staging pass (no separate launch)."""
-        hrow = self.b_h[M - 1] if M > 1 else self.b_h[0]
+        hrow = self.b_h[M - 1]
         kw = dict(stage=ho.STAGE_NORM, g=self.g_final,
                   eps=self.config.rms_norm_eps, softcap=self.final_softcap)
         if self.wq4:
@@ -1189,25 +1208,85 @@ class GPUModel(DecodeLoop):
                              f"{self.max_seq} pool")
         self.reset()
         self.bt_nout.zero_()
-        for b in range(B):
+        for segs in self._chunks(lens):
+            if len(segs) > 1:
+                self._read_pack(segs, seqs)
+                continue
+            (b, done, M), = segs
             self._pb = b
-            P = lens[b]
-            done = 0
-            while done < P:
-                M = min(P - done, self.PC)
-                self.ids_buf[:M].copy_(
-                    torch.from_numpy(seqs[b][done:done + M]))
-                ho.i32_set(self.len_buf, done)
-                ho.embed(self.embed, self.ids_buf, self.b_h, M,
-                         self.config.embed_scale)
-                self._layers_forward(M, keys=done + M)
-                done += M
-            self._lm_head_last(M)
-            self.bt_logits32[b].copy_(self.b_logits)
+            self.ids_buf[:M].copy_(torch.from_numpy(seqs[b][done:done + M]))
+            ho.i32_set(self.len_buf, done)
+            ho.embed(self.embed, self.ids_buf, self.b_h, M,
+                     self.config.embed_scale)
+            self._layers_forward(M, keys=done + M)
+            if done + M == lens[b]:
+                self._lm_head_last(M)
+                self.bt_logits32[b].copy_(self.b_logits)
         self._pb = 0
         self.bt_lens[:B].copy_(torch.tensor(lens, dtype=torch.int32))
         self._host_lens = lens
         self._batch_n = B
+
+    def _chunks(self, lens):
+        """The prompts in chunks of up to PC rows, each a list of (sequence,
+        first position, rows).  Several prompts share a chunk, so that its
+        products have the rows of all: read one by one, 16 prompts of 305 to
+        611 rows beside e4m3 weights left tiles half empty and W was streamed
+        16 times (with 31 steps behind them 17.5 -> 13.4 ms; six of 167 to
+        333 in bf16 with 23 steps 10.1 -> 8.4).  The ones whose last chunk is
+        a single row beside e4m3 weights go alone, for that row is not
+        rounded to e4m3, and those beside MXFP4, whose few rows are gated in
+        fp32."""
+        apart = self.wq4 or self.hd not in (64, 128, 256)
+        chunks, room = [], 0
+        for b, n in enumerate(lens):
+            alone = apart or (self.fp8 and n % self.PC == 1)
+            done = 0
+            while done < n:
+                if alone or room == 0:
+                    chunks.append([])
+                    room = self.PC
+                M = min(n - done, room)
+                chunks[-1].append((b, done, M))
+                done += M
+                room = 0 if alone else room - M
+        return chunks
+
+    def _read_pack(self, segs, seqs) -> None:
+        """One chunk of several prompts through the layers, and the logits of
+        those that it ends."""
+        M = sum(n for _, _, n in segs)
+        ends, row = [], 0
+        for b, done, n in segs:
+            row += n
+            if done + n == len(seqs[b]):
+                ends.append((b, row - 1))
+        tiles = ho.attn_tiles(segs, self.nh_l // self.kvh_l)
+        parts = [np.concatenate([seqs[b][p:p + n] for b, p, n in segs]),
+                 np.concatenate([np.arange(p, p + n) for _, p, n in segs]),
+                 np.repeat([b for b, _, _ in segs], [n for _, _, n in segs]),
+                 tiles.ravel(), np.array([r for _, r in ends])]
+        host = np.concatenate(parts).astype(np.int32)
+        buf = self.pack_buf[:len(host)]
+        buf.copy_(torch.from_numpy(host))
+        ids, rows, tiles, last = buf.split(
+            [M, 2 * M, tiles.size, len(ends)])
+        ho.embed(self.embed, ids, self.b_h, M, self.config.embed_scale)
+        self._layers_forward(
+            M, keys=max(p + n for _, p, n in segs),
+            pack=(rows, tiles.view(-1, 5), max(n for _, _, n in segs)))
+        if self.fp8 or self.tp_branch or len(ends) == 1:
+            for b, r in ends:
+                self._lm_head_last(r + 1)
+                self.bt_logits32[b].copy_(self.b_logits)
+            return
+        # bf16: a row is the same among others, W is read once for 16
+        for i in range(0, len(ends), ho.FEW_ROWS):
+            n = min(len(ends) - i, ho.FEW_ROWS)
+            b = ends[i][0]
+            ho.embed(self.b_h, last[i:], self.b_t1, n)
+            self._rows(self._head, "", self.b_t1, self.bt_logits32[b:b + n],
+                       n, g=self.g_final, softcap=self.final_softcap)
 
     # ---- continuous batching primitives (rows join/leave the group) ----
     def prefill_row(self, b: int, ids, greedy: bool = True,

@@ -17,6 +17,7 @@ from __future__ import annotations
 import ctypes
 import os
 
+import numpy as np
 import torch
 
 _LIB = None
@@ -31,13 +32,13 @@ _SIGS = {
     "launch_rmsnorm": [ctypes.c_void_p] * 8 + [ctypes.c_int] * 2 +
                       [ctypes.c_float, ctypes.c_void_p],
     "launch_rope_cache": [ctypes.c_void_p] * 7 + [ctypes.c_int] +
-                         [ctypes.c_void_p] * 3 + [ctypes.c_int] * 7 +
+                         [ctypes.c_void_p] * 4 + [ctypes.c_int] * 7 +
                          [ctypes.c_void_p],
     "launch_attn": [ctypes.c_void_p] * 7 + [ctypes.c_int] * 7 +
                    [ctypes.c_float, ctypes.c_float, ctypes.c_int,
                     ctypes.c_void_p],
-    "launch_attn_prefill_mfma": [ctypes.c_void_p] * 8 + [ctypes.c_long] +
-                                [ctypes.c_int] * 8 +
+    "launch_attn_prefill_mfma": [ctypes.c_void_p] * 9 + [ctypes.c_long] +
+                                [ctypes.c_int] * 10 +
                                 [ctypes.c_float, ctypes.c_float,
                                  ctypes.c_int, ctypes.c_void_p],
     "launch_attn_dec": [ctypes.c_void_p] * 9 + [ctypes.c_int] +
@@ -230,17 +231,20 @@ def rope_cache(q: torch.Tensor, k_in: torch.Tensor, v_in: torch.Tensor,
                cos_t: torch.Tensor, sin_t: torch.Tensor,
                pos_ptr: torch.Tensor, M: int, nh: int, kvh: int, hd: int,
                kS: torch.Tensor | None = None,
-               vS: torch.Tensor | None = None):
+               vS: torch.Tensor | None = None,
+               rows: torch.Tensor | None = None):
     """kS/vS given => fp8 (e4m3) KV pool with per-(head,pos) scales.
     q, k_in, v_in: M rows, which may lie in one fused buffer (k_in and v_in
-    equally far apart)."""
-    S = k_cache.shape[1]
+    equally far apart).  rows (int32 [2, M]): the position of each row and
+    which pool of several it belongs to (caches [pools, kvh, S, hd])."""
+    S = k_cache.shape[-2]
+    assert rows is None or (rows.numel() == 2 * M and k_cache.dim() == 4)
     assert _ld(v_in, kvh * hd) == _ld(k_in, kvh * hd)
     _check(lib().launch_rope_cache(
         _ptr(q), _ptr(k_in), _ptr(v_in), _ptr(k_cache), _ptr(v_cache),
         _ptr(kS), _ptr(vS), 1 if kS is not None else 0,
-        _ptr(cos_t), _ptr(sin_t), _ptr(pos_ptr), M, nh, kvh, hd, S,
-        _ld(q, nh * hd), _ld(k_in, kvh * hd), _stream()), "rope_cache")
+        _ptr(cos_t), _ptr(sin_t), _ptr(pos_ptr), _ptr(rows), M, nh, kvh, hd,
+        S, _ld(q, nh * hd), _ld(k_in, kvh * hd), _stream()), "rope_cache")
 
 
 def attn(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -262,20 +266,41 @@ def attn_prefill_mfma(q: torch.Tensor, k_cache: torch.Tensor,
                       hd: int, scale: float, softcap: float = 0.0,
                       window: int = 0, kS: torch.Tensor | None = None,
                       vS: torch.Tensor | None = None,
-                      part: torch.Tensor | None = None, keys: int = 0):
+                      part: torch.Tensor | None = None, keys: int = 0,
+                      tiles: torch.Tensor | None = None, most: int = 0):
     """Flash prefill attention (MFMA, online softmax); q already roped,
     caches already written for [0, pos0+M).  With part (fp32 scratch) few
     rows split their keys over more blocks; keys (pos0+M, as far as the
-    host knows) sizes that split."""
-    S = k_cache.shape[1]
+    host knows) sizes that split.  tiles (``attn_tiles``): rows of several
+    sequences, the longest of ``most`` rows, caches [pools, kvh, S, hd]."""
+    S = k_cache.shape[-2]
+    assert tiles is None or (tiles.shape[-1] == 5 and tiles.is_contiguous()
+                             and k_cache.dim() == 4)
     _check(lib().launch_attn_prefill_mfma(
         _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(len_ptr),
-        _ptr(kS), _ptr(vS), _ptr(part),
+        _ptr(tiles), _ptr(kS), _ptr(vS), _ptr(part),
         ctypes.c_long(0 if part is None else part.numel()),
         1 if kS is not None else 0,
-        M, nh, kvh, hd, _ld(q, nh * hd), S, max(keys, M),
-        ctypes.c_float(scale),
+        M, nh, kvh, hd, _ld(q, nh * hd), S, max(keys, M if not most else 1),
+        most, 0 if tiles is None else tiles.shape[0], ctypes.c_float(scale),
         ctypes.c_float(softcap), window, _stream()), "attn_prefill_mfma")
+
+
+def attn_tiles(segs, group: int) -> np.ndarray:
+    """The tiles of attn_prefill_mfma for segs [(pool, position, rows)],
+    which follow each other in the batch, ``group`` query heads to a kv head:
+    those that see the most keys first."""
+    per = 32 if max(n for _, _, n in segs) * group <= 32 else 128
+    out, row0 = [], 0
+    for pool, pos, n in segs:
+        t = np.arange(-(-n * group // per))
+        last = pos + np.minimum(n, -(-(t + 1) * per // group))   # keys seen
+        out.append(np.stack([t, np.full_like(t, row0), np.full_like(t, n),
+                             np.full_like(t, pos), np.full_like(t, pool),
+                             last]))
+        row0 += n
+    t = np.concatenate(out, axis=1)
+    return t[:5, np.argsort(-t[5], kind="stable")].T.astype(np.int32)
 
 
 def attn_dec(qkv: torch.Tensor, k_cache: torch.Tensor,

@@ -107,3 +107,22 @@ def test_chunks_shorter_than_the_group(dtype):
         assert m.b_att.shape[0] >= 20 and m.PC == chunk
     assert (h[0] - h[1]).norm() < 0.05 * h[1].norm()
     assert (ids[0] == ids[1]).mean() > 0.9          # ties of close logits
+
+
+# several prompts in a chunk, one over two chunks, single tokens: the same
+# logits as each prompt by itself
+@pytest.mark.parametrize("dtype", ["bf16", "fp8", "fp4"])
+def test_prompts_read_together(dtype):
+    rng = np.random.default_rng(0)
+    prompts = [rng.integers(0, 256, size=n) for n in (5, 40, 1, 33, 65, 2)]
+    m = engine(hidden=128, max_batch=6, dtype=dtype, prefill_chunk=64,
+               max_seq=80)
+    m.prefill_batch(prompts)
+    got = m.bt_logits32[:6].clone()
+    for b, p in enumerate(prompts):
+        m.prefill_row(b, p)
+        want = m.b_logits
+        # products in another order, rounded to 8 bits a layer (e4m3 rows: 4)
+        bound = 2.0 ** -4 if dtype == "fp8" else 2.0 ** -6
+        assert (got[b] - want).norm() < bound * want.norm(), b
+    assert m.bt_lens.tolist() == [len(p) for p in prompts]

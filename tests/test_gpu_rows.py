@@ -666,3 +666,62 @@ def test_rotated_rows(hd, nh, kvh, M, pos0, kv8):
             assert off(new, ref) < 2 ** -8
         before = got[:, :pos0].float() if not kv8 else got[:, :pos0]
         assert not before.any() and not got[:, pos0 + M:].any()
+
+
+# prompts of one batch: one wave a tile and four, a sequence that goes on
+# behind earlier keys, windows, keys split over blocks, pools out of order
+@pytest.mark.parametrize("hd,nh,kvh", [(64, 8, 2), (128, 3, 1), (256, 2, 2)])
+@pytest.mark.parametrize("segs,window,cap", [
+    ([(0, 0, 1), (2, 0, 4)], 0, 0.0),
+    ([(1, 700, 3), (0, 0, 2), (2, 31, 8)], 40, 50.0),
+    ([(2, 0, 33), (0, 130, 1), (1, 0, 129)], 0, 0.0),
+    ([(0, 2000, 9), (1, 0, 43), (2, 3, 300)], 64, 0.0)])
+@pytest.mark.parametrize("kv8", [False, True])
+def test_prompts_of_one_batch(hd, nh, kvh, segs, window, cap, kv8):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    M, S = sum(n for _, _, n in segs), max(p + n for _, p, n in segs) + 3
+    pool = torch.cat([torch.full((n,), b) for b, _, n in segs])
+    pos = torch.cat([torch.arange(p, p + n) for _, p, n in segs])
+    rows = torch.stack([pos, pool]).int().cuda()
+    kc, vc = (normal(3, kvh, S, hd, seed=s) for s in (2, 3))
+    kS = vS = None
+    if kv8:
+        (kc, kS, _), (vc, vS, _) = e4m3(kc), e4m3(vc)
+    a = torch.rand(S, hd // 2, device="cuda", dtype=torch.float64) * 6
+    cos, sin = torch.cos(a).float(), torch.sin(a).float()
+    part = torch.zeros(1 << 22, device="cuda")
+    kw = dict(softcap=cap, window=window, part=part)
+
+    def run(x, packed):
+        q, k, v = x.split([nh * hd, kvh * hd, kvh * hd], dim=1)
+        caches = [t if t is None else t.clone() for t in (kc, vc, kS, vS)]
+        out = torch.full((M, nh * hd), 7.0, device="cuda").bfloat16()
+        if packed:
+            K, V, ks, vs = caches
+            ho.rope_cache(q, k, v, K, V, cos, sin, None, M, nh, kvh, hd,
+                          kS=ks, vS=vs, rows=rows)
+            tiles = torch.from_numpy(ho.attn_tiles(segs, nh // kvh)).cuda()
+            ho.attn_prefill_mfma(
+                q, K, V, out, None, M, nh, kvh, hd, hd ** -0.5, kS=ks, vS=vs,
+                keys=S - 3, tiles=tiles, most=max(n for _, _, n in segs),
+                **kw)
+            return out, caches
+        at = 0
+        for b, p, n in segs:                      # each by itself
+            K, V, ks, vs = (t if t is None else t[b] for t in caches)
+            i = slice(at, at + n)
+            p0 = torch.tensor([p], dtype=torch.int32, device="cuda")
+            ho.rope_cache(q[i], k[i], v[i], K, V, cos, sin, p0, n, nh, kvh,
+                          hd, kS=ks, vS=vs)
+            ho.attn_prefill_mfma(q[i], K, V, out[i], p0, n, nh, kvh, hd,
+                                 hd ** -0.5, kS=ks, vS=vs, keys=p + n, **kw)
+            at += n
+        return out, caches
+
+    x = normal(M, (nh + 2 * kvh) * hd, seed=1, scale=2.0)
+    (got, c0), (want, c1) = run(x.clone(), True), run(x.clone(), False)
+    for t, u in zip(c0, c1):
+        assert t is None or torch.equal(t, u)
+    # keys in other ranges: sums in another order, rounded to bf16 at the end
+    assert off(got, want.double()) < 2 ** -8

@@ -1,0 +1,50 @@
+"""Which rows of a group's prompts share a chunk, and their tiles."""
+
+import types
+
+import numpy as np
+import pytest
+
+from llm_np_cp_amd.models.engine import GPUModel
+from llm_np_cp_amd.ops import hip_ops as ho
+
+
+def chunks(lens, PC=64, fp8=False, wq4=False, hd=64):
+    m = types.SimpleNamespace(PC=PC, fp8=fp8, wq4=wq4, hd=hd)
+    return GPUModel._chunks(m, lens)
+
+
+@pytest.mark.parametrize("kind", [{}, {"fp8": True},
+                                  {"fp8": True, "wq4": True}, {"hd": 80}])
+@pytest.mark.parametrize("lens", [[1], [64, 64], [5, 40, 1, 33, 64, 2],
+                                  [200, 3, 65, 129], [1, 1, 1]])
+def test_every_row_once_in_order(lens, kind):
+    out = chunks(lens, **kind)
+    assert all(0 < sum(n for _, _, n in c) <= 64 for c in out)
+    seen = {}
+    for c in out:
+        for b, p, n in c:
+            assert n > 0 and p == seen.get(b, 0)
+            seen[b] = p + n
+    assert [seen[b] for b in range(len(lens))] == lens
+    if "wq4" in kind or "hd" in kind:
+        assert all(len(c) == 1 for c in out)
+    for c in out:                  # as ever: one row beside e4m3 by itself
+        if kind == {"fp8": True} and len(c) > 1:
+            assert all(lens[b] % 64 != 1 for b, _, _ in c)
+
+
+@pytest.mark.parametrize("group", [1, 3, 7])
+@pytest.mark.parametrize("segs", [
+    [(0, 0, 1)], [(3, 7, 4), (1, 0, 2)], [(0, 0, 200), (2, 900, 33)],
+    [(1, 0, 43), (0, 5, 1), (2, 0, 129)]])
+def test_tiles_cover_their_rows(segs, group):
+    t = ho.attn_tiles(segs, group)
+    per = 32 if max(n for _, _, n in segs) * group <= 32 else 128
+    want, row0 = set(), 0
+    for b, p, n in segs:
+        want |= {(i, row0, n, p, b) for i in range(-(-n * group // per))}
+        row0 += n
+    assert len(t) == len(want) and {tuple(r) for r in t.tolist()} == want
+    last = [p + min(n, -(-(i + 1) * per // group)) for i, _, n, p, _ in t]
+    assert (np.diff(last) <= 0).all()
