@@ -120,6 +120,7 @@ class GPUModel(DecodeLoop):
             max_seq = self._auto_max_seq()
         self.max_seq = max_seq
         self._alloc_state(prefill_chunk)
+        self._stack = self._native_stack()
         self._graph = None
         self._graph_mode = None
         # side-stream weight prefetcher — measured NEGATIVE (the fork's
@@ -444,6 +445,60 @@ class GPUModel(DecodeLoop):
         self.final_softcap = float(cfg.final_logit_softcapping or 0.0)
         self.scale = float(cfg.attn_scale)
 
+    def _native_stack(self) -> ho.Stack:
+        """The layers for the native launcher of a prompt's rows."""
+        cfg = self.config
+
+        def lin(lw, name):
+            many = self.moe and name in ("wgu", "wdown")
+            if self.wq4:
+                return lw[name + "_q4"], None, lw[name + "_e4"]
+            if self.fp8:
+                end = "_all" if many else ""
+                return lw[name + "_q" + end], lw[name + "_s" + end], None
+            return lw[name + ("_all" if many else "")], None, None
+
+        layers = []
+        for i, lw in enumerate(self.layers):
+            layers.append(dict(
+                {n: lw.get(n) for n in ("g_in", "g_post", "g_preffn",
+                                        "g_postffn", "bqkv", "wg")},
+                qkv=lin(lw, "wqkv"), o=lin(lw, "wo"), gu=lin(lw, "wgu"),
+                down=lin(lw, "wdown"), kc=self.k_cache[i],
+                vc=self.v_cache[i], kS=self.k_scale[i], vS=self.v_scale[i],
+                window=(cfg.sliding_window or 0) if cfg.is_sliding(i)
+                else 0))
+        own = {n: getattr(self, a, None) for n, a in dict(
+            embed="embed", cos="cos_t", sin="sin_t", h="b_h", xn="b_xn",
+            t1="b_t1", qkv="b_rqkv", att="b_att", gate="b_gate", up="b_up",
+            acc="b_gemm_acc", row_cnt="row_cnt", tile_cnt="tile_cnt",
+            xq="b_xq", sx="b_sx", len="len_buf", moe_idx="moe_idx",
+            moe_w="moe_w", moe_order="moe_order", pairs="b_pairs",
+            aq="b_aq", sa="b_sa").items()}
+        return ho.Stack(
+            layers, **own, acc_floats=self.b_gemm_acc.numel(),
+            order_room=self.moe_order.numel() if self.moe else 0, H=self.H,
+            I=self.inter_l, nh=self.nh_l, kvh=self.kvh_l, hd=self.hd,
+            S=self.max_seq, wt=2 if self.wq4 else 1 if self.fp8 else 0,
+            kv8=int(self.kv8), gemma=int(self.gemma), act=self.act,
+            E=cfg.num_local_experts if self.moe else 0,
+            topk=self.topk if self.moe else 0, nrow_cnt=self.row_cnt.numel(),
+            ntile_cnt=self.tile_cnt.numel(),
+            mfma=int(self.hd in (64, 128, 256)), eps=cfg.rms_norm_eps,
+            scale=self.scale, softcap=self.attn_softcap,
+            escale=cfg.embed_scale)
+
+    def _read(self, ids: np.ndarray, pos0: int, layer_hook=None) -> None:
+        """A chunk of a prompt (int32, up to PC tokens) from position pos0 of
+        sequence _pb through all layers; its rows are in b_h."""
+        M = len(ids)
+        if M > ho.STACK_IDS:
+            self.ids_buf[:M].copy_(torch.from_numpy(ids.astype(np.int32)))
+            self._stack.embed(self.ids_buf, M, pos0)
+        else:
+            self._stack.embed(ids, M, pos0)
+        self._layers_forward(M, layer_hook=layer_hook, keys=pos0 + M)
+
     # ------------------------------------------------------------------
     # cache interface (generate()-compatible)
     # ------------------------------------------------------------------
@@ -603,6 +658,24 @@ class GPUModel(DecodeLoop):
         INDEPENDENT sequences at the same position (lockstep batched
         decode) — the fused decode-attention kernel runs per row over
         per-sequence KV pools instead of the prefill attention."""
+        if not batch_attn and not self.tp_branch:
+            rows, tiles, most = pack or (None, None, 0)
+            kw = dict(keys=keys, pool=self._pb, rows=rows, tiles=tiles,
+                      most=most)
+            if layer_hook is None:
+                self._stack.forward(M, **kw)
+                return
+            layer_hook(-1, self.b_h[:M])
+            for i in range(len(self.layers)):
+                self._stack.forward(M, first=i, last=i + 1, **kw)
+                layer_hook(i, self.b_h[:M])
+            return
+        self._layers_by_launch(M, layer_hook, batch_attn, keys, pack)
+
+    def _layers_by_launch(self, M: int, layer_hook=None,
+                          batch_attn: bool = False, keys: int = 0, pack=None):
+        """The same with a call a launch: steps of a group (captured once)
+        and layers that reduce over ranks in between."""
         cfg = self.config
         eps = cfg.rms_norm_eps
         h, xn, t1 = self.b_h, self.b_xn, self.b_t1
@@ -808,18 +881,13 @@ class GPUModel(DecodeLoop):
         done = 0
         while done < n:
             M = min(n - done, self.PC)
-            self.ids_buf[:M].copy_(
-                torch.from_numpy(ids[done:done + M].astype(np.int32)))
-            ho.i32_set(self.len_buf, done)
-            ho.embed(self.embed, self.ids_buf, self.b_h, M,
-                     self.config.embed_scale)
             d0 = done
 
             def hook(i, h):
                 torch.cuda.synchronize()
                 hidden[i + 1][d0:d0 + h.shape[0]] = \
                     h.float().cpu().numpy()
-            self._layers_forward(M, layer_hook=hook, keys=done + M)
+            self._read(ids[done:done + M], done, layer_hook=hook)
             self._head_rows(M, logits_buf)
             if self.world > 1:
                 # gather vocab shards on-device (each rank holds the
@@ -862,12 +930,7 @@ class GPUModel(DecodeLoop):
         done = 0
         while done < n:
             M = min(n - done, self.PC)
-            self.ids_buf[:M].copy_(
-                torch.from_numpy(ids[done:done + M].astype(np.int32)))
-            ho.i32_set(self.len_buf, pos0 + done)
-            ho.embed(self.embed, self.ids_buf, self.b_h, M,
-                     self.config.embed_scale)
-            self._layers_forward(M, keys=pos0 + done + M)
+            self._read(ids[done:done + M], pos0 + done)
             self._head_rows(M, logits_buf)
             if self.world > 1:
                 # gather vocab shards on-device (each rank holds the
@@ -914,12 +977,7 @@ class GPUModel(DecodeLoop):
         done = 0
         while done < n:
             M = min(n - done, self.PC)
-            self.ids_buf[:M].copy_(
-                torch.from_numpy(ids[done:done + M].astype(np.int32)))
-            ho.i32_set(self.len_buf, pos0 + done)
-            ho.embed(self.embed, self.ids_buf, self.b_h, M,
-                     self.config.embed_scale)
-            self._layers_forward(M, keys=pos0 + done + M)
+            self._read(ids[done:done + M], pos0 + done)
             done += M
         ho.i32_set(self.len_buf, pos0 + n)
         self._host_len = pos0 + n
@@ -1214,11 +1272,7 @@ class GPUModel(DecodeLoop):
                 continue
             (b, done, M), = segs
             self._pb = b
-            self.ids_buf[:M].copy_(torch.from_numpy(seqs[b][done:done + M]))
-            ho.i32_set(self.len_buf, done)
-            ho.embed(self.embed, self.ids_buf, self.b_h, M,
-                     self.config.embed_scale)
-            self._layers_forward(M, keys=done + M)
+            self._read(seqs[b][done:done + M], done)
             if done + M == lens[b]:
                 self._lm_head_last(M)
                 self.bt_logits32[b].copy_(self.b_logits)
@@ -1271,7 +1325,7 @@ class GPUModel(DecodeLoop):
         buf.copy_(torch.from_numpy(host))
         ids, rows, tiles, last = buf.split(
             [M, 2 * M, tiles.size, len(ends)])
-        ho.embed(self.embed, ids, self.b_h, M, self.config.embed_scale)
+        self._stack.embed(ids, M, 0)
         self._layers_forward(
             M, keys=max(p + n for _, p, n in segs),
             pack=(rows, tiles.view(-1, 5), max(n for _, _, n in segs)))
@@ -1306,11 +1360,7 @@ class GPUModel(DecodeLoop):
         done = 0
         while done < P:
             M = min(P - done, self.PC)
-            self.ids_buf[:M].copy_(torch.from_numpy(ids[done:done + M]))
-            ho.i32_set(self.len_buf, done)
-            ho.embed(self.embed, self.ids_buf, self.b_h, M,
-                     self.config.embed_scale)
-            self._layers_forward(M, keys=done + M)
+            self._read(ids[done:done + M], done)
             done += M
         self._lm_head_last(M)
         self._pb = 0

@@ -95,6 +95,11 @@ _SIGS = {
     "launch_moe_scale_add": [ctypes.c_void_p] * 3 +
                             [ctypes.c_long, ctypes.c_int, ctypes.c_int,
                              ctypes.c_void_p],
+    "stack_forward": [ctypes.c_void_p] + [ctypes.c_int] * 5 +
+                     [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2 +
+                     [ctypes.c_void_p],
+    "stack_embed": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 2 +
+                   [ctypes.c_void_p],
     # one-shot xGMI collectives (csrc/xgmi_comm.hip)
     "launch_xgmi_coll": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                          ctypes.c_int, ctypes.c_int, ctypes.c_long,
@@ -584,6 +589,84 @@ def addinto(y: torch.Tensor, a: torch.Tensor):
 
 def i32_set(buf: torch.Tensor, v: int):
     _check(lib().launch_i32_set(_ptr(buf), v, _stream()), "i32_set")
+
+
+# ----------------------------------------------------------------------
+# a prompt's rows through all layers in one call (csrc/stack.hip)
+# ----------------------------------------------------------------------
+
+STACK_IDS = 128      # tokens that come with the embedding's launch
+
+
+class _StackLin(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("w", "s", "e")]
+
+
+class _StackLayer(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in (
+        "g_in", "g_post", "g_preffn", "g_postffn", "bqkv", "wg")] + \
+        [(n, _StackLin) for n in ("qkv", "o", "gu", "down")] + \
+        [(n, ctypes.c_void_p) for n in ("kc", "vc", "kS", "vS")] + \
+        [("window", ctypes.c_long)]
+
+
+class _StackPlan(ctypes.Structure):
+    _fields_ = [("layers", ctypes.POINTER(_StackLayer))] + \
+        [(n, ctypes.c_void_p) for n in (
+            "embed", "cos", "sin", "h", "xn", "t1", "qkv", "att", "gate",
+            "up", "acc", "row_cnt", "tile_cnt", "xq", "sx", "len", "moe_idx",
+            "moe_w", "moe_order", "pairs", "aq", "sa")] + \
+        [(n, ctypes.c_long) for n in ("acc_floats", "order_room")] + \
+        [(n, ctypes.c_int) for n in (
+            "nlayers", "H", "I", "nh", "kvh", "hd", "S", "wt", "kv8",
+            "gemma", "act", "E", "topk", "nrow_cnt", "ntile_cnt", "mfma")] + \
+        [(n, ctypes.c_float) for n in ("eps", "scale", "softcap", "escale")]
+
+
+class Stack:
+    """An engine's layers as the native launcher reads them.  ``layers``: of
+    each layer its tensors by field (a linear's as (w, scales, exponents));
+    ``fields``: the plan's, tensors or numbers.  Holds what it points to."""
+
+    def __init__(self, layers, **fields):
+        self._held = (layers, fields)
+
+        def put(to, values):
+            for n, v in values.items():
+                if isinstance(v, tuple):
+                    v = _StackLin(*[None if t is None else _ptr(t)
+                                    for t in v])
+                elif v is None or isinstance(v, torch.Tensor):
+                    v = None if v is None else _ptr(v)
+                setattr(to, n, v)
+
+        self._layers = (_StackLayer * len(layers))()
+        for to, l in zip(self._layers, layers):
+            put(to, l)
+        self._plan = _StackPlan(layers=self._layers, nlayers=len(layers))
+        put(self._plan, fields)
+        self._at = ctypes.addressof(self._plan)
+
+    def embed(self, ids, M: int, pos0: int):
+        """Rows of M tokens into h, and pos0 into len: ids on the host (int32
+        numpy, up to STACK_IDS) or on the device."""
+        host = isinstance(ids, np.ndarray)
+        assert not host or (ids.dtype == np.int32 and len(ids) == M
+                            and ids.flags.c_contiguous)
+        _check(lib().stack_embed(
+            self._at, ids.ctypes.data if host else None,
+            None if host else ids.data_ptr(), M, pos0, _stream()),
+            "stack_embed")
+
+    def forward(self, M: int, keys: int, pool: int = 0, first: int = 0,
+                last: int | None = None, rows=None, tiles=None, most: int = 0):
+        """Rows [0, M) of h through layers [first, last); rows, tiles, most
+        as for rope_cache and attn_prefill_mfma."""
+        _check(lib().stack_forward(
+            self._at, M, keys, pool, first,
+            len(self._layers) if last is None else last, _ptr(rows),
+            _ptr(tiles), 0 if tiles is None else tiles.shape[0], most,
+            _stream()), "stack_forward")
 
 
 # ----------------------------------------------------------------------
