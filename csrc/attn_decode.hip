@@ -91,30 +91,16 @@ DEVINL void ad_merge(const AdArgs& a, const float* part, u16* out, int ng,
   __shared__ float wt[GB][AD_MAX_SPLIT], sum[GB];
   const int tid = threadIdx.x;
   const size_t rowp = (size_t)gridDim.y * (HD + 2);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  int* cnt = a.cnt + blockIdx.z * gridDim.x + blockIdx.x;
-  if (tid == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const int t = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-    *last_flag = t == eff - 1;
-  }
-  __syncthreads();
-  if (!*last_flag) return;
-  if (tid == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    *cnt = 0;                                  // for the next step
-  }
-  __syncthreads();
+  if (!last_block(a.cnt + blockIdx.z * gridDim.x + blockIdx.x, eff,
+                  last_flag))
+    return;
   // a wave a head: the weights of its parts and their sum
   for (int g = tid >> 6; g < ng; g += blockDim.x >> 6) {
     const int c = tid & 63;
     float m = -INFINITY, l = 0.f;
     if (c < eff) {
-      m = part[g * rowp + c * (HD + 2)];
-      l = part[g * rowp + c * (HD + 2) + 1];
+      m = part_get(part + g * rowp + c * (HD + 2));
+      l = part_get(part + g * rowp + c * (HD + 2) + 1);
     }
     float mt = m;
 #pragma unroll
@@ -133,7 +119,7 @@ DEVINL void ad_merge(const AdArgs& a, const float* part, u16* out, int ng,
       float x[Q];
 #pragma unroll
       for (int i = 0; i < Q; i++)
-        x[i] = pp[(size_t)min(c0 + i, eff - 1) * (HD + 2)];
+        x[i] = part_get(pp + (size_t)min(c0 + i, eff - 1) * (HD + 2));
       if (e0 == 0 && c0 == 0) __syncthreads();
 #pragma unroll
       for (int i = 0; i < Q; i++)
@@ -415,8 +401,11 @@ __global__ void __launch_bounds__(64 * AD_NW) k_attn_dec_any(AdArgs a) {
       out[e] = f2b(v / lt);
     } else {
       float* pp = part + g * rowp + chunk * (HD + 2);
-      pp[2 + d] = v;
-      if (d == 0) { pp[0] = mt; pp[1] = lt; }
+      part_put(pp + 2 + d, v);
+      if (d == 0) {
+        part_put(pp, mt);
+        part_put(pp + 1, lt);
+      }
     }
   }
   if (eff == 1) return;
@@ -758,8 +747,11 @@ k_attn_dec(AdArgs a) {
       out[e] = f2b(v / lt);
     } else {
       float* pp = parts + h * rowp + chunk * (HD + 2);
-      pp[2 + d] = v;
-      if (d == 0) { pp[0] = mt; pp[1] = lt; }
+      part_put(pp + 2 + d, v);
+      if (d == 0) {
+        part_put(pp, mt);
+        part_put(pp + 1, lt);
+      }
     }
   }
   if (eff == 1) return;

@@ -294,24 +294,9 @@ k_gemm_prompt(GpArgs a) {
     for (int i = 0; i < FM; i++)
 #pragma unroll
       for (int j = 0; j < FN; j++)
-        *(f4v*)(pp + (size_t)blockIdx.y * (BM * BN) +
-                (i * FN + j) * (NW * 256)) = acc[i][j];
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (tid == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      const int t = __hip_atomic_fetch_add(&a.cnt[tile], 1, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-      last_flag = t == SK - 1;
-    }
-    __syncthreads();
-    if (!last_flag) return;
-    if (tid == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      a.cnt[tile] = 0;                                  // for the next launch
-    }
-    __syncthreads();
+        part_put4(pp + (size_t)blockIdx.y * (BM * BN) +
+                  (i * FN + j) * (NW * 256), acc[i][j]);
+    if (!last_block(&a.cnt[tile], SK, &last_flag)) return;
     // up to 16 fragments of a part on the way at a time: a part a trip, not
     // a fragment of one
     constexpr int G = FM * FN > 16 ? 16 / FN : FM;
@@ -327,8 +312,8 @@ k_gemm_prompt(GpArgs a) {
         for (int i = 0; i < G; i++)
 #pragma unroll
           for (int j = 0; j < FN; j++)
-            t[i][j] = *(const f4v*)(pp + (size_t)q * (BM * BN) +
-                                    ((i0 + i) * FN + j) * (NW * 256));
+            t[i][j] = part_get4(pp + (size_t)q * (BM * BN) +
+                                ((i0 + i) * FN + j) * (NW * 256));
 #pragma unroll
         for (int i = 0; i < G; i++)
 #pragma unroll

@@ -1074,16 +1074,16 @@ k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
   if (threadIdx.x == 0) {
     uint64_t b = ws[0];
     for (int w = 1; w < NT / 64; w++) if (ws[w] > b) b = ws[w];
+    // atomics of the device both, one after the other: nothing to write back
     atomicMax(pick, (unsigned long long)b);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    int t = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_ACQ_REL,
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    int t = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
     lastflag = (t == (int)gridDim.x - 1);
   }
   __syncthreads();
   if (!lastflag || threadIdx.x != 0) return;
   // last arriver: commit the winner, reset scratch, advance state
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   *cnt = 0;
   int winner = unpack_idx(
       __hip_atomic_load(pick, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));

@@ -419,31 +419,15 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
         finish(e, v, up, o[j]);
       } else {
         float* pp = parts + ((size_t)t * KS + blockIdx.y) * (P * 256) + (e & 255);
-        pp[0] = v;
-        if (GLU) pp[256] = up;
+        part_put(pp, v);
+        if (GLU) part_put(pp + 256, up);
       }
     }
   }
   if (KS == 1) return;
 
   // the last of the blocks that share these columns adds the parts
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (tid == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const int t = __hip_atomic_fetch_add(&a.cnt[blockIdx.x], 1,
-                                         __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-    last_flag = t == KS - 1;
-  }
-  __syncthreads();
-  if (!last_flag) return;
-  if (tid == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    a.cnt[blockIdx.x] = 0;                   // for the next launch
-  }
-  __syncthreads();
+  if (!last_block(&a.cnt[blockIdx.x], KS, &last_flag)) return;
   for (int e = tid; e < ntile * 256; e += 64 * RG_NW) {
     if (((e >> 4) & 15) >= a.M) continue;
     const float* pp = parts + (size_t)(e >> 8) * KS * (P * 256) + (e & 255);
@@ -453,8 +437,9 @@ __global__ void __launch_bounds__(64 * RG_NW) k_row_gemm(RgArgs a) {
       float x[8], y[8];
 #pragma unroll
       for (int q = 0; q < 8; q++) {
-        x[q] = pp[(size_t)min(q0 + q, KS - 1) * (P * 256)];
-        if (GLU) y[q] = pp[(size_t)min(q0 + q, KS - 1) * (P * 256) + 256];
+        const float* at = pp + (size_t)min(q0 + q, KS - 1) * (P * 256);
+        x[q] = part_get(at);
+        if (GLU) y[q] = part_get(at + 256);
       }
 #pragma unroll
       for (int q = 0; q < 8; q++)
