@@ -32,7 +32,7 @@ PKG = os.path.join(ROOT, "llm_np_cp_amd")
 LIBS = {
     "llmops": ["llm_ops.hip", "gemv.hip", "attn_decode.hip",
                "attn_prefill.hip", "row_gemm.hip", "gemm_prompt.hip",
-               "stack.hip", "xgmi_comm.hip"],
+               "mid_gemm.hip", "stack.hip", "xgmi_comm.hip"],
     "linear": ["linear.hip"],
     "latent": ["latent_attn.hip"],
     "gqa": ["gqa_attn.hip"],
@@ -44,7 +44,7 @@ LIBS = {
     "moe": ["moe.hip"],
 }
 HEADERS = ["attn_prefill.h", "attn_split.h", "common.h", "gemm_tile.h",
-           "gemv.h", "hybrid.h", "mingru.h", "moe.h"]
+           "gemv.h", "hybrid.h", "mid_gemm.h", "mingru.h", "moe.h"]
 # Packed fp32 VALU forms are kept out of all device code: some of them
 # have returned wrong results on this hardware.  (The host pass warns that
 # it does not know the feature.)

@@ -24,6 +24,7 @@
 // With few tiles K is split over blocks; the last block of a tile to arrive
 // adds the parts in their order (the result does not depend on timing).
 #include "common.h"
+#include "mid_gemm.h"
 
 typedef short gp_s8 __attribute__((ext_vector_type(8)));
 typedef int gp_i8 __attribute__((ext_vector_type(8)));
@@ -477,6 +478,10 @@ extern "C" hipError_t launch_gemm_prompt(
               (const u16*)bias, (u16*)y, (float*)part, (int*)cnt, M, N, K,
               act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
   if (!part || !cnt) part_floats = 0;
+  if (mid_takes(sx, M, N, K, act >= 0))
+    return launch_mid_gemm(x, w, sx, sw, res, bias, y, part, cnt, part_floats,
+                           ncnt, M, N, K, K, res ? N : 0, N, act, 0, 0.f,
+                           stream);
   return sx ? gp_run<true>(a, part_floats, ncnt, stream)
             : gp_run<false>(a, part_floats, ncnt, stream);
 }

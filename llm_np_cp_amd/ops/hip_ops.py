@@ -59,6 +59,8 @@ _SIGS = {
     "launch_row_gemm": [ctypes.c_void_p] * 11 + [ctypes.c_long] +
                        [ctypes.c_int] * 11 +
                        [ctypes.c_float, ctypes.c_float, ctypes.c_void_p],
+    "launch_mid_gemm": [ctypes.c_void_p] * 9 + [ctypes.c_long] +
+                       [ctypes.c_int] * 9 + [ctypes.c_float, ctypes.c_void_p],
     "row_gemm_plan": [ctypes.c_int] * 6 + [ctypes.c_long, ctypes.c_int,
                                            ctypes.c_void_p],
     "launch_prefetch": [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p,
@@ -447,6 +449,29 @@ def row_gemm(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, M: int,
         res.stride(0) if res is not None else 0, y.stride(0), act,
         1 if y.dtype == torch.float32 else 0, int(norm16),
         ctypes.c_float(eps), ctypes.c_float(softcap), _stream()), "row_gemm")
+
+
+def mid_gemm(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, M: int,
+             ws: torch.Tensor | None = None, sx: torch.Tensor | None = None,
+             bias: torch.Tensor | None = None,
+             res: torch.Tensor | None = None, act: int = -1,
+             softcap: float = 0.0, part: torch.Tensor | None = None,
+             cnt: torch.Tensor | None = None):
+    """Y[M<=64, N] = X W^T, bf16 or e4m3 (x bytes, sx and ws scales of rows),
+    the rest as for row_gemm without a norm (gate: up to 32 rows).  row_gemm
+    and gemm hand on what it is faster for."""
+    K, N = x.shape[-1], w.shape[0] // (2 if act >= 0 else 1)
+    assert w.shape[1] == K and w.is_contiguous() and (sx is None) == \
+        (ws is None)
+    assert x.stride(-1) == 1 and y.stride(-1) == 1
+    _check(lib().launch_mid_gemm(
+        _ptr(x), _ptr(w), _ptr(sx), _ptr(ws), _ptr(res), _ptr(bias), _ptr(y),
+        _ptr(part), _ptr(cnt),
+        ctypes.c_long(0 if part is None else part.numel()),
+        0 if cnt is None else cnt.numel(), M, N, K, x.stride(0),
+        res.stride(0) if res is not None else 0, y.stride(0), act,
+        1 if y.dtype == torch.float32 else 0, ctypes.c_float(softcap),
+        _stream()), "mid_gemm")
 
 
 def row_gemm_plan(kind: str, M: int, N: int, K: int, glu: bool = False,

@@ -725,3 +725,56 @@ def test_prompts_of_one_batch(hd, nh, kvh, segs, window, cap, kv8):
         assert t is None or torch.equal(t, u)
     # keys in other ranges: sums in another order, rounded to bf16 at the end
     assert off(got, want.double()) < 2 ** -8
+
+
+# row tiles of 16, outputs that end inside a tile (also where four do not fit),
+# one slab, fewer slabs than waves, half a slab at the end, K split over two
+# and more blocks, rows apart
+@pytest.mark.parametrize("f8", [False, True])
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(16, 64), (40, 192), (4130, 320),
+                                 (70, 9280), (33, 16448), (256, 4096)])
+@pytest.mark.parametrize("kind", ["plain", "all", "gate"])
+def test_some_rows(f8, M, N, K, kind):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    if kind == "gate" and M > 32:
+        pytest.skip("a gate takes up to 32 rows")
+    act = 1 if kind == "gate" else -1
+    X = normal(M, K + 32, seed=1)[:, :K]
+    W = normal(N * (2 if act >= 0 else 1), K, seed=2, scale=K ** -0.5)
+    Xd, Wd, kw = X.double(), W.double(), {}
+    if f8:
+        (X, kw["sx"], Xd), (W, kw["ws"], Wd) = e4m3(X), e4m3(W)
+    ref = Xd @ Wd.T
+    # fp32 sums: as many roundings as products, of the sum of magnitudes
+    far = Xd.abs() @ Wd.abs().T * (K * 2.0 ** -23)
+    if kind == "gate":
+        g, u = ref.chunk(2, 1)
+        gf, uf = far.chunk(2, 1)
+        t = torch.nn.functional.gelu(g, approximate="tanh")
+        # the activation's slope is at most 1.13, and 2^-20 of tanh
+        far = (gf * 1.13 + g.abs() * 2.0 ** -20) * (u.abs() + uf) + \
+            t.abs() * uf
+        ref = t * u
+    Y = torch.full((M + 1, N + 4), 7.0, device="cuda").bfloat16()
+    if kind == "all":
+        kw["bias"], kw["softcap"] = normal(N, seed=3), 3.0
+        kw["res"] = normal(M, N + 12, seed=4)[:, :N]
+        ref = 3.0 * torch.tanh(ref / 3.0) + kw["bias"].double() + \
+            kw["res"].double()
+        far = far + 2.0 ** -20
+        Y = Y.float()
+    part = torch.full((1 << 21,), float("nan"), device="cuda")
+    cnt = torch.zeros(256, dtype=torch.int32, device="cuda")
+    for _ in range(2):               # the counters are left zero
+        ho.mid_gemm(X, W, Y[:M, :N], M, act=act, part=part, cnt=cnt, **kw)
+        if f8:
+            # e4m3 products are cut off at the largest one's place before
+            # they are added (2^-18 of the sum seen): like more rows'
+            assert off(Y[:M, :N], ref) < 2.0 ** (-9 if act < 0 else -8)
+        err = (Y[:M, :N].double() - ref).abs()
+        round_ = 0.0 if kind == "all" else ref.abs() * 2.0 ** -8
+        assert f8 or (err <= far + round_ + 1e-30).all()
+        assert (Y[M] == 7.0).all() and (Y[:, N:] == 7.0).all()
+        assert not cnt.any()
