@@ -20,7 +20,7 @@
 // Measured (32/8 heads of 128, 2048 rows behind 6139 keys): 291 us,
 // 827 TFLOP/s; a wave per head and 16 queries took 1422 us.  (With both
 // buffers in one array the DMA drained ahead of every tile's reads: 314 us.)
-// 5 rows of 24/8 heads over 906 keys, split: 18 us, unsplit per-head waves
+// 5 rows of 24/8 heads over 906 keys, split: 14 us, unsplit per-head waves
 // 74 us.  Head dim 256 at two waves a SIMD just fits the registers without a
 // soft cap; with one it spills 7, beside an e4m3 pool 36 (12 to 14 where one
 // wave has all rows).  One wave a SIMD without spills was slower (2048 rows
@@ -407,19 +407,33 @@ __global__ void __launch_bounds__(256) k_attn_rows_merge(ApArgs a, int split) {
   const int kvhead = w / nrows, row = w % nrows;
   const size_t stride = (size_t)a.kvh * nrows * (HD + 4);
   const float* p = a.part + ((size_t)kvhead * nrows + row) * (HD + 4);
-  float m = -INFINITY;
-  for (int z = 0; z < split; z++) m = fmaxf(m, p[z * stride + HD]);
-  float l = 0.f, v[HD / 64];
+  // a lane a part: all maxima and sums in one trip, then eight parts a trip
+  const int zl = min(lane, split - 1);
+  const float mz = lane < split ? p[zl * stride + HD] : -INFINITY;
+  const float lz = p[zl * stride + HD + 1];
+  float m = mz;
+#pragma unroll
+  for (int w = 1; w < 64; w <<= 1) m = fmaxf(m, __shfl_xor(m, w));
+  // a part without keys of this row holds nothing
+  const float al = mz == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mz - m);
+  const float l = wave_reduce_sum(mz == -INFINITY ? 0.f : lz * al);
+  float v[HD / 64];
 #pragma unroll
   for (int i = 0; i < HD / 64; i++) v[i] = 0.f;
-  for (int z = 0; z < split; z++) {
-    const float mz = p[z * stride + HD];
-    if (mz == -INFINITY) continue;
-    const float al = __builtin_amdgcn_exp2f(mz - m);
-    l += p[z * stride + HD + 1] * al;
+  for (int z0 = 0; z0 < split; z0 += 8) {
+    float x[8][HD / 64];
 #pragma unroll
-    for (int i = 0; i < HD / 64; i++)
-      v[i] += p[z * stride + i * 64 + lane] * al;
+    for (int z = 0; z < 8; z++)
+#pragma unroll
+      for (int i = 0; i < HD / 64; i++)
+        x[z][i] = p[min(z0 + z, split - 1) * stride + i * 64 + lane];
+#pragma unroll
+    for (int z = 0; z < 8; z++) {
+      const float w = __shfl(al, min(z0 + z, 63));
+      if (z0 + z < split && w > 0.f)
+#pragma unroll
+        for (int i = 0; i < HD / 64; i++) v[i] += x[z][i] * w;
+    }
   }
   u16* op = a.out + ((size_t)(row / grp) * a.nh + kvhead * grp + row % grp) * HD;
 #pragma unroll
@@ -444,15 +458,20 @@ static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
   // up to 32 rows are one wave's; more share their tiles among four
   const int nw = most * (a.nh / a.kvh) <= 32 ? 1 : 4;
   const int tiles = a.tiles ? ntiles : (rows + nw * 32 - 1) / (nw * 32);
-  // Too few blocks for 256 CUs of two each: the keys are split too, down
-  // to four tiles a block.
+  // Too few blocks for 256 CUs of two each: the keys are split too, down to
+  // four tiles a block, where blocks are very few to one (from four tiles on:
+  // a part costs the launch that adds them).  us, attention and sum, by four
+  // -> here: five rows of 24/8 heads of 128 over 906 keys 19.3 -> 13.6, over
+  // 6000 of 32/8 e4m3 heads 39.9 -> 23.1, seven of 8/4 of 256 over 900 25.0 ->
+  // 16.8, nine of 28/4 of 128 over 500 16.9 -> 13.0.
   int split = 1;
   const int want = nw == 1 ? 1024 : 512;
   if (tiles * a.kvh * 2 <= want && a.part) {
     split = want / (tiles * a.kvh);
     const int span = a.window > 0 && a.window + most < keys ? a.window + most
                                                             : keys;
-    const int worth = span / (4 * BKV);
+    const int one = span / BKV;
+    const int worth = tiles * a.kvh > 64 ? one / 4 : one < 4 ? 1 : one;
     if (split > worth) split = worth;
     if (split > 64) split = 64;
     const long each = (long)a.kvh * rows * (HD + 4);
