@@ -924,14 +924,17 @@ class GPUModel(DecodeLoop):
         if pos0 + n > self.max_seq:
             raise ValueError(f"sequence {pos0}+{n} exceeds max_seq "
                              f"{self.max_seq}")
-        out = np.empty((n, self.config.vocab_size), dtype=np.float32)
-        logits_buf = torch.empty(self.PC, self.vocab_l,
+        out = None
+        logits_buf = torch.empty(min(n, self.PC), self.vocab_l,
                                  dtype=torch.bfloat16, device=self.device)
         done = 0
         while done < n:
             M = min(n - done, self.PC)
             self._read(ids[done:done + M], pos0 + done)
             self._head_rows(M, logits_buf)
+            if done + M == n:
+                ho.i32_set(self.len_buf, pos0 + n)
+                self._host_len = pos0 + n
             if self.world > 1:
                 # gather vocab shards on-device (each rank holds the
                 # columns [r*vocab_l, (r+1)*vocab_l) of rows [0, M))
@@ -941,12 +944,13 @@ class GPUModel(DecodeLoop):
                 dist.all_gather(chunks, t)
                 loc = torch.cat(chunks, dim=1).cpu().numpy()
             else:
-                torch.cuda.synchronize()
                 loc = logits_buf[:M].float().cpu().numpy()
+            if M == n:           # widened on the device, copied once
+                return loc
+            if out is None:
+                out = np.empty((n, self.config.vocab_size), dtype=np.float32)
             out[done:done + M] = loc
             done += M
-        ho.i32_set(self.len_buf, pos0 + n)
-        self._host_len = pos0 + n
         return out
 
     def rewind(self, n: int):
@@ -979,12 +983,11 @@ class GPUModel(DecodeLoop):
             M = min(n - done, self.PC)
             self._read(ids[done:done + M], pos0 + done)
             done += M
+        self._lm_head_last(M)
         ho.i32_set(self.len_buf, pos0 + n)
         self._host_len = pos0 + n
-        self._lm_head_last(M)
         cache.seq_len = pos0 + n
-        torch.cuda.synchronize()
-        return self.b_logits.float().cpu().numpy()[None, :]
+        return self.b_logits.cpu().numpy()[None, :]     # waits for it
 
     # ------------------------------------------------------------------
     # fast device-side decode loop (graph-replayable)
