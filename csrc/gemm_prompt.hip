@@ -399,24 +399,34 @@ static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
 }
 
 // Tile sizes, and microseconds that a slab takes on a CU that runs one block
-// of them or as many as fit (measured with a full chip, bf16; e4m3 slabs move
-// the same bytes and differ by a tenth).  Large tiles ask L2 for the fewest
-// bytes a product: 128x128 by four waves wants 64 bytes a clock, all that a
-// CU gets.  They win where there are rounds of them; where tiles are fewer
-// than the chip has CUs a smaller one that is deep in flight does.
-struct GpTile { int bm, bn, occ; float one, full; };
+// of them or as many as fit, in bf16 and in e4m3, and those that a round costs
+// besides (first slabs, epilogue).  Large tiles ask L2 for the fewest bytes a
+// product: 128x128 by four waves wants 64 bytes a clock, all that a CU gets.
+// They win where there are rounds of them; where tiles are fewer than the chip
+// has CUs a smaller one that is deep in flight does.
+// The numbers are fitted to the times of every tile and split (1 to 8 parts)
+// for 324 products: 70 to 2048 rows of 27 shapes of both types (2048x2048 to
+// 18944x3584).  Chosen by them a product takes 0.9% more than with its best
+// tile and split on average; by bf16 slab times for both types and splits of
+// 1, 2, 4, 8 at what they cost while parts were flushed, 6.0% (70x3584x14336
+// e4m3 26.8 us, here 19.1; 907x2304x9216 102, 72; 611x3584x18944 160, 115).
+struct GpTile {
+  int bm, bn, occ;
+  float one[2], full[2], round;
+};
 static const GpTile gp_tiles[] = {
-    {256, 256, 1, 1.60f, 1.60f},    // bf16 only: e4m3 fragments would spill
-    {128, 256, 1, 0.94f, 0.94f}, {128, 128, 2, 0.82f, 1.10f},
-    {128, 128, 1, 0.56f, 0.56f},    // eight waves, four buffers
-    {64, 128, 2, 0.41f, 0.665f}, {128, 64, 2, 0.41f, 0.665f},
-    {64, 64, 2, 0.26f, 0.47f},   {32, 64, 2, 0.17f, 0.40f},
+    // bf16 only (e4m3 fragments would spill), not split: its parts cost most
+    {256, 256, 1, {1.48f, 1.311f}, {1.48f, 1.311f}, 6.2f},
+    {128, 256, 1, {0.87f, 1.225f}, {0.87f, 1.225f}, 4.0f},
+    {128, 128, 2, {0.546f, 1.385f}, {1.032f, 2.773f}, 3.2f},
+    // eight waves, four buffers
+    {128, 128, 1, {0.494f, 0.718f}, {0.494f, 0.718f}, 3.4f},
+    {64, 128, 2, {0.652f, 0.758f}, {0.73f, 0.834f}, 1.8f},
+    {128, 64, 2, {0.734f, 0.881f}, {0.918f, 1.407f}, 1.6f},
+    {64, 64, 2, {0.261f, 0.472f}, {0.499f, 0.563f}, 1.4f},
+    {32, 64, 2, {0.231f, 0.286f}, {0.288f, 0.459f}, 1.8f},
 };
 
-// us, chosen by rates of one block on an otherwise idle chip -> by these:
-//   1999x2048x8192 110 -> 72, 2048x6144x4096 132 -> 101, 2048x2304x9216 194 ->
-//   125, 907x2304x9216 92 -> 83, 300x3584x18944 189 -> 84, 60x4608x3584 35 ->
-//   18, 37x2048x8192 25 -> 18
 template <bool F8>
 static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
                          hipStream_t s) {
@@ -428,21 +438,23 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
     const GpTile& g = gp_tiles[c];
     const long tiles = (long)((a.M + g.bm - 1) / g.bm) *
                        ((width + g.bn - 1) / g.bn);
-    for (int sk = 1; sk <= 8; sk *= 2) {
+    for (int sk = 1; sk <= 8; sk++) {
       const double parts = (double)tiles * sk * g.bm * g.bn;
-      if (sk > 1 && (tiles > ncnt || parts > part_floats || slabs / sk < 4))
+      if (sk > 1 && (c == 0 || tiles > ncnt || tiles * sk > 700 ||
+                     parts > part_floats || slabs / sk < 4))
         break;
-      // Full rounds and a rest.  Blocks alone on their CU share L2 and
-      // memory with fewer others where not all CUs have one; a few CUs with
-      // two set the time for all.
+      // Full rounds and a rest.  A few CUs with two blocks set the time for
+      // all.
+      const float one = g.one[F8], full = g.full[F8];
       const float x = (float)(tiles * sk) / 256.f;       // blocks of a CU
-      const float rest = x - (int)(x / g.occ) * g.occ;
-      float t = (int)(x / g.occ) * g.full;
-      if (rest > 1.f) t += g.one + (g.full - g.one) * (0.35f + 0.65f * (rest - 1.f));
-      else if (rest > 0.f) t += g.one * (0.8f + 0.2f * rest);
-      t *= (slabs + sk - 1) / sk;
-      // parts written and read (2.6 TB/s), a trip for each
-      if (sk > 1) t += 3.f + 0.7f * sk + (float)(parts * 1.54e-6);
+      const int rounds = (int)(x / g.occ);
+      const float rest = x - rounds * g.occ;
+      float t = rounds * full;
+      if (rest > 1.f) t += one + (full - one) * (0.42f + 0.58f * (rest - 1.f));
+      else if (rest > 0.f) t += one * (0.96f + 0.04f * rest);
+      t = t * ((slabs + sk - 1) / sk) + (rounds + (rest > 0.f)) * g.round;
+      // parts written and read, and a trip for each
+      if (sk > 1) t += 2.1f + (float)(parts * 5.0e-6);
       if (best < 0 || t < best_t) {
         best = c;
         best_sk = sk;
