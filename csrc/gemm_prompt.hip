@@ -1,5 +1,6 @@
 // gemm_prompt.hip — linears of many rows: Y[M,N] = X[M,K] W[N,K]^T, bf16 or
-// e4m3 with row scales, fp32 sums, bf16 out.
+// e4m3 with row scales, or bf16 rows beside MXFP4 weights; fp32 sums, bf16
+// out.
 //
 // Slabs of 128 bytes a row (64 bf16, 128 e4m3) go straight into LDS, two to
 // six buffers, one barrier a slab that waits for the next slab only and
@@ -21,6 +22,16 @@
 // 16 in a tile (GLU): a lane has both halves of its outputs and stores
 // act(gate) * up, half the bytes and one launch instead of three.
 //
+// MXFP4 weights are widened to bf16 (exact) on their way into LDS, once a
+// block, between the operands of the next products and the products at hand.
+// A thread asks for its piece of a slab as many slabs ahead as there are
+// buffers: two ahead, and put down before the operands are read, 2048 rows of
+// 37888x3584 with the gate took 881 us, so 605.  With double-buffered tiles of
+// 128x128 alone, a wait for all each slab, parts of K that were added by
+// atomics to zeroed sums and a launch for each half of a gate it was 911; 130
+// rows 194 us, here 91; 600 rows of 3584x18944 266, 130.  The halves of a gate
+// are not rounded to bf16 any more on their way to it.
+//
 // With few tiles K is split over blocks; the last block of a tile to arrive
 // adds the parts in their order (the result does not depend on timing).
 #include "common.h"
@@ -35,6 +46,7 @@ struct GpArgs {
   const void* w;       // [N, K], GLU: [2N, K] gate then up
   const float* sx;     // e4m3: row scales
   const float* sw;
+  const uint8_t* we;   // MXFP4: exponents [rows of w, K/32]
   const u16* res;      // [M, N]
   const u16* bias;     // [N]
   u16* y;              // [M, N]
@@ -66,14 +78,15 @@ template <int N> DEVINL void gp_meet() {
 }
 
 template <bool F8, int BM, int BN, int WM, int WN, int NS, bool GLU,
-          bool MOE = false>
+          bool MOE = false, bool W4 = false>
 __global__ void __launch_bounds__(64 * WM * WN)
 k_gemm_prompt(GpArgs a) {
   constexpr int NW = WM * WN;
   constexpr int FM = BM / WM / 16, FN = BN / WN / 16;   // fragments of a wave
   constexpr int AI = BM / 8 / NW, BI = BN / 8 / NW;     // DMA of a wave
   static_assert(AI > 0 && BI > 0 && FM > 0 && FN % (GLU ? 2 : 1) == 0);
-  constexpr int PS = AI + BI;
+  // loads of a wave for a slab (MXFP4: a piece of W and its exponent)
+  constexpr int PS = W4 ? AI + 2 : AI + BI;
   // An array a buffer, and the loop unrolled over them: the compiler sees
   // that a DMA into one does not touch what is read from another, and puts
   // no wait for it before the reads.
@@ -117,24 +130,55 @@ k_gemm_prompt(GpArgs a) {
 
   const int g_r = lane >> 3, g_s = lane & 7;
   const char* pa[AI];
-  const char* pb[BI];
+  [[maybe_unused]] const char* pb[BI];
 #pragma unroll
   for (int i = 0; i < AI; i++) {
     const int r = (wave * AI + i) * 8 + g_r;
     pa[i] = (const char*)a.x + (size_t)x_row(min(bm + r, rows - 1)) * rowb;
   }
+  auto w_row = [&](int r) {                  // of W, row r of the tile
+    if (!GLU) return (size_t)min(bn + r, a.N - 1);
+    const int n = min(bn + (r >> 5) * 16 + (r & 15), a.N - 1);
+    return ((r >> 4) & 1) ? (size_t)a.N + n : (size_t)n;
+  };
+  if constexpr (!W4)
 #pragma unroll
-  for (int i = 0; i < BI; i++) {
-    const int r = (wave * BI + i) * 8 + g_r;
-    size_t row;
-    if (GLU) {
-      const int n = min(bn + (r >> 5) * 16 + (r & 15), a.N - 1);
-      row = ((r >> 4) & 1) ? (size_t)a.N + n : (size_t)n;
-    } else {
-      row = min(bn + r, a.N - 1);
-    }
-    pb[i] = (const char*)a.w + (w0 + row) * rowb;
+    for (int i = 0; i < BI; i++)
+      pb[i] = (const char*)a.w + (w0 + w_row((wave * BI + i) * 8 + g_r)) * rowb;
+  // MXFP4: a thread's piece of a slab, 32 or 16 values of a row
+  constexpr int WB = W4 ? BN * 32 / (64 * NW) : 16, WT = 32 / WB;
+  static_assert(WB == 16 || WB == 8);
+  const int w_r = tid / WT, w_p = tid % WT;
+  [[maybe_unused]] const uint8_t *p4 = nullptr, *pe = nullptr;
+  if constexpr (W4) {
+    p4 = (const uint8_t*)a.w + w_row(w_r) * (a.K / 2) + w_p * WB;
+    pe = a.we + w_row(w_r) * (a.K / 32) + w_p * WB / 16;
   }
+  [[maybe_unused]] uint32_t raw[NS][WB / 4], rexp[NS];
+  auto ask = [&](int b, int s) {             // the piece of slab s
+    s = min(s, s_hi - 1);
+    if constexpr (WB == 16) *(u4v_*)raw[b] = *(const u4v_*)(p4 + s * 32);
+    else *(uint2*)raw[b] = *(const uint2*)(p4 + s * 32);
+    rexp[b] = pe[s * 2];
+  };
+  auto widen = [&](int b, char* B) {         // and into LDS
+    const float sc = __uint_as_float(rexp[b] << 23);
+#pragma unroll
+    for (int d = 0; d < WB / 4; d++) {
+      union { gp_b2 p[4]; u4v_ u; } o;
+      o.p[0] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw[b][d], sc, 0);
+      o.p[1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw[b][d], sc, 1);
+      o.p[2] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw[b][d], sc, 2);
+      o.p[3] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(raw[b][d], sc, 3);
+      const int slot = (w_p * (WB / 4) + d) ^ ((w_r >> 1) & 7);
+      *(u4v_*)(B + w_r * 128 + slot * 16) = o.u;
+    }
+  };
+  auto put = [&](int b, char* B, int s) {
+    widen(b, B);
+    ask(b, s + NS);
+    asm volatile("" ::: "memory");
+  };
   // row r of a tile keeps slot q at q ^ ((r >> 1) & 7)
   const int src0 = (g_s ^ (g_r >> 1)) * 16, src1 = src0 ^ 64;
   auto stage = [&](char* A, char* B, int s) {
@@ -148,6 +192,10 @@ k_gemm_prompt(GpArgs a) {
               pa[i] + (((wave * AI + i) & 1) ? k1 : k0)),
           (__attribute__((address_space(3))) uint32_t*)(
               A + (wave * AI + i) * 1024), 16, 0, 0);
+    if constexpr (W4) {
+      asm volatile("" ::: "memory");       // the waits count loads in order
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < BI; i++)
       __builtin_amdgcn_global_load_lds(
@@ -172,9 +220,14 @@ k_gemm_prompt(GpArgs a) {
   // conditions while there are slabs to ask for; the last few wait for all.
   int s = s_lo;
   if (s_lo < s_hi) {
+    if constexpr (W4)
 #pragma unroll
-    for (int u = 0; u < NS; u++)
+      for (int u = 0; u < NS; u++) ask(u, s_lo + u);
+#pragma unroll
+    for (int u = 0; u < NS; u++) {
       if (s_lo + u < s_hi) stage(A[u], B[u], s_lo + u);
+      if constexpr (W4) put(u, B[u], s_lo + u);
+    }
     // all but the first may still be in flight
     if (s_lo + NS <= s_hi) gp_meet<PS * (NS - 1)>();
     else gp_meet<0>();
@@ -259,7 +312,7 @@ k_gemm_prompt(GpArgs a) {
         __builtin_amdgcn_sched_barrier(0);
       };
       auto slab = [&](char* A, char* B, const char* An, const char* Bn,
-                      int s, bool steady) {
+                      int s, int u, bool steady) {
         fetch(1, A, B);
         mma(0);
         if (steady) {
@@ -271,19 +324,23 @@ k_gemm_prompt(GpArgs a) {
           if (s + NS < s_hi) stage(A, B, s + NS);
           fetch(0, An, Bn);
         }
+        if constexpr (W4)
+          if (steady || s + NS < s_hi) put(u, B, s + NS);
         mma(1);
       };
       fetch(0, A[0], B[0]);
       for (; s + 2 * NS <= s_hi; s += NS) {
 #pragma unroll
         for (int u = 0; u < NS; u++)
-          slab(A[u], B[u], A[(u + 1) % NS], B[(u + 1) % NS], s + u, true);
+          slab(A[u], B[u], A[(u + 1) % NS], B[(u + 1) % NS], s + u, u,
+               true);
       }
       for (; s < s_hi; s += NS) {
 #pragma unroll
         for (int u = 0; u < NS; u++)
           if (s + u < s_hi)
-            slab(A[u], B[u], A[(u + 1) % NS], B[(u + 1) % NS], s + u, false);
+            slab(A[u], B[u], A[(u + 1) % NS], B[(u + 1) % NS], s + u, u,
+                 false);
       }
     }
   }
@@ -397,60 +454,71 @@ k_gemm_prompt(GpArgs a) {
   }
 }
 
-template <bool F8, int BM, int BN, int WM, int WN, int NS>
+enum { GP_BF16, GP_E4M3, GP_MXFP4 };           // of W
+
+template <int T, int BM, int BN, int WM, int WN, int NS>
 static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
+  constexpr bool F8 = T == GP_E4M3, W4 = T == GP_MXFP4;
   const bool glu = a.act >= 0;
   const int wide = glu ? BN / 2 : BN;
   a.tm = (a.M + BM - 1) / BM;
   a.tn = (a.N + wide - 1) / wide;
   const dim3 grid((a.tm * a.tn + 7) / 8 * 8, sk);
   if (glu)
-    hipLaunchKernelGGL((k_gemm_prompt<F8, BM, BN, WM, WN, NS, true>), grid,
-                       dim3(64 * WM * WN), 0, s, a);
+    hipLaunchKernelGGL(
+        (k_gemm_prompt<F8, BM, BN, WM, WN, NS, true, false, W4>), grid,
+        dim3(64 * WM * WN), 0, s, a);
   else
-    hipLaunchKernelGGL((k_gemm_prompt<F8, BM, BN, WM, WN, NS, false>), grid,
-                       dim3(64 * WM * WN), 0, s, a);
+    hipLaunchKernelGGL(
+        (k_gemm_prompt<F8, BM, BN, WM, WN, NS, false, false, W4>), grid,
+        dim3(64 * WM * WN), 0, s, a);
   return hipGetLastError();
 }
 
 // Tile sizes, and microseconds that a slab takes on a CU that runs one block
-// of them or as many as fit, in bf16 and in e4m3, and those that a round costs
-// besides (first slabs, epilogue).  Large tiles ask L2 for the fewest bytes a
-// product: 128x128 by four waves wants 64 bytes a clock, all that a CU gets.
-// They win where there are rounds of them; where tiles are fewer than the chip
-// has CUs a smaller one that is deep in flight does.
-// The numbers are fitted to the times of every tile and split (1 to 8 parts)
-// for 324 products: 70 to 2048 rows of 27 shapes of both types (2048x2048 to
-// 18944x3584).  Chosen by them a product takes 0.9% more than with its best
-// tile and split on average; by bf16 slab times for both types and splits of
-// 1, 2, 4, 8 at what they cost while parts were flushed, 6.0% (70x3584x14336
-// e4m3 26.8 us, here 19.1; 907x2304x9216 102, 72; 611x3584x18944 160, 115).
+// of them or as many as fit, in bf16, e4m3 and MXFP4, and those that a round
+// costs besides (first slabs, epilogue); 0: not for that type.  Large tiles
+// ask L2 for the fewest bytes a product: 128x128 by four waves wants 64 bytes
+// a clock, all that a CU gets.  They win where there are rounds of them; where
+// tiles are fewer than the chip has CUs a smaller one that is deep in flight
+// does.  256x256 spills in e4m3 (fragments) and MXFP4 (W on its way to LDS:
+// 467 TFLOP/s at 2048x37888x3584, 128x128 944).
+// The numbers of bf16 and e4m3 are fitted to the times of every tile and split
+// (1 to 8 parts) for 324 products: 70 to 2048 rows of 27 shapes of both types
+// (2048x2048 to 18944x3584).  Chosen by them a product takes 0.9% more than
+// with its best tile and split on average; by bf16 slab times for both types
+// and splits of 1, 2, 4, 8 at what they cost while parts were flushed, 6.0%
+// (70x3584x14336 e4m3 26.8 us, here 19.1; 907x2304x9216 102, 72; 611x3584x18944
+// 160, 115).  Those of MXFP4 are fitted to 64, 130, 600 and 2048 rows of five
+// shapes.
 struct GpTile {
   int bm, bn, occ;
-  float one[2], full[2], round;
+  float one[3], full[3], round;
 };
 static const GpTile gp_tiles[] = {
-    // bf16 only (e4m3 fragments would spill), not split: its parts cost most
-    {256, 256, 1, {1.48f, 1.311f}, {1.48f, 1.311f}, 6.2f},
-    {128, 256, 1, {0.87f, 1.225f}, {0.87f, 1.225f}, 4.0f},
-    {128, 128, 2, {0.546f, 1.385f}, {1.032f, 2.773f}, 3.2f},
+    // not split: its parts cost most
+    {256, 256, 1, {1.48f, 0.f, 0.f}, {1.48f, 0.f, 0.f}, 6.2f},
+    {128, 256, 1, {0.87f, 1.225f, 0.96f}, {0.87f, 1.225f, 0.96f}, 4.0f},
+    {128, 128, 2, {0.546f, 1.385f, 0.654f}, {1.032f, 2.773f, 1.08f}, 3.2f},
     // eight waves, four buffers
-    {128, 128, 1, {0.494f, 0.718f}, {0.494f, 0.718f}, 3.4f},
-    {64, 128, 2, {0.652f, 0.758f}, {0.73f, 0.834f}, 1.8f},
-    {128, 64, 2, {0.734f, 0.881f}, {0.918f, 1.407f}, 1.6f},
-    {64, 64, 2, {0.261f, 0.472f}, {0.499f, 0.563f}, 1.4f},
-    {32, 64, 2, {0.231f, 0.286f}, {0.288f, 0.459f}, 1.8f},
+    {128, 128, 1, {0.494f, 0.718f, 0.562f}, {0.494f, 0.718f, 0.562f}, 3.4f},
+    {64, 128, 2, {0.652f, 0.758f, 0.44f}, {0.73f, 0.834f, 0.773f}, 1.8f},
+    {128, 64, 2, {0.734f, 0.881f, 0.f}, {0.918f, 1.407f, 0.f}, 1.6f},
+    {64, 64, 2, {0.261f, 0.472f, 0.292f}, {0.499f, 0.563f, 0.538f}, 1.4f},
+    {32, 64, 2, {0.231f, 0.286f, 0.f}, {0.288f, 0.459f, 0.f}, 1.8f},
 };
 
-template <bool F8>
+template <int T>
 static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
                          hipStream_t s) {
   const int width = a.act >= 0 ? 2 * a.N : a.N;
-  const int slabs = (int)(((long)a.K * (F8 ? 1 : 2) + 127) / 128);
+  const int slabs = (int)(((long)a.K * (T == GP_E4M3 ? 1 : 2) + 127) / 128);
   int best = -1, best_sk = 1;
   float best_t = 0.f;
-  for (int c = F8 ? 1 : 0; c < (int)(sizeof(gp_tiles) / sizeof(GpTile)); c++) {
+  for (int c = 0; c < (int)(sizeof(gp_tiles) / sizeof(GpTile)); c++) {
     const GpTile& g = gp_tiles[c];
+    const float one = g.one[T], full = g.full[T];
+    if (one == 0.f) continue;
     const long tiles = (long)((a.M + g.bm - 1) / g.bm) *
                        ((width + g.bn - 1) / g.bn);
     for (int sk = 1; sk <= 8; sk++) {
@@ -459,9 +527,10 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
                      parts > part_floats || slabs / sk < 4))
         break;
       // Full rounds and a rest.  A few CUs with two blocks set the time for
-      // all.
-      const float one = g.one[F8], full = g.full[F8];
-      const float x = (float)(tiles * sk) / 256.f;       // blocks of a CU
+      // all: blocks are counted on the XCD that has most, 32 CUs of it (three
+      // parts of 84 tiles are 252 blocks, but 33 on four of the XCDs:
+      // 130x3584x18944 MXFP4 80 us; in parts of four 68).
+      const float x = (float)((tiles + 7) / 8 * sk) / 32.f;   // of a CU
       const int rounds = (int)(x / g.occ);
       const float rest = x - rounds * g.occ;
       float t = rounds * full;
@@ -479,15 +548,22 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
   }
   switch (best) {
     case 0:
-      if constexpr (!F8) return gp_go<F8, 256, 256, 2, 4, 2>(a, best_sk, s);
+      if constexpr (T == GP_BF16)
+        return gp_go<T, 256, 256, 2, 4, 2>(a, best_sk, s);
       break;
-    case 1: return gp_go<F8, 128, 256, 2, 4, 3>(a, best_sk, s);
-    case 2: return gp_go<F8, 128, 128, 2, 2, 2>(a, best_sk, s);
-    case 3: return gp_go<F8, 128, 128, 2, 4, 4>(a, best_sk, s);
-    case 4: return gp_go<F8, 64, 128, 2, 2, 3>(a, best_sk, s);
-    case 5: return gp_go<F8, 128, 64, 2, 2, 3>(a, best_sk, s);
-    case 6: return gp_go<F8, 64, 64, 2, 2, 4>(a, best_sk, s);
-    case 7: return gp_go<F8, 32, 64, 2, 2, 6>(a, best_sk, s);
+    case 1: return gp_go<T, 128, 256, 2, 4, 3>(a, best_sk, s);
+    case 2: return gp_go<T, 128, 128, 2, 2, 2>(a, best_sk, s);
+    case 3: return gp_go<T, 128, 128, 2, 4, 4>(a, best_sk, s);
+    case 4: return gp_go<T, 64, 128, 2, 2, 3>(a, best_sk, s);
+    case 5:
+      if constexpr (T != GP_MXFP4)
+        return gp_go<T, 128, 64, 2, 2, 3>(a, best_sk, s);
+      break;
+    case 6: return gp_go<T, 64, 64, 2, 2, 4>(a, best_sk, s);
+    case 7:
+      if constexpr (T != GP_MXFP4)
+        return gp_go<T, 32, 64, 2, 2, 6>(a, best_sk, s);
+      break;
   }
   return hipErrorInvalidValue;
 }
@@ -501,16 +577,28 @@ extern "C" hipError_t launch_gemm_prompt(
     hipStream_t stream) {
   if (M < 1 || N < 1 || K < 64 || K % 64 || (!sx != !sw))
     return hipErrorInvalidValue;
-  GpArgs a = {x, w, (const float*)sx, (const float*)sw, (const u16*)res,
-              (const u16*)bias, (u16*)y, (float*)part, (int*)cnt, M, N, K,
-              act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
+  GpArgs a = {x, w, (const float*)sx, (const float*)sw, nullptr,
+              (const u16*)res, (const u16*)bias, (u16*)y, (float*)part,
+              (int*)cnt, M, N, K, act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
   if (!part || !cnt) part_floats = 0;
   if (mid_takes(sx, M, N, K, act >= 0))
     return launch_mid_gemm(x, w, sx, sw, res, bias, y, part, cnt, part_floats,
                            ncnt, M, N, K, K, res ? N : 0, N, act, 0, 0.f,
                            stream);
-  return sx ? gp_run<true>(a, part_floats, ncnt, stream)
-            : gp_run<false>(a, part_floats, ncnt, stream);
+  return sx ? gp_run<GP_E4M3>(a, part_floats, ncnt, stream)
+            : gp_run<GP_BF16>(a, part_floats, ncnt, stream);
+}
+
+// The same of bf16 rows and MXFP4 weights: w [N, K/2], we [N, K/32]
+extern "C" hipError_t launch_gemm_fp4w(
+    const void* x, const void* w, const void* we, const void* res,
+    const void* bias, void* y, void* part, void* cnt, long part_floats,
+    int ncnt, int M, int N, int K, int act, hipStream_t stream) {
+  if (M < 1 || N < 1 || K < 64 || K % 64 || !we) return hipErrorInvalidValue;
+  GpArgs a = {x, w, nullptr, nullptr, (const uint8_t*)we, (const u16*)res,
+              (const u16*)bias, (u16*)y, (float*)part, (int*)cnt, M, N, K,
+              act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
+  return gp_run<GP_MXFP4>(a, part && cnt ? part_floats : 0, ncnt, stream);
 }
 
 // ---- routed experts --------------------------------------------------------
@@ -638,8 +726,8 @@ extern "C" hipError_t launch_expert_gemm(
   const int bm = expert_bm(pairs, E), tiles = pairs / bm + E;
   const int* p = (const int*)sorted;
   GpArgs a = {x, w, (const float*)sx, (const float*)sw, nullptr, nullptr,
-              (u16*)y, nullptr, nullptr, pairs, N, K, act, tiles, 0, p,
-              p + pairs, p + pairs + tiles, p + pairs + 2 * tiles, top,
+              nullptr, (u16*)y, nullptr, nullptr, pairs, N, K, act, tiles, 0,
+              p, p + pairs, p + pairs + tiles, p + pairs + 2 * tiles, top,
               gather};
 #define EXPERTS(F8)                                                          \
   return bm == 128  ? gp_experts<F8, 128, 128, 2, 4, 4>(a, stream)           \

@@ -24,7 +24,7 @@ struct StackLayer {
 struct StackPlan {
   const StackLayer* layers;
   const void *embed, *cos, *sin;
-  void *h, *xn, *t1, *qkv, *att, *gate, *up, *acc, *row_cnt, *tile_cnt, *xq,
+  void *h, *xn, *t1, *qkv, *att, *gate, *acc, *row_cnt, *tile_cnt, *xq,
       *sx, *len, *moe_idx, *moe_w, *moe_order, *pairs, *aq, *sa;
   long acc_floats, order_room;
   int nlayers, H, I, nh, kvh, hd, S, wt, kv8, gemma, act, E, topk, nrow_cnt,
@@ -59,8 +59,6 @@ hipError_t launch_attn_prefill_mfma(
     void* part, long part_floats, int kv8, int M, int nh, int kvh, int hd,
     int ldq, int S, int keys, int most, int ntiles, float scale,
     float softcap, int window, hipStream_t);
-hipError_t launch_glu(const void* gate, const void* up, void* out, long total,
-                      int act, hipStream_t);
 hipError_t launch_gemm_prompt(
     const void* x, const void* w, const void* sx, const void* sw,
     const void* res, const void* bias, void* y, void* part, void* cnt,
@@ -73,11 +71,10 @@ hipError_t launch_row_gemm(
     float eps, float softcap, hipStream_t);
 hipError_t launch_quant_fp8(const void* X, void* Q, void* S, int f32, int M,
                             int K, hipStream_t);
-hipError_t launch_gemm_fp4w(const void* X, const void* W4, const void* WE,
-                            void* Y, const void* res, void* accbuf, int M,
-                            int N, int K, hipStream_t);
-hipError_t launch_bias_add(void* y, const void* bias, int M, int N,
-                           hipStream_t);
+hipError_t launch_gemm_fp4w(
+    const void* x, const void* w, const void* we, const void* res,
+    const void* bias, void* y, void* part, void* cnt, long part_floats,
+    int ncnt, int M, int N, int K, int act, hipStream_t);
 hipError_t launch_moe_route(const void* h, const void* g, const void* wg,
                             int M, int H, int E, int topk, float eps,
                             void* idx, void* wout, void* dense, hipStream_t);
@@ -110,20 +107,9 @@ hipError_t st_linear(const StackPlan& p, const StackLin& w, const void* x,
                      const void* res, const void* bias, int act,
                      hipStream_t s) {
   if (M > ST_FEW) {
-    if (p.wt == ST_FP4) {
-      auto one = [&](size_t row0, void* out) {
-        return launch_gemm_fp4w(
-            x, (const char*)w.w + row0 * (K / 2),
-            (const char*)w.e + row0 * (K / 32), out, res,
-            p.acc_floats >= (long)M * N ? p.acc : nullptr, M, N, K, s);
-      };
-      ST(one(0, y));
-      if (act >= 0) {
-        ST(one(N, p.up));
-        ST(launch_glu(y, p.up, y, (long)M * N, act, s));
-      }
-      return bias ? launch_bias_add(y, bias, M, N, s) : hipSuccess;
-    }
+    if (p.wt == ST_FP4)
+      return launch_gemm_fp4w(x, w.w, w.e, res, bias, y, p.acc, p.tile_cnt,
+                              p.acc_floats, p.ntile_cnt, M, N, K, act, s);
     const void* sx = nullptr;
     if (p.wt == ST_FP8) {
       ST(launch_quant_fp8(x, p.xq, p.sx, 0, M, K, s));

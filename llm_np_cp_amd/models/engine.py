@@ -333,8 +333,6 @@ class GPUModel(DecodeLoop):
         # act(gate) * up; of each of a row's experts
         pairs = R * (self.topk if self.moe else 1)
         self.b_gate = torch.zeros(pairs, I, **bf)
-        if self.wq4:          # its prompts have gate and up apart
-            self.b_up = torch.zeros(R, I, **bf)
         # fp32 parts of products that split K, and of attention that splits
         # its keys.  A few long rows beside many outputs can take more than a
         # short chunk of a prompt does.
@@ -470,7 +468,7 @@ class GPUModel(DecodeLoop):
                 else 0))
         own = {n: getattr(self, a, None) for n, a in dict(
             embed="embed", cos="cos_t", sin="sin_t", h="b_h", xn="b_xn",
-            t1="b_t1", qkv="b_rqkv", att="b_att", gate="b_gate", up="b_up",
+            t1="b_t1", qkv="b_rqkv", att="b_att", gate="b_gate",
             acc="b_gemm_acc", row_cnt="row_cnt", tile_cnt="tile_cnt",
             xq="b_xq", sx="b_sx", len="len_buf", moe_idx="moe_idx",
             moe_w="moe_w", moe_order="moe_order", pairs="b_pairs",
@@ -570,21 +568,13 @@ class GPUModel(DecodeLoop):
                        batch=batch)
             return
         res = res[:M] if res is not None else None
-        kw = dict(res=res, accbuf=self.b_gemm_acc)
+        kw = dict(res=res, accbuf=self.b_gemm_acc, bias=bias, act=act,
+                  cnt=self.tile_cnt)
         if self.wq4:
-            q, e = lw[name + "_q4"], lw[name + "_e4"]
-            if act >= 0:
-                assert res is None, "a gate beside MXFP4 adds nothing"
-                n = q.shape[0] // 2
-                ho.gemm_fp4w(x[:M], q[:n], e[:n], y[:M], **kw)
-                ho.gemm_fp4w(x[:M], q[n:], e[n:], self.b_up[:M], **kw)
-                ho.glu(y[:M], self.b_up[:M], y[:M], act)
-            else:
-                ho.gemm_fp4w(x[:M], q, e, y[:M], **kw)
-            if bias is not None:
-                ho.bias_add(y[:M], bias, M)
+            assert act < 0 or res is None, "a gate beside MXFP4 adds nothing"
+            ho.gemm_fp4w(x[:M], lw[name + "_q4"], lw[name + "_e4"], y[:M],
+                         **kw)
             return
-        kw.update(bias=bias, act=act, cnt=self.tile_cnt)
         if self.fp8:
             ho.quant_fp8(x[:M], self.b_xq, self.b_sx)
             ho.gemm_fp8(self.b_xq, self.b_sx, lw[name + "_q"],
@@ -611,7 +601,8 @@ class GPUModel(DecodeLoop):
         for a, b in ((0, M2), (M2, M)):
             if self.wq4:
                 ho.gemm_fp4w(x[a:b], lw[name + "_q4"], lw[name + "_e4"],
-                             y[a:b], accbuf=self.b_gemm_acc)
+                             y[a:b], accbuf=self.b_gemm_acc,
+                             cnt=self.tile_cnt)
             elif self.fp8:
                 ho.gemm_fp8(self.b_xq[a * K:], self.b_sx[a:],
                             lw[name + "_q"], lw[name + "_s"], y[a:b],
@@ -830,7 +821,8 @@ class GPUModel(DecodeLoop):
                    eps=self.config.rms_norm_eps)
         if self.wq4 and not batch:
             ho.gemm_fp4w(self.b_xn[:M], self.lm_head_q4, self.lm_head_e4,
-                         out[:M], accbuf=self.b_gemm_acc)
+                         out[:M], accbuf=self.b_gemm_acc,
+                         cnt=self.tile_cnt)
         elif self.fp8:
             ho.quant_fp8(self.b_xn[:M], self.b_xq, self.b_sx)
             ho.gemm_fp8(self.b_xq, self.b_sx, self.lm_head_q, self.lm_head_s,

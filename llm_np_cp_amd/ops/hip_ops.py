@@ -84,8 +84,8 @@ _SIGS = {
                           [ctypes.c_int] * 5 +
                           [ctypes.c_float, ctypes.c_int, ctypes.c_float,
                            ctypes.c_float, ctypes.c_void_p],
-    "launch_gemm_fp4w": [ctypes.c_void_p] * 6 + [ctypes.c_int] * 3 +
-                        [ctypes.c_void_p],
+    "launch_gemm_fp4w": [ctypes.c_void_p] * 8 + [ctypes.c_long] +
+                        [ctypes.c_int] * 5 + [ctypes.c_void_p],
     "launch_moe_route": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4 +
                         [ctypes.c_float] + [ctypes.c_void_p] * 4,
     "launch_expert_sort": [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2 +
@@ -569,18 +569,22 @@ def gemv_fp8_mx(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
 
 def gemm_fp4w(X: torch.Tensor, Wq4: torch.Tensor, We4: torch.Tensor,
               Y: torch.Tensor, res: torch.Tensor | None = None,
-              accbuf: torch.Tensor | None = None):
-    """Y[M,N] = X[M,K] @ dequant(W4)[N,K]^T (+res): bf16-MFMA prefill
+              accbuf: torch.Tensor | None = None,
+              bias: torch.Tensor | None = None, act: int = -1,
+              cnt: torch.Tensor | None = None):
+    """Y[M,N] = X[M,K] @ dequant(W4)[N,K]^T (+bias, +res): bf16-MFMA prefill
     over MXFP4 weights (single-copy fp4 engines; activations unquantized
-    -> more accurate than the fp8 prefill path)."""
+    -> more accurate than the fp8 prefill path).  act, accbuf and cnt as
+    gemm's."""
     M, K = X.shape
-    N = Wq4.shape[0]
+    N = Wq4.shape[0] // (2 if act >= 0 else 1)
     assert Wq4.shape[1] * 2 == K and K % 64 == 0
-    if accbuf is not None and accbuf.numel() < M * N:
-        accbuf = None
     _check(lib().launch_gemm_fp4w(
-        _ptr(X), _ptr(Wq4), _ptr(We4), _ptr(Y), _ptr(res), _ptr(accbuf),
-        M, N, K, _stream()), "gemm_fp4w")
+        _ptr(X), _ptr(Wq4), _ptr(We4), _ptr(res), _ptr(bias), _ptr(Y),
+        _ptr(accbuf), _ptr(cnt),
+        ctypes.c_long(0 if accbuf is None else accbuf.numel()),
+        0 if cnt is None else cnt.numel(), M, N, K, act, _stream()),
+        "gemm_fp4w")
 
 
 def prefetch(t: torch.Tensor, sink: torch.Tensor):
@@ -639,7 +643,7 @@ class _StackPlan(ctypes.Structure):
     _fields_ = [("layers", ctypes.POINTER(_StackLayer))] + \
         [(n, ctypes.c_void_p) for n in (
             "embed", "cos", "sin", "h", "xn", "t1", "qkv", "att", "gate",
-            "up", "acc", "row_cnt", "tile_cnt", "xq", "sx", "len", "moe_idx",
+            "acc", "row_cnt", "tile_cnt", "xq", "sx", "len", "moe_idx",
             "moe_w", "moe_order", "pairs", "aq", "sa")] + \
         [(n, ctypes.c_long) for n in ("acc_floats", "order_room")] + \
         [(n, ctypes.c_int) for n in (

@@ -271,6 +271,42 @@ def test_many_rows(M, N, K, kind, act):
     assert (Y[M] == 7.0).all() and not cnt.any()
 
 
+# the tiles that the device chooses among beside MXFP4 (64x64, 64x128, 128x128
+# of eight and of four waves, 128x256) with a rest both ways; fewer slabs of 64
+# than buffers, as many, one more; parts of K, also with a short last one
+@pytest.mark.parametrize("M,N,K", [
+    (17, 70, 64), (33, 200, 8192), (64, 64, 256), (130, 1000, 320),
+    (290, 900, 6144), (513, 4100, 256), (1030, 2050, 64), (1100, 2000, 4096),
+    (2050, 6200, 128), (2050, 6200, 192), (2049, 3700, 1024)])
+@pytest.mark.parametrize("act", [-1, 0, 1])
+def test_many_rows_beside_mxfp4(M, N, K, act):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    rows = N * (2 if act >= 0 else 1)
+    W = normal(rows, K, seed=11, scale=K ** -0.5)
+    X, bias, res = normal(M, K, seed=12), normal(N, seed=13), \
+        normal(M, N, seed=14)
+    q = torch.empty(rows, K // 2, dtype=torch.uint8, device="cuda")
+    e = torch.empty(rows, K // 32, dtype=torch.uint8, device="cuda")
+    ho.quant_fp4(W, q, e)
+    z = X.double() @ mxfp4_values(q, e).double().T
+    if act >= 0:
+        f = (torch.nn.functional.silu if act == 0 else lambda t:
+             torch.nn.functional.gelu(t, approximate="tanh"))
+        z = f(z[:, :N]) * z[:, N:]
+    part = torch.zeros(1 << 24, device="cuda")
+    cnt = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    Y = torch.full((M + 1, N), 7.0, device="cuda").bfloat16()
+    for kw, want in ((dict(), z), (dict(bias=bias, res=res, accbuf=part,
+                                        cnt=cnt),
+                                   z + bias.double() + res.double())):
+        for _ in range(2):                          # counters are left zero
+            ho.gemm_fp4w(X, q, e, Y[:M], act=act, **kw)
+        # exact products, fp32 sums, bf16 results: 2^-9 at most
+        assert off(Y[:M], want) < 2.0 ** -9
+        assert (Y[M] == 7.0).all() and not cnt.any()
+
+
 # histories of nothing, one key, a part of a tile, a block's range and one
 # key more, ranges of several tiles; heads that fill no group of four; a
 # window; head dims of both kernels
