@@ -1282,14 +1282,15 @@ class GPUModel(DecodeLoop):
         products have the rows of all: read one by one, 16 prompts of 305 to
         611 rows beside e4m3 weights left tiles half empty and W was streamed
         16 times (with 31 steps behind them 17.5 -> 13.4 ms; six of 167 to
-        333 in bf16 with 23 steps 10.1 -> 8.4).  The ones whose last chunk is
+        333 in bf16 with 23 steps 10.1 -> 8.4; prompts alone beside MXFP4,
+        eight layers of 3584: 16 of 305 to 611 rows 74 ms one by one in
+        products of their own, 27 so).  The ones whose last chunk is
         a single row beside e4m3 weights go alone, for that row is not
-        rounded to e4m3, and those beside MXFP4, whose few rows are gated in
-        fp32."""
-        apart = self.wq4 or self.hd not in (64, 128, 256)
+        rounded to e4m3."""
+        apart = self.hd not in (64, 128, 256)
         chunks, room = [], 0
         for b, n in enumerate(lens):
-            alone = apart or (self.fp8 and n % self.PC == 1)
+            alone = apart or (self.fp8 and not self.wq4 and n % self.PC == 1)
             done = 0
             while done < n:
                 if alone or room == 0:
