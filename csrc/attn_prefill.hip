@@ -414,8 +414,9 @@ __global__ void __launch_bounds__(256) k_attn_rows_merge(ApArgs a, int split) {
   float m = mz;
 #pragma unroll
   for (int w = 1; w < 64; w <<= 1) m = fmaxf(m, __shfl_xor(m, w));
-  // a part without keys of this row holds nothing
-  const float al = mz == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mz - m);
+  // a part without keys of this row holds nothing, one that weighs nothing
+  // may hold values without a number
+  const float al = mz == -INFINITY ? -1.f : __builtin_amdgcn_exp2f(mz - m);
   const float l = wave_reduce_sum(mz == -INFINITY ? 0.f : lz * al);
   float v[HD / 64];
 #pragma unroll
@@ -430,7 +431,7 @@ __global__ void __launch_bounds__(256) k_attn_rows_merge(ApArgs a, int split) {
 #pragma unroll
     for (int z = 0; z < 8; z++) {
       const float w = __shfl(al, min(z0 + z, 63));
-      if (z0 + z < split && w > 0.f)
+      if (z0 + z < split && !(w < 0.f))
 #pragma unroll
         for (int i = 0; i < HD / 64; i++) v[i] += x[z][i] * w;
     }

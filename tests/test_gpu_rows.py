@@ -65,6 +65,29 @@ def test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8):
     assert (out[M] == 7.0).all()
 
 
+# a part of the keys whose weight beside the others' underflows, with values
+# that are no number: as in one softmax, 0 times them is none either
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_prompt_attention_without_a_number(hd):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    M, pos0, nh, kvh = 5, 901, 4, 2
+    T = pos0 + M
+    q = torch.ones(M, nh, hd, device="cuda").bfloat16()
+    K, V = (normal(kvh, T, hd, seed=s) for s in (2, 3))
+    K[:, :128] = -40.0
+    V[:, 10, 3], V[:, 70, 5] = math.nan, math.inf
+    out = torch.empty(M, nh, hd, device="cuda").bfloat16()
+    ho.attn_prefill_mfma(
+        q, K, V, out, torch.tensor([pos0], dtype=torch.int32, device="cuda"),
+        M, nh, kvh, hd, hd ** -0.5,
+        part=torch.zeros(1 << 22, device="cuda"), keys=T)
+    bad = out.isnan()
+    assert bad[..., 3].all() and bad[..., 5].all()
+    bad[..., 3] = bad[..., 5] = False
+    assert not bad.any()
+
+
 def mxfp4_values(q, e):
     """MXFP4 bytes and exponents as 64-bit values."""
     grid = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0],
