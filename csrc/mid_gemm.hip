@@ -178,6 +178,8 @@ __global__ void __launch_bounds__(64 * MG_NW) k_mid_gemm(MgArgs a) {
     }
     mul(p, X0, i);
     if (i + 1 < n) mul(q, X1, i + 1);
+    // nothing is on its way into LDS when the block ends
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   f4v* const sums = (f4v*)X0;
 #pragma unroll
