@@ -991,18 +991,19 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs a) {
   });
 }
 
-// up to 16*MF rows: a tile of NB (16, or 8 to have more blocks) outputs per
-// block, K over NW waves, both operands straight from memory (the weights are
+// up to 16*MF rows: NB (8, 16 or 32) outputs per block, K over NW waves of U
+// slabs at a time, both operands straight from memory (the weights are
 // read once).  A load of W takes 8 rows x 128 bytes, whole lines, and an
 // exchange with lane ^ 8 makes operands of two of them (row_gemm.hip); in 16
 // rows x 64 bytes, and half of the lanes idle for eight outputs, 4 rows of
-// 32000x2048 took 28.6 us, now 24.3, 8192x2048 9.8 -> 8.9, 2048x8192 (in two
-// trips of loads, now one) 11.0 -> 9.6.
-template <typename T, int MF, int NW, int NB = 16>
+// 32000x2048 took 28.6 us, so 24.3, 8192x2048 9.8 -> 8.9, 2048x8192 (in two
+// trips of loads, so one) 11.0 -> 9.6.
+template <typename T, int MF, int NW, int NB = 16,
+          int U = MF == 1 ? 64 / NB : MF == 2 ? 4 : 2>
 __global__ void __launch_bounds__(64 * NW) k_gemm_skinny(GemmArgs a) {
-  __shared__ float red[NW * MF * 256];
   constexpr int R = NB / 8;                  // loads of a slab of W
-  constexpr int U = MF == 1 ? 8 / R : MF == 2 ? 4 : 2;
+  constexpr int TN = R > 1 ? R / 2 : 1;      // tiles of 16 outputs
+  __shared__ float red[NW * MF * TN * 256];
   const int tid = threadIdx.x, wave = wave_index(), lane = tid & 63;
   const int lr = lane & 15, gq = lane >> 4, z = blockIdx.z;
   const bool low = lr < 8;
@@ -1019,9 +1020,11 @@ __global__ void __launch_bounds__(64 * NW) k_gemm_skinny(GemmArgs a) {
   for (int i = 0; i < MF; i++)
     xr[i] = (const char*)((const T*)a.X + (size_t)z * a.xz +
                           (size_t)min(i * 16 + lr, a.M - 1) * a.ldx) + gq * 32;
-  f4v acc[MF];
+  f4v acc[MF][TN];
 #pragma unroll
-  for (int i = 0; i < MF; i++) acc[i] = {0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < MF; i++)
+#pragma unroll
+    for (int t = 0; t < TN; t++) acc[i][t] = {0.f, 0.f, 0.f, 0.f};
   auto turn = [](float v) {                  // the value of lane ^ 8
     return dpp_from<0x128>(v);
   };
@@ -1045,36 +1048,44 @@ __global__ void __launch_bounds__(64 * NW) k_gemm_skinny(GemmArgs a) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
       if (s + u * NW >= nsl) break;          // alike in a wave
-      f4v c[2];                              // row lr, chunks 2gq and 2gq + 1
 #pragma unroll
-      for (int d = 0; d < 4; d++) {
-        if constexpr (R == 1) {
-          c[0][d] = w[u][0][d];              // rows 8-15 are not there
-          c[1][d] = turn(w[u][0][d]);
-        } else {
-          const float got = turn(low ? w[u][1][d] : w[u][0][d]);
-          c[0][d] = low ? w[u][0][d] : got;
-          c[1][d] = low ? got : w[u][1][d];
+      for (int t = 0; t < TN; t++) {
+        f4v c[2];                            // row lr, chunks 2gq and 2gq + 1
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+          if constexpr (R == 1) {
+            c[0][d] = w[u][0][d];            // rows 8-15 are not there
+            c[1][d] = turn(w[u][0][d]);
+          } else {
+            const float w0 = w[u][2 * t][d], w1 = w[u][2 * t + 1][d];
+            const float got = turn(low ? w1 : w0);
+            c[0][d] = low ? w0 : got;
+            c[1][d] = low ? got : w1;
+          }
         }
+#pragma unroll
+        for (int i = 0; i < MF; i++)
+#pragma unroll
+          for (int q = 0; q < 2; q++)
+            acc[i][t] = GemmMma<T>::mma(xv[u][i][q], c[q], acc[i][t]);
       }
-#pragma unroll
-      for (int i = 0; i < MF; i++)
-#pragma unroll
-        for (int q = 0; q < 2; q++)
-          acc[i] = GemmMma<T>::mma(xv[u][i][q], c[q], acc[i]);
     }
   }
 #pragma unroll
   for (int i = 0; i < MF; i++)
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-      red[(wave * MF + i) * 256 + (gq * 4 + r) * 16 + lr] = acc[i][r];
+    for (int t = 0; t < TN; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        red[((wave * MF + i) * TN + t) * 256 + (gq * 4 + r) * 16 + lr] =
+            acc[i][t][r];
   __syncthreads();
-  for (int e = tid; e < MF * 256; e += 64 * NW) {
+  for (int e = tid; e < MF * TN * 256; e += 64 * NW) {
     float v = 0.f;
 #pragma unroll
-    for (int u = 0; u < NW; u++) v += red[u * MF * 256 + e];
-    const int row = e >> 4, col = (e & 15) < NB ? n0 + (e & 15) : a.N;
+    for (int u = 0; u < NW; u++) v += red[u * MF * TN * 256 + e];
+    const int row = (e >> 8) / TN * 16 + ((e >> 4) & 15);
+    const int c = (e >> 8) % TN * 16 + (e & 15), col = c < NB ? n0 + c : a.N;
     if (a.bias) v += a.bias[min(col, a.N - 1)];
     with_epilogue(a.epi, [&](auto epi) {
       gemm_store_rows<T, decltype(epi)::value, 1>(a, z, row, col, &v);
@@ -1370,13 +1381,42 @@ template <typename T>
 static void gemm_go(const GemmArgs& a, int Z, hipStream_t s) {
   long b128 = (long)((a.M + 127) / 128) * ((a.N + 127) / 128) * Z;
   dim3 sk((a.N + 15) / 16, 1, Z);
+  // Up to 16 rows, us for 4 and 16 of them, bf16, by eight waves and 16
+  // outputs a block -> here.  What a CU streams sets the time, so blocks are
+  // as narrow as it takes for every CU to have one, and as wide as fits where
+  // they are more than that: 32 outputs read X half as often.  Sixteen waves
+  // have two slabs each on the way and take the deeper K.
+  //   128 blocks of 16   2048x2048  5.1 -> 4.3, 6.1 -> 5.3
+  //   256                4096x2048  5.8 -> 5.5, 7.0 -> 6.4 (192: 3072x3072
+  //                      8 rows 7.5 -> 7.1; 160: 2560x2048 4 rows 5.1, 5.3)
+  //   512                5120x2048  8.4 -> 7.3, 10.4 -> 8.2; 8192x2048  9.0 ->
+  //                      8.1, 11.2 -> 8.9; 5120x8192  25 -> 22, 31 -> 25
+  //     from K 4096 on two trips of 32 outputs are as long as three of 16
+  //     (8192x4096 16 and 13), but where half of the CUs have a block
+  //   more               8192x8192 27 -> 24, 33 -> 32; 32000x2048  25.8 ->
+  //                      23.2, 33 -> 29 (more than eight rows: 32 outputs, by
+  //                      16 30.9; 10240x2048 15.0 and 13.4)
+  // One slab a wave gains nothing (9216x512 fp32 6.9, 7.3), nor does K
+  // beyond 8192 (5120x16384 51, 54 by 16 outputs).
+  const int slabs = (int)(a.K * sizeof(T) / 128);
+  const unsigned n = Z == 1 && slabs >= 16 ? sk.x : 0;
+#define SKINNY(NW, NB, ...)                                                  \
+  hipLaunchKernelGGL((k_gemm_skinny<T, 1, NW, NB, ##__VA_ARGS__>),           \
+                     dim3((a.N + NB - 1) / NB, 1, Z), dim3(64 * NW), 0, s, a)
   if (a.M <= 16 && sk.x * Z <= 128 && a.K >= 4096) {   // few blocks, deep K
-    hipLaunchKernelGGL((k_gemm_skinny<T, 1, 16, 8>), dim3((a.N + 7) / 8, 1, Z),
-                       dim3(1024), 0, s, a);
+    SKINNY(16, 8);
   } else if (a.M <= 16 && sk.x * Z <= 256 && a.K >= 4096) {
-    hipLaunchKernelGGL((k_gemm_skinny<T, 1, 16>), sk, dim3(1024), 0, s, a);
+    SKINNY(16, 16);
   } else if (a.M <= 16) {
-    hipLaunchKernelGGL((k_gemm_skinny<T, 1, 8>), sk, dim3(512), 0, s, a);
+    const bool deep = slabs >= 32 && slabs <= 128;
+    if (n >= 1 && n <= 128) SKINNY(8, 8, 4);
+    else if (n >= 192 && n <= 256 && deep) SKINNY(16, 16);
+    else if (n > 256 && (n <= 384 || (n <= 512 && slabs < 64) ||
+                         (n >= 1024 && deep && a.M > 8 && sizeof(T) == 2)))
+      SKINNY(16, 32, 2);
+    else if (n > 384 && deep) SKINNY(16, 16, 2);
+    else SKINNY(8, 16);
+#undef SKINNY
   } else if (a.M <= 32) {
     hipLaunchKernelGGL((k_gemm_skinny<T, 2, 8>), sk, dim3(512), 0, s, a);
   } else if (a.M <= 64) {

@@ -49,6 +49,54 @@ def test_tiles_of_row_products(hy, dtype, M, N, K):
     assert (Y[M] == 7.0).all()
 
 
+# blocks of 8, 16 and 32 outputs by 8 and 16 waves, with a rest of outputs and
+# of slabs: the first and last numbers of blocks of 16, and of slabs, of each
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("M", [2, 8, 9, 16])
+@pytest.mark.parametrize("N,slabs", [
+    (40, 16), (2044, 19), (2050, 16), (3058, 32), (4092, 33), (4100, 16),
+    (6140, 70), (6150, 16), (6150, 64), (8190, 63), (8200, 31), (8200, 32),
+    (8200, 129), (16372, 33), (16390, 32), (16390, 31)])
+def test_few_rows_by_blocks(hy, dtype, M, N, slabs):
+    K = slabs * (64 if dtype == "bf16" else 32)
+    K += K % 64                          # rows are padded to 64
+    X, W = draw(M, M, K, dtype=DT[dtype]), draw(N, N, K, dtype=DT[dtype])
+    b = draw(3, N, dtype=torch.float32)
+    Y = torch.full((M + 1, N), 7.0, device="cuda")
+    hy.gemm_rows(X, W, Y, M, K, N, hy.EPI_F32, bias=b)
+    want, far = product(X, W)
+    want = want + b.double()
+    assert ((Y[:M].double() - want).abs() <= far + want.abs() * 2.0 ** -23).all()
+    assert (Y[M] == 7.0).all()
+
+
+# pairs of columns that turn in each kind of block
+@pytest.mark.parametrize("N", [264, 2584, 4168, 8264])
+def test_few_rows_turned(hy, N):
+    M, K, RT, dims, split = 5, 2048, 8, 6, N - 64
+    X, W = (draw(k, n, K, dtype=DT["bf16"]) for k, n in ((1, M), (2, N)))
+    ang = torch.rand(40, dims // 2, device="cuda", dtype=torch.float64) * 6
+    pos = torch.arange(7, 7 + M, dtype=torch.int32, device="cuda")
+    cos, sin = torch.cos(ang).float(), torch.sin(ang).float()
+    Y = torch.full((M + 1, N), 7.0, device="cuda").bfloat16()
+    R = torch.full((M + 1, 8, 16), 7.0, device="cuda").bfloat16()
+    rot = hy.Rotary().put(pos=pos, cosT=cos, sinT=sin, y=R, split=split,
+                          RT=RT, dims=dims, ld=128, hs=16)
+    hy.gemm_rows(X, W, Y, M, K, N, hy.EPI_ROTARY, rotary=rot)
+    want, far = product(X, W)
+    t = want[:, split:].view(M, 8, RT).clone()
+    c, s = (f[pos.long(), None].double() for f in (cos, sin))
+    a, b = t[..., :dims:2].clone(), t[..., 1:dims:2].clone()
+    t[..., :dims:2], t[..., 1:dims:2] = a * c - b * s, b * c + a * s
+    # rounded to bf16 at the end; a turn adds up two products
+    for got, w, f in ((Y[:M, :split], want[:, :split], far[:, :split]),
+                      (R[:M, :, :RT], t, 2 * far[:, split:].view(M, 8, RT)
+                       .amax(-1, keepdim=True) + t.abs() * 2.0 ** -22)):
+        assert ((got.double() - w).abs() <= f + w.abs() * 2.0 ** -8).all()
+    assert (Y[:, split:] == 7.0).all() and (R[..., RT:] == 7.0).all()
+    assert (Y[M] == 7.0).all() and (R[M] == 7.0).all()
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize("M", [2, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(72, 64), (528, 512), (2056, 1088)])
