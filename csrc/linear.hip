@@ -71,8 +71,8 @@ __global__ void __launch_bounds__(256) k_last_tokens(PairEmbed a) {
 // A row of up to NT*U elements stays in the registers of NT threads.
 // X says whether there may be an xadd or a gate: none; some, asked for with x;
 // some, read when they are due (rows that are longer than the registers).
-// Their registers cost where there is none (2048 rows of 4096, norm alone:
-// 11.8 us, with them 15.1).
+// Their registers cost where there is none (2048 rows of 4096, norm alone, by
+// four waves a row: 11.8 us, with them 15.1).
 enum { ST_NONE, ST_AHEAD, ST_LATE };
 struct RowStage {
   const float* x;
@@ -392,12 +392,12 @@ k_group_rows(RowStage s, int groups, T* __restrict__ out) {
 
 // one block per row; `rows` (nullable) picks the source row of each output
 // row.  out rows have Kp elements; the padding is written as zero.
-template <typename T, int U, int X>
-__global__ void __launch_bounds__(256)
+template <typename T, int U, int X, int NT>
+__global__ void __launch_bounds__(NT)
 k_norm_rows(RowStage s, const int* __restrict__ rows, T* __restrict__ out) {
-  __shared__ float red[8];
+  __shared__ float red[NT / 32];
   T* o = out + (size_t)blockIdx.x * s.Kp;
-  stage_row<256, U, X>(s, rows ? rows[blockIdx.x] : blockIdx.x, true, red,
+  stage_row<NT, U, X>(s, rows ? rows[blockIdx.x] : blockIdx.x, true, red,
                [&](int i, float v) { o[i] = El<T>::st(v); });
 }
 
@@ -1186,19 +1186,28 @@ static bool bad_stage(const RowStage& s) {
 template <typename T>
 static void norm_rows(const RowStage& s, const void* rows, void* out, int M,
                       hipStream_t st) {
-#define NORM_ROWS(U, X)                                                      \
-  hipLaunchKernelGGL((k_norm_rows<T, U, X>), dim3(M), dim3(256), 0, st, s,   \
-                     (const int*)rows, (T*)out)
+#define NORM_ROWS(U, X, NT)                                                  \
+  hipLaunchKernelGGL((k_norm_rows<T, U, X, NT>), dim3(M), dim3(NT), 0, st,   \
+                     s, (const int*)rows, (T*)out)
+  // Eight waves a row: a thread has half as much to ask for and to add up.
+  // us by four and by eight, with the norm and addition ahead and with a
+  // gate: 4 rows of 2048 3.5 -> 3.1, 4.2 -> 3.1, of 4096 4.7 -> 3.8, 6.3 ->
+  // 4.2; 2048 of 4096 22.9 -> 21.8, 22.0 -> 17.1.  Many short rows fill the
+  // chip by four (600 of 2048 5.9 both, 2048 of 2048 10.6 and 11.6).
   const bool some = s.gate || s.xadd;
-  if (s.W <= 2048) {
-    if (some) NORM_ROWS(8, ST_AHEAD);
-    else NORM_ROWS(8, ST_NONE);
-  } else if (!some) {
-    NORM_ROWS(16, ST_NONE);
+  if (s.W <= 2048 && M <= 512) {
+    if (some) NORM_ROWS(4, ST_AHEAD, 512);
+    else NORM_ROWS(4, ST_NONE, 512);
+  } else if (s.W <= 2048) {
+    if (some) NORM_ROWS(8, ST_AHEAD, 256);
+    else NORM_ROWS(8, ST_NONE, 256);
   } else if (s.W <= 4096) {
-    NORM_ROWS(16, ST_AHEAD);
+    if (some) NORM_ROWS(8, ST_AHEAD, 512);
+    else NORM_ROWS(8, ST_NONE, 512);
+  } else if (!some) {
+    NORM_ROWS(16, ST_NONE, 256);
   } else {
-    NORM_ROWS(16, ST_LATE);
+    NORM_ROWS(16, ST_LATE, 256);
   }
 #undef NORM_ROWS
 }

@@ -145,6 +145,34 @@ def test_staged_rows(hy, dtype, W, form):
         assert ((xout.double() - v).abs() <= far * size).all()
 
 
+# the last number of short rows that eight waves take each, and the first that
+# four do
+@pytest.mark.parametrize("M", [512, 513])
+@pytest.mark.parametrize("W", [1030, 2048])
+@pytest.mark.parametrize("form", ["norm", "gate", "sum"])
+def test_many_staged_rows(hy, M, W, form):
+    Kp, eps = -(-W // 64) * 64, 1e-5
+    x, y, gate = (draw(i, M, W) for i in range(3))
+    g, gb = draw(3, W), draw(4, W)
+    out = torch.full((M + 1, Kp), 7.0, device="cuda")
+    v, size, kw = x.double(), x.double().abs(), {}
+    if form == "sum":
+        kw.update(y=y, gb=gb, xout=x)                 # in its place
+        t = y.double()
+        t = t / (t * t).mean(-1, keepdim=True).add(eps).sqrt() * gb.double()
+        v, size = v + t, size + t.abs()
+    by = g.double() / (v * v).mean(-1, keepdim=True).add(eps).sqrt()
+    if form == "gate":
+        kw.update(gate=gate, ldg=W)
+        by = by * torch.sigmoid(gate.double())
+    hy.norm_rows(x, g, out, M, W, Kp, eps, **kw)
+    far = 2.0 ** -18                    # as for few rows
+    assert ((out[:M, :W].double() - v * by).abs()
+            <= far * size * by.abs()).all()
+    assert (out[:M, W:] == 0).all() and (out[M] == 7.0).all()
+    assert ((x.double() - v).abs() <= far * size).all()
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 @pytest.mark.parametrize("T,bm", [
     (5, 32), (90, 32), (150, 64),
