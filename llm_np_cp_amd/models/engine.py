@@ -1284,20 +1284,25 @@ class GPUModel(DecodeLoop):
         16 times (with 31 steps behind them 17.5 -> 13.4 ms; six of 167 to
         333 in bf16 with 23 steps 10.1 -> 8.4; prompts alone beside MXFP4,
         eight layers of 3584: 16 of 305 to 611 rows 74 ms one by one in
-        products of their own, 27 so).  The ones whose last chunk is
-        a single row beside e4m3 weights go alone, for that row is not
-        rounded to e4m3."""
-        apart = self.hd not in (64, 128, 256)
+        products of their own, 27 so).  Beside e4m3 weights a row in a chunk
+        by itself is not rounded to e4m3, so which rows are must not depend on
+        a prompt's neighbours: the ones that end with such a row go alone, and
+        of the others none is left with one (the cut before it moves up)."""
+        e4m3 = self.fp8 and not self.wq4
+        apart = self.hd not in (64, 128, 256) or (e4m3 and self.PC < 3)
         chunks, room = [], 0
         for b, n in enumerate(lens):
-            alone = apart or (self.fp8 and not self.wq4 and n % self.PC == 1)
+            alone = apart or (e4m3 and n % self.PC == 1)
             done = 0
             while done < n:
                 if alone or room == 0:
                     chunks.append([])
                     room = self.PC
                 M = min(n - done, room)
-                chunks[-1].append((b, done, M))
+                if e4m3 and not alone and n - done - M == 1:
+                    M, room = M - 1, M - 1
+                if M:
+                    chunks[-1].append((b, done, M))
                 done += M
                 room = 0 if alone else room - M
         return chunks

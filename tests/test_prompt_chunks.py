@@ -36,6 +36,27 @@ def test_every_row_once_in_order(lens, kind):
             assert all(lens[b] % 64 != 1 for b, _, _ in c)
 
 
+# a row beside e4m3 weights is in a chunk by itself, and so not rounded, where
+# it is when its prompt is read alone, and nowhere else
+@pytest.mark.parametrize("PC", [1, 2, 3, 4, 5, 64])
+def test_a_row_by_itself_whatever_its_neighbours(PC):
+    rng = np.random.default_rng(PC)
+    lists = [[40, 25], [63, 2], [63, 3], [2, 63], [62, 2, 2], [64, 65, 66]]
+    lists += [rng.integers(1, 3 * PC + 4, size=rng.integers(1, 9)).tolist()
+              for _ in range(500)]
+    for lens in lists:
+        out, seen = chunks(lens, PC=PC, fp8=True), [0] * len(lens)
+        single = [c[0][:2] for c in out if sum(n for _, _, n in c) == 1]
+        for c in out:
+            assert 0 < sum(n for _, _, n in c) <= PC
+            for b, p, n in c:
+                assert n > 0 and p == seen[b]
+                seen[b] += n
+        assert seen == lens
+        assert single == [(b, p) for b, n in enumerate(lens)
+                          for p in range(0, n, PC) if n - p == 1 or PC == 1]
+
+
 @pytest.mark.parametrize("group", [1, 3, 7])
 @pytest.mark.parametrize("segs", [
     [(0, 0, 1)], [(3, 7, 4), (1, 0, 2)], [(0, 0, 200), (2, 900, 33)],
