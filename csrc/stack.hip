@@ -28,7 +28,7 @@ struct StackPlan {
       *sx, *len, *moe_idx, *moe_w, *moe_order, *pairs, *aq, *sa;
   long acc_floats, order_room;
   int nlayers, H, I, nh, kvh, hd, S, wt, kv8, gemma, act, E, topk, nrow_cnt,
-      ntile_cnt, mfma;
+      ntile_cnt, mfma, rows, pools;        // rows that fit, sequences
   float eps, scale, softcap, escale;
 };
 
@@ -181,7 +181,11 @@ extern "C" hipError_t stack_forward(const StackPlan* plan, int M, int keys,
                                     const void* rows, const void* tiles,
                                     int ntiles, int most, hipStream_t s) {
   const StackPlan& p = *plan;
-  if (M < 1 || first < 0 || last > p.nlayers || (ntiles && !p.mfma))
+  // a chunk of one sequence ends inside its cache, one of several brings the
+  // positions and pools of its rows
+  if (M < 1 || M > p.rows || keys > p.S || first < 0 || last > p.nlayers ||
+      (ntiles ? ntiles < 0 || !p.mfma || !rows || !tiles || most < 1 || most > M
+              : M > p.S || pool < 0 || pool >= p.pools))
     return hipErrorInvalidValue;
   const bool few = M <= ST_FEW;
   const int nq = p.nh * p.hd, nkv = p.kvh * p.hd, nqkv = nq + 2 * nkv;
@@ -259,13 +263,15 @@ k_embed_list(const u16* __restrict__ embed, StackIds ids,
   }
 }
 
-// ids: the tokens on the host, M <= 128, or list: on the device
+// ids: the tokens on the host, M <= 128, or list: on the device.  pos0 is a
+// position of the cache; where several sequences share the rows it is not used.
 extern "C" hipError_t stack_embed(const StackPlan* plan, const int* ids,
                                   const void* list, int M, int pos0,
                                   hipStream_t s) {
   const StackPlan& p = *plan;
   StackIds v = {};
-  if (M < 1 || !ids == !list || (ids && M > ST_IDS))
+  if (M < 1 || M > p.rows || pos0 < 0 || pos0 >= p.S || !ids == !list ||
+      (ids && M > ST_IDS))
     return hipErrorInvalidValue;
   for (int i = 0; ids && i < M; i++) v.v[i] = ids[i];
   hipLaunchKernelGGL(k_embed_list, dim3(M), dim3(256), 0, s,

@@ -482,7 +482,8 @@ class GPUModel(DecodeLoop):
             E=cfg.num_local_experts if self.moe else 0,
             topk=self.topk if self.moe else 0, nrow_cnt=self.row_cnt.numel(),
             ntile_cnt=self.tile_cnt.numel(),
-            mfma=int(self.hd in (64, 128, 256)), eps=cfg.rms_norm_eps,
+            mfma=int(self.hd in (64, 128, 256)), rows=self.b_h.shape[0],
+            pools=self.max_batch, eps=cfg.rms_norm_eps,
             scale=self.scale, softcap=self.attn_softcap,
             escale=cfg.embed_scale)
 

@@ -648,7 +648,8 @@ class _StackPlan(ctypes.Structure):
         [(n, ctypes.c_long) for n in ("acc_floats", "order_room")] + \
         [(n, ctypes.c_int) for n in (
             "nlayers", "H", "I", "nh", "kvh", "hd", "S", "wt", "kv8",
-            "gemma", "act", "E", "topk", "nrow_cnt", "ntile_cnt", "mfma")] + \
+            "gemma", "act", "E", "topk", "nrow_cnt", "ntile_cnt", "mfma",
+            "rows", "pools")] + \
         [(n, ctypes.c_float) for n in ("eps", "scale", "softcap", "escale")]
 
 
@@ -682,6 +683,7 @@ class Stack:
         host = isinstance(ids, np.ndarray)
         assert not host or (ids.dtype == np.int32 and len(ids) == M
                             and ids.flags.c_contiguous)
+        assert host or ids.numel() >= M
         _check(lib().stack_embed(
             self._at, ids.ctypes.data if host else None,
             None if host else ids.data_ptr(), M, pos0, _stream()),
@@ -691,6 +693,8 @@ class Stack:
                 last: int | None = None, rows=None, tiles=None, most: int = 0):
         """Rows [0, M) of h through layers [first, last); rows, tiles, most
         as for rope_cache and attn_prefill_mfma."""
+        assert tiles is None or (rows.numel() == 2 * M and
+                                 tiles.shape[-1] == 5)
         _check(lib().stack_forward(
             self._at, M, keys, pool, first,
             len(self._layers) if last is None else last, _ptr(rows),
