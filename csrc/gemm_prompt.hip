@@ -34,6 +34,8 @@
 //
 // With few tiles K is split over blocks; the last block of a tile to arrive
 // adds the parts in their order (the result does not depend on timing).
+#include <type_traits>
+
 #include "common.h"
 #include "mid_gemm.h"
 
@@ -85,6 +87,9 @@ k_gemm_prompt(GpArgs a) {
   constexpr int FM = BM / WM / 16, FN = BN / WN / 16;   // fragments of a wave
   constexpr int AI = BM / 8 / NW, BI = BN / 8 / NW;     // DMA of a wave
   static_assert(AI > 0 && BI > 0 && FM > 0 && FN % (GLU ? 2 : 1) == 0);
+  // The K of the largest tile is not split: the epilogue that adds
+  // parts would cost the former two spilled registers.
+  constexpr bool SPLIT = BM * BN < 256 * 256;
   // loads of a wave for a slab (MXFP4: a piece of W and its exponent)
   constexpr int PS = W4 ? AI + 2 : AI + BI;
   // An array a buffer, and the loop unrolled over them: the compiler sees
@@ -98,7 +103,7 @@ k_gemm_prompt(GpArgs a) {
 #undef GP_BUF
   char* const A[6] = {A0, A1, A2, A3, A4, A5};
   char* const B[6] = {B0, B1, B2, B3, B4, B5};
-  __shared__ int last_flag;
+  [[maybe_unused]] __shared__ int last_flag;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -129,30 +134,36 @@ k_gemm_prompt(GpArgs a) {
   const bool half = F8 && (rowb & 127) && s_hi == slabs;
 
   const int g_r = lane >> 3, g_s = lane & 7;
-  const char* pa[AI];
-  [[maybe_unused]] const char* pb[BI];
+  // Where a lane's rows lie behind the tile's first: 32 bits beside a base in
+  // scalar registers (an expert's rows of x are anywhere).  With 64-bit
+  // addresses the 256x256 tiles spill.
+  typedef typename std::conditional<MOE, size_t, uint32_t>::type Off;
+  const char* const x_at = (const char*)a.x + (MOE ? 0 : (size_t)bm * rowb);
+  const char* const w_at = (const char*)a.w + (w0 + bn) * rowb;
+  Off pa[AI];
+  [[maybe_unused]] uint32_t pb[BI];
 #pragma unroll
   for (int i = 0; i < AI; i++) {
-    const int r = (wave * AI + i) * 8 + g_r;
-    pa[i] = (const char*)a.x + (size_t)x_row(min(bm + r, rows - 1)) * rowb;
+    const int r = min(bm + (wave * AI + i) * 8 + g_r, rows - 1);
+    pa[i] = MOE ? (Off)x_row(r) * (Off)rowb : (Off)(r - bm) * (Off)rowb;
   }
-  auto w_row = [&](int r) {                  // of W, row r of the tile
-    if (!GLU) return (size_t)min(bn + r, a.N - 1);
-    const int n = min(bn + (r >> 5) * 16 + (r & 15), a.N - 1);
-    return ((r >> 4) & 1) ? (size_t)a.N + n : (size_t)n;
+  auto w_out = [&](int r) {                  // output of row r of the tile
+    return min(bn + (GLU ? (r >> 5) * 16 + (r & 15) : r), a.N - 1);
   };
   if constexpr (!W4)
 #pragma unroll
     for (int i = 0; i < BI; i++)
-      pb[i] = (const char*)a.w + (w0 + w_row((wave * BI + i) * 8 + g_r)) * rowb;
+      pb[i] = (uint32_t)(w_out((wave * BI + i) * 8 + g_r) - bn) *
+              (uint32_t)rowb;
   // MXFP4: a thread's piece of a slab, 32 or 16 values of a row
   constexpr int WB = W4 ? BN * 32 / (64 * NW) : 16, WT = 32 / WB;
   static_assert(WB == 16 || WB == 8);
   const int w_r = tid / WT, w_p = tid % WT;
   [[maybe_unused]] const uint8_t *p4 = nullptr, *pe = nullptr;
   if constexpr (W4) {
-    p4 = (const uint8_t*)a.w + w_row(w_r) * (a.K / 2) + w_p * WB;
-    pe = a.we + w_row(w_r) * (a.K / 32) + w_p * WB / 16;
+    const size_t row = (GLU && ((w_r >> 4) & 1) ? a.N : 0) + (size_t)w_out(w_r);
+    p4 = (const uint8_t*)a.w + row * (a.K / 2) + w_p * WB;
+    pe = a.we + row * (a.K / 32) + w_p * WB / 16;
   }
   [[maybe_unused]] uint32_t raw[NS][WB / 4], rexp[NS];
   auto ask = [&](int b, int s) {             // the piece of slab s
@@ -184,12 +195,12 @@ k_gemm_prompt(GpArgs a) {
   auto stage = [&](char* A, char* B, int s) {
     int o0 = src0, o1 = src1;
     if (F8 && half && s == slabs - 1) o0 &= 63, o1 &= 63;   // stay in the row
-    const size_t k0 = (size_t)s * 128 + o0, k1 = (size_t)s * 128 + o1;
+    const char* const xs = x_at + (size_t)s * 128;
 #pragma unroll
     for (int i = 0; i < AI; i++)
       __builtin_amdgcn_global_load_lds(
           (const __attribute__((address_space(1))) uint32_t*)(
-              pa[i] + (((wave * AI + i) & 1) ? k1 : k0)),
+              xs + (Off)(pa[i] + (((wave * AI + i) & 1) ? o1 : o0))),
           (__attribute__((address_space(3))) uint32_t*)(
               A + (wave * AI + i) * 1024), 16, 0, 0);
     if constexpr (W4) {
@@ -197,12 +208,16 @@ k_gemm_prompt(GpArgs a) {
       return;
     }
 #pragma unroll
-    for (int i = 0; i < BI; i++)
+    for (int i = 0; i < BI; i++) {
+      // 16 rows of the gate, 16 of what it gates
+      const char* const ws = w_at + (size_t)s * 128 +
+          (GLU && (((wave * BI + i) >> 1) & 1) ? (size_t)a.N * rowb : 0);
       __builtin_amdgcn_global_load_lds(
           (const __attribute__((address_space(1))) uint32_t*)(
-              pb[i] + (((wave * BI + i) & 1) ? k1 : k0)),
+              ws + (uint32_t)(pb[i] + (((wave * BI + i) & 1) ? o1 : o0))),
           (__attribute__((address_space(3))) uint32_t*)(
               B + (wave * BI + i) * 1024), 16, 0, 0);
+    }
   };
 
   f4v acc[FM][FN];
@@ -345,7 +360,7 @@ k_gemm_prompt(GpArgs a) {
     }
   }
 
-  if (SK > 1) {
+  if (SPLIT && SK > 1) {
     // fragments as they lie in registers: the last block reads them alike
     float* pp = a.part + (size_t)tile * SK * (BM * BN) + tid * 4;
 #pragma unroll
