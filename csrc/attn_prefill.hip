@@ -451,6 +451,56 @@ static void ap_go(const ApArgs& a, dim3 grid, hipStream_t s) {
                        dim3(64 * NW), 0, s, a);
 }
 
+// Into how many ranges the keys are split where blocks are too few for 256
+// CUs of two each (four of one wave).  A range more takes tiles off the
+// longest block, and writes and reads a part more of every row; blocks that
+// share a CU slow each other down.  The numbers are fitted to the times of
+// 3660 calls at up to 16 splits each (11 head layouts, both pools, 1 to 1400
+// rows behind 0 to 20000 keys, from memory): 1.1% above each call's best split
+// on average.  Four tiles a block at least, as it once was: 13.0%; one, where
+// blocks are at most 64: 6.9%, since many rows' parts cost more than they save.
+// us by four tiles, by one tile, here:
+//   head dim 128   5 rows of 24/8 heads over 905 keys  18.0 12.5 12.5
+//     120 of 28/4 over 1020                            20.5 24.6 19.5
+//     300 of 24/8 over 300                             14.2 20.0 14.2
+//   256  300 of 16/8 over 430                          27.2 34.2 27.2
+//   64   200 of 4/1 over 4200                          24.1 21.7 15.0
+template <int HD, int BKV>
+static int ap_split(const ApArgs& a, int kv8, int keys, long part_floats,
+                    int most, int nw, int blocks) {
+  const int want = nw == 1 ? 1024 : 512;
+  if (blocks * 2 > want || !a.part) return 1;
+  const int span = a.window > 0 && a.window + most < keys ? a.window + most
+                                                          : keys;
+  const int tiles = (span + BKV - 1) / BKV;
+  const long each = (long)a.kvh * a.M * (a.nh / a.kvh) * (HD + 4);
+  int cap = want / blocks < 64 ? want / blocks : 64;
+  if (cap > tiles) cap = tiles;
+  if (cap > part_floats / each) cap = (int)(part_floats / each);
+  // us of a tile, by one wave and by four, and how much longer with another
+  // block on the CU; of a part that is a block's, and of a MB of them
+  const float one = HD == 64 ? 0.77f : HD == 128 ? 1.41f : 1.31f;
+  const float four = HD == 64 ? 0.75f : HD == 128 ? 1.00f : 0.95f;
+  const float tile = (nw == 1 ? one : four) * (kv8 ? 1.70f : 1.f);
+  const float more = nw == 1 ? 0.40f : 0.15f;
+  const float mb = HD == 64 ? 0.50f : HD == 128 ? 0.30f : 0.215f;
+  const float part = 0.058f + mb * (float)each * 4e-6f;
+  int split = 1, last = 0;
+  float best = 0.f;
+  for (int s = 1; s == 1 || s <= cap; s++) {
+    const int per = (tiles + s - 1) / s;
+    if (per == last) continue;
+    last = per;
+    float t = per * tile * (1.f + more * ((blocks * s + 255) / 256 - 1));
+    if (s > 1) t += 2.16f + part * s;
+    if (s == 1 || t < best) {
+      best = t;
+      split = s;
+    }
+  }
+  return split;
+}
+
 // most: rows of the longest sequence; ntiles: of several sequences
 template <int HD, int BKV>
 static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
@@ -459,26 +509,8 @@ static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
   // up to 32 rows are one wave's; more share their tiles among four
   const int nw = most * (a.nh / a.kvh) <= 32 ? 1 : 4;
   const int tiles = a.tiles ? ntiles : (rows + nw * 32 - 1) / (nw * 32);
-  // Too few blocks for 256 CUs of two each: the keys are split too, down to
-  // four tiles a block, where blocks are very few to one (from four tiles on:
-  // a part costs the launch that adds them).  us, attention and sum, by four
-  // -> here: five rows of 24/8 heads of 128 over 906 keys 19.3 -> 13.6, over
-  // 6000 of 32/8 e4m3 heads 39.9 -> 23.1, seven of 8/4 of 256 over 900 25.0 ->
-  // 16.8, nine of 28/4 of 128 over 500 16.9 -> 13.0.
-  int split = 1;
-  const int want = nw == 1 ? 1024 : 512;
-  if (tiles * a.kvh * 2 <= want && a.part) {
-    split = want / (tiles * a.kvh);
-    const int span = a.window > 0 && a.window + most < keys ? a.window + most
-                                                            : keys;
-    const int one = span / BKV;
-    const int worth = tiles * a.kvh > 64 ? one / 4 : one < 4 ? 1 : one;
-    if (split > worth) split = worth;
-    if (split > 64) split = 64;
-    const long each = (long)a.kvh * rows * (HD + 4);
-    if (split > part_floats / each) split = (int)(part_floats / each);
-    if (split < 1) split = 1;
-  }
+  const int split = ap_split<HD, BKV>(a, kv8, keys, part_floats, most, nw,
+                                      tiles * a.kvh);
   a.fold = !a.tiles && split == 1 && tiles % 2 == 0 && tiles * a.kvh <= 512;
   dim3 grid(a.kvh, tiles, split);
   if (nw == 1) {

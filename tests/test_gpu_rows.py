@@ -28,12 +28,14 @@ def e4m3(x):
 
 
 # rows of a kv head: one short of, at and past 32 (one wave) and 128 (four);
-# keys: a partial tile, a window inside one, enough to be split
+# keys: a partial tile, a window inside one, enough to be split, into parts of
+# one tile and of some
 @pytest.mark.parametrize("hd,nh,kvh", [(64, 8, 2), (128, 3, 1), (256, 2, 2)])
 @pytest.mark.parametrize("M,pos0,window,cap", [
     (1, 0, 0, 0.0), (2, 63, 0, 50.0), (5, 901, 0, 0.0), (8, 700, 40, 0.0),
     (11, 2000, 0, 0.0), (32, 0, 7, 0.0), (33, 1, 0, 0.0), (43, 3, 0, 50.0),
-    (129, 64, 33, 0.0)])
+    (129, 64, 33, 0.0), (64, 2000, 0, 0.0), (90, 500, 300, 50.0),
+    (300, 100, 0, 0.0)])
 @pytest.mark.parametrize("kv8", [False, True])
 def test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8):
     from llm_np_cp_amd.ops import hip_ops as ho
