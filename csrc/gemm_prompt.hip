@@ -470,6 +470,7 @@ k_gemm_prompt(GpArgs a) {
 }
 
 enum { GP_BF16, GP_E4M3, GP_MXFP4 };           // of W
+#define GP_MAX_K (1 << 23)     // a tile's rows lie within 32 bits of its first
 
 template <int T, int BM, int BN, int WM, int WN, int NS>
 static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
@@ -490,44 +491,60 @@ static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Tile sizes, and microseconds that a slab takes on a CU that runs one block
-// of them or as many as fit, in bf16, e4m3 and MXFP4, and those that a round
-// costs besides (first slabs, epilogue); 0: not for that type.  Large tiles
-// ask L2 for the fewest bytes a product: 128x128 by four waves wants 64 bytes
-// a clock, all that a CU gets.  They win where there are rounds of them; where
-// tiles are fewer than the chip has CUs a smaller one that is deep in flight
-// does.  256x256 spills in e4m3 (fragments) and MXFP4 (W on its way to LDS:
-// 467 TFLOP/s at 2048x37888x3584, 128x128 944).
-// The numbers of bf16 and e4m3 are fitted to the times of every tile and split
-// (1 to 8 parts) for 324 products: 70 to 2048 rows of 27 shapes of both types
-// (2048x2048 to 18944x3584).  Chosen by them a product takes 0.9% more than
-// with its best tile and split on average; by bf16 slab times for both types
-// and splits of 1, 2, 4, 8 at what they cost while parts were flushed, 6.0%
-// (70x3584x14336 e4m3 26.8 us, here 19.1; 907x2304x9216 102, 72; 611x3584x18944
-// 160, 115).  Those of MXFP4 are fitted to 64, 130, 600 and 2048 rows of five
-// shapes.
+// Tile sizes, and by type (bf16, e4m3, MXFP4) what a slab costs a CU that
+// runs one block of them or as many as fit, and a round besides (first slabs,
+// epilogue); 0: not for that type.  Large tiles ask L2 for the fewest bytes a
+// product: 128x128 by four waves wants 64 bytes a clock, all that a CU gets.
+// They win where there are rounds of them; where tiles are fewer than the chip
+// has CUs a smaller one that is deep in flight does.  256x256 spills in e4m3
+// (fragments) and MXFP4 (W on its way to LDS: 467 TFLOP/s at 2048x37888x3584,
+// 128x128 944).
+// The numbers are about us, but fitted, with those of mid_time, to what they
+// choose: the times of every likely tile, split (1 to 8 parts) and of mid_gemm,
+// W from memory, for 17 to 2000 rows of 126 shapes, with and without a gate,
+// and for 14 numbers of rows each of 30 shapes of models.  By them a product
+// takes 1.4% (bf16) and 1.1% (e4m3) more than it does at best; fitted to the
+// latter 27 alone, with mid_gemm by limits of its own, 3.0% and 2.5%, and 69 and
+// 66 of 2268 products each took longer than by whole rounds and splits of 1, 2,
+// 4 and 8 (64x256x3584 15.3 us, at best 10.6; 128x9216x2048 e4m3 with a gate
+// 21.4, so 20.3).  Those of MXFP4 are fitted to 64, 130, 600 and 2048 rows of
+// five shapes (2.2%).
 struct GpTile {
   int bm, bn, occ;
-  float one[3], full[3], round;
+  float one[3], full[3], round[3];
 };
 static const GpTile gp_tiles[] = {
     // not split: its parts cost most
-    {256, 256, 1, {1.48f, 0.f, 0.f}, {1.48f, 0.f, 0.f}, 6.2f},
-    {128, 256, 1, {0.87f, 1.225f, 0.96f}, {0.87f, 1.225f, 0.96f}, 4.0f},
-    {128, 128, 2, {0.546f, 1.385f, 0.654f}, {1.032f, 2.773f, 1.08f}, 3.2f},
+    {256, 256, 1, {1.43f, 0.f, 0.f}, {1.43f, 0.f, 0.f}, {10.4f, 0.f, 0.f}},
+    {128, 256, 1, {0.821f, 1.25f, 0.96f}, {0.821f, 1.25f, 0.96f},
+     {6.88f, 3.34f, 4.0f}},
+    {128, 128, 2, {0.805f, 1.17f, 0.654f}, {1.07f, 2.82f, 1.08f},
+     {4.17f, 2.65f, 3.2f}},
     // eight waves, four buffers
-    {128, 128, 1, {0.494f, 0.718f, 0.562f}, {0.494f, 0.718f, 0.562f}, 3.4f},
-    {64, 128, 2, {0.652f, 0.758f, 0.44f}, {0.73f, 0.834f, 0.773f}, 1.8f},
-    {128, 64, 2, {0.734f, 0.881f, 0.f}, {0.918f, 1.407f, 0.f}, 1.6f},
-    {64, 64, 2, {0.261f, 0.472f, 0.292f}, {0.499f, 0.563f, 0.538f}, 1.4f},
-    {32, 64, 2, {0.231f, 0.286f, 0.f}, {0.288f, 0.459f, 0.f}, 1.8f},
+    {128, 128, 1, {0.524f, 0.763f, 0.562f}, {0.524f, 0.763f, 0.562f},
+     {4.58f, 1.94f, 3.4f}},
+    {64, 128, 2, {0.488f, 0.657f, 0.44f}, {0.857f, 0.911f, 0.773f},
+     {3.72f, 3.27f, 1.8f}},
+    {128, 64, 2, {0.516f, 1.25f, 0.f}, {3.88f, 3.47f, 0.f},
+     {1.91f, 1.9f, 0.f}},
+    {64, 64, 2, {0.283f, 0.425f, 0.292f}, {0.536f, 0.497f, 0.538f},
+     {1.74f, 1.33f, 1.4f}},
+    {32, 64, 2, {0.233f, 0.346f, 0.f}, {0.509f, 0.425f, 0.f},
+     {1.91f, 1.33f, 0.f}},
 };
+// A second block on some CUs, the first on few; K in parts, and each of their
+// floats.
+struct GpCost { float second, first, split, part; };
+static const GpCost gp_cost[3] = {{0.882f, 1.f, 1.02f, 5.32e-6f},
+                                  {1.f, 1.f, 1.12f, 4.14e-6f},
+                                  {0.42f, 0.96f, 2.1f, 5.0e-6f}};
 
 template <int T>
 static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
                          hipStream_t s) {
   const int width = a.act >= 0 ? 2 * a.N : a.N;
   const int slabs = (int)(((long)a.K * (T == GP_E4M3 ? 1 : 2) + 127) / 128);
+  const GpCost& k = gp_cost[T];
   int best = -1, best_sk = 1;
   float best_t = 0.f;
   for (int c = 0; c < (int)(sizeof(gp_tiles) / sizeof(GpTile)); c++) {
@@ -549,11 +566,13 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
       const int rounds = (int)(x / g.occ);
       const float rest = x - rounds * g.occ;
       float t = rounds * full;
-      if (rest > 1.f) t += one + (full - one) * (0.42f + 0.58f * (rest - 1.f));
-      else if (rest > 0.f) t += one * (0.96f + 0.04f * rest);
-      t = t * ((slabs + sk - 1) / sk) + (rounds + (rest > 0.f)) * g.round;
+      if (rest > 1.f)
+        t += one + (full - one) * (k.second + (1.f - k.second) * (rest - 1.f));
+      else if (rest > 0.f)
+        t += one * (k.first + (1.f - k.first) * rest);
+      t = t * ((slabs + sk - 1) / sk) + (rounds + (rest > 0.f)) * g.round[T];
       // parts written and read, and a trip for each
-      if (sk > 1) t += 2.1f + (float)(parts * 5.0e-6);
+      if (sk > 1) t += k.split + (float)(parts * k.part);
       if (best < 0 || t < best_t) {
         best = c;
         best_sk = sk;
@@ -561,6 +580,12 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
       }
     }
   }
+  if (T != GP_MXFP4 &&
+      mid_time(T == GP_E4M3, a.M, a.N, a.K, a.act >= 0, part_floats, ncnt) <
+          best_t)
+    return launch_mid_gemm(a.x, a.w, a.sx, a.sw, a.res, a.bias, a.y, a.part,
+                           a.cnt, part_floats, ncnt, a.M, a.N, a.K, a.K,
+                           a.res ? a.N : 0, a.N, a.act, 0, 0.f, s);
   switch (best) {
     case 0:
       if constexpr (T == GP_BF16)
@@ -590,16 +615,12 @@ extern "C" hipError_t launch_gemm_prompt(
     const void* res, const void* bias, void* y, void* part, void* cnt,
     long part_floats, int ncnt, int M, int N, int K, int act,
     hipStream_t stream) {
-  if (M < 1 || N < 1 || K < 64 || K % 64 || (!sx != !sw))
+  if (M < 1 || N < 1 || K < 64 || K % 64 || K > GP_MAX_K || (!sx != !sw))
     return hipErrorInvalidValue;
   GpArgs a = {x, w, (const float*)sx, (const float*)sw, nullptr,
               (const u16*)res, (const u16*)bias, (u16*)y, (float*)part,
               (int*)cnt, M, N, K, act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
   if (!part || !cnt) part_floats = 0;
-  if (mid_takes(sx, M, N, K, act >= 0))
-    return launch_mid_gemm(x, w, sx, sw, res, bias, y, part, cnt, part_floats,
-                           ncnt, M, N, K, K, res ? N : 0, N, act, 0, 0.f,
-                           stream);
   return sx ? gp_run<GP_E4M3>(a, part_floats, ncnt, stream)
             : gp_run<GP_BF16>(a, part_floats, ncnt, stream);
 }
@@ -609,7 +630,8 @@ extern "C" hipError_t launch_gemm_fp4w(
     const void* x, const void* w, const void* we, const void* res,
     const void* bias, void* y, void* part, void* cnt, long part_floats,
     int ncnt, int M, int N, int K, int act, hipStream_t stream) {
-  if (M < 1 || N < 1 || K < 64 || K % 64 || !we) return hipErrorInvalidValue;
+  if (M < 1 || N < 1 || K < 64 || K % 64 || K > GP_MAX_K || !we)
+    return hipErrorInvalidValue;
   GpArgs a = {x, w, nullptr, nullptr, (const uint8_t*)we, (const u16*)res,
               (const u16*)bias, (u16*)y, (float*)part, (int*)cnt, M, N, K,
               act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
@@ -736,7 +758,7 @@ extern "C" hipError_t launch_expert_gemm(
     const void* sorted, int pairs, int E, int top, int gather, int N, int K,
     int act, hipStream_t stream) {
   if (pairs < 1 || E < 1 || E > 64 || top < 1 || pairs % top || N < 1 ||
-      K < 64 || K % 64 || (!sx != !sw))
+      K < 64 || K % 64 || K > GP_MAX_K || (!sx != !sw))
     return hipErrorInvalidValue;
   const int bm = expert_bm(pairs, E), tiles = pairs / bm + E;
   const int* p = (const int*)sorted;

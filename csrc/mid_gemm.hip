@@ -20,6 +20,8 @@
 // lane l^8 makes operands of two of them: row l&15, 16-byte chunks 2(l>>4)
 // and 2(l>>4)+1.  X is read in that order.  W is the first operand, so a lane
 // ends with four neighbouring outputs of one row.
+#include <cmath>
+
 #include "common.h"
 #include "mid_gemm.h"
 
@@ -309,30 +311,58 @@ static MgPlan mg_plan(bool f8, int M, int N, int K, bool glu,
   return p;
 }
 
-// us, row_gemm (to 16 rows) or gemm_prompt (above) / here:
-//   bf16  2048x2048  5 rows 6.6/5.4, 17 9.4/6.1, 64 9.6/9.0
-//         4096x2304  5 8.7/6.7, 48 12.0/9.7; 3584x3584  17 17.0/9.5
-//         8192x3584  33 16.9/16.5, 64 19.1/19.7; 4608x3584  5 11.5/13.2
-//         3072x8192  5 12.9/14.0, 16 16.9/14.2, 48 19.6/19.2, 64 20.5/21.1
-//         3584x14336 16 35.9/22.1, 17 24.9/23.2, 32 25.8/26.5, 64 29.9/33.8
-//   e4m3  3072x2048  5 6.0/4.4, 37 8.1/5.5; 3584x3584  17 13.7/6.4
-//         3072x8192  5 9.0/9.7, 16 10.7/9.8, 64 25.2/13.8
-//         3584x18944 16 18.5/16.9, 64 27.5/25.4
-//   gate, bf16  8192x2048  17 18.6/14.3, 32 18.7/16.3; 8192x3072 32
-//         21.5/22.8; 14336x3584  5 36.5/40.2, 17 39.2/43.5
-//   wide  32768x3072  5 35.8/33.9 (21.4/22.2 in e4m3), 33 40.1/50.2
-// X is read once a block, so what has many blocks or many rows of X for a row
-// of W is better off with tiles.
-bool mid_takes(bool f8, int M, int N, int K, bool glu) {
-  if (glu) return M > 16 && M <= 32 && N <= 8192 && K <= 2048;
-  if (M <= 16) return N <= (f8 ? 8192 : 4096) && (K <= 4096 || M > 8);
-  if (M > 64 || N > 8192) return false;
-  if (f8) return true;
-  return M <= (K > 8192 ? 24 : K > 4096 || N > 4096 ? 48 : 64);
+// us, row_gemm / here, W from memory (15 widths by 11 lengths at 12 numbers of
+// rows each):
+//   rows of up to 4.5 KB  bf16 2048x2048 5 rows 7.5/6.7, 6144x2048 10.6/9.7;
+//     e4m3 2048x2048 7.5/5.6, 4608x4096 10.1/9.1.  More than 384 blocks of 16
+//     rows of W read X too often: bf16 10240x2048 12.2/14.3
+//   up to 8 KB  where row_gemm cannot share out few columns (bf16 1024x4096
+//     10.2/8.8) and where every CU has a block here (3584x3584 9.7/9.1, e4m3
+//     4096x8192 11.1/10.4); between them K in one stretch a block is too long
+//     (bf16 2048x3584 7.9/8.8) unless row_gemm has many rows to stage (16 of
+//     them 9.7/9.5), past them 32 rows of W a block are (4608x4096 12.0/14.1)
+//   longer  row_gemm stages more than eight rows in parts (bf16 2304x14336 5
+//     rows 16.9/17.0, 9 21.3/17.4); fewer than 1024 or more than 2560 columns
+//     are too few or too many blocks (4096x8192 9 rows 17.3/20.4)
+bool mid_takes(bool f8, int M, int N, int K) {
+  const long rowb = (long)K * (f8 ? 1 : 2);
+  const int blocks = (N + 15) / 16;
+  if (rowb <= 4608) return blocks <= 384;
+  if (rowb <= 8192)
+    return blocks <= 64 || (blocks <= 256 && (blocks > 160 || M > 12));
+  return M > 8 && blocks >= 64 && blocks <= 160;
 }
 
-// Y [M, N], M up to 64 (32 with a gate); sx, sw: row scales of e4m3 x and w.  act < 0: no
-// gate.  part and cnt (zero, left zero) let K be split.
+// What a round of slabs costs by the rows of W and X that a block has, what
+// more blocks than CUs do, and parts of K.  Fitted together with the numbers
+// of gemm_prompt's tiles, by what is chosen, so not by themselves us.
+// us, its best tile / here:
+//   bf16  2304x2048  17 rows 10.2/7.5, 64 11.7/10.3; 3584x3584 17 12.8/10.5,
+//         64 15.9/16.3; 3072x8192 24 17.4/17.1, 48 19.9/20.4; 3584x14336 17
+//         25.6/24.4, 32 26.2/27.7
+//   e4m3  4096x4096  17 12.1/8.0, 64 13.0/11.1; 3584x14336 17 18.8/16.4, 64
+//         22.5/22.4
+//   gate  4096x4096  17 19.2/15.0 (e4m3 14.4/10.9); 8192x3584 17 24.4/25.5
+//         (17.7/15.0)
+float mid_time(bool f8, int M, int N, int K, bool glu, long part_floats,
+               int ncnt) {
+  if (M > (glu ? 32 : 64)) return INFINITY;
+  static const struct {
+    float narrow, wide, rows, all, more, split, part;
+  } cost[2] = {{0.0852f, 0.725f, 0.229f, 1.44f, 1.32f, 0.45f, 0.247f},
+               {0.259f, 0.885f, 0.159f, 0.768f, 6.32f, 0.916f, 0.521f}};
+  const auto& c = cost[f8];
+  const MgPlan p = mg_plan(f8, M, N, K, glu, part_floats, ncnt);
+  const int mt = glu ? 2 : (M + 15) / 16, blocks = p.groups * p.ks;
+  float t = (p.nt == 1 ? c.narrow : c.wide) + c.rows * mt;
+  if (blocks > 256) t *= 1.f + c.more * (blocks / 256.f - 1.f);
+  t = c.all + t * ((p.per + MG_NW - 1) / MG_NW);
+  if (p.ks > 1) t += c.split + c.part * blocks * mt * p.nt * 1e-3f;
+  return t;
+}
+
+// Y [M, N], M up to 64 (32 with a gate); sx, sw: row scales of e4m3 x and w.
+// act < 0: no gate.  part and cnt (zero, left zero) let K be split.
 extern "C" hipError_t launch_mid_gemm(
     const void* x, const void* w, const void* sx, const void* sw,
     const void* res, const void* bias, void* y, void* part, void* cnt,
@@ -363,8 +393,7 @@ extern "C" hipError_t launch_mid_gemm(
     default: MG_GO(F8, 4, NT, GLU);                                          \
   }
 #define MG_KIND(F8)                                                          \
-  if (glu && M > 16) MG_GO(F8, 2, 2, true);                                  \
-  else if (glu) MG_GO(F8, 1, 2, true);                                       \
+  if (glu) MG_GO(F8, 2, 2, true);                                            \
   else if (p.nt == 2) MG_ROWS(F8, 2, false)                                  \
   else MG_ROWS(F8, 1, false)
   if (sx) { MG_KIND(true) } else { MG_KIND(false) }
