@@ -575,8 +575,10 @@ def gemm_fp4w(X: torch.Tensor, Wq4: torch.Tensor, We4: torch.Tensor,
     """Y[M,N] = X[M,K] @ dequant(W4)[N,K]^T (+bias, +res): bf16-MFMA prefill
     over MXFP4 weights (single-copy fp4 engines; activations unquantized
     -> more accurate than the fp8 prefill path).  act, accbuf and cnt as
-    gemm's."""
+    gemm's; accbuf alone brings counters of the call's own."""
     M, K = X.shape
+    if accbuf is not None and cnt is None:
+        cnt = torch.zeros(1024, dtype=torch.int32, device=X.device)
     N = Wq4.shape[0] // (2 if act >= 0 else 1)
     assert Wq4.shape[1] * 2 == K and K % 64 == 0
     _check(lib().launch_gemm_fp4w(

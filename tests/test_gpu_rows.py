@@ -839,3 +839,48 @@ def test_some_rows(f8, M, N, K, kind):
         assert f8 or (err <= far + round_ + 1e-30).all()
         assert (Y[M] == 7.0).all() and (Y[:, N:] == 7.0).all()
         assert not cnt.any()
+
+
+# e4m3 products by instructions of 32 and of 128 values of K: both cut their
+# products off at the same place, so one is as far from 64 bits as the other
+@pytest.mark.parametrize("M,K", [(2, 512), (9, 2048), (16, 8192)])
+@pytest.mark.parametrize("kind", ["normal", "outliers", "cubes", "positive"])
+def test_e4m3_sums_of_both_instructions(M, K, kind):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    N = 16384                        # row_gemm does not hand it on
+    X = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).cuda()
+    W = torch.randn(N, K, generator=torch.Generator().manual_seed(K)).cuda()
+    if kind == "outliers":
+        X[:, ::97] *= 30
+    elif kind == "cubes":
+        X, W = X ** 3, W ** 3
+    elif kind == "positive":
+        X, W = X.abs(), W.abs()
+    (x, sx, Xd), (w, ws, Wd) = e4m3(X), e4m3(W)
+    ref, far = Xd @ Wd.T, []
+    for f in (ho.row_gemm, ho.mid_gemm):
+        Y = torch.empty(M, N, device="cuda")
+        f(x, w, Y, M, ws=ws, sx=sx)
+        far.append(off(Y, ref))
+    assert far[0] < 2.0 ** -13           # 6e-5 seen, of cubes
+    assert far[1] <= far[0] * 1.01
+
+
+# counters are the caller's or the call's own
+def test_mxfp4_products_without_counters():
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    M, N, K = 33, 200, 8192
+    W, X = normal(N, K, seed=1, scale=K ** -0.5), normal(M, K, seed=2)
+    q = torch.empty(N, K // 2, dtype=torch.uint8, device="cuda")
+    e = torch.empty(N, K // 32, dtype=torch.uint8, device="cuda")
+    ho.quant_fp4(W, q, e)
+    part = torch.full((1 << 22,), float("nan"), device="cuda")
+    cnt = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    a, b = (torch.empty(M, N, device="cuda").bfloat16() for _ in "ab")
+    ho.gemm_fp4w(X, q, e, a, accbuf=part, cnt=cnt)
+    assert not part[0].isnan()                   # K is split
+    part.fill_(float("nan"))
+    ho.gemm_fp4w(X, q, e, b, accbuf=part)
+    assert not part[0].isnan() and torch.equal(a, b)
