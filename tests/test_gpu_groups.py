@@ -15,7 +15,7 @@ def _build():
 
 
 def engine(family="llama", hidden=4608, layers=2, heads=(4, 2), max_seq=64,
-           max_batch=4, **kw):
+           max_batch=4, more={}, **kw):
     import llm_np_cp_amd as L
     from llm_np_cp_amd.io.loader import random_weights
     from llm_np_cp_amd.models.engine import GPUModel
@@ -27,7 +27,7 @@ def engine(family="llama", hidden=4608, layers=2, heads=(4, 2), max_seq=64,
         head_dim=64,
         hidden_act="gelu_pytorch_tanh" if family == "gemma2" else "silu",
         attn_logit_softcapping=50.0 if family == "gemma2" else None,
-        final_logit_softcapping=30.0 if family == "gemma2" else None)
+        final_logit_softcapping=30.0 if family == "gemma2" else None, **more)
     return GPUModel(cfg, random_weights(cfg, seed=3), max_seq=max_seq,
                     max_batch=max_batch, **kw)
 
@@ -110,13 +110,21 @@ def test_chunks_shorter_than_the_group(dtype):
 
 
 # several prompts in a chunk, one over two chunks, single tokens: the same
-# logits as each prompt by itself
+# logits as each prompt by itself; a window that ends inside a prompt, norms
+# behind the branches, a bias, experts, an e4m3 cache
 @pytest.mark.parametrize("dtype", ["bf16", "fp8", "fp4"])
-def test_prompts_read_together(dtype):
+@pytest.mark.parametrize("family,kv,more", [
+    ("llama", "bf16", {}), ("llama", "fp8", {}),
+    ("gemma2", "bf16", dict(sliding_window=24)),
+    ("qwen2", "fp8", dict(attention_bias=True)),
+    ("mixtral", "bf16", dict(num_local_experts=4, num_experts_per_tok=2))])
+def test_prompts_read_together(family, kv, more, dtype):
+    if family == "mixtral" and dtype == "fp4":
+        pytest.skip("experts are bf16 or e4m3")
     rng = np.random.default_rng(0)
     prompts = [rng.integers(0, 256, size=n) for n in (5, 40, 1, 33, 65, 2)]
-    m = engine(hidden=128, max_batch=6, dtype=dtype, prefill_chunk=64,
-               max_seq=80)
+    m = engine(family, hidden=128, max_batch=6, dtype=dtype, kv_dtype=kv,
+               prefill_chunk=64, max_seq=80, more=more)
     m.prefill_batch(prompts)
     got = m.bt_logits32[:6].clone()
     for b, p in enumerate(prompts):

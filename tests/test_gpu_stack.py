@@ -74,3 +74,30 @@ def test_one_call_or_one_a_launch(kind):
         for a, b in zip(*got):
             assert torch.isfinite(a.float()).all()
             assert torch.equal(a, b), chunks
+
+
+# rows of both sequences in a chunk, the second going on behind another
+@pytest.mark.parametrize("kind", [k for k in KINDS if k.get("hd") != 80],
+                         ids=lambda k: "-".join(
+                             str(v) for v in k.values()) or "plain")
+@pytest.mark.parametrize("lens", [(3, 4), (40, 60)])
+def test_shared_chunk_by_one_call_or_one_a_launch(kind, lens):
+    m = engine(**kind)
+    rng = np.random.default_rng(sum(lens))
+    seqs = [rng.integers(0, 512, size=n).astype(np.int32) for n in lens]
+    got = []
+    for one in (True, False):
+        if not one:
+            m._layers_forward = m._layers_by_launch
+        for t in m.k_cache + m.v_cache:
+            t.zero_()
+        cut, h = lens[1] - 2, []
+        for segs in ([(1, 0, cut)], [(0, 0, lens[0]), (1, cut, 2)]):
+            m._read_pack(segs, seqs)
+            h.append(m.b_h[:sum(n for _, _, n in segs)].clone())
+        got.append(h + [m.bt_logits32.clone()] +
+                   [t[:, :, :max(lens)].clone()
+                    for t in m.k_cache + m.v_cache])
+    for a, b in zip(*got):
+        assert torch.isfinite(a.float()).all()
+        assert torch.equal(a, b)
