@@ -18,8 +18,9 @@
 //                               k_attn_rows / k_attn
 //  K2 cuBLAS GEMM/GEMV       -> k_gemv (decode), k_row_gemm (few rows),
 //                               k_gemm_prompt (prefill)
-//  K3 elementwise ufuncs     -> fused GEMV staging (NORM/GLU/NORM2),
-//                               k_rmsnorm, k_glu, k_softcap, k_addinto
+//  K3 elementwise ufuncs     -> fused GEMV staging (NORM/GLU/NORM2), epilogues
+//                               of products, k_rmsnorm, k_softcap, k_addinto,
+//                               k_glu
 //  K4 KV concat              -> in-place pool writes
 //  K5 repeat_kv              -> attention indexes kv_head = q_head/groups
 //  K7 torch.multinomial      -> k_logit_max + k_sample_pick (last-block commit)
@@ -864,7 +865,8 @@ extern "C" hipError_t launch_attn(const void* q, const void* kc,
 }
 
 // ====================================================================
-// GLU activations: out = act(gate) * up ; act 0 = SiLU, 1 = tanh-GELU
+// GLU activations: out = act(gate) * up ; act 0 = SiLU, 1 = tanh-GELU, for
+// halves that are there already (products take theirs as they store)
 // ====================================================================
 
 extern "C" __global__ void __launch_bounds__(256)
@@ -1334,35 +1336,6 @@ extern "C" hipError_t launch_softcap(void* y, long total, float cap,
   long blocks = (total / 8 + 255) / 256;
   hipLaunchKernelGGL(k_softcap, dim3((uint32_t)blocks), dim3(256), 0, stream,
                      (u16*)y, total, cap);
-  return hipGetLastError();
-}
-
-// ====================================================================
-// y[M,N] += bias[N] (bf16): Qwen-2 qkv-bias epilogue on the prefill /
-// batched GEMM path (the decode GEMV adds bias via its `res` slot).
-// ====================================================================
-
-extern "C" __global__ void __launch_bounds__(256)
-k_bias_add(u16* __restrict__ y, const u16* __restrict__ bias, long total,
-           int N) {
-  long i = ((long)blockIdx.x * 256 + threadIdx.x) * 8;
-  if (i >= total) return;
-  s8v yv = *(const s8v*)(y + i);
-  s8v bv = *(const s8v*)(bias + (i % N));
-  u16 o[8];
-#pragma unroll
-  for (int j = 0; j < 8; j++)
-    o[j] = f2b(b2f(((u16*)&yv)[j]) + b2f(((u16*)&bv)[j]));
-  *(s8v*)(y + i) = *(s8v*)o;
-}
-
-extern "C" hipError_t launch_bias_add(void* y, const void* bias, int M,
-                                      int N, hipStream_t stream) {
-  if (N % 8 != 0) return hipErrorInvalidValue;
-  long total = (long)M * N;
-  hipLaunchKernelGGL(k_bias_add, dim3((uint32_t)((total / 8 + 255) / 256)),
-                     dim3(256), 0, stream, (u16*)y, (const u16*)bias, total,
-                     N);
   return hipGetLastError();
 }
 

@@ -24,7 +24,7 @@ def fake(**kw):
         config=types.SimpleNamespace(rms_norm_eps=1e-5), fp8=False,
         wq4=False, b_gemm_acc=None, row_cnt=None, tile_cnt=None,
         b_xn=torch.zeros(32, 64), b_xq=torch.zeros(32 * 64),
-        b_sx=torch.zeros(32), b_up=torch.zeros(32, 64))
+        b_sx=torch.zeros(32))
     m.__dict__.update(kw)
     m._rows = types.MethodType(eng.GPUModel._rows, m)
     return m
