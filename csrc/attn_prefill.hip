@@ -456,10 +456,10 @@ static void ap_go(const ApArgs& a, dim3 grid, hipStream_t s) {
 // longest block, and writes and reads a part more of every row; blocks that
 // share a CU slow each other down.  The numbers are fitted to the times of
 // 3660 calls at up to 16 splits each (11 head layouts, both pools, 1 to 1400
-// rows behind 0 to 20000 keys, from memory): 1.1% above each call's best split
-// on average.  Four tiles a block at least, as it once was: 13.0%; one, where
-// blocks are at most 64: 6.9%, since many rows' parts cost more than they save.
-// us by four tiles, by one tile, here:
+// rows behind 0 to 20000 keys, from memory).  Above each call's best split, on
+// average where more rows than a tile make up to 64 blocks: 1.2% here, by four
+// tiles a block at least, as it once was, or by one, 8.2% and 8.4%, since many
+// rows' parts cost more than they save.  us by four tiles, by one tile, here:
 //   head dim 128   5 rows of 24/8 heads over 905 keys  18.0 12.5 12.5
 //     120 of 28/4 over 1020                            20.5 24.6 19.5
 //     300 of 24/8 over 300                             14.2 20.0 14.2
@@ -477,6 +477,16 @@ static int ap_split(const ApArgs& a, int kv8, int keys, long part_floats,
   int cap = want / blocks < 64 ? want / blocks : 64;
   if (cap > tiles) cap = tiles;
   if (cap > part_floats / each) cap = (int)(part_floats / each);
+  // Where neither was slower before, it stays: beside e4m3 rounding parts of
+  // other lengths are other values.  Few rows, a tile of them a kv head: a tile
+  // of keys a block from four on.  More blocks: four tiles at least.
+  if (blocks == a.kvh || blocks > 64) {
+    int s = span / BKV;
+    if (blocks > 64) s /= 4;
+    else if (s < 4) s = 1;
+    if (s > cap) s = cap;
+    return s < 1 ? 1 : s;
+  }
   // us of a tile, by one wave and by four, and how much longer with another
   // block on the CU; of a part that is a block's, and of a MB of them
   const float one = HD == 64 ? 0.77f : HD == 128 ? 1.41f : 1.31f;
