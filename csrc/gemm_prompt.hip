@@ -499,16 +499,17 @@ static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
 // has CUs a smaller one that is deep in flight does.  256x256 spills in e4m3
 // (fragments) and MXFP4 (W on its way to LDS: 467 TFLOP/s at 2048x37888x3584,
 // 128x128 944).
-// The numbers are about us, but fitted, with those of mid_time, to what they
-// choose: the times of every likely tile, split (1 to 8 parts) and of mid_gemm,
-// W from memory, for 17 to 2000 rows of 126 shapes, with and without a gate,
-// and for 14 numbers of rows each of 30 shapes of models.  By them a product
-// takes 1.4% (bf16) and 1.1% (e4m3) more than it does at best; fitted to the
-// latter 27 alone, with mid_gemm by limits of its own, 3.0% and 2.5%, and 69 and
-// 66 of 2268 products each took longer than by whole rounds and splits of 1, 2,
-// 4 and 8 (64x256x3584 15.3 us, at best 10.6; 128x9216x2048 e4m3 with a gate
-// 21.4, so 20.3).  Those of MXFP4 are fitted to 64, 130, 600 and 2048 rows of
-// five shapes (2.2%).
+// The numbers are about us, but fitted (bf16 with those of mid_time) to what
+// they choose: the times of every likely tile, split (1 to 8 parts) and of
+// mid_gemm, W from memory, for 17 to 2000 rows of 126 shapes, with and without
+// a gate, and for 14 numbers of rows each of 30 shapes of models.  By them a
+// product takes 1.4% (bf16) and 2.0% (e4m3) more than it does at best; fitted
+// to 27 of the latter alone 2.9% and 2.3%, and 94 and 78 of 2684 products each
+// took longer than by whole rounds and splits of 1, 2, 4 and 8, where 20 and 6
+// do so (64x256x3584 15.3 us, now 10.6; 128x6144x3584 e4m3 19.1, 16.6).  In
+// e4m3 that is mostly tiles of 32 rows where 64 are faster; K is split as it
+// was but for 3% of the products.  Those of MXFP4 are fitted to 64, 130, 600 and
+// 2048 rows of five shapes (2.2%).
 struct GpTile {
   int bm, bn, occ;
   float one[3], full[3], round[3];
@@ -516,27 +517,27 @@ struct GpTile {
 static const GpTile gp_tiles[] = {
     // not split: its parts cost most
     {256, 256, 1, {1.43f, 0.f, 0.f}, {1.43f, 0.f, 0.f}, {10.4f, 0.f, 0.f}},
-    {128, 256, 1, {0.821f, 1.25f, 0.96f}, {0.821f, 1.25f, 0.96f},
-     {6.88f, 3.34f, 4.0f}},
-    {128, 128, 2, {0.805f, 1.17f, 0.654f}, {1.07f, 2.82f, 1.08f},
-     {4.17f, 2.65f, 3.2f}},
+    {128, 256, 1, {0.821f, 1.02f, 0.96f}, {0.821f, 1.18f, 0.96f},
+     {6.88f, 5.07f, 4.0f}},
+    {128, 128, 2, {0.805f, 1.4f, 0.654f}, {1.07f, 3.03f, 1.08f},
+     {4.17f, 2.14f, 3.2f}},
     // eight waves, four buffers
-    {128, 128, 1, {0.524f, 0.763f, 0.562f}, {0.524f, 0.763f, 0.562f},
-     {4.58f, 1.94f, 3.4f}},
-    {64, 128, 2, {0.488f, 0.657f, 0.44f}, {0.857f, 0.911f, 0.773f},
-     {3.72f, 3.27f, 1.8f}},
-    {128, 64, 2, {0.516f, 1.25f, 0.f}, {3.88f, 3.47f, 0.f},
-     {1.91f, 1.9f, 0.f}},
-    {64, 64, 2, {0.283f, 0.425f, 0.292f}, {0.536f, 0.497f, 0.538f},
-     {1.74f, 1.33f, 1.4f}},
-    {32, 64, 2, {0.233f, 0.346f, 0.f}, {0.509f, 0.425f, 0.f},
-     {1.91f, 1.33f, 0.f}},
+    {128, 128, 1, {0.524f, 0.724f, 0.562f}, {0.524f, 0.724f, 0.562f},
+     {4.58f, 3.1f, 3.4f}},
+    {64, 128, 2, {0.488f, 0.687f, 0.44f}, {0.857f, 0.807f, 0.773f},
+     {3.72f, 3.02f, 1.8f}},
+    {128, 64, 2, {0.516f, 1.07f, 0.f}, {3.88f, 1.48f, 0.f},
+     {1.91f, 0.75f, 0.f}},
+    {64, 64, 2, {0.283f, 0.398f, 0.292f}, {0.536f, 0.563f, 0.538f},
+     {1.74f, 1.35f, 1.4f}},
+    {32, 64, 2, {0.233f, 0.274f, 0.f}, {0.509f, 0.474f, 0.f},
+     {1.91f, 1.55f, 0.f}},
 };
 // A second block on some CUs, the first on few; K in parts, and each of their
 // floats.
 struct GpCost { float second, first, split, part; };
 static const GpCost gp_cost[3] = {{0.882f, 1.f, 1.02f, 5.32e-6f},
-                                  {1.f, 1.f, 1.12f, 4.14e-6f},
+                                  {0.42f, 0.96f, 2.1f, 5.0e-6f},
                                   {0.42f, 0.96f, 2.1f, 5.0e-6f}};
 
 template <int T>

@@ -6,8 +6,8 @@
 // Whether it is faster than row_gemm, up to 16 rows without a gate.
 bool mid_takes(bool f8, int M, int N, int K);
 
-// How long it takes, to be compared with gemm_prompt's tiles; without end for
-// more rows than it takes.
+// How long it takes, to be compared with gemm_prompt's tiles: without end for
+// more rows than it takes, nothing where it is faster than any.
 float mid_time(bool f8, int M, int N, int K, bool glu, long part_floats,
                int ncnt);
 
