@@ -135,9 +135,10 @@ k_gemm_prompt(GpArgs a) {
 
   const int g_r = lane >> 3, g_s = lane & 7;
   // Where a lane's rows lie behind the tile's first: 32 bits beside a base in
-  // scalar registers (an expert's rows of x are anywhere).  With 64-bit
-  // addresses the 256x256 tiles spill.
-  typedef typename std::conditional<MOE, size_t, uint32_t>::type Off;
+  // scalar registers (an expert's rows of x are anywhere; beside MXFP4 weights
+  // a launch takes 0.35 us longer so).  With 64-bit addresses the 256x256 tiles
+  // spill.
+  typedef typename std::conditional<MOE || W4, size_t, uint32_t>::type Off;
   const char* const x_at = (const char*)a.x + (MOE ? 0 : (size_t)bm * rowb);
   const char* const w_at = (const char*)a.w + (w0 + bn) * rowb;
   Off pa[AI];
@@ -491,66 +492,75 @@ static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Tile sizes, and by type (bf16, e4m3, MXFP4) what a slab costs a CU that
-// runs one block of them or as many as fit, and a round besides (first slabs,
-// epilogue); 0: not for that type.  Large tiles ask L2 for the fewest bytes a
-// product: 128x128 by four waves wants 64 bytes a clock, all that a CU gets.
-// They win where there are rounds of them; where tiles are fewer than the chip
-// has CUs a smaller one that is deep in flight does.  256x256 spills in e4m3
-// (fragments) and MXFP4 (W on its way to LDS: 467 TFLOP/s at 2048x37888x3584,
-// 128x128 944).
-// The numbers are about us, but fitted (bf16 with those of mid_time) to what
-// they choose: the times of every likely tile, split (1 to 8 parts) and of
-// mid_gemm, W from memory, for 17 to 2000 rows of 126 shapes, with and without
-// a gate, and for 14 numbers of rows each of 30 shapes of models.  By them a
-// product takes 1.4% (bf16) and 2.0% (e4m3) more than it does at best; fitted
-// to 27 of the latter alone 2.9% and 2.3%, and 94 and 78 of 2684 products each
-// took longer than by whole rounds and splits of 1, 2, 4 and 8, where 20 and 6
-// do so (64x256x3584 15.3 us, now 10.6; 128x6144x3584 e4m3 19.1, 16.6).  In
-// e4m3 that is mostly tiles of 32 rows where 64 are faster; K is split as it
-// was but for 3% of the products.  Those of MXFP4 are fitted to 64, 130, 600 and
-// 2048 rows of five shapes (2.2%).
-struct GpTile {
-  int bm, bn, occ;
-  float one[3], full[3], round[3];
+// Large tiles ask L2 for the fewest bytes a product: 128x128 by four waves
+// wants 64 bytes a clock, all that a CU gets.  They win where there are rounds
+// of them; where tiles are fewer than the chip has CUs a smaller one that is
+// deep in flight does.  256x256 (never split: its parts cost most) spills in
+// e4m3 (fragments) and MXFP4 (W on its way to LDS: 467 TFLOP/s at
+// 2048x37888x3584, 128x128 944).  The second 128x128 has eight waves and four
+// buffers.
+struct GpTile { int bm, bn, occ; };              // occ: blocks that fit on a CU
+static const GpTile gp_tiles[8] = {
+    {256, 256, 1}, {128, 256, 1}, {128, 128, 2}, {128, 128, 1},
+    {64, 128, 2},  {128, 64, 2},  {64, 64, 2},   {32, 64, 2}};
+
+// What a slab of each tile costs a CU with one block and with as many as fit,
+// a round besides (first slabs, epilogue); the second block on some CUs, the
+// first on few; K in parts, and each of their floats.  0: not for that type.
+// The numbers are about us, but fitted to what they choose: the times of every
+// likely tile and split (1 to 8 parts), W from memory, for 17 to 2000 rows of
+// 126 shapes and for 14 numbers of rows each of 30 shapes of models, so that
+// few products take longer than by the numbers before, or than by whole rounds
+// and splits of 1, 2, 4 and 8.  Of 1804 products, and 880 with a gate, above
+// the best, and how many took 4% longer than by the latter, before -> now:
+//   bf16 2.8% -> 1.5%, 51 -> 13; with a gate 2.8% -> 1.9%, 50 -> 7
+//   e4m3 2.0% -> 1.4%, 51 -> 1; with a gate 2.9% -> 1.8%, 29 -> 1
+// (us: 64x256x3584 15.3 -> 10.6; 128x6144x3584 e4m3 19.1 -> 16.6; before, they
+// were fitted to 27 shapes of models, with and without gates alike).  Beside
+// e4m3 rounding sums in another order are other values: K is split as it was
+// but for 2% of the products.  MXFP4 is fitted to 64, 130, 600 and 2048 rows of
+// five shapes (2.2%).
+struct GpCost {
+  float one[8], full[8], round[8], second, first, split, part;
 };
-static const GpTile gp_tiles[] = {
-    // not split: its parts cost most
-    {256, 256, 1, {1.43f, 0.f, 0.f}, {1.43f, 0.f, 0.f}, {10.4f, 0.f, 0.f}},
-    {128, 256, 1, {0.821f, 1.02f, 0.96f}, {0.821f, 1.18f, 0.96f},
-     {6.88f, 5.07f, 4.0f}},
-    {128, 128, 2, {0.805f, 1.4f, 0.654f}, {1.07f, 3.03f, 1.08f},
-     {4.17f, 2.14f, 3.2f}},
-    // eight waves, four buffers
-    {128, 128, 1, {0.524f, 0.724f, 0.562f}, {0.524f, 0.724f, 0.562f},
-     {4.58f, 3.1f, 3.4f}},
-    {64, 128, 2, {0.488f, 0.687f, 0.44f}, {0.857f, 0.807f, 0.773f},
-     {3.72f, 3.02f, 1.8f}},
-    {128, 64, 2, {0.516f, 1.07f, 0.f}, {3.88f, 1.48f, 0.f},
-     {1.91f, 0.75f, 0.f}},
-    {64, 64, 2, {0.283f, 0.398f, 0.292f}, {0.536f, 0.563f, 0.538f},
-     {1.74f, 1.35f, 1.4f}},
-    {32, 64, 2, {0.233f, 0.274f, 0.f}, {0.509f, 0.474f, 0.f},
-     {1.91f, 1.55f, 0.f}},
-};
-// A second block on some CUs, the first on few; K in parts, and each of their
-// floats.
-struct GpCost { float second, first, split, part; };
-static const GpCost gp_cost[3] = {{0.882f, 1.f, 1.02f, 5.32e-6f},
-                                  {0.42f, 0.96f, 2.1f, 5.0e-6f},
-                                  {0.42f, 0.96f, 2.1f, 5.0e-6f}};
+static const GpCost gp_cost[5] = {
+    {// bf16
+     {1.29f, 0.87f, 0.62f, 0.483f, 1.24f, 0.485f, 0.261f, 0.251f},
+     {1.29f, 0.87f, 1.09f, 0.483f, 1.24f, 0.85f, 0.49f, 0.438f},
+     {7.85f, 4.92f, 2.87f, 3.78f, 2.01f, 1.53f, 1.33f, 0.787f},
+     0.7f, 1.f, 1.61f, 4.94e-6f},
+    {// bf16 with a gate
+     {1.46f, 0.87f, 0.592f, 0.5f, 0.854f, 0.481f, 0.261f, 0.234f},
+     {1.48f, 0.87f, 1.22f, 0.5f, 0.854f, 0.75f, 0.598f, 0.312f},
+     {4.86f, 3.2f, 2.75f, 3.37f, 2.56f, 2.98f, 1.09f, 1.56f},
+     0.616f, 0.96f, 2.1f, 4.79e-6f},
+    {// e4m3
+     {0.f, 1.1f, 2.04f, 0.752f, 0.633f, 0.892f, 0.405f, 0.286f},
+     {0.f, 1.43f, 4.27f, 0.752f, 0.817f, 0.892f, 0.556f, 0.449f},
+     {0.f, 3.81f, 3.68f, 2.16f, 2.07f, 2.84f, 1.14f, 1.21f},
+     0.626f, 0.952f, 0.273f, 5.43e-6f},
+    {// e4m3 with a gate
+     {0.f, 1.17f, 2.54f, 0.677f, 1.07f, 0.572f, 0.45f, 0.286f},
+     {0.f, 1.17f, 2.54f, 0.769f, 1.07f, 0.851f, 0.57f, 0.474f},
+     {0.f, 3.98f, 2.81f, 2.42f, 1.8f, 1.77f, 1.4f, 1.85f},
+     0.632f, 1.f, 0.778f, 4.63e-6f},
+    {// MXFP4
+     {0.f, 0.96f, 0.654f, 0.562f, 0.44f, 0.f, 0.292f, 0.f},
+     {0.f, 0.96f, 1.08f, 0.562f, 0.773f, 0.f, 0.538f, 0.f},
+     {0.f, 4.f, 3.2f, 3.4f, 1.8f, 0.f, 1.4f, 0.f},
+     0.42f, 0.96f, 2.1f, 5e-6f}};
 
 template <int T>
 static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
                          hipStream_t s) {
   const int width = a.act >= 0 ? 2 * a.N : a.N;
   const int slabs = (int)(((long)a.K * (T == GP_E4M3 ? 1 : 2) + 127) / 128);
-  const GpCost& k = gp_cost[T];
+  const GpCost& k = gp_cost[T == GP_MXFP4 ? 4 : T * 2 + (a.act >= 0)];
   int best = -1, best_sk = 1;
   float best_t = 0.f;
-  for (int c = 0; c < (int)(sizeof(gp_tiles) / sizeof(GpTile)); c++) {
+  for (int c = 0; c < 8; c++) {
     const GpTile& g = gp_tiles[c];
-    const float one = g.one[T], full = g.full[T];
+    const float one = k.one[c], full = k.full[c];
     if (one == 0.f) continue;
     const long tiles = (long)((a.M + g.bm - 1) / g.bm) *
                        ((width + g.bn - 1) / g.bn);
@@ -571,7 +581,7 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
         t += one + (full - one) * (k.second + (1.f - k.second) * (rest - 1.f));
       else if (rest > 0.f)
         t += one * (k.first + (1.f - k.first) * rest);
-      t = t * ((slabs + sk - 1) / sk) + (rounds + (rest > 0.f)) * g.round[T];
+      t = t * ((slabs + sk - 1) / sk) + (rounds + (rest > 0.f)) * k.round[c];
       // parts written and read, and a trip for each
       if (sk > 1) t += k.split + (float)(parts * k.part);
       if (best < 0 || t < best_t) {
@@ -581,12 +591,6 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
       }
     }
   }
-  if (T != GP_MXFP4 &&
-      mid_time(T == GP_E4M3, a.M, a.N, a.K, a.act >= 0, part_floats, ncnt) <
-          best_t)
-    return launch_mid_gemm(a.x, a.w, a.sx, a.sw, a.res, a.bias, a.y, a.part,
-                           a.cnt, part_floats, ncnt, a.M, a.N, a.K, a.K,
-                           a.res ? a.N : 0, a.N, a.act, 0, 0.f, s);
   switch (best) {
     case 0:
       if constexpr (T == GP_BF16)
@@ -622,6 +626,10 @@ extern "C" hipError_t launch_gemm_prompt(
               (const u16*)res, (const u16*)bias, (u16*)y, (float*)part,
               (int*)cnt, M, N, K, act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
   if (!part || !cnt) part_floats = 0;
+  if (mid_takes(sx, M, N, K, act >= 0))
+    return launch_mid_gemm(x, w, sx, sw, res, bias, y, part, cnt, part_floats,
+                           ncnt, M, N, K, K, res ? N : 0, N, act, 0, 0.f,
+                           stream);
   return sx ? gp_run<GP_E4M3>(a, part_floats, ncnt, stream)
             : gp_run<GP_BF16>(a, part_floats, ncnt, stream);
 }

@@ -3,13 +3,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-// Whether it is faster than row_gemm, up to 16 rows without a gate.
-bool mid_takes(bool f8, int M, int N, int K);
-
-// How long it takes, to be compared with gemm_prompt's tiles: without end for
-// more rows than it takes, nothing where it is faster than any.
-float mid_time(bool f8, int M, int N, int K, bool glu, long part_floats,
-               int ncnt);
+// Whether it is the faster one: gate, and M at most 16 beside row_gemm, more
+// beside gemm_prompt.
+bool mid_takes(bool f8, int M, int N, int K, bool glu);
 
 extern "C" hipError_t launch_mid_gemm(
     const void* x, const void* w, const void* sx, const void* sw,

@@ -20,8 +20,6 @@
 // lane l^8 makes operands of two of them: row l&15, 16-byte chunks 2(l>>4)
 // and 2(l>>4)+1.  X is read in that order.  W is the first operand, so a lane
 // ends with four neighbouring outputs of one row.
-#include <cmath>
-
 #include "common.h"
 #include "mid_gemm.h"
 
@@ -313,64 +311,53 @@ static MgPlan mg_plan(bool f8, int M, int N, int K, bool glu,
 
 // us, row_gemm / here, W from memory (15 widths by 11 lengths at 12 numbers of
 // rows each):
-//   bf16  rows of up to 4.5 KB  2048x2048 5 rows 7.5/6.7, 6144x2048 10.6/9.7;
-//       more than 384 blocks of 16 rows of W read X too often: 10240x2048
-//       12.2/14.3
-//     up to 8 KB  where row_gemm cannot share out few columns (1024x4096
-//       10.2/8.8) and where every CU has a block here (3584x3584 9.7/9.1);
-//       between them K in one stretch a block is too long (2048x3584 7.9/8.8)
-//       unless row_gemm has many rows to stage (16 of them 9.7/9.5), past them
-//       32 rows of W a block are (4608x4096 12.0/14.1)
-//     longer  row_gemm stages more than eight rows in parts (2304x14336 5 rows
-//       16.9/17.0, 9 21.3/17.4); fewer than 1024 or more than 2560 columns are
-//       too few or too many blocks (4096x8192 9 rows 17.3/20.4)
-//   e4m3  2048x2048 7.5/5.6, 8192x3584 8 rows 10.1/9.4; not
-//       8192x4096 (10.4/11.1) nor 4608x8192 9 rows (13.1/14.2); 2048x8192 5 rows
-//       8.7/9.1, 16 10.7/9.7
-bool mid_takes(bool f8, int M, int N, int K) {
-  const int blocks = (N + 15) / 16;
+//   bf16  up to 4096 columns: 2048x2048 5 rows 7.5/6.7, 3584x3584 9.7/9.1; where
+//       rows are 6 to 8 KB and blocks neither few, as row_gemm has it then
+//       (1024x4096 10.2/8.8), nor one for most CUs, K in one stretch a block is
+//       too long (2048x3584 7.9/8.8)
+//     longer rows  row_gemm stages more than eight rows of X in parts
+//       (2304x14336 5 rows 16.9/17.0, 9 21.3/17.4), but not beside few columns
+//       (9x512x14336 12.2/13.1); 16 KB apart they stand in each other's way
+//       here (9x4096x8192 17.3/20.4)
+//   e4m3  2048x2048 7.5/5.6, 8192x3584 8 rows 10.1/9.4; 2048x8192 5 rows
+//       8.7/9.1, 16 10.7/9.7; many rows not 4 and 8 KB apart (5x8192x4096
+//       10.4/11.1, 9x4608x8192 13.1/14.2)
+static bool mid_takes_few(bool f8, int M, int N, int K) {
+  if (N > (f8 ? 8192 : 4096) || (K > 4096 && M <= 8)) return false;
   if (f8)
-    return blocks <= (K >= 8192 ? 256 : K >= 4096 ? 384 : 512) &&
-           (K <= 4096 || M > 8);
-  if (K <= 2304) return blocks <= 384;
+    return N <= 4096 || (K % 8192 && (K % 4096 || N <= 6144) &&
+                         (K <= 16384 || N > 7168));
   if (K <= 4096)
-    return blocks <= 64 || (blocks <= 256 && (blocks > 160 || M > 12));
-  return M > 8 && blocks >= 64 && blocks <= 160;
+    return K <= 2304 || M > 12 || N <= 1024 || N > (K <= 3072 ? 2048 : 2560);
+  if (K > 8192 && N < 1024) return false;
+  return K % 8192 || N <= (M > 12 ? 3584 : 2560);
 }
 
-// bf16: what a round of slabs costs by the rows of W and X that a block has,
-// what more blocks than CUs do, and parts of K.  Fitted together with the
-// numbers of gemm_prompt's tiles, by what is chosen, so not by themselves us.
-// e4m3 by limits: next to e4m3 rounding, sums in another order are other
-// values (logits 0.05 apart after 16 layers), so the order is left as it is
-// where that costs nothing.
-// us, its best tile / here:
-//   bf16  2304x2048  17 rows 10.2/7.5, 64 11.7/10.3; 3584x3584 17 12.8/10.5,
-//         64 15.9/16.3; 3072x8192 24 17.4/17.1, 48 19.9/20.4; 3584x14336 17
-//         25.6/24.4, 32 26.2/27.7
-//   e4m3  4096x4096  17 12.1/8.0, 64 13.0/11.1; 3584x14336 17 18.8/16.4, 64
-//         22.5/22.4; 512x8192 64 12.1/15.5
-//   gate  bf16 4096x4096  17 19.2/15.0; 8192x3584 17 24.4/25.5; e4m3 8192x2048
-//         17 12.5/10.2, 6144x1024 32 8.5/9.7
-float mid_time(bool f8, int M, int N, int K, bool glu, long part_floats,
-               int ncnt) {
-  if (M > (glu ? 32 : 64)) return INFINITY;
-  if (f8) {
-    const bool yes = glu ? M > 16 && N <= 8192 && K <= 2048 &&
-                               (K > 1024 || N <= 4096)
-                     : M <= 16 ? mid_takes(f8, M, N, K)
-                               : N <= 8192 && (K < 8192 || N > 1024 || M < 48);
-    return yes ? 0.f : INFINITY;
-  }
-  const float narrow = 0.0852f, wide = 0.725f, rows = 0.229f, all = 1.44f,
-              more = 1.32f, split = 0.45f, part = 0.247f;
-  const MgPlan p = mg_plan(f8, M, N, K, glu, part_floats, ncnt);
-  const int mt = glu ? 2 : (M + 15) / 16, blocks = p.groups * p.ks;
-  float t = (p.nt == 1 ? narrow : wide) + rows * mt;
-  if (blocks > 256) t *= 1.f + more * (blocks / 256.f - 1.f);
-  t = all + t * ((p.per + MG_NW - 1) / MG_NW);
-  if (p.ks > 1) t += split + part * blocks * mt * p.nt * 1e-3f;
-  return t;
+// More rows and gates: us, the best tile / here, W from memory, 17 to 64 rows
+// of 126 shapes:
+//   bf16  rows of up to 4.5 KB  2304x2048 17 rows 10.2/7.5, 64 11.7/10.3;
+//       6144x2048 48 1.07 of the time here, 64 1.03
+//     up to 8 KB  17x3584x3584 12.8/10.5, 48 15.2/14.5; the more rows of X, the
+//       more columns it takes to be worth their way (48x1024x4096 0.85,
+//       48x3072x4096 1.04, 64x3072x4096 0.94 of the time here), and 4608 make
+//       144 blocks of 32, too few (33x4608x3584 0.96)
+//     longer  3072x8192 24 rows 17.4/17.1, 48 19.9/20.4; 3584x14336 17
+//       25.6/24.4, 32 26.2/27.7; 17x4608x14336 0.78
+//   e4m3  4096x4096 17 12.1/8.0, 64 13.0/11.1; 3584x14336 17 18.8/16.4, 64
+//       22.5/22.4; 512x8192 64 12.1/15.5
+//   gate  8192x2048 17 19.2/15.4, 32 19.2/17.1; 17x8192x3584 24.4/25.5; e4m3
+//       8192x2048 17 12.5/10.2, 6144x1024 32 8.5/9.7
+bool mid_takes(bool f8, int M, int N, int K, bool glu) {
+  if (glu)
+    return M > 16 && M <= 32 && N <= 8192 && K <= 2048 &&
+           !(f8 && K <= 1024 && N > 4096);
+  if (M <= 16) return mid_takes_few(f8, M, N, K);
+  if (M > 64 || N > 8192) return false;
+  if (f8) return K <= 7168 || K > 8192 || N > 1024 || M < 48;
+  if (K <= 2304) return N <= 4096 || M <= 48;
+  if (K > 8192) return M <= 24 && (N <= 4096 || N >= 7168);
+  if (M > 48 || (N > 4096 && N < 5120)) return false;
+  return K > 4096 || M <= 32 || N >= 48 * M;
 }
 
 // Y [M, N], M up to 64 (32 with a gate); sx, sw: row scales of e4m3 x and w.

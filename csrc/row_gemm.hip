@@ -589,7 +589,7 @@ extern "C" hipError_t launch_row_gemm(
               (float*)part, (int*)cnt, M, N, K, ldx, ldr, ldy, act, out_f32,
               0, 0, n16, eps, softcap};
   if (!part || !cnt) part_floats = 0;
-  if (!g && wt != RG_FP4 && act < 0 && mid_takes(wt == RG_FP8, M, N, K))
+  if (!g && wt != RG_FP4 && act < 0 && mid_takes(wt == RG_FP8, M, N, K, false))
     return launch_mid_gemm(x, w, wt == RG_FP8 ? sx : nullptr, ws, res, bias,
                            y, part, cnt, part_floats, ncnt, M, N, K, ldx, ldr,
                            ldy, act, out_f32, softcap, stream);
