@@ -457,7 +457,7 @@ static void ap_go(const ApArgs& a, dim3 grid, hipStream_t s) {
 // share a CU slow each other down.  The numbers are fitted to the times of
 // 3660 calls at up to 16 splits each (11 head layouts, both pools, 1 to 1400
 // rows behind 0 to 20000 keys, from memory).  Above each call's best split, on
-// average where more rows than a tile make up to 64 blocks: 1.2% here, by four
+// average where more rows than a tile make up to 64 blocks: 1.1% here, by four
 // tiles a block at least, as it once was, or by one, 8.2% and 8.4%, since many
 // rows' parts cost more than they save.  us by four tiles, by one tile, here:
 //   head dim 128   5 rows of 24/8 heads over 905 keys  18.0 12.5 12.5
@@ -489,12 +489,12 @@ static int ap_split(const ApArgs& a, int kv8, int keys, long part_floats,
   }
   // us of a tile, by one wave and by four, and how much longer with another
   // block on the CU; of a part that is a block's, and of a MB of them
-  const float one = HD == 64 ? 0.77f : HD == 128 ? 1.41f : 1.31f;
-  const float four = HD == 64 ? 0.75f : HD == 128 ? 1.00f : 0.95f;
-  const float tile = (nw == 1 ? one : four) * (kv8 ? 1.70f : 1.f);
-  const float more = nw == 1 ? 0.40f : 0.15f;
-  const float mb = HD == 64 ? 0.50f : HD == 128 ? 0.30f : 0.215f;
-  const float part = 0.058f + mb * (float)each * 4e-6f;
+  const float one = HD == 64 ? 0.76f : HD == 128 ? 2.58f : 1.73f;
+  const float four = HD == 64 ? 0.82f : HD == 128 ? 1.04f : 0.95f;
+  const float tile = (nw == 1 ? one : four) * (kv8 ? 1.78f : 1.f);
+  const float more = nw == 1 ? 0.40f : 0.20f;
+  const float mb = HD == 64 ? 0.50f : HD == 128 ? 0.30f : 0.20f;
+  const float part = 0.042f + mb * (float)each * 4e-6f;
   int split = 1, last = 0;
   float best = 0.f;
   for (int s = 1; s == 1 || s <= cap; s++) {
@@ -502,7 +502,7 @@ static int ap_split(const ApArgs& a, int kv8, int keys, long part_floats,
     if (per == last) continue;
     last = per;
     float t = per * tile * (1.f + more * ((blocks * s + 255) / 256 - 1));
-    if (s > 1) t += 2.16f + part * s;
+    if (s > 1) t += 2.43f + part * s;
     if (s == 1 || t < best) {
       best = t;
       split = s;
