@@ -1400,17 +1400,17 @@ static void gemm_go(const GemmArgs& a, int Z, hipStream_t s) {
   //                      8 rows 7.5 -> 7.1; 160: 2560x2048 4 rows 5.1, 5.3)
   //   512                5120x2048  8.4 -> 7.3, 10.4 -> 8.2; 8192x2048  9.0 ->
   //                      8.1, 11.2 -> 8.9; 5120x8192  25 -> 22, 31 -> 25
-  //     from rows of 8 KB on up to 384, and up to eight rows of X beside rows
-  //     of 8 to 12 KB up to 320: there sixteen waves take 16 outputs each
+  //     from rows of 8 KB on up to 384, and up to six rows of X beside rows of
+  //     8 to 12 KB up to 320: there sixteen waves take 16 outputs each
   //     (6144x4096 2 rows 13.0, by 32 outputs 14.8, so 12.8; fp32 6144x2048
   //     14.1, 16.2, 13.5; 8192x4096 16 and 13)
   //   more               8192x8192 27 -> 24, 33 -> 32; 32000x2048  25.8 ->
-  //                      23.2, 33 -> 29 (more than eight rows, rows of W of
-  //                      less than 8 KB: 32 outputs, by 16 30.9; 10240x2048
-  //                      15.0 and 13.4; but 16384x4096 9 rows by eight waves
-  //                      27.6, by 32 outputs 33.7, by 16 26.8).  fp32 rows of
-  //                      less than 8 KB stay by eight waves (24576x1536 2 rows
-  //                      25.5, by sixteen 26.6)
+  //                      23.2, 33 -> 29 (more than eight rows: 32 outputs, by
+  //                      16 30.9; 10240x2048 15.0 and 13.4; not beside rows of
+  //                      8 KB, which stand in each other's way: 16384x4096 9
+  //                      rows by eight waves 27.6, by 32 outputs 33.7, by 16
+  //                      26.8).  fp32 rows of 6 to 8 KB stay by eight waves
+  //                      (24576x1536 2 rows 25.5, by sixteen 26.6)
   // One slab a wave gains nothing (9216x512 fp32 6.9, 7.3), nor does K
   // beyond 8192 (5120x16384 51, 54 by 16 outputs).
   const int slabs = (int)(a.K * sizeof(T) / 128);
@@ -1427,11 +1427,12 @@ static void gemm_go(const GemmArgs& a, int Z, hipStream_t s) {
     if (n >= 1 && n <= 128) SKINNY(8, 8, 4);
     else if (n >= 192 && n <= 256 && deep) SKINNY(16, 16);
     else if (n > 256 && n <= (slabs < 64 ? 512 : 384) &&
-             !(n >= 320 && slabs >= 64 && slabs < 96 && a.M <= 8))
+             !(n >= 320 && slabs >= 64 && slabs < 96 && a.M <= 6))
       SKINNY(16, 32, 2);
-    else if (n >= 1024 && deep && slabs < 64 && a.M > 8 && sizeof(T) == 2)
+    else if (n >= 1024 && deep && slabs != 64 && a.M > 8 && sizeof(T) == 2)
       SKINNY(16, 32, 2);
-    else if (n > 256 && deep && (sizeof(T) == 2 || slabs >= 64))
+    else if (n > 256 && deep &&
+             (sizeof(T) == 2 || slabs < 48 || slabs >= 64))
       SKINNY(16, 16, 2);
     else SKINNY(8, 16);
 #undef SKINNY
