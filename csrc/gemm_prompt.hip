@@ -80,7 +80,7 @@ template <int N> DEVINL void gp_meet() {
 }
 
 template <bool F8, int BM, int BN, int WM, int WN, int NS, bool GLU,
-          bool MOE = false, bool W4 = false>
+          bool MOE = false, bool W4 = false, bool FAR = false>
 __global__ void __launch_bounds__(64 * WM * WN)
 k_gemm_prompt(GpArgs a) {
   constexpr int NW = WM * WN;
@@ -137,12 +137,13 @@ k_gemm_prompt(GpArgs a) {
   // Where a lane's rows lie behind the tile's first: 32 bits beside a base in
   // scalar registers (an expert's rows of x are anywhere; beside MXFP4 weights
   // a launch takes 0.35 us longer so).  With 64-bit addresses the 256x256 tiles
-  // spill.
-  typedef typename std::conditional<MOE || W4, size_t, uint32_t>::type Off;
+  // spill.  FAR: rows so long that 32 bits are not enough.
+  typedef typename std::conditional<MOE || W4 || FAR, size_t, uint32_t>::type
+      Off;
   const char* const x_at = (const char*)a.x + (MOE ? 0 : (size_t)bm * rowb);
   const char* const w_at = (const char*)a.w + (w0 + bn) * rowb;
   Off pa[AI];
-  [[maybe_unused]] uint32_t pb[BI];
+  [[maybe_unused]] Off pb[BI];
 #pragma unroll
   for (int i = 0; i < AI; i++) {
     const int r = min(bm + (wave * AI + i) * 8 + g_r, rows - 1);
@@ -154,8 +155,7 @@ k_gemm_prompt(GpArgs a) {
   if constexpr (!W4)
 #pragma unroll
     for (int i = 0; i < BI; i++)
-      pb[i] = (uint32_t)(w_out((wave * BI + i) * 8 + g_r) - bn) *
-              (uint32_t)rowb;
+      pb[i] = (Off)(w_out((wave * BI + i) * 8 + g_r) - bn) * (Off)rowb;
   // MXFP4: a thread's piece of a slab, 32 or 16 values of a row
   constexpr int WB = W4 ? BN * 32 / (64 * NW) : 16, WT = 32 / WB;
   static_assert(WB == 16 || WB == 8);
@@ -215,7 +215,7 @@ k_gemm_prompt(GpArgs a) {
           (GLU && (((wave * BI + i) >> 1) & 1) ? (size_t)a.N * rowb : 0);
       __builtin_amdgcn_global_load_lds(
           (const __attribute__((address_space(1))) uint32_t*)(
-              ws + (uint32_t)(pb[i] + (((wave * BI + i) & 1) ? o1 : o0))),
+              ws + (Off)(pb[i] + (((wave * BI + i) & 1) ? o1 : o0))),
           (__attribute__((address_space(3))) uint32_t*)(
               B + (wave * BI + i) * 1024), 16, 0, 0);
     }
@@ -471,9 +471,9 @@ k_gemm_prompt(GpArgs a) {
 }
 
 enum { GP_BF16, GP_E4M3, GP_MXFP4 };           // of W
-#define GP_MAX_K (1 << 23)     // a tile's rows lie within 32 bits of its first
+#define GP_FAR (1 << 23)       // K up to which 32 bits reach all rows of a tile
 
-template <int T, int BM, int BN, int WM, int WN, int NS>
+template <int T, int BM, int BN, int WM, int WN, int NS, bool FAR = false>
 static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
   constexpr bool F8 = T == GP_E4M3, W4 = T == GP_MXFP4;
   const bool glu = a.act >= 0;
@@ -483,11 +483,11 @@ static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
   const dim3 grid((a.tm * a.tn + 7) / 8 * 8, sk);
   if (glu)
     hipLaunchKernelGGL(
-        (k_gemm_prompt<F8, BM, BN, WM, WN, NS, true, false, W4>), grid,
+        (k_gemm_prompt<F8, BM, BN, WM, WN, NS, true, false, W4, FAR>), grid,
         dim3(64 * WM * WN), 0, s, a);
   else
     hipLaunchKernelGGL(
-        (k_gemm_prompt<F8, BM, BN, WM, WN, NS, false, false, W4>), grid,
+        (k_gemm_prompt<F8, BM, BN, WM, WN, NS, false, false, W4, FAR>), grid,
         dim3(64 * WM * WN), 0, s, a);
   return hipGetLastError();
 }
@@ -556,12 +556,13 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
   const int width = a.act >= 0 ? 2 * a.N : a.N;
   const int slabs = (int)(((long)a.K * (T == GP_E4M3 ? 1 : 2) + 127) / 128);
   const GpCost& k = gp_cost[T == GP_MXFP4 ? 4 : T * 2 + (a.act >= 0)];
+  const bool far = T != GP_MXFP4 && a.K > GP_FAR;        // 64x64 alone
   int best = -1, best_sk = 1;
   float best_t = 0.f;
   for (int c = 0; c < 8; c++) {
     const GpTile& g = gp_tiles[c];
     const float one = k.one[c], full = k.full[c];
-    if (one == 0.f) continue;
+    if (one == 0.f || (far && c != 6)) continue;
     const long tiles = (long)((a.M + g.bm - 1) / g.bm) *
                        ((width + g.bn - 1) / g.bn);
     for (int sk = 1; sk <= 8; sk++) {
@@ -604,7 +605,10 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
       if constexpr (T != GP_MXFP4)
         return gp_go<T, 128, 64, 2, 2, 3>(a, best_sk, s);
       break;
-    case 6: return gp_go<T, 64, 64, 2, 2, 4>(a, best_sk, s);
+    case 6:
+      if constexpr (T != GP_MXFP4)
+        if (far) return gp_go<T, 64, 64, 2, 2, 4, true>(a, best_sk, s);
+      return gp_go<T, 64, 64, 2, 2, 4>(a, best_sk, s);
     case 7:
       if constexpr (T != GP_MXFP4)
         return gp_go<T, 32, 64, 2, 2, 6>(a, best_sk, s);
@@ -620,7 +624,7 @@ extern "C" hipError_t launch_gemm_prompt(
     const void* res, const void* bias, void* y, void* part, void* cnt,
     long part_floats, int ncnt, int M, int N, int K, int act,
     hipStream_t stream) {
-  if (M < 1 || N < 1 || K < 64 || K % 64 || K > GP_MAX_K || (!sx != !sw))
+  if (M < 1 || N < 1 || K < 64 || K % 64 || (!sx != !sw))
     return hipErrorInvalidValue;
   GpArgs a = {x, w, (const float*)sx, (const float*)sw, nullptr,
               (const u16*)res, (const u16*)bias, (u16*)y, (float*)part,
@@ -639,7 +643,7 @@ extern "C" hipError_t launch_gemm_fp4w(
     const void* x, const void* w, const void* we, const void* res,
     const void* bias, void* y, void* part, void* cnt, long part_floats,
     int ncnt, int M, int N, int K, int act, hipStream_t stream) {
-  if (M < 1 || N < 1 || K < 64 || K % 64 || K > GP_MAX_K || !we)
+  if (M < 1 || N < 1 || K < 64 || K % 64 || !we)
     return hipErrorInvalidValue;
   GpArgs a = {x, w, nullptr, nullptr, (const uint8_t*)we, (const u16*)res,
               (const u16*)bias, (u16*)y, (float*)part, (int*)cnt, M, N, K,
@@ -767,7 +771,7 @@ extern "C" hipError_t launch_expert_gemm(
     const void* sorted, int pairs, int E, int top, int gather, int N, int K,
     int act, hipStream_t stream) {
   if (pairs < 1 || E < 1 || E > 64 || top < 1 || pairs % top || N < 1 ||
-      K < 64 || K % 64 || K > GP_MAX_K || (!sx != !sw))
+      K < 64 || K % 64 || (!sx != !sw))
     return hipErrorInvalidValue;
   const int bm = expert_bm(pairs, E), tiles = pairs / bm + E;
   const int* p = (const int*)sorted;

@@ -296,6 +296,16 @@ def test_many_rows(M, N, K, kind, act):
     assert (Y[M] == 7.0).all() and not cnt.any()
 
 
+# rows so long that 32 bits do not reach those of a tile: of the largest (256
+# rows of 2^24 bytes), and of the one that takes them (64 rows of 66 MB)
+@pytest.mark.parametrize("kind,act,K", [
+    ("bf16", -1, (1 << 23) + 64), ("bf16", 0, (1 << 23) + 64),
+    ("fp8", -1, (1 << 23) + 64), ("fp8", 0, (1 << 23) + 64),
+    ("bf16", -1, 33 << 20)])
+def test_long_rows(kind, act, K):
+    test_many_rows(65, 70, K, kind, act)
+
+
 # the tiles that the device chooses among beside MXFP4 (64x64, 64x128, 128x128
 # of eight and of four waves, 128x256) with a rest both ways; fewer slabs of 64
 # than buffers, as many, one more; parts of K, also with a short last one
