@@ -296,6 +296,25 @@ def test_many_rows(M, N, K, kind, act):
     assert (Y[M] == 7.0).all() and not cnt.any()
 
 
+# each tile by itself and with K split over blocks, where the sizes above leave
+# it out: 256x256 (bf16), 128x256, 128x128 of eight waves, 64x128, 128x64;
+# parts of 128x128, 64x128, 64x64 and 32x64
+@pytest.mark.parametrize("M,N,K,kind,act", [
+    (1037, 10902, 192, "bf16", -1), (525, 11405, 704, "bf16", -1),
+    (513, 3878, 512, "bf16", -1), (1601, 598, 5632, "bf16", -1),
+    (132, 16809, 64, "bf16", -1), (429, 376, 2112, "bf16", -1),
+    (66, 58, 896, "bf16", -1), (517, 1812, 448, "bf16", 0),
+    (589, 418, 7552, "bf16", 0), (130, 8243, 128, "bf16", 0),
+    (33, 8564, 6720, "bf16", 0), (582, 1621, 1152, "bf16", 0),
+    (43, 65, 960, "bf16", 0), (26, 129, 2112, "bf16", 0),
+    (584, 5294, 192, "fp8", -1), (871, 4614, 448, "fp8", -1),
+    (425, 340, 6400, "fp8", -1), (67, 70, 960, "fp8", -1),
+    (137, 7852, 448, "fp8", 0), (596, 845, 7680, "fp8", 0),
+    (19, 16845, 64, "fp8", 0), (378, 193, 5056, "fp8", 0)])
+def test_many_rows_of_each_tile(M, N, K, kind, act):
+    test_many_rows(M, N, K, kind, act)
+
+
 # rows so long that 32 bits do not reach those of a tile: of the largest (256
 # rows of 2^24 bytes), and of the one that takes them (64 rows of 66 MB)
 @pytest.mark.parametrize("kind,act,K", [
