@@ -30,7 +30,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "csrc")
 PKG = os.path.join(ROOT, "llm_np_cp_amd")
 LIBS = {
-    "llmops": ["llm_ops.hip", "gemv.hip", "attn_decode.hip",
+    "llmops": ["llm_ops.hip", "gemv.hip", "chain.hip", "attn_decode.hip",
                "attn_prefill.hip", "row_gemm.hip", "gemm_prompt.hip",
                "mid_gemm.hip", "stack.hip", "xgmi_comm.hip"],
     "linear": ["linear.hip"],

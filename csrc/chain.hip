@@ -1,0 +1,816 @@
+// chain.hip — the products between two attentions of one row in one launch:
+// W_o, gate and up, W_down, and the next layer's q, k and v.
+//
+// A launch of its own costs each of them 3 to 4 us in which no weights move:
+// the dispatch, x and its norm, the first loads, the last rows.  Here the
+// weights never stop: a block's loader waves fill rings in LDS by DMA and run
+// ahead into the next product while its x is still being computed, so what is
+// left between two products is the way of x from block to block.
+//
+// A block of 12 waves on each CU:
+//   4 that multiply: four rows at a time, a KB of each, off their ring; the
+//     waves share out K, or rows, whichever leaves fewer rounds;
+//   4 that load, one for each of these;
+//   4 that bring x (the norm's weights on the way) and finish the outputs.
+// They meet at counters in LDS.  A norm's factor is a number for all of x and
+// comes in behind the product, so no one waits for a sum over x.
+//
+// From block to block there is neither a counter nor a fence (an arrival at a
+// counter takes 25 ns, one after the other): outputs go past the L2 into
+// memory that was filled with ones before the step, which no value is made
+// of, and who needs them reads until none is left.  Every word is written
+// once a step, so no reader meets an old one.
+//
+// All 256 blocks need not run at once.  A wave that has read `limit` times
+// computes what it misses by itself, product by product, in the order of sums
+// of the others (ch_help), and waits for no one: blocks that come late find
+// their work done.  So the launch ends whatever else holds CUs.
+//
+// What is in flight is kept small: what x needs queues behind it.  us for a
+// layer's four products, four launches -> here (weights cold):
+//   2048 wide, 8192 in the middle, bf16        32.9 -> 25.7, e4m3 25.7 -> 19.9
+//   3072, 8192, bf16                           46.9 -> 35.9, MXFP4 27.5 -> 24.2
+//   4096, 14336, bf16 83.5 -> 72.9 (6 TB/s), e4m3 49.4 -> 43.5, MXFP4 39.8 -> 31.3
+//   2304, 9216, bf16, two norms                41.9 -> 35.3
+//   3584, 14336, e4m3, two norms               47.6 -> 43.2
+//   3584, 18944, e4m3                          55.1 -> 49.4
+// Of the first: two slots of a loader in flight ahead of the newest 28.1 (one
+// 25.7), weights kept in the caches 27.3, x read 8 bytes a lane 28.3, in
+// copies for each die 29.1, eight waves that multiply 29.4.  With no x to wait
+// for its weights alone take 17.3 (7 TB/s): a hand-over is 2 to 3 us from the
+// last block's sums to the next product's first, and the rings hold 4 us.
+#include <type_traits>
+
+#include "common.h"
+#include "gemv.h"
+
+typedef unsigned long long ch_u8;
+typedef __bf16 ch_b2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) uint32_t* ch_lp;
+
+enum { CH_RAW = 0, CH_NORM = 1, CH_NORM2 = 2 };
+#define CH_MAX 4                           // products of a launch
+#define CH_BLOCKS 256
+#define CH_NC 4                            // waves: multiply, load, bring x
+#define CH_NL CH_NC
+#define CH_NS 4
+#define CH_NT (64 * CH_NS)
+#define CH_NORM_K (2 * 8 * CH_NT)          // the longest row that is normed
+#define CH_SLOTS 8                         // of a ring, at most
+#define CH_LDS (160 * 1024 - 4096)         // 4 KB beside it
+
+// A product as the caller gives it.  What is marked (*) is read until it is
+// there; such words held ones before the step.
+struct ChStage {
+  const void* w;         // [N, K], with a gate [2N, K]: gate, then up
+  const float* ws;       // e4m3: scales of rows
+  const uint8_t* we;     // MXFP4: exponents [rows, K/32]
+  const void* x;         // bf16 or fp32; with wait (*)
+  const u16* h;          // NORM2: the stream; null: what the last one left
+  const float* g;        // weights of the norm; NORM2: of the first,
+  const float* g2;       //   of the second
+  const u16* add;        // bias or residual; own: y of an earlier product
+  void* y;
+  u16* hout;             // NORM2: the stream behind it, or null
+  int N, K, kind, x_f32, wait, glu, y_f32, own;
+};
+// and how it is shared out
+struct ChStep {
+  ChStage s;
+  int rpb, kwl, cols, groups, ngate, ng, keep, pad;
+};
+struct ChArgs {
+  ChStep st[CH_MAX];
+  int n, act, total, slots, xbytes, hbytes, rbytes, limit;
+  float eps;
+};
+
+DEVINL int ch_s(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <class T> DEVINL T* ch_p(T* p) {
+  const ch_u8 u = (ch_u8)p;
+  return (T*)((ch_u8)(uint32_t)ch_s((int)u) |
+              (ch_u8)(uint32_t)ch_s((int)(u >> 32)) << 32);
+}
+// Counters in LDS, by hand: beside loads into LDS the compiler waits for all
+// of these first.
+DEVINL int ch_get(ch_lp p) {
+  uint32_t v;
+  asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+               : "=v"(v) : "v"(p) : "memory");
+  return ch_s((int)v);
+}
+DEVINL void ch_set(ch_lp p, uint32_t v) {
+  asm volatile("ds_write_b32 %0, %1" :: "v"(p), "v"(v) : "memory");
+}
+DEVINL void ch_done(ch_lp p, int lane) {   // one more wave, its LDS behind it
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if (lane == 0)
+    asm volatile("ds_add_u32 %0, %1" :: "v"(p), "v"(1u) : "memory");
+}
+template <int N> DEVINL void ch_arrived() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+
+DEVINL ch_u8 ch_word(const void* p) {
+  return __hip_atomic_load((const ch_u8*)p, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+// 16 bytes of x past the L2 (sc1, as that load has it; each value in them is
+// looked at by itself, so they need not be of one moment)
+DEVINL u4v_ ch_fresh(__amdgpu_buffer_rsrc_t r, int at) {
+  return __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 16);
+}
+template <bool F32> DEVINL bool ch_there(u4v_ v) {
+  bool all = true;
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    all = all && (F32 ? v[k] != ~0u
+                      : v[k] < 0xffff0000u && (v[k] & 0xffffu) != 0xffffu);
+  return all;
+}
+DEVINL float ch_value(const ChStage& s, const void* y, int n, bool* there) {
+  if (s.y_f32) {
+    const uint32_t v = __hip_atomic_load((const uint32_t*)y + n,
+                                         __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    *there = v != ~0u;
+    return __uint_as_float(v);
+  }
+  const u16 v = __hip_atomic_load((const u16*)y + n, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+  *there = v != 0xffff;
+  return b2f(v);
+}
+DEVINL void ch_put(void* y, int f32, int n, float v) {
+  // a NaN is never all ones (f2b makes its own)
+  if (f32)
+    __hip_atomic_store((uint32_t*)y + n,
+                       v != v ? 0x7fc00000u : __float_as_uint(v),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    __hip_atomic_store((u16*)y + n, f2b(v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+DEVINL f4v ch_quad(uint32_t a, uint32_t b) {    // four bf16
+  return f4v{__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u),
+             __uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u)};
+}
+DEVINL f4v ch_quad(ch_u8 v) { return ch_quad((uint32_t)v, (uint32_t)(v >> 32)); }
+DEVINL ch_u8 ch_pack(f4v v) {
+  return (ch_u8)(f2b(v[0]) | (uint32_t)f2b(v[1]) << 16) |
+         (ch_u8)(f2b(v[2]) | (uint32_t)f2b(v[3]) << 16) << 32;
+}
+// the same for x in LDS, by the unit's own conversion
+DEVINL ch_u8 ch_pack_x(f4v v) {
+  union { __bf16 b[4]; ch_u8 u; } r;
+#pragma unroll
+  for (int k = 0; k < 4; k++) r.b[k] = (__bf16)v[k];
+  return r.u;
+}
+DEVINL float ch_squares(f4v a, f4v b) {
+  return a[0] * a[0] + a[1] * a[1] + a[2] * a[2] + a[3] * a[3] +
+         (b[0] * b[0] + b[1] * b[1] + b[2] * b[2] + b[3] * b[3]);
+}
+
+// Adds to R rows' sums a 16-byte piece of each times x: bf16 as it is (xb),
+// else fp32.  Row by row the same bits whatever R is.
+template <int WT, int R>
+DEVINL void ch_dot(const u4v_* w, u4v_ xb, const f4v* x, const uint32_t* e,
+                   bool in, float* acc) {
+  float p[R], o[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    p[r] = acc[r];
+    o[r] = 0.f;
+  }
+#pragma unroll
+  for (int d = 0; d < 4; d++)
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const uint32_t v = w[r][d];
+      if constexpr (WT == GV_BF16) {
+        union { uint32_t u; ch_b2 b; } s = {v}, t = {xb[d]};
+        p[r] = __builtin_amdgcn_fdot2_f32_bf16(s.b, t.b, p[r], false);
+      } else if constexpr (WT == GV_FP8) {
+        const f2v l = __builtin_amdgcn_cvt_pk_f32_fp8(v, false);
+        const f2v h = __builtin_amdgcn_cvt_pk_f32_fp8(v, true);
+        p[r] += l[0] * x[d][0];
+        o[r] += l[1] * x[d][1];
+        p[r] += h[0] * x[d][2];
+        o[r] += h[1] * x[d][3];
+      } else {
+        const float s = __uint_as_float(e[r] << 23);
+        const f2v t[4] = {__builtin_amdgcn_cvt_scalef32_pk_f32_fp4(v, s, 0),
+                          __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(v, s, 1),
+                          __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(v, s, 2),
+                          __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(v, s, 3)};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          p[r] += t[i][0] * x[d * 2 + i / 2][i % 2 * 2];
+          o[r] += t[i][1] * x[d * 2 + i / 2][i % 2 * 2 + 1];
+        }
+      }
+    }
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    if constexpr (WT != GV_BF16) p[r] += o[r];
+    acc[r] = in ? p[r] : acc[r];           // nothing behind the row's end
+  }
+}
+
+// An output from its sums, on either way
+template <int WT>
+DEVINL float ch_finish(const ChStage& s, int act, float v, float up, float rn,
+                       float s1, float s2, float add) {
+  v *= rn;
+  if constexpr (WT == GV_FP8) v *= s1;
+  if (s.glu) {
+    up *= rn;
+    if constexpr (WT == GV_FP8) up *= s2;
+    v = gate_act(v, act) * up;
+  }
+  return v + add;
+}
+
+// What is missing of the products ahead of `upto`, by a wave by itself: slow,
+// and the same bits.
+template <int WT>
+DEVINL void ch_help(const ChStep* st, int upto, int start, int lane, int act,
+                    float eps) {
+  constexpr int E = gv_e<WT>(), Q = E / 4;
+  for (int t = 0; t < upto; t++) {
+    const ChStep& q = st[t];
+    const ChStage& s = q.s;
+    const int P = s.K / E, C = (P + 63) / 64;
+    auto raw = [&](int i) {                // quad i of x
+      const char* p = (const char*)s.x;
+      if (!s.x_f32) return ch_quad(ch_word(p + (size_t)i * 8));
+      union { ch_u8 u[2]; f4v v; } r;
+      r.u[0] = ch_word(p + (size_t)i * 16);
+      r.u[1] = ch_word(p + (size_t)i * 16 + 8);
+      return r.v;
+    };
+    // sums of squares in the order of the waves that bring x
+    auto over_all = [&](auto quad) {
+      float all = 0.f;
+      for (int w = 0; w < CH_NS; w++) {
+        float ss = 0.f;
+        for (int i = w * 64 + lane; i < s.K / 8; i += CH_NT)
+          ss += ch_squares(quad(i * 2), quad(i * 2 + 1));
+        all += wave_reduce_sum(ss);
+      }
+      return rsqrtf(all / (float)s.K + eps);
+    };
+    float r1 = 1.f, rn = 1.f;
+    auto stream = [&](int i) {             // NORM2: the stream behind it
+      const f4v v = raw(i), h = ch_quad(ch_word(s.h + (size_t)i * 4));
+      const f4v g = *(const f4v*)(s.g + i * 4);
+      f4v o;
+#pragma unroll
+      for (int k = 0; k < 4; k++) o[k] = b2f(f2b(v[k] * r1 * g[k] + h[k]));
+      return o;
+    };
+    if (s.kind == CH_NORM) rn = over_all(raw);
+    if (s.kind == CH_NORM2) {
+      r1 = over_all(raw);
+      rn = over_all(stream);
+    }
+    auto value = [&](int i) {
+      f4v v = s.kind == CH_NORM2 ? stream(i) : raw(i);
+      if (s.kind != CH_RAW) {
+        const f4v g = *(const f4v*)((s.kind == CH_NORM2 ? s.g2 : s.g) + i * 4);
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] *= g[k];
+      }
+      return v;
+    };
+    auto sum = [&](int row) {              // of a row of W
+      float all = 0.f;
+      for (int kw = 0; kw < 1 << q.kwl; kw++) {
+        float acc = 0.f;
+        for (int cc = 0; cc < q.cols; cc++) {
+          const int col = min((cc << q.kwl) + kw, C - 1);
+          const int pc = (cc << q.kwl) + kw < C ? col * 64 + lane : P;
+          const int at = min(pc, P - 1);
+          f4v x[Q];
+          u4v_ xb = {};
+#pragma unroll
+          for (int i = 0; i < Q; i++) x[i] = value(at * Q + i);
+          if constexpr (WT == GV_BF16) {
+            union { ch_u8 u[2]; u4v_ v; } b = {{ch_pack_x(x[0]), ch_pack_x(x[1])}};
+            xb = b.v;
+          }
+          const u4v_ w =
+              *((const u4v_*)((const char*)s.w + (size_t)row * P * 16) + at);
+          const uint32_t e =
+              WT == GV_FP4 ? s.we[(size_t)row * (s.K / 32) + at] : 0;
+          ch_dot<WT, 1>(&w, xb, x, &e, pc < P, &acc);
+        }
+        acc += gv_from<2>(acc);
+        acc += gv_from<1>(acc);
+        acc += gv_from<8>(acc);
+        acc += gv_from<12>(acc);
+        all += gv_halves(acc);
+      }
+      return all;
+    };
+    for (int b0 = 0; b0 < s.N; b0 += 64) {
+      // every wave from another place on, so that they share the work
+      const int base = (b0 + start * 64) % ((s.N + 63) / 64 * 64);
+      bool there;
+      ch_value(s, s.y, min(base + lane, s.N - 1), &there);
+      ch_u8 todo = __ballot(!there && base + lane < s.N);
+      while (todo) {
+        const int n = base + __builtin_ctzll(todo);
+        todo &= todo - 1;
+        float add = 0.f, s1 = 1.f, s2 = 1.f;
+        if (s.add) {
+          if (s.own) {
+            bool yes;
+            add = ch_value(st[0].s, s.add, n, &yes);
+          } else {
+            add = b2f(s.add[n]);
+          }
+        }
+        if (WT == GV_FP8) {
+          s1 = s.ws[n];
+          if (s.glu) s2 = s.ws[s.N + n];
+        }
+        const float v = sum(n), up = s.glu ? sum(s.N + n) : 0.f;
+        const float o = ch_finish<WT>(s, act, v, up, rn, s1, s2, add);
+        if (lane == 0) ch_put(s.y, s.y_f32, n, o);
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+}
+
+// a product as a block's loaders and multipliers see it
+struct ChCur {
+  const char* w;         // first row of the block
+  const char* we;
+  int N, P, C, rpb, nn, kwl, cols, groups, ngate, ng;
+};
+DEVINL ChCur ch_take(const ChStep* st, int i, int wt) {
+  const ChStep* q = st + i;
+  ChCur c;
+  const int K = ch_s(q->s.K), E = 8 << wt, rpb = ch_s(q->rpb);
+  c.N = ch_s(q->s.N);
+  c.P = K / E;
+  c.C = (c.P + 63) / 64;
+  c.rpb = rpb;
+  // a block without rows of its own sees the last one again
+  const int n0 = min((int)blockIdx.x * rpb, c.N - 1);
+  c.nn = min(rpb, c.N - n0);
+  c.w = ch_p((const char*)q->s.w) + (size_t)n0 * c.P * 16;
+  c.we = ch_p((const char*)q->s.we) + (size_t)n0 * (K / 32);
+  c.kwl = ch_s(q->kwl);
+  c.cols = ch_s(q->cols);
+  c.groups = ch_s(q->groups);
+  c.ngate = ch_s(q->ngate);
+  c.ng = ch_s(q->ng);
+  return c;
+}
+// the g-th four rows of a wave: the first, and whether they are up rows
+DEVINL int ch_rows(const ChCur& c, int g, int wave, bool* up) {
+  const int G = min(g * (CH_NC >> c.kwl) + (wave >> c.kwl), c.ng - 1);
+  *up = G >= c.ngate;
+  return (G - (*up ? c.ngate : 0)) * 4;
+}
+
+template <int WT>
+__global__ void __launch_bounds__(64 * (CH_NC + CH_NL + CH_NS))
+k_chain(ChArgs a) {
+  constexpr int E = gv_e<WT>(), Q = E / 4;
+  constexpr int SLOT = WT == GV_FP4 ? 4096 + 256 : 4096;
+  constexpr int LD = WT == GV_FP4 ? 5 : 4; // loads of a slot
+  __shared__ ChStep st[CH_MAX];
+  __shared__ float ssq[4][CH_NS], own[CH_NT];
+  __shared__ uint32_t full[CH_NC], freed[CH_NC], xcnt, scnt, sub;
+  // x | the stream | sums [row][wave] | rings
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = ch_s(tid >> 6);
+  char* const xs = lds;
+  char* const hs = xs + a.xbytes;
+  float* const red = (float*)(hs + a.hbytes);
+  char* const ring = hs + a.hbytes + a.rbytes;
+
+  if (tid < CH_NC) full[tid] = freed[tid] = 0;
+  if (tid == 0) xcnt = scnt = sub = 0;
+  {
+    typedef const __attribute__((address_space(4))) uint32_t* kp;
+    const kp from = (kp)__builtin_amdgcn_kernarg_segment_ptr();
+    for (int i = tid; i < (int)sizeof(st) / 4; i += blockDim.x)
+      ((uint32_t*)st)[i] = from[i];
+  }
+  __syncthreads();
+
+  if (wave < CH_NC) {                      // ---- multiply
+    const ch_lp fullp = (ch_lp)&full[wave], freep = (ch_lp)&freed[wave];
+    int at = 0, have = 0, u = 0;           // slot, slots told, rounds
+    for (int i = 0; i < a.n; i++) {
+      const ChCur c = ch_take(st, i, WT);
+      const int kw = wave & ((1 << c.kwl) - 1);
+      while (ch_get((ch_lp)&xcnt) < CH_NS * (i + 1))
+        __builtin_amdgcn_s_sleep(1);
+      for (int g = 0; g < c.groups; g++) {
+        float acc[4] = {};
+        for (int cc = 0; cc < c.cols; cc++) {
+          while (have <= u) {
+            have = ch_get(fullp);
+            if (have <= u) __builtin_amdgcn_s_sleep(1);
+          }
+          const int col = (cc << c.kwl) + kw;
+          const char* x0 = xs + min(col, c.C - 1) *
+                                (WT == GV_BF16 ? 1024 : 256 * E) + lane * 16;
+          const char* sl = ring + (wave * a.slots + at) * SLOT;
+          if (++at == a.slots) at = 0;
+          u4v_ w[4], xb = {};
+          f4v x[Q];
+          uint32_t e[4] = {};
+          if constexpr (WT == GV_BF16) {
+            xb = *(const u4v_*)x0;
+          } else {
+#pragma unroll
+            for (int k = 0; k < Q; k++) x[k] = *(const f4v*)(x0 + k * 1024);
+          }
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            w[r] = *(const u4v_*)(sl + r * 1024 + lane * 16);
+            if constexpr (WT == GV_FP4)
+              e[r] = *(const uint8_t*)(sl + 4096 + r * 64 + lane);
+          }
+          ch_set(freep, ++u);              // LDS keeps a wave's order
+          ch_dot<WT, 4>(w, xb, x, e, col * 64 + lane < c.P, acc);
+        }
+        const float s = gv_rows<4>(acc, lane);
+        bool up;
+        const int r0 = ch_rows(c, g, wave, &up);
+        if (lane < 4 && r0 + lane < c.rpb)
+          red[((up ? c.rpb : 0) + r0 + lane) * CH_NC + kw] = s;
+      }
+      ch_done((ch_lp)&scnt, lane);
+    }
+  } else if (wave < CH_NC + CH_NL) {       // ---- load
+    const int wv = wave - CH_NC;
+    const ch_lp fullp = (ch_lp)&full[wv], freep = (ch_lp)&freed[wv];
+    int ps = 0, pg = 0, pc = 0, at = 0, freedv = 0;
+    ChCur c = ch_take(st, 0, WT);
+    // slots that have arrived are told as the next one is asked for: one in
+    // flight behind the newest
+    __builtin_amdgcn_s_sleep(12);          // x of the first product goes ahead
+    for (int u = 0; u < a.total; u++) {
+      if (u - freedv >= a.slots) {
+        freedv = ch_get(freep);
+        if (u - freedv >= a.slots) {       // none free: wait for the newest
+          ch_arrived<0>();
+          ch_set(fullp, u);
+          while (u - (freedv = ch_get(freep)) >= a.slots)
+            __builtin_amdgcn_s_sleep(1);
+        }
+      }
+      bool up;
+      const int r0 = ch_rows(c, pg, wv, &up);
+      const int col =
+          min((pc << c.kwl) + (wv & ((1 << c.kwl) - 1)), c.C - 1);
+      const int piece = min(col * 64 + lane, c.P - 1);
+      char* const sl = ring + (wv * a.slots + at) * SLOT;
+      const char* w = c.w + (up ? (size_t)c.N * c.P * 16 : 0);
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) uint32_t*)(
+                w + (size_t)min(r0 + r, c.nn - 1) * c.P * 16 +
+                (size_t)piece * 16),
+            (__attribute__((address_space(3))) uint32_t*)(sl + r * 1024), 16,
+            0, 2);
+      if constexpr (WT == GV_FP4) {        // four bytes a lane
+        const int row = min(r0 + (lane >> 4), c.nn - 1);
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) uint32_t*)(
+                c.we + (up ? (size_t)c.N * c.P : 0) + (size_t)row * c.P +
+                min(col * 64 + (lane & 15) * 4, c.P - 4)),
+            (__attribute__((address_space(3))) uint32_t*)(sl + 4096), 4, 0, 2);
+      }
+      if (u > 0) {
+        ch_arrived<LD>();
+        ch_set(fullp, u);
+      }
+      if (++at == a.slots) at = 0;
+      if (++pc < c.cols) continue;
+      pc = 0;
+      if (++pg < c.groups) continue;
+      pg = 0;
+      if (++ps < a.n) c = ch_take(st, ps, WT);
+    }
+    ch_arrived<0>();
+    ch_set(fullp, a.total);
+  } else {                                 // ---- bring x, finish outputs
+    __builtin_amdgcn_s_setprio(3);         // what all others wait for
+    const int t = tid - 64 * (CH_NC + CH_NL), sw = wave - CH_NC - CH_NL;
+    int limit = a.limit, sums = 0;         // sums: over all of x, so far
+    auto add_up = [&](float v) {           // one more: this wave's share
+      v = wave_reduce_sum(v);
+      if (lane == 0) ssq[sums & 3][sw] = v;
+      sums++;
+      ch_done((ch_lp)&sub, lane);
+    };
+    auto factor = [&](int K) {             // of the last one
+      while (ch_get((ch_lp)&sub) < CH_NS * sums) __builtin_amdgcn_s_sleep(0);
+      float v = 0.f;
+#pragma unroll
+      for (int k = 0; k < CH_NS; k++)
+        v += ((volatile float*)ssq[(sums - 1) & 3])[k];
+      return rsqrtf(v / (float)K + a.eps);
+    };
+    for (int i = 0; i < a.n; i++) {
+      const ChStage& s = st[i].s;
+      const int K = ch_s(s.K), kind = ch_s(s.kind);
+      const int rpb = ch_s(st[i].rpb), n0 = blockIdx.x * rpb;
+      const int nn = max(0, min(rpb, ch_s(s.N) - n0));
+      const bool wait = ch_s(s.wait), glu = ch_s(s.glu);
+      const char* const src = (const char*)ch_p(s.x);
+      const float *const g = ch_p(s.g), *const g2 = ch_p(s.g2);
+      const u16* const hsrc = ch_p(s.h);
+      const u16* const addp = ch_p(s.add);
+      u16* const hout = ch_p(s.hout);
+      const bool fromown = ch_s(s.own), keep = ch_s(st[i].keep);
+      const int kw = 1 << ch_s(st[i].kwl);
+      const float* const wsp = ch_p(s.ws) + n0;
+      const int N = ch_s(s.N), yf32 = ch_s(s.y_f32);
+      void* const y = ch_p(s.y);
+      // what an output needs besides its sums
+      float add = 0.f, s1 = 1.f, s2 = 1.f;
+      auto rest = [&](int r) {
+        if (addp) add = fromown ? own[r] : b2f(addp[n0 + r]);
+        if constexpr (WT == GV_FP8) {
+          s1 = wsp[r];
+          if (glu) s2 = wsp[N + r];
+        }
+      };
+      if (t < nn) rest(t);
+
+      // G pieces of 16 bytes a thread at a time; norms take all of x in one
+      auto bring = [&](auto gn, auto f32, auto norms) {
+        constexpr int G = decltype(gn)::value;
+        constexpr bool F32 = decltype(f32)::value;
+        constexpr bool NORMS = decltype(norms)::value;
+        constexpr int V = F32 ? 1 : 2;     // quads of a piece
+        const int np = K / (4 * V);
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)src, 0, np * 16, 0x00027000);
+        for (int b0 = 0; b0 < np; b0 += G * CH_NT) {
+          auto piece = [&](int j) { return min(b0 + j * CH_NT + t, np - 1); };
+          auto real = [&](int j) { return b0 + j * CH_NT + t < np; };
+          f4v ga[G][V], gb[G][V];
+          ch_u8 hv[G][V];
+          if constexpr (NORMS)             // asked for ahead of x
+#pragma unroll
+            for (int j = 0; j < G; j++)
+#pragma unroll
+              for (int k = 0; k < V; k++) {
+                const int q = piece(j) * V + k;
+                ga[j][k] = *(const f4v*)(g + q * 4);
+                if (kind == CH_NORM2) {
+                  gb[j][k] = *(const f4v*)(g2 + q * 4);
+                  hv[j][k] = hsrc ? *(const ch_u8*)(hsrc + q * 4)
+                                  : *(const ch_u8*)(hs + q * 8);
+                }
+              }
+          u4v_ v[G];
+          uint32_t todo = wait ? (1u << G) - 1 : 0;
+          if (!wait)
+#pragma unroll
+            for (int j = 0; j < G; j++) v[j] = ((const u4v_*)src)[piece(j)];
+          // what the other blocks are still at is not there at once
+          if (wait && b0 == 0) __builtin_amdgcn_s_sleep(12);
+          for (int tries = 0; todo;) {
+            asm volatile("" ::: "memory");  // read again each time
+#pragma unroll
+            for (int j = 0; j < G; j++)
+              if (todo >> j & 1) v[j] = ch_fresh(rs, piece(j) * 16);
+#pragma unroll
+            for (int j = 0; j < G; j++)
+              if (todo >> j & 1 && __all(ch_there<F32>(v[j])))
+                todo &= ~(1u << j);
+            if (todo && ++tries > limit) return false;
+          }
+          f4v x[G][V];
+#pragma unroll
+          for (int j = 0; j < G; j++) {
+            if constexpr (F32) {
+              union { u4v_ u; f4v f; } r = {v[j]};
+              x[j][0] = r.f;
+            } else {
+              x[j][0] = ch_quad(v[j][0], v[j][1]);
+              x[j][V - 1] = ch_quad(v[j][2], v[j][3]);
+            }
+          }
+          auto squares = [&]() {
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < G; j++)
+              ss += real(j) ? ch_squares(x[j][0], x[j][V - 1]) : 0.f;
+            return ss;
+          };
+          float ss = 0.f;
+          if constexpr (NORMS) {
+            if (kind == CH_NORM2) {
+              add_up(squares());
+              const float r1 = factor(K);
+#pragma unroll
+              for (int j = 0; j < G; j++)
+#pragma unroll
+                for (int k = 0; k < V; k++) {
+                  const f4v h = ch_quad(hv[j][k]);
+#pragma unroll
+                  for (int e = 0; e < 4; e++)
+                    x[j][k][e] = x[j][k][e] * r1 * ga[j][k][e] + h[e];
+                  const ch_u8 o = ch_pack(x[j][k]);
+                  x[j][k] = ch_quad(o);
+                  const int q = piece(j) * V + k;
+                  if (real(j)) {
+                    *(ch_u8*)(hs + q * 8) = o;
+                    if (hout && blockIdx.x == 0) *(ch_u8*)(hout + q * 4) = o;
+                  }
+                  ga[j][k] = gb[j][k];
+                }
+            }
+            ss = squares();
+          }
+#pragma unroll
+          for (int j = 0; j < G; j++)
+#pragma unroll
+            for (int k = 0; k < V; k++) {
+              if constexpr (NORMS)
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[j][k][e] *= ga[j][k][e];
+              if (!real(j)) continue;
+              const int q = piece(j) * V + k;
+              if constexpr (WT == GV_BF16)
+                *(ch_u8*)(xs + q * 8) = ch_pack_x(x[j][k]);
+              else                         // a lane's quads a KB apart
+                *(f4v*)(xs + q / (Q * 64) * (256 * E) + q % Q * 1024 +
+                        q / Q % 64 * 16) = x[j][k];
+            }
+          if (b0 + G * CH_NT >= np) {
+            ch_done((ch_lp)&xcnt, lane);
+            if constexpr (NORMS) add_up(ss);
+          }
+        }
+        return true;
+      };
+      using yes = std::true_type;
+      using no = std::false_type;
+      for (;;) {
+        const bool all =
+            ch_s(s.x_f32)     ? bring(std::integral_constant<int, 7>(), yes(), no())
+            : kind == CH_RAW  ? bring(std::integral_constant<int, 4>(), no(), no())
+            : K <= 8 * CH_NT  ? bring(std::integral_constant<int, 1>(), no(), yes())
+                              : bring(std::integral_constant<int, 2>(), no(), yes());
+        if (all) break;
+        ch_help<WT>(st, i, blockIdx.x * CH_NS + sw, lane, a.act, a.eps);
+        limit = min(limit, 8);
+      }
+
+      const float rn = kind == CH_RAW ? 1.f : factor(K);
+      while (ch_get((ch_lp)&scnt) < CH_NC * (i + 1))
+        __builtin_amdgcn_s_sleep(0);
+      for (int r = t; r < nn; r += CH_NT) {
+        if (r != t) rest(r);
+        const f4v p = *(const f4v*)&red[r * CH_NC];
+        const f4v o = *(const f4v*)&red[((glu ? rpb : 0) + r) * CH_NC];
+        float v = 0.f, up = 0.f;
+#pragma unroll
+        for (int k = 0; k < CH_NC; k++)
+          if (k < kw) {
+            v += p[k];
+            up += o[k];
+          }
+        v = ch_finish<WT>(s, a.act, v, up, rn, s1, s2, add);
+        if (keep) own[r] = b2f(f2b(v));
+        ch_put(y, yf32, n0 + r, v);
+      }
+    }
+  }
+}
+
+// How a step's rows of K weights are shared out: the split of K over the
+// waves that multiply with the fewest rounds.
+static ChStep ch_share(const ChStage& s, int wt) {
+  ChStep q = {};
+  q.s = s;
+  const int C = (s.K / (8 << wt) + 63) / 64;
+  q.rpb = (s.N + CH_BLOCKS - 1) / CH_BLOCKS;
+  q.ngate = (q.rpb + 3) / 4;
+  q.ng = s.glu ? 2 * q.ngate : q.ngate;
+  int best = 1 << 30;
+  for (int l = 0; 1 << l <= CH_NC; l++) {
+    const int cols = (C + (1 << l) - 1) >> l, nw = CH_NC >> l;
+    const int groups = (q.ng + nw - 1) / nw;
+    if (cols * groups >= best) continue;
+    best = cols * groups;
+    q.kwl = l;
+    q.cols = cols;
+    q.groups = groups;
+  }
+  return q;
+}
+
+static int ch_plan(ChArgs* a, const ChStage* s, int n, int wt) {
+  const int E = 8 << wt, slot = wt == GV_FP4 ? 4096 + 256 : 4096;
+  int x = 0, h = 0, rows = 0;
+  a->n = n;
+  a->total = 0;
+  for (int i = 0; i < n; i++) {
+    if (s[i].N < 1 || s[i].K < E || s[i].K % E || s[i].K % 8 ||
+        (wt == GV_FP4 && s[i].K % 128) ||
+        (s[i].kind != CH_RAW && (s[i].K > CH_NORM_K || s[i].x_f32)))
+      return 0;
+    a->st[i] = ch_share(s[i], wt);
+    const int C = (s[i].K / E + 63) / 64;
+    const int xb = C * 64 * E * (wt == GV_BF16 ? 2 : 4);
+    const int r = a->st[i].rpb * (s[i].glu ? 2 : 1);
+    x = xb > x ? xb : x;
+    rows = r > rows ? r : rows;
+    if (s[i].kind == CH_NORM2 && s[i].K * 2 > h) h = s[i].K * 2;
+    a->total += a->st[i].cols * a->st[i].groups;
+  }
+  a->xbytes = x;
+  a->hbytes = (h + 15) / 16 * 16;
+  a->rbytes = rows * CH_NC * 4;
+  const long left = (long)CH_LDS - x - a->hbytes - a->rbytes;
+  const int slots = left < 0 ? 0 : (int)(left / (CH_NC * slot));
+  a->slots = slots < CH_SLOTS ? slots : CH_SLOTS;
+  return a->slots;
+}
+
+// Slots of a ring that these products leave room for: with fewer than two
+// they are not taken.
+extern "C" int chain_slots(const ChStage* s, int n, int wt) {
+  ChArgs a = {};
+  if (!s || n < 1 || n > CH_MAX || wt < GV_BF16 || wt > GV_FP4) return 0;
+  return ch_plan(&a, s, n, wt);
+}
+
+template <int WT>
+static hipError_t ch_launch(const ChArgs& a, size_t bytes, hipStream_t s) {
+  static const hipError_t raised = hipFuncSetAttribute(
+      (const void*)&k_chain<WT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      CH_LDS);
+  (void)raised;
+  hipLaunchKernelGGL((k_chain<WT>), dim3(CH_BLOCKS),
+                     dim3(64 * (CH_NC + CH_NL + CH_NS)), bytes, s, a);
+  return hipGetLastError();
+}
+
+// wt as of launch_gemv; limit: reads of a word ahead of computing it.
+extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
+                                   float eps, int limit, hipStream_t stream) {
+  ChArgs a = {};
+  if (!s || n < 1 || n > CH_MAX || wt < GV_BF16 || wt > GV_FP4 || limit < 0 ||
+      ch_plan(&a, s, n, wt) < 2)
+    return hipErrorInvalidValue;
+  int left = -1;                           // who left the stream in LDS
+  for (int i = 0; i < n; i++) {
+    if (!s[i].w || !s[i].x || !s[i].y || (wt == GV_FP8 && !s[i].ws) ||
+        (wt == GV_FP4 && !s[i].we) || s[i].kind < CH_RAW ||
+        s[i].kind > CH_NORM2 || (s[i].kind != CH_RAW && !s[i].g) ||
+        (s[i].kind == CH_NORM2 &&
+         (!s[i].g2 || (!s[i].h && (left < 0 || s[left].K != s[i].K)))) ||
+        // only the first product's outputs are kept, for as many rows
+        (s[i].own && (i == 0 || s[i].add != s[0].y || s[0].glu || s[0].y_f32 ||
+                      s[i].N != s[0].N || a.st[0].rpb > CH_NT)) ||
+        // help reads a stream from memory
+        (s[i].kind == CH_NORM2 && !s[i].h && i != n - 1))
+      return hipErrorInvalidValue;
+    if (s[i].kind == CH_NORM2) left = i;
+    if (s[i].own) a.st[0].keep = 1;
+  }
+  a.act = act;
+  a.eps = eps;
+  a.limit = limit;
+  const size_t bytes = (size_t)a.xbytes + a.hbytes + a.rbytes +
+                       (size_t)a.slots * CH_NC * (wt == GV_FP4 ? 4352 : 4096);
+  switch (wt) {
+    case GV_BF16: return ch_launch<GV_BF16>(a, bytes, stream);
+    case GV_FP8: return ch_launch<GV_FP8>(a, bytes, stream);
+    case GV_FP4: return ch_launch<GV_FP4>(a, bytes, stream);
+  }
+  return hipErrorInvalidValue;
+}
+
+// ones in all of words [0, n) of 16 bytes: what is read until it is there
+__global__ void __launch_bounds__(256) k_chain_clear(u4v_* p, long n) {
+  for (long i = blockIdx.x * 256l + threadIdx.x; i < n; i += gridDim.x * 256l)
+    p[i] = u4v_{~0u, ~0u, ~0u, ~0u};
+}
+
+extern "C" hipError_t launch_chain_clear(void* p, long bytes, hipStream_t s) {
+  if (!p || bytes < 16 || bytes % 16) return hipErrorInvalidValue;
+  const long n = bytes / 16, blocks = (n + 255) / 256;
+  hipLaunchKernelGGL(k_chain_clear, dim3(blocks < 1024 ? blocks : 1024),
+                     dim3(256), 0, s, (u4v_*)p, n);
+  return hipGetLastError();
+}

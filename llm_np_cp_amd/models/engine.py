@@ -121,6 +121,7 @@ class GPUModel(DecodeLoop):
         self.max_seq = max_seq
         self._alloc_state(prefill_chunk)
         self._stack = self._native_stack()
+        self._chains = self._decode_chains()
         self._graph = None
         self._graph_mode = None
         # side-stream weight prefetcher — measured NEGATIVE (the fork's
@@ -486,6 +487,67 @@ class GPUModel(DecodeLoop):
             pools=self.max_batch, eps=cfg.rms_norm_eps,
             scale=self.scale, softcap=self.attn_softcap,
             escale=cfg.embed_scale)
+
+    def _decode_chains(self):
+        """Of each layer the products behind its attention and those into the
+        next one's, as one launch of a decode step; None where sizes or ranks
+        do not let them be one.  What its products leave each other stands in
+        chain_buf, a stretch of its own for every layer."""
+        # its blocks are one a CU: with fewer CUs they would wait for turns
+        cus = torch.cuda.get_device_properties(self.device) \
+            .multi_processor_count
+        if self.moe or self.tp_branch or cus < ho.CHAIN_BLOCKS:
+            return None
+        H, I, n = self.H, self.inter_l, len(self.layers)
+        act = self.b_act.dtype
+        kinds = (H, torch.bfloat16), (I, act), (H, torch.bfloat16)
+        size = [ho.chain_room(*k) for k in kinds]
+        self.chain_buf = torch.zeros(n * sum(size), dtype=torch.uint8,
+                                     device=self.device)
+        self.chain_h = torch.zeros(n, H, dtype=torch.bfloat16,
+                                   device=self.device)
+
+        def weight(lw, name):
+            if self.wq4:
+                return lw[name + "_q4"], None, lw[name + "_e4"]
+            if self.fp8:
+                return lw[name + "_q"], lw[name + "_s"], None
+            return lw[name], None, None
+
+        chains, h = [], self.b_h[0]
+        for i, lw in enumerate(self.layers):
+            at = i * sum(size)
+            o, mid, dn = (ho.chain_part(self.chain_buf, at + sum(size[:k]), *v)
+                          for k, v in enumerate(kinds))
+            nxt = self.layers[i + 1] if i + 1 < n else None
+            gu = dict(W=weight(lw, "wgu"), x=o, y=mid, glu=True)
+            down = dict(W=weight(lw, "wdown"), x=mid, y=dn)
+            st = [dict(W=weight(lw, "wo"), x=self.b_att[0], y=o), gu, down]
+            qkv = nxt and dict(W=weight(nxt, "wqkv"), x=dn, y=self.b_qkv,
+                               add=nxt.get("bqkv"))
+            if self.gemma:
+                gu.update(kind=ho.CHAIN_NORM2, h=h, g=lw["g_post"],
+                          g2=lw["g_preffn"])
+                h = self.chain_h[i]
+                if nxt:
+                    qkv.update(kind=ho.CHAIN_NORM2, g=lw["g_postffn"],
+                               g2=nxt["g_in"], hout=h)
+                else:
+                    gu.update(hout=h)
+            else:
+                st[0].update(add=h)
+                gu.update(kind=ho.CHAIN_NORM, g=lw["g_post"])
+                down.update(add=o)
+                h = dn
+                if nxt:
+                    qkv.update(kind=ho.CHAIN_NORM, g=nxt["g_in"])
+            if nxt:
+                st.append(qkv)
+            chains.append(ho.Chain(st, 2 if self.wq4 else int(self.fp8),
+                                   self.act, self.config.rms_norm_eps))
+        # what the head reads: the stream, Gemma's last branch
+        self.chain_out = (h, dn)
+        return chains if all(c.fits() for c in chains) else None
 
     def _read(self, ids: np.ndarray, pos0: int, layer_hook=None) -> None:
         """A chunk of a prompt (int32, up to PC tokens) from position pos0 of
@@ -1004,7 +1066,8 @@ class GPUModel(DecodeLoop):
 
     def _decode_step(self, greedy: bool, min_p: float,
                      temperature: float = 1.0):
-        """Fused decode path: 5 kernels/layer — RMSNorm lives in the
+        """Fused decode path: 2 kernels a layer where its products run as
+        one launch (``_decode_chains``), else 5 — RMSNorm lives in the
         staging of a product, GLU in the epilogue of gate and up, RoPE +
         KV write inside the attention kernel; a side stream prefetches the
         next layer's weights through MALL, paced by per-layer events."""
@@ -1016,6 +1079,9 @@ class GPUModel(DecodeLoop):
         t2 = self.b_t2
         s0 = torch.cuda.current_stream()
         pf = self.prefetch_on
+        chains = None if pf else self._chains
+        if chains:
+            ho.chain_clear(self.chain_buf)
         self._pf_events = []
         prev = None  # previous gemma layer (its postffn norm fused here)
         for i, lw in enumerate(self.layers):
@@ -1028,7 +1094,9 @@ class GPUModel(DecodeLoop):
                     for t in self._pf_tensors(self.layers[i + 1]):
                         ho.prefetch(t, self._pf_sink)
             window = cfg.sliding_window if cfg.is_sliding(i) else 0
-            if self.gemma and prev is not None:
+            if chains and i > 0:
+                pass                      # with the layer before
+            elif self.gemma and prev is not None:
                 # h' = h + norm(t2_prev)*g_postffn_prev; stage norm(h')*g_in
                 self._dgemv(lw, "wqkv", t2, self.b_qkv,
                             stage=ho.STAGE_NORM2, x2=h,
@@ -1056,6 +1124,9 @@ class GPUModel(DecodeLoop):
                         softcap=self.attn_softcap, window=window or 0,
                         split=self.attn_split,
                         kS=self.k_scale[i], vS=self.v_scale[i])
+            if chains:
+                chains[i].run()
+                continue
             if self.gemma:
                 self._dgemv(lw, "wo", self.b_att[0], t1)
                 tpu.all_reduce(t1)
@@ -1109,6 +1180,8 @@ class GPUModel(DecodeLoop):
             ev.record(self._pf_stream)
             self._pf_events.append(ev)
             s0.wait_event(ev)  # join the fork before the step ends
+        if chains:
+            h, t2 = self.chain_out
         if self.gemma:
             # last layer's post-ffn sandwich norm + final norm, both
             # fused into the lm_head staging (NORM2: h' = h + norm(t2)*

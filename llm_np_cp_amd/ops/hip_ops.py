@@ -100,6 +100,10 @@ _SIGS = {
                      [ctypes.c_void_p],
     "stack_embed": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 2 +
                    [ctypes.c_void_p],
+    "chain_slots": [ctypes.c_void_p] + [ctypes.c_int] * 2,
+    "launch_chain": [ctypes.c_void_p] + [ctypes.c_int] * 3 +
+                    [ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
+    "launch_chain_clear": [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p],
     # one-shot xGMI collectives (csrc/xgmi_comm.hip)
     "launch_xgmi_coll": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                          ctypes.c_int, ctypes.c_int, ctypes.c_long,
@@ -693,6 +697,92 @@ class Stack:
             len(self._layers) if last is None else last, _ptr(rows),
             _ptr(tiles), 0 if tiles is None else tiles.shape[0], most,
             _stream()), "stack_forward")
+
+
+# ----------------------------------------------------------------------
+# the products between two attentions of one row (csrc/chain.hip)
+# ----------------------------------------------------------------------
+
+CHAIN_RAW, CHAIN_NORM, CHAIN_NORM2 = 0, 1, 2
+# reads of a word that another block is at, about a microsecond each, before
+# a wave computes it by itself: beyond what blocks that run are apart
+CHAIN_LIMIT = 64
+CHAIN_BLOCKS = 256
+
+
+def chain_room(n: int, dtype) -> int:
+    """Bytes of n values that products of a chain leave each other."""
+    return -(-n * dtype.itemsize // 256) * 256
+
+
+def chain_part(buf: torch.Tensor, at: int, n: int, dtype) -> torch.Tensor:
+    """n values at byte `at` of buf."""
+    return buf[at:at + n * dtype.itemsize].view(dtype)
+
+
+class _ChainStage(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in (
+        "w", "ws", "we", "x", "h", "g", "g2", "add", "y", "hout")] + \
+        [(n, ctypes.c_int) for n in (
+            "N", "K", "kind", "x_f32", "wait", "glu", "y_f32", "own")]
+
+
+class Chain:
+    """Products that follow each other, in one launch.  ``stages``: of each,
+    its weight ``W`` (w, scales, exponents), ``x`` (of an earlier one of them:
+    its y), ``y`` and, where it has them, kind, g, g2, h, hout, add, glu, as
+    csrc/chain.hip has them.  Every y but the last lies in memory that
+    ``chain_clear`` filled before the step.  Holds what it points to."""
+
+    def __init__(self, stages, wt: int, act: int, eps: float):
+        self._held = stages
+        self.wt, self.act, self.eps = wt, act, eps
+        self._stages = (_ChainStage * len(stages))()
+        f32 = torch.float32
+        for i, (to, s) in enumerate(zip(self._stages, stages)):
+            w, ws, we = s["W"]
+            x, y, add = s["x"], s["y"], s.get("add")
+            to.w, to.ws, to.we = w.data_ptr(), _ptr(ws) or None, \
+                _ptr(we) or None
+            rows, K = w.shape[0], w.shape[1] * (2 if wt == 2 else 1)
+            to.glu = int(s.get("glu", False))
+            to.N, to.K = rows // (2 if to.glu else 1), K
+            to.kind = s.get("kind", CHAIN_RAW)
+            to.x, to.y = x.data_ptr(), y.data_ptr()
+            to.x_f32, to.y_f32 = int(x.dtype == f32), int(y.dtype == f32)
+            to.wait = int(any(x is t["y"] for t in stages[:i]))
+            to.own = int(add is not None and
+                         any(add is t["y"] for t in stages[:i]))
+            to.add = _ptr(add) or None
+            assert w.is_contiguous() and x.is_contiguous() and \
+                y.is_contiguous()
+            assert x.numel() >= K and y.numel() >= to.N
+            assert add is None or (add.dtype == torch.bfloat16 and
+                                   add.numel() >= to.N)
+            assert x.dtype in (f32, torch.bfloat16) and \
+                y.dtype in (f32, torch.bfloat16)
+            for n, dt in dict(h=torch.bfloat16, hout=torch.bfloat16, g=f32,
+                              g2=f32).items():
+                t = s.get(n)
+                assert t is None or (t.dtype == dt and t.numel() >= K)
+                setattr(to, n, _ptr(t) or None)
+
+    def fits(self) -> bool:
+        """Whether the sizes are ones that the kernel takes."""
+        return lib().chain_slots(self._stages, len(self._stages),
+                                 self.wt) >= 2
+
+    def run(self, limit: int = CHAIN_LIMIT):
+        _check(lib().launch_chain(
+            self._stages, len(self._stages), self.wt, self.act,
+            ctypes.c_float(self.eps), limit, _stream()), "chain")
+
+
+def chain_clear(buf: torch.Tensor):
+    """Ones in all of buf: what products of a chain leave is not there yet."""
+    _check(lib().launch_chain_clear(
+        _ptr(buf), buf.numel() * buf.element_size(), _stream()),
+        "chain_clear")
 
 
 # ----------------------------------------------------------------------
