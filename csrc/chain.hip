@@ -1,5 +1,5 @@
 // chain.hip — the products between two attentions of one row in one launch:
-// W_o, gate and up, W_down, and the next layer's q, k and v.
+// W_o, gate and up, W_down, and the next layer's q, k and v, or the head.
 //
 // A launch of its own costs each of them 3 to 4 us in which no weights move:
 // the dispatch, x and its norm, the first loads, the last rows.  Here the
@@ -73,6 +73,8 @@ struct ChStage {
   void* y;
   u16* hout;             // NORM2: the stream behind it, or null
   int N, K, kind, x_f32, wait, glu, y_f32, own;
+  float softcap;         // of the outputs, or 0
+  int pad;
 };
 // and how it is shared out
 struct ChStep {
@@ -222,6 +224,7 @@ DEVINL void ch_dot(const u4v_* w, u4v_ xb, const f4v* x, const uint32_t* e,
 template <int WT>
 DEVINL float ch_finish(const ChStage& s, int act, float v, float up, float rn,
                        float s1, float s2, float add) {
+  const float cap = s.softcap;
   v *= rn;
   if constexpr (WT == GV_FP8) v *= s1;
   if (s.glu) {
@@ -229,6 +232,7 @@ DEVINL float ch_finish(const ChStage& s, int act, float v, float up, float rn,
     if constexpr (WT == GV_FP8) up *= s2;
     v = gate_act(v, act) * up;
   }
+  if (cap > 0.f) v = cap * tanhf(v / cap);
   return v + add;
 }
 
@@ -565,7 +569,7 @@ k_chain(ChArgs a) {
           auto real = [&](int j) { return b0 + j * CH_NT + t < np; };
           f4v ga[G][V], gb[G][V];
           ch_u8 hv[G][V];
-          if constexpr (NORMS)             // asked for ahead of x
+          if (NORMS && kind != CH_RAW)     // asked for ahead of x
 #pragma unroll
             for (int j = 0; j < G; j++)
 #pragma unroll
@@ -637,13 +641,13 @@ k_chain(ChArgs a) {
                   ga[j][k] = gb[j][k];
                 }
             }
-            ss = squares();
+            if (kind != CH_RAW) ss = squares();
           }
 #pragma unroll
           for (int j = 0; j < G; j++)
 #pragma unroll
             for (int k = 0; k < V; k++) {
-              if constexpr (NORMS)
+              if (NORMS && kind != CH_RAW)
 #pragma unroll
                 for (int e = 0; e < 4; e++) x[j][k][e] *= ga[j][k][e];
               if (!real(j)) continue;
@@ -656,7 +660,7 @@ k_chain(ChArgs a) {
             }
           if (b0 + G * CH_NT >= np) {
             ch_done((ch_lp)&xcnt, lane);
-            if constexpr (NORMS) add_up(ss);
+            if (NORMS && kind != CH_RAW) add_up(ss);
           }
         }
         return true;
@@ -666,7 +670,7 @@ k_chain(ChArgs a) {
       for (;;) {
         const bool all =
             ch_s(s.x_f32)     ? bring(std::integral_constant<int, 7>(), yes(), no())
-            : kind == CH_RAW  ? bring(std::integral_constant<int, 4>(), no(), no())
+            : K > CH_NORM_K   ? bring(std::integral_constant<int, 4>(), no(), no())
             : K <= 8 * CH_NT  ? bring(std::integral_constant<int, 1>(), no(), yes())
                               : bring(std::integral_constant<int, 2>(), no(), yes());
         if (all) break;

@@ -47,6 +47,8 @@ struct GvArgs {
   int N, K, stage, act, glu, x_f32, out_f32, kw, nw, rpb, ne;
   int kwl, nwl, kwel;    // log2 of kw, nw, kw / ne
   float eps, softcap, escale;
+  u4v_* ones;            // filled with ones, words of 16 bytes
+  long nones;
 };
 
 // LDS only: weights stay in flight across it
@@ -383,6 +385,9 @@ __global__ void __launch_bounds__(512) k_gemv(GvArgs a) {
     if (a.out_f32) ((float*)a.y)[at] = v;
     else ((u16*)a.y)[at] = f2b(v);
   }
+  for (long i = (long)blockIdx.x * blockDim.x + tid; i < a.nones;
+       i += (long)gridDim.x * blockDim.x)
+    a.ones[i] = u4v_{~0u, ~0u, ~0u, ~0u};
 }
 
 #define GV_ROOM (80 * 1024)                // LDS for the sums of a block
@@ -507,25 +512,29 @@ static hipError_t gv_run(GvArgs a, int maxblocks, hipStream_t s) {
 // wt: 0 bf16, 1 e4m3 with ws, 2 MXFP4 with we.  glu: W holds 2N rows, gate
 // then up, and y = act(gate) * up.  eidx: ne experts' W; their results stand
 // in y one after the other with glu, else they are added up, x [ne, K].
+// ones: bytes that are filled with ones besides (what a later launch leaves
+// there is not there yet; a launch for that alone takes 2 us).
 extern "C" hipError_t launch_gemv(
     const void* W, const void* ws, const void* we, const void* x,
     const void* x2, const void* g, const void* g2, void* y, const void* res,
     int wt, int N, int K, int stage, int act, int glu, int x_f32, int out_f32,
     float eps, float softcap, float escale, int maxblocks, const void* eidx,
-    int ne, long wstride, long sstride, const void* oscale,
-    hipStream_t stream) {
+    int ne, long wstride, long sstride, const void* oscale, void* ones,
+    long ones_bytes, hipStream_t stream) {
   const bool keeps = stage == STAGE_NORM2 || stage == STAGE_NORM_EMBED;
   if (N < 1 || K < 1 || K % (wt == GV_BF16 ? 8 : wt == GV_FP8 ? 16 : 32) ||
       stage < 0 || stage > STAGE_NORM_EMBED || ne < 1 || ne > 8 ||
       (ne > 1 && (!eidx || (!glu && stage != STAGE_RAW) || keeps)) ||
       (x_f32 && stage != STAGE_RAW) || (keeps && !res) ||
-      (wt == GV_FP8 && !ws) || (wt == GV_FP4 && (!we || eidx)))
+      (wt == GV_FP8 && !ws) || (wt == GV_FP4 && (!we || eidx)) ||
+      (ones ? ones_bytes < 16 || ones_bytes % 16 || ne > 1 : ones_bytes != 0))
     return hipErrorInvalidValue;
   GvArgs a = {W, (const float*)ws, (const uint8_t*)we, x, (const u16*)x2,
               (const float*)g, (const float*)g2, y,
               keeps ? nullptr : (const u16*)res, (u16*)res, (const int*)eidx,
               (const float*)oscale, wstride, sstride, N, K, stage, act, glu,
-              x_f32, out_f32, 0, 0, 0, ne, 0, 0, 0, eps, softcap, escale};
+              x_f32, out_f32, 0, 0, 0, ne, 0, 0, 0, eps, softcap, escale,
+              (u4v_*)ones, ones_bytes / 16};
   switch (wt) {
     case GV_BF16: return gv_run<GV_BF16>(a, maxblocks, stream);
     case GV_FP8: return gv_run<GV_FP8>(a, maxblocks, stream);

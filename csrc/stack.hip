@@ -38,7 +38,8 @@ hipError_t launch_gemv(
     const void* x2, const void* g, const void* g2, void* y, const void* res,
     int wt, int N, int K, int stage, int act, int glu, int x_f32, int out_f32,
     float eps, float softcap, float escale, int maxblocks, const void* eidx,
-    int ne, long wstride, long sstride, const void* oscale, hipStream_t);
+    int ne, long wstride, long sstride, const void* oscale, void* ones,
+    long ones_bytes, hipStream_t);
 hipError_t launch_rmsnorm(const void* x, const void* g, const void* res,
                           void* y, const void* g2, void* y2, void* q2,
                           void* s2, int M, int H, float eps, hipStream_t);
@@ -130,7 +131,7 @@ hipError_t st_linear(const StackPlan& p, const StackLin& w, const void* x,
     return launch_gemv(w.w, w.s, nullptr, x, nullptr, nullptr, nullptr, y,
                        bias ? bias : res, ST_FP8, N, K, 0, act > 0 ? act : 0,
                        act >= 0, 0, 0, 1e-5f, 0.f, 1.f, 0, nullptr, 1, 0, 0,
-                       nullptr, s);
+                       nullptr, nullptr, 0, s);
   }
   if (g && K > ST_NORM_K) {
     ST(launch_rmsnorm(x, g, nullptr, p.xn, nullptr, nullptr, nullptr, nullptr,

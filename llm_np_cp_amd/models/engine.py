@@ -490,9 +490,9 @@ class GPUModel(DecodeLoop):
 
     def _decode_chains(self):
         """Of each layer the products behind its attention and those into the
-        next one's, as one launch of a decode step; None where sizes or ranks
-        do not let them be one.  What its products leave each other stands in
-        chain_buf, a stretch of its own for every layer."""
+        next one's, or the head, as one launch of a decode step; None where
+        sizes or ranks do not let them be one.  What its products leave each
+        other stands in chain_buf, a stretch of its own for every layer."""
         # its blocks are one a CU: with fewer CUs they would wait for turns
         cus = torch.cuda.get_device_properties(self.device) \
             .multi_processor_count
@@ -519,34 +519,33 @@ class GPUModel(DecodeLoop):
             at = i * sum(size)
             o, mid, dn = (ho.chain_part(self.chain_buf, at + sum(size[:k]), *v)
                           for k, v in enumerate(kinds))
-            nxt = self.layers[i + 1] if i + 1 < n else None
             gu = dict(W=weight(lw, "wgu"), x=o, y=mid, glu=True)
             down = dict(W=weight(lw, "wdown"), x=mid, y=dn)
             st = [dict(W=weight(lw, "wo"), x=self.b_att[0], y=o), gu, down]
-            qkv = nxt and dict(W=weight(nxt, "wqkv"), x=dn, y=self.b_qkv,
-                               add=nxt.get("bqkv"))
+            if i + 1 < n:
+                nxt = self.layers[i + 1]
+                g_next = nxt["g_in"]
+                last = dict(W=weight(nxt, "wqkv"), y=self.b_qkv,
+                            add=nxt.get("bqkv"))
+            else:
+                g_next = self.g_final
+                last = dict(W=weight(vars(self), "lm_head"), y=self.b_logits_l,
+                            softcap=self.final_softcap)
             if self.gemma:
                 gu.update(kind=ho.CHAIN_NORM2, h=h, g=lw["g_post"],
                           g2=lw["g_preffn"])
                 h = self.chain_h[i]
-                if nxt:
-                    qkv.update(kind=ho.CHAIN_NORM2, g=lw["g_postffn"],
-                               g2=nxt["g_in"], hout=h)
-                else:
-                    gu.update(hout=h)
+                last.update(kind=ho.CHAIN_NORM2, g=lw["g_postffn"], g2=g_next,
+                            hout=h)
             else:
                 st[0].update(add=h)
                 gu.update(kind=ho.CHAIN_NORM, g=lw["g_post"])
                 down.update(add=o)
+                last.update(kind=ho.CHAIN_NORM, g=g_next)
                 h = dn
-                if nxt:
-                    qkv.update(kind=ho.CHAIN_NORM, g=nxt["g_in"])
-            if nxt:
-                st.append(qkv)
-            chains.append(ho.Chain(st, 2 if self.wq4 else int(self.fp8),
+            chains.append(ho.Chain(st + [dict(x=dn, **last)],
+                                   2 if self.wq4 else int(self.fp8),
                                    self.act, self.config.rms_norm_eps))
-        # what the head reads: the stream, Gemma's last branch
-        self.chain_out = (h, dn)
         return chains if all(c.fits() for c in chains) else None
 
     def _read(self, ids: np.ndarray, pos0: int, layer_hook=None) -> None:
@@ -1066,11 +1065,12 @@ class GPUModel(DecodeLoop):
 
     def _decode_step(self, greedy: bool, min_p: float,
                      temperature: float = 1.0):
-        """Fused decode path: 2 kernels a layer where its products run as
-        one launch (``_decode_chains``), else 5 — RMSNorm lives in the
-        staging of a product, GLU in the epilogue of gate and up, RoPE +
-        KV write inside the attention kernel; a side stream prefetches the
-        next layer's weights through MALL, paced by per-layer events."""
+        """Fused decode path: 2 kernels a layer where its products, and with
+        the last layer's the head, run as one launch (``_decode_chains``),
+        else 5 — RMSNorm lives in the staging of a product, GLU in the
+        epilogue of gate and up, RoPE + KV write inside the attention kernel;
+        a side stream prefetches the next layer's weights through MALL, paced
+        by per-layer events."""
         cfg = self.config
         eps = cfg.rms_norm_eps
         h = self.b_h[0]
@@ -1080,8 +1080,8 @@ class GPUModel(DecodeLoop):
         s0 = torch.cuda.current_stream()
         pf = self.prefetch_on
         chains = None if pf else self._chains
-        if chains:
-            ho.chain_clear(self.chain_buf)
+        # what the chains' products leave each other is not there yet
+        ones = dict(ones=self.chain_buf) if chains else {}
         self._pf_events = []
         prev = None  # previous gemma layer (its postffn norm fused here)
         for i, lw in enumerate(self.layers):
@@ -1109,13 +1109,13 @@ class GPUModel(DecodeLoop):
                 self._dgemv(lw, "wqkv", self.embed, self.b_qkv,
                             stage=ho.STAGE_NORM_EMBED, x2=self.next_token,
                             g=lw["g_in"], res=h, eps=eps,
-                            escale=cfg.embed_scale)
+                            escale=cfg.embed_scale, **ones)
             else:
                 if i == 0:  # bias models keep the separate embed gather
                     ho.embed(self.embed, self.next_token, self.b_h, 1,
                              cfg.embed_scale)
                 self._dgemv(lw, "wqkv", h, self.b_qkv, stage=ho.STAGE_NORM,
-                            g=lw["g_in"], res=lw.get("bqkv"), eps=eps)
+                            g=lw["g_in"], res=lw.get("bqkv"), eps=eps, **ones)
             prev = lw
             ho.attn_dec(self.b_qkv, self.k_cache[i], self.v_cache[i],
                         self.b_att[0], self.len_buf, self.cos_t, self.sin_t,
@@ -1181,8 +1181,8 @@ class GPUModel(DecodeLoop):
             self._pf_events.append(ev)
             s0.wait_event(ev)  # join the fork before the step ends
         if chains:
-            h, t2 = self.chain_out
-        if self.gemma:
+            pass                          # the head with the last layer
+        elif self.gemma:
             # last layer's post-ffn sandwich norm + final norm, both
             # fused into the lm_head staging (NORM2: h' = h + norm(t2)*
             # g_postffn, then stage norm(h')*g_final)

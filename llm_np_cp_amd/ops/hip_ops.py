@@ -28,7 +28,8 @@ _SIGS = {
     "launch_gemv": [ctypes.c_void_p] * 9 + [ctypes.c_int] * 8 +
                    [ctypes.c_float] * 3 +
                    [ctypes.c_int, ctypes.c_void_p, ctypes.c_int] +
-                   [ctypes.c_long] * 2 + [ctypes.c_void_p] * 2,
+                   [ctypes.c_long] * 2 + [ctypes.c_void_p] * 2 +
+                   [ctypes.c_long, ctypes.c_void_p],
     "launch_rmsnorm": [ctypes.c_void_p] * 8 + [ctypes.c_int] * 2 +
                       [ctypes.c_float, ctypes.c_void_p],
     "launch_rope_cache": [ctypes.c_void_p] * 7 + [ctypes.c_int] +
@@ -167,7 +168,8 @@ STAGE_NORM_EMBED = 4
 
 
 def _gemv(wt, W, ws, we, K, x, y, res, softcap, stage, x2, g, act, eps,
-          maxblocks, g2, escale, eidx, wstride, sstride, oscale, glu):
+          maxblocks, g2, escale, eidx, wstride, sstride, oscale, glu,
+          ones=None):
     N, ne = W.shape[0] // (2 if glu else 1), 1
     if eidx is not None:        # experts that there are rows for
         ne = min(eidx.numel(), y.numel() // N if glu else x.numel() // K)
@@ -179,7 +181,9 @@ def _gemv(wt, W, ws, we, K, x, y, res, softcap, stage, x2, g, act, eps,
         int(y.dtype == torch.float32), ctypes.c_float(eps),
         ctypes.c_float(softcap), ctypes.c_float(escale), maxblocks,
         _ptr(eidx), ne, ctypes.c_long(wstride), ctypes.c_long(sstride),
-        _ptr(oscale), _stream()), "gemv")
+        _ptr(oscale), _ptr(ones) or None,
+        0 if ones is None else ones.numel() * ones.itemsize, _stream()),
+        "gemv")
 
 
 def gemv(W: torch.Tensor, x: torch.Tensor, y: torch.Tensor,
@@ -189,7 +193,8 @@ def gemv(W: torch.Tensor, x: torch.Tensor, y: torch.Tensor,
          nt: int = 1, rpw: int = 1, maxblocks: int = 0,
          g2: torch.Tensor | None = None, escale: float = 1.0,
          eidx: torch.Tensor | None = None, wstride: int = 0,
-         oscale: torch.Tensor | None = None, glu: bool = False):
+         oscale: torch.Tensor | None = None, glu: bool = False,
+             ones: torch.Tensor | None = None):
     """y[N] = W[N,K] @ stage(x)[K] (+res); stage takes RMSNorm / GLU /
     the Gemma sandwich (NORM2: x2 = h_in, g/g2 = post/pre gammas, res =
     h_out ping-pong) / the embed gather (NORM_EMBED: x = embed table,
@@ -197,10 +202,11 @@ def gemv(W: torch.Tensor, x: torch.Tensor, y: torch.Tensor,
     (RAW).  glu: W holds gate rows, then up rows: y[N/2] = act(gate) * up.
     eidx/wstride/oscale: W of expert *eidx, its result times *oscale; of
     several experts (x [n, K]) the results are added up, with glu they stand
-    one after the other (y [n, N/2]).  nt and rpw are kept for callers: the kernel streams
+    one after the other (y [n, N/2]).  ones: a buffer filled with ones besides
+    (``chain_clear``).  nt and rpw are kept for callers: the kernel streams
     W past the caches and picks its rows by itself."""
     _gemv(0, W, None, None, W.shape[1], x, y, res, softcap, stage, x2, g,
-          act, eps, maxblocks, g2, escale, eidx, wstride, 0, oscale, glu)
+          act, eps, maxblocks, g2, escale, eidx, wstride, 0, oscale, glu, ones)
 
 
 def gemv_fp8(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
@@ -211,12 +217,13 @@ def gemv_fp8(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
              maxblocks: int = 0, g2: torch.Tensor | None = None,
              escale: float = 1.0, eidx: torch.Tensor | None = None,
              wstride: int = 0, sstride: int = 0,
-             oscale: torch.Tensor | None = None, glu: bool = False):
+             oscale: torch.Tensor | None = None, glu: bool = False,
+             ones: torch.Tensor | None = None):
     """y[N] = scales * (Wq[N,K] @ stage(x)); Wq = e4m3fn bytes; the rest
     as for gemv (sstride: scales of an expert)."""
     _gemv(1, Wq, scales, None, Wq.shape[1], x, y, res, softcap, stage, x2, g,
           act, eps, maxblocks, g2, escale, eidx, wstride, sstride, oscale,
-          glu)
+          glu, ones)
 
 
 def rmsnorm(x: torch.Tensor, g: torch.Tensor, y: torch.Tensor | None,
@@ -525,12 +532,13 @@ def gemv_fp4(Wq: torch.Tensor, We: torch.Tensor, x: torch.Tensor,
              x2: torch.Tensor | None = None, g: torch.Tensor | None = None,
              act: int = 0, eps: float = 1e-5, nt: int = 1, rpw: int = 1,
              maxblocks: int = 0, g2: torch.Tensor | None = None,
-             escale: float = 1.0, glu: bool = False):
+             escale: float = 1.0, glu: bool = False,
+             ones: torch.Tensor | None = None):
     """y[N] = W4[N,K] @ stage(x): MXFP4 weights (Wq: N x K/2 packed
     bytes, We: N x K/32 e8m0 scale bytes) — half the fp8 stream; the rest
     as for gemv."""
     _gemv(2, Wq, None, We, Wq.shape[1] * 2, x, y, res, softcap, stage, x2, g,
-          act, eps, maxblocks, g2, escale, None, 0, 0, None, glu)
+          act, eps, maxblocks, g2, escale, None, 0, 0, None, glu, ones)
 
 
 def gemm_fp8(xq: torch.Tensor, sx: torch.Tensor, Wq: torch.Tensor,
@@ -724,13 +732,14 @@ class _ChainStage(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in (
         "w", "ws", "we", "x", "h", "g", "g2", "add", "y", "hout")] + \
         [(n, ctypes.c_int) for n in (
-            "N", "K", "kind", "x_f32", "wait", "glu", "y_f32", "own")]
+            "N", "K", "kind", "x_f32", "wait", "glu", "y_f32", "own")] + \
+        [("softcap", ctypes.c_float), ("pad", ctypes.c_int)]
 
 
 class Chain:
     """Products that follow each other, in one launch.  ``stages``: of each,
     its weight ``W`` (w, scales, exponents), ``x`` (of an earlier one of them:
-    its y), ``y`` and, where it has them, kind, g, g2, h, hout, add, glu, as
+    its y), ``y`` and, where it has them, kind, g, g2, h, hout, add, glu, softcap, as
     csrc/chain.hip has them.  Every y but the last lies in memory that
     ``chain_clear`` filled before the step.  Holds what it points to."""
 
@@ -748,6 +757,7 @@ class Chain:
             to.glu = int(s.get("glu", False))
             to.N, to.K = rows // (2 if to.glu else 1), K
             to.kind = s.get("kind", CHAIN_RAW)
+            to.softcap = s.get("softcap", 0.0)
             to.x, to.y = x.data_ptr(), y.data_ptr()
             to.x_f32, to.y_f32 = int(x.dtype == f32), int(y.dtype == f32)
             to.wait = int(any(x is t["y"] for t in stages[:i]))

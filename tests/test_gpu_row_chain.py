@@ -48,8 +48,9 @@ class Layer:
     from what the one before it left in memory (so that a rounding in one is
     no error of the next)."""
 
-    def __init__(self, ho, wt, H, I, A, Q, gemma=False, last=False, seed=0):
-        self.ho, self.gemma, self.last = ho, gemma, last
+    def __init__(self, ho, wt, H, I, A, Q, gemma=False, last=False, seed=0,
+                 head=0.0):
+        self.ho, self.gemma, self.last, self.head = ho, gemma, last, head
         act = F32 if wt else BF
         self.W = [weight(ho, wt, seed + 1, H, A), weight(ho, wt, seed + 2,
                   2 * I, H), weight(ho, wt, seed + 3, H, I),
@@ -64,12 +65,14 @@ class Layer:
         o, mid, dn = (ho.chain_part(self.buf, sum(size[:k]), *v)
                       for k, v in enumerate(kinds))
         self.o, self.mid, self.dn = o, mid, dn
-        self.qkv = torch.zeros(Q + 8, dtype=BF, device="cuda")
+        self.qkv = torch.zeros(Q + 8, dtype=F32 if head else BF,
+                               device="cuda")
         self.hout = torch.zeros(H, dtype=BF, device="cuda")
         gu = dict(W=self.W[1][0], x=o, y=mid, glu=True)
         down = dict(W=self.W[2][0], x=mid, y=dn)
         st = [dict(W=self.W[0][0], x=self.att, y=o), gu, down]
-        qkv = dict(W=self.W[3][0], x=dn, y=self.qkv, add=self.bias)
+        qkv = dict(W=self.W[3][0], x=dn, y=self.qkv, softcap=head,
+                   add=None if head else self.bias)
         if gemma:
             gu.update(kind=ho.CHAIN_NORM2, h=self.h, g=self.g[0],
                       g2=self.g[1])
@@ -153,7 +156,12 @@ class Layer:
             x = norm(dn) * self.g[1].double()
         if not self.last:
             n = self.bias.numel()
-            near(qkv[:n], x, W[3], add=self.bias.double(), xbf=True)
+            if self.head:                     # |d cap tanh(z / cap)| <= |dz|
+                near(qkv[:n], x, W[3], lambda z, far: (
+                    self.head * torch.tanh(z / self.head),
+                    far + self.head * 2.0 ** -20), bf=False, xbf=True)
+            else:
+                near(qkv[:n], x, W[3], add=self.bias.double(), xbf=True)
             assert (qkv[n:] == 0).all()       # nothing behind its end
 
 
@@ -184,6 +192,16 @@ def test_chain(ho, wt, gemma, H, I, A, Q):
     for _ in range(3):                        # a pass gives the same bits
         for a, b in zip(first, l.run()):
             assert torch.equal(a, b)
+
+
+# more rows a block than threads that finish them, one each, and a rest
+@pytest.mark.parametrize("wt", [0, 1, 2])
+@pytest.mark.parametrize("gemma", [False, True])
+@pytest.mark.parametrize("V", [512, 32768, 66000, 128256])
+def test_head(ho, wt, gemma, V):
+    l = Layer(ho, wt, 256, 768, 256, V, gemma, head=30.0)
+    assert l.chain.fits()
+    l.check(l.run())
 
 
 @pytest.mark.parametrize("wt", [0, 1, 2])
