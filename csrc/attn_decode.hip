@@ -27,7 +27,7 @@
 // 4.3 us at no history, 128 dims.  us, blocks a head apart and two fixed
 // ranges (as before) -> here:
 //   32/8 heads of 64, 90 keys 7.6 -> 4.6; 4000 keys 22.2 -> 10.0
-//   32/8 of 128, 6040 e4m3 keys 39.2 -> 15.5; 160 keys 9.8 -> 6.4
+//   32/8 of 128, 6040 e4m3 keys 39.2 -> 14.1; 160 keys 9.8 -> 6.4
 //   16/8 of 256, 16 sequences of 620 keys, softcap 52.3 -> 25.4 (two ranges)
 //   64/8 of 128, 4 sequences of 2000 keys 97 -> 23
 //   16/4 of 128, 32000 keys 131 -> 38 (1.7 TB/s: few blocks, long ranges)
@@ -413,6 +413,19 @@ __global__ void __launch_bounds__(64 * AD_NW) k_attn_dec_any(AdArgs a) {
   ad_merge<HD, GB>(a, part, out, ng, eff, &last_flag);
 }
 
+// eight e4m3 numbers as bf16, exact (by way of fp32 and f2b, as keys went
+// before, 6040 of 32/8 heads of 128 took 16.6 us, 15.2 like this)
+DEVINL s8v ad_widen(unsigned long long v) {
+  union { ad_b2 p[4]; s8v s; } w;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const uint32_t u = (uint32_t)(v >> (32 * i));
+    w.p[i * 2] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u, 1.0f, false);
+    w.p[i * 2 + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(u, 1.0f, true);
+  }
+  return w.s;
+}
+
 // value * (1, 2^-8, 2^-16, 0): part `part` of its split into bf16 numbers
 DEVINL float ad_part(float v, int part) {
   const float r1 = v - (float)(__bf16)v;
@@ -606,15 +619,9 @@ k_attn_dec(AdArgs a) {
         const int x = HD == 64 ? (r >> 1) & 1 : r & 3;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-          union { ad_b2 p[4]; s8v v; } w;
-#pragma unroll
-          for (int d = 0; d < 2; d++) {
-            w.p[d * 2] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
-                v8[i][h * 2 + d], 1.0f, false);
-            w.p[d * 2 + 1] = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
-                v8[i][h * 2 + d], 1.0f, true);
-          }
-          *(s8v*)(&Vs[wave][r * RB + ((s2 * 2 + h) ^ (x << 2)) * 16]) = w.v;
+          const s8v w = ad_widen((unsigned long long)v8[i][h * 2] |
+                                 (unsigned long long)v8[i][h * 2 + 1] << 32);
+          *(s8v*)(&Vs[wave][r * RB + ((s2 * 2 + h) ^ (x << 2)) * 16]) = w;
         }
       }
     }
@@ -625,7 +632,7 @@ k_attn_dec(AdArgs a) {
 #pragma unroll
       for (int c = 0; c < KC; c++) {
         Op k;
-        if constexpr (KV8) k.s = fp8x8_to_bf16(k8[n][c]);
+        if constexpr (KV8) k.s = ad_widen(k8[n][c]);
         else k.s = kf[n][c];
         s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k.v, qf[c].v, s, 0, 0, 0);
       }
