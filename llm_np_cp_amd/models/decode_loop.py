@@ -9,8 +9,8 @@ An engine supplies the forward pass and the one-token step:
 
 and the device-side decode state (sampled token, RNG counter, output ring,
 sequence lengths).  The loops here prefill, sample the first token from
-the prefill logits, capture the step in a hipGraph and replay it; the host
-sees token ids only once per chunk.  ``_reserve(lens)`` runs before any
+the prefill logits, keep the step (its launches, or a hipGraph) and replay it;
+the host sees token ids only once per chunk.  ``_reserve(lens)`` runs before any
 step that lets row b grow to lens[b] tokens, for engines whose cache is
 allocated on demand.
 """
@@ -36,6 +36,41 @@ class DeviceCacheHandle:
 
 
 class DecodeLoop:
+    # a step is launches and nothing else: they are kept and made again from
+    # native code; else it is captured in a hipGraph
+    launches_only = False
+
+    def _keep_step(self, step):
+        """Runs step() once, for real, and returns what replays it (None and
+        the exception where neither way does)."""
+        if self.launches_only:
+            tape = ho.record(step)
+            if tape is not None:
+                return tape, None
+        else:
+            s = torch.cuda.Stream()
+            s.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(s):
+                step()
+            torch.cuda.current_stream().wait_stream(s)
+        torch.cuda.synchronize()
+        try:
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                step()
+            return g, None
+        except Exception as e:
+            torch.cuda.synchronize()
+            return None, e
+
+    @staticmethod
+    def _replay(kept, n: int) -> None:
+        if isinstance(kept, torch.cuda.CUDAGraph):
+            for _ in range(n):
+                kept.replay()
+        else:
+            kept.replay(n)
+
     def _reserve(self, lens: List[int]) -> None:
         """Cache room for row b up to lens[b] tokens (preallocated pools
         have it already)."""
@@ -62,7 +97,8 @@ class DecodeLoop:
                         greedy: bool = True, min_p: float = 0.1,
                         eos_id=None, chunk: int = 16, on_ids=None,
                         temperature: float = 1.0, stop_fn=None):
-        """Fast generate: device-side hipGraph decode in chunks, host
+        """Fast generate: device-side decode in chunks (of 256 where nobody
+        looks at tokens in between), host
         sees ids every `chunk` tokens (streaming + EOS stop).  Used by
         runtime.generate() for greedy/min-p on GPU models.
         ``eos_id`` may be an int or a collection of ints (HF configs
@@ -80,6 +116,9 @@ class DecodeLoop:
         eos_set = (set() if eos_id is None else
                    {int(eos_id)} if np.isscalar(eos_id) else
                    {int(e) for e in eos_id})
+        # nobody looks at the tokens in between
+        if not (eos_set or on_ids or stop_fn):
+            chunk = max(chunk, 256)
         t0 = _time.perf_counter()
         with trace_range("prefill"):
             self.prefill(prompt_ids)
@@ -133,26 +172,16 @@ class DecodeLoop:
         key = ("batch", B, greedy, min_p, temperature)
         if use_graph and n_steps > 0 and self._graph_mode != key \
                 and not getattr(self, "_graph_failed", False):
-            s = torch.cuda.Stream()
-            s.wait_stream(torch.cuda.current_stream())
-            with torch.cuda.stream(s):
-                self._decode_batch_step(B, greedy, min_p, temperature)
-            torch.cuda.current_stream().wait_stream(s)
-            torch.cuda.synchronize()
+            kept, error = self._keep_step(lambda: self._decode_batch_step(
+                B, greedy, min_p, temperature))
             n_steps -= 1
-            try:
-                g = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(g):
-                    self._decode_batch_step(B, greedy, min_p, temperature)
-                self._graph = g
-                self._graph_mode = key
-            except Exception as e:
-                self._graph_failed = True
-                self._graph_error = e
+            if kept is not None:
+                self._graph, self._graph_mode = kept, key
+            else:
+                self._graph_failed, self._graph_error = True, error
                 use_graph = False
         if use_graph and self._graph_mode == key:
-            for _ in range(n_steps):
-                self._graph.replay()
+            self._replay(self._graph, n_steps)
         else:
             for _ in range(n_steps):
                 self._decode_batch_step(B, greedy, min_p, temperature)
@@ -180,26 +209,16 @@ class DecodeLoop:
         executed = 0
         if (use_graph and g is None and n > 1
                 and not getattr(self, "_graph_failed", False)):
-            s = torch.cuda.Stream()
-            s.wait_stream(torch.cuda.current_stream())
-            with torch.cuda.stream(s):
-                self._decode_batch_step(B, greedy, min_p, temperature)
-            torch.cuda.current_stream().wait_stream(s)
-            torch.cuda.synchronize()
-            executed += 1  # the warm-up was a real step
-            try:
-                g = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(g):
-                    self._decode_batch_step(B, greedy, min_p, temperature)
+            g, error = self._keep_step(lambda: self._decode_batch_step(
+                B, greedy, min_p, temperature))
+            executed += 1  # that was a real step
+            if g is not None:
                 self._bgraphs[key] = g
-            except Exception as e:
-                self._graph_failed = True
-                self._graph_error = e
-                g = None
+            else:
+                self._graph_failed, self._graph_error = True, error
         remaining = n - executed
         if g is not None and use_graph:
-            for _ in range(remaining):
-                g.replay()
+            self._replay(g, remaining)
         else:
             for _ in range(remaining):
                 self._decode_batch_step(B, greedy, min_p, temperature)
@@ -223,11 +242,11 @@ class DecodeLoop:
 
     def capture_decode_graph(self, greedy: bool = True, min_p: float = 0.1,
                              temperature: float = 1.0):
-        """Capture one decode step into a hipGraph (fixed shapes: KV pool
-        is preallocated and the position is a device scalar, so the graph
-        is shape-stable).
+        """Keep one decode step for replay, as its launches or as a hipGraph
+        (fixed shapes: KV pool is preallocated and the position is a device
+        scalar, so a step is shape-stable).
 
-        NOTE: the warm-up executes ONE REAL decode step (advances the
+        NOTE: this executes ONE REAL decode step (advances the
         sequence by one token).  Returns ``(steps_taken, ok)``:
         ``steps_taken`` is the number of real decode steps executed here
         (1 whenever the warm-up ran, 0 when the cached graph is reused)
@@ -240,24 +259,12 @@ class DecodeLoop:
             return 0, True
         if getattr(self, "_graph_failed", False):
             return 0, False
-        # warm-up (a real step) on a side stream, then capture
-        s = torch.cuda.Stream()
-        s.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(s):
-            self._decode_step(greedy, min_p, temperature)
-        torch.cuda.current_stream().wait_stream(s)
-        torch.cuda.synchronize()
-        try:
-            g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g):
-                self._decode_step(greedy, min_p, temperature)
-        except Exception as e:
-            # the warm-up step above DID run (token committed to
-            # out_ring, len_buf advanced) — report it so decode() does
-            # not double-count
-            self._graph_failed = True
-            self._graph_error = e
-            torch.cuda.synchronize()
+        g, error = self._keep_step(
+            lambda: self._decode_step(greedy, min_p, temperature))
+        if g is None:
+            # the step DID run (token committed to out_ring, len_buf
+            # advanced) — report it so decode() does not double-count
+            self._graph_failed, self._graph_error = True, error
             return 1, False
         self._graph = g
         self._graph_mode = mode
@@ -296,8 +303,7 @@ class DecodeLoop:
             if not ok:
                 use_graph = False
         if use_graph and n_steps > 0:
-            for _ in range(n_steps):
-                self._graph.replay()
+            self._replay(self._graph, n_steps)
         else:
             for _ in range(n_steps):
                 self._decode_step(greedy, min_p, temperature)

@@ -134,6 +134,7 @@ class GPUModel(DecodeLoop):
         self._pf_sink = torch.zeros(256, dtype=torch.float32,
                                     device=self.device)
         self._pf_events = []
+        self.launches_only = not (self.tp_branch or self.prefetch_on)
 
     # ------------------------------------------------------------------
     def _auto_max_seq(self) -> int:

@@ -63,6 +63,8 @@ class Rows:
 
 
 class LayeredModel(DecodeLoop):
+    launches_only = True
+
     def __init__(self, config: LayeredConfig, weights, dtype: str = "bf16",
                  max_seq: Optional[int] = 4096, prefill_chunk: int = 2048,
                  device: Optional[str] = None, seed: int = 0,

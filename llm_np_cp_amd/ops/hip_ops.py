@@ -20,6 +20,8 @@ import os
 import numpy as np
 import torch
 
+from . import tape as _tape
+
 _LIB = None
 _LIB_PATH = os.path.join(os.path.dirname(os.path.dirname(
     os.path.abspath(__file__))), "_libllmops.so")
@@ -105,6 +107,8 @@ _SIGS = {
     "launch_chain": [ctypes.c_void_p] + [ctypes.c_int] * 3 +
                     [ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
     "launch_chain_clear": [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p],
+    "tape_run": [ctypes.c_void_p] + [ctypes.c_int] * 2 +
+                [ctypes.c_void_p] * 2,
     # one-shot xGMI collectives (csrc/xgmi_comm.hip)
     "launch_xgmi_coll": [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                          ctypes.c_int, ctypes.c_int, ctypes.c_long,
@@ -133,7 +137,12 @@ def lib():
             fn = getattr(_LIB, name)
             fn.argtypes = argtypes
             fn.restype = ctypes.c_int  # hipError_t
-    return _LIB
+    return _tape.library(_LIB)
+
+
+def record(step):
+    """Runs step() and keeps its launches (see ops/tape.py)."""
+    return _tape.record(step, lib())
 
 
 def _stream() -> int:

@@ -14,6 +14,8 @@ import os
 
 import torch
 
+from . import tape as _tape
+
 _PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 _FNS = {}
 
@@ -192,7 +194,7 @@ def _fn(launcher):
             f.argtypes = argtypes
             f.restype = ctypes.c_int
             _FNS[fn] = f
-    return _FNS[launcher]
+    return _tape.noted(launcher, _FNS[launcher])
 
 
 def _go(name, *args):
