@@ -26,6 +26,17 @@
 // of the others (ch_help), and waits for no one: blocks that come late find
 // their work done.  So the launch ends whatever else holds CUs.
 //
+// Routed experts are products like the others, of weights that are known once
+// the router has chosen: every block dots its x with the router as it brings
+// it, and its loaders wait for the choice, not for a launch of the router's
+// own.  Up to eight experts: their router rows stand in registers ahead of x.
+// W_o, router, gate and up, down, q, k and v, five launches -> here, us:
+//   2048 wide, two of 4096, bf16 39.5 -> 34.8, e4m3 35.1 -> 30.6
+//   4096, two of 14336, bf16 144 -> 129, e4m3 90.2 -> 80.7
+// (Of the first, x of both down products brought at once 34.6; x of one
+// brought while the last is multiplied 35.3, as a read past the L2 takes 3 to
+// 5 us while weights stream.)
+//
 // What is in flight is kept small: what x needs queues behind it.  us for a
 // layer's four products, four launches -> here (weights cold):
 //   2048 wide, 8192 in the middle, bf16        32.9 -> 25.7, e4m3 25.7 -> 19.9
@@ -49,7 +60,9 @@ typedef __bf16 ch_b2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) uint32_t* ch_lp;
 
 enum { CH_RAW = 0, CH_NORM = 1, CH_NORM2 = 2 };
-#define CH_MAX 4                           // products of a launch
+#define CH_MAX 6                           // products of a launch
+#define CH_TOP 2                           // experts of a row, at most
+#define CH_EXPERTS 8                       // to choose from
 #define CH_BLOCKS 256
 #define CH_NC 4                            // waves: multiply, load, bring x
 #define CH_NL CH_NC
@@ -74,7 +87,16 @@ struct ChStage {
   u16* hout;             // NORM2: the stream behind it, or null
   int N, K, kind, x_f32, wait, glu, y_f32, own;
   float softcap;         // of the outputs, or 0
-  int pad;
+  // Routed experts.  slot 1 .. CH_TOP: the product of one that was chosen, W
+  // and ws of expert e wstep bytes and sstep floats on; scaled: its result by
+  // its weight.  route, with slot 1: the router [experts, K] in bf16, dotted
+  // with the normed x; `top` are chosen.  same: x is what the last product
+  // had.  add2: y, in fp32, of the product before this one.
+  int slot;
+  const u16* route;
+  const float* add2;
+  long wstep, sstep;
+  int scaled, same, experts, top;
 };
 // and how it is shared out
 struct ChStep {
@@ -223,10 +245,11 @@ DEVINL void ch_dot(const u4v_* w, u4v_ xb, const f4v* x, const uint32_t* e,
 // An output from its sums, on either way
 template <int WT>
 DEVINL float ch_finish(const ChStage& s, int act, float v, float up, float rn,
-                       float s1, float s2, float add) {
+                       float s1, float s2, float add, float scale = 1.f) {
   const float cap = s.softcap;
   v *= rn;
   if constexpr (WT == GV_FP8) v *= s1;
+  v *= scale;
   if (s.glu) {
     up *= rn;
     if constexpr (WT == GV_FP8) up *= s2;
@@ -240,12 +263,17 @@ DEVINL float ch_finish(const ChStage& s, int act, float v, float up, float rn,
 // and the same bits.
 template <int WT>
 DEVINL void ch_help(const ChStep* st, int upto, int start, int lane, int act,
-                    float eps) {
+                    float eps, const int* eid, const float* ew) {
   constexpr int E = gv_e<WT>(), Q = E / 4;
   for (int t = 0; t < upto; t++) {
     const ChStep& q = st[t];
     const ChStage& s = q.s;
     const int P = s.K / E, C = (P + 63) / 64;
+    // whoever is at a product behind the router's has its choice
+    const int ex = s.slot ? eid[s.slot - 1] : 0;
+    const float scale = s.scaled ? ew[s.slot - 1] : 1.f;
+    const char* const W = (const char*)s.w + ex * s.wstep;
+    const float* const ws = WT == GV_FP8 ? s.ws + ex * s.sstep : nullptr;
     auto raw = [&](int i) {                // quad i of x
       const char* p = (const char*)s.x;
       if (!s.x_f32) return ch_quad(ch_word(p + (size_t)i * 8));
@@ -305,7 +333,7 @@ DEVINL void ch_help(const ChStep* st, int upto, int start, int lane, int act,
             xb = b.v;
           }
           const u4v_ w =
-              *((const u4v_*)((const char*)s.w + (size_t)row * P * 16) + at);
+              *((const u4v_*)(W + (size_t)row * P * 16) + at);
           const uint32_t e =
               WT == GV_FP4 ? s.we[(size_t)row * (s.K / 32) + at] : 0;
           ch_dot<WT, 1>(&w, xb, x, &e, pc < P, &acc);
@@ -336,12 +364,16 @@ DEVINL void ch_help(const ChStep* st, int upto, int start, int lane, int act,
             add = b2f(s.add[n]);
           }
         }
+        if (s.add2) {
+          bool yes;
+          add += ch_value(st[t - 1].s, s.add2, n, &yes);
+        }
         if (WT == GV_FP8) {
-          s1 = s.ws[n];
-          if (s.glu) s2 = s.ws[s.N + n];
+          s1 = ws[n];
+          if (s.glu) s2 = ws[s.N + n];
         }
         const float v = sum(n), up = s.glu ? sum(s.N + n) : 0.f;
-        const float o = ch_finish<WT>(s, act, v, up, rn, s1, s2, add);
+        const float o = ch_finish<WT>(s, act, v, up, rn, s1, s2, add, scale);
         if (lane == 0) ch_put(s.y, s.y_f32, n, o);
       }
     }
@@ -355,7 +387,8 @@ struct ChCur {
   const char* we;
   int N, P, C, rpb, nn, kwl, cols, groups, ngate, ng;
 };
-DEVINL ChCur ch_take(const ChStep* st, int i, int wt) {
+template <bool MOE = false>
+DEVINL ChCur ch_take(const ChStep* st, int i, int wt, const int* eid = nullptr) {
   const ChStep* q = st + i;
   ChCur c;
   const int K = ch_s(q->s.K), E = 8 << wt, rpb = ch_s(q->rpb);
@@ -367,6 +400,8 @@ DEVINL ChCur ch_take(const ChStep* st, int i, int wt) {
   const int n0 = min((int)blockIdx.x * rpb, c.N - 1);
   c.nn = min(rpb, c.N - n0);
   c.w = ch_p((const char*)q->s.w) + (size_t)n0 * c.P * 16;
+  if (MOE && ch_s(q->s.slot))
+    c.w += (size_t)ch_s(eid[ch_s(q->s.slot) - 1]) * q->s.wstep;
   c.we = ch_p((const char*)q->s.we) + (size_t)n0 * (K / 32);
   c.kwl = ch_s(q->kwl);
   c.cols = ch_s(q->cols);
@@ -382,7 +417,7 @@ DEVINL int ch_rows(const ChCur& c, int g, int wave, bool* up) {
   return (G - (*up ? c.ngate : 0)) * 4;
 }
 
-template <int WT>
+template <int WT, bool MOE>
 __global__ void __launch_bounds__(64 * (CH_NC + CH_NL + CH_NS))
 k_chain(ChArgs a) {
   constexpr int E = gv_e<WT>(), Q = E / 4;
@@ -391,6 +426,11 @@ k_chain(ChArgs a) {
   __shared__ ChStep st[CH_MAX];
   __shared__ float ssq[4][CH_NS], own[CH_NT];
   __shared__ uint32_t full[CH_NC], freed[CH_NC], xcnt, scnt, sub;
+  // routed experts: the router's sums, the choice, what add2 is
+  __shared__ float rsum[MOE ? CH_NS : 1][CH_EXPERTS], ew[CH_TOP];
+  __shared__ float own2[MOE ? CH_NT : 1];
+  __shared__ int eid[CH_TOP];
+  __shared__ uint32_t dots, routed;
   // x | the stream | sums [row][wave] | rings
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -401,7 +441,7 @@ k_chain(ChArgs a) {
   char* const ring = hs + a.hbytes + a.rbytes;
 
   if (tid < CH_NC) full[tid] = freed[tid] = 0;
-  if (tid == 0) xcnt = scnt = sub = 0;
+  if (tid == 0) xcnt = scnt = sub = dots = routed = 0;
   {
     typedef const __attribute__((address_space(4))) uint32_t* kp;
     const kp from = (kp)__builtin_amdgcn_kernarg_segment_ptr();
@@ -506,7 +546,14 @@ k_chain(ChArgs a) {
       pc = 0;
       if (++pg < c.groups) continue;
       pg = 0;
-      if (++ps < a.n) c = ch_take(st, ps, WT);
+      if (++ps >= a.n) continue;
+      if constexpr (MOE)
+        if (ch_s(st[ps].s.slot) && !ch_get((ch_lp)&routed)) {
+          ch_arrived<0>();
+          ch_set(fullp, u + 1);            // all that the router waits for
+          while (!ch_get((ch_lp)&routed)) __builtin_amdgcn_s_sleep(1);
+        }
+      c = ch_take<MOE>(st, ps, WT, eid);
     }
     ch_arrived<0>();
     ch_set(fullp, a.total);
@@ -528,9 +575,15 @@ k_chain(ChArgs a) {
         v += ((volatile float*)ssq[(sums - 1) & 3])[k];
       return rsqrtf(v / (float)K + a.eps);
     };
+    float rn = 1.f;
     for (int i = 0; i < a.n; i++) {
       const ChStage& s = st[i].s;
-      const int K = ch_s(s.K), kind = ch_s(s.kind);
+      const int K = ch_s(s.K), skind = ch_s(s.kind);
+      const u16* const route = MOE ? ch_p(s.route) : nullptr;
+      const int slot = MOE ? ch_s(s.slot) : 0;
+      const bool add2 = MOE && ch_p(s.add2);
+      [[maybe_unused]] float scale = 1.f;
+
       const int rpb = ch_s(st[i].rpb), n0 = blockIdx.x * rpb;
       const int nn = max(0, min(rpb, ch_s(s.N) - n0));
       const bool wait = ch_s(s.wait), glu = ch_s(s.glu);
@@ -539,27 +592,38 @@ k_chain(ChArgs a) {
       const u16* const hsrc = ch_p(s.h);
       const u16* const addp = ch_p(s.add);
       u16* const hout = ch_p(s.hout);
-      const bool fromown = ch_s(s.own), keep = ch_s(st[i].keep);
+      const bool fromown = ch_s(s.own);
+      const int keep = ch_s(st[i].keep);
       const int kw = 1 << ch_s(st[i].kwl);
-      const float* const wsp = ch_p(s.ws) + n0;
+      const float* wsp = ch_p(s.ws) + n0;
       const int N = ch_s(s.N), yf32 = ch_s(s.y_f32);
       void* const y = ch_p(s.y);
       // what an output needs besides its sums
       float add = 0.f, s1 = 1.f, s2 = 1.f;
       auto rest = [&](int r) {
         if (addp) add = fromown ? own[r] : b2f(addp[n0 + r]);
+        if (MOE && add2) add += own2[r];
         if constexpr (WT == GV_FP8) {
           s1 = wsp[r];
           if (glu) s2 = wsp[N + r];
         }
       };
-      if (t < nn) rest(t);
+      // an expert's are known only behind its router
+      if (t < nn && !(MOE && route)) {
+        if constexpr (MOE) {
+          if (slot && WT == GV_FP8) wsp += (size_t)ch_s(eid[slot - 1]) * s.sstep;
+          if (s.scaled) scale = ew[slot - 1];
+        }
+        rest(t);
+      }
 
       // G pieces of 16 bytes a thread at a time; norms take all of x in one
-      auto bring = [&](auto gn, auto f32, auto norms) {
+      auto bring = [&](auto gn, auto f32, auto norms, auto routes) {
         constexpr int G = decltype(gn)::value;
         constexpr bool F32 = decltype(f32)::value;
         constexpr bool NORMS = decltype(norms)::value;
+        constexpr bool ROUTES = decltype(routes)::value;   // by NORM alone
+        const int kind = ROUTES ? CH_NORM : skind;
         constexpr int V = F32 ? 1 : 2;     // quads of a piece
         const int np = K / (4 * V);
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -582,6 +646,17 @@ k_chain(ChArgs a) {
                                   : *(const ch_u8*)(hs + q * 8);
                 }
               }
+          [[maybe_unused]] ch_u8 wg[ROUTES ? CH_EXPERTS : 1][G][V];
+          if constexpr (ROUTES)
+#pragma unroll
+            for (int e = 0; e < CH_EXPERTS; e++)
+#pragma unroll
+              for (int j = 0; j < G; j++)
+#pragma unroll
+                for (int k = 0; k < V; k++)
+                  wg[e][j][k] = *(const ch_u8*)(
+                      route + (size_t)min(e, ch_s(s.experts) - 1) * K +
+                      (piece(j) * V + k) * 4);
           u4v_ v[G];
           uint32_t todo = wait ? (1u << G) - 1 : 0;
           if (!wait)
@@ -658,6 +733,25 @@ k_chain(ChArgs a) {
                 *(f4v*)(xs + q / (Q * 64) * (256 * E) + q % Q * 1024 +
                         q / Q % 64 * 16) = x[j][k];
             }
+          if constexpr (ROUTES) {
+            float d[CH_EXPERTS];
+#pragma unroll
+            for (int e = 0; e < CH_EXPERTS; e++) {
+              d[e] = 0.f;
+#pragma unroll
+              for (int j = 0; j < G; j++)
+#pragma unroll
+                for (int k = 0; k < V; k++) {
+                  const f4v w = ch_quad(wg[e][j][k]);
+                  if (real(j))
+                    d[e] += x[j][k][0] * w[0] + x[j][k][1] * w[1] +
+                            (x[j][k][2] * w[2] + x[j][k][3] * w[3]);
+                }
+            }
+            const float r = gv_rows<CH_EXPERTS>(d, lane);
+            if (lane < CH_EXPERTS) rsum[sw][lane] = r;
+            ch_done((ch_lp)&dots, lane);
+          }
           if (b0 + G * CH_NT >= np) {
             ch_done((ch_lp)&xcnt, lane);
             if (NORMS && kind != CH_RAW) add_up(ss);
@@ -667,18 +761,59 @@ k_chain(ChArgs a) {
       };
       using yes = std::true_type;
       using no = std::false_type;
-      for (;;) {
+      const std::integral_constant<int, 1> one;
+      const std::integral_constant<int, 2> two;
+      const std::integral_constant<bool, MOE> moe;
+      if (MOE && ch_s(s.same)) ch_done((ch_lp)&xcnt, lane);
+      else for (;;) {
         const bool all =
-            ch_s(s.x_f32)     ? bring(std::integral_constant<int, 7>(), yes(), no())
-            : K > CH_NORM_K   ? bring(std::integral_constant<int, 4>(), no(), no())
-            : K <= 8 * CH_NT  ? bring(std::integral_constant<int, 1>(), no(), yes())
-                              : bring(std::integral_constant<int, 2>(), no(), yes());
+            MOE && route ? K <= 8 * CH_NT ? bring(one, no(), yes(), moe)
+                                          : bring(two, no(), yes(), moe)
+            : ch_s(s.x_f32)   ? bring(std::integral_constant<int, 7>(), yes(), no(), no())
+            : K > CH_NORM_K   ? bring(std::integral_constant<int, 4>(), no(), no(), no())
+            : K <= 8 * CH_NT  ? bring(one, no(), yes(), no())
+                              : bring(two, no(), yes(), no());
         if (all) break;
-        ch_help<WT>(st, i, blockIdx.x * CH_NS + sw, lane, a.act, a.eps);
+        ch_help<WT>(st, i, blockIdx.x * CH_NS + sw, lane, a.act, a.eps, eid, ew);
         limit = min(limit, 8);
       }
 
-      const float rn = kind == CH_RAW ? 1.f : factor(K);
+      if (!(MOE && ch_s(s.same))) rn = skind == CH_RAW ? 1.f : factor(K);
+      if (MOE && route) {
+        // Every wave by itself, to the same: probabilities of all experts,
+        // the largest of them (the first of equals), by their sum.
+        while (ch_get((ch_lp)&dots) < CH_NS) __builtin_amdgcn_s_sleep(0);
+        const int ne = ch_s(s.experts), top = ch_s(s.top);
+        const int e = lane & (CH_EXPERTS - 1);
+        auto most = [&](float v) {         // over eight lanes
+          v = fmaxf(v, gv_from<1>(v));
+          v = fmaxf(v, gv_from<2>(v));
+          return fmaxf(v, gv_from<7>(v));
+        };
+        float z = 0.f;
+#pragma unroll
+        for (int k = 0; k < CH_NS; k++) z += ((volatile float*)rsum[k])[e];
+        z = e < ne ? z * rn : -INFINITY;
+        float p = __expf(z - most(z)), sum = 0.f, pv[CH_TOP];
+        if (!(p == p)) p = 0.f;            // an index is one of an expert
+        p = e < ne ? p : -2.f;
+#pragma unroll
+        for (int j = 0; j < CH_TOP; j++) {
+          pv[j] = most(p);
+          const int best =
+              __builtin_ctz((uint32_t)__ballot(p == pv[j]) & 0xff | 256) & 7;
+          if (j < top) sum += pv[j];
+          if (e == best) p = -1.f;
+          ((volatile int*)eid)[j] = j < top ? best : 0;
+        }
+#pragma unroll
+        for (int j = 0; j < CH_TOP; j++) ((volatile float*)ew)[j] = pv[j] / sum;
+        ch_done((ch_lp)&routed, lane);
+        if (t < nn) {
+          if (WT == GV_FP8) wsp += (size_t)ch_s(eid[slot - 1]) * s.sstep;
+          rest(t);
+        }
+      }
       while (ch_get((ch_lp)&scnt) < CH_NC * (i + 1))
         __builtin_amdgcn_s_sleep(0);
       for (int r = t; r < nn; r += CH_NT) {
@@ -692,8 +827,9 @@ k_chain(ChArgs a) {
             v += p[k];
             up += o[k];
           }
-        v = ch_finish<WT>(s, a.act, v, up, rn, s1, s2, add);
-        if (keep) own[r] = b2f(f2b(v));
+        v = ch_finish<WT>(s, a.act, v, up, rn, s1, s2, add, scale);
+        if (keep == 1) own[r] = b2f(f2b(v));
+        if (MOE && keep == 2) own2[r] = v;
         ch_put(y, yf32, n0 + r, v);
       }
     }
@@ -758,13 +894,13 @@ extern "C" int chain_slots(const ChStage* s, int n, int wt) {
   return ch_plan(&a, s, n, wt);
 }
 
-template <int WT>
+template <int WT, bool MOE>
 static hipError_t ch_launch(const ChArgs& a, size_t bytes, hipStream_t s) {
   static const hipError_t raised = hipFuncSetAttribute(
-      (const void*)&k_chain<WT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-      CH_LDS);
+      (const void*)&k_chain<WT, MOE>,
+      hipFuncAttributeMaxDynamicSharedMemorySize, CH_LDS);
   (void)raised;
-  hipLaunchKernelGGL((k_chain<WT>), dim3(CH_BLOCKS),
+  hipLaunchKernelGGL((k_chain<WT, MOE>), dim3(CH_BLOCKS),
                      dim3(64 * (CH_NC + CH_NL + CH_NS)), bytes, s, a);
   return hipGetLastError();
 }
@@ -777,12 +913,29 @@ extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
       ch_plan(&a, s, n, wt) < 2)
     return hipErrorInvalidValue;
   int left = -1;                           // who left the stream in LDS
+  int chosen = 0;                          // experts that a router has chosen
   for (int i = 0; i < n; i++) {
+    if (s[i].route) {
+      if (chosen || i == 0 || s[i].slot != 1 || s[i].kind != CH_NORM ||
+          s[i].experts < 1 || s[i].experts > CH_EXPERTS || s[i].top < 1 ||
+          s[i].top > CH_TOP || s[i].top > s[i].experts)
+        return hipErrorInvalidValue;
+      chosen = s[i].top;
+    }
     if (!s[i].w || !s[i].x || !s[i].y || (wt == GV_FP8 && !s[i].ws) ||
         (wt == GV_FP4 && !s[i].we) || s[i].kind < CH_RAW ||
         s[i].kind > CH_NORM2 || (s[i].kind != CH_RAW && !s[i].g) ||
         (s[i].kind == CH_NORM2 &&
          (!s[i].g2 || (!s[i].h && (left < 0 || s[left].K != s[i].K)))) ||
+        (s[i].slot && (wt == GV_FP4 || s[i].slot < 0 || !chosen ||
+                       s[i].slot > chosen || s[i].kind == CH_NORM2)) ||
+        (!s[i].slot && s[i].scaled) ||
+        // the last product's x, and its norm
+        (s[i].same && (i == 0 || s[i].x != s[i - 1].x || s[i].K != s[i - 1].K ||
+                       s[i].kind != s[i - 1].kind || s[i].g != s[i - 1].g)) ||
+        (s[i].add2 && (i < 2 || s[i].add2 != s[i - 1].y || !s[i - 1].y_f32 ||
+                       s[i].N != s[i - 1].N || a.st[0].rpb > CH_NT ||
+                       a.st[i].rpb > CH_NT || s[i - 1].glu)) ||
         // only the first product's outputs are kept, for as many rows
         (s[i].own && (i == 0 || s[i].add != s[0].y || s[0].glu || s[0].y_f32 ||
                       s[i].N != s[0].N || a.st[0].rpb > CH_NT)) ||
@@ -791,6 +944,7 @@ extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
       return hipErrorInvalidValue;
     if (s[i].kind == CH_NORM2) left = i;
     if (s[i].own) a.st[0].keep = 1;
+    if (s[i].add2) a.st[i - 1].keep = 2;
   }
   a.act = act;
   a.eps = eps;
@@ -798,9 +952,13 @@ extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
   const size_t bytes = (size_t)a.xbytes + a.hbytes + a.rbytes +
                        (size_t)a.slots * CH_NC * (wt == GV_FP4 ? 4352 : 4096);
   switch (wt) {
-    case GV_BF16: return ch_launch<GV_BF16>(a, bytes, stream);
-    case GV_FP8: return ch_launch<GV_FP8>(a, bytes, stream);
-    case GV_FP4: return ch_launch<GV_FP4>(a, bytes, stream);
+    case GV_BF16:
+      return chosen ? ch_launch<GV_BF16, true>(a, bytes, stream)
+                    : ch_launch<GV_BF16, false>(a, bytes, stream);
+    case GV_FP8:
+      return chosen ? ch_launch<GV_FP8, true>(a, bytes, stream)
+                    : ch_launch<GV_FP8, false>(a, bytes, stream);
+    case GV_FP4: return ch_launch<GV_FP4, false>(a, bytes, stream);
   }
   return hipErrorInvalidValue;
 }

@@ -497,11 +497,16 @@ class GPUModel(DecodeLoop):
         # its blocks are one a CU: with fewer CUs they would wait for turns
         cus = torch.cuda.get_device_properties(self.device) \
             .multi_processor_count
-        if self.moe or self.tp_branch or cus < ho.CHAIN_BLOCKS:
+        if self.tp_branch or cus < ho.CHAIN_BLOCKS:
             return None
         H, I, n = self.H, self.inter_l, len(self.layers)
         act = self.b_act.dtype
-        kinds = (H, torch.bfloat16), (I, act), (H, torch.bfloat16)
+        E, top = self.config.num_local_experts, self.topk if self.moe else 1
+        if self.moe and (top > ho.CHAIN_TOP or E > ho.CHAIN_EXPERTS or
+                         self.wq4):
+            return None
+        kinds = [(H, torch.bfloat16), (H, torch.bfloat16)] + \
+            [(I, act)] * top + [(H, torch.float32)] * (top - 1)
         size = [ho.chain_room(*k) for k in kinds]
         self.chain_buf = torch.zeros(n * sum(size), dtype=torch.uint8,
                                      device=self.device)
@@ -509,19 +514,22 @@ class GPUModel(DecodeLoop):
                                    device=self.device)
 
         def weight(lw, name):
+            end = "_all" if self.moe and name in ("wgu", "wdown") else ""
             if self.wq4:
                 return lw[name + "_q4"], None, lw[name + "_e4"]
             if self.fp8:
-                return lw[name + "_q"], lw[name + "_s"], None
-            return lw[name], None, None
+                return lw[name + "_q" + end], lw[name + "_s" + end], None
+            return lw[name + end], None, None
 
         chains, h = [], self.b_h[0]
         for i, lw in enumerate(self.layers):
             at = i * sum(size)
-            o, mid, dn = (ho.chain_part(self.chain_buf, at + sum(size[:k]), *v)
-                          for k, v in enumerate(kinds))
-            gu = dict(W=weight(lw, "wgu"), x=o, y=mid, glu=True)
-            down = dict(W=weight(lw, "wdown"), x=mid, y=dn)
+            o, dn, *rest = (
+                ho.chain_part(self.chain_buf, at + sum(size[:k]), *v)
+                for k, v in enumerate(kinds))
+            mid, part = rest[:top], rest[top:]
+            gu = dict(W=weight(lw, "wgu"), x=o, y=mid[0], glu=True)
+            down = dict(W=weight(lw, "wdown"), x=mid[-1], y=dn)
             st = [dict(W=weight(lw, "wo"), x=self.b_att[0], y=o), gu, down]
             if i + 1 < n:
                 nxt = self.layers[i + 1]
@@ -544,6 +552,17 @@ class GPUModel(DecodeLoop):
                 down.update(add=o)
                 last.update(kind=ho.CHAIN_NORM, g=g_next)
                 h = dn
+            if self.moe:
+                # gate and up of each of a row's experts, then their sums
+                gu.update(experts=E, slot=1)
+                down.update(experts=E, slot=top, scaled=True)
+                more = [dict(gu, slot=j + 1, y=mid[j]) for j in range(1, top)]
+                gu.update(route=lw["wg"], top=top)
+                sums = [dict(down, slot=j + 1, x=mid[j], y=part[j], add=None)
+                        for j in range(top - 1)]
+                if part:
+                    down.update(add2=part[-1])
+                st[2:] = more + sums + [down]
             chains.append(ho.Chain(st + [dict(x=dn, **last)],
                                    2 if self.wq4 else int(self.fp8),
                                    self.act, self.config.rms_norm_eps))

@@ -742,14 +742,22 @@ class _ChainStage(ctypes.Structure):
         "w", "ws", "we", "x", "h", "g", "g2", "add", "y", "hout")] + \
         [(n, ctypes.c_int) for n in (
             "N", "K", "kind", "x_f32", "wait", "glu", "y_f32", "own")] + \
-        [("softcap", ctypes.c_float), ("pad", ctypes.c_int)]
+        [("softcap", ctypes.c_float), ("slot", ctypes.c_int),
+         ("route", ctypes.c_void_p), ("add2", ctypes.c_void_p),
+         ("wstep", ctypes.c_long), ("sstep", ctypes.c_long)] + \
+        [(n, ctypes.c_int) for n in ("scaled", "same", "experts", "top")]
+
+
+CHAIN_TOP, CHAIN_EXPERTS = 2, 8           # routed experts of a row, of at most
 
 
 class Chain:
     """Products that follow each other, in one launch.  ``stages``: of each,
     its weight ``W`` (w, scales, exponents), ``x`` (of an earlier one of them:
     its y), ``y`` and, where it has them, kind, g, g2, h, hout, add, glu, softcap, as
-    csrc/chain.hip has them.  Every y but the last lies in memory that
+    csrc/chain.hip has them; of routed experts, W of all ``experts`` one below
+    the other, ``slot`` from 1, ``route`` and ``top`` with the first, scaled,
+    add2.  Every y but the last lies in memory that
     ``chain_clear`` filled before the step.  Holds what it points to."""
 
     def __init__(self, stages, wt: int, act: int, eps: float):
@@ -763,6 +771,21 @@ class Chain:
             to.w, to.ws, to.we = w.data_ptr(), _ptr(ws) or None, \
                 _ptr(we) or None
             rows, K = w.shape[0], w.shape[1] * (2 if wt == 2 else 1)
+            to.slot = s.get("slot", 0)
+            if to.slot:
+                rows //= s["experts"]
+                to.wstep = rows * w.shape[1] * w.element_size()
+                to.sstep, to.experts = rows, s["experts"]
+                to.scaled = int(s.get("scaled", False))
+                to.same = int(i > 0 and x is stages[i - 1]["x"])
+                route, add2 = s.get("route"), s.get("add2")
+                to.route, to.add2 = _ptr(route) or None, _ptr(add2) or None
+                to.top = s.get("top", 0)
+                assert route is None or (
+                    route.dtype == torch.bfloat16 and route.is_contiguous()
+                    and route.shape == (to.experts, K))
+                assert add2 is None or (add2.dtype == f32 and
+                                        add2.numel() >= rows)
             to.glu = int(s.get("glu", False))
             to.N, to.K = rows // (2 if to.glu else 1), K
             to.kind = s.get("kind", CHAIN_RAW)

@@ -281,3 +281,123 @@ def test_two_at_a_time(ho):
     for l, w in zip(ls, want):
         for a, b in zip(w, (l.o, l.mid, l.dn, l.qkv)):
             assert torch.equal(a, b)
+
+
+class Experts(Layer):
+    """Routed experts between W_o and the next layer's q, k and v."""
+
+    def __init__(self, ho, wt, H, I, E, top, seed=0, tie=False):
+        super().__init__(ho, wt, H, I, 256, 192, seed=seed)
+        st = self.chain._held
+        act = F32 if wt else BF
+        self.E, self.top = E, top
+        self.wg = rand(seed + 20, E, H, scale=H ** -0.5).bfloat16()
+        if tie:
+            self.wg[:] = self.wg[0]
+        up, dn = weight(ho, wt, seed + 21, E * 2 * I, H), \
+            weight(ho, wt, seed + 22, E * H, I)
+        self.Wup, self.Wdn = up[1].view(E, 2 * I, H), dn[1].view(E, H, I)
+        kinds = [(H, BF), (H, BF)] + [(I, act)] * top + [(H, F32)] * (top - 1)
+        size = [ho.chain_room(*k) for k in kinds]
+        self.buf = torch.zeros(sum(size), dtype=U8, device="cuda")
+        self.o, self.dn, *rest = (
+            ho.chain_part(self.buf, sum(size[:k]), *v)
+            for k, v in enumerate(kinds))
+        self.mids, self.parts = rest[:top], rest[top:]
+        new = [dict(st[0], y=self.o)]
+        for j in range(top):
+            new.append(dict(W=up[0], x=self.o, y=self.mids[j], glu=True,
+                            kind=ho.CHAIN_NORM, g=self.g[0], experts=E,
+                            slot=j + 1))
+        new[1].update(route=self.wg, top=top)
+        for j in range(top):
+            last = j == top - 1
+            new.append(dict(W=dn[0], x=self.mids[j], experts=E, slot=j + 1,
+                            y=self.dn if last else self.parts[j], scaled=True,
+                            add=self.o if last else None,
+                            add2=self.parts[0] if last and top > 1 else None))
+        new.append(dict(st[3], x=self.dn))
+        self.chain = ho.Chain(new, wt, 0, 1e-5)
+
+    def run(self, **kw):
+        super().run(**kw)
+        return [t.clone() for t in [self.o, self.dn, self.qkv] + self.mids +
+                self.parts]
+
+    def check(self, out):
+        top, wt = self.top, self.wt
+        o, dn, qkv, *rest = (t.double() for t in out)
+        mids, parts = rest[:top], rest[top:]
+
+        def norm(x):
+            return x / torch.sqrt((x * x).mean() + 1e-5)
+
+        def near(got, want, far, bf):
+            far = far + want.abs() * 2.0 ** -8 * bf + 1e-30
+            assert ((got - want).abs() <= far).all(), \
+                ((got - want).abs() / far).max()
+
+        def dot(w, x, bf=True):               # and its error, as in Layer
+            return w @ x, w.abs() @ x.abs() * (
+                2.0 ** -9 * (bf and wt == 0) + x.numel() * 2.0 ** -23 +
+                2.0 ** -19)
+
+        z, far = dot(self.W[0][1], self.att.double(), False)
+        near(o, z + self.h.double(), far, True)
+        x = norm(o) * self.g[0].double()
+        p = torch.softmax(self.wg.double() @ x, 0)
+        pw, pe = torch.sort(p, descending=True, stable=True)
+        pw, pe = pw[:top] / pw[:top].sum(), pe[:top].tolist()
+        want, err = self.o.double() * 0, 0
+        for j in range(top):
+            I = mids[j].numel()
+            z, far = dot(self.Wup[pe[j]], x)
+            t = z[:I].clone().requires_grad_()
+            s = torch.nn.functional.silu(t)
+            s.sum().backward()
+            s = s.detach()
+            near(mids[j], s * z[I:], (t.grad.abs() * far[:I] + far[:I] ** 2) *
+                 (z[I:].abs() + far[I:]) + s.abs() * (
+                     far[I:] + 2.0 ** -18 * z[I:].abs()), wt == 0)
+            z, far = dot(self.Wdn[pe[j]], mids[j], False)
+            want, err = want + pw[j] * z, err + pw[j] * far + \
+                2.0 ** -16 * z.abs()
+            if j < top - 1:
+                near(parts[j], want, err, False)
+        near(dn, want + o, err, True)
+        z, far = dot(self.W[3][1], norm(dn) * self.g[1].double())
+        near(qkv[:192], z + self.bias.double(), far, True)
+
+
+@pytest.mark.parametrize("wt", [0, 1])
+@pytest.mark.parametrize("H,I,E,top", [
+    (256, 512, 8, 2), (1152, 640, 3, 2), (2048, 4096, 8, 2),
+    (2304, 1280, 5, 1), (4096, 2048, 8, 2), (128, 256, 1, 1)])
+def test_experts(ho, wt, H, I, E, top):
+    for seed in (0, 100, 200):
+        l = Experts(ho, wt, H, I, E, top, seed)
+        assert l.chain.fits()
+        first = l.run()
+        l.check(first)
+        for kw in ({}, dict(limit=0)):
+            for a, b in zip(first, l.run(**kw)):
+                assert torch.equal(a, b)
+
+
+def test_experts_alike(ho):
+    """The first of equals, as ``moe_route`` has it; and none that is not
+    there where the router's input is no number."""
+    l = Experts(ho, 0, 256, 512, 8, 2, tie=True)
+    l.check(l.run())
+    l.att[3] = float("nan")
+    o, dn, qkv, *rest = l.run()
+    assert not dn.isfinite().any() and qkv[:192].isnan().all()
+
+
+def test_experts_refused(ho):
+    for field, bad in (("experts", 9), ("top", 3), ("top", 0), ("slot", 2),
+                       ("kind", 0)):
+        l = Experts(ho, 0, 256, 512, 8, 2)
+        setattr(l.chain._stages[1], field, bad)
+        with pytest.raises(RuntimeError):
+            l.chain.run()
