@@ -8,8 +8,8 @@ MI355X-first design:
     extension is missing);
   - preallocated KV pool per layer (in-place writes, no concat);
   - decode state (seq length, sampled token, RNG counter, output ring)
-    lives in device memory so a decode step is hipGraph-replayable with
-    zero host round-trips (torch.cuda.CUDAGraph == hipGraph on ROCm);
+    lives in device memory so a decode step has zero host round-trips and
+    is replayed: its launches, or a hipGraph of them (torch.cuda.CUDAGraph);
   - tensor parallelism: head/row/col-sharded weights per rank, RCCL
     all-reduce after o_proj and down_proj, all-gather for logits
     (world_size==1 skips collectives — same code path).

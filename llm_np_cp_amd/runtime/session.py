@@ -8,7 +8,7 @@ transcript — turn latency stays O(new tokens), not O(conversation).
 Engine-agnostic by construction: both engines expose the same
 continuation primitives (``forward(ids, cache, pos0)`` writes KV at
 [pos0, pos0+n) and returns last-position logits; the GPU engine
-additionally runs its device-side hipGraph ``decode`` loop from that
+additionally runs its device-side ``decode`` loop from that
 state).  The reference re-prefills from scratch every call
 (``llama3.2_model.py:865-902`` — and when caching, feeds back
 re-tokenized text); this is a beyond-parity capability.
@@ -90,7 +90,7 @@ class ChatSession:
         if (hasattr(self.model, "decode") and greedy_or_minp
                 and not self.params.logit_bias
                 and not getattr(self.model, "no_rewind", False)):
-            # GPU engine: continue with the device-side hipGraph loop
+            # GPU engine: continue with the device-side loop
             # (the prefill logits above are already in b_logits)
             produced = 0
             first = True
