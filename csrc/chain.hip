@@ -37,6 +37,9 @@
 // brought while the last is multiplied 35.3, as a read past the L2 takes 3 to
 // 5 us while weights stream.)
 //
+// Behind the head, the largest logit of each wave's share goes to memory too,
+// for a sampler that need not look for it (k_sample_pick).
+//
 // What is in flight is kept small: what x needs queues behind it.  us for a
 // layer's four products, four launches -> here (weights cold):
 //   2048 wide, 8192 in the middle, bf16        32.9 -> 25.7, e4m3 25.7 -> 19.9
@@ -62,6 +65,7 @@ typedef __attribute__((address_space(3))) uint32_t* ch_lp;
 enum { CH_RAW = 0, CH_NORM = 1, CH_NORM2 = 2 };
 #define CH_MAX 6                           // products of a launch
 #define CH_TOP 2                           // experts of a row, at most
+#define CH_TOPS (CH_BLOCKS * CH_NS)
 #define CH_EXPERTS 8                       // to choose from
 #define CH_BLOCKS 256
 #define CH_NC 4                            // waves: multiply, load, bring x
@@ -97,6 +101,7 @@ struct ChStage {
   const float* add2;
   long wstep, sstep;
   int scaled, same, experts, top;
+  float* tops;           // the largest output of each wave's, CH_TOPS of them
 };
 // and how it is shared out
 struct ChStep {
@@ -779,7 +784,7 @@ k_chain(ChArgs a) {
       }
 
       if (!(MOE && ch_s(s.same))) rn = skind == CH_RAW ? 1.f : factor(K);
-      if (MOE && route) {
+      if constexpr (MOE) if (route) {
         // Every wave by itself, to the same: probabilities of all experts,
         // the largest of them (the first of equals), by their sum.
         while (ch_get((ch_lp)&dots) < CH_NS) __builtin_amdgcn_s_sleep(0);
@@ -816,6 +821,8 @@ k_chain(ChArgs a) {
       }
       while (ch_get((ch_lp)&scnt) < CH_NC * (i + 1))
         __builtin_amdgcn_s_sleep(0);
+      float* const tops = ch_p(s.tops);
+      float most = -INFINITY;
       for (int r = t; r < nn; r += CH_NT) {
         if (r != t) rest(r);
         const f4v p = *(const f4v*)&red[r * CH_NC];
@@ -831,6 +838,11 @@ k_chain(ChArgs a) {
         if (keep == 1) own[r] = b2f(f2b(v));
         if (MOE && keep == 2) own2[r] = v;
         ch_put(y, yf32, n0 + r, v);
+        most = fmaxf(most, v);
+      }
+      if (tops) {                          // not a NaN
+        most = wave_reduce_max(most);
+        if (lane == 0) tops[blockIdx.x * CH_NS + sw] = most;
       }
     }
   }
@@ -931,6 +943,7 @@ extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
                        s[i].slot > chosen || s[i].kind == CH_NORM2)) ||
         (!s[i].slot && s[i].scaled) ||
         // the last product's x, and its norm
+        (s[i].tops && (!s[i].y_f32 || i != n - 1)) ||
         (s[i].same && (i == 0 || s[i].x != s[i - 1].x || s[i].K != s[i - 1].K ||
                        s[i].kind != s[i - 1].kind || s[i].g != s[i - 1].g)) ||
         (s[i].add2 && (i < 2 || s[i].add2 != s[i - 1].y || !s[i - 1].y_f32 ||

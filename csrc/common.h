@@ -45,6 +45,11 @@ DEVINL float wave_reduce_sum(float v) {
   const auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
+DEVINL float wave_reduce_max(float v) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v = fmaxf(v, __shfl_xor(v, m));
+  return v;
+}
 
 // act 0: SiLU, 1: tanh-GELU
 DEVINL float gate_act(float x, int act) {

@@ -56,12 +56,6 @@ DEVINL f4v ld16nt(const void* p) {
   return __builtin_nontemporal_load((const f4v*)p);
 }
 
-DEVINL float wave_reduce_max(float v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v = fmaxf(v, __shfl_xor(v, m));
-  return v;
-}
-
 // orders LDS traffic between the lanes of one wave
 DEVINL void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");

@@ -1011,7 +1011,14 @@ k_logit_max(const void* __restrict__ logits, int V, int lbf16,
 // Temperature folds into both the min-p keep-set and the Gumbel score:
 //   p_i(T) >= min_p * p_max(T)  <=>  l_i >= l_max + T*ln(min_p)
 //   Gumbel-argmax over p(T)     <=>  argmax of l_i/T + G_i
-template <int NT>
+//
+// TOPS: one row, whose logits' producer left the largest of several shares of
+// them (`tops`), so that no launch goes through all of them ahead: each block
+// goes through the shares, its first logits already on the way.  The last to
+// arrive advances the RNG counter, which all have read by then.
+// us a step by min-p, both launches -> here: 32000 logits 7.6 -> 5.1, 128256
+// 8.2 -> 5.2, 256000 8.6 -> 5.5.
+template <int NT, bool TOPS>
 __global__ void __launch_bounds__(NT)
 k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
               long ring_stride, float min_p,
@@ -1021,26 +1028,44 @@ k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
               unsigned long long* __restrict__ pick,
               int* __restrict__ cnt, int* __restrict__ next_token,
               int* __restrict__ out_ring, int* __restrict__ nout,
-              int* __restrict__ len_ptr, int bump_len) {
+              int* __restrict__ len_ptr, int bump_len,
+              const float* __restrict__ tops, int ntops) {
   const int b = blockIdx.y;
   gmax += b; pick += b; cnt += b; nout += b;
   out_ring += (size_t)b * ring_stride;
   const float* lf = (const float*)logits + (size_t)b * V;
   const u16* lh = (const u16*)logits + (size_t)b * V;
-  float thresh = -INFINITY;
-  if (!greedy)
-    thresh = fkey_inv((uint32_t)(*gmax >> 32)) + __logf(min_p) / inv_temp;
-  const uint32_t c = (uint32_t)(*ctr) ^ ((uint32_t)b * 0x85ebca6bu);
-  float bv = -INFINITY;
-  int bi = 0x7fffffff;
-  for (int i0 = blockIdx.x * NT * SMP_U + threadIdx.x; i0 < V;
-       i0 += gridDim.x * NT * SMP_U) {
-    float vs[SMP_U];
+  float vs[SMP_U];
+  auto load = [&](int i0) {
 #pragma unroll
     for (int u = 0; u < SMP_U; u++) {
       const int i = min(i0 + u * NT, V - 1);
       vs[u] = lbf16 ? b2f(lh[i]) : lf[i];
     }
+  };
+  const int step = gridDim.x * NT * SMP_U;
+  int i0 = blockIdx.x * NT * SMP_U + threadIdx.x;
+  load(i0);
+  float thresh = -INFINITY;
+  if constexpr (TOPS) {
+    __shared__ float top[NT / 64];
+    float m = -INFINITY;
+    for (int i = threadIdx.x; i < ntops; i += NT) m = fmaxf(m, tops[i]);
+    m = wave_reduce_max(m);
+    if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NT / 64; w++) m = fmaxf(m, top[w]);
+    thresh = m + __logf(min_p) / inv_temp;
+  } else if (!greedy) {
+    thresh = fkey_inv((uint32_t)(*gmax >> 32)) + __logf(min_p) / inv_temp;
+  }
+  const uint32_t c = ((uint32_t)(*ctr) + (TOPS ? 1u : 0u)) ^
+                     ((uint32_t)b * 0x85ebca6bu);
+  float bv = -INFINITY;
+  int bi = 0x7fffffff;
+  for (; i0 < V; i0 += step) {
+    if (i0 >= step) load(i0);
 #pragma unroll
     for (int u = 0; u < SMP_U; u++) {
       const int i = min(i0 + u * NT, V - 1);
@@ -1089,6 +1114,7 @@ k_sample_pick(const void* __restrict__ logits, int V, int lbf16,
   *nout = n + 1;
   // per-row position advances (ragged batch); the shared RNG counter
   // was already advanced by k_logit_max ahead of this kernel
+  if (TOPS) *ctr += 1;
   if (bump_len) len_ptr[b] += 1;
   *pick = 0ull;
   *gmax = 0ull;
@@ -1101,7 +1127,9 @@ extern "C" hipError_t launch_sample(const void* logits, int V, int lbf16,
                                     void* cnt, void* next_token,
                                     void* out_ring, void* nout,
                                     void* len_ptr, int bump_len,
+                                    const void* tops, int ntops,
                                     hipStream_t stream) {
+  if (tops && (batch != 1 || ntops < 1)) return hipErrorInvalidValue;
   // Every block queues up at a word of its row, twice in the pick, and the
   // words of a group's rows share lines: some 25 ns a block, of whatever row.
   // A trip of a block through its logits takes some 0.65 us.  One row: 63
@@ -1119,23 +1147,31 @@ extern "C" hipError_t launch_sample(const void* logits, int V, int lbf16,
                    : batch > 4 ? 16
                                : 64 / (batch > 0 ? batch : 1);
   if (blocks > most) blocks = most;
+#define SMP_PICK(NT, TOPS)                                                   \
+  hipLaunchKernelGGL((k_sample_pick<NT, TOPS>), dim3(blocks, batch),         \
+                     dim3(NT), 0, stream, logits, V, lbf16, ring_stride,     \
+                     min_p, greedy, seed, inv_temp,                          \
+                     (unsigned long long*)gmax, (uint64_t*)ctr,              \
+                     (unsigned long long*)pick, (int*)cnt,                   \
+                     (int*)next_token, (int*)out_ring, (int*)nout,           \
+                     (int*)len_ptr, bump_len, (const float*)tops, ntops)
+  if (tops && !greedy) {
+    SMP_PICK(512, true);
+    return hipGetLastError();
+  }
 #define SMP_GO(NT)                                                           \
   if (!greedy)                                                               \
     hipLaunchKernelGGL(k_logit_max<NT>, dim3(blocks, batch), dim3(NT), 0,    \
                        stream, logits, V, lbf16, (unsigned long long*)gmax,  \
                        (uint64_t*)ctr);                                      \
-  hipLaunchKernelGGL(k_sample_pick<NT>, dim3(blocks, batch), dim3(NT), 0,    \
-                     stream, logits, V, lbf16, ring_stride, min_p, greedy,   \
-                     seed, inv_temp, (unsigned long long*)gmax,              \
-                     (uint64_t*)ctr, (unsigned long long*)pick, (int*)cnt,   \
-                     (int*)next_token, (int*)out_ring, (int*)nout,           \
-                     (int*)len_ptr, bump_len)
+  SMP_PICK(NT, false)
   if (nt == 1024) {
     SMP_GO(1024);
   } else {
     SMP_GO(512);
   }
 #undef SMP_GO
+#undef SMP_PICK
   return hipGetLastError();
 }
 

@@ -399,6 +399,8 @@ class GPUModel(DecodeLoop):
             device=dev)
         self.attn_cnt = torch.zeros(self.nh_l, dtype=torch.int32, device=dev)
         self.s_gmax = torch.zeros(1, dtype=torch.int64, device=dev)
+        self.s_tops = torch.zeros(ho.CHAIN_TOPS, dtype=torch.float32,
+                                  device=dev)
         self.s_pick = torch.zeros(1, dtype=torch.int64, device=dev)
         self.s_cnt = torch.zeros(1, dtype=torch.int32, device=dev)
         i32 = dict(dtype=torch.int32, device=dev)
@@ -539,7 +541,7 @@ class GPUModel(DecodeLoop):
             else:
                 g_next = self.g_final
                 last = dict(W=weight(vars(self), "lm_head"), y=self.b_logits_l,
-                            softcap=self.final_softcap)
+                            softcap=self.final_softcap, tops=self.s_tops)
             if self.gemma:
                 gu.update(kind=ho.CHAIN_NORM2, h=h, g=lw["g_post"],
                           g2=lw["g_preffn"])
@@ -1234,7 +1236,8 @@ class GPUModel(DecodeLoop):
         ho.sample(self.b_logits, min_p, greedy, self.seed, self.rng_ctr,
                   self.s_gmax, self.s_pick, self.next_token, self.out_ring,
                   self.nout, self.len_buf, bump_len=True,
-                  temperature=temperature, cnt=self.s_cnt)
+                  temperature=temperature, cnt=self.s_cnt,
+                  tops=self.s_tops if chains else None)
 
     # ------------------------------------------------------------------
     # lockstep batched decode (throughput mode; beyond-parity capability)

@@ -56,7 +56,8 @@ _SIGS = {
                       ctypes.c_int, ctypes.c_long, ctypes.c_float,
                       ctypes.c_int, ctypes.c_uint64, ctypes.c_float] +
                      [ctypes.c_void_p] * 8 +
-                     [ctypes.c_int, ctypes.c_void_p],
+                     [ctypes.c_int, ctypes.c_void_p, ctypes.c_int,
+                      ctypes.c_void_p],
     "launch_gemm_prompt": [ctypes.c_void_p] * 9 + [ctypes.c_long] +
                           [ctypes.c_int] * 5 + [ctypes.c_void_p],
     "launch_row_gemm": [ctypes.c_void_p] * 11 + [ctypes.c_long] +
@@ -371,11 +372,13 @@ def sample(logits: torch.Tensor, min_p: float, greedy: bool, seed: int,
            next_token: torch.Tensor, out_ring: torch.Tensor,
            nout: torch.Tensor, len_ptr: torch.Tensor,
            bump_len: bool = True, temperature: float = 1.0,
-           cnt: torch.Tensor | None = None, batch: int = 1):
+           cnt: torch.Tensor | None = None, batch: int = 1,
+           tops: torch.Tensor | None = None):
     """min-p / greedy sampler: parallel max + Gumbel-argmax; the
     last-arriving pick block commits the winner (no 1-thread fin
     launch).  gmax/pick are u64 scratch (zeroed once; the commit path
-    re-zeros); cnt is an i32 ticket counter (zeroed once, re-armed).
+    re-zeros); tops (fp32, one row): the largest of shares that make up all
+    logits, where their producer left them; cnt is an i32 ticket counter (zeroed once, re-armed).
     Temperature scales device-side (min-p keep-set + Gumbel score), so
     the GPU fast path matches the CPU sample_token() semantics."""
     V = logits.shape[-1]
@@ -403,7 +406,8 @@ def sample(logits: torch.Tensor, min_p: float, greedy: bool, seed: int,
         ctypes.c_uint64(seed), ctypes.c_float(inv_temp),
         _ptr(ctr), _ptr(gmax), _ptr(pick), _ptr(cnt),
         _ptr(next_token), _ptr(out_ring), _ptr(nout), _ptr(len_ptr),
-        1 if bump_len else 0, _stream()), "sample")
+        1 if bump_len else 0, _ptr(tops),
+        0 if tops is None else tops.numel(), _stream()), "sample")
 
 
 def _gemm_prompt(name, x, w, sx, sw, y, M, K, res, bias, act, accbuf, cnt):
@@ -745,9 +749,11 @@ class _ChainStage(ctypes.Structure):
         [("softcap", ctypes.c_float), ("slot", ctypes.c_int),
          ("route", ctypes.c_void_p), ("add2", ctypes.c_void_p),
          ("wstep", ctypes.c_long), ("sstep", ctypes.c_long)] + \
-        [(n, ctypes.c_int) for n in ("scaled", "same", "experts", "top")]
+        [(n, ctypes.c_int) for n in ("scaled", "same", "experts", "top")] + \
+        [("tops", ctypes.c_void_p)]
 
 
+CHAIN_TOPS = CHAIN_BLOCKS * 4             # shares of the last product's outputs
 CHAIN_TOP, CHAIN_EXPERTS = 2, 8           # routed experts of a row, of at most
 
 
@@ -757,7 +763,7 @@ class Chain:
     its y), ``y`` and, where it has them, kind, g, g2, h, hout, add, glu, softcap, as
     csrc/chain.hip has them; of routed experts, W of all ``experts`` one below
     the other, ``slot`` from 1, ``route`` and ``top`` with the first, scaled,
-    add2.  Every y but the last lies in memory that
+    add2; ``tops``, of the last: the largest of CHAIN_TOPS shares of y.  Every y but the last lies in memory that
     ``chain_clear`` filled before the step.  Holds what it points to."""
 
     def __init__(self, stages, wt: int, act: int, eps: float):
@@ -772,6 +778,10 @@ class Chain:
                 _ptr(we) or None
             rows, K = w.shape[0], w.shape[1] * (2 if wt == 2 else 1)
             to.slot = s.get("slot", 0)
+            tops = s.get("tops")
+            assert tops is None or (tops.dtype == f32 and
+                                    tops.numel() >= CHAIN_TOPS)
+            to.tops = _ptr(tops) or None
             if to.slot:
                 rows //= s["experts"]
                 to.wstep = rows * w.shape[1] * w.element_size()

@@ -401,3 +401,62 @@ def test_experts_refused(ho):
         setattr(l.chain._stages[1], field, bad)
         with pytest.raises(RuntimeError):
             l.chain.run()
+
+
+# blocks of many rows, of a few, with none; waves without a row
+@pytest.mark.parametrize("wt", [0, 1, 2])
+@pytest.mark.parametrize("V", [130, 512, 66000, 128256])
+def test_largest_outputs(ho, wt, V):
+    l = Layer(ho, wt, 256, 768, 256, V, head=30.0)
+    tops = torch.full((ho.CHAIN_TOPS,), 1e9, device="cuda")
+    l.chain._stages[3].tops = tops.data_ptr()
+    out = l.run()
+    l.check(out)
+    assert tops.max() == out[3][:V].max()
+    per = -(-V // ho.CHAIN_BLOCKS)            # a block's rows, its waves'
+    for b in (0, 1, V // per - 1, ho.CHAIN_BLOCKS - 1):
+        rows = out[3][b * per:min(V, (b + 1) * per)]
+        assert tops.view(-1, 4)[b].max() == \
+            (rows.max() if rows.numel() else float("-inf"))
+    l.chain._stages[0].tops = tops.data_ptr()  # of the last, in fp32
+    with pytest.raises(RuntimeError):
+        l.chain.run()
+
+
+# one trip of a block through its logits and more; shares of none
+@pytest.mark.parametrize("V,n", [(1, 1), (7, 3), (2048, 1024), (2049, 1024),
+                                 (32000, 1024), (300001, 1024)])
+@pytest.mark.parametrize("temperature", [1.0, 0.3])
+def test_picks_by_shares(ho, V, n, temperature):
+    """The picks that a pass through all logits ahead gives, and the counter
+    that it leaves."""
+    logits = 3 * rand(V, V)
+    for bad in (None, float("-inf"), float("nan")):
+        if bad is not None:
+            logits[V // 2] = bad
+        tops = torch.full((n,), float("-inf"), device="cuda")
+        for i, share in enumerate(logits.chunk(n)):
+            tops[i] = share[~share.isnan()].max() if \
+                (~share.isnan()).any() else float("-inf")
+        got = []
+        for kw in ({}, dict(tops=tops)):
+            st = [torch.zeros(k, dtype=dt, device="cuda") for k, dt in (
+                (1, torch.int64), (1, torch.int64), (1, torch.int64),
+                (1, torch.int32), (64, torch.int32), (1, torch.int32),
+                (1, torch.int32))]
+            for _ in range(40):
+                ho.sample(logits, 0.1, False, 5, *st, bump_len=True,
+                          temperature=temperature, **kw)
+            got.append(st)
+        for a, b in zip(*got):
+            assert torch.equal(a, b)
+        assert got[0][0].item() == 40
+
+
+def test_shares_of_more_rows_refused(ho):
+    z = [torch.zeros(2, dtype=dt, device="cuda") for dt in (
+        torch.int64, torch.int64, torch.int64, torch.int32, torch.int32,
+        torch.int32, torch.int32, torch.int32)]
+    with pytest.raises(RuntimeError):
+        ho.sample(torch.zeros(2, 64, device="cuda"), 0.1, False, 5, *z[:7],
+                  cnt=z[7], batch=2, tops=torch.zeros(4, device="cuda"))
