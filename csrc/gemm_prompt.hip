@@ -551,9 +551,11 @@ static const GpCost gp_cost[5] = {
      {0.f, 4.f, 3.2f, 3.4f, 1.8f, 0.f, 1.4f, 0.f},
      0.42f, 0.96f, 2.1f, 5e-6f}};
 
+// the tile and split of a product, and what it takes by the numbers
+struct GpPick { int tile, sk; float time; };
+
 template <int T>
-static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
-                         hipStream_t s) {
+static GpPick gp_pick(const GpArgs& a, long part_floats, int ncnt) {
   const int width = a.act >= 0 ? 2 * a.N : a.N;
   const int slabs = (int)(((long)a.K * (T == GP_E4M3 ? 1 : 2) + 127) / 128);
   const GpCost& k = gp_cost[T == GP_MXFP4 ? 4 : T * 2 + (a.act >= 0)];
@@ -593,7 +595,16 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
       }
     }
   }
-  switch (best) {
+  return {best, best_sk, best_t};
+}
+
+template <int T>
+static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
+                         hipStream_t s) {
+  const bool far = T != GP_MXFP4 && a.K > GP_FAR;        // 64x64 alone
+  const GpPick pick = gp_pick<T>(a, part_floats, ncnt);
+  const int best_sk = pick.sk;
+  switch (pick.tile) {
     case 0:
       if constexpr (T == GP_BF16)
         return gp_go<T, 256, 256, 2, 4, 2>(a, best_sk, s);
@@ -653,6 +664,18 @@ extern "C" hipError_t launch_gemm_fp4w(
               (const u16*)bias, (u16*)y, (float*)part, (int*)cnt, M, N, K,
               act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
   return gp_run<GP_MXFP4>(a, part && cnt ? part_floats : 0, ncnt, stream);
+}
+
+// About what a product of bf16 rows takes, us, W bf16 or MXFP4
+extern "C" float gemm_prompt_time(int fp4, int M, int N, int K, int act,
+                                  long part_floats, int ncnt) {
+  GpArgs a = {};
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.act = act;
+  return fp4 ? gp_pick<GP_MXFP4>(a, part_floats, ncnt).time
+             : gp_pick<GP_BF16>(a, part_floats, ncnt).time;
 }
 
 // ---- routed experts --------------------------------------------------------

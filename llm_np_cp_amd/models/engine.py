@@ -570,6 +570,11 @@ class GPUModel(DecodeLoop):
                                    self.act, self.config.rms_norm_eps))
         return chains if all(c.fits() for c in chains) else None
 
+    def _chunk_rows(self, n: int) -> int:
+        """Rows of the chunks that a prompt of n tokens is read in."""
+        return self.PC if self.tp_branch or n <= self.PC else \
+            self._stack.chunk_rows(n, self.PC)
+
     def _read(self, ids: np.ndarray, pos0: int, layer_hook=None) -> None:
         """A chunk of a prompt (int32, up to PC tokens) from position pos0 of
         sequence _pb through all layers; its rows are in b_h."""
@@ -1004,8 +1009,9 @@ class GPUModel(DecodeLoop):
         logits_buf = torch.empty(min(n, self.PC), self.vocab_l,
                                  dtype=torch.bfloat16, device=self.device)
         done = 0
+        rows = self._chunk_rows(n)
         while done < n:
-            M = min(n - done, self.PC)
+            M = min(n - done, rows)
             self._read(ids[done:done + M], pos0 + done)
             self._head_rows(M, logits_buf)
             if done + M == n:
@@ -1055,8 +1061,9 @@ class GPUModel(DecodeLoop):
             raise ValueError(f"sequence {pos0}+{n} exceeds max_seq "
                              f"{self.max_seq}")
         done = 0
+        rows = self._chunk_rows(n)
         while done < n:
-            M = min(n - done, self.PC)
+            M = min(n - done, rows)
             self._read(ids[done:done + M], pos0 + done)
             done += M
         self._lm_head_last(M)
@@ -1456,8 +1463,9 @@ class GPUModel(DecodeLoop):
             raise ValueError(f"prompt {P} fills the {self.max_seq} pool")
         self._pb = b
         done = 0
+        rows = self._chunk_rows(P)
         while done < P:
-            M = min(P - done, self.PC)
+            M = min(P - done, rows)
             self._read(ids[done:done + M], done)
             done += M
         self._lm_head_last(M)

@@ -102,6 +102,7 @@ _SIGS = {
     "stack_forward": [ctypes.c_void_p] + [ctypes.c_int] * 5 +
                      [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2 +
                      [ctypes.c_void_p],
+    "stack_chunk_rows": [ctypes.c_void_p, ctypes.c_int, ctypes.c_int],
     "stack_embed": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 2 +
                    [ctypes.c_void_p],
     "chain_slots": [ctypes.c_void_p] + [ctypes.c_int] * 2,
@@ -706,6 +707,11 @@ class Stack:
             self._at, ids.ctypes.data if host else None,
             None if host else ids.data_ptr(), M, pos0, _stream()),
             "stack_embed")
+
+    def chunk_rows(self, n: int, most: int) -> int:
+        """Rows of the chunks that n rows of a prompt are best read in, at
+        most ``most``."""
+        return lib().stack_chunk_rows(self._at, n, most)
 
     def forward(self, M: int, keys: int, pool: int = 0, first: int = 0,
                 last: int | None = None, rows=None, tiles=None, most: int = 0):
