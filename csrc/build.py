@@ -32,7 +32,7 @@ PKG = os.path.join(ROOT, "llm_np_cp_amd")
 LIBS = {
     "llmops": ["llm_ops.hip", "gemv.hip", "chain.hip", "attn_decode.hip",
                "attn_prefill.hip", "row_gemm.hip", "gemm_prompt.hip",
-               "mid_gemm.hip", "stack.hip", "tape.hip", "xgmi_comm.hip"],
+               "mid_gemm.hip", "head_rows.hip", "stack.hip", "tape.hip", "xgmi_comm.hip"],
     "linear": ["linear.hip"],
     "latent": ["latent_attn.hip"],
     "gqa": ["gqa_attn.hip"],

@@ -418,6 +418,9 @@ class GPUModel(DecodeLoop):
             pairs = PC * (self.nh_l // self.kvh_l)
             self.pack_buf = torch.zeros(
                 3 * PC + 5 * (-(-pairs // 128) + B) + B, **i32)
+            # the heads of its prompts, beside e4m3 weights
+            self.b_parts = torch.zeros(
+                3 * ho.HEAD_ROWS * H if self.fp8 and not self.wq4 else 0, **bf)
             i64 = dict(dtype=torch.int64, device=dev)
             self.bt_qkv = self.b_rqkv[:B]
             self.bt_logits = torch.zeros(B, self.vocab_l, **bf)
@@ -1434,10 +1437,22 @@ class GPUModel(DecodeLoop):
         self._layers_forward(
             M, keys=max(p + n for _, p, n in segs),
             pack=(rows, tiles.view(-1, 5), max(n for _, _, n in segs)))
-        if self.fp8 or self.tp_branch or len(ends) == 1:
+        if len(ends) == 1 or self.wq4 or self.tp_branch or (
+                self.fp8 and self.H % 64):
             for b, r in ends:
                 self._lm_head_last(r + 1)
                 self.bt_logits32[b].copy_(self.b_logits)
+            return
+        if self.fp8:
+            # as rows alone: not rounded to e4m3, W read once for 16
+            for i in range(0, len(ends), ho.HEAD_ROWS):
+                n = min(len(ends) - i, ho.HEAD_ROWS)
+                b = ends[i][0]
+                ho.head_rows(self.b_h, last[i:], self.lm_head_q,
+                             self.lm_head_s, self.bt_logits32[b:b + n], n,
+                             self.g_final, self.b_parts,
+                             eps=self.config.rms_norm_eps,
+                             softcap=self.final_softcap)
             return
         # bf16: a row is the same among others, W is read once for 16
         for i in range(0, len(ends), ho.FEW_ROWS):

@@ -78,6 +78,8 @@ _SIGS = {
                         [ctypes.c_void_p],
     "launch_quant_fp4": [ctypes.c_void_p] * 3 + [ctypes.c_int] * 2 +
                         [ctypes.c_void_p],
+    "launch_head_rows": [ctypes.c_void_p] * 7 + [ctypes.c_int] * 3 +
+                        [ctypes.c_float] * 2 + [ctypes.c_void_p],
     "launch_gemv_fp8_mx": [ctypes.c_void_p] * 3 + [ctypes.c_long] +
                           [ctypes.c_void_p, ctypes.c_long] +
                           [ctypes.c_void_p] * 3 + [ctypes.c_long] +
@@ -589,6 +591,28 @@ def gemv_fp8_mx(Wq: torch.Tensor, scales: torch.Tensor, x: torch.Tensor,
         _ptr(hout), ctypes.c_long(hstride), N, K, B, stage, act,
         ctypes.c_float(eps), out_f32, ctypes.c_float(softcap),
         ctypes.c_float(escale), _stream()), "gemv_fp8_mx")
+
+
+HEAD_ROWS = 16       # rows that head_rows takes
+
+
+def head_rows(x: torch.Tensor, rows: torch.Tensor, Wq: torch.Tensor,
+              scales: torch.Tensor, y: torch.Tensor, M: int, g: torch.Tensor,
+              parts: torch.Tensor, eps: float = 1e-5, softcap: float = 0.0):
+    """y[i] = softcap(norm(x[rows[i]]) Wq^T), M <= HEAD_ROWS rows beside e4m3
+    weights that are not rounded to e4m3 themselves, W streamed once; y fp32.
+    parts: scratch of 3 * HEAD_ROWS * K bf16."""
+    N, K = Wq.shape
+    assert x.is_contiguous() and x.shape[-1] == K and \
+        x.dtype == parts.dtype == torch.bfloat16
+    assert rows.dtype == torch.int32 and rows.numel() >= M
+    assert y.dtype == torch.float32 and y.is_contiguous() and \
+        y.numel() >= M * N and scales.numel() >= N
+    assert parts.numel() >= 3 * HEAD_ROWS * K and g.numel() >= K
+    _check(lib().launch_head_rows(
+        _ptr(x), _ptr(rows), _ptr(g), _ptr(Wq), _ptr(scales), _ptr(parts),
+        _ptr(y), M, N, K, ctypes.c_float(eps), ctypes.c_float(softcap),
+        _stream()), "head_rows")
 
 
 def gemm_fp4w(X: torch.Tensor, Wq4: torch.Tensor, We4: torch.Tensor,
