@@ -975,17 +975,3 @@ extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
   }
   return hipErrorInvalidValue;
 }
-
-// ones in all of words [0, n) of 16 bytes: what is read until it is there
-__global__ void __launch_bounds__(256) k_chain_clear(u4v_* p, long n) {
-  for (long i = blockIdx.x * 256l + threadIdx.x; i < n; i += gridDim.x * 256l)
-    p[i] = u4v_{~0u, ~0u, ~0u, ~0u};
-}
-
-extern "C" hipError_t launch_chain_clear(void* p, long bytes, hipStream_t s) {
-  if (!p || bytes < 16 || bytes % 16) return hipErrorInvalidValue;
-  const long n = bytes / 16, blocks = (n + 255) / 256;
-  hipLaunchKernelGGL(k_chain_clear, dim3(blocks < 1024 ? blocks : 1024),
-                     dim3(256), 0, s, (u4v_*)p, n);
-  return hipGetLastError();
-}

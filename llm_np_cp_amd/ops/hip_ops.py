@@ -110,7 +110,6 @@ _SIGS = {
     "chain_slots": [ctypes.c_void_p] + [ctypes.c_int] * 2,
     "launch_chain": [ctypes.c_void_p] + [ctypes.c_int] * 3 +
                     [ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
-    "launch_chain_clear": [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p],
     "tape_run": [ctypes.c_void_p] + [ctypes.c_int] * 2 +
                 [ctypes.c_void_p] * 2,
     # one-shot xGMI collectives (csrc/xgmi_comm.hip)
@@ -216,7 +215,7 @@ def gemv(W: torch.Tensor, x: torch.Tensor, y: torch.Tensor,
     eidx/wstride/oscale: W of expert *eidx, its result times *oscale; of
     several experts (x [n, K]) the results are added up, with glu they stand
     one after the other (y [n, N/2]).  ones: a buffer filled with ones besides
-    (``chain_clear``).  nt and rpw are kept for callers: the kernel streams
+    (``Chain``).  nt and rpw are kept for callers: the kernel streams
     W past the caches and picks its rows by itself."""
     _gemv(0, W, None, None, W.shape[1], x, y, res, softcap, stage, x2, g,
           act, eps, maxblocks, g2, escale, eidx, wstride, 0, oscale, glu, ones)
@@ -790,11 +789,13 @@ CHAIN_TOP, CHAIN_EXPERTS = 2, 8           # routed experts of a row, of at most
 class Chain:
     """Products that follow each other, in one launch.  ``stages``: of each,
     its weight ``W`` (w, scales, exponents), ``x`` (of an earlier one of them:
-    its y), ``y`` and, where it has them, kind, g, g2, h, hout, add, glu, softcap, as
-    csrc/chain.hip has them; of routed experts, W of all ``experts`` one below
-    the other, ``slot`` from 1, ``route`` and ``top`` with the first, scaled,
-    add2; ``tops``, of the last: the largest of CHAIN_TOPS shares of y.  Every y but the last lies in memory that
-    ``chain_clear`` filled before the step.  Holds what it points to."""
+    its y), ``y`` and, where it has them, kind, g, g2, h, hout, add, glu,
+    softcap, as csrc/chain.hip has them; of routed experts, W of all
+    ``experts`` one below the other, ``slot`` from 1, ``route`` and ``top``
+    with the first, scaled, add2; of the last, ``tops``: the largest of
+    CHAIN_TOPS shares of y.  Every y but the last lies in memory that held
+    ones, all bits of them, before the step (``ones`` of ``gemv``).  Holds
+    what it points to."""
 
     def __init__(self, stages, wt: int, act: int, eps: float):
         self._held = stages
@@ -858,13 +859,6 @@ class Chain:
         _check(lib().launch_chain(
             self._stages, len(self._stages), self.wt, self.act,
             ctypes.c_float(self.eps), limit, _stream()), "chain")
-
-
-def chain_clear(buf: torch.Tensor):
-    """Ones in all of buf: what products of a chain leave is not there yet."""
-    _check(lib().launch_chain_clear(
-        _ptr(buf), buf.numel() * buf.element_size(), _stream()),
-        "chain_clear")
 
 
 # ----------------------------------------------------------------------
