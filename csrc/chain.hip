@@ -21,10 +21,21 @@
 // of, and who needs them reads until none is left.  Every word is written
 // once a step, so no reader meets an old one.
 //
-// All 256 blocks need not run at once.  A wave that has read `limit` times
-// computes what it misses by itself, product by product, in the order of sums
-// of the others (ch_help), and waits for no one: blocks that come late find
-// their work done.  So the launch ends whatever else holds CUs.
+// All 256 blocks need not run at once.  Another stream's kernels may hold CUs,
+// and a block that waits for one that cannot start would hold its own for
+// nothing.  So each block has a word (`claims`) and marks there that it has
+// started; waves that wait in vain for `limit` take over a block that has not,
+// a quarter of its rows each, for all products (ch_unit), and it ends as soon as
+// it starts.  What has started waits for nothing that has not, so the launch
+// ends whatever else holds CUs.  (Beside that, waves whose patience is at an end
+// compute what is missing of anyone's.)
+// It waits a while first, and as long as blocks still start or fewer than half
+// have: CUs come free as others' blocks end, and of two launches of this kind
+// that hold some each, one is to go on.  ms for 200 tokens of a 1B model, alone
+// 117: beside prompts of 2000 rows on another stream 440 (each product in a
+// launch of its own 555; where waves that waited computed whatever was missing,
+// many of them the same, 3150), beside another model's decode 230 to 350 (198;
+// 420 to 890).  With half of its blocks gone a launch of 26 us takes 150.
 //
 // Routed experts are products like the others, of weights that are known once
 // the router has chosen: every block dots its x with the router as it brings
@@ -42,15 +53,16 @@
 //
 // What is in flight is kept small: what x needs queues behind it.  us for a
 // layer's four products, four launches -> here (weights cold):
-//   2048 wide, 8192 in the middle, bf16        32.9 -> 25.7, e4m3 25.7 -> 19.9
-//   3072, 8192, bf16                           46.9 -> 35.9, MXFP4 27.5 -> 24.2
-//   4096, 14336, bf16 83.5 -> 72.9 (6 TB/s), e4m3 49.4 -> 43.5, MXFP4 39.8 -> 31.3
-//   2304, 9216, bf16, two norms                41.9 -> 35.3
-//   3584, 14336, e4m3, two norms               47.6 -> 43.2
-//   3584, 18944, e4m3                          55.1 -> 49.4
-// Of the first: two slots of a loader in flight ahead of the newest 28.1 (one
-// 25.7), weights kept in the caches 27.3, x read 8 bytes a lane 28.3, in
-// copies for each die 29.1, eight waves that multiply 29.4.  With no x to wait
+//   2048 wide, 8192 in the middle, bf16        32.9 -> 26.2, e4m3 25.6 -> 21.3
+//   3072, 8192, bf16                           47.4 -> 36.6, MXFP4 27.8 -> 24.7
+//   4096, 14336, bf16 83.9 -> 76.3 (5.7 TB/s), e4m3 51.8 -> 47.3, MXFP4 39.5 -> 31.5
+//   2304, 9216, bf16, two norms                40.2 -> 36.0
+//   3584, 14336, e4m3, two norms               48.0 -> 44.9
+//   3584, 18944, e4m3                          55.8 -> 51.5
+// Of the first (25.7 before blocks marked their start): two slots of a loader
+// in flight ahead of the newest 28.1, weights kept in the caches 27.3, x read 8
+// bytes a lane 28.3, in copies for each die 29.1, eight waves that multiply
+// 29.4.  With no x to wait
 // for its weights alone take 17.3 (7 TB/s): a hand-over is 2 to 3 us from the
 // last block's sums to the next product's first, and the rings hold 4 us.
 #include <type_traits>
@@ -61,6 +73,8 @@
 typedef unsigned long long ch_u8;
 typedef __bf16 ch_b2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) uint32_t* ch_lp;
+#define CH_LDS_OF(T) const __attribute__((address_space(3))) T
+#define CH_VOL(T) volatile __attribute__((address_space(3))) T
 
 enum { CH_RAW = 0, CH_NORM = 1, CH_NORM2 = 2 };
 #define CH_MAX 6                           // products of a launch
@@ -74,6 +88,15 @@ enum { CH_RAW = 0, CH_NORM = 1, CH_NORM2 = 2 };
 #define CH_NT (64 * CH_NS)
 #define CH_NORM_K (2 * 8 * CH_NT)          // the longest row that is normed
 #define CH_SLOTS 8                         // of a ring, at most
+#define CH_READS 8                         // ahead of a look whether to go on
+#define CH_MINOR 64                        // looks in vain while fewer than half have
+#define CH_PATIENCE 1024                   // and of all
+#define CH_QUIT (1 << 30)                  // in the counters of a block that ends
+// A block's word, of which bits go as things happen: it has started; another
+// has its rows; the host's own, its rows are for others.
+#define CH_STARTED 1u
+#define CH_GIVEN 2u
+#define CH_ABSENT 4u
 #define CH_LDS (160 * 1024 - 4096)         // 4 KB beside it
 
 // A product as the caller gives it.  What is marked (*) is read until it is
@@ -112,6 +135,7 @@ struct ChArgs {
   ChStep st[CH_MAX];
   int n, act, total, slots, xbytes, hbytes, rbytes, limit;
   float eps;
+  uint32_t* claims;      // CH_BLOCKS words that held ones, or null
 };
 
 DEVINL int ch_s(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -136,6 +160,12 @@ DEVINL void ch_done(ch_lp p, int lane) {   // one more wave, its LDS behind it
   if (lane == 0)
     asm volatile("ds_add_u32 %0, %1" :: "v"(p), "v"(1u) : "memory");
 }
+// until n have; whether the block goes on
+template <int NAP> DEVINL bool ch_wait(ch_lp p, int n) {
+  int v;
+  while ((v = ch_get(p)) < n) __builtin_amdgcn_s_sleep(NAP);
+  return v < CH_QUIT;
+}
 template <int N> DEVINL void ch_arrived() {
   asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
 }
@@ -157,8 +187,8 @@ template <bool F32> DEVINL bool ch_there(u4v_ v) {
                       : v[k] < 0xffff0000u && (v[k] & 0xffffu) != 0xffffu);
   return all;
 }
-DEVINL float ch_value(const ChStage& s, const void* y, int n, bool* there) {
-  if (s.y_f32) {
+DEVINL float ch_value(const void* y, int f32, int n, bool* there) {
+  if (f32) {
     const uint32_t v = __hip_atomic_load((const uint32_t*)y + n,
                                          __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
@@ -264,125 +294,178 @@ DEVINL float ch_finish(const ChStage& s, int act, float v, float up, float rn,
   return v + add;
 }
 
-// What is missing of the products ahead of `upto`, by a wave by itself: slow,
-// and the same bits.
+// Rows of product t that are quarter q of block b's, by one wave: every 16 rows
+// four of them, in the order of sums of the waves that multiply, so the same
+// bits.  r1 and rn: the factors of its norms.  hs: the last product's stream,
+// where it stands in LDS alone.  look: only what is not there yet.
 template <int WT>
-DEVINL void ch_help(const ChStep* st, int upto, int start, int lane, int act,
-                    float eps, const int* eid, const float* ew) {
+DEVINL void ch_unit(CH_LDS_OF(ChStep)* st, int t, int b, int q, int lane,
+                    int act, float r1, float rn, CH_LDS_OF(int)* eid,
+                    CH_LDS_OF(float)* ew, CH_LDS_OF(char)* hs, bool look) {
   constexpr int E = gv_e<WT>(), Q = E / 4;
-  for (int t = 0; t < upto; t++) {
-    const ChStep& q = st[t];
-    const ChStage& s = q.s;
-    const int P = s.K / E, C = (P + 63) / 64;
-    // whoever is at a product behind the router's has its choice
-    const int ex = s.slot ? eid[s.slot - 1] : 0;
-    const float scale = s.scaled ? ew[s.slot - 1] : 1.f;
-    const char* const W = (const char*)s.w + ex * s.wstep;
-    const float* const ws = WT == GV_FP8 ? s.ws + ex * s.sstep : nullptr;
-    auto raw = [&](int i) {                // quad i of x
-      const char* p = (const char*)s.x;
-      if (!s.x_f32) return ch_quad(ch_word(p + (size_t)i * 8));
-      union { ch_u8 u[2]; f4v v; } r;
-      r.u[0] = ch_word(p + (size_t)i * 16);
-      r.u[1] = ch_word(p + (size_t)i * 16 + 8);
-      return r.v;
-    };
-    // sums of squares in the order of the waves that bring x
-    auto over_all = [&](auto quad) {
-      float all = 0.f;
-      for (int w = 0; w < CH_NS; w++) {
-        float ss = 0.f;
-        for (int i = w * 64 + lane; i < s.K / 8; i += CH_NT)
-          ss += ch_squares(quad(i * 2), quad(i * 2 + 1));
-        all += wave_reduce_sum(ss);
-      }
-      return rsqrtf(all / (float)s.K + eps);
-    };
-    float r1 = 1.f, rn = 1.f;
-    auto stream = [&](int i) {             // NORM2: the stream behind it
-      const f4v v = raw(i), h = ch_quad(ch_word(s.h + (size_t)i * 4));
-      const f4v g = *(const f4v*)(s.g + i * 4);
-      f4v o;
-#pragma unroll
-      for (int k = 0; k < 4; k++) o[k] = b2f(f2b(v[k] * r1 * g[k] + h[k]));
-      return o;
-    };
-    if (s.kind == CH_NORM) rn = over_all(raw);
-    if (s.kind == CH_NORM2) {
-      r1 = over_all(raw);
-      rn = over_all(stream);
+  ChStep p;
+  for (int i = 0; i < (int)sizeof(p) / 4; i++)
+    ((uint32_t*)&p)[i] = ch_s(((CH_LDS_OF(uint32_t)*)(st + t))[i]);
+  const ChStage& s = p.s;
+  const int K = s.K, N = s.N, rpb = p.rpb, kwl = p.kwl;
+  const int P = K / E, kind = s.kind;
+  const int n0 = b * rpb, nn = min(rpb, N - n0);
+  const bool glu = s.glu, f32 = s.x_f32;
+  // whoever is at a product behind the router's has its choice
+  const int ex = s.slot ? ch_s(eid[s.slot - 1]) : 0;
+  const float scale = s.scaled ? ew[s.slot - 1] : 1.f;
+  const char* const W = (const char*)s.w + ex * s.wstep;
+  const float* const ws = WT == GV_FP8 ? s.ws + ex * s.sstep : nullptr;
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)s.x, 0, K * (f32 ? 4 : 2), 0x00027000);
+  // quads 2i and 2i + 1 of x, by its norm but for the factor behind the product
+  auto pair = [&](int i, f4v* v, bool stream) {
+    if (f32) {
+      union { u4v_ u; f4v f; } a = {ch_fresh(xr, i * 32)},
+                               c = {ch_fresh(xr, i * 32 + 16)};
+      v[0] = a.f;
+      v[1] = c.f;
+      return;
     }
-    auto value = [&](int i) {
-      f4v v = s.kind == CH_NORM2 ? stream(i) : raw(i);
-      if (s.kind != CH_RAW) {
-        const f4v g = *(const f4v*)((s.kind == CH_NORM2 ? s.g2 : s.g) + i * 4);
+    if (kind == CH_NORM2 && !s.h) {        // behind its first norm
+      const u4v_ h = *(CH_LDS_OF(u4v_)*)(hs + i * 16);
+      v[0] = ch_quad(h[0], h[1]);
+      v[1] = ch_quad(h[2], h[3]);
+    } else {
+      const u4v_ a = ch_fresh(xr, i * 16);
+      v[0] = ch_quad(a[0], a[1]);
+      v[1] = ch_quad(a[2], a[3]);
+      if (kind == CH_NORM2) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) v[k] *= g[k];
-      }
-      return v;
-    };
-    auto sum = [&](int row) {              // of a row of W
-      float all = 0.f;
-      for (int kw = 0; kw < 1 << q.kwl; kw++) {
-        float acc = 0.f;
-        for (int cc = 0; cc < q.cols; cc++) {
-          const int col = min((cc << q.kwl) + kw, C - 1);
-          const int pc = (cc << q.kwl) + kw < C ? col * 64 + lane : P;
-          const int at = min(pc, P - 1);
-          f4v x[Q];
-          u4v_ xb = {};
+        for (int j = 0; j < 2; j++) {
+          const f4v h = ch_quad(*(const ch_u8*)(s.h + i * 8 + j * 4));
+          const f4v g = *(const f4v*)(s.g + i * 8 + j * 4);
 #pragma unroll
-          for (int i = 0; i < Q; i++) x[i] = value(at * Q + i);
-          if constexpr (WT == GV_BF16) {
-            union { ch_u8 u[2]; u4v_ v; } b = {{ch_pack_x(x[0]), ch_pack_x(x[1])}};
-            xb = b.v;
-          }
-          const u4v_ w =
-              *((const u4v_*)(W + (size_t)row * P * 16) + at);
-          const uint32_t e =
-              WT == GV_FP4 ? s.we[(size_t)row * (s.K / 32) + at] : 0;
-          ch_dot<WT, 1>(&w, xb, x, &e, pc < P, &acc);
+          for (int k = 0; k < 4; k++)
+            v[j][k] = b2f(f2b(v[j][k] * r1 * g[k] + h[k]));
         }
-        acc += gv_from<2>(acc);
-        acc += gv_from<1>(acc);
-        acc += gv_from<8>(acc);
-        acc += gv_from<12>(acc);
-        all += gv_halves(acc);
-      }
-      return all;
-    };
-    for (int b0 = 0; b0 < s.N; b0 += 64) {
-      // every wave from another place on, so that they share the work
-      const int base = (b0 + start * 64) % ((s.N + 63) / 64 * 64);
-      bool there;
-      ch_value(s, s.y, min(base + lane, s.N - 1), &there);
-      ch_u8 todo = __ballot(!there && base + lane < s.N);
-      while (todo) {
-        const int n = base + __builtin_ctzll(todo);
-        todo &= todo - 1;
-        float add = 0.f, s1 = 1.f, s2 = 1.f;
-        if (s.add) {
-          if (s.own) {
-            bool yes;
-            add = ch_value(st[0].s, s.add, n, &yes);
-          } else {
-            add = b2f(s.add[n]);
-          }
-        }
-        if (s.add2) {
-          bool yes;
-          add += ch_value(st[t - 1].s, s.add2, n, &yes);
-        }
-        if (WT == GV_FP8) {
-          s1 = ws[n];
-          if (s.glu) s2 = ws[s.N + n];
-        }
-        const float v = sum(n), up = s.glu ? sum(s.N + n) : 0.f;
-        const float o = ch_finish<WT>(s, act, v, up, rn, s1, s2, add, scale);
-        if (lane == 0) ch_put(s.y, s.y_f32, n, o);
       }
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (kind == CH_RAW || stream) return;
+    const float* const g = kind == CH_NORM2 ? s.g2 : s.g;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const f4v m = *(const f4v*)(g + i * 8 + j * 4);
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[j][k] *= m[k];
+    }
+  };
+  if (b == 0 && s.hout)
+    for (int i = q * 64 + lane; i < K / 8; i += 256) {
+      f4v v[2];
+      pair(i, v, true);
+      *(ch_u8*)(s.hout + i * 8) = ch_pack(v[0]);
+      *(ch_u8*)(s.hout + i * 8 + 4) = ch_pack(v[1]);
+    }
+  float most = -INFINITY;
+  for (int r0 = q * 4; r0 < nn; r0 += 4 * CH_NS) {
+    const int n = n0 + r0 + lane;
+    const bool mine = lane < 4 && r0 + lane < nn;
+    if (look) {
+      bool there = true;
+      if (mine) ch_value(s.y, s.y_f32, n, &there);
+      if (__all(there)) continue;
+    }
+    // U columns on their way at a time: a read past the L2 takes 6 us here
+    constexpr int U = WT == GV_BF16 ? 4 : WT == GV_FP8 ? 1 : 2;
+    float v = 0.f, up = 0.f;
+    for (int side = 0; side <= glu; side++) {
+      float sum = 0.f;
+      for (int kw = 0; kw < 1 << kwl; kw++) {
+        float acc[4] = {};
+        for (int cc = 0; cc < p.cols; cc += U) {
+          f4v x[U][Q];
+          u4v_ w[U][4];
+          uint32_t e[U][4] = {};
+#pragma unroll
+          for (int j = 0; j < U; j++) {
+            const int at = min((((cc + j) << kwl) + kw) * 64 + lane, P - 1);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const size_t row = n0 + min(r0 + r, nn - 1) + (side ? N : 0);
+              w[j][r] = __builtin_nontemporal_load(
+                  (const u4v_*)(W + row * P * 16) + at);
+              if constexpr (WT == GV_FP4) e[j][r] = s.we[row * P + at];
+            }
+#pragma unroll
+            for (int i = 0; i < Q; i += 2)
+              pair(at * (Q / 2) + i / 2, x[j] + i, false);
+          }
+#pragma unroll
+          for (int j = 0; j < U; j++) {    // nothing behind the row's end
+            u4v_ xb = {};
+            if constexpr (WT == GV_BF16) {
+              union { ch_u8 u[2]; u4v_ v; } o = {
+                  {ch_pack_x(x[j][0]), ch_pack_x(x[j][1])}};
+              xb = o.v;
+            }
+            ch_dot<WT, 4>(w[j], xb, x[j], e[j],
+                          (((cc + j) << kwl) + kw) * 64 + lane < P, acc);
+          }
+        }
+        sum += gv_rows<4>(acc, lane);
+      }
+      (side ? up : v) = sum;
+    }
+    if (!mine) continue;
+    float add = 0.f, s1 = 1.f, s2 = 1.f;
+    bool yes;                              // own: bf16, add2: fp32
+    if (s.add) add = s.own ? ch_value(s.add, 0, n, &yes) : b2f(s.add[n]);
+    if (s.add2) add += ch_value(s.add2, 1, n, &yes);
+    if (WT == GV_FP8) {
+      s1 = ws[n];
+      if (glu) s2 = ws[N + n];
+    }
+    const float o = ch_finish<WT>(s, act, v, up, rn, s1, s2, add, scale);
+    ch_put(s.y, s.y_f32, n, o);
+    most = fmaxf(most, o);
+  }
+  if (s.tops) {
+    most = wave_reduce_max(most);
+    if (lane == 0) s.tops[b * CH_NS + q] = most;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// A block that has not started, for good, or -1; while fewer than half have, -1
+// but for `any`: then another launch of the kind may have most CUs, and it is
+// better that one of the two goes on.  Ends: each turn that fails has seen a bit
+// of a word go.
+DEVINL int ch_adopt(uint32_t* claims, int lane, bool any, int* seen) {
+  for (;;) {
+    uint32_t w[4], free = 0;
+    int cared = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      w[k] = __hip_atomic_load(claims + lane * 4 + k, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+      if ((w[k] & CH_GIVEN) && ((w[k] & CH_STARTED) || !(w[k] & CH_ABSENT)))
+        free |= 1u << k;
+      cared += __builtin_popcountll(__ballot((w[k] & (CH_STARTED | CH_GIVEN)) !=
+                                             (CH_STARTED | CH_GIVEN)));
+    }
+    const ch_u8 some = __ballot(free != 0);
+    const bool more = cared > *seen;       // blocks still come
+    *seen = cared;
+    if (!some || (!any && (more || cared < CH_BLOCKS / 2))) return -1;
+    // every block from another place on
+    const int l0 = blockIdx.x >> 2, k0 = blockIdx.x & 3;
+    const int l = (__builtin_ctzll(some >> l0 | some << (-l0 & 63)) + l0) & 63;
+    const uint32_t f = __builtin_amdgcn_readlane(free, l);
+    const int k = (__builtin_ctz((f >> k0 | f << (4 - k0)) & 15) + k0) & 3;
+    bool got = false;
+    if (lane == l) {
+      uint32_t old = k == 0 ? w[0] : k == 1 ? w[1] : k == 2 ? w[2] : w[3];
+      got = __hip_atomic_compare_exchange_strong(
+          claims + lane * 4 + k, &old, old & ~CH_GIVEN, __ATOMIC_RELAXED,
+          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (__ballot(got)) return l * 4 + k;
   }
 }
 
@@ -431,6 +514,10 @@ k_chain(ChArgs a) {
   __shared__ ChStep st[CH_MAX];
   __shared__ float ssq[4][CH_NS], own[CH_NT];
   __shared__ uint32_t full[CH_NC], freed[CH_NC], xcnt, scnt, sub;
+  // it stays; products whose norms are there; blocks taken over, whether all
+  __shared__ uint32_t stays, ncnt, nothers, closed;
+  __shared__ float norms[CH_MAX][2];         // factors of each product's
+  __shared__ uint8_t others[CH_BLOCKS];
   // routed experts: the router's sums, the choice, what add2 is
   __shared__ float rsum[MOE ? CH_NS : 1][CH_EXPERTS], ew[CH_TOP];
   __shared__ float own2[MOE ? CH_NT : 1];
@@ -446,7 +533,7 @@ k_chain(ChArgs a) {
   char* const ring = hs + a.hbytes + a.rbytes;
 
   if (tid < CH_NC) full[tid] = freed[tid] = 0;
-  if (tid == 0) xcnt = scnt = sub = dots = routed = 0;
+  if (tid == 0) xcnt = scnt = sub = stays = ncnt = nothers = closed = dots = routed = 0;
   {
     typedef const __attribute__((address_space(4))) uint32_t* kp;
     const kp from = (kp)__builtin_amdgcn_kernarg_segment_ptr();
@@ -458,11 +545,14 @@ k_chain(ChArgs a) {
   if (wave < CH_NC) {                      // ---- multiply
     const ch_lp fullp = (ch_lp)&full[wave], freep = (ch_lp)&freed[wave];
     int at = 0, have = 0, u = 0;           // slot, slots told, rounds
-    for (int i = 0; i < a.n; i++) {
-      const ChCur c = ch_take(st, i, WT);
+    // looked at behind the first product (a read past the L2 ahead of x, by
+    // the waves that bring it, held each launch up by 2 us)
+    uint32_t word = ~0u;
+    if (a.claims && tid == 0)
+      word = __hip_atomic_fetch_and(a.claims + blockIdx.x, ~CH_STARTED,
+                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    auto multiply = [&](const ChCur& c) {
       const int kw = wave & ((1 << c.kwl) - 1);
-      while (ch_get((ch_lp)&xcnt) < CH_NS * (i + 1))
-        __builtin_amdgcn_s_sleep(1);
       for (int g = 0; g < c.groups; g++) {
         float acc[4] = {};
         for (int cc = 0; cc < c.cols; cc++) {
@@ -500,6 +590,93 @@ k_chain(ChArgs a) {
           red[((up ? c.rpb : 0) + r0 + lane) * CH_NC + kw] = s;
       }
       ch_done((ch_lp)&scnt, lane);
+    };
+    // A wave that has waited for long goes on below: what it does for others
+    // has registers of its own there (in one loop with the products it cost
+    // each launch 2 to 3 us).
+    int i = 0;
+    for (; i < a.n; i++) {
+      const ChCur c = ch_take(st, i, WT);
+      // The block's rows are another's: all counters say so, what multipliers
+      // and loaders look at behind what outputs wait for.
+      if (i == 1 && wave == 0) {
+        if (~ch_s((int)word) & (CH_GIVEN | CH_ABSENT)) {
+          ch_set((ch_lp)&scnt, CH_QUIT);
+          ch_set((ch_lp)&sub, CH_QUIT);
+          ch_set((ch_lp)&dots, CH_QUIT);
+          ch_set((ch_lp)&routed, CH_QUIT);
+          ch_set((ch_lp)&xcnt, CH_QUIT);
+          return;
+        }
+        ch_set((ch_lp)&stays, 1);
+      }
+      int v, polls = 0;
+      while ((v = ch_get((ch_lp)&xcnt)) < CH_NS * (i + 1)) {
+        if (++polls >= a.limit && ch_get((ch_lp)&stays)) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      if (v >= CH_QUIT) return;
+      if (__builtin_expect(v < CH_NS * (i + 1), 0)) break;
+      if (i == a.n - 1 && wave == 0) ch_set((ch_lp)&closed, 1);
+      multiply(c);
+    }
+    if (__builtin_expect(i == a.n, 1)) {
+      ch_wait<1>((ch_lp)&closed, 1);
+      if (__builtin_expect(!ch_get((ch_lp)&nothers), 1)) return;
+    }
+    // blocks taken over, of which `kept` are as far as this one; looks in vain;
+    // the next of all blocks, where their turn has come
+    int kept = 0, looks = 0, all = CH_BLOCKS, seen = 0;
+    for (; i <= a.n; i++) {
+      // Until x is there (behind the last product: to the end of those taken
+      // over) a quarter of another block's rows, products from t0 on.
+      for (int k = 0, polls = a.limit, had = ch_get((ch_lp)&nothers);;) {
+        int b, t0 = 0;
+        const bool look = all < CH_BLOCKS;
+        if (k < had) {
+          b = ch_s(((CH_VOL(uint8_t)*)others)[k]);
+          if (k < kept) t0 = i - 1;
+          k++;
+        } else if (look) {
+          b = (int)(blockIdx.x + all++ * 101) & (CH_BLOCKS - 1);
+        } else if (i < a.n) {
+          const int v = ch_get((ch_lp)&xcnt);
+          if (v >= CH_QUIT) return;
+          if (v >= CH_NS * (i + 1)) break;
+          __builtin_amdgcn_s_sleep(1);
+          if (++polls < a.limit) continue;
+          // someone's rows are not there
+          polls = a.limit / 4 * 3;
+          had = ch_get((ch_lp)&nothers);
+          if (k < had) continue;
+          b = wave == 0 && a.claims
+                  ? ch_adopt(a.claims, lane, looks >= CH_MINOR, &seen) : -1;
+          if (b >= 0) {
+            if (lane == 0) ((CH_VOL(uint8_t)*)others)[k] = b;
+            ch_set((ch_lp)&nothers, ++had);   // LDS keeps a wave's order
+            polls = a.limit;
+          } else if (++looks > (a.limit == 0 ? 0 : a.claims ? CH_PATIENCE : 8)) {
+            all = 0;
+          }
+          continue;
+        } else {
+          // wave 0 has taken over its last one
+          ch_wait<1>((ch_lp)&closed, 1);
+          had = ch_get((ch_lp)&nothers);
+          if (k < had) continue;
+          break;
+        }
+        ch_wait<1>((ch_lp)&ncnt, i);
+        for (int t = t0; t < i; t++)
+          ch_unit<WT>((CH_LDS_OF(ChStep)*)st, t, b, wave, lane, a.act,
+                      ((CH_VOL(float)*)norms[t])[1],
+                      ((CH_VOL(float)*)norms[t])[0], (CH_LDS_OF(int)*)eid,
+                      (CH_LDS_OF(float)*)ew, (CH_LDS_OF(char)*)hs, look);
+        kept = max(kept, k);
+      }
+      if (i == a.n) break;
+      if (i == a.n - 1 && wave == 0) ch_set((ch_lp)&closed, 1);
+      multiply(ch_take(st, i, WT));
     }
   } else if (wave < CH_NC + CH_NL) {       // ---- load
     const int wv = wave - CH_NC;
@@ -515,8 +692,13 @@ k_chain(ChArgs a) {
         if (u - freedv >= a.slots) {       // none free: wait for the newest
           ch_arrived<0>();
           ch_set(fullp, u);
-          while (u - (freedv = ch_get(freep)) >= a.slots)
+          for (int n = 1; u - (freedv = ch_get(freep)) >= a.slots; n++) {
+            if (!(n & 15) && ch_get((ch_lp)&xcnt) >= CH_QUIT) {
+              ch_set(fullp, CH_QUIT);      // who still multiplies, for nothing
+              return;
+            }
             __builtin_amdgcn_s_sleep(1);
+          }
         }
       }
       bool up;
@@ -553,10 +735,16 @@ k_chain(ChArgs a) {
       pg = 0;
       if (++ps >= a.n) continue;
       if constexpr (MOE)
-        if (ch_s(st[ps].s.slot) && !ch_get((ch_lp)&routed)) {
-          ch_arrived<0>();
-          ch_set(fullp, u + 1);            // all that the router waits for
-          while (!ch_get((ch_lp)&routed)) __builtin_amdgcn_s_sleep(1);
+        if (ch_s(st[ps].s.slot)) {
+          if (!ch_get((ch_lp)&routed)) {
+            ch_arrived<0>();
+            ch_set(fullp, u + 1);          // all that the router waits for
+          }
+          if (!ch_wait<1>((ch_lp)&routed, 1)) {
+            ch_arrived<0>();               // none on its way when a block ends
+            ch_set(fullp, CH_QUIT);
+            return;
+          }
         }
       c = ch_take<MOE>(st, ps, WT, eid);
     }
@@ -565,7 +753,7 @@ k_chain(ChArgs a) {
   } else {                                 // ---- bring x, finish outputs
     __builtin_amdgcn_s_setprio(3);         // what all others wait for
     const int t = tid - 64 * (CH_NC + CH_NL), sw = wave - CH_NC - CH_NL;
-    int limit = a.limit, sums = 0;         // sums: over all of x, so far
+    int sums = 0;                          // over all of x, so far
     auto add_up = [&](float v) {           // one more: this wave's share
       v = wave_reduce_sum(v);
       if (lane == 0) ssq[sums & 3][sw] = v;
@@ -573,14 +761,14 @@ k_chain(ChArgs a) {
       ch_done((ch_lp)&sub, lane);
     };
     auto factor = [&](int K) {             // of the last one
-      while (ch_get((ch_lp)&sub) < CH_NS * sums) __builtin_amdgcn_s_sleep(0);
+      ch_wait<0>((ch_lp)&sub, CH_NS * sums);   // (or others have the rows)
       float v = 0.f;
 #pragma unroll
       for (int k = 0; k < CH_NS; k++)
-        v += ((volatile float*)ssq[(sums - 1) & 3])[k];
+        v += ((CH_VOL(float)*)ssq[(sums - 1) & 3])[k];
       return rsqrtf(v / (float)K + a.eps);
     };
-    float rn = 1.f;
+    float rn = 1.f, r1 = 1.f;
     for (int i = 0; i < a.n; i++) {
       const ChStage& s = st[i].s;
       const int K = ch_s(s.K), skind = ch_s(s.kind);
@@ -678,7 +866,7 @@ k_chain(ChArgs a) {
             for (int j = 0; j < G; j++)
               if (todo >> j & 1 && __all(ch_there<F32>(v[j])))
                 todo &= ~(1u << j);
-            if (todo && ++tries > limit) return false;
+            if (todo && ++tries > CH_READS) return false;
           }
           f4v x[G][V];
 #pragma unroll
@@ -702,7 +890,7 @@ k_chain(ChArgs a) {
           if constexpr (NORMS) {
             if (kind == CH_NORM2) {
               add_up(squares());
-              const float r1 = factor(K);
+              r1 = factor(K);
 #pragma unroll
               for (int j = 0; j < G; j++)
 #pragma unroll
@@ -771,23 +959,29 @@ k_chain(ChArgs a) {
       const std::integral_constant<bool, MOE> moe;
       if (MOE && ch_s(s.same)) ch_done((ch_lp)&xcnt, lane);
       else for (;;) {
-        const bool all =
+        const bool there =
             MOE && route ? K <= 8 * CH_NT ? bring(one, no(), yes(), moe)
                                           : bring(two, no(), yes(), moe)
             : ch_s(s.x_f32)   ? bring(std::integral_constant<int, 7>(), yes(), no(), no())
             : K > CH_NORM_K   ? bring(std::integral_constant<int, 4>(), no(), no(), no())
             : K <= 8 * CH_NT  ? bring(one, no(), yes(), no())
                               : bring(two, no(), yes(), no());
-        if (all) break;
-        ch_help<WT>(st, i, blockIdx.x * CH_NS + sw, lane, a.act, a.eps, eid, ew);
-        limit = min(limit, 8);
+        if (there) break;
+        if (ch_get((ch_lp)&xcnt) >= CH_QUIT) return;
       }
 
       if (!(MOE && ch_s(s.same))) rn = skind == CH_RAW ? 1.f : factor(K);
+      if (sw == 0) {
+        if (lane == 0) {
+          ((CH_VOL(float)*)norms[i])[0] = rn;
+          ((CH_VOL(float)*)norms[i])[1] = r1;
+        }
+        ch_set((ch_lp)&ncnt, i + 1);       // LDS keeps a wave's order
+      }
       if constexpr (MOE) if (route) {
         // Every wave by itself, to the same: probabilities of all experts,
         // the largest of them (the first of equals), by their sum.
-        while (ch_get((ch_lp)&dots) < CH_NS) __builtin_amdgcn_s_sleep(0);
+        if (!ch_wait<0>((ch_lp)&dots, CH_NS)) return;
         const int ne = ch_s(s.experts), top = ch_s(s.top);
         const int e = lane & (CH_EXPERTS - 1);
         auto most = [&](float v) {         // over eight lanes
@@ -797,7 +991,7 @@ k_chain(ChArgs a) {
         };
         float z = 0.f;
 #pragma unroll
-        for (int k = 0; k < CH_NS; k++) z += ((volatile float*)rsum[k])[e];
+        for (int k = 0; k < CH_NS; k++) z += ((CH_VOL(float)*)rsum[k])[e];
         z = e < ne ? z * rn : -INFINITY;
         float p = __expf(z - most(z)), sum = 0.f, pv[CH_TOP];
         if (!(p == p)) p = 0.f;            // an index is one of an expert
@@ -809,18 +1003,17 @@ k_chain(ChArgs a) {
               __builtin_ctz((uint32_t)__ballot(p == pv[j]) & 0xff | 256) & 7;
           if (j < top) sum += pv[j];
           if (e == best) p = -1.f;
-          ((volatile int*)eid)[j] = j < top ? best : 0;
+          ((CH_VOL(int)*)eid)[j] = j < top ? best : 0;
         }
 #pragma unroll
-        for (int j = 0; j < CH_TOP; j++) ((volatile float*)ew)[j] = pv[j] / sum;
+        for (int j = 0; j < CH_TOP; j++) ((CH_VOL(float)*)ew)[j] = pv[j] / sum;
         ch_done((ch_lp)&routed, lane);
         if (t < nn) {
           if (WT == GV_FP8) wsp += (size_t)ch_s(eid[slot - 1]) * s.sstep;
           rest(t);
         }
       }
-      while (ch_get((ch_lp)&scnt) < CH_NC * (i + 1))
-        __builtin_amdgcn_s_sleep(0);
+      if (!ch_wait<0>((ch_lp)&scnt, CH_NC * (i + 1))) return;
       float* const tops = ch_p(s.tops);
       float most = -INFINITY;
       for (int r = t; r < nn; r += CH_NT) {
@@ -898,8 +1091,8 @@ static int ch_plan(ChArgs* a, const ChStage* s, int n, int wt) {
   return a->slots;
 }
 
-// Slots of a ring that these products leave room for: with fewer than two
-// they are not taken.
+// Slots of a ring that these products leave room for: with fewer than two they
+// are not taken.
 extern "C" int chain_slots(const ChStage* s, int n, int wt) {
   ChArgs a = {};
   if (!s || n < 1 || n > CH_MAX || wt < GV_BF16 || wt > GV_FP4) return 0;
@@ -917,12 +1110,15 @@ static hipError_t ch_launch(const ChArgs& a, size_t bytes, hipStream_t s) {
   return hipGetLastError();
 }
 
-// wt as of launch_gemv; limit: reads of a word ahead of computing it.
+// wt as of launch_gemv; limit: how long a wave waits, in steps of some 1.6 us,
+// ahead of looking for blocks that have not started; claims: CH_BLOCKS words of
+// ones, or null.
 extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
-                                   float eps, int limit, hipStream_t stream) {
+                                   float eps, int limit, void* claims,
+                                   hipStream_t stream) {
   ChArgs a = {};
   if (!s || n < 1 || n > CH_MAX || wt < GV_BF16 || wt > GV_FP4 || limit < 0 ||
-      ch_plan(&a, s, n, wt) < 2)
+      (size_t)claims % 16 || ch_plan(&a, s, n, wt) < 2)
     return hipErrorInvalidValue;
   int left = -1;                           // who left the stream in LDS
   int chosen = 0;                          // experts that a router has chosen
@@ -934,6 +1130,8 @@ extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
         return hipErrorInvalidValue;
       chosen = s[i].top;
     }
+    // a block that ends leaves no stream behind, not even a wrong one
+    if (claims && s[i].hout && i < 2) return hipErrorInvalidValue;
     if (!s[i].w || !s[i].x || !s[i].y || (wt == GV_FP8 && !s[i].ws) ||
         (wt == GV_FP4 && !s[i].we) || s[i].kind < CH_RAW ||
         s[i].kind > CH_NORM2 || (s[i].kind != CH_RAW && !s[i].g) ||
@@ -952,7 +1150,7 @@ extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
         // only the first product's outputs are kept, for as many rows
         (s[i].own && (i == 0 || s[i].add != s[0].y || s[0].glu || s[0].y_f32 ||
                       s[i].N != s[0].N || a.st[0].rpb > CH_NT)) ||
-        // help reads a stream from memory
+        // who takes over rows reads a stream from memory, or the last one's
         (s[i].kind == CH_NORM2 && !s[i].h && i != n - 1))
       return hipErrorInvalidValue;
     if (s[i].kind == CH_NORM2) left = i;
@@ -961,7 +1159,8 @@ extern "C" hipError_t launch_chain(const ChStage* s, int n, int wt, int act,
   }
   a.act = act;
   a.eps = eps;
-  a.limit = limit;
+  a.limit = (limit < 1 << 20 ? limit : 1 << 20) * 16;  // looks at LDS
+  a.claims = (uint32_t*)claims;
   const size_t bytes = (size_t)a.xbytes + a.hbytes + a.rbytes +
                        (size_t)a.slots * CH_NC * (wt == GV_FP4 ? 4352 : 4096);
   switch (wt) {

@@ -513,7 +513,8 @@ class GPUModel(DecodeLoop):
         kinds = [(H, torch.bfloat16), (H, torch.bfloat16)] + \
             [(I, act)] * top + [(H, torch.float32)] * (top - 1)
         size = [ho.chain_room(*k) for k in kinds]
-        self.chain_buf = torch.zeros(n * sum(size), dtype=torch.uint8,
+        each = sum(size) + ho.CHAIN_CLAIMS
+        self.chain_buf = torch.zeros(n * each, dtype=torch.uint8,
                                      device=self.device)
         self.chain_h = torch.zeros(n, H, dtype=torch.bfloat16,
                                    device=self.device)
@@ -528,7 +529,7 @@ class GPUModel(DecodeLoop):
 
         chains, h = [], self.b_h[0]
         for i, lw in enumerate(self.layers):
-            at = i * sum(size)
+            at = i * each
             o, dn, *rest = (
                 ho.chain_part(self.chain_buf, at + sum(size[:k]), *v)
                 for k, v in enumerate(kinds))
@@ -570,7 +571,8 @@ class GPUModel(DecodeLoop):
                 st[2:] = more + sums + [down]
             chains.append(ho.Chain(st + [dict(x=dn, **last)],
                                    2 if self.wq4 else int(self.fp8),
-                                   self.act, self.config.rms_norm_eps))
+                                   self.act, self.config.rms_norm_eps,
+                                   self.chain_buf[at + sum(size):at + each]))
         return chains if all(c.fits() for c in chains) else None
 
     def _chunk_rows(self, n: int) -> int:

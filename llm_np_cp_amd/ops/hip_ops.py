@@ -109,7 +109,7 @@ _SIGS = {
                    [ctypes.c_void_p],
     "chain_slots": [ctypes.c_void_p] + [ctypes.c_int] * 2,
     "launch_chain": [ctypes.c_void_p] + [ctypes.c_int] * 3 +
-                    [ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
+                    [ctypes.c_float, ctypes.c_int] + [ctypes.c_void_p] * 2,
     "tape_run": [ctypes.c_void_p] + [ctypes.c_int] * 2 +
                 [ctypes.c_void_p] * 2,
     # one-shot xGMI collectives (csrc/xgmi_comm.hip)
@@ -754,10 +754,12 @@ class Stack:
 # ----------------------------------------------------------------------
 
 CHAIN_RAW, CHAIN_NORM, CHAIN_NORM2 = 0, 1, 2
-# reads of a word that another block is at, about a microsecond each, before
-# a wave computes it by itself: beyond what blocks that run are apart
-CHAIN_LIMIT = 64
+# how long a wave waits for others' words before it looks for blocks that have
+# not started, in steps of some 1.6 us.  ms for 200 tokens beside another
+# stream's prompts and decode: 4 steps 537 and 270, 16 440 and 260, 32 414 and 360
+CHAIN_LIMIT = 16
 CHAIN_BLOCKS = 256
+CHAIN_CLAIMS = CHAIN_BLOCKS * 4           # bytes of a launch's claims
 
 
 def chain_room(n: int, dtype) -> int:
@@ -794,11 +796,14 @@ class Chain:
     ``experts`` one below the other, ``slot`` from 1, ``route`` and ``top``
     with the first, scaled, add2; of the last, ``tops``: the largest of
     CHAIN_TOPS shares of y.  Every y but the last lies in memory that held
-    ones, all bits of them, before the step (``ones`` of ``gemv``).  Holds
-    what it points to."""
+    ones, all bits of them, before the step (``ones`` of ``gemv``), and so
+    does ``claims``, CHAIN_CLAIMS bytes by which waves take over the rows of
+    blocks that find no CU.  Holds what it points to."""
 
-    def __init__(self, stages, wt: int, act: int, eps: float):
-        self._held = stages
+    def __init__(self, stages, wt: int, act: int, eps: float, claims=None):
+        self._held, self._claims = stages, claims
+        assert claims is None or (claims.is_contiguous() and claims.numel() *
+                                  claims.itemsize >= CHAIN_CLAIMS)
         self.wt, self.act, self.eps = wt, act, eps
         self._stages = (_ChainStage * len(stages))()
         f32 = torch.float32
@@ -858,7 +863,8 @@ class Chain:
     def run(self, limit: int = CHAIN_LIMIT):
         _check(lib().launch_chain(
             self._stages, len(self._stages), self.wt, self.act,
-            ctypes.c_float(self.eps), limit, _stream()), "chain")
+            ctypes.c_float(self.eps), limit, _ptr(self._claims) or None,
+            _stream()), "chain")
 
 
 # ----------------------------------------------------------------------

@@ -223,6 +223,55 @@ def test_what_is_missing_is_computed(ho, wt, gemma, H, I, A, Q):
         assert torch.equal(a, b)
 
 
+def claims(ho, absent=()):
+    """A word a block, of ones; without bit 2 it leaves its rows to others."""
+    c = torch.full((ho.CHAIN_BLOCKS,), -1, dtype=torch.int32, device="cuda")
+    c[list(absent)] = ~4
+    return c
+
+
+# blocks that do nothing, as where another stream's kernels hold their CUs:
+# the first (the stream's), the last, half, all but a few, all but one
+@pytest.mark.parametrize("wt", [0, 1, 2])
+@pytest.mark.parametrize("gemma", [False, True])
+@pytest.mark.parametrize("absent", [(), (0,), (255, 7), range(0, 256, 2),
+                                    range(8, 256), range(1, 256)])
+@pytest.mark.parametrize("H,I,A,Q", [(128, 256, 128, 192),
+                                     (1152, 2048, 640, 1290),
+                                     (2304, 2560, 2048, 2310)])
+def test_rows_are_taken_over(ho, wt, gemma, absent, H, I, A, Q):
+    l = Layer(ho, wt, H, I, A, Q, gemma)
+    want = l.run()
+    l.chain._claims = c = claims(ho, absent)
+    for a, b in zip(want, l.run()):
+        assert torch.equal(a, b)
+    # bit 0: it has started; bit 1: another block has its rows
+    assert not (c & 1).any()
+    gone = torch.zeros(256, dtype=torch.bool, device="cuda")
+    gone[list(absent)] = True
+    assert ((c & 2 == 0) == gone).all()
+
+
+@pytest.mark.parametrize("wt", [0, 1, 2])
+@pytest.mark.parametrize("V", [130, 66000])
+def test_outputs_are_taken_over(ho, wt, V):
+    """And the largest of their shares."""
+    l = Layer(ho, wt, 256, 768, 256, V, head=30.0)
+    want = l.run()
+    tops = torch.full((ho.CHAIN_TOPS,), 1e9, device="cuda")
+    l.chain._stages[3].tops = tops.data_ptr()
+    for absent in ((), (1, 255), range(0, 256, 2), range(16, 256)):
+        tops.fill_(1e9)
+        l.chain._claims = claims(ho, absent)
+        for a, b in zip(want, l.run()):
+            assert torch.equal(a, b)
+        per = -(-V // ho.CHAIN_BLOCKS)
+        for b in (0, 1, 2, 64, 255):
+            rows = want[3][b * per:max(b * per, min(V, (b + 1) * per))]
+            assert tops.view(-1, 4)[b].max() == \
+                (rows.max() if rows.numel() else float("-inf"))
+
+
 def test_refused(ho):
     l = Layer(ho, 0, 128, 256, 128, 192)
     long = Layer(ho, 0, 4352, 256, 128, 192)  # a norm of more than 4096
@@ -281,6 +330,45 @@ def test_two_at_a_time(ho):
     for l, w in zip(ls, want):
         for a, b in zip(w, (l.o, l.mid, l.dn, l.qkv)):
             assert torch.equal(a, b)
+
+
+def test_engines_on_two_streams(ho):
+    """Two models at once, each in a thread with a stream of its own: what
+    each answers alone."""
+    import threading
+
+    import llm_np_cp_amd as L
+    from llm_np_cp_amd.io.loader import random_weights
+    from llm_np_cp_amd.models.engine import GPUModel
+
+    ms = []
+    for hidden, dtype in ((1024, "bf16"), (2048, "fp8")):
+        cfg = L.ModelConfig(
+            model_type="llama", vocab_size=512, hidden_size=hidden,
+            intermediate_size=2 * hidden, num_hidden_layers=3,
+            num_attention_heads=8, num_key_value_heads=4, head_dim=128)
+        ms.append(GPUModel(cfg, random_weights(cfg, seed=3), max_seq=700,
+                           dtype=dtype))
+        assert ms[-1]._chains is not None
+
+    def answer(m, to):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(3):
+                ids = m.generate_tokens([3, 1, 4, 1, 5], 200)
+                to.append((ids, m.b_logits.clone()))
+            torch.cuda.synchronize()
+
+    got = [[], [], [], []]
+    for m, to in zip(ms, got):
+        answer(m, to)
+    ts = [threading.Thread(target=answer, args=a) for a in zip(ms, got[2:])]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for alone, beside in zip(got[:2], got[2:]):
+        for (i, z), (j, y) in zip(alone, beside):
+            assert i == j and torch.equal(z, y)
 
 
 class Experts(Layer):
@@ -382,6 +470,17 @@ def test_experts(ho, wt, H, I, E, top):
         for kw in ({}, dict(limit=0)):
             for a, b in zip(first, l.run(**kw)):
                 assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("wt", [0, 1])
+@pytest.mark.parametrize("E,top", [(8, 2), (3, 2), (5, 1)])
+def test_experts_are_taken_over(ho, wt, E, top):
+    l = Experts(ho, wt, 1152, 640, E, top)
+    want = l.run()
+    for absent in ((0,), range(1, 256, 2), range(16, 256)):
+        l.chain._claims = claims(ho, absent)
+        for a, b in zip(want, l.run()):
+            assert torch.equal(a, b)
 
 
 def test_experts_alike(ho):
