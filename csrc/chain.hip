@@ -1091,8 +1091,12 @@ static int ch_plan(ChArgs* a, const ChStage* s, int n, int wt) {
   return a->slots;
 }
 
-// Slots of a ring that these products leave room for: with fewer than two they
-// are not taken.
+// Slots of a ring that these products leave room for.  With fewer than two they
+// are not taken, with two they should not be: us, four launches -> here, 4096
+// wide, as many in the middle as leave 4, 3 and 2 slots:
+//   bf16  36864 168 -> 157, 45056 198 -> 196, 52224 223 -> 250
+//   e4m3  19456 61.7 -> 58.1, 23552 69.1 -> 68.6, 27648 77.7 -> 85.7
+//   MXFP4 17408 46.3 -> 37.2, 21504 49.9 -> 42.9, 25600 54.0 -> 57.3
 extern "C" int chain_slots(const ChStage* s, int n, int wt) {
   ChArgs a = {};
   if (!s || n < 1 || n > CH_MAX || wt < GV_BF16 || wt > GV_FP4) return 0;

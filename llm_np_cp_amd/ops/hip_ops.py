@@ -856,9 +856,10 @@ class Chain:
                 setattr(to, n, _ptr(t) or None)
 
     def fits(self) -> bool:
-        """Whether the sizes are ones that the kernel takes."""
+        """Whether the sizes are ones that the kernel takes, and faster than
+        a launch for each."""
         return lib().chain_slots(self._stages, len(self._stages),
-                                 self.wt) >= 2
+                                 self.wt) >= 3
 
     def run(self, limit: int = CHAIN_LIMIT):
         _check(lib().launch_chain(

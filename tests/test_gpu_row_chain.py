@@ -285,6 +285,19 @@ def test_refused(ho):
         l.chain.run()
 
 
+# the middle that leaves a ring three slots, and two: right but slower than a
+# launch for each product
+@pytest.mark.parametrize("wt,three,two", [(0, 45056, 52224),
+                                          (1, 23552, 27648),
+                                          (2, 21504, 25600)])
+def test_few_slots(ho, wt, three, two):
+    for I, slots in ((three, 3), (two, 2)):
+        l = Layer(ho, wt, 4096, I, 256, 192)
+        assert ho.lib().chain_slots(l.chain._stages, 4, wt) == slots
+        assert l.chain.fits() == (slots == 3)
+        l.check(l.run())
+
+
 def test_values_that_are_no_numbers(ho):
     """inf and NaN go through, and end no wait."""
     for bad in (float("inf"), float("nan")):
