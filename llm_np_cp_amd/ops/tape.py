@@ -5,7 +5,9 @@ native code (csrc/tape.hip) as often as asked.
 through the kernel libraries: the launcher and its arguments, blocks of
 arguments by value.  What it cannot keep makes it return None, and the caller
 captures the step instead: an operation of torch that is no view (new memory
-among them), a launch on another stream.  The addresses are those of the
+among them), a launch on another stream, any other native function but those
+that only answer, an argument that is neither whole number, pointer, block nor
+c_float.  The addresses are those of the
 engine's own buffers, as in a captured graph.
 """
 
@@ -18,6 +20,8 @@ import torch
 from torch.utils._python_dispatch import TorchDispatchMode
 
 INTS, FLOATS = 32, 8
+# native functions that enqueue nothing
+ASKS = frozenset(("row_gemm_plan", "chain_slots", "stack_chunk_rows"))
 _local = threading.local()
 
 
@@ -37,7 +41,9 @@ def _word(v, held) -> int:
         copy = type(obj).from_buffer_copy(obj)
         held.append(copy)
         return ctypes.addressof(copy)
-    return obj.value or 0 if hasattr(obj, "value") else int(v)
+    if obj is v and isinstance(getattr(v, "value", v), (int, type(None))):
+        return v.value or 0
+    raise ValueError(f"an argument that is {v!r}")
 
 
 class Tape:
@@ -56,6 +62,8 @@ class Tape:
         for t, v in zip(fn.argtypes, args):
             if t is ctypes.c_float:
                 floats.append(float(getattr(v, "value", v)))
+            elif t in (ctypes.c_double, ctypes.c_longdouble):
+                raise ValueError(f"{fn.__name__}: a fraction of more bits")
             else:
                 ints.append(_word(v, self._held))
         if len(args) != len(fn.argtypes) or len(ints) > INTS or \
@@ -116,11 +124,15 @@ class _Library:
 
 
 def noted(name: str, fn, recorder=None):
-    """fn, or while this thread records a step and fn launches, fn noted."""
+    """fn, or while this thread records a step and fn launches, fn noted.
+    Work under another name cannot be kept, and then the step is not."""
     recorder = recorder or getattr(_local, "recorder", None)
-    if recorder is None or not name.startswith("launch_"):
+    if recorder is None or name in ASKS:
         return fn
-    return recorder.launch(fn)
+    if name.startswith("launch_"):
+        return recorder.launch(fn)
+    recorder.other = recorder.other or name
+    return fn
 
 
 def library(lib):

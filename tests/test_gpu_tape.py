@@ -98,6 +98,70 @@ def test_what_is_no_launch_is_not_kept(ho):
     assert (c.h == 2.0 ** 5).all()
 
 
+def model(design="dense", **kw):
+    import llm_np_cp_amd as L
+    from llm_np_cp_amd.io.loader import LazyRandomWeights, random_weights
+    from llm_np_cp_amd.models.registry import engine_class
+
+    if design != "dense":
+        cfg = L.preset_config(design)
+        return engine_class(cfg)(cfg, LazyRandomWeights(cfg, seed=3),
+                                 max_seq=256, max_batch=4, **kw)
+    cfg = L.ModelConfig(
+        model_type="llama", vocab_size=512, hidden_size=256,
+        intermediate_size=768, num_hidden_layers=3, num_attention_heads=4,
+        num_key_value_heads=2, head_dim=64)
+    return engine_class(cfg)(cfg, random_weights(cfg, seed=3), max_seq=256,
+                             max_batch=4, **kw)
+
+
+def test_other_work_of_the_library_is_not_kept(ho):
+    """A native call of many launches that has no place on the list."""
+    c, m = Count(ho), model()
+
+    def step():
+        c.step()
+        m._stack.forward(1, keys=1)
+
+    assert ho.record(step) is None
+    assert ho.record(lambda: (c.step(), m._stack.chunk_rows(9, 4))) is not None
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+def test_steps_of_an_engine_are_kept(ho, dtype):
+    """As launches: q, k and v, two a layer and the pick of one row, some a
+    layer of a group; and they go on as a step by itself does."""
+    m = model(dtype=dtype)
+    m.prefill([1, 2, 3])
+    ids = list(m.decode(9))
+    assert type(m._graph).__name__ == "Tape" and len(m._graph) == 3 * 2 + 2
+    m.prefill([1, 2, 3])
+    assert list(m.decode(9, use_graph=False)) == ids
+    m.prefill_batch([[1, 2, 3], [4, 5]])
+    ids = m.decode_batch(9)
+    assert type(m._graph).__name__ == "Tape" and len(m._graph) > 3 * 4
+    m.prefill_batch([[1, 2, 3], [4, 5]])
+    assert (m.decode_batch(9, use_graph=False) == ids).all()
+    m.prefill_row(0, [1, 2, 3])
+    m.prefill_row(1, [4, 5])
+    m.decode_rows(2, 4)
+    (g,) = m._bgraphs.values()
+    assert type(g).__name__ == "Tape"
+
+
+def test_steps_of_a_layer_list_are_kept(ho):
+    m = model("garupel-2k")
+    m.prefill([1, 2, 3])
+    ids = list(m.decode(5))
+    assert type(m._graph).__name__ == "Tape" and len(m._graph) > 40
+    m.prefill([1, 2, 3])
+    assert list(m.decode(5, use_graph=False)) == ids
+    m.prefill_batch([[1, 2, 3], [4, 5]])
+    m.decode_batch(5)
+    assert type(m._graph).__name__ == "Tape" and len(m._graph) > 40
+
+
 def test_only_this_thread_records(ho):
     import threading
     c, d = Count(ho), Count(ho)
