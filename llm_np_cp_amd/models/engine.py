@@ -1370,7 +1370,7 @@ class GPUModel(DecodeLoop):
                              f"{self.max_seq} pool")
         self.reset()
         self.bt_nout.zero_()
-        for segs in self._chunks(lens):
+        for segs in self._chunks(lens, self._chunk_rows):
             if len(segs) > 1:
                 self._read_pack(segs, seqs)
                 continue
@@ -1385,9 +1385,11 @@ class GPUModel(DecodeLoop):
         self._host_lens = lens
         self._batch_n = B
 
-    def _chunks(self, lens):
+    def _chunks(self, lens, rows=None):
         """The prompts in chunks of up to PC rows, each a list of (sequence,
-        first position, rows).  Several prompts share a chunk, so that its
+        first position, rows); a prompt whose chunks are its own in chunks of
+        rows(its length), as it is read elsewhere.  Several prompts share a
+        chunk, so that its
         products have the rows of all: read one by one, 16 prompts of 305 to
         611 rows beside e4m3 weights left tiles half empty and W was streamed
         16 times (with 31 steps behind them 17.5 -> 13.4 ms; six of 167 to
@@ -1402,11 +1404,13 @@ class GPUModel(DecodeLoop):
         chunks, room = [], 0
         for b, n in enumerate(lens):
             alone = apart or (e4m3 and n % self.PC == 1)
+            own = rows and (alone or len(lens) == 1)
+            most = rows(n) if own else self.PC
             done = 0
             while done < n:
                 if alone or room == 0:
                     chunks.append([])
-                    room = self.PC
+                    room = most
                 M = min(n - done, room)
                 if e4m3 and not alone and n - done - M == 1:
                     M, room = M - 1, M - 1

@@ -6,7 +6,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def engine(family="llama", hidden=2304, dtype="bf16", **more):
+def engine(family="llama", hidden=2304, dtype="bf16", max_batch=1, **more):
     import llm_np_cp_amd as L
     from llm_np_cp_amd.io.loader import random_weights
     from llm_np_cp_amd.models.engine import GPUModel
@@ -18,7 +18,7 @@ def engine(family="llama", hidden=2304, dtype="bf16", **more):
         num_key_value_heads=4, head_dim=256,
         hidden_act="gelu_pytorch_tanh" if gemma else "silu", **more)
     return GPUModel(cfg, random_weights(cfg, seed=3), max_seq=4200,
-                    dtype=dtype)
+                    dtype=dtype, max_batch=max_batch)
 
 
 @pytest.mark.parametrize("kind", [
@@ -57,3 +57,17 @@ def test_the_same_prompt(kind):
     for other in got[1:]:
         assert np.linalg.norm(other - got[0]) < \
             2.0 ** -6 * np.linalg.norm(got[0])
+
+
+@pytest.mark.parametrize("kind", [dict(), dict(dtype="fp4"),
+                                  dict(dtype="fp8")])
+def test_the_same_by_each_entry_point(kind):
+    """A long prompt alone: prefill, a row of a pool, a group of one."""
+    m = engine(max_batch=2, **kind)
+    ids = np.arange(3001) * 7 % 512
+    _, want = m.prefill(ids)
+    want = want.copy()
+    m.prefill_batch([ids])
+    assert np.array_equal(m.bt_logits32[0].cpu().numpy(), want)
+    m.prefill_row(1, ids)
+    assert np.array_equal(m.b_logits.cpu().numpy(), want)

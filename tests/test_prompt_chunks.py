@@ -9,9 +9,9 @@ from llm_np_cp_amd.models.engine import GPUModel
 from llm_np_cp_amd.ops import hip_ops as ho
 
 
-def chunks(lens, PC=64, fp8=False, wq4=False, hd=64):
+def chunks(lens, PC=64, fp8=False, wq4=False, hd=64, rows=None):
     m = types.SimpleNamespace(PC=PC, fp8=fp8, wq4=wq4, hd=hd)
-    return GPUModel._chunks(m, lens)
+    return GPUModel._chunks(m, lens, rows)
 
 
 @pytest.mark.parametrize("kind", [{}, {"fp8": True},
@@ -55,6 +55,21 @@ def test_a_row_by_itself_whatever_its_neighbours(PC):
         assert seen == lens
         assert single == [(b, p) for b, n in enumerate(lens)
                           for p in range(0, n, PC) if n - p == 1 or PC == 1]
+
+
+def test_a_long_prompt_with_chunks_of_its_own():
+    """In the chunks that it is read in without a group."""
+    def rows(n):
+        return 64 if n <= 64 else 48
+
+    def cut(b, n, most):
+        return [[(b, p, min(most, n - p))] for p in range(0, n, most)]
+
+    for n in (1, 64, 65, 100, 200):
+        assert chunks([n], rows=rows) == cut(0, n, rows(n))
+        assert chunks([n, 70], hd=80, rows=rows) == \
+            cut(0, n, rows(n)) + cut(1, 70, 48)
+        assert chunks([n, 70], rows=rows) == chunks([n, 70])
 
 
 @pytest.mark.parametrize("group", [1, 3, 7])
