@@ -419,6 +419,7 @@ class GPUModel(DecodeLoop):
             self.pack_buf = torch.zeros(
                 3 * PC + 5 * (-(-pairs // 128) + B) + B, **i32)
             # the heads of its prompts, beside e4m3 weights
+            self.b_row0 = torch.zeros(1, **i32)
             self.b_parts = torch.zeros(
                 3 * ho.HEAD_ROWS * H if self.fp8 and not self.wq4 else 0, **bf)
             i64 = dict(dtype=torch.int64, device=dev)
@@ -1378,8 +1379,7 @@ class GPUModel(DecodeLoop):
             self._pb = b
             self._read(seqs[b][done:done + M], done)
             if done + M == lens[b]:
-                self._lm_head_last(M)
-                self.bt_logits32[b].copy_(self.b_logits)
+                self._heads([(b, M - 1)], B)
         self._pb = 0
         self.bt_lens[:B].copy_(torch.tensor(lens, dtype=torch.int32))
         self._host_lens = lens
@@ -1443,21 +1443,33 @@ class GPUModel(DecodeLoop):
         self._layers_forward(
             M, keys=max(p + n for _, p, n in segs),
             pack=(rows, tiles.view(-1, 5), max(n for _, _, n in segs)))
-        if len(ends) == 1 or self.wq4 or self.tp_branch or (
-                self.fp8 and self.H % 64):
+        self._heads(ends, len(seqs), last)
+
+    def _heads(self, ends, B: int, last=None) -> None:
+        """The logits of sequences b whose last row is r, `ends` of them (b,
+        r), of a group of B; last: the r, int32 on the device."""
+        if self.wq4 or self.tp_branch or B == 1 or (
+                self.H % 64 if self.fp8 else len(ends) == 1):
             for b, r in ends:
                 self._lm_head_last(r + 1)
                 self.bt_logits32[b].copy_(self.b_logits)
             return
         if self.fp8:
-            # as rows alone: not rounded to e4m3, W read once for 16
+            # Not rounded to e4m3, W read once for 16.  By itself a row's sums
+            # would go in another order, so a single one of a group goes here
+            # too (40 us instead of 22, 32768x3584): its logits do not depend
+            # on which prompts end beside it.  A prompt without a group has
+            # the product of one row.
+            x = self.b_h
+            if last is None:
+                (_, r), = ends
+                x, last = x[r:r + 1], self.b_row0
             for i in range(0, len(ends), ho.HEAD_ROWS):
                 n = min(len(ends) - i, ho.HEAD_ROWS)
                 b = ends[i][0]
-                ho.head_rows(self.b_h, last[i:], self.lm_head_q,
-                             self.lm_head_s, self.bt_logits32[b:b + n], n,
-                             self.g_final, self.b_parts,
-                             eps=self.config.rms_norm_eps,
+                ho.head_rows(x, last[i:], self.lm_head_q, self.lm_head_s,
+                             self.bt_logits32[b:b + n], n, self.g_final,
+                             self.b_parts, eps=self.config.rms_norm_eps,
                              softcap=self.final_softcap)
             return
         # bf16: a row is the same among others, W is read once for 16

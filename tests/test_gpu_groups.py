@@ -134,3 +134,26 @@ def test_prompts_read_together(family, kv, more, dtype):
         bound = 2.0 ** -4 if dtype == "fp8" else 2.0 ** -6
         assert (got[b] - want).norm() < bound * want.norm(), b
     assert m.bt_lens.tolist() == [len(p) for p in prompts]
+
+
+# more prompts end in a chunk than a launch of heads takes, two, and one by
+# itself: a row's logits beside e4m3 weights do not depend on its neighbours
+@pytest.mark.parametrize("family", ["llama", "gemma2"])
+def test_heads_whatever_the_neighbours(family):
+    rng = np.random.default_rng(1)
+    prompts = [rng.integers(0, 256, size=2 + b % 3) for b in range(19)]
+    full = rng.integers(0, 256, size=64)
+    m = engine(family, hidden=128, max_batch=19, dtype="fp8",
+               prefill_chunk=64, max_seq=80)
+    m.prefill_batch(prompts)
+    together = m.bt_logits32[:19].clone()
+    for b, p in enumerate(prompts):
+        for group in ([p, prompts[0]], [prompts[3], p], [full, p]):
+            at = 0 if group[0] is p else 1
+            if group[0] is full:              # p in a chunk of its own
+                assert [len(c) for c in m._chunks([64, len(p)])] == [1, 1]
+            m.prefill_batch(group)
+            assert torch.equal(m.bt_logits32[at], together[b]), b
+        m.prefill_row(0, p)                   # one row's sums, in their order
+        off = (m.b_logits - together[b]).norm() / together[b].norm()
+        assert off < 128 * 2.0 ** -23, b
