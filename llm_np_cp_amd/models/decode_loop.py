@@ -97,9 +97,9 @@ class DecodeLoop:
                         greedy: bool = True, min_p: float = 0.1,
                         eos_id=None, chunk: int = 16, on_ids=None,
                         temperature: float = 1.0, stop_fn=None):
-        """Fast generate: device-side decode in chunks (of 256 where nobody
-        looks at tokens in between), host
-        sees ids every `chunk` tokens (streaming + EOS stop).  Used by
+        """Fast generate: device-side decode in chunks, host sees ids every
+        `chunk` tokens (streaming + EOS stop; every 256 by default where there
+        is neither callback, end token nor stop function).  Used by
         runtime.generate() for greedy/min-p on GPU models.
         ``eos_id`` may be an int or a collection of ints (HF configs
         often store a list, e.g. Llama-3.2-Instruct).  ``stop_fn``
@@ -116,9 +116,9 @@ class DecodeLoop:
         eos_set = (set() if eos_id is None else
                    {int(eos_id)} if np.isscalar(eos_id) else
                    {int(e) for e in eos_id})
-        # nobody looks at the tokens in between
-        if not (eos_set or on_ids or stop_fn):
-            chunk = max(chunk, 256)
+        # nobody looks at the tokens in between, nor asked for another size
+        if chunk == 16 and not (eos_set or on_ids or stop_fn):
+            chunk = 256
         t0 = _time.perf_counter()
         with trace_range("prefill"):
             self.prefill(prompt_ids)

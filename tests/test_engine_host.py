@@ -5,9 +5,11 @@ import os
 import re
 import types
 
+import numpy as np
 import pytest
 import torch
 
+from llm_np_cp_amd.models import decode_loop
 from llm_np_cp_amd.models import engine as eng
 
 
@@ -105,3 +107,30 @@ def test_experts_there_are_rows_for(monkeypatch, listed, rows, glu, taken):
     idx, p = torch.zeros(listed, dtype=torch.int32), torch.zeros(listed)
     ho.gemv(W, x, y, eidx=idx, wstride=N * K, oscale=p, glu=glu)
     assert args[0][22] == taken and args[0][10] == N and args[0][11] == K
+
+
+class Loop(decode_loop.DecodeLoop):
+    max_seq = 1000
+
+    def __init__(self):
+        self.sizes = []
+
+    def prefill(self, ids):
+        pass
+
+    def decode(self, n, **kw):
+        self.sizes.append(n)
+        return np.arange(n)
+
+
+@pytest.mark.parametrize("kw,sizes", [
+    (dict(), [256, 44]), (dict(chunk=8), [8] * 37 + [4]),
+    (dict(chunk=100), [100, 100, 100]), (dict(chunk=300), [300]),
+    (dict(on_ids=lambda ids: None), [16] * 18 + [12]),
+    (dict(eos_id=999), [16] * 18 + [12]),
+    (dict(eos_id=[999], chunk=150), [150, 150]),
+    (dict(stop_fn=lambda ids: len(ids) >= 40), [16] * 3)])
+def test_tokens_are_fetched_in_the_chunks_asked_for(kw, sizes):
+    m = Loop()
+    assert len(m.generate_tokens([1, 2], 300, **kw)) == sum(sizes)
+    assert m.sizes == sizes
