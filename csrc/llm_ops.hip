@@ -1551,7 +1551,8 @@ k_moe_route(const u16* __restrict__ h, const float* __restrict__ g,
     for (int w = 1; w < 64; w <<= 1) x = fmaxf(x, __shfl_xor(x, w));
     return x;
   };
-  float p = lane < E ? __expf(v - most(v)) : 0.f;
+  const float top = most(v);          // by all lanes, also those without one
+  float p = lane < E ? __expf(v - top) : 0.f;
   if (!(p == p)) p = 0.f;             // an index is one of an expert, whatever
   if (dense && lane < E) dense[(size_t)m * E + lane] = 0.f;
   // top-k by repeated argmax (ties -> smallest index, matching the

@@ -713,6 +713,24 @@ def test_router_of_rows_without_a_number(E, top, bad):
     assert off(w[good], p / p.sum(1, keepdim=True)) < 2.0 ** -16
 
 
+# a wave has an expert a lane: numbers that leave a butterfly of lanes short
+@pytest.mark.parametrize("E", [1, 2, 3, 5, 6, 7, 9, 10, 12, 17, 33, 60, 63])
+def test_router_of_any_number_of_experts(E):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    M, H, top = 40, 192, min(3, E)
+    h, g = normal(M, H, seed=1), torch.ones(H, device="cuda")
+    wg = normal(E, H, seed=2)
+    idx = torch.full((M, top), -9, dtype=torch.int32, device="cuda")
+    w = torch.zeros(M, top, device="cuda")
+    ho.moe_route(h, g, wg, M, top, idx, w)
+    x = h.double()
+    z = (x * torch.rsqrt(x.pow(2).mean(1, keepdim=True) + 1e-5)) @ wg.double().T
+    p, i = torch.softmax(z, 1).topk(top, 1)
+    assert (idx.long() == i).all()
+    assert off(w, p / p.sum(1, keepdim=True)) < 2.0 ** -16
+
+
 # a thread has 16 values of a head (of 24: one at a time); rows that end
 # inside a block; a head's threads that are no power of two
 @pytest.mark.parametrize("hd,nh,kvh", [(16, 4, 2), (24, 2, 1), (48, 3, 1),
