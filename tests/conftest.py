@@ -21,6 +21,13 @@ def pytest_configure(config):
 
 
 def pytest_collection_modifyitems(config, items):
+    # The eight streams of the comm tests need a hardware queue each, and
+    # streams get theirs in turn as they are first used: behind tests that
+    # use streams of their own two of the eight may share one, and ranks that
+    # spin for each other on it time out.  So these tests go first, whatever
+    # the files are called.
+    items.sort(key=lambda i: os.path.basename(str(i.fspath)) !=
+               "test_gpu_comm.py")
     try:
         import torch
         has_gpu = torch.cuda.is_available()

@@ -31,7 +31,8 @@ def _ho():
 # must be co-resident, and HIP maps streams round-robin onto a bounded
 # set of hardware queues (GPU_MAX_HW_QUEUES, raised in conftest.py) — a
 # fresh 8 streams per test would eventually collide two spinners onto
-# one queue and serialize them into a timeout.
+# one queue and serialize them into a timeout.  So would streams that other
+# tests used before: conftest.py puts this file's tests first.
 _STREAMS = []
 
 
