@@ -685,7 +685,6 @@ k_chain(ChArgs a) {
     ChCur c = ch_take(st, 0, WT);
     // slots that have arrived are told as the next one is asked for: one in
     // flight behind the newest
-    __builtin_amdgcn_s_sleep(12);          // x of the first product goes ahead
     for (int u = 0; u < a.total; u++) {
       if (u - freedv >= a.slots) {
         freedv = ch_get(freep);
