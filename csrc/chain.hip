@@ -25,16 +25,16 @@
 // and a block that waits for one that cannot start would hold its own for
 // nothing.  So each block has a word (`claims`) and marks there that it has
 // started; waves that wait in vain for `limit` take over a block that has not,
-// a quarter of its rows each, for all products (ch_unit), and it ends as soon as
-// it starts.  What has started waits for nothing that has not, so the launch
-// ends whatever else holds CUs.  (Beside that, waves whose patience is at an end
-// compute what is missing of anyone's.)
+// a quarter of its rows each, for all products (ch_unit), and it does nothing
+// where it starts at last.  What has started waits for nothing that has not, so
+// the launch ends whatever else holds CUs.  (Beside that, waves whose patience
+// is at an end compute what is missing of anyone's.)
 // It waits a while first, and as long as blocks still start or fewer than half
 // have: CUs come free as others' blocks end, and of two launches of this kind
 // that hold some each, one is to go on.  ms for 200 tokens of a 1B model, alone
-// 117: beside prompts of 2000 rows on another stream 440 (each product in a
+// 117: beside prompts of 2000 rows on another stream 460 (each product in a
 // launch of its own 555; where waves that waited computed whatever was missing,
-// many of them the same, 3150), beside another model's decode 230 to 350 (198;
+// many of them the same, 3150), beside another model's decode 230 to 280 (198;
 // 420 to 890).  With half of its blocks gone a launch of 26 us takes 150.
 //
 // Routed experts are products like the others, of weights that are known once
@@ -53,18 +53,22 @@
 //
 // What is in flight is kept small: what x needs queues behind it.  us for a
 // layer's four products, four launches -> here (weights cold):
-//   2048 wide, 8192 in the middle, bf16        32.9 -> 26.2, e4m3 25.6 -> 21.3
-//   3072, 8192, bf16                           47.4 -> 36.6, MXFP4 27.8 -> 24.7
-//   4096, 14336, bf16 83.9 -> 76.3 (5.7 TB/s), e4m3 51.8 -> 47.3, MXFP4 39.5 -> 31.5
-//   2304, 9216, bf16, two norms                40.2 -> 36.0
-//   3584, 14336, e4m3, two norms               48.0 -> 44.9
-//   3584, 18944, e4m3                          55.8 -> 51.5
-// Of the first (25.7 before blocks marked their start): two slots of a loader
-// in flight ahead of the newest 28.1, weights kept in the caches 27.3, x read 8
-// bytes a lane 28.3, in copies for each die 29.1, eight waves that multiply
-// 29.4.  With no x to wait
-// for its weights alone take 17.3 (7 TB/s): a hand-over is 2 to 3 us from the
-// last block's sums to the next product's first, and the rings hold 4 us.
+//   2048 wide, 8192 in the middle, bf16        32.9 -> 25.7, e4m3 25.5 -> 20.5
+//   3072, 8192, bf16                           47.3 -> 36.5, MXFP4 28.0 -> 24.3
+//   4096, 14336, bf16 83.7 -> 76.3 (5.7 TB/s), e4m3 51.7 -> 46.5, MXFP4 39.3 -> 31.7
+//   2304, 9216, bf16, two norms                40.2 -> 35.5
+//   3584, 14336, e4m3, two norms               48.2 -> 43.6
+//   3584, 18944, e4m3                          55.6 -> 50.5
+// Of the first: two slots of a loader in flight ahead of the newest 28.1,
+// weights kept in the caches 27.3, x read 8 bytes a lane 28.3, in copies for
+// each die 29.1, eight waves that multiply 29.4.  With no x to wait for its
+// weights alone take 17.3 (7 TB/s): a hand-over is 2 to 3 us from the last
+// block's sums to the next product's first, and the rings hold 4 us.
+//
+// The waves that bring x have one way through: a return where others have the
+// block's rows, out of their reads or ahead of an output, cost each launch 0.5
+// us and 0.4 to 0.9; with the standing in in the same loop as the products it
+// was 2 to 3, out of line 0.3 to 2.5.
 #include <type_traits>
 
 #include "common.h"
@@ -88,7 +92,6 @@ enum { CH_RAW = 0, CH_NORM = 1, CH_NORM2 = 2 };
 #define CH_NT (64 * CH_NS)
 #define CH_NORM_K (2 * 8 * CH_NT)          // the longest row that is normed
 #define CH_SLOTS 8                         // of a ring, at most
-#define CH_READS 8                         // ahead of a look whether to go on
 #define CH_MINOR 64                        // looks in vain while fewer than half have
 #define CH_PATIENCE 1024                   // and of all
 #define CH_QUIT (1 << 30)                  // in the counters of a block that ends
@@ -597,10 +600,17 @@ k_chain(ChArgs a) {
     int i = 0;
     for (; i < a.n; i++) {
       const ChCur c = ch_take(st, i, WT);
-      // The block's rows are another's: all counters say so, what multipliers
-      // and loaders look at behind what outputs wait for.
+      // The block's rows are another's: multipliers and loaders end, and the
+      // others go through what is left without waiting or writing.  All
+      // counters say so, what the former look at behind what the latter do.
       if (i == 1 && wave == 0) {
         if (~ch_s((int)word) & (CH_GIVEN | CH_ABSENT)) {
+          if (lane < a.n) {                // what waits and writes besides
+            st[lane].s.wait = 0;
+            st[lane].s.hout = nullptr;
+            st[lane].s.tops = nullptr;
+          }
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
           ch_set((ch_lp)&scnt, CH_QUIT);
           ch_set((ch_lp)&sub, CH_QUIT);
           ch_set((ch_lp)&dots, CH_QUIT);
@@ -683,8 +693,12 @@ k_chain(ChArgs a) {
     const ch_lp fullp = (ch_lp)&full[wv], freep = (ch_lp)&freed[wv];
     int ps = 0, pg = 0, pc = 0, at = 0, freedv = 0;
     ChCur c = ch_take(st, 0, WT);
-    // slots that have arrived are told as the next one is asked for: one in
-    // flight behind the newest
+    // Slots that have arrived are told as the next one is asked for: one in
+    // flight behind the newest.
+    // x of the first product ahead of weights that are soon through: us a launch
+    // at once, after 6 and 12 x 64 cycles, e4m3 1B 20.9, 20.5, 20.2, 8B 46.4, 46.2,
+    // 46.4, bf16 1B 25.7, 26.1, 26.3.
+    if constexpr (WT == GV_FP8) __builtin_amdgcn_s_sleep(6);
     for (int u = 0; u < a.total; u++) {
       if (u - freedv >= a.slots) {
         freedv = ch_get(freep);
@@ -856,7 +870,7 @@ k_chain(ChArgs a) {
             for (int j = 0; j < G; j++) v[j] = ((const u4v_*)src)[piece(j)];
           // what the other blocks are still at is not there at once
           if (wait && b0 == 0) __builtin_amdgcn_s_sleep(12);
-          for (int tries = 0; todo;) {
+          while (todo) {
             asm volatile("" ::: "memory");  // read again each time
 #pragma unroll
             for (int j = 0; j < G; j++)
@@ -865,7 +879,6 @@ k_chain(ChArgs a) {
             for (int j = 0; j < G; j++)
               if (todo >> j & 1 && __all(ch_there<F32>(v[j])))
                 todo &= ~(1u << j);
-            if (todo && ++tries > CH_READS) return false;
           }
           f4v x[G][V];
 #pragma unroll
@@ -949,25 +962,21 @@ k_chain(ChArgs a) {
             if (NORMS && kind != CH_RAW) add_up(ss);
           }
         }
-        return true;
       };
       using yes = std::true_type;
       using no = std::false_type;
       const std::integral_constant<int, 1> one;
       const std::integral_constant<int, 2> two;
+      const std::integral_constant<int, 4> four;
+      const std::integral_constant<int, 7> seven;
       const std::integral_constant<bool, MOE> moe;
       if (MOE && ch_s(s.same)) ch_done((ch_lp)&xcnt, lane);
-      else for (;;) {
-        const bool there =
-            MOE && route ? K <= 8 * CH_NT ? bring(one, no(), yes(), moe)
-                                          : bring(two, no(), yes(), moe)
-            : ch_s(s.x_f32)   ? bring(std::integral_constant<int, 7>(), yes(), no(), no())
-            : K > CH_NORM_K   ? bring(std::integral_constant<int, 4>(), no(), no(), no())
-            : K <= 8 * CH_NT  ? bring(one, no(), yes(), no())
-                              : bring(two, no(), yes(), no());
-        if (there) break;
-        if (ch_get((ch_lp)&xcnt) >= CH_QUIT) return;
-      }
+      else if (MOE && route) K <= 8 * CH_NT ? bring(one, no(), yes(), moe)
+                                            : bring(two, no(), yes(), moe);
+      else if (ch_s(s.x_f32)) bring(seven, yes(), no(), no());
+      else if (K > CH_NORM_K) bring(four, no(), no(), no());
+      else K <= 8 * CH_NT ? bring(one, no(), yes(), no())
+                          : bring(two, no(), yes(), no());
 
       if (!(MOE && ch_s(s.same))) rn = skind == CH_RAW ? 1.f : factor(K);
       if (sw == 0) {
@@ -980,7 +989,7 @@ k_chain(ChArgs a) {
       if constexpr (MOE) if (route) {
         // Every wave by itself, to the same: probabilities of all experts,
         // the largest of them (the first of equals), by their sum.
-        if (!ch_wait<0>((ch_lp)&dots, CH_NS)) return;
+        ch_wait<0>((ch_lp)&dots, CH_NS);
         const int ne = ch_s(s.experts), top = ch_s(s.top);
         const int e = lane & (CH_EXPERTS - 1);
         auto most = [&](float v) {         // over eight lanes
@@ -998,8 +1007,8 @@ k_chain(ChArgs a) {
 #pragma unroll
         for (int j = 0; j < CH_TOP; j++) {
           pv[j] = most(p);
-          const int best =
-              __builtin_ctz((uint32_t)__ballot(p == pv[j]) & 0xff | 256) & 7;
+          const int best = min(
+              __builtin_ctz((uint32_t)__ballot(p == pv[j]) & 0xff | 256), ne - 1);
           if (j < top) sum += pv[j];
           if (e == best) p = -1.f;
           ((CH_VOL(int)*)eid)[j] = j < top ? best : 0;
@@ -1012,10 +1021,11 @@ k_chain(ChArgs a) {
           rest(t);
         }
       }
-      if (!ch_wait<0>((ch_lp)&scnt, CH_NC * (i + 1))) return;
-      float* const tops = ch_p(s.tops);
+      // nothing to finish where the block's rows are another's
+      const int mine = ch_wait<0>((ch_lp)&scnt, CH_NC * (i + 1)) ? nn : 0;
+      float* const tops = ch_p(((CH_VOL(ChStep)*)st)[i].s.tops);
       float most = -INFINITY;
-      for (int r = t; r < nn; r += CH_NT) {
+      for (int r = t; r < mine; r += CH_NT) {
         if (r != t) rest(r);
         const f4v p = *(const f4v*)&red[r * CH_NC];
         const f4v o = *(const f4v*)&red[((glu ? rpb : 0) + r) * CH_NC];

@@ -756,7 +756,7 @@ class Stack:
 CHAIN_RAW, CHAIN_NORM, CHAIN_NORM2 = 0, 1, 2
 # how long a wave waits for others' words before it looks for blocks that have
 # not started, in steps of some 1.6 us.  ms for 200 tokens beside another
-# stream's prompts and decode: 4 steps 537 and 270, 16 440 and 260, 32 414 and 360
+# stream's prompts and decode: 4 steps 537 and 270, 16 460 and 260, 32 414 and 360
 CHAIN_LIMIT = 16
 CHAIN_BLOCKS = 256
 CHAIN_CLAIMS = CHAIN_BLOCKS * 4           # bytes of a launch's claims
