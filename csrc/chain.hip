@@ -696,9 +696,10 @@ k_chain(ChArgs a) {
     // Slots that have arrived are told as the next one is asked for: one in
     // flight behind the newest.
     // x of the first product ahead of weights that are soon through: us a launch
-    // at once, after 6 and 12 x 64 cycles, e4m3 1B 20.9, 20.5, 20.2, 8B 46.4, 46.2,
-    // 46.4, bf16 1B 25.7, 26.1, 26.3.
-    if constexpr (WT == GV_FP8) __builtin_amdgcn_s_sleep(6);
+    // at once, after 6 and 12 x 64 cycles, MXFP4 1B 20.0, 18.6, 18.4, 8B 32.4,
+    // 32.1, 32.4, e4m3 1B 20.9, 20.5, 20.2, 8B 46.4, 46.3, 46.7, bf16 1B 25.7,
+    // 26.1, 26.3.
+    if constexpr (WT != GV_BF16) __builtin_amdgcn_s_sleep(6);
     for (int u = 0; u < a.total; u++) {
       if (u - freedv >= a.slots) {
         freedv = ch_get(freep);
