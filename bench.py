@@ -6,7 +6,7 @@ weights, bf16.  Default model is Llama-3.2-1B at
 EVERY N (TP=N) so the driver's 1/2/4/8-GPU curve compares like with
 like; the metric's second config (Gemma-2-9B TP=8, fp8) runs via
 ``--model gemma-2-9b --dtype fp8``.  A "step" is one decoded token; the
-timed region is K hipGraph-replayed decode steps (full forward incl.
+timed region is K replayed decode steps (full forward incl.
 lm_head + sampling).
 
 Usage: python bench.py [--gpus N] [--steps K] [--warmup W] [--model M]

@@ -27,7 +27,7 @@
 // 4.3 us at no history, 128 dims.  us, blocks a head apart and two fixed
 // ranges (as before) -> here:
 //   32/8 heads of 64, 90 keys 7.6 -> 4.6; 4000 keys 22.2 -> 10.0
-//   32/8 of 128, 6040 e4m3 keys 39.2 -> 14.1; 160 keys 9.8 -> 6.4
+//   32/8 of 128, 6040 e4m3 keys 39.2 -> 13.5; 160 keys 9.8 -> 6.4
 //   16/8 of 256, 16 sequences of 620 keys, softcap 52.3 -> 25.4 (two ranges)
 //   64/8 of 128, 4 sequences of 2000 keys 97 -> 23
 //   16/4 of 128, 32000 keys 131 -> 38 (1.7 TB/s: few blocks, long ranges)
@@ -414,7 +414,7 @@ __global__ void __launch_bounds__(64 * AD_NW) k_attn_dec_any(AdArgs a) {
 }
 
 // eight e4m3 numbers as bf16, exact (by way of fp32 and f2b, as keys went
-// before, 6040 of 32/8 heads of 128 took 16.6 us, 15.2 like this)
+// before, 6040 of 32/8 heads of 128 took 1.4 us longer)
 DEVINL s8v ad_widen(unsigned long long v) {
   union { ad_b2 p[4]; s8v s; } w;
 #pragma unroll

@@ -90,7 +90,10 @@ enum { CH_RAW = 0, CH_NORM = 1, CH_NORM2 = 2 };
 #define CH_NL CH_NC
 #define CH_NS 4
 #define CH_NT (64 * CH_NS)
-#define CH_NORM_K (2 * 8 * CH_NT)          // the longest row that is normed
+// The longest row that is normed.  Its pieces are in registers until the sum of
+// squares is there, with the norm's weights and, behind two norms, the stream's
+// and theirs: two pieces a thread.  Four (4608, 8192 wide) were not built.
+#define CH_NORM_K (2 * 8 * CH_NT)
 #define CH_SLOTS 8                         // of a ring, at most
 #define CH_MINOR 64                        // looks in vain while fewer than half have
 #define CH_PATIENCE 1024                   // and of all

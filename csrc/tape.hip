@@ -2,16 +2,25 @@
 //
 // A step is the same launches each time, its state on the device.  As a graph
 // it runs without gaps inside, but 8 us pass between one graph's last kernel
-// and the next one's first, and a first pass paid 1 to 2 ms for the capture.
-// Called again from here a launch takes the host 3 us, less than its kernel
-// runs (4 to 80), and the stream never runs dry.  us a step, a graph each ->
-// launch by launch (graphs of four steps):
-//   6 launches, 4096 wide MXFP4, 2 layers        99.3 ->  96.8 ( 95.9)
-//   14 launches, experts                        128.1 -> 126.4 (124.7)
-//   64 launches, layer list, 4 rows             391.4 -> 387.0 (387.8)
-//   34 launches, 2048 wide bf16, 16 layers      558.6 -> 564 to 566 (564.1)
-// Four steps a graph are half a percent less, and 0.2 to 0.5 ms of a first
-// pass more.
+// and the next one's first, and a first pass pays for the capture.  Called again
+// from here a launch takes the host 3 us; it makes them while earlier ones run
+// (kernels take 4 to 80) and waits for none.  us a step, a graph each -> launch
+// by launch, and what the first two steps of a pass take, ms:
+//   6 launches, 4096 wide MXFP4, 2 layers           97.8 ->   94.3   0.77 -> 0.40
+//   21, 9B e4m3, 2 layers, 16 rows                 211.2 ->  204.5   1.20 -> 0.88
+//   18, 8B e4m3, 8 layers                          457.7 ->  454.0   1.68 -> 1.08
+//   66, 8B e4m3, 32 layers                        1734.2 -> 1730.5   4.87 -> 3.73
+//   83, 1B bf16, 16 layers, 16 rows                901.5 ->  895.1   3.61 -> 2.85
+//   143, 7B bf16, 28 layers, 6 rows               3024.6 -> 3018.4   8.12 -> 6.32
+//   381, 9B e4m3, 42 layers, 16 rows              3601.1 -> 3597.2  12.44 -> 11.97
+//   64, layer list, 4 rows                         391.2 ->  387.4   2.23 -> 1.69
+//   45, layer list, one row                        372.5 ->  374.7   2.03 -> 1.32
+//   34, 1B bf16, 16 layers, one row                557.9 ->  562.0   2.00 -> 1.30
+// So all are made from here.  The last two lose 0.6% of a step and are behind
+// once a pass has made some 300 and 170 of them; the others gain at any depth.
+// The device depends on the host's thread for it, which is in C for all steps
+// of a call.  Graphs of several steps are no faster and take 0.2 to 0.7 ms more
+// to capture.
 #include "common.h"
 
 // A launcher with its arguments.  Numbers and pointers go in eight bytes

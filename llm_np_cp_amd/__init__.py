@@ -4,8 +4,8 @@ A from-scratch re-design of the capabilities of ``githubpradeep/llm_np_cp``
 (single-file Llama-3.2 / Gemma-2 inference: HF safetensors loader,
 ``generate()`` with per-token streaming, KV cache, min-p sampling) built
 MI355X-first: hand-written HIP/CDNA4 (gfx950) kernels for the whole
-forward pass, PyTorch-ROCm tensors as memory containers, decode
-without the host, tensor parallelism over RCCL/xGMI, fp8/MXFP4 weight paths.
+forward pass, PyTorch-ROCm tensors as memory containers, decode steps
+that wait for no host result, tensor parallelism over RCCL/xGMI, fp8/MXFP4 weight paths.
 
 Families: Llama-3.x, Gemma-2, Qwen-2.5, Mistral, Mixtral sparse MoE.
 
