@@ -310,8 +310,10 @@ DEVINL void ch_unit(CH_LDS_OF(ChStep)* st, int t, int b, int q, int lane,
                     CH_LDS_OF(float)* ew, CH_LDS_OF(char)* hs, bool look) {
   constexpr int E = gv_e<WT>(), Q = E / 4;
   ChStep p;
+  uint32_t words[sizeof(p) / 4];
   for (int i = 0; i < (int)sizeof(p) / 4; i++)
-    ((uint32_t*)&p)[i] = ch_s(((CH_LDS_OF(uint32_t)*)(st + t))[i]);
+    words[i] = ch_s(((CH_LDS_OF(uint32_t)*)(st + t))[i]);
+  __builtin_memcpy(&p, words, sizeof(p));
   const ChStage& s = p.s;
   const int K = s.K, N = s.N, rpb = p.rpb, kwl = p.kwl;
   const int P = K / E, kind = s.kind;
@@ -377,7 +379,9 @@ DEVINL void ch_unit(CH_LDS_OF(ChStep)* st, int t, int b, int q, int lane,
       if (mine) ch_value(s.y, s.y_f32, n, &there);
       if (__all(there)) continue;
     }
-    // U columns on their way at a time: a read past the L2 takes 6 us here
+    // U columns on their way at a time: a read past the L2 takes some 6 us while
+    // weights stream (200 tokens of 1B bf16 beside another stream's prompts 446
+    // ms, a column at a time 472; e4m3 alike)
     constexpr int U = WT == GV_BF16 ? 4 : WT == GV_FP8 ? 1 : 2;
     float v = 0.f, up = 0.f;
     for (int side = 0; side <= glu; side++) {
