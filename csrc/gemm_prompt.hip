@@ -2,13 +2,13 @@
 // e4m3 with row scales, or bf16 rows beside MXFP4 weights; fp32 sums, bf16
 // out.
 //
-// Slabs of 128 bytes a row (64 bf16, 128 e4m3) go straight into LDS, two to
-// six buffers, one barrier a slab that waits for the next slab only and
-// leaves the DMA behind it in flight.  That wait is what bounds these
-// products (a slab is back from L2 or memory after one to two microseconds,
-// the matrix cores want one a microsecond): with every DMA drained at each
-// barrier 2048x4096x14336 ran at 1030 TFLOP/s in bf16 and 870 in e4m3, with
-// 128x256 tiles and three buffers it runs at 1160 and 2180.
+// Slabs of 128 bytes a row (64 bf16, 128 e4m3) go straight into LDS.  What
+// bounds these products is the way there: a slab is back from L2 or memory
+// after one to two microseconds, the matrix cores want one a microsecond, and
+// a CU gets 45 to 55 GB/s from its L2 and what is behind it.  So tiles are as
+// large as fits, and loads stay in flight across the barriers.  Tiles 256 wide
+// are k_gemm_wide's; the others have two to six buffers and one barrier a slab
+// that waits for the next slab only.
 //
 // Rows are XOR-swizzled by 16-byte slots; the DMA writes lane-linear, so the
 // swizzle sits in the address that a lane reads and in the fragment reads.
@@ -54,13 +54,21 @@ struct GpArgs {
   u16* y;              // [M, N]
   float* part;         // split K: [tile, split, BM*BN]
   int* cnt;            // split K: blocks of a tile that are done
-  int M, N, K, act, tm, tn;
+  int M, N, K, act, tm, tn, band;
   // Routed experts: a row tile has n[t] rows of expert e[t]; row r of it is
   // pair perm[row0[t] + r].  x by token (a pair / top) and y in that order
   // (gather), or x in that order and y by pair.
   const int *perm, *tile_e, *tile_row0, *tile_n;
   int top, gather;
 };
+
+// Row and column of a tile: bands of rows of tiles, rows fastest in each.
+struct GpAt { int row, col; };
+DEVINL GpAt gp_at(const GpArgs& a, int tile) {
+  const int all = a.band * a.tn, b = tile / all, r = tile - b * all;
+  const int h = min(a.band, a.tm - b * a.band);
+  return {b * a.band + r % h, r / h};
+}
 
 // gate_act with tanh by exp: an epilogue has some hundred of them a lane
 DEVINL float gp_act(float x, int act) {
@@ -79,6 +87,123 @@ template <int N> DEVINL void gp_meet() {
   asm volatile("" ::: "memory");
 }
 
+// The sums of a tile on their way out: parts of K meet, scales, the gate, bias,
+// residual.  Fragment (i, j) of a wave holds rows row_of(i) + (lane & 15) and
+// outputs col_of(j) + (lane >> 4) * 4 + 0..3 of the tile.
+template <bool F8, int BM, int BN, int NW, int FM, int FN, bool GLU, bool MOE,
+          bool SPLIT, class RowOf, class ColOf, class XRow>
+DEVINL void gp_finish(const GpArgs& a, f4v (&acc)[FM][FN], int tile, int part,
+                      int SK, int bm, int bn, int rows, int first, const int* perm, size_t w0,
+                      int* last_flag, RowOf row_of, ColOf col_of, XRow x_row) {
+  const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fk = lane >> 4;
+  if (SPLIT && SK > 1) {
+    // fragments as they lie in registers: the last block reads them alike
+    float* pp = a.part + (size_t)tile * SK * (BM * BN) + tid * 4;
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++)
+        part_put4(pp + (size_t)part * (BM * BN) +
+                  (i * FN + j) * (NW * 256), acc[i][j]);
+    if (!last_block(&a.cnt[tile], SK, last_flag)) return;
+    // up to 16 fragments of a part on the way at a time: a part a trip, not
+    // a fragment of one
+    constexpr int G = FM * FN > 16 ? 16 / FN : FM;
+#pragma unroll
+    for (int i0 = 0; i0 < FM; i0 += G) {
+#pragma unroll
+      for (int i = 0; i < G; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) acc[i0 + i][j] = {0.f, 0.f, 0.f, 0.f};
+      for (int q = 0; q < SK; q++) {
+        f4v t[G][FN];
+#pragma unroll
+        for (int i = 0; i < G; i++)
+#pragma unroll
+          for (int j = 0; j < FN; j++)
+            t[i][j] = part_get4(pp + (size_t)q * (BM * BN) +
+                                ((i0 + i) * FN + j) * (NW * 256));
+#pragma unroll
+        for (int i = 0; i < G; i++)
+#pragma unroll
+          for (int j = 0; j < FN; j++) acc[i0 + i][j] += t[i][j];
+      }
+    }
+  }
+
+  constexpr int P = GLU ? 2 : 1;
+  const bool wide = a.N % 4 == 0;
+  // e4m3 scales, all asked for ahead of the stores, behind which each would
+  // be waited for (2048x14336x3584 with a gate 285 us, so 273)
+  [[maybe_unused]] float sx[FM], sv[FN / P][4], su[FN / P][4];
+  if constexpr (F8) {
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+      sx[i] = a.sx[x_row(min(bm + row_of(i) + fr, rows - 1))];
+#pragma unroll
+    for (int j = 0; j < FN / P; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int n = min(bn + col_of(j * P) / P + fk * 4 + r, a.N - 1);
+        sv[j][r] = a.sw[w0 + n];
+        if (GLU) su[j][r] = a.sw[w0 + a.N + n];
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < FM; i++) {
+    const int r_in = bm + row_of(i) + fr;
+    if (r_in >= rows) continue;
+    const int row = !MOE ? r_in : a.gather ? first + r_in : perm[r_in];
+#pragma unroll
+    for (int j = 0; j < FN; j += P) {
+      const int n = bn + col_of(j) / P + fk * 4;
+      if (n >= a.N) continue;
+      f4v v = acc[i][j];
+      if (F8) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] *= sx[i] * sv[j / P][r];
+      }
+      if constexpr (GLU) {
+        f4v u = acc[i][j + 1];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          if (F8) {
+            // to be rounded to e4m3 next, where a value's last bits decide
+            // which of two it takes: from bf16 halves, as by single launches
+            u[r] = (float)(__bf16)(u[r] * sx[i] * su[j / P][r]);
+            v[r] = (float)(__bf16)v[r];
+          }
+          v[r] = gp_act(v[r], a.act) * u[r];
+        }
+      }
+      const size_t at = (size_t)row * a.N + n;
+      if (wide) {
+        union { gp_b2 b[2]; u16 h[4]; unsigned long long q; } o;
+        if (a.bias) {
+          o.q = *(const unsigned long long*)(a.bias + n);
+#pragma unroll
+          for (int r = 0; r < 4; r++) v[r] += b2f(o.h[r]);
+        }
+        if (a.res) {
+          o.q = *(const unsigned long long*)(a.res + at);
+#pragma unroll
+          for (int r = 0; r < 4; r++) v[r] += b2f(o.h[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) o.b[r / 2][r % 2] = (__bf16)v[r];
+        *(unsigned long long*)(a.y + at) = o.q;
+      } else {
+        for (int r = 0; r < 4 && n + r < a.N; r++) {
+          float f = v[r];
+          if (a.bias) f += b2f(a.bias[n + r]);
+          if (a.res) f += b2f(a.res[at + r]);
+          a.y[at + r] = f2b(f);
+        }
+      }
+    }
+  }
+}
+
 template <bool F8, int BM, int BN, int WM, int WN, int NS, bool GLU,
           bool MOE = false, bool W4 = false, bool FAR = false>
 __global__ void __launch_bounds__(64 * WM * WN)
@@ -87,9 +212,6 @@ k_gemm_prompt(GpArgs a) {
   constexpr int FM = BM / WM / 16, FN = BN / WN / 16;   // fragments of a wave
   constexpr int AI = BM / 8 / NW, BI = BN / 8 / NW;     // DMA of a wave
   static_assert(AI > 0 && BI > 0 && FM > 0 && FN % (GLU ? 2 : 1) == 0);
-  // The K of the largest tile is not split: the epilogue that adds
-  // parts would cost the former two spilled registers.
-  constexpr bool SPLIT = BM * BN < 256 * 256;
   // loads of a wave for a slab (MXFP4: a piece of W and its exponent)
   constexpr int PS = W4 ? AI + 2 : AI + BI;
   // An array a buffer, and the loop unrolled over them: the compiler sees
@@ -112,14 +234,15 @@ k_gemm_prompt(GpArgs a) {
   const int tiles = a.tm * a.tn, chunk = (tiles + 7) / 8;
   const int tile = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= chunk || tile >= tiles) return;
-  const int bm = MOE ? 0 : tile % a.tm * BM;
-  const int bn = tile / a.tm * (GLU ? BN / 2 : BN);
+  const GpAt at = gp_at(a, tile);
+  const int bm = MOE ? 0 : at.row * BM;
+  const int bn = at.col * (GLU ? BN / 2 : BN);
   // the rows of a tile that are there
-  const int rows = MOE ? a.tile_n[tile % a.tm] : a.M;
+  const int rows = MOE ? a.tile_n[at.row] : a.M;
   if (MOE && rows == 0) return;
-  const int* perm = MOE ? a.perm + a.tile_row0[tile % a.tm] : nullptr;
-  const int first = MOE ? a.tile_row0[tile % a.tm] : 0;
-  const size_t w0 = MOE ? (size_t)a.tile_e[tile % a.tm] * (GLU ? 2 : 1) * a.N
+  const int* perm = MOE ? a.perm + a.tile_row0[at.row] : nullptr;
+  const int first = MOE ? a.tile_row0[at.row] : 0;
+  const size_t w0 = MOE ? (size_t)a.tile_e[at.row] * (GLU ? 2 : 1) * a.N
                         : 0;                 // first row of the expert's W
   auto x_row = [&](int r) {
     if (!MOE) return r;
@@ -136,8 +259,8 @@ k_gemm_prompt(GpArgs a) {
   const int g_r = lane >> 3, g_s = lane & 7;
   // Where a lane's rows lie behind the tile's first: 32 bits beside a base in
   // scalar registers (an expert's rows of x are anywhere; beside MXFP4 weights
-  // a launch takes 0.35 us longer so).  With 64-bit addresses the 256x256 tiles
-  // spill.  FAR: rows so long that 32 bits are not enough.
+  // a launch takes 0.35 us longer so).  FAR: rows so long that 32 bits are not
+  // enough.
   typedef typename std::conditional<MOE || W4 || FAR, size_t, uint32_t>::type
       Off;
   const char* const x_at = (const char*)a.x + (MOE ? 0 : (size_t)bm * rowb);
@@ -257,7 +380,7 @@ k_gemm_prompt(GpArgs a) {
             wb[j].q[0] = *(const u4v_*)(cb + j * 2048 + x0);
             wb[j].q[1] = *(const u4v_*)(cb + j * 2048 + x1);
           }
-          // block scales of one (e8m0 127): the row scales come at the end
+          // no block scales: the row scales come at the end
 #pragma unroll
           for (int i = 0; i < FM; i++) {
             union { u4v_ q[2]; gp_i8 v; } xa;
@@ -266,8 +389,7 @@ k_gemm_prompt(GpArgs a) {
 #pragma unroll
             for (int j = 0; j < FN; j++)
               acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                  wb[j].v, xa.v, acc[i][j], 0, 0, 0, 0x7f7f7f7f, 0,
-                  0x7f7f7f7f);
+                  wb[j].v, xa.v, acc[i][j], 0, 0, 0, 0, 0, 0);
           }
         } else {
 #pragma unroll
@@ -361,125 +483,286 @@ k_gemm_prompt(GpArgs a) {
     }
   }
 
-  if (SPLIT && SK > 1) {
-    // fragments as they lie in registers: the last block reads them alike
-    float* pp = a.part + (size_t)tile * SK * (BM * BN) + tid * 4;
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-      for (int j = 0; j < FN; j++)
-        part_put4(pp + (size_t)blockIdx.y * (BM * BN) +
-                  (i * FN + j) * (NW * 256), acc[i][j]);
-    if (!last_block(&a.cnt[tile], SK, &last_flag)) return;
-    // up to 16 fragments of a part on the way at a time: a part a trip, not
-    // a fragment of one
-    constexpr int G = FM * FN > 16 ? 16 / FN : FM;
-#pragma unroll
-    for (int i0 = 0; i0 < FM; i0 += G) {
-#pragma unroll
-      for (int i = 0; i < G; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) acc[i0 + i][j] = {0.f, 0.f, 0.f, 0.f};
-      for (int q = 0; q < SK; q++) {
-        f4v t[G][FN];
-#pragma unroll
-        for (int i = 0; i < G; i++)
-#pragma unroll
-          for (int j = 0; j < FN; j++)
-            t[i][j] = part_get4(pp + (size_t)q * (BM * BN) +
-                                ((i0 + i) * FN + j) * (NW * 256));
-#pragma unroll
-        for (int i = 0; i < G; i++)
-#pragma unroll
-          for (int j = 0; j < FN; j++) acc[i0 + i][j] += t[i][j];
-      }
-    }
-  }
+  gp_finish<F8, BM, BN, NW, FM, FN, GLU, MOE, true>(
+      a, acc, tile, blockIdx.y, SK, bm, bn, rows, first, perm, w0, &last_flag,
+      [&](int i) { return (wm * FM + i) * 16; },
+      [&](int j) { return (wn * FN + j) * 16; }, x_row);
+}
 
-  // fragment (i, j): row i*16 + fr, outputs j*16 + fk*4 + 0..3
-  constexpr int P = GLU ? 2 : 1;
-  const bool wide = a.N % 4 == 0;
-  // e4m3 scales, all asked for ahead of the stores, behind which each would
-  // be waited for (2048x14336x3584 with a gate 285 us, so 273)
-  [[maybe_unused]] float sx[FM], sv[FN / P][4], su[FN / P][4];
-  if constexpr (F8) {
+// Tiles 256 wide, by two groups of four waves that take turns: while one has
+// the matrix cores, the other brings its next operands from LDS and asks for
+// slabs to come.
+//
+// A slab comes in pieces of 128 rows of 128 bytes: two of W (B0, B1) and HA of
+// X (A0, A1), read and asked for in the order B0, A0, B1, A1.  Pieces lie in a
+// ring of nine.  A turn is 64 rows by 32 outputs of a wave's tile, 16
+// products: it brings what the next products need, asks for pieces where both
+// groups have theirs in registers, waits for the pieces that the turn after it
+// reads, with all those behind them still in flight, and meets the others
+// twice, ahead of its products and behind them.  The groups are one meeting
+// apart.
+//
+// A block takes tile after tile, and the pieces that are asked for are those
+// of the next tile where a tile ends: none waits for its first slabs but the
+// first.  Behind the last one loads go on, to one line, so that the waits
+// count alike.
+#define GW_RING 9
+DEVINL void gw_load(const char* base, uint32_t off, uint32_t lds) {
+  // 64 lanes of 16 bytes to lds and behind it
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+               "global_load_lds_dwordx4 %1, %0"
+               :: "s"(base), "v"(off), "s"(lds) : "memory");
+}
+DEVINL void gw_meet() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+// LDS reads are over, and all loads but the last N
+template <int N> DEVINL void gw_wait() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | 7 << 4);
+  asm volatile("" ::: "memory");
+}
+
+template <bool F8, int HA, bool GLU>
+__global__ void __launch_bounds__(512) k_gemm_wide(GpArgs a, int SK) {
+  constexpr int BM = 128 * HA, BN = 256, FM = 4 * HA, FN = 4;
+  __shared__ __attribute__((aligned(16))) char ring[GW_RING * 16384];
+  __shared__ int last_flag;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  // Work of an XCD (block id modulo 8): neighbouring tiles, rows fastest, in
+  // each part of K.  A block takes every step-th item of it.
+  const int tiles = a.tm * a.tn, chunk = (tiles + 7) / 8, items = chunk * SK;
+  const int step = gridDim.x >> 3, t0 = (blockIdx.x & 7) * chunk;
+  auto there = [&](int k) {                  // the next item from k on
+    while (k < items && t0 + k % chunk >= tiles) k += step;
+    return k;
+  };
+  int item = there(blockIdx.x >> 3);
+  if (item >= items) return;
+
+  const size_t rowb = (size_t)a.K * (F8 ? 1 : 2);       // bytes of a row
+  const int slabs = (int)((rowb + 127) / 128), per = (slabs + SK - 1) / SK;
+
+  // ---- what is asked for: a slab of an item, then the next one ----
+  const int g_r = lane >> 3, g_s = lane & 7;
+  // row r of a piece keeps slot q at q ^ ((r >> 1) & 7)
+  const uint32_t src = (g_s ^ (g_r >> 1)) * 16;
+  const char *xp, *wp;
+  uint32_t pa[HA][2], pb[2][2];
+  int ahead = item, left, adv = 128;
+  auto aim = [&] {
+    left = 1 << 30;
+    if (ahead >= items) {                    // no more: one line of each
+      adv = 0;
+      xp = (const char*)a.x;
+      wp = (const char*)a.w;
 #pragma unroll
-    for (int i = 0; i < FM; i++)
-      sx[i] = a.sx[x_row(min(bm + (wm * FM + i) * 16 + fr, rows - 1))];
+      for (int t = 0; t < 2; t++) {
 #pragma unroll
-    for (int j = 0; j < FN / P; j++)
+        for (int h = 0; h < HA; h++) pa[h][t] = 0;
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int n = min(bn + (wn * FN / P + j) * 16 + fk * 4 + r, a.N - 1);
-        sv[j][r] = a.sw[w0 + n];
-        if (GLU) su[j][r] = a.sw[w0 + a.N + n];
+        for (int h = 0; h < 2; h++) pb[h][t] = 0;
       }
-  }
+      return;
+    }
+    const int tile = t0 + ahead % chunk, lo = ahead / chunk * per;
+    left = min(per, slabs - lo);
+    const GpAt at = gp_at(a, tile);
+    const int bm = at.row * BM, bn = at.col * (GLU ? BN / 2 : BN);
+    xp = (const char*)a.x + (size_t)bm * rowb + (size_t)lo * 128;
+    // 16 rows of the gate, 16 of what it gates
+    wp = (const char*)a.w + (size_t)bn * rowb + (size_t)lo * 128 +
+         (GLU && (wave & 1) ? (size_t)a.N * rowb : 0);
 #pragma unroll
-  for (int i = 0; i < FM; i++) {
-    const int r_in = bm + (wm * FM + i) * 16 + fr;
-    if (r_in >= rows) continue;
-    const int row = !MOE ? r_in : a.gather ? first + r_in : perm[r_in];
+    for (int t = 0; t < 2; t++) {
+      const int r = (wave * 2 + t) * 8 + g_r;
+      const uint32_t o = t ? src ^ 64 : src;
 #pragma unroll
-    for (int j = 0; j < FN; j += P) {
-      const int n = bn + (wn * FN + j) / P * 16 + fk * 4;
-      if (n >= a.N) continue;
-      f4v v = acc[i][j];
-      if (F8) {
+      for (int h = 0; h < HA; h++)
+        pa[h][t] = (uint32_t)min(h * 128 + r, a.M - 1 - bm) * (uint32_t)rowb + o;
 #pragma unroll
-        for (int r = 0; r < 4; r++) v[r] *= sx[i] * sv[j / P][r];
-      }
-      if constexpr (GLU) {
-        f4v u = acc[i][j + 1];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          if (F8) {
-            // to be rounded to e4m3 next, where a value's last bits decide
-            // which of two it takes: from bf16 halves, as by single launches
-            u[r] = (float)(__bf16)(u[r] * sx[i] * su[j / P][r]);
-            v[r] = (float)(__bf16)v[r];
-          }
-          v[r] = gp_act(v[r], a.act) * u[r];
-        }
-      }
-      const size_t at = (size_t)row * a.N + n;
-      if (wide) {
-        union { gp_b2 b[2]; u16 h[4]; unsigned long long q; } o;
-        if (a.bias) {
-          o.q = *(const unsigned long long*)(a.bias + n);
-#pragma unroll
-          for (int r = 0; r < 4; r++) v[r] += b2f(o.h[r]);
-        }
-        if (a.res) {
-          o.q = *(const unsigned long long*)(a.res + at);
-#pragma unroll
-          for (int r = 0; r < 4; r++) v[r] += b2f(o.h[r]);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; r++) o.b[r / 2][r % 2] = (__bf16)v[r];
-        *(unsigned long long*)(a.y + at) = o.q;
-      } else {
-        for (int r = 0; r < 4 && n + r < a.N; r++) {
-          float f = v[r];
-          if (a.bias) f += b2f(a.bias[n + r]);
-          if (a.res) f += b2f(a.res[at + r]);
-          a.y[at + r] = f2b(f);
-        }
+      for (int h = 0; h < 2; h++) {
+        const int c = h * 128 + r;
+        pb[h][t] = (uint32_t)min(GLU ? (c >> 5) * 16 + (c & 15) : c,
+                                 a.N - 1 - bn) * (uint32_t)rowb + o;
       }
     }
+  };
+  const uint32_t ring0 = __builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring +
+      wave * 2048);
+  uint32_t put = 0, get = 0;
+  auto turned = [](uint32_t at) {
+    return at == (GW_RING - 1) * 16384 ? 0 : at + 16384;
+  };
+  auto ask = [&](const char* base, const uint32_t (&off)[2]) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) gw_load(base, off[t], ring0 + put + t * 1024);
+    put = turned(put);
+  };
+  // piece 0: B0, 1: A0, 2: B1, 3: A1
+  auto ask_piece = [&](int u) {
+    if (u & 1) ask(xp, pa[HA == 2 ? u >> 1 : 0]);
+    else ask(wp, pb[u >> 1]);
+    if (u == HA + 1) {                       // the slab's last
+      xp += adv;
+      wp += adv;
+      if (--left == 0) {
+        ahead = there(ahead + step);
+        aim();
+      }
+    }
+  };
+
+  // ---- products ----
+  f4v acc[FM][FN];
+  const int fr = lane & 15, fk = lane >> 4;
+  const int x0 = (fk ^ (fr >> 1)) * 16, x1 = x0 ^ 64;
+  const int la = (wm * 64 + fr) * 128, lb = (wn * 32 + fr) * 128;
+  union Frag { u4v_ q[2]; gp_i8 v; gp_s8 h[2]; };
+  Frag xa[4], wb[2][2];
+  auto get_a = [&] {
+    const char* const c = ring + get + la;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      xa[i].q[0] = *(const u4v_*)(c + i * 2048 + x0);
+      xa[i].q[1] = *(const u4v_*)(c + i * 2048 + x1);
+    }
+    get = turned(get);
+  };
+  auto get_b = [&](int h) {
+    const char* const c = ring + get + lb;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      wb[h][j].q[0] = *(const u4v_*)(c + j * 2048 + x0);
+      wb[h][j].q[1] = *(const u4v_*)(c + j * 2048 + x1);
+    }
+    get = turned(get);
+  };
+  auto mma = [&](int ha, int hb) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int k = 0; k < (F8 ? 1 : 2); k++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          f4v& c = acc[ha * 4 + i][hb * 2 + j];
+          // e4m3: without block scales, which would take an instruction more
+          // each (2048x16384x8192 270 us, so 239); row scales at the end
+          if constexpr (F8)
+            c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                wb[hb][j].v, xa[i].v, c, 0, 0, 0, 0, 0, 0);
+          else
+            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                wb[hb][j].h[k], xa[i].h[k], c, 0, 0, 0);
+        }
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  aim();
+  // the slabs that fit in the ring, as if turns before had asked for them
+  constexpr int P = HA == 2 ? GW_RING : GW_RING - 1;
+#pragma unroll
+  for (int n = 0; n < P; n++) ask_piece(n % (HA + 2));
+  gw_wait<2 * (P - 2)>();
+  gw_meet();
+  get_b(0);
+  gw_wait<2 * (P - 2)>();
+  gw_meet();
+  for (;;) {
+    const int tile = t0 + item % chunk, part = item / chunk;
+    const GpAt at = gp_at(a, tile);
+    const int bm = at.row * BM, bn = at.col * (GLU ? BN / 2 : BN);
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++) acc[i][j] = {0.f, 0.f, 0.f, 0.f};
+    if (wm) gw_meet();
+    for (int n = min(per, slabs - part * per); n > 0; n--) {
+      if constexpr (HA == 2) {
+        constexpr int N = 2 * (GW_RING - 2);
+        get_a();
+        ask_piece(1);
+        gw_wait<N>();
+        gw_meet();
+        mma(0, 0);
+        gw_meet();
+        get_b(1);
+        ask_piece(2);
+        gw_wait<N>();
+        gw_meet();
+        mma(0, 1);
+        gw_meet();
+        get_a();
+        ask_piece(3);
+        gw_wait<N>();
+        gw_meet();
+        mma(1, 0);
+        gw_meet();
+        get_b(0);                            // of the next slab
+        ask_piece(0);
+        gw_wait<N>();
+        gw_meet();
+        mma(1, 1);
+        gw_meet();
+      } else {
+        constexpr int N = 2 * (GW_RING - 3);
+        get_a();
+        ask_piece(2);
+        ask_piece(0);
+        gw_wait<N>();
+        gw_meet();
+        mma(0, 0);
+        gw_meet();
+        get_b(1);
+        get_b(0);                            // of the next slab
+        ask_piece(1);
+        gw_wait<N>();
+        gw_meet();
+        mma(0, 1);
+        gw_meet();
+      }
+    }
+    if (!wm) gw_meet();
+    item = there(item + step);
+    gp_finish<F8, BM, BN, 8, FM, FN, GLU, false, HA == 1>(
+        a, acc, tile, part, SK, bm, bn, a.M, 0, nullptr, 0, &last_flag,
+        [&](int i) { return (i >> 2) * 128 + wm * 64 + (i & 3) * 16; },
+        [&](int j) { return (j >> 1) * 128 + wn * 32 + (j & 1) * 16; },
+        [](int r) { return r; });
+    if (item >= items) break;
   }
+  gw_wait<0>();
 }
 
 enum { GP_BF16, GP_E4M3, GP_MXFP4 };           // of W
 #define GP_FAR (1 << 23)       // K up to which 32 bits reach all rows of a tile
+
+// Tiles, in bands of rows that are about as high as what the CUs of an XCD work
+// on is wide: its L2 then misses least (2048x4096x14336 in 128x256 207 -> 202
+// us, e4m3 125 -> 119; 1999x2048x8192 in 128x128 76 -> 72; no difference from
+// 4 to 8 rows of tiles).  256x256 is best in one band of 2048 rows.
+static void gp_tiling(GpArgs& a, int bm, int wide) {
+  a.tm = (a.M + bm - 1) / bm;
+  a.tn = (a.N + wide - 1) / wide;
+  const int most = bm == 256 ? 8 : 1024 / bm, bands = (a.tm + most - 1) / most;
+  a.band = (a.tm + bands - 1) / bands;
+}
 
 template <int T, int BM, int BN, int WM, int WN, int NS, bool FAR = false>
 static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
   constexpr bool F8 = T == GP_E4M3, W4 = T == GP_MXFP4;
   const bool glu = a.act >= 0;
   const int wide = glu ? BN / 2 : BN;
-  a.tm = (a.M + BM - 1) / BM;
-  a.tn = (a.N + wide - 1) / wide;
+  gp_tiling(a, BM, wide);
   const dim3 grid((a.tm * a.tn + 7) / 8 * 8, sk);
   if (glu)
     hipLaunchKernelGGL(
@@ -492,13 +775,34 @@ static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
   return hipGetLastError();
 }
 
+// by k_gemm_wide; e4m3 rows of whole slabs
+template <int T, int HA>
+static hipError_t gp_go_wide(GpArgs a, int sk, hipStream_t s) {
+  constexpr bool F8 = T == GP_E4M3;
+  const bool glu = a.act >= 0;
+  gp_tiling(a, 128 * HA, glu ? 128 : 256);
+  // as many parts as have slabs
+  const int slabs = (int)((long)a.K * (F8 ? 1 : 2) / 128);
+  const int per = (slabs + sk - 1) / sk;
+  sk = (slabs + per - 1) / per;
+  const int share = (a.tm * a.tn + 7) / 8 * sk;          // of an XCD
+  const dim3 grid(8 * (share < 32 ? share : 32));        // a block a CU
+  if (glu)
+    hipLaunchKernelGGL((k_gemm_wide<F8, HA, true>), grid, dim3(512), 0, s, a,
+                       sk);
+  else
+    hipLaunchKernelGGL((k_gemm_wide<F8, HA, false>), grid, dim3(512), 0, s, a,
+                       sk);
+  return hipGetLastError();
+}
+
 // Large tiles ask L2 for the fewest bytes a product: 128x128 by four waves
 // wants 64 bytes a clock, all that a CU gets.  They win where there are rounds
 // of them; where tiles are fewer than the chip has CUs a smaller one that is
-// deep in flight does.  256x256 (never split: its parts cost most) spills in
-// e4m3 (fragments) and MXFP4 (W on its way to LDS: 467 TFLOP/s at
-// 2048x37888x3584, 128x128 944).  The second 128x128 has eight waves and four
-// buffers.
+// deep in flight does.  256x256 is never split (1999x2048x8192 in four parts
+// 107 us, 128x128 76: its parts cost most) and not for MXFP4 (W on its way to
+// LDS spills: 467 TFLOP/s at 2048x37888x3584, 128x128 944).  The second 128x128
+// has eight waves and four buffers.
 struct GpTile { int bm, bn, occ; };              // occ: blocks that fit on a CU
 static const GpTile gp_tiles[8] = {
     {256, 256, 1}, {128, 256, 1}, {128, 128, 2}, {128, 128, 1},
@@ -521,14 +825,19 @@ static const GpTile gp_tiles[8] = {
 // e4m3 rounding sums in another order are other values: K is split as it was
 // but for 2% of the products.  MXFP4 is fitted to 64, 130, 600 and 2048 rows of
 // five shapes (2.2%).
+// The numbers of the 256-wide tiles (and of bf16 128x128 of eight waves) were
+// fitted again when k_gemm_wide took them over, to 432 products of 100 to 2048
+// rows of 27 shapes.  Above the best, and how many by more than 4%, by the
+// numbers that were -> now: bf16 1.0% -> 0.8%, 14 -> 9; with a gate 0.2%, 1;
+// e4m3 1.9% -> 0.3%, 14 -> 3; with a gate 9.4% -> 0.2%, 29 -> 1.
 struct GpCost {
   float one[8], full[8], round[8], second, first, split, part;
 };
 static const GpCost gp_cost[5] = {
     {// bf16
-     {1.29f, 0.87f, 0.62f, 0.483f, 1.24f, 0.485f, 0.261f, 0.251f},
-     {1.29f, 0.87f, 1.09f, 0.483f, 1.24f, 0.85f, 0.49f, 0.438f},
-     {7.85f, 4.92f, 2.87f, 3.78f, 2.01f, 1.53f, 1.33f, 0.787f},
+     {1.29f, 0.665f, 0.62f, 0.51f, 1.24f, 0.485f, 0.261f, 0.251f},
+     {1.29f, 0.665f, 1.09f, 0.51f, 1.24f, 0.85f, 0.49f, 0.438f},
+     {7.85f, 3.82f, 2.87f, 4.5f, 2.01f, 1.53f, 1.33f, 0.787f},
      0.7f, 1.f, 1.61f, 4.94e-6f},
     {// bf16 with a gate
      {1.46f, 0.87f, 0.592f, 0.5f, 0.854f, 0.481f, 0.261f, 0.234f},
@@ -536,14 +845,14 @@ static const GpCost gp_cost[5] = {
      {4.86f, 3.2f, 2.75f, 3.37f, 2.56f, 2.98f, 1.09f, 1.56f},
      0.616f, 0.96f, 2.1f, 4.79e-6f},
     {// e4m3
-     {0.f, 1.1f, 0.f, 0.752f, 0.633f, 0.892f, 0.405f, 0.286f},
-     {0.f, 1.43f, 0.f, 0.752f, 0.817f, 0.892f, 0.556f, 0.449f},
-     {0.f, 3.81f, 0.f, 2.16f, 2.07f, 2.84f, 1.14f, 1.21f},
+     {1.76f, 0.954f, 0.f, 0.752f, 0.633f, 0.892f, 0.405f, 0.286f},
+     {1.76f, 0.954f, 0.f, 0.752f, 0.817f, 0.892f, 0.556f, 0.449f},
+     {6.f, 3.81f, 0.f, 2.16f, 2.07f, 2.84f, 1.14f, 1.21f},
      0.626f, 0.952f, 0.273f, 5.43e-6f},
     {// e4m3 with a gate
-     {0.f, 1.17f, 0.f, 0.677f, 1.07f, 0.572f, 0.45f, 0.286f},
-     {0.f, 1.17f, 0.f, 0.769f, 1.07f, 0.851f, 0.57f, 0.474f},
-     {0.f, 3.98f, 0.f, 2.42f, 1.8f, 1.77f, 1.4f, 1.85f},
+     {1.87f, 1.17f, 0.f, 0.677f, 1.07f, 0.572f, 0.45f, 0.286f},
+     {1.87f, 1.17f, 0.f, 0.769f, 1.07f, 0.851f, 0.57f, 0.474f},
+     {6.f, 3.98f, 0.f, 2.42f, 1.8f, 1.77f, 1.4f, 1.85f},
      0.632f, 1.f, 0.778f, 4.63e-6f},
     {// MXFP4
      {0.f, 0.96f, 0.654f, 0.562f, 0.44f, 0.f, 0.292f, 0.f},
@@ -565,7 +874,9 @@ static GpPick gp_pick(const GpArgs& a, long part_floats, int ncnt) {
   for (int c = 0; c < 8; c++) {
     const GpTile& g = gp_tiles[c];
     const float one = k.one[c], full = k.full[c];
-    if (one == 0.f || (far && c != 6)) continue;
+    if (one == 0.f || (far && c != 6) ||
+        (c == 0 && T == GP_E4M3 && a.K % 128))
+      continue;
     const long tiles = (long)((a.M + g.bm - 1) / g.bm) *
                        ((width + g.bn - 1) / g.bn);
     for (int sk = 1; sk <= 8; sk++) {
@@ -602,14 +913,19 @@ template <int T>
 static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
                          hipStream_t s) {
   const bool far = T != GP_MXFP4 && a.K > GP_FAR;        // 64x64 alone
+  const bool odd = T == GP_E4M3 && a.K % 128;            // half a slab
   const GpPick pick = gp_pick<T>(a, part_floats, ncnt);
   const int best_sk = pick.sk;
   switch (pick.tile) {
     case 0:
-      if constexpr (T == GP_BF16)
-        return gp_go<T, 256, 256, 2, 4, 2>(a, best_sk, s);
+      if constexpr (T != GP_MXFP4) return gp_go_wide<T, 2>(a, best_sk, s);
       break;
-    case 1: return gp_go<T, 128, 256, 2, 4, 3>(a, best_sk, s);
+    case 1:
+      if constexpr (T != GP_MXFP4)
+        if (!odd) return gp_go_wide<T, 1>(a, best_sk, s);
+      if constexpr (T != GP_BF16)
+        return gp_go<T, 128, 256, 2, 4, 3>(a, best_sk, s);
+      break;
     case 2:
       if constexpr (T != GP_E4M3)
         return gp_go<T, 128, 128, 2, 2, 2>(a, best_sk, s);
@@ -643,7 +959,7 @@ extern "C" hipError_t launch_gemm_prompt(
     return hipErrorInvalidValue;
   GpArgs a = {x, w, (const float*)sx, (const float*)sw, nullptr,
               (const u16*)res, (const u16*)bias, (u16*)y, (float*)part,
-              (int*)cnt, M, N, K, act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
+              (int*)cnt, M, N, K, act, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
   if (!part || !cnt) part_floats = 0;
   if (mid_takes(sx, M, N, K, act >= 0))
     return launch_mid_gemm(x, w, sx, sw, res, bias, y, part, cnt, part_floats,
@@ -662,7 +978,7 @@ extern "C" hipError_t launch_gemm_fp4w(
     return hipErrorInvalidValue;
   GpArgs a = {x, w, nullptr, nullptr, (const uint8_t*)we, (const u16*)res,
               (const u16*)bias, (u16*)y, (float*)part, (int*)cnt, M, N, K,
-              act, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
+              act, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, 1, 0};
   return gp_run<GP_MXFP4>(a, part && cnt ? part_floats : 0, ncnt, stream);
 }
 
@@ -803,7 +1119,7 @@ extern "C" hipError_t launch_expert_gemm(
   const int bm = expert_bm(pairs, E), tiles = pairs / bm + E;
   const int* p = (const int*)sorted;
   GpArgs a = {x, w, (const float*)sx, (const float*)sw, nullptr, nullptr,
-              nullptr, (u16*)y, nullptr, nullptr, pairs, N, K, act, tiles, 0,
+              nullptr, (u16*)y, nullptr, nullptr, pairs, N, K, act, tiles, 0, tiles,
               p, p + pairs, p + pairs + tiles, p + pairs + 2 * tiles, top,
               gather};
 #define EXPERTS(F8)                                                          \

@@ -315,6 +315,29 @@ def test_many_rows_of_each_tile(M, N, K, kind, act):
     test_many_rows(M, N, K, kind, act)
 
 
+# tiles 256 wide: slabs fewer than the ring holds, one, two and three, and
+# several tiles a block (more than 256), so that one's slabs are asked for
+# while another is multiplied; 256 and 128 rows, with a rest both ways; parts
+# of K, also with a short last one
+@pytest.mark.parametrize("M,N,K,kind,act", [
+    (905, 8494, 384, "bf16", -1), (391, 10822, 192, "bf16", -1),
+    (1045, 11186, 192, "bf16", -1), (675, 10949, 320, "bf16", -1),
+    (153, 11205, 12864, "bf16", -1), (199, 8994, 8192, "bf16", -1),
+    (223, 2589, 17600, "bf16", 0),
+    (385, 8380, 64, "bf16", 0), (1188, 9848, 64, "bf16", 0),
+    (1159, 9732, 128, "bf16", 0), (1052, 10895, 192, "bf16", 0),
+    (1025, 10942, 256, "bf16", 0), (259, 8593, 128, "bf16", 0),
+    (566, 10887, 128, "bf16", 0), (555, 11005, 192, "bf16", 0),
+    (793, 10086, 128, "fp8", -1), (840, 9423, 384, "fp8", -1),
+    (332, 11127, 128, "fp8", -1), (330, 10970, 256, "fp8", -1),
+    (340, 11179, 384, "fp8", -1), (1167, 9842, 128, "fp8", 0),
+    (1164, 9823, 256, "fp8", 0), (1156, 10068, 384, "fp8", 0),
+    (547, 11509, 128, "fp8", 0), (542, 11246, 256, "fp8", 0),
+    (521, 11510, 384, "fp8", 0)])
+def test_many_rows_of_wide_tiles(M, N, K, kind, act):
+    test_many_rows(M, N, K, kind, act)
+
+
 # rows so long that 32 bits do not reach those of a tile: of the largest (256
 # rows of 2^24 bytes), and of the one that takes them (64 rows of 66 MB)
 @pytest.mark.parametrize("kind,act,K", [
