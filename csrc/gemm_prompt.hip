@@ -205,7 +205,7 @@ DEVINL void gp_finish(const GpArgs& a, f4v (&acc)[FM][FN], int tile, int part,
 }
 
 template <bool F8, int BM, int BN, int WM, int WN, int NS, bool GLU,
-          bool MOE = false, bool W4 = false, bool FAR = false>
+          bool MOE = false, bool W4 = false, bool FAR = false, bool NT = false>
 __global__ void __launch_bounds__(64 * WM * WN)
 k_gemm_prompt(GpArgs a) {
   constexpr int NW = WM * WN;
@@ -340,7 +340,7 @@ k_gemm_prompt(GpArgs a) {
           (const __attribute__((address_space(1))) uint32_t*)(
               ws + (Off)(pb[i] + (((wave * BI + i) & 1) ? o1 : o0))),
           (__attribute__((address_space(3))) uint32_t*)(
-              B + (wave * BI + i) * 1024), 16, 0, 0);
+              B + (wave * BI + i) * 1024), 16, 0, NT ? 2 : 0);
     }
   };
 
@@ -507,11 +507,17 @@ k_gemm_prompt(GpArgs a) {
 // first.  Behind the last one loads go on, to one line, so that the waits
 // count alike.
 #define GW_RING 9
+// 64 lanes of 16 bytes to lds and behind it
+template <bool NT = false>
 DEVINL void gw_load(const char* base, uint32_t off, uint32_t lds) {
-  // 64 lanes of 16 bytes to lds and behind it
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
-               "global_load_lds_dwordx4 %1, %0"
-               :: "s"(base), "v"(off), "s"(lds) : "memory");
+  if constexpr (NT)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %1, %0 nt"
+                 :: "s"(base), "v"(off), "s"(lds) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %1, %0"
+                 :: "s"(base), "v"(off), "s"(lds) : "memory");
 }
 DEVINL void gw_meet() {
   asm volatile("" ::: "memory");
@@ -525,7 +531,7 @@ template <int N> DEVINL void gw_wait() {
   asm volatile("" ::: "memory");
 }
 
-template <bool F8, int HA, bool GLU>
+template <bool F8, int HA, bool GLU, bool NT>
 __global__ void __launch_bounds__(512) k_gemm_wide(GpArgs a, int SK) {
   constexpr int BM = 128 * HA, BN = 256, FM = 4 * HA, FN = 4;
   __shared__ __attribute__((aligned(16))) char ring[GW_RING * 16384];
@@ -600,15 +606,16 @@ __global__ void __launch_bounds__(512) k_gemm_wide(GpArgs a, int SK) {
   auto turned = [](uint32_t at) {
     return at == (GW_RING - 1) * 16384 ? 0 : at + 16384;
   };
-  auto ask = [&](const char* base, const uint32_t (&off)[2]) {
+  auto ask = [&](auto nt, const char* base, const uint32_t (&off)[2]) {
 #pragma unroll
-    for (int t = 0; t < 2; t++) gw_load(base, off[t], ring0 + put + t * 1024);
+    for (int t = 0; t < 2; t++)
+      gw_load<decltype(nt)::value>(base, off[t], ring0 + put + t * 1024);
     put = turned(put);
   };
   // piece 0: B0, 1: A0, 2: B1, 3: A1
   auto ask_piece = [&](int u) {
-    if (u & 1) ask(xp, pa[HA == 2 ? u >> 1 : 0]);
-    else ask(wp, pb[u >> 1]);
+    if (u & 1) ask(std::false_type(), xp, pa[HA == 2 ? u >> 1 : 0]);
+    else ask(std::integral_constant<bool, NT>(), wp, pb[u >> 1]);
     if (u == HA + 1) {                       // the slab's last
       xp += adv;
       wp += adv;
@@ -757,21 +764,36 @@ static void gp_tiling(GpArgs& a, int bm, int wide) {
   a.band = (a.tm + bands - 1) / bands;
 }
 
+// One row of tiles reads W once: past the caches, where there is much of it
+// (us, W of 16 to 155 MB, in them -> past: 64 rows of 28672x4096 54.0 -> 47.1,
+// of 16384x2048 17.4 -> 16.9, 128 rows of 28672x4096 by 128x128 58.9 -> 51.5;
+// 6144x2304 of 28 MB 17.8 -> 18.1, and e4m3 3072x2048 of 6 MB, which the last
+// level may still hold, 10.9 -> 13.0).
+template <int T> static bool gp_once(const GpArgs& a) {
+  return a.tm == 1 && (a.act >= 0 ? 2.f : 1.f) * a.N * a.K *
+                              (T == GP_E4M3 ? 1 : 2) >= 32 << 20;
+}
+
 template <int T, int BM, int BN, int WM, int WN, int NS, bool FAR = false>
 static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
   constexpr bool F8 = T == GP_E4M3, W4 = T == GP_MXFP4;
   const bool glu = a.act >= 0;
   const int wide = glu ? BN / 2 : BN;
   gp_tiling(a, BM, wide);
-  const dim3 grid((a.tm * a.tn + 7) / 8 * 8, sk);
-  if (glu)
-    hipLaunchKernelGGL(
-        (k_gemm_prompt<F8, BM, BN, WM, WN, NS, true, false, W4, FAR>), grid,
-        dim3(64 * WM * WN), 0, s, a);
-  else
-    hipLaunchKernelGGL(
-        (k_gemm_prompt<F8, BM, BN, WM, WN, NS, false, false, W4, FAR>), grid,
-        dim3(64 * WM * WN), 0, s, a);
+  const dim3 grid((a.tm * a.tn + 7) / 8 * 8, sk), nt(64 * WM * WN);
+#define GP_GO(GLU, NT)                                                       \
+  hipLaunchKernelGGL((k_gemm_prompt<F8, BM, BN, WM, WN, NS, GLU, false, W4,  \
+                                    FAR, NT>), grid, nt, 0, s, a)
+  if constexpr (!W4 && !FAR) {
+    if (gp_once<T>(a)) {
+      if (glu) GP_GO(true, true);
+      else GP_GO(false, true);
+      return hipGetLastError();
+    }
+  }
+  if (glu) GP_GO(true, false);
+  else GP_GO(false, false);
+#undef GP_GO
   return hipGetLastError();
 }
 
@@ -787,12 +809,19 @@ static hipError_t gp_go_wide(GpArgs a, int sk, hipStream_t s) {
   sk = (slabs + per - 1) / per;
   const int share = (a.tm * a.tn + 7) / 8 * sk;          // of an XCD
   const dim3 grid(8 * (share < 32 ? share : 32));        // a block a CU
-  if (glu)
-    hipLaunchKernelGGL((k_gemm_wide<F8, HA, true>), grid, dim3(512), 0, s, a,
-                       sk);
-  else
-    hipLaunchKernelGGL((k_gemm_wide<F8, HA, false>), grid, dim3(512), 0, s, a,
-                       sk);
+#define GW_GO(GLU, NT)                                                       \
+  hipLaunchKernelGGL((k_gemm_wide<F8, HA, GLU, NT>), grid, dim3(512), 0, s,  \
+                     a, sk)
+  if constexpr (HA == 1) {
+    if (gp_once<T>(a)) {
+      if (glu) GW_GO(true, true);
+      else GW_GO(false, true);
+      return hipGetLastError();
+    }
+  }
+  if (glu) GW_GO(true, false);
+  else GW_GO(false, false);
+#undef GW_GO
   return hipGetLastError();
 }
 
@@ -829,30 +858,35 @@ static const GpTile gp_tiles[8] = {
 // fitted again when k_gemm_wide took them over, to 432 products of 100 to 2048
 // rows of 27 shapes.  Above the best, and how many by more than 4%, by the
 // numbers that were -> now: bf16 1.0% -> 0.8%, 14 -> 9; with a gate 0.2%, 1;
-// e4m3 1.9% -> 0.3%, 14 -> 3; with a gate 9.4% -> 0.2%, 29 -> 1.
+// e4m3 1.9% -> 0.3%, 14 -> 3; with a gate 9.4% -> 0.2%, 29 -> 1.  And, to 648
+// of 20 to 2048 rows, those of the others when 64x64, 64x128 and 128x64 went
+// from four waves to eight (64 rows of 16384x2048 18.5 -> 17.4, 100 of
+// 8192x2048 21.4 to 24.4 -> 12.8 to 21.4; over all 4% in bf16, 5% in e4m3):
+// bf16 2.0% -> 1.3%, with a gate 1.2% -> 0.8%, e4m3 as it was 1.5%, with a gate
+// 1.1% -> 0.5%.
 struct GpCost {
   float one[8], full[8], round[8], second, first, split, part;
 };
 static const GpCost gp_cost[5] = {
     {// bf16
-     {1.29f, 0.665f, 0.62f, 0.51f, 1.24f, 0.485f, 0.261f, 0.251f},
-     {1.29f, 0.665f, 1.09f, 0.51f, 1.24f, 0.85f, 0.49f, 0.438f},
-     {7.85f, 3.82f, 2.87f, 4.5f, 2.01f, 1.53f, 1.33f, 0.787f},
-     0.7f, 1.f, 1.61f, 4.94e-6f},
+     {1.29f, 0.665f, 0.62f, 0.51f, 1.24f, 0.443f, 0.261f, 0.257f},
+     {1.29f, 0.665f, 1.09f, 0.51f, 1.37f, 1.07f, 0.501f, 0.438f},
+     {7.85f, 3.82f, 2.87f, 4.5f, 2.1f, 1.21f, 1.54f, 1.24f},
+     0.7f, 1.f, 2.22f, 4.94e-6f},
     {// bf16 with a gate
-     {1.46f, 0.87f, 0.592f, 0.5f, 0.854f, 0.481f, 0.261f, 0.234f},
-     {1.48f, 0.87f, 1.22f, 0.5f, 0.854f, 0.75f, 0.598f, 0.312f},
-     {4.86f, 3.2f, 2.75f, 3.37f, 2.56f, 2.98f, 1.09f, 1.56f},
-     0.616f, 0.96f, 2.1f, 4.79e-6f},
+     {1.46f, 0.87f, 0.592f, 0.518f, 0.854f, 0.481f, 0.261f, 0.234f},
+     {1.46f, 0.87f, 1.22f, 0.518f, 0.854f, 0.822f, 0.576f, 0.312f},
+     {4.86f, 3.2f, 2.36f, 3.37f, 2.56f, 2.98f, 1.09f, 1.56f},
+     0.616f, 0.96f, 1.77f, 4.79e-6f},
     {// e4m3
      {1.76f, 0.954f, 0.f, 0.752f, 0.633f, 0.892f, 0.405f, 0.286f},
      {1.76f, 0.954f, 0.f, 0.752f, 0.817f, 0.892f, 0.556f, 0.449f},
      {6.f, 3.81f, 0.f, 2.16f, 2.07f, 2.84f, 1.14f, 1.21f},
      0.626f, 0.952f, 0.273f, 5.43e-6f},
     {// e4m3 with a gate
-     {1.87f, 1.17f, 0.f, 0.677f, 1.07f, 0.572f, 0.45f, 0.286f},
-     {1.87f, 1.17f, 0.f, 0.769f, 1.07f, 0.851f, 0.57f, 0.474f},
-     {6.f, 3.98f, 0.f, 2.42f, 1.8f, 1.77f, 1.4f, 1.85f},
+     {1.87f, 1.17f, 0.f, 0.745f, 0.651f, 0.78f, 0.45f, 0.286f},
+     {1.87f, 1.17f, 0.f, 0.745f, 0.878f, 0.78f, 0.45f, 0.474f},
+     {6.f, 3.98f, 0.f, 2.18f, 1.8f, 1.28f, 1.68f, 1.85f},
      0.632f, 1.f, 0.778f, 4.63e-6f},
     {// MXFP4
      {0.f, 0.96f, 0.654f, 0.562f, 0.44f, 0.f, 0.292f, 0.f},
@@ -916,6 +950,8 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
   const bool odd = T == GP_E4M3 && a.K % 128;            // half a slab
   const GpPick pick = gp_pick<T>(a, part_floats, ncnt);
   const int best_sk = pick.sk;
+  // eight waves, four beside MXFP4, whose pieces of W a thread would be halves
+  constexpr int WM = T == GP_MXFP4 ? 2 : 4;
   switch (pick.tile) {
     case 0:
       if constexpr (T != GP_MXFP4) return gp_go_wide<T, 2>(a, best_sk, s);
@@ -931,15 +967,15 @@ static hipError_t gp_run(const GpArgs& a, long part_floats, int ncnt,
         return gp_go<T, 128, 128, 2, 2, 2>(a, best_sk, s);
       break;
     case 3: return gp_go<T, 128, 128, 2, 4, 4>(a, best_sk, s);
-    case 4: return gp_go<T, 64, 128, 2, 2, 3>(a, best_sk, s);
+    case 4: return gp_go<T, 64, 128, WM, 2, 3>(a, best_sk, s);
     case 5:
       if constexpr (T != GP_MXFP4)
-        return gp_go<T, 128, 64, 2, 2, 3>(a, best_sk, s);
+        return gp_go<T, 128, 64, WM, 2, 3>(a, best_sk, s);
       break;
     case 6:
       if constexpr (T != GP_MXFP4)
-        if (far) return gp_go<T, 64, 64, 2, 2, 4, true>(a, best_sk, s);
-      return gp_go<T, 64, 64, 2, 2, 4>(a, best_sk, s);
+        if (far) return gp_go<T, 64, 64, WM, 2, 4, true>(a, best_sk, s);
+      return gp_go<T, 64, 64, WM, 2, 4>(a, best_sk, s);
     case 7:
       if constexpr (T != GP_MXFP4)
         return gp_go<T, 32, 64, 2, 2, 6>(a, best_sk, s);
@@ -1124,7 +1160,7 @@ extern "C" hipError_t launch_expert_gemm(
               gather};
 #define EXPERTS(F8)                                                          \
   return bm == 128  ? gp_experts<F8, 128, 128, 2, 4, 4>(a, stream)           \
-         : bm == 64 ? gp_experts<F8, 64, 64, 2, 2, 4>(a, stream)             \
+         : bm == 64 ? gp_experts<F8, 64, 64, 4, 2, 4>(a, stream)             \
                     : gp_experts<F8, 32, 64, 2, 2, 6>(a, stream)
   if (sx) EXPERTS(true);
   EXPERTS(false);
