@@ -83,19 +83,23 @@ DEVINL void part_put(float* p, float v) {
 DEVINL float part_get(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Four of them, the last two `far` floats behind the first: lanes side by side
+// leave whole lines (16 bytes a lane in two halves of their own left half lines
+// twice: 1999x2048x8192 in two parts of K by 128x256 81 us, so 72; 300 rows in
+// three 36.6, 33.9; 700x3584x14336 in three 103, 95).
 union PartSums { f4v v; unsigned long long u[2]; };
-DEVINL void part_put4(float* p, f4v v) {     // 8-byte aligned
+DEVINL void part_put4(float* p, int far, f4v v) {     // 8-byte aligned
   const PartSums s = {v};
 #pragma unroll
   for (int i = 0; i < 2; i++)
-    __hip_atomic_store((unsigned long long*)p + i, s.u[i], __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store((unsigned long long*)(p + i * far), s.u[i],
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-DEVINL f4v part_get4(const float* p) {
+DEVINL f4v part_get4(const float* p, int far) {
   PartSums s;
 #pragma unroll
   for (int i = 0; i < 2; i++)
-    s.u[i] = __hip_atomic_load((const unsigned long long*)p + i,
+    s.u[i] = __hip_atomic_load((const unsigned long long*)(p + i * far),
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return s.v;
 }

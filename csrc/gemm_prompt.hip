@@ -98,13 +98,13 @@ DEVINL void gp_finish(const GpArgs& a, f4v (&acc)[FM][FN], int tile, int part,
   const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fk = lane >> 4;
   if (SPLIT && SK > 1) {
     // fragments as they lie in registers: the last block reads them alike
-    float* pp = a.part + (size_t)tile * SK * (BM * BN) + tid * 4;
+    float* pp = a.part + (size_t)tile * SK * (BM * BN) + tid * 2;
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
       for (int j = 0; j < FN; j++)
         part_put4(pp + (size_t)part * (BM * BN) +
-                  (i * FN + j) * (NW * 256), acc[i][j]);
+                  (i * FN + j) * (NW * 256), NW * 128, acc[i][j]);
     if (!last_block(&a.cnt[tile], SK, last_flag)) return;
     // up to 16 fragments of a part on the way at a time: a part a trip, not
     // a fragment of one
@@ -122,7 +122,7 @@ DEVINL void gp_finish(const GpArgs& a, f4v (&acc)[FM][FN], int tile, int part,
 #pragma unroll
           for (int j = 0; j < FN; j++)
             t[i][j] = part_get4(pp + (size_t)q * (BM * BN) +
-                                ((i0 + i) * FN + j) * (NW * 256));
+                                ((i0 + i) * FN + j) * (NW * 256), NW * 128);
 #pragma unroll
         for (int i = 0; i < G; i++)
 #pragma unroll
@@ -829,7 +829,7 @@ static hipError_t gp_go_wide(GpArgs a, int sk, hipStream_t s) {
 // wants 64 bytes a clock, all that a CU gets.  They win where there are rounds
 // of them; where tiles are fewer than the chip has CUs a smaller one that is
 // deep in flight does.  256x256 is never split (1999x2048x8192 in four parts
-// 107 us, 128x128 76: its parts cost most) and not for MXFP4 (W on its way to
+// 85 us, 128x128 72: its parts cost most) and not for MXFP4 (W on its way to
 // LDS spills: 467 TFLOP/s at 2048x37888x3584, 128x128 944).  The second 128x128
 // has eight waves and four buffers.
 struct GpTile { int bm, bn, occ; };              // occ: blocks that fit on a CU

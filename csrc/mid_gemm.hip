@@ -263,12 +263,22 @@ __global__ void __launch_bounds__(64 * MG_NW) k_mid_gemm(MgArgs a) {
   }
   float* part = a.part + (size_t)blockIdx.x * KS * ITEMS * 4;
   for (int e = tid; e < ITEMS; e += 64 * MG_NW)
-    part_put4(part + ((size_t)blockIdx.y * ITEMS + e) * 4, meet(e));
+    part_put4(part + (size_t)blockIdx.y * ITEMS * 4 + e * 2, ITEMS * 2,
+              meet(e));
   if (!last_block(&a.cnt[blockIdx.x], KS, &last_flag)) return;
+  // four parts on the way at a time (one after the other, and in halves of
+  // lines: 37x2048x8192 12.7 us, so 12.2)
   auto parts = [&](int at) {
-    f4v v = part_get4(part + at * 4);
-    for (int k = 1; k < KS; k++)
-      v += part_get4(part + ((size_t)k * ITEMS + at) * 4);
+    f4v v, t[4];
+    for (int k = 0; k < KS; k += 4) {
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        t[q] = part_get4(part + (size_t)min(k + q, KS - 1) * ITEMS * 4 +
+                             at * 2, ITEMS * 2);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (k + q < KS) v = k + q ? v + t[q] : t[q];
+    }
     return v;
   };
   for (int e = tid; e < DONE; e += 64 * MG_NW) {
