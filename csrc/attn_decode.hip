@@ -17,10 +17,11 @@
 //
 // A wave takes 32 keys at a time by itself: K in operand order straight from
 // the pool, V through its own stretch of LDS, turned by ds_read_b64_tr_b16
-// (see attn_prefill.hip).  Loads are hidden by the eight waves of a block
-// (four of 256 dims: registers), not by a pipeline in one: a wave rarely has
-// a second tile, since a block's range is a tile for each wave.  64 keys in
-// four waves took 1.7 us more at 90 keys and as long at 6000.
+// (see attn_prefill.hip).  Loads are hidden by the eight waves of a block, not
+// by a pipeline in one: a wave rarely has a second tile, since a block's range
+// is a tile for each wave.  64 keys in four waves took 1.7 us more at 90 keys
+// and as long at 6000.  Of 256 dims, where eight waves are a CU's whole LDS,
+// short histories come in ranges of four tiles.
 //
 // What is left at a short history is one trip for the position, one for the
 // loads it allows, the score -> probability -> value chain and the launch:
@@ -28,7 +29,9 @@
 // ranges (as before) -> here:
 //   32/8 heads of 64, 90 keys 7.6 -> 4.6; 4000 keys 22.2 -> 10.0
 //   32/8 of 128, 6040 e4m3 keys 39.2 -> 13.5; 160 keys 9.8 -> 6.4
-//   16/8 of 256, 16 sequences of 620 keys, softcap 52.3 -> 25.4 (two ranges)
+//   16/8 of 256, 16 sequences of 620 keys, softcap 52.3 -> 25.4 (two ranges);
+//     by eight waves a block for four 23.5 -> 20.0 (3.1 TB/s), 16 of 1500 keys
+//     46.6 -> 40.7, one of 2000 13.5 -> 12.2, 8/4 heads, 220 keys 11.7 -> 10.1
 //   64/8 of 128, 4 sequences of 2000 keys 97 -> 23
 //   16/4 of 128, 32000 keys 131 -> 38 (1.7 TB/s: few blocks, long ranges)
 //
@@ -434,9 +437,9 @@ DEVINL float ad_part(float v, int part) {
 }
 
 template <int HD, bool KV8>
-__global__ void __launch_bounds__(64 * (HD == 256 ? 4 : 8))
+__global__ void __launch_bounds__(64 * 8)
 k_attn_dec(AdArgs a) {
-  constexpr int NW = HD == 256 ? 4 : 8, NS = 2, TK = 16 * NS;  // keys of a tile
+  constexpr int NW = 8, NS = 2, TK = 16 * NS;  // keys of a tile
   constexpr int KC = HD / 32, DT = HD / 16, HD2 = HD / 2, RB = HD * 2;
   constexpr int VT = TK * RB;                // bytes of a wave's V tile
   __shared__ __attribute__((aligned(16))) char Vs[NW][VT];
@@ -457,10 +460,14 @@ k_attn_dec(AdArgs a) {
   const int hist = pos - start;
   // A tile for every wave of a block, more where the grid ends; one range as
   // long as two rounds will do (345 keys of 128, 6 sequences: 8.9 us, two
-  // ranges and their merge 10.0).
+  // ranges and their merge 10.0; of 256 dims one round: 300 keys 12.1, three
+  // ranges 9.9).  Of 256 dims up to 2048 keys are in ranges of four tiles (700
+  // keys, 4 sequences 13.9, so 11.4; 2000 keys 14.4, 12.2; 5000 15.6 both).
+  constexpr int ONE = HD == 256 ? NW : 2 * NW;
   const int tiles = (hist + TK - 1) / TK;
-  const int eff = tiles <= 2 * NW ? 1
-                                  : min((tiles + NW - 1) / NW, (int)gridDim.y);
+  const int most = HD == 256 && tiles <= 64 ? 4 : NW;
+  const int eff = tiles <= ONE ? 1 : min((tiles + most - 1) / most,
+                                         (int)gridDim.y);
   if (chunk >= eff) return;
   const int per = (tiles + eff - 1) / eff;
   const int c0 = start + chunk * per * TK, c1 = min(c0 + per * TK, pos);
@@ -769,12 +776,11 @@ template <int HD>
 static hipError_t ad_mfma(AdArgs a, int kv8, int split, int batch,
                           hipStream_t s) {
   a.hg = (a.nh / a.kvh + 3) / 4;
-  const int nt = HD == 256 ? 256 : 512;
   const dim3 grid(a.kvh * a.hg, split, batch);
   if (kv8)
-    hipLaunchKernelGGL((k_attn_dec<HD, true>), grid, dim3(nt), 0, s, a);
+    hipLaunchKernelGGL((k_attn_dec<HD, true>), grid, dim3(512), 0, s, a);
   else
-    hipLaunchKernelGGL((k_attn_dec<HD, false>), grid, dim3(nt), 0, s, a);
+    hipLaunchKernelGGL((k_attn_dec<HD, false>), grid, dim3(512), 0, s, a);
   return hipGetLastError();
 }
 

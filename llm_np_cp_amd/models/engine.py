@@ -391,9 +391,9 @@ class GPUModel(DecodeLoop):
         import os as _os
         _sp = _os.environ.get("LLM_ATTN_SPLIT")
         # ranges of the history that a step may take: the kernel takes one
-        # for some 256 keys, up to so many
-        self.attn_split = (int(_sp) if _sp else
-                           min(64, max(1, -(-self.max_seq // 256))))
+        # for some 256 keys (128 of 256 dims), up to so many
+        self.attn_split = (int(_sp) if _sp else min(64, max(
+            1, -(-self.max_seq // (128 if hd == 256 else 256)))))
         self.attn_scratch = torch.zeros(
             self.nh_l * self.attn_split * (hd + 2), dtype=torch.float32,
             device=dev)

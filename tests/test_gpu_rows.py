@@ -407,6 +407,12 @@ def test_new_tokens(hd, nh, kvh, pos, kv8):
     (128, 5, 1, [16400, 3], (80, 5000, 0.0)),
     (256, 4, 2, [2300, 8200], (64, 0, 50.0)),
     (256, 2, 1, [3000, 2177], (20, 2176, 0.0)),
+    # of 256 dims: one round in one range, a key more in ranges of four
+    # tiles, the last length that has those and the first that has not; where
+    # the grid ends ahead of them
+    (256, 4, 2, [256, 257], (64, 0, 50.0)),
+    (256, 4, 2, [2048, 2049], (64, 0, 0.0)),
+    (256, 8, 2, [611, 2048], (2, 0, 50.0)),
     (512, 2, 1, [1500, 1088], (80, 0, 0.0)),
     (512, 4, 2, [4500, 65], (80, 4000, 30.0)),
     (16, 4, 2, [40000, 2049], (80, 0, 0.0))])
