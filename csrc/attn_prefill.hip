@@ -26,6 +26,18 @@
 // wave has all rows).  One wave a SIMD without spills was slower (2048 rows
 // behind 2048 keys: 219 us to 163 when it still spilled 20, now 118).
 //
+// Where a block's own keys are what takes long (the last rows of a prompt see
+// all of them, and a block goes through its tiles one after the other), two
+// groups of four waves take its tiles in turn and meet in LDS at the end: a
+// chain half as long and nothing past the L2, where ranges of keys leave parts
+// of every row.  us, ranges or one block as before -> two groups:
+//   64 dims   32/8 heads  611 rows 22.8 -> 12.7, 1000 34.9 -> 17.1, 1999 34.1 ->
+//             29.9; 700 behind 1300 keys 37.5 -> 27.6
+//   128 dims  32/8 1000 rows 40.5 -> 24.4, 1999 54.1 -> 49.6; 24/8 1999 52.7 ->
+//             40.8; 16/4 1999 51.6 -> 39.7
+// Of 256 dims a CU is bound by its LDS (each wave reads all of K and V for 32
+// rows of its own): 1999 rows of 8/4 heads 111.7 by one group and by two.
+//
 // Rows of several sequences (a group's prompts in one batch) bring a table:
 // which rows, position and pool a block's tile belongs to, the ones with the
 // most keys first.  A scalar load a block; nothing else differs.
@@ -56,8 +68,19 @@ template <int HD> DEVINL int v_slot(int row, int slot) {
   return slot ^ (x << 2);
 }
 
-template <int HD, int BKV, int NW, bool KV8, bool CAP>
-__global__ void __launch_bounds__(64 * NW, 2)
+// A kv head's part of a range of keys, in the (HD + 4) floats a row that it has.
+// A wave's 32 rows or fewer: row by row.  More: four dims of all rows, the next
+// four, .., then maxima, then sums.  Where that
+// leaves room, rows are counted up to whole lines and parts begin with one.
+struct ApPart { uint32_t rows; size_t size; };
+template <int HD> DEVINL ApPart ap_part(uint32_t rows) {
+  const size_t size = (size_t)rows * (HD + 4);
+  if (rows < 4 * (HD + 2)) return {rows, size};
+  return {(rows + 7) / 8 * 8, size / 32 * 32};
+}
+
+template <int HD, int BKV, int NW, int KG, bool KV8, bool CAP>
+__global__ void __launch_bounds__(64 * NW * KG, KG == 2 && HD == 64 ? 4 : 2)
 k_attn_rows(ApArgs a) {
   constexpr int RB = HD * 2;                 // LDS bytes of a row
   constexpr int TILE = BKV * RB;
@@ -68,23 +91,30 @@ k_attn_rows(ApArgs a) {
   // an array a buffer, and the loop unrolled over the two: the compiler sees
   // that the DMA into one does not touch what is read from the other, and
   // does not wait for it before the reads
-  __shared__ __attribute__((aligned(16))) char K0[TILE], K1[TILE];
-  __shared__ __attribute__((aligned(16))) char V0[TILE], V1[TILE];
-  __shared__ __attribute__((aligned(16))) float S0[2][KV8 ? BKV : 4],
-      S1[2][KV8 ? BKV : 4];
+  __shared__ __attribute__((aligned(16))) char KA[KG * TILE], KB[KG * TILE];
+  __shared__ __attribute__((aligned(16))) char VA[KG * TILE], VB[KG * TILE];
+  __shared__ __attribute__((aligned(16))) float SA[KG][2][KV8 ? BKV : 4],
+      SB[KG][2][KV8 ? BKV : 4];
 
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = KG == 1 ? threadIdx.x : threadIdx.x & (NT - 1);
+  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // tiles of keys go to the groups of waves in turn
+  const int kg = KG == 1 ? 0
+                         : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
+  char *const K0 = KA + kg * TILE, *const K1 = KB + kg * TILE;
+  char *const V0 = VA + kg * TILE, *const V1 = VB + kg * TILE;
+  float(*const S0)[KV8 ? BKV : 4] = SA[kg], (*const S1)[KV8 ? BKV : 4] = SB[kg];
   const int hh = lane >> 5, col = lane & 31;
   const int grp = a.nh / a.kvh;
   // heads vary fastest, so that with a multiple of eight of them the
   // blocks of a kv head land on one XCD and share its L2
   const int kvhead = blockIdx.x;
   const int nq = gridDim.y;
-  // longest rows first; where two blocks a CU hold the whole grid, a long
-  // one shares its CU with a short one
+  // longest rows first; where two blocks a CU hold the whole grid, the second
+  // of a CU come shortest first
   int qt = nq - 1 - (int)blockIdx.y;
-  if (a.fold && (int)blockIdx.y >= nq / 2) qt = (int)blockIdx.y - nq / 2;
+  if ((int)blockIdx.y >= a.fold) qt = (int)blockIdx.y - a.fold;
 
   int base = 0, M = a.M, pool = 0, pos0;
   if (a.tiles) {
@@ -215,16 +245,21 @@ k_attn_rows(ApArgs a) {
   };
 
   // LDS offsets of fragments that the swizzle makes differ by more than a
-  // constant: 8 of K (16-byte slots of a row), 4 of V (64-byte chunks)
+  // constant: 8 of K (16-byte slots of a row), 4 of V (64-byte chunks).  Of 256
+  // dims, where registers are short, they are made for each tile of the first
+  // ones: kept, some were spilled, and their way back waited for the next
+  // tile's DMA (1792 rows of 8/4 heads with a cap, parts
+  // left as they are now: 54.9 us, so 50.4).
   constexpr int KC = HD / 16 < 8 ? HD / 16 : 8, VD = HD / 32 < 4 ? HD / 32 : 4;
+  constexpr bool FEW = HD == 256;
   const int vrow = hh * 4 + ((lane & 15) >> 2);
   const int vcol = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
-  int kb[KC], vb[VD];
+  int kb[FEW ? 1 : KC], vb[FEW ? 1 : VD];
 #pragma unroll
-  for (int c = 0; c < KC; c++)
+  for (int c = 0; c < (FEW ? 1 : KC); c++)
     kb[c] = col * RB + k_slot<HD>(col, c * 2 + hh) * 16;
 #pragma unroll
-  for (int d = 0; d < VD; d++)
+  for (int d = 0; d < (FEW ? 1 : VD); d++)
     vb[d] = vrow * RB + v_slot<HD>(vrow, d * 4 + (vcol >> 3)) * 16 +
             (vcol & 7) * 2;
 
@@ -239,14 +274,18 @@ k_attn_rows(ApArgs a) {
 
   auto tile = [&](char* Ks, char* Vs, float (*Sc)[KV8 ? BKV : 4], char* Kn,
                   char* Vn, float (*Sn)[KV8 ? BKV : 4], int t0) {
-    const bool more = t0 + BKV < k_hi;
+    const bool more = t0 + KG * BKV < k_hi;
     if (more) {
-      if constexpr (KV8) load8(t0 + BKV);
-      else stage16(Kn, Vn, t0 + BKV);
+      if constexpr (KV8) load8(t0 + KG * BKV);
+      else stage16(Kn, Vn, t0 + KG * BKV);
     }
-    const bool some = live && t0 <= q_hi &&
+    const bool some = live && t0 <= q_hi && (KG == 1 || t0 < k_hi) &&
                       (a.window <= 0 || t0 + BKV > q_lo - a.window);
     if (some) {
+      int k0 = kb[0], v0 = vb[0];
+      if constexpr (FEW) asm volatile("" : "+v"(k0), "+v"(v0));
+      auto k_at = [&](int c) { return FEW ? k0 ^ c % KC << 5 : kb[FEW ? 0 : c % KC]; };
+      auto v_at = [&](int d) { return FEW ? v0 ^ d % VD << 6 : vb[FEW ? 0 : d % VD]; };
       ap_f16 s[NS];
 #pragma unroll
       for (int n = 0; n < NS; n++) {
@@ -255,7 +294,7 @@ k_attn_rows(ApArgs a) {
 #pragma unroll
         for (int c = 0; c < HD / 16; c++) {
           const ap_b8 kf = *(const ap_b8*)(
-              Ks + kb[c % KC] + c / KC * 256 + n * 32 * RB);
+              Ks + k_at(c) + c / KC * 256 + n * 32 * RB);
           s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[c], s[n], 0,
                                                          0, 0);
         }
@@ -345,7 +384,7 @@ k_attn_rows(ApArgs a) {
             for (int h = 0; h < 2; h++)
               vf.h[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                   (__attribute__((address_space(3))) ap_s4*)(
-                      Vs + vb[d % VD] + d / VD * 256 +
+                      Vs + v_at(d) + d / VD * 256 +
                       (n * 32 + sl * 16 + h * 8) * RB));
             o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf.v, o[d],
                                                            0, 0, 0);
@@ -356,17 +395,55 @@ k_attn_rows(ApArgs a) {
     if constexpr (KV8) { if (more) store8(Kn, Vn, Sn); }
     __syncthreads();
   };
-  if (k_lo < k_hi) {
-    if constexpr (KV8) { load8(k_lo); store8(K0, V0, S0); }
-    else stage16(K0, V0, k_lo);
+  const int first = k_lo + kg * BKV;         // of the group
+  if (first < k_hi) {
+    if constexpr (KV8) { load8(first); store8(K0, V0, S0); }
+    else stage16(K0, V0, first);
   }
   __syncthreads();
-  for (int t0 = k_lo; t0 < k_hi; t0 += 2 * BKV) {
-    tile(K0, V0, S0, K1, V1, S1, t0);
-    if (t0 + BKV < k_hi) tile(K1, V1, S1, K0, V0, S0, t0 + BKV);
+  for (int t0 = k_lo; t0 < k_hi; t0 += 2 * KG * BKV) {
+    tile(K0, V0, S0, K1, V1, S1, t0 + kg * BKV);
+    if (t0 + KG * BKV < k_hi)
+      tile(K1, V1, S1, K0, V0, S0, t0 + (KG + kg) * BKV);
   }
 
   l += __shfl_xor(l, 32);
+  if constexpr (KG == 2) {
+    // what the second group has, through the LDS that held the keys; lanes of
+    // a wave beside each other
+    static_assert(NW == 4 && 32 * HD * 4 <= KG * TILE);
+    __shared__ float ml[NW][2][64];
+    char* const to = wave == 0 ? KA : wave == 1 ? KB : wave == 2 ? VA : VB;
+    float* const at = (float*)to + lane * 4;
+    if (kg == 1) {
+#pragma unroll
+      for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; q4++)
+          *(f4v*)(at + (d * 4 + q4) * 256) =
+              f4v{o[d][q4 * 4], o[d][q4 * 4 + 1], o[d][q4 * 4 + 2],
+                  o[d][q4 * 4 + 3]};
+      ml[wave][0][lane] = m;
+      ml[wave][1][lane] = l;
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = ml[wave][0][lane], l1 = ml[wave][1][lane];
+    const float mt = fmaxf(m, m1);
+    const float w0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mt);
+    const float w1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mt);
+#pragma unroll
+    for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4++) {
+        const f4v v = *(const f4v*)(at + (d * 4 + q4) * 256);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+          o[d][q4 * 4 + j] = o[d][q4 * 4 + j] * w0 + v[j] * w1;
+      }
+    l = l * w0 + l1 * w1;
+    m = mt;
+  }
   if (row >= nrows) return;
   if (gridDim.z == 1) {
     const float inv = 1.f / l;
@@ -382,7 +459,7 @@ k_attn_rows(ApArgs a) {
           w.b[j / 2][j % 2] = (__bf16)(o[d][q4 * 4 + j] * inv);
         *(unsigned long long*)(op + d * 32 + q4 * 8 + hh * 4) = w.u;
       }
-  } else {
+  } else if constexpr (NW == 1) {
     // unnormalised part of this key range: HD values, maximum, sum
     float* pp = a.part + (((size_t)blockIdx.z * a.kvh + kvhead) * a.M * grp +
                           base * grp + row) * (HD + 4);
@@ -394,9 +471,30 @@ k_attn_rows(ApArgs a) {
             f4v{o[d][q4 * 4], o[d][q4 * 4 + 1], o[d][q4 * 4 + 2],
                 o[d][q4 * 4 + 3]};
     if (hh == 0) { pp[HD] = m; pp[HD + 1] = l; }
+  } else {
+    // Unnormalised part of this key range: the lanes of a store, which are
+    // rows, leave whole lines (each row for itself, 16 bytes a lane: 1000 rows of
+    // 32/8 heads of 64 in two ranges 35.2 us, so 26.7, of 128 40.7, 35.7).
+    const ApPart part = ap_part<HD>(a.M * grp);
+    const uint32_t nr = part.rows, at = base * grp + row;
+    float* pp = a.part + ((size_t)blockIdx.z * a.kvh + kvhead) * part.size;
+    float* to = pp + ((size_t)hh * nr + at) * 4;
+#pragma unroll
+    for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; q4++) {
+        *(f4v*)to = f4v{o[d][q4 * 4], o[d][q4 * 4 + 1], o[d][q4 * 4 + 2],
+                        o[d][q4 * 4 + 3]};
+        to += (size_t)nr * 8;
+      }
+    if (hh == 0) {
+      pp[(size_t)HD * nr + at] = m;
+      pp[(size_t)(HD + 1) * nr + at] = l;
+    }
   }
 }
 
+#define AP_MAX_SPLIT 64
 // the parts of a row, one wave a row
 template <int HD>
 __global__ void __launch_bounds__(256) k_attn_rows_merge(ApArgs a, int split) {
@@ -441,14 +539,76 @@ __global__ void __launch_bounds__(256) k_attn_rows_merge(ApArgs a, int split) {
   for (int i = 0; i < HD / 64; i++) op[i * 64 + lane] = f2b(v[i] / l);
 }
 
-template <int HD, int BKV, int NW, bool KV8>
+// The same of more rows than a wave's, as they lie then: 16 rows of a kv head a
+// block, four where blocks are few, a thread takes ND times four dims of a row.
+// All maxima and sums and the first eight parts are on the way together.  (Two
+// rows of 8/4 heads of 256 over 3000 keys in 47 ranges take 1.1 us longer so, of
+// 64 dims 2.1, than by a wave a row.)
+template <int HD, int R>
+__global__ void __launch_bounds__(256) k_attn_rows_merge_many(ApArgs a, int split) {
+  constexpr int ND = R == 16 ? HD / 64 : 1, NG = HD / 4 / ND;
+  __shared__ float ms[AP_MAX_SPLIT][R], ls[AP_MAX_SPLIT][R];
+  const int tid = threadIdx.x, r = tid % R, g = tid / R;
+  const int grp = a.nh / a.kvh, kvhead = blockIdx.y, all = a.M * grp;
+  const int row = blockIdx.x * R + r, at = min(row, all - 1);
+  const ApPart part = ap_part<HD>(all);
+  const size_t nr = part.rows, stride = a.kvh * part.size;
+  const float* p = a.part + kvhead * part.size;
+  for (int z = g; z < split; z += NG) {
+    ms[z][r] = p[z * stride + HD * nr + at];
+    ls[z][r] = p[z * stride + (HD + 1) * nr + at];
+  }
+  f4v x[8][ND], v[ND];
+  auto ask = [&](int z0) {
+#pragma unroll
+    for (int z = 0; z < 8; z++)
+#pragma unroll
+      for (int i = 0; i < ND; i++)
+        x[z][i] = *(const f4v*)(p + min(z0 + z, split - 1) * stride +
+                                ((g + i * NG) * nr + at) * 4);
+  };
+  ask(0);
+  __syncthreads();
+  float m = -INFINITY, l = 0.f;
+  for (int z0 = 0; z0 < split; z0 += 8)
+#pragma unroll
+    for (int z = 0; z < 8; z++) m = fmaxf(m, ms[min(z0 + z, split - 1)][r]);
+#pragma unroll
+  for (int i = 0; i < ND; i++) v[i] = {0.f, 0.f, 0.f, 0.f};
+  for (int z0 = 0; z0 < split; z0 += 8) {
+    if (z0) ask(z0);
+#pragma unroll
+    for (int z = 0; z < 8; z++) {
+      // a part without keys of this row holds nothing, one that weighs nothing
+      // may hold values without a number
+      const float mz = ms[min(z0 + z, split - 1)][r];
+      const float lz = ls[min(z0 + z, split - 1)][r];
+      if (z0 + z >= split || mz == -INFINITY) continue;
+      const float w = __builtin_amdgcn_exp2f(mz - m);
+      l += lz * w;
+#pragma unroll
+      for (int i = 0; i < ND; i++) v[i] += x[z][i] * w;
+    }
+  }
+  if (row >= all) return;
+  u16* op = a.out + ((size_t)(row / grp) * a.nh + kvhead * grp + row % grp) * HD;
+#pragma unroll
+  for (int i = 0; i < ND; i++) {
+    union { ap_b2 b[2]; unsigned long long u; } o;
+#pragma unroll
+    for (int j = 0; j < 4; j++) o.b[j / 2][j % 2] = (__bf16)(v[i][j] / l);
+    *(unsigned long long*)(op + (g + i * NG) * 4) = o.u;
+  }
+}
+
+template <int HD, int BKV, int NW, int KG, bool KV8>
 static void ap_go(const ApArgs& a, dim3 grid, hipStream_t s) {
   if (a.softcap > 0.f)
-    hipLaunchKernelGGL((k_attn_rows<HD, BKV, NW, KV8, true>), grid,
-                       dim3(64 * NW), 0, s, a);
+    hipLaunchKernelGGL((k_attn_rows<HD, BKV, NW, KG, KV8, true>), grid,
+                       dim3(64 * NW * KG), 0, s, a);
   else
-    hipLaunchKernelGGL((k_attn_rows<HD, BKV, NW, KV8, false>), grid,
-                       dim3(64 * NW), 0, s, a);
+    hipLaunchKernelGGL((k_attn_rows<HD, BKV, NW, KG, KV8, false>), grid,
+                       dim3(64 * NW * KG), 0, s, a);
 }
 
 // Into how many ranges the keys are split where blocks are too few for 256
@@ -474,7 +634,7 @@ static int ap_split(const ApArgs& a, int kv8, int keys, long part_floats,
                                                           : keys;
   const int tiles = (span + BKV - 1) / BKV;
   const long each = (long)a.kvh * a.M * (a.nh / a.kvh) * (HD + 4);
-  int cap = want / blocks < 64 ? want / blocks : 64;
+  int cap = want / blocks < AP_MAX_SPLIT ? want / blocks : AP_MAX_SPLIT;
   if (cap > tiles) cap = tiles;
   if (cap > part_floats / each) cap = (int)(part_floats / each);
   // Where neither was slower before, it stays: beside e4m3 rounding parts of
@@ -511,6 +671,42 @@ static int ap_split(const ApArgs& a, int kv8, int keys, long part_floats,
   return split;
 }
 
+// Whether two groups of waves share a block's keys, rather than `split` ranges.
+// More blocks than CUs: of 64 dims (two such blocks fit a CU) always; of 128 (one
+// does) where blocks differ in length enough that the short ones fill what the
+// long ones leave: few keys ahead of the rows (32/8 heads of 128, 1999 rows
+// 54.1 -> 49.6, behind 2000 keys 114 -> 118, 1365 behind 4000 137 -> 156).  Up
+// to a block a CU, by numbers (us; tiles of the longest block, tiles of a CU,
+// parts of rows in MB) fitted to 255 calls of 11 head layouts, 40 to 2048 rows
+// behind 0 to 6000 keys: 1.25 (64 dims), 1.16 and, e4m3, 1.12 times as fast as
+// ranges alone, none slower (but 80 blocks of 64 dims, five tiles, 9.1 -> 9.5:
+// not below eight).
+// More blocks than 512 and 64 dims of e4m3 (which spill) were not measured.
+template <int HD, int BKV>
+static bool ap_two(const ApArgs& a, int kv8, int keys, int most, int blocks,
+                   int split) {
+  if (HD == 256 || (HD == 64 && kv8) || blocks <= 64 || blocks > 512)
+    return false;
+  const bool bound = a.window > 0 && a.window < keys;
+  if (blocks > 256) return HD == 64 || (2 * (keys - most) < most && !bound);
+  const int span = bound && a.window + most < keys ? a.window + most : keys;
+  const int tiles = (span + BKV - 1) / BKV, per = (tiles + split - 1) / split;
+  if (HD == 64 && tiles < 8) return false;
+  const float mean = bound && a.window < keys - most / 2 ? a.window
+                                                         : keys - most / 2;
+  const float all = blocks * mean / BKV / 256;
+  const float mb = (float)a.kvh * a.M * (a.nh / a.kvh) * (HD + 4) * 4e-6f;
+  static const float fit[3][8] = {
+      {4.49f, 0.6f, 0.244f, 7.f, 0.799f, 0.517f, 2.62f, 0.358f},
+      {5.99f, 0.95f, 0.439f, 9.f, 1.32f, 0.731f, 2.03f, 0.254f},
+      {8.9f, 0.95f, 0.254f, 9.74f, 0.963f, 0.827f, 2.03f, 0.241f}};
+  const float* f = fit[HD == 64 ? 0 : kv8 ? 2 : 1];
+  const float two = f[0] + f[1] * tiles + f[2] * all;
+  const float one = f[3] + f[4] * per + f[5] * all +
+                    (split > 1 ? f[6] + f[7] * split * mb : 0.f);
+  return two < one;
+}
+
 // most: rows of the longest sequence; ntiles: of several sequences
 template <int HD, int BKV>
 static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
@@ -519,20 +715,40 @@ static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
   // up to 32 rows are one wave's; more share their tiles among four
   const int nw = most * (a.nh / a.kvh) <= 32 ? 1 : 4;
   const int tiles = a.tiles ? ntiles : (rows + nw * 32 - 1) / (nw * 32);
-  const int split = ap_split<HD, BKV>(a, kv8, keys, part_floats, most, nw,
-                                      tiles * a.kvh);
-  a.fold = !a.tiles && split == 1 && tiles % 2 == 0 && tiles * a.kvh <= 512;
+  int split = ap_split<HD, BKV>(a, kv8, keys, part_floats, most, nw,
+                                tiles * a.kvh);
+  const bool two = nw == 4 && ap_two<HD, BKV>(a, kv8, keys, most,
+                                              tiles * a.kvh, split);
+  if (two) split = 1;
+  // A block a CU, then the second of each (two groups of 128 dims have a CU to
+  // themselves).  us, longest first -> so: 64 dims 1999 rows of 32/8 heads 32.4
+  // -> 29.9, 2000 behind 2000 keys 72.3 -> 68.0; 128 dims 54.1 -> 52.3.
+  a.fold = tiles;
+  if (!a.tiles && split == 1 && tiles * a.kvh <= 512 && !(two && HD == 128))
+    a.fold = a.kvh < 256 ? 256 / a.kvh : 1;
   dim3 grid(a.kvh, tiles, split);
   if (nw == 1) {
-    if (kv8) ap_go<HD, BKV, 1, true>(a, grid, s);
-    else ap_go<HD, BKV, 1, false>(a, grid, s);
+    if (kv8) ap_go<HD, BKV, 1, 1, true>(a, grid, s);
+    else ap_go<HD, BKV, 1, 1, false>(a, grid, s);
+  } else if (two) {
+    if constexpr (HD == 128)
+      if (kv8) ap_go<HD, BKV, 4, 2, true>(a, grid, s);
+    if constexpr (HD <= 128)
+      if (!kv8) ap_go<HD, BKV, 4, 2, false>(a, grid, s);
   } else {
-    if (kv8) ap_go<HD, BKV, 4, true>(a, grid, s);
-    else ap_go<HD, BKV, 4, false>(a, grid, s);
+    if (kv8) ap_go<HD, BKV, 4, 1, true>(a, grid, s);
+    else ap_go<HD, BKV, 4, 1, false>(a, grid, s);
   }
-  if (split > 1)
+  if (split > 1 && nw == 1)
     hipLaunchKernelGGL((k_attn_rows_merge<HD>), dim3((rows * a.kvh + 3) / 4),
                        dim3(256), 0, s, a, split);
+  else if (split > 1 && (long)rows * a.kvh < 16 * 256)
+    hipLaunchKernelGGL((k_attn_rows_merge_many<HD, 4>),
+                       dim3((rows + 3) / 4, a.kvh), dim3(HD), 0, s, a, split);
+  else if (split > 1)
+    hipLaunchKernelGGL((k_attn_rows_merge_many<HD, 16>),
+                       dim3((rows + 15) / 16, a.kvh), dim3(256), 0, s, a,
+                       split);
   return hipGetLastError();
 }
 

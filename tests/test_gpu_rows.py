@@ -67,6 +67,25 @@ def test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8):
     assert (out[M] == 7.0).all()
 
 
+# blocks of which two groups of waves take the keys in turn: up to a block a CU
+# and more, one tile of keys (the second group has none), an odd number, keys
+# ahead of the rows, windows, a cap; rows that end inside a wave; and as many
+# blocks in ranges, of 256 dims and of e4m3 keys of 64
+@pytest.mark.parametrize("hd,nh,kvh,M,pos0,window,cap,kv8", [
+    (64, 80, 80, 50, 0, 0, 0.0, False), (64, 32, 8, 333, 0, 0, 0.0, False),
+    (64, 32, 8, 611, 70, 0, 30.0, False), (64, 40, 8, 1037, 0, 0, 0.0, False),
+    (64, 32, 8, 500, 300, 200, 0.0, False),
+    (64, 32, 8, 611, 0, 0, 0.0, True),
+    (128, 72, 72, 64, 0, 0, 0.0, False), (128, 32, 8, 430, 0, 0, 0.0, False),
+    (128, 16, 4, 1100, 33, 0, 50.0, False), (128, 24, 8, 1450, 0, 0, 0.0, False),
+    (128, 32, 8, 480, 100, 130, 0.0, False),
+    (128, 32, 8, 430, 5, 0, 0.0, True), (128, 24, 8, 1450, 0, 0, 0.0, True),
+    (256, 16, 8, 601, 0, 0, 50.0, False)])
+def test_prompt_attention_of_many_blocks(hd, nh, kvh, M, pos0, window, cap,
+                                         kv8):
+    test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8)
+
+
 # a part of the keys whose weight beside the others' underflows, with values
 # that are no number: as in one softmax, 0 times them is none either
 @pytest.mark.parametrize("hd", [64, 128, 256])
