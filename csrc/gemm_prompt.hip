@@ -506,6 +506,10 @@ k_gemm_prompt(GpArgs a) {
 // of the next tile where a tile ends: none waits for its first slabs but the
 // first.  Behind the last one loads go on, to one line, so that the waits
 // count alike.
+//
+// Of routed experts (MOE) the blocks share the row tiles that have rows: with
+// the empty ones left in place some had a tile more than others (1100 rows, 8
+// experts, 2048->2x4096: 130 us, so 107).
 #define GW_RING 9
 // 64 lanes of 16 bytes to lds and behind it
 template <bool NT = false>
@@ -531,7 +535,7 @@ template <int N> DEVINL void gw_wait() {
   asm volatile("" ::: "memory");
 }
 
-template <bool F8, int HA, bool GLU, bool NT>
+template <bool F8, int HA, bool GLU, bool NT, bool MOE = false>
 __global__ void __launch_bounds__(512) k_gemm_wide(GpArgs a, int SK) {
   constexpr int BM = 128 * HA, BN = 256, FM = 4 * HA, FN = 4;
   __shared__ __attribute__((aligned(16))) char ring[GW_RING * 16384];
@@ -540,6 +544,12 @@ __global__ void __launch_bounds__(512) k_gemm_wide(GpArgs a, int SK) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
+  if constexpr (MOE) {
+    // row tiles that have rows: the last E of those counted on may have none
+    const int t = a.tm - 1 - lane;
+    a.tm -= __popcll(__ballot(t >= 0 && a.tile_n[max(t, 0)] == 0));
+    a.band = a.tm;
+  }
   // Work of an XCD (block id modulo 8): neighbouring tiles, rows fastest, in
   // each part of K.  A block takes every step-th item of it.
   const int tiles = a.tm * a.tn, chunk = (tiles + 7) / 8, items = chunk * SK;
@@ -579,18 +589,26 @@ __global__ void __launch_bounds__(512) k_gemm_wide(GpArgs a, int SK) {
     const int tile = t0 + ahead % chunk, lo = ahead / chunk * per;
     left = min(per, slabs - lo);
     const GpAt at = gp_at(a, tile);
-    const int bm = at.row * BM, bn = at.col * (GLU ? BN / 2 : BN);
+    const int bm = MOE ? 0 : at.row * BM, bn = at.col * (GLU ? BN / 2 : BN);
+    const int rows = MOE ? a.tile_n[at.row] : a.M - bm;
+    const int first = MOE ? a.tile_row0[at.row] : 0;
     xp = (const char*)a.x + (size_t)bm * rowb + (size_t)lo * 128;
     // 16 rows of the gate, 16 of what it gates
     wp = (const char*)a.w + (size_t)bn * rowb + (size_t)lo * 128 +
          (GLU && (wave & 1) ? (size_t)a.N * rowb : 0);
+    if (MOE)
+      wp += (size_t)__builtin_amdgcn_readfirstlane(a.tile_e[at.row]) *
+            (GLU ? 2 : 1) * a.N * rowb;
 #pragma unroll
     for (int t = 0; t < 2; t++) {
       const int r = (wave * 2 + t) * 8 + g_r;
       const uint32_t o = t ? src ^ 64 : src;
 #pragma unroll
-      for (int h = 0; h < HA; h++)
-        pa[h][t] = (uint32_t)min(h * 128 + r, a.M - 1 - bm) * (uint32_t)rowb + o;
+      for (int h = 0; h < HA; h++) {
+        int x = min(h * 128 + r, rows - 1);
+        if (MOE) x = a.gather ? a.perm[first + x] / a.top : first + x;
+        pa[h][t] = (uint32_t)x * (uint32_t)rowb + o;
+      }
 #pragma unroll
       for (int h = 0; h < 2; h++) {
         const int c = h * 128 + r;
@@ -687,7 +705,12 @@ __global__ void __launch_bounds__(512) k_gemm_wide(GpArgs a, int SK) {
   for (;;) {
     const int tile = t0 + item % chunk, part = item / chunk;
     const GpAt at = gp_at(a, tile);
-    const int bm = at.row * BM, bn = at.col * (GLU ? BN / 2 : BN);
+    const int bm = MOE ? 0 : at.row * BM, bn = at.col * (GLU ? BN / 2 : BN);
+    const int rows = MOE ? a.tile_n[at.row] : a.M;
+    const int first = MOE ? a.tile_row0[at.row] : 0;
+    const int* const perm = MOE ? a.perm + first : nullptr;
+    const size_t w0 =
+        MOE ? (size_t)a.tile_e[at.row] * (GLU ? 2 : 1) * a.N : 0;
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
@@ -740,11 +763,13 @@ __global__ void __launch_bounds__(512) k_gemm_wide(GpArgs a, int SK) {
     }
     if (!wm) gw_meet();
     item = there(item + step);
-    gp_finish<F8, BM, BN, 8, FM, FN, GLU, false, HA == 1>(
-        a, acc, tile, part, SK, bm, bn, a.M, 0, nullptr, 0, &last_flag,
+    gp_finish<F8, BM, BN, 8, FM, FN, GLU, MOE, HA == 1 && !MOE>(
+        a, acc, tile, part, SK, bm, bn, rows, first, perm, w0, &last_flag,
         [&](int i) { return (i >> 2) * 128 + wm * 64 + (i & 3) * 16; },
         [&](int j) { return (j >> 1) * 128 + wn * 32 + (j & 1) * 16; },
-        [](int r) { return r; });
+        [&](int r) {
+          return !MOE ? r : a.gather ? perm[r] / a.top : first + r;
+        });
     if (item >= items) break;
   }
   gw_wait<0>();
@@ -1158,6 +1183,29 @@ extern "C" hipError_t launch_expert_gemm(
               nullptr, (u16*)y, nullptr, nullptr, pairs, N, K, act, tiles, 0, tiles,
               p, p + pairs, p + pairs + tiles, p + pairs + 2 * tiles, top,
               gather};
+  // 128x256 tiles in turns with more than a 128x128 tile a CU to do, half a
+  // row tile an expert counted on for the last of its rows: 8 experts, 1100
+  // rows, 2 each, 2048->2x4096 143 us, so 107 (e4m3 101, 69), 4096->2048 80,
+  // 64; 700 rows 4096->2x14336 594, 478; 16 experts of 1024 30, 21.  With a
+  // tile a CU or less the small ones end sooner: 700 rows 4096->2048 46,
+  // 60.  Row offsets have 32 bits.
+  const int glu = act >= 0 ? 2 : 1;
+  if (bm == 128 && (!sx || K % 128 == 0) &&
+      (size_t)pairs * K * (sx ? 1 : 2) <= UINT32_MAX &&
+      (pairs / 128 + E / 2) * ((N * glu + 127L) / 128) > 256) {
+    a.tn = (N * glu + 255) / 256;
+    const int share = (tiles * a.tn + 7) / 8;
+    const dim3 grid(8 * (share < 32 ? share : 32)), nt(512);
+#define WIDE(F8, GLU)                                                        \
+  hipLaunchKernelGGL((k_gemm_wide<F8, 1, GLU, false, true>), grid, nt, 0,    \
+                     stream, a, 1)
+    if (sx && act >= 0) WIDE(true, true);
+    else if (sx) WIDE(true, false);
+    else if (act >= 0) WIDE(false, true);
+    else WIDE(false, false);
+#undef WIDE
+    return hipGetLastError();
+  }
 #define EXPERTS(F8)                                                          \
   return bm == 128  ? gp_experts<F8, 128, 128, 2, 4, 4>(a, stream)           \
          : bm == 64 ? gp_experts<F8, 64, 64, 4, 2, 4>(a, stream)             \

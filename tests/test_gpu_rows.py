@@ -648,10 +648,9 @@ def test_two_norms(M, H):
 @pytest.mark.parametrize("M,E,top", [(1, 8, 2), (40, 8, 3), (200, 9, 2),
                                      (330, 4, 2), (70, 64, 8)])
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
-def test_experts_of_many_rows(M, E, top, kind):
+def test_experts_of_many_rows(M, E, top, kind, H=192, I=320):
     from llm_np_cp_amd.ops import hip_ops as ho
 
-    H, I = 192, 320
     up, dn = (normal(E * r, k, seed=s, scale=k ** -0.5)
               for r, k, s in ((2 * I, H, 1), (H, I, 2)))
     x, h = normal(M, H, seed=3), normal(M, H, seed=4)
@@ -699,6 +698,16 @@ def test_experts_of_many_rows(M, E, top, kind):
                       * p.double()[..., None]).sum(1)
     assert off(out, z) < 2.0 ** -8 * top            # bf16 after each expert
     assert (a[pairs] == 7.0).all() and (y[pairs] == 7.0).all()
+
+
+# more 128x128 tiles than CUs: outputs that end within a tile 256 wide, one
+# slab, experts without rows, the first product alone past the line
+@pytest.mark.parametrize("M,E,top,H,I", [
+    (1500, 4, 2, 1408, 704), (1500, 4, 2, 1408, 768), (900, 64, 8, 64, 192),
+    (2200, 1, 1, 2112, 1088), (520, 8, 2, 384, 1536), (300, 3, 1, 640, 5504)])
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+def test_experts_of_wide_tiles(M, E, top, H, I, kind):
+    test_experts_of_many_rows(M, E, top, kind, H, I)
 
 
 # a row, a few, a group in larger blocks, a large one in fewer; a vocabulary of
