@@ -17,14 +17,14 @@
 //
 // What bounds it: head_dim 128 spends 512 MFMA cycles and about 450 VALU
 // cycles on 32 keys x 32 rows; two blocks of 64 KB LDS on a CU overlap them.
-// Measured (32/8 heads of 128, 2048 rows behind 6139 keys): 291 us,
-// 827 TFLOP/s; a wave per head and 16 queries took 1422 us.  (With both
+// Measured (32/8 heads of 128, 2048 rows behind 6139 keys): 270 us,
+// 890 TFLOP/s; a wave per head and 16 queries took 1422 us.  (With both
 // buffers in one array the DMA drained ahead of every tile's reads: 314 us.)
-// 5 rows of 24/8 heads over 906 keys, split: 14 us, unsplit per-head waves
-// 74 us.  Head dim 256 at two waves a SIMD just fits the registers without a
-// soft cap; with one it spills 7, beside an e4m3 pool 36 (12 to 14 where one
-// wave has all rows).  One wave a SIMD without spills was slower (2048 rows
-// behind 2048 keys: 219 us to 163 when it still spilled 20, now 118).
+// 5 rows of 24/8 heads over 906 keys, split: 11 us, unsplit per-head waves
+// 74 us.  Head dim 256 at two waves a SIMD just fits the registers where LDS
+// addresses are made again for each tile (2048 rows of 16/8 heads behind 2048
+// keys with a soft cap 181 us, so 177); beside an e4m3 pool it spills 27 (6
+// where one wave has all rows).  One wave a SIMD without spills was slower.
 //
 // Where a block's own keys are what takes long (the last rows of a prompt see
 // all of them, and a block goes through its tiles one after the other), two

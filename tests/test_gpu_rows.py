@@ -357,6 +357,20 @@ def test_many_rows_of_wide_tiles(M, N, K, kind, act):
     test_many_rows(M, N, K, kind, act)
 
 
+# one row of tiles beside 32 MB of W or just less of it: read past the caches
+# by each tile of up to 128 rows, with a rest both ways and parts of K
+@pytest.mark.parametrize("M,N,K,kind,act", [
+    (37, 8203, 2048, "bf16", 0), (61, 2050, 8256, "bf16", -1),
+    (65, 16850, 1088, "bf16", -1), (99, 9001, 2048, "bf16", -1),
+    (128, 14300, 2048, "bf16", 0), (128, 28690, 640, "bf16", -1),
+    (128, 8190, 2048, "bf16", -1), (70, 4110, 8192, "bf16", -1),
+    (33, 8203, 4096, "fp8", 0), (57, 16500, 2176, "fp8", -1),
+    (128, 8400, 2176, "fp8", 0), (121, 17010, 2112, "fp8", -1),
+    (128, 34000, 1024, "fp8", -1), (128, 4099, 8320, "fp8", -1)])
+def test_many_rows_beside_large_weights(M, N, K, kind, act):
+    test_many_rows(M, N, K, kind, act)
+
+
 # rows so long that 32 bits do not reach those of a tile: of the largest (256
 # rows of 2^24 bytes), and of the one that takes them (64 rows of 66 MB)
 @pytest.mark.parametrize("kind,act,K", [
