@@ -54,27 +54,6 @@ DEVINL int v_place(int j) {
   return (j & 32) | ((j >> 2) & 3) << 3 | ((j >> 4) & 1) << 2 | (j & 3);
 }
 
-DEVINL float sum_squares(const float* p, int n, float* red) {
-  float ss = 0.f;
-#pragma unroll 4
-  for (int i = threadIdx.x; i < n; i += blockDim.x) ss += p[i] * p[i];
-  return block_sum(ss, red);
-}
-
-// key and value of key/value head g, written to the cache
-template <typename T>
-DEVINL void write_kv(const GqaArgs& a, const float* p, int page, int at, int g,
-                     float rk) {
-  T* K = (T*)a.K + (((size_t)page * a.G + g) * PAGE + at) * a.DP;
-  const float* k = p + a.ok + g * a.d;
-  for (int i = threadIdx.x; i < a.DP; i += blockDim.x)
-    K[i] = El<T>::st(i < a.d ? k[i] * rk * a.knorm[g * a.d + i] : 0.f);
-  T* V = (T*)a.V + ((size_t)page * a.G + g) * a.VP * PAGE + v_place(at);
-  const float* v = p + a.ov + g * a.vd;
-  for (int i = threadIdx.x; i < a.vd; i += blockDim.x)
-    V[(size_t)i * PAGE] = El<T>::st(v[i]);
-}
-
 // ---- runs: normed queries, keys and values -------------------------------
 // a block per row for queries and keys; blocks of PREP_ROWS rows for the
 // values, since those of neighbouring positions share a line of V
@@ -207,18 +186,45 @@ DEVINL void drop_unwritten(f4v* v, int k0, int g, int kend) {
   }
 }
 
+// one key's value among them, before any that no token has written
+template <typename T>
+DEVINL void put_value(f4v* v, int k0, int g, int key, T val) {
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const bool at = k0 + (i >> 2) * 16 + g * 4 + (i & 3) == key;
+    if constexpr (sizeof(T) == 2) {
+      union { f4v f; u16 h[8]; } o;
+      o.f = v[0];
+      o.h[i] = at ? val : o.h[i];
+      v[0] = o.f;
+    } else {
+      v[i >> 2][i & 3] = at ? val : v[i >> 2][i & 3];
+    }
+  }
+}
+
 // ---- single tokens --------------------------------------------------------
 // A block takes one row, key/value head and share of the keys: group s of
 // 128 keys, then s + NS, ...; its 4 waves take 32 keys each, straight from
 // the cache, and merge at the end.  The blocks normalise the query
-// themselves; the one whose share ends with the new token writes its key
-// and value first.
+// themselves; the one whose share ends with the new token makes its key and
+// value too, and puts them in their places among those that it has read.
+//
+// What bounds it is a chain of trips to memory, so each is asked for as soon as
+// its place is known: keys and values were read behind the query's norm, and
+// behind the new token's key on its way through the cache.  us, 4 rows of 16/4
+// heads of 128 behind 520 keys 9.9 -> 8.8, 64 of them 37.4 -> 34.7 at 1500
+// keys, 8 of 32/8 of 64 at 2000 15.1 -> 11.8, one of 32/8 of 128 at 30000 31.5
+// -> 27.1; in fp32 12.9 -> 12.3.
+#define TOKEN_U 8            // query elements that a thread asks for at once
 template <typename T, int DP, int VP>
 __global__ void __launch_bounds__(256) k_gqa_token(GqaArgs a) {
   constexpr int SZ = sizeof(T), NC = DP * SZ / 64, ND = VP / 16, VV = SZ / 2;
   constexpr int XS = 32 * VP > 4 * DP * SZ ? 32 * VP : 4 * DP * SZ;
   __shared__ __attribute__((aligned(16))) float xs[XS];
-  __shared__ float red[4], ms[4][16], ls[4][16];
+  constexpr int QU = 16 * DP / 256;     // staged query elements of a thread
+  __shared__ float red[2][4], ms[4][16], ls[4][16];
+  __shared__ __attribute__((aligned(16))) T newk[DP], newv[VP];
   T* qs = (T*)xs;                       // [16][DP], then partials [2][16][VP]
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int qc = lane & 15, g = lane >> 4;
@@ -227,8 +233,18 @@ __global__ void __launch_bounds__(256) k_gqa_token(GqaArgs a) {
   const int r = blockIdx.x / (nqt * a.G);       // from rbase, which is 0
   const int nq = min(16, R - qt * 16), h0 = kv * R + qt * 16;
   const float* p = a.P + (size_t)r * a.ldp;
-  const int pos = a.pos[r], kend = pos + 1;
-  const int* pages = a.table + (size_t)a.slot[r] * a.ldt;
+  // All that comes from memory is asked for as soon as its place is known: the
+  // projections, keys and values of the first group, the new token's.
+  const int nqd = a.H * a.d, nkd = a.G * a.d;
+  float pv[TOKEN_U];
+#pragma unroll
+  for (int u = 0; u < TOKEN_U; u++) {
+    const int i = tid + u * 256;
+    pv[u] = i < nqd ? p[a.oq + i] : 0.f;
+  }
+  const int pos = a.pos[r], slot = a.slot[r], kend = pos + 1;
+  asm volatile("" :: "s"(slot));       // on its way with pos, not behind it
+  const int* pages = a.table + (size_t)slot * a.ldt;
   // groups from the first key that is seen
   const int k_lo = first_seen(a, pos), g0 = k_lo / 128;
   const int ngroup = (kend + 127) / 128 - g0, split = blockIdx.y;
@@ -239,21 +255,93 @@ __global__ void __launch_bounds__(256) k_gqa_token(GqaArgs a) {
     if (tid < nq) a.ml[(split * n + orow + tid) * 2 + 1] = 0.f;
     return;
   }
-  const float rq =
-      (a.temp ? a.temp[pos] : 1.f) / sqrtf(sum_squares(p + a.oq, a.H * a.d, red) /
-                              (float)(a.H * a.d) + a.eps);
-  if ((ngroup - 1) % a.NS == split) {
-    // blocks of one key/value head (nqt > 1) write the same values
-    const float rk =
-        1.f / sqrtf(sum_squares(p + a.ok, a.G * a.d, red) /
-                        (float)(a.G * a.d) + a.eps);
-    write_kv<T>(a, p, pages[pos / PAGE], pos % PAGE, kv, rk);
+  // the block whose share ends with the new token
+  const bool fresh = (ngroup - 1) % a.NS == split;
+  const int page = fresh ? pages[pos / PAGE] : 0;
+  float qv[QU], qn[QU], kx = 0.f, kn = 0.f, vx = 0.f, sk = 0.f;
+#pragma unroll
+  for (int u = 0; u < QU; u++) {
+    const int i = tid + u * 256, c = i / DP, j = i - c * DP;
+    const int e = (h0 + c) * a.d + j;
+    const bool in = c < nq && j < a.d;
+    qv[u] = in ? p[a.oq + e] : 0.f;
+    qn[u] = in ? a.qnorm[e] : 0.f;
   }
-  for (int i = tid; i < 16 * DP; i += 256) {
-    const int c = i / DP, j = i - c * DP, s = (h0 + c) * a.d + j;
-    qs[i] = El<T>::st(c < nq && j < a.d ? p[a.oq + s] * rq * a.qnorm[s] : 0.f);
+  if (fresh) {
+    if (tid < a.d) {
+      kx = p[a.ok + kv * a.d + tid];
+      kn = a.knorm[kv * a.d + tid];
+    }
+    if (tid < a.vd) vx = p[a.ov + kv * a.vd + tid];
+#pragma unroll 4
+    for (int i = tid; i < nkd; i += 256) sk += p[a.ok + i] * p[a.ok + i];
   }
-  __syncthreads();              // publishes qs, and the new key to the block
+  const float* bias =
+      a.bias ? a.bias + (size_t)(h0 + min(qc, nq - 1)) * a.nbias : nullptr;
+  f4v kf[2][NC], vf[ND][VV];
+  float bv[8];
+  auto fetch = [&](int k0) {
+    const size_t pg = (size_t)pages[k0 / PAGE] * a.G + kv;
+    const char* K = (const char*)((const T*)a.K +
+                                  (pg * PAGE + k0 % PAGE + qc) * DP) + g * 16;
+    const char* V = (const char*)((const T*)a.V + (pg * VP + qc) * PAGE +
+                                  k0 % PAGE + g * 8);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int c = 0; c < NC; c++)
+        kf[i][c] = ld16(K + (size_t)i * 16 * DP * SZ + c * 64);
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+      for (int u = 0; u < VV; u++)
+        vf[d][u] = ld16(V + (size_t)d * 16 * PAGE * SZ + u * 16);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int n = pos - (k0 + (i >> 2) * 16 + g * 4 + (i & 3));
+      bv[i] = bias ? bias[min(max(n, 0), a.nbias - 1)] : 0.f;
+    }
+  };
+  const int first = (g0 + split) * 128 + wave * 32;
+  if (first < kend && first + 32 > k_lo) fetch(first);
+
+  float sq = 0.f;
+#pragma unroll
+  for (int u = 0; u < TOKEN_U; u++) sq += pv[u] * pv[u];
+#pragma unroll 4
+  for (int i = tid + TOKEN_U * 256; i < nqd; i += 256)
+    sq += p[a.oq + i] * p[a.oq + i];
+  sq = wave_reduce_sum(sq);
+  if (fresh) sk = wave_reduce_sum(sk);
+  if (lane == 0) {
+    red[0][wave] = sq;
+    red[1][wave] = sk;
+  }
+  __syncthreads();
+  sq = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+  sk = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+  const float rq = (a.temp ? a.temp[pos] : 1.f) / sqrtf(sq / (float)nqd + a.eps);
+#pragma unroll
+  for (int u = 0; u < QU; u++)
+    qs[tid + u * 256] = El<T>::st(qv[u] * rq * qn[u]);
+  if (fresh) {
+    // to the cache (blocks of one key/value head, nqt > 1, write the same
+    // values), and to where the waves take it from
+    const float rk = 1.f / sqrtf(sk / (float)nkd + a.eps);
+    const size_t at = (size_t)page * a.G + kv;
+    if (tid < DP) {
+      const T v = El<T>::st(tid < a.d ? kx * rk * kn : 0.f);
+      newk[tid] = v;
+      ((T*)a.K)[(at * PAGE + pos % PAGE) * DP + tid] = v;
+    }
+    if (tid < VP) {
+      const T v = El<T>::st(vx);
+      newv[tid] = v;
+      if (tid < a.vd)
+        ((T*)a.V)[(at * VP + tid) * PAGE + v_place(pos % PAGE)] = v;
+    }
+  }
+  __syncthreads();              // publishes qs, and the new token to the block
   f4v qf[NC];
 #pragma unroll
   for (int c = 0; c < NC; c++)
@@ -268,33 +356,22 @@ __global__ void __launch_bounds__(256) k_gqa_token(GqaArgs a) {
     mrun = a.sink[hq];
     lrun = 1.f;
   }
-  const float* bias = a.bias ? a.bias + (size_t)hq * a.nbias : nullptr;
 
   for (int grp = g0 + split; grp < g0 + ngroup; grp += a.NS) {
     const int k0 = grp * 128 + wave * 32;
     if (k0 >= kend) break;
     if (k0 + 32 <= k_lo) continue;
-    const size_t pg = (size_t)pages[k0 / PAGE] * a.G + kv;
-    const char* K = (const char*)((const T*)a.K +
-                                  (pg * PAGE + k0 % PAGE + qc) * DP) + g * 16;
-    const char* V = (const char*)((const T*)a.V + (pg * VP + qc) * PAGE +
-                                  k0 % PAGE + g * 8);
-    f4v kf[2][NC], vf[ND][VV];
+    if (k0 != first) fetch(k0);
+    if (fresh && k0 + 32 > pos) {        // the new token's, not there when asked
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+      for (int i = 0; i < 2; i++)
+        if (k0 + i * 16 + qc == pos)
 #pragma unroll
-      for (int c = 0; c < NC; c++)
-        kf[i][c] = ld16(K + (size_t)i * 16 * DP * SZ + c * 64);
+          for (int c = 0; c < NC; c++)
+            kf[i][c] = ld16((const char*)newk + c * 64 + g * 16);
 #pragma unroll
-    for (int d = 0; d < ND; d++)
-#pragma unroll
-      for (int u = 0; u < VV; u++)
-        vf[d][u] = ld16(V + (size_t)d * 16 * PAGE * SZ + u * 16);
-    float bv[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int n = pos - (k0 + (i >> 2) * 16 + g * 4 + (i & 3));
-      bv[i] = bias ? bias[min(max(n, 0), a.nbias - 1)] : 0.f;
+      for (int d = 0; d < ND; d++)
+        put_value<T>(vf[d], k0, g, pos, newv[d * 16 + qc]);
     }
     f4v st[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll

@@ -129,6 +129,69 @@ def test_launchers_refuse_bad_shapes():
                                                  nvt=1))
 
 
+# the new token first, last and amid a share's 32 keys, a page, 128 keys; in a
+# share's first group and in a later one; a cache that holds anything where no
+# token has written
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H, G, d, vd", [(6, 2, 40, 72), (17, 1, 64, 30),
+                                         (4, 4, 130, 20)])
+@pytest.mark.parametrize("pos, NS", [([0, 31, 32], 1), ([63, 64, 127], 2),
+                                     ([128, 500, 255], 2), ([300, 1, 17], 5)])
+def test_new_token_among_keys_read_before_it(dtype, H, G, d, vd, pos, NS):
+    from llm_np_cp_amd.ops import hybrid_ops as hy
+
+    g = torch.Generator(device="cuda").manual_seed(d)
+    R = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    DP, VP = (256, 256) if d > 128 else (64, 64 if vd <= 64 else 128)
+    n, per, R_ = len(pos), max(pos) // 64 + 1, H // G
+    ov = H * d + G * d
+    P, qn, kn = R(n, ov + G * vd), R(H * d), R(G * d)
+    table = i32(*torch.randperm(n * per).tolist()).view(n, per)
+    K = torch.full((n * per, G, 64, DP), float("nan"), device="cuda",
+                   dtype=dtype)
+    V = torch.full((n * per, G, VP, 64), float("nan"), device="cuda",
+                   dtype=dtype)
+    K[..., d:] = 0
+    V[:, :, vd:] = 0
+    norm = lambda x: x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-5)
+    q = (norm(P[:, :H * d]) * qn).to(dtype).double().view(n, H, d)
+    k1 = (norm(P[:, H * d:ov]) * kn).to(dtype).view(n, G, d)
+    v1 = P[:, ov:].to(dtype).view(n, G, vd)
+    want = torch.zeros(n, H, vd, dtype=torch.float64)
+    for r in range(n):
+        ks, vs = R(pos[r], G, d).to(dtype), R(pos[r], G, vd).to(dtype)
+        for j in range(pos[r]):
+            at, o = int(table[r, j // 64]), j % 64
+            K[at, :, o, :d] = ks[j]
+            V[at, :, :vd, (o & 32) | ((o >> 2) & 3) << 3 | ((o >> 4) & 1) << 2
+              | (o & 3)] = vs[j]
+        ks, vs = torch.cat([ks, k1[r:r + 1]]), torch.cat([vs, v1[r:r + 1]])
+        for h in range(H):
+            s = ks[:, h // R_].double() @ q[r, h] * d ** -0.5
+            want[r, h] = (s.softmax(0) @ vs[:, h // R_].double()).cpu()
+    part = torch.zeros(NS, n * H, VP, device="cuda")
+    ml = torch.zeros(NS, n * H, 2, device="cuda")
+    out = torch.zeros(n, H * vd, device="cuda", dtype=dtype)
+    f32, slot, at = int(dtype == torch.float32), i32(*range(n)), i32(*pos)
+    a = hy.GqaArgs().put(
+        P=P, qnorm=qn, knorm=kn, slot=slot, pos=at,
+        table=table, K=K, V=V, part=part, ml=ml, o=out, ldp=P.shape[1], oq=0,
+        ok=H * d, ov=ov, og=-1, H=H, G=G, d=d, vd=vd, DP=DP, VP=VP,
+        ldo=H * vd, ldt=per, rows=n, rbase=0, NS=NS, eps=1e-5,
+        scale=d ** -0.5)
+    hy.gqa_token(f32, a)
+    hy.gqa_merge(f32, a)
+    # bf16: keys and queries a unit apart where the norm's sum has another
+    # order (2^-8 of some), probabilities and results rounded (2^-9 each)
+    assert rel(_np(out), want.view(n, -1).numpy()) < (
+        1e-5 if f32 else 2.0 ** -7)
+    for r in range(n):
+        o = pos[r] % 64
+        new = K[table[r, pos[r] // 64], :, o, :d]
+        assert rel(_np(new), _np(k1[r])) < (1e-5 if f32 else 2.0 ** -8)
+
+
 # -------------------------------------------------------- mechanisms alone
 
 def check_alone(cfg, n=150, seed=0, cuts=None):
