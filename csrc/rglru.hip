@@ -52,13 +52,14 @@ DEVINL float one_minus_exp(float x, float e) {
   return x * s;
 }
 
-// decay and input weight of one channel from the gate sums
-DEVINL void recur(const RglruArgs& a, int c, float r, float i, float u,
+// decay and input weight of one channel from the gate sums, their biases and
+// its rate
+DEVINL void recur(float rb, float ib, float nl, float r, float i, float u,
                   float& dec, float& add) {
-  const float la = fast_sigmoid(r + a.rb[c]) * a.nl[c];
+  const float la = fast_sigmoid(r + rb) * nl;
   dec = fast_exp(la);
   add = __builtin_amdgcn_sqrtf(one_minus_exp(-2.f * la, dec * dec)) *
-        fast_sigmoid(i + a.ib[c]) * u;
+        fast_sigmoid(i + ib) * u;
 }
 
 // C += A B^T of 16 rows of fp32 `u` (LDS, this lane's row) and 16 rows of
@@ -100,7 +101,12 @@ template <> struct GateMma<u16> {
 
 // ---- one token per row ------------------------------------------------
 // a block: 16 channels of one part; 16 lanes per channel share its two dot
-// products over the part's convolved inputs
+// products over the part's convolved inputs.  What bounds it is the way of all
+// that it reads, so nothing waits for something else: taps, states and what
+// the epilogue takes are asked for ahead of the convolution (us, 16 parts of
+// 128, 4 taps: 4 rows 4.2 -> 3.3, 16 rows 6.3 -> 5.2, 64 rows 16.8 -> 13.1; tap
+// after tap, behind a division of its own each, and the state at the end).
+#define STEP_TAPS 4
 template <typename T>
 __global__ void __launch_bounds__(256) k_rglru_step(RglruArgs a) {
   constexpr int V = El<T>::V;
@@ -117,17 +123,32 @@ __global__ void __launch_bounds__(256) k_rglru_step(RglruArgs a) {
   const T* wi = wr + (size_t)a.KP * a.KP;
   f4v pr = ld16(wr + (l * V < a.KP ? l * V : 0));     // on their way early
   f4v pi = ld16(wi + (l * V < a.KP ? l * V : 0));
+  const int cn = b * a.bw + nc, place = pos % a.taps;
+  float* const S = a.S + slot * a.C + cn;
+  const float s0 = *S, xn = x[nc], yn = a.P[(size_t)r * a.ldp + a.oy + cn];
+  const float rb = a.rb[cn], ib = a.ib[cn], nl = a.nl[cn];
   for (int j = tid; j < a.KP; j += 256) {
     float u = 0.f;
     if (j < a.bw) {
       const int c = b * a.bw + j;
+      const float wx = a.cw[(a.taps - 1) * a.C + c], xj = x[j];
       u = a.cb[c];
-      for (int t = 1; t < a.taps; t++) {
-        const int p = pos - a.taps + t;
-        if (p >= 0)
-          u = fmaf(a.cw[(t - 1) * a.C + c], ring[(p % a.taps) * a.C + j], u);
+      // STEP_TAPS of them on the way at a time; those ahead of the first
+      // position are read, in some place of the ring, and left out
+      for (int t0 = 1; t0 < a.taps; t0 += STEP_TAPS) {
+        float w[STEP_TAPS], v[STEP_TAPS];
+#pragma unroll
+        for (int i = 0; i < STEP_TAPS; i++) {
+          const int t = min(t0 + i, a.taps - 1), at = place + t;
+          w[i] = a.cw[(t - 1) * a.C + c];
+          v[i] = ring[(at < a.taps ? at : at - a.taps) * a.C + j];
+        }
+#pragma unroll
+        for (int i = 0; i < STEP_TAPS; i++)
+          if (t0 + i < a.taps && pos - a.taps + t0 + i >= 0)
+            u = fmaf(w[i], v[i], u);
       }
-      u = fmaf(a.cw[(a.taps - 1) * a.C + c], x[j], u);
+      u = fmaf(wx, xj, u);
     }
     us[j] = u;
   }
@@ -151,13 +172,11 @@ __global__ void __launch_bounds__(256) k_rglru_step(RglruArgs a) {
   if (l == 0 && n < a.bw) {
     const int c = b * a.bw + n;
     float dec, add;
-    recur(a, c, sr, si, us[n], dec, add);
-    float* S = a.S + slot * a.C + c;
-    const float s = pos == 0 ? add : dec * *S + add;
+    recur(rb, ib, nl, sr, si, us[n], dec, add);
+    const float s = pos == 0 ? add : dec * s0 + add;
     *S = s;
-    ring[(pos % a.taps) * a.C + n] = x[n];
-    ((T*)a.out)[(size_t)r * a.ldo + c] =
-        El<T>::st(s * gelu_tanh_f(a.P[(size_t)r * a.ldp + a.oy + c]));
+    ring[place * a.C + n] = xn;
+    ((T*)a.out)[(size_t)r * a.ldo + c] = El<T>::st(s * gelu_tanh_f(yn));
   }
 }
 
@@ -267,9 +286,11 @@ __global__ void __launch_bounds__(256) k_rglru_local(RglruArgs a) {
     for (int r = 0; r < 4; r++) {
       const int t = wave * 16 + g * 4 + r, n = q * 16 + lr;
       float dec = 1.f, add = 0.f;
-      if (t < len && n0 + n < a.bw)
-        recur(a, b * a.bw + n0 + n, ar[q][r], ai[q][r], us[t * LS + n], dec,
-              add);
+      if (t < len && n0 + n < a.bw) {
+        const int c = b * a.bw + n0 + n;
+        recur(a.rb[c], a.ib[c], a.nl[c], ar[q][r], ai[q][r], us[t * LS + n],
+              dec, add);
+      }
       ds[t * LS + n] = dec;
       us[t * LS + n] = add;
     }
