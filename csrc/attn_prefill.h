@@ -15,7 +15,7 @@ struct ApArgs {
   const float* kS;       // [kvh, S]
   const float* vS;
   float* part;           // split keys: [split, kvh, rows, head_dim + 4]
-  int M, nh, kvh, ldq, S, fold;
+  int M, nh, kvh, ldq, S, fold, by_row;
   float scale, softcap;
   int window;
 };

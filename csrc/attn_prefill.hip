@@ -69,9 +69,9 @@ template <int HD> DEVINL int v_slot(int row, int slot) {
 }
 
 // A kv head's part of a range of keys, in the (HD + 4) floats a row that it has.
-// A wave's 32 rows or fewer: row by row.  More: four dims of all rows, the next
-// four, .., then maxima, then sums.  Where that
-// leaves room, rows are counted up to whole lines and parts begin with one.
+// Row by row, or (in lines) four dims of all rows, the next four, .., then
+// maxima, then sums.  Where that leaves room, rows are counted up to whole lines
+// and parts begin with one.
 struct ApPart { uint32_t rows; size_t size; };
 template <int HD> DEVINL ApPart ap_part(uint32_t rows) {
   const size_t size = (size_t)rows * (HD + 4);
@@ -459,7 +459,7 @@ k_attn_rows(ApArgs a) {
           w.b[j / 2][j % 2] = (__bf16)(o[d][q4 * 4 + j] * inv);
         *(unsigned long long*)(op + d * 32 + q4 * 8 + hh * 4) = w.u;
       }
-  } else if constexpr (NW == 1) {
+  } else if (NW == 1 || a.by_row) {
     // unnormalised part of this key range: HD values, maximum, sum
     float* pp = a.part + (((size_t)blockIdx.z * a.kvh + kvhead) * a.M * grp +
                           base * grp + row) * (HD + 4);
@@ -539,14 +539,12 @@ __global__ void __launch_bounds__(256) k_attn_rows_merge(ApArgs a, int split) {
   for (int i = 0; i < HD / 64; i++) op[i * 64 + lane] = f2b(v[i] / l);
 }
 
-// The same of more rows than a wave's, as they lie then: 16 rows of a kv head a
-// block, four where blocks are few, a thread takes ND times four dims of a row.
-// All maxima and sums and the first eight parts are on the way together.  (Two
-// rows of 8/4 heads of 256 over 3000 keys in 47 ranges take 1.1 us longer so, of
-// 64 dims 2.1, than by a wave a row.)
-template <int HD, int R>
+// The same of parts in lines: 16 rows of a kv head a block, a thread takes ND
+// times four dims of a row.  All maxima and sums and the first eight parts are
+// on the way together.
+template <int HD>
 __global__ void __launch_bounds__(256) k_attn_rows_merge_many(ApArgs a, int split) {
-  constexpr int ND = R == 16 ? HD / 64 : 1, NG = HD / 4 / ND;
+  constexpr int R = 16, ND = HD / 64, NG = 16;
   __shared__ float ms[AP_MAX_SPLIT][R], ls[AP_MAX_SPLIT][R];
   const int tid = threadIdx.x, r = tid % R, g = tid / R;
   const int grp = a.nh / a.kvh, kvhead = blockIdx.y, all = a.M * grp;
@@ -707,19 +705,35 @@ static bool ap_two(const ApArgs& a, int kv8, int keys, int most, int blocks,
   return two < one;
 }
 
-// most: rows of the longest sequence; ntiles: of several sequences
+// How a call runs: waves that share a tile of rows, such tiles, ranges of keys,
+// whether two groups of waves share a block's.  most: rows of the longest
+// sequence; ntiles: of several sequences.
+struct ApPlan { int nw, tiles, split; bool two, by_row; };
 template <int HD, int BKV>
-static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
-                         int most, int ntiles, hipStream_t s) {
+static ApPlan ap_plan(const ApArgs& a, int kv8, int keys, long part_floats,
+                      int most, int ntiles) {
   const int rows = a.M * (a.nh / a.kvh);
   // up to 32 rows are one wave's; more share their tiles among four
   const int nw = most * (a.nh / a.kvh) <= 32 ? 1 : 4;
-  const int tiles = a.tiles ? ntiles : (rows + nw * 32 - 1) / (nw * 32);
-  int split = ap_split<HD, BKV>(a, kv8, keys, part_floats, most, nw,
-                                tiles * a.kvh);
+  const int tiles = ntiles ? ntiles : (rows + nw * 32 - 1) / (nw * 32);
+  const int split = ap_split<HD, BKV>(a, kv8, keys, part_floats, most, nw,
+                                      tiles * a.kvh);
   const bool two = nw == 4 && ap_two<HD, BKV>(a, kv8, keys, most,
                                               tiles * a.kvh, split);
-  if (two) split = 1;
+  // Many parts of few rows lie row by row: a wave adds those of one row, where
+  // 16 rows a block would leave most CUs without any (us, so / in lines: 64 dims,
+  // 16 parts of 256 rows 13.6 / 16.1, 8 of 256 10.9 / 11.2, of 4096 -4%, 4 parts
+  // of 256 -1%, of 4096 -6%; 8000 calls)
+  return {nw, tiles, two ? 1 : split, two,
+          nw == 1 || (split >= 8 && (long)rows * a.kvh < 128 * split)};
+}
+
+template <int HD, int BKV>
+static hipError_t ap_run(ApArgs a, int kv8, const ApPlan& plan,
+                         hipStream_t s) {
+  const auto [nw, tiles, split, two, by_row] = plan;
+  const int rows = a.M * (a.nh / a.kvh);
+  a.by_row = by_row;
   // A block a CU, then the second of each (two groups of 128 dims have a CU to
   // themselves).  us, longest first -> so: 64 dims 1999 rows of 32/8 heads 32.4
   // -> 29.9, 2000 behind 2000 keys 72.3 -> 68.0; 128 dims 54.1 -> 52.3.
@@ -739,14 +753,11 @@ static hipError_t ap_run(ApArgs a, int kv8, int keys, long part_floats,
     if (kv8) ap_go<HD, BKV, 4, 1, true>(a, grid, s);
     else ap_go<HD, BKV, 4, 1, false>(a, grid, s);
   }
-  if (split > 1 && nw == 1)
+  if (split > 1 && by_row)
     hipLaunchKernelGGL((k_attn_rows_merge<HD>), dim3((rows * a.kvh + 3) / 4),
                        dim3(256), 0, s, a, split);
-  else if (split > 1 && (long)rows * a.kvh < 16 * 256)
-    hipLaunchKernelGGL((k_attn_rows_merge_many<HD, 4>),
-                       dim3((rows + 3) / 4, a.kvh), dim3(HD), 0, s, a, split);
   else if (split > 1)
-    hipLaunchKernelGGL((k_attn_rows_merge_many<HD, 16>),
+    hipLaunchKernelGGL((k_attn_rows_merge_many<HD>),
                        dim3((rows + 15) / 16, a.kvh), dim3(256), 0, s, a,
                        split);
   return hipGetLastError();
@@ -766,16 +777,49 @@ extern "C" hipError_t launch_attn_prefill_mfma(
   if (M < 1 || kvh < 1 || nh % kvh || ldq < nh * hd || ldq % 8 ||
       (tiles && (ntiles < 1 || most < 1)))
     return hipErrorInvalidValue;
-  if (!tiles) most = M;
+  if (!tiles) {
+    most = M;
+    ntiles = 0;
+  }
   ApArgs a = {(const u16*)q, kc, vc, (u16*)out, (const int*)len_ptr,
               (const int*)tiles,
               (const float*)kS, (const float*)vS, (float*)part, M, nh, kvh,
-              ldq, S, 0, scale, softcap, window};
+              ldq, S, 0, 0, scale, softcap, window};
   if (hd == 64)
-    return ap_run<64, 64>(a, kv8, keys, part_floats, most, ntiles, stream);
+    return ap_run<64, 64>(
+        a, kv8, ap_plan<64, 64>(a, kv8, keys, part_floats, most, ntiles),
+        stream);
   if (hd == 128)
-    return ap_run<128, 64>(a, kv8, keys, part_floats, most, ntiles, stream);
+    return ap_run<128, 64>(
+        a, kv8, ap_plan<128, 64>(a, kv8, keys, part_floats, most, ntiles),
+        stream);
   if (hd == 256)
-    return ap_run<256, 32>(a, kv8, keys, part_floats, most, ntiles, stream);
+    return ap_run<256, 32>(
+        a, kv8, ap_plan<256, 32>(a, kv8, keys, part_floats, most, ntiles),
+        stream);
   return hipErrorInvalidValue;
+}
+
+// How such a call runs, on the host alone: ranges of keys, whether two groups of
+// waves share a block's, whether parts lie row by row.  1: a head dim that is
+// none of the kernels'.
+extern "C" int attn_prefill_plan(int kv8, int M, int nh, int kvh, int hd,
+                                 int keys, int most, int ntiles, int window,
+                                 long part_floats, int* out) {
+  ApArgs a = {};
+  a.M = M;
+  a.nh = nh;
+  a.kvh = kvh;
+  a.window = window;
+  a.part = part_floats > 0 ? (float*)out : nullptr;      // is there or not
+  if (!ntiles) most = M;
+  if (hd != 64 && hd != 128 && hd != 256) return 1;
+  const ApPlan p =
+      hd == 64 ? ap_plan<64, 64>(a, kv8, keys, part_floats, most, ntiles)
+      : hd == 128 ? ap_plan<128, 64>(a, kv8, keys, part_floats, most, ntiles)
+                  : ap_plan<256, 32>(a, kv8, keys, part_floats, most, ntiles);
+  out[0] = p.split;
+  out[1] = p.two;
+  out[2] = p.by_row;
+  return 0;
 }

@@ -65,6 +65,8 @@ _SIGS = {
                        [ctypes.c_float, ctypes.c_float, ctypes.c_void_p],
     "launch_mid_gemm": [ctypes.c_void_p] * 9 + [ctypes.c_long] +
                        [ctypes.c_int] * 9 + [ctypes.c_float, ctypes.c_void_p],
+    "attn_prefill_plan": [ctypes.c_int] * 9 + [ctypes.c_long,
+                                               ctypes.c_void_p],
     "row_gemm_plan": [ctypes.c_int] * 6 + [ctypes.c_long, ctypes.c_int,
                                            ctypes.c_void_p],
     "launch_prefetch": [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p,
@@ -312,6 +314,20 @@ def attn_prefill_mfma(q: torch.Tensor, k_cache: torch.Tensor,
         M, nh, kvh, hd, _ld(q, nh * hd), S, max(keys, M if not most else 1),
         most, 0 if tiles is None else tiles.shape[0], ctypes.c_float(scale),
         ctypes.c_float(softcap), window, _stream()), "attn_prefill_mfma")
+
+
+def attn_prefill_plan(M: int, nh: int, kvh: int, hd: int, keys: int,
+                      window: int = 0, kv8: bool = False, part: int = 1 << 62,
+                      most: int = 0, ntiles: int = 0) -> dict:
+    """How attn_prefill_mfma goes about a call with so many floats of part:
+    ranges of keys, whether two groups of waves share a block's (two), whether
+    parts of the ranges lie row by row (by_row).  Host arithmetic only."""
+    out = (ctypes.c_int * 3)()
+    _check(lib().attn_prefill_plan(
+        int(kv8), M, nh, kvh, hd, max(keys, M if not most else 1), most,
+        ntiles, window, ctypes.c_long(part),
+        ctypes.cast(out, ctypes.c_void_p)), "attn_prefill_plan")
+    return dict(ranges=out[0], two=bool(out[1]), by_row=bool(out[2]))
 
 
 def attn_tiles(segs, group: int) -> np.ndarray:

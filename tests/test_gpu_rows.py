@@ -86,6 +86,27 @@ def test_prompt_attention_of_many_blocks(hd, nh, kvh, M, pos0, window, cap,
     test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8)
 
 
+# parts of the keys in lines, 16 rows a block of their sum: rows that end inside
+# one and with one, fewer parts than are on the way together (eight), as many, one
+# more; and row by row, also as few rows as that goes by
+@pytest.mark.parametrize("hd,nh,kvh,M,pos0,window,cap,ranges,by_row", [
+    (64, 4, 2, 67, 220, 0, 0.0, 5, False), (64, 8, 2, 300, 2000, 0, 0.0, 9, False),
+    (64, 4, 4, 400, 900, 0, 30.0, 7, False), (128, 3, 1, 43, 190, 0, 0.0, 4, False),
+    (128, 8, 1, 144, 300, 0, 0.0, 7, False), (128, 6, 2, 400, 900, 700, 0.0, 6, False),
+    (256, 2, 2, 130, 30, 0, 50.0, 5, False), (256, 4, 1, 330, 200, 0, 0.0, 9, False),
+    (256, 8, 1, 200, 500, 0, 0.0, 8, False), (64, 9, 3, 21, 1800, 0, 0.0, 28, True),
+    (128, 4, 2, 210, 800, 0, 0.0, 8, True), (256, 4, 1, 270, 700, 0, 0.0, 11, True)])
+@pytest.mark.parametrize("kv8", [False, True])
+def test_prompt_attention_in_parts(hd, nh, kvh, M, pos0, window, cap, ranges,
+                                   by_row, kv8):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    p = ho.attn_prefill_plan(M, nh, kvh, hd, pos0 + M, window, kv8, 1 << 22)
+    if not kv8:
+        assert p == dict(ranges=ranges, two=False, by_row=by_row)
+    test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8)
+
+
 # a part of the keys whose weight beside the others' underflows, with values
 # that are no number: as in one softmax, 0 times them is none either
 @pytest.mark.parametrize("hd", [64, 128, 256])
