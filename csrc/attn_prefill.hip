@@ -669,40 +669,53 @@ static int ap_split(const ApArgs& a, int kv8, int keys, long part_floats,
   return split;
 }
 
-// Whether two groups of waves share a block's keys, rather than `split` ranges.
-// More blocks than CUs: of 64 dims (two such blocks fit a CU) always; of 128 (one
-// does) where blocks differ in length enough that the short ones fill what the
-// long ones leave: few keys ahead of the rows (32/8 heads of 128, 1999 rows
-// 54.1 -> 49.6, behind 2000 keys 114 -> 118, 1365 behind 4000 137 -> 156).  Up
-// to a block a CU, by numbers (us; tiles of the longest block, tiles of a CU,
-// parts of rows in MB) fitted to 255 calls of 11 head layouts, 40 to 2048 rows
-// behind 0 to 6000 keys: 1.25 (64 dims), 1.16 and, e4m3, 1.12 times as fast as
-// ranges alone, none slower (but 80 blocks of 64 dims, five tiles, 9.1 -> 9.5:
-// not below eight).
-// More blocks than 512 and 64 dims of e4m3 (which spill) were not measured.
+// Whether two groups of waves share a block's keys, rather than `split` ranges
+// or one group alone.  By the tiles that the longest block goes through (under a
+// window those of a block's rows and of the window) and by how many a CU gets,
+// fitted to 26700 calls timed both ways: 26 head layouts, 65 to 512 blocks, 40
+// to 2048 rows behind 0 to 8000 keys, windows, and two to eight sequences, a
+// part of them behind keys of their own.  Above the better way 0.9% on average
+// (never two groups 10.7%); 176 calls take 4% longer than by ranges whose parts
+// were left row by row, the others up to 2.6 times less.
+//   More blocks than CUs: of 64 dims (two such blocks fit a CU) from eight tiles
+// on (72/8 heads, one tile a block, 6.1 us by one group, 7.6); of 128 (one does)
+// where blocks differ in length enough that the short ones fill what the long
+// ones leave: few keys ahead of the rows (32/8 heads, 1999 rows 54.1 -> 49.6,
+// behind 2000 keys 114 -> 118), and of several sequences, which may be short but
+// for one, where the longest is long (8 of up to 50 rows, 40/40 heads, 7.6 by one
+// group, 12.8 by two).
+//   Up to a block a CU by numbers for what two groups take more: of one sequence
+// and of several; each of 64 dims, 128, 128 beside e4m3.
+// 64 dims of e4m3 (which spill) and more than 512 blocks were not measured.
 template <int HD, int BKV>
 static bool ap_two(const ApArgs& a, int kv8, int keys, int most, int blocks,
-                   int split) {
+                   int split, bool several) {
   if (HD == 256 || (HD == 64 && kv8) || blocks <= 64 || blocks > 512)
     return false;
-  const bool bound = a.window > 0 && a.window < keys;
-  if (blocks > 256) return HD == 64 || (2 * (keys - most) < most && !bound);
-  const int span = bound && a.window + most < keys ? a.window + most : keys;
+  const int grp = a.nh / a.kvh, own = (128 + grp - 1) / grp;
+  const int span = a.window > 0 && a.window + own < keys ? a.window + own
+                                                         : keys;
   const int tiles = (span + BKV - 1) / BKV, per = (tiles + split - 1) / split;
-  if (HD == 64 && tiles < 8) return false;
-  const float mean = bound && a.window < keys - most / 2 ? a.window
-                                                         : keys - most / 2;
+  const float mean = fminf(keys - 0.5f * most, span);
   const float all = blocks * mean / BKV / 256;
-  const float mb = (float)a.kvh * a.M * (a.nh / a.kvh) * (HD + 4) * 4e-6f;
-  static const float fit[3][8] = {
-      {4.49f, 0.6f, 0.244f, 7.f, 0.799f, 0.517f, 2.62f, 0.358f},
-      {5.99f, 0.95f, 0.439f, 9.f, 1.32f, 0.731f, 2.03f, 0.254f},
-      {8.9f, 0.95f, 0.254f, 9.74f, 0.963f, 0.827f, 2.03f, 0.241f}};
-  const float* f = fit[HD == 64 ? 0 : kv8 ? 2 : 1];
-  const float two = f[0] + f[1] * tiles + f[2] * all;
-  const float one = f[3] + f[4] * per + f[5] * all +
-                    (split > 1 ? f[6] + f[7] * split * mb : 0.f);
-  return two < one;
+  if (blocks > 256) {
+    if (HD == 64) return tiles >= 8;
+    if (several) return tiles >= (kv8 ? 8 : 11);
+    if (kv8) return tiles - 0.8f * all > 1.6f;
+    return tiles - all > 4.f && 2 * (keys - most) < most;
+  }
+  // parts of the rows, MB
+  const float mb = split > 1 ? (float)a.M * a.nh * (HD + 4) * 4e-6f : 0.f;
+  static const float fit[6][5] = {
+      {0.646f, -0.329f, -0.907f, -0.518f, -0.39f},
+      {0.563f, -0.0799f, -0.821f, -1.42f, -0.162f},
+      {1.49f, -0.152f, -2.22f, -1.71f, -0.372f},
+      {0.212f, 0.0593f, -0.421f, -0.567f, -0.158f},
+      {0.186f, -0.0126f, -0.233f, -1.14f, -0.0603f},
+      {0.397f, 0.121f, -0.842f, 0.397f, -0.133f}};
+  const float* f = fit[several * 3 + (HD == 64 ? 0 : kv8 ? 2 : 1)];
+  return 1.f + f[0] * tiles + f[1] * all + f[2] * per + f[3] * (split > 1) +
+             f[4] * split * mb < 0.f;
 }
 
 // How a call runs: waves that share a tile of rows, such tiles, ranges of keys,
@@ -719,7 +732,7 @@ static ApPlan ap_plan(const ApArgs& a, int kv8, int keys, long part_floats,
   const int split = ap_split<HD, BKV>(a, kv8, keys, part_floats, most, nw,
                                       tiles * a.kvh);
   const bool two = nw == 4 && ap_two<HD, BKV>(a, kv8, keys, most,
-                                              tiles * a.kvh, split);
+                                              tiles * a.kvh, split, ntiles);
   // Many parts of few rows lie row by row: a wave adds those of one row, where
   // 16 rows a block would leave most CUs without any (us, so / in lines: 64 dims,
   // 16 parts of 256 rows 13.6 / 16.1, 8 of 256 10.9 / 11.2, of 4096 -4%, 4 parts

@@ -44,3 +44,40 @@ def test_one_wave_of_rows_lies_row_by_row():
     p = plan(64, 32, 8, [(300, 5)])
     assert p["ranges"] > 1 and p["by_row"]
     assert plan(64, 32, 8, [(300, 5)], part=0)["ranges"] == 1
+
+
+# Two groups of waves a block wait for each other and meet at the end: not worth
+# it for a few tiles, which several short sequences have, however many blocks
+# they are, nor where the longest block is hardly longer than the others.
+@pytest.mark.parametrize("hd,nh,kvh,segs,window,kv8", [
+    (64, 128, 8, [(0, 300)], 0, False),                 # five tiles
+    (64, 64, 64, [(0, 600)], 100, False),               # three in a window
+    (64, 40, 8, [(0, 50)] * 7 + [(1500, 30)], 0, False),
+    (64, 16, 4, [(0, 199), (2849, 484), (0, 572)], 0, False),
+    (128, 40, 40, [(0, 50)] * 8, 0, False),
+    (128, 40, 40, [(0, 50)] * 8, 152, True),
+    (128, 28, 4, [(0, 333)] * 6, 0, False),
+    (128, 64, 8, [(0, 376)], 40, False),
+    (128, 8, 1, [(0, 1066)], 0, False),
+    (128, 32, 8, [(2000, 1999)], 0, False)])
+def test_one_group_of_waves(hd, nh, kvh, segs, window, kv8):
+    assert not plan(hd, nh, kvh, segs, window, kv8)["two"]
+
+
+# and where a chain half as long is
+@pytest.mark.parametrize("hd,nh,kvh,segs,window,kv8", [
+    (64, 32, 8, [(0, 611)], 0, False), (64, 32, 8, [(0, 1999)], 0, False),
+    (64, 32, 8, [(1300, 700)], 0, False), (64, 32, 8, [(300, 500)], 200, False),
+    (64, 32, 8, [(0, 400), (60, 480), (0, 20)], 0, False),
+    (128, 32, 8, [(0, 1000)], 0, False), (128, 24, 8, [(0, 1999)], 0, False),
+    (128, 24, 8, [(0, 1999)], 0, True), (128, 32, 8, [(100, 480)], 130, False),
+    (128, 64, 8, [(0, 750), (0, 101)], 0, False),
+    (128, 32, 8, [(0, 400), (60, 480), (0, 20)], 0, True)])
+def test_two_groups_of_waves(hd, nh, kvh, segs, window, kv8):
+    assert plan(hd, nh, kvh, segs, window, kv8)["two"]
+
+
+def test_two_groups_of_waves_have_two_halves_at_most():
+    assert not plan(256, 16, 8, [(0, 1999)])["two"]
+    assert not plan(64, 32, 8, [(0, 1999)], kv8=True)["two"]
+    assert not plan(64, 32, 8, [(0, 2048)] * 2)["two"]    # 1024 blocks

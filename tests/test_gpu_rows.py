@@ -68,9 +68,10 @@ def test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8):
 
 
 # blocks of which two groups of waves take the keys in turn: up to a block a CU
-# and more, one tile of keys (the second group has none), an odd number, keys
-# ahead of the rows, windows, a cap; rows that end inside a wave; and as many
-# blocks in ranges, of 256 dims and of e4m3 keys of 64
+# and more, first rows with one tile of keys (the second group has none), an odd
+# number, keys ahead of the rows, windows, a cap; rows that end inside a wave.
+# And as many blocks whose way is another: one tile in all, ranges, 256 dims,
+# e4m3 keys of 64
 @pytest.mark.parametrize("hd,nh,kvh,M,pos0,window,cap,kv8", [
     (64, 80, 80, 50, 0, 0, 0.0, False), (64, 32, 8, 333, 0, 0, 0.0, False),
     (64, 32, 8, 611, 70, 0, 30.0, False), (64, 40, 8, 1037, 0, 0, 0.0, False),
@@ -84,6 +85,57 @@ def test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8):
 def test_prompt_attention_of_many_blocks(hd, nh, kvh, M, pos0, window, cap,
                                          kv8):
     test_prompt_attention(hd, nh, kvh, M, pos0, window, cap, kv8)
+
+
+# the same of several sequences, of ragged lengths, one of them behind keys of its
+# own: up to a block a CU and more, sequences that leave the second group without
+# a tile, windows, a cap, pools out of order
+@pytest.mark.parametrize("hd,nh,kvh,segs,window,cap,kv8", [
+    (64, 32, 8, [(2, 0, 333), (0, 70, 301), (1, 0, 65)], 0, 0.0, False),
+    (64, 32, 8, [(2, 0, 533), (0, 70, 301), (1, 0, 5)], 470, 30.0, False),
+    (64, 40, 8, [(2, 0, 640), (0, 0, 410), (1, 100, 33)], 520, 0.0, False),
+    (64, 72, 8, [(0, 0, 300), (2, 300, 250), (1, 0, 2)], 0, 50.0, False),
+    (128, 16, 4, [(0, 0, 600), (1, 30, 60), (2, 0, 3)], 0, 0.0, False),
+    (128, 12, 2, [(1, 0, 900), (0, 300, 60), (2, 0, 40)], 0, 50.0, False),
+    (128, 64, 8, [(1, 0, 650), (0, 600, 101), (2, 0, 17)], 0, 0.0, False),
+    (128, 64, 8, [(1, 0, 750), (0, 0, 101), (2, 0, 17)], 700, 0.0, False),
+    (128, 32, 8, [(2, 0, 333), (0, 70, 301), (1, 0, 65)], 200, 0.0, True),
+    (128, 64, 8, [(1, 0, 450), (0, 600, 101), (2, 0, 17)], 0, 30.0, True)])
+def test_prompts_of_one_batch_by_two_groups_of_waves(hd, nh, kvh, segs, window,
+                                                     cap, kv8):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    M, keys = sum(n for _, _, n in segs), max(p + n for _, p, n in segs)
+    most, S = max(n for _, _, n in segs), keys + 3
+    tiles = torch.from_numpy(ho.attn_tiles(segs, nh // kvh)).cuda()
+    assert ho.attn_prefill_plan(M, nh, kvh, hd, keys, window, kv8, 1 << 22,
+                                most, len(tiles))["two"]
+    q = normal(M, nh, hd, seed=1, scale=2.0)
+    K, V = (normal(3, kvh, S, hd, seed=s) for s in (2, 3))
+    kS = vS = None
+    Kd, Vd = K.double(), V.double()
+    if kv8:
+        (K, kS, Kd), (V, vS, Vd) = e4m3(K), e4m3(V)
+    out = torch.full((M + 1, nh * hd), 7.0, device="cuda").bfloat16()
+    ho.attn_prefill_mfma(
+        q, K, V, out, None, M, nh, kvh, hd, hd ** -0.5, softcap=cap,
+        window=window, kS=kS, vS=vS, part=torch.zeros(1 << 22, device="cuda"),
+        keys=keys, tiles=tiles, most=most)
+    ref, at = torch.empty(M, nh, hd, dtype=torch.float64, device="cuda"), 0
+    for b, p, n in segs:
+        i = p + torch.arange(n, device="cuda")[:, None]
+        j = torch.arange(p + n, device="cuda")
+        bad = (j > i) | ((j <= i - window) if window else False)
+        for h in range(nh):
+            g = h * kvh // nh
+            s = q[at:at + n, h].double() @ Kd[b, g, :p + n].T * hd ** -0.5
+            s = cap * torch.tanh(s / cap) if cap else s
+            w = torch.softmax(s.masked_fill(bad, -math.inf), -1)
+            ref[at:at + n, h] = w @ Vd[b, g, :p + n]
+        # bf16 probabilities and results: 2^-9 at most each
+        assert off(out[at:at + n], ref[at:at + n].view(n, -1)) < 2.0 ** -8
+        at += n
+    assert (out[M] == 7.0).all()
 
 
 # parts of the keys in lines, 16 rows a block of their sum: rows that end inside
