@@ -672,17 +672,17 @@ static int ap_split(const ApArgs& a, int kv8, int keys, long part_floats,
 // Whether two groups of waves share a block's keys, rather than `split` ranges
 // or one group alone.  By the tiles that the longest block goes through (under a
 // window those of a block's rows and of the window) and by how many a CU gets,
-// fitted to 26700 calls timed both ways: 26 head layouts, 65 to 512 blocks, 40
+// fitted to 26700 calls timed both ways: 17 head layouts, 65 to 512 blocks, 40
 // to 2048 rows behind 0 to 8000 keys, windows, and two to eight sequences, a
 // part of them behind keys of their own.  Above the better way 0.9% on average
 // (never two groups 10.7%); 176 calls take 4% longer than by ranges whose parts
-// were left row by row, the others up to 2.6 times less.
+// were left row by row, the others up to 3.4 times less.
 //   More blocks than CUs: of 64 dims (two such blocks fit a CU) from eight tiles
-// on (72/8 heads, one tile a block, 6.1 us by one group, 7.6); of 128 (one does)
+// on (8 prompts of up to 40 rows, 64/64 heads, 6.2 us by one group, 7.6); of 128 (one does)
 // where blocks differ in length enough that the short ones fill what the long
 // ones leave: few keys ahead of the rows (32/8 heads, 1999 rows 54.1 -> 49.6,
 // behind 2000 keys 114 -> 118), and of several sequences, which may be short but
-// for one, where the longest is long (8 of up to 50 rows, 40/40 heads, 7.6 by one
+// for one, where the longest is long (8 of up to 40 rows, 40/40 heads, 7.6 by one
 // group, 12.8 by two).
 //   Up to a block a CU by numbers for what two groups take more: of one sequence
 // and of several; each of 64 dims, 128, 128 beside e4m3.
