@@ -731,10 +731,15 @@ class GPUModel(DecodeLoop):
     def _ranges(self, M: int) -> int:
         """Ranges of the history that a step of M rows may take: the more
         rows, the fewer fill the chip.  us, 8000 keys of 8 heads of 128, by
-        1, 2, 4, 8, 16 ranges: one row 76 44 27 18 15, four 81 49 31 28 35,
-        16 117 101 111 137 184; 16 rows of 620 keys, 8 heads of 256: 2 ranges
-        25, 3 35."""
-        return min(self.attn_split, max(1, 256 // (M * self.kvh_l)))
+        1, 2, 4, 8, 16 ranges: one row 80 47 28 19 15, four 103 61 37 32 31,
+        16 127 99 102 102 103; 16 rows of 620 keys, 8 heads of 256: one range
+        25, two 23, three 30.  A block of 256 dims is all that a CU holds, so
+        there each four query heads of a kv head count: 16 rows of 109 and 2031
+        keys, 8/1 heads, by 8 ranges 9.8 and 22, by 16 17 and 30."""
+        blocks = M * self.kvh_l
+        if self.hd == 256:
+            blocks *= -(-self.nh_l // (4 * self.kvh_l))
+        return min(self.attn_split, max(1, 256 // blocks))
 
     def _layers_forward(self, M: int, layer_hook=None,
                         batch_attn: bool = False, keys: int = 0, pack=None):

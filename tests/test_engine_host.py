@@ -134,3 +134,15 @@ def test_tokens_are_fetched_in_the_chunks_asked_for(kw, sizes):
     m = Loop()
     assert len(m.generate_tokens([1, 2], 300, **kw)) == sum(sizes)
     assert m.sizes == sizes
+
+
+# a block of 256 dims has a CU to itself, one for every four query heads of a kv
+# head; of other dims two share one and heads are not counted
+@pytest.mark.parametrize("hd,nh,kvh,rows,most,ranges", [
+    (256, 8, 1, 16, 16, 8), (256, 8, 1, 32, 8, 4), (256, 8, 1, 64, 64, 2),
+    (256, 8, 1, 200, 64, 1), (256, 4, 1, 16, 64, 16), (256, 16, 8, 16, 64, 2),
+    (256, 20, 4, 8, 64, 4), (256, 8, 4, 1, 20, 20), (128, 8, 1, 16, 64, 16),
+    (64, 32, 4, 16, 64, 4)])
+def test_ranges_of_a_step(hd, nh, kvh, rows, most, ranges):
+    m = types.SimpleNamespace(hd=hd, nh_l=nh, kvh_l=kvh, attn_split=most)
+    assert eng.GPUModel._ranges(m, rows) == ranges
