@@ -217,8 +217,10 @@ DEVINL void put_value(f4v* v, int k0, int g, int key, T val) {
 // keys, 8 of 32/8 of 64 at 2000 15.1 -> 11.8, one of 32/8 of 128 at 30000 31.5
 // -> 27.1; in fp32 12.9 -> 12.3.
 #define TOKEN_U 8            // query elements that a thread asks for at once
+// (fp32 of 64 dims: else one register more than lets three blocks on a CU)
 template <typename T, int DP, int VP>
-__global__ void __launch_bounds__(256) k_gqa_token(GqaArgs a) {
+__global__ void __launch_bounds__(256, sizeof(T) == 4 && DP + VP == 128 ? 3 : 1)
+k_gqa_token(GqaArgs a) {
   constexpr int SZ = sizeof(T), NC = DP * SZ / 64, ND = VP / 16, VV = SZ / 2;
   constexpr int XS = 32 * VP > 4 * DP * SZ ? 32 * VP : 4 * DP * SZ;
   __shared__ __attribute__((aligned(16))) float xs[XS];
@@ -303,7 +305,10 @@ __global__ void __launch_bounds__(256) k_gqa_token(GqaArgs a) {
     }
   };
   const int first = (g0 + split) * 128 + wave * 32;
-  if (first < kend && first + 32 > k_lo) fetch(first);
+  // not fp32 of 256 dims, whose keys and values fill the registers: early ones
+  // were spilled (16 rows of 16/4 heads, 3000 keys 92 us, so 100)
+  constexpr bool EARLY = DP * SZ + VP * SZ < 2048;
+  if (EARLY && first < kend && first + 32 > k_lo) fetch(first);
 
   float sq = 0.f;
 #pragma unroll
@@ -361,7 +366,7 @@ __global__ void __launch_bounds__(256) k_gqa_token(GqaArgs a) {
     const int k0 = grp * 128 + wave * 32;
     if (k0 >= kend) break;
     if (k0 + 32 <= k_lo) continue;
-    if (k0 != first) fetch(k0);
+    if (!EARLY || k0 != first) fetch(k0);
     if (fresh && k0 + 32 > pos) {        // the new token's, not there when asked
 #pragma unroll
       for (int i = 0; i < 2; i++)
