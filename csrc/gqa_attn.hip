@@ -312,10 +312,10 @@ k_gqa_token(GqaArgs a) {
 
   float sq = 0.f;
 #pragma unroll
-  for (int u = 0; u < TOKEN_U; u++) sq += pv[u] * pv[u];
+  for (int u = 0; u < TOKEN_U; u++) sq = fmaf(pv[u], pv[u], sq);
 #pragma unroll 4
   for (int i = tid + TOKEN_U * 256; i < nqd; i += 256)
-    sq += p[a.oq + i] * p[a.oq + i];
+    sq = fmaf(p[a.oq + i], p[a.oq + i], sq);
   sq = wave_reduce_sum(sq);
   if (fresh) sk = wave_reduce_sum(sk);
   if (lane == 0) {
