@@ -511,18 +511,23 @@ k_gemm_prompt(GpArgs a) {
 // the empty ones left in place some had a tile more than others (1100 rows, 8
 // experts, 2048->2x4096: 130 us, so 107).
 #define GW_RING 9
-// 64 lanes of 16 bytes to lds and behind it
+// 64 lanes of 16 bytes to lds and behind it.  By asm: ahead of a builtin's load
+// the compiler would wait for those in flight.  m0 is named, so that one that it
+// sets for a builtin is set again behind this; it warns that it keeps m0 itself.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <bool NT = false>
 DEVINL void gw_load(const char* base, uint32_t off, uint32_t lds) {
   if constexpr (NT)
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
                  "global_load_lds_dwordx4 %1, %0 nt"
-                 :: "s"(base), "v"(off), "s"(lds) : "memory");
+                 :: "s"(base), "v"(off), "s"(lds) : "memory", "m0");
   else
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\t"
                  "global_load_lds_dwordx4 %1, %0"
-                 :: "s"(base), "v"(off), "s"(lds) : "memory");
+                 :: "s"(base), "v"(off), "s"(lds) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 DEVINL void gw_meet() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();

@@ -74,6 +74,21 @@ def test_every_header_is_known_to_the_build():
     assert {s for src in LIBS.values() for s in src} <= set(there)
 
 
+def test_asm_that_sets_m0_says_so():
+    """LDS loads of builtins go by m0 too, and the compiler keeps it."""
+    from csrc.build import CSRC
+
+    found = 0
+    for f in os.listdir(CSRC):
+        if f.endswith((".h", ".hip")):
+            text = open(os.path.join(CSRC, f)).read()
+            for asm in re.findall(r"\basm\b[^(]*\((.*?)\);", text, re.S):
+                if re.search(r"\bs_mov_b32 m0\b", asm):
+                    found += 1
+                    assert '"m0"' in asm, f
+    assert found
+
+
 # one piece of any shape: rows follow one another; parts of a fused row: they
 # are as far apart as it is long (a single row may say anything)
 def test_distance_of_rows():
