@@ -827,16 +827,20 @@ static hipError_t gp_go(GpArgs a, int sk, hipStream_t s) {
   return hipGetLastError();
 }
 
+// of parts of K as many as have slabs
+template <int T> static int gw_parts(int K, int sk) {
+  const int slabs = (int)((long)K * (T == GP_E4M3 ? 1 : 2) / 128);
+  const int per = (slabs + sk - 1) / sk;
+  return (slabs + per - 1) / per;
+}
+
 // by k_gemm_wide; e4m3 rows of whole slabs
 template <int T, int HA>
 static hipError_t gp_go_wide(GpArgs a, int sk, hipStream_t s) {
   constexpr bool F8 = T == GP_E4M3;
   const bool glu = a.act >= 0;
   gp_tiling(a, 128 * HA, glu ? 128 : 256);
-  // as many parts as have slabs
-  const int slabs = (int)((long)a.K * (F8 ? 1 : 2) / 128);
-  const int per = (slabs + sk - 1) / sk;
-  sk = (slabs + per - 1) / per;
+  sk = gw_parts<T>(a.K, sk);
   const int share = (a.tm * a.tn + 7) / 8 * sk;          // of an XCD
   const dim3 grid(8 * (share < 32 ? share : 32));        // a block a CU
 #define GW_GO(GLU, NT)                                                       \
@@ -869,8 +873,9 @@ static const GpTile gp_tiles[8] = {
 
 // What a slab of each tile costs a CU with one block and with as many as fit,
 // a round besides (first slabs, epilogue); the second block on some CUs, the
-// first on few; K in parts, and each of their floats.  0: not for that type
-// (e4m3 in 128x128 by four waves: no product of the fits chose it).
+// first on few; K in parts, and each of their floats; a round where outputs are
+// no multiple of four and leave one by one.  0: not for that type (e4m3 in
+// 128x128 by four waves: no product of the fits chose it).
 // The numbers are about us, but fitted to what they choose: the times of every
 // likely tile and split (1 to 8 parts), W from memory, for 17 to 2000 rows of
 // 126 shapes and for 14 numbers of rows each of 30 shapes of models, so that
@@ -894,35 +899,49 @@ static const GpTile gp_tiles[8] = {
 // 8192x2048 21.4 to 24.4 -> 12.8 to 21.4; over all 4% in bf16, 5% in e4m3):
 // bf16 2.0% -> 1.3%, with a gate 1.2% -> 0.8%, e4m3 as it was 1.5%, with a gate
 // 1.1% -> 0.5%.
+// e4m3 rows with half a slab at their end, which k_gemm_wide does not take, have
+// numbers of their own, fitted to half of 8474 products: above the best of the
+// others' 3.2% -> 1.7%, 4% longer than before k_gemm_wide 57 -> 30 of 1647; with a
+// gate 2.0% -> 0.9%, 61 -> 14 of 1067 (1792x4786x704 63.5 us, so 41.9).
 struct GpCost {
-  float one[8], full[8], round[8], second, first, split, part;
+  float one[8], full[8], round[8], second, first, split, part, off;
 };
-static const GpCost gp_cost[5] = {
+static const GpCost gp_cost[7] = {
     {// bf16
      {1.29f, 0.665f, 0.62f, 0.51f, 1.24f, 0.443f, 0.261f, 0.257f},
      {1.29f, 0.665f, 1.09f, 0.51f, 1.37f, 1.07f, 0.501f, 0.438f},
      {7.85f, 3.82f, 2.87f, 4.5f, 2.1f, 1.21f, 1.54f, 1.24f},
-     0.7f, 1.f, 2.22f, 4.94e-6f},
+     0.7f, 1.f, 2.22f, 4.94e-6f, 1.f},
     {// bf16 with a gate
      {1.46f, 0.87f, 0.592f, 0.518f, 0.854f, 0.481f, 0.261f, 0.234f},
      {1.46f, 0.87f, 1.22f, 0.518f, 0.854f, 0.822f, 0.576f, 0.312f},
      {4.86f, 3.2f, 2.36f, 3.37f, 2.56f, 2.98f, 1.09f, 1.56f},
-     0.616f, 0.96f, 1.77f, 4.79e-6f},
+     0.616f, 0.96f, 1.77f, 4.79e-6f, 1.f},
     {// e4m3
      {1.76f, 0.954f, 0.f, 0.752f, 0.633f, 0.892f, 0.405f, 0.286f},
      {1.76f, 0.954f, 0.f, 0.752f, 0.817f, 0.892f, 0.556f, 0.449f},
      {6.f, 3.81f, 0.f, 2.16f, 2.07f, 2.84f, 1.14f, 1.21f},
-     0.626f, 0.952f, 0.273f, 5.43e-6f},
+     0.626f, 0.952f, 0.273f, 5.43e-6f, 1.f},
     {// e4m3 with a gate
      {1.87f, 1.17f, 0.f, 0.745f, 0.651f, 0.78f, 0.45f, 0.286f},
      {1.87f, 1.17f, 0.f, 0.745f, 0.878f, 0.78f, 0.45f, 0.474f},
      {6.f, 3.98f, 0.f, 2.18f, 1.8f, 1.28f, 1.68f, 1.85f},
-     0.632f, 1.f, 0.778f, 4.63e-6f},
+     0.632f, 1.f, 0.778f, 4.63e-6f, 1.f},
+    {// e4m3, half a slab at the end of a row
+     {0.f, 1.84f, 0.f, 1.03f, 0.903f, 0.842f, 0.589f, 0.374f},
+     {0.f, 1.84f, 0.f, 1.03f, 1.29f, 1.22f, 0.836f, 0.618f},
+     {0.f, 3.41f, 0.f, 6.f, 2.52f, 1.29f, 0.647f, 0.626f},
+     0.824f, 0.852f, 1.27f, 4.33e-6f, 1.98f},
+    {// the same with a gate
+     {0.f, 1.18f, 0.f, 0.739f, 0.648f, 0.555f, 0.38f, 0.217f},
+     {0.f, 1.18f, 0.f, 0.739f, 0.891f, 0.8f, 0.511f, 0.387f},
+     {0.f, 3.87f, 0.f, 2.18f, 1.64f, 1.16f, 1.11f, 1.34f},
+     0.99f, 0.856f, 0.944f, 2.79e-6f, 1.f},
     {// MXFP4
      {0.f, 0.96f, 0.654f, 0.562f, 0.44f, 0.f, 0.292f, 0.f},
      {0.f, 0.96f, 1.08f, 0.562f, 0.773f, 0.f, 0.538f, 0.f},
      {0.f, 4.f, 3.2f, 3.4f, 1.8f, 0.f, 1.4f, 0.f},
-     0.42f, 0.96f, 2.1f, 5e-6f}};
+     0.42f, 0.96f, 2.1f, 5e-6f, 1.f}};
 
 // the tile and split of a product, and what it takes by the numbers
 struct GpPick { int tile, sk; float time; };
@@ -931,16 +950,16 @@ template <int T>
 static GpPick gp_pick(const GpArgs& a, long part_floats, int ncnt) {
   const int width = a.act >= 0 ? 2 * a.N : a.N;
   const int slabs = (int)(((long)a.K * (T == GP_E4M3 ? 1 : 2) + 127) / 128);
-  const GpCost& k = gp_cost[T == GP_MXFP4 ? 4 : T * 2 + (a.act >= 0)];
+  const bool half = T == GP_E4M3 && a.K % 128;
+  const GpCost& k = gp_cost[T == GP_MXFP4 ? 6 : (half ? 4 : T * 2) + (a.act >= 0)];
   const bool far = T != GP_MXFP4 && a.K > GP_FAR;        // 64x64 alone
   int best = -1, best_sk = 1;
   float best_t = 0.f;
   for (int c = 0; c < 8; c++) {
     const GpTile& g = gp_tiles[c];
     const float one = k.one[c], full = k.full[c];
-    if (one == 0.f || (far && c != 6) ||
-        (c == 0 && T == GP_E4M3 && a.K % 128))
-      continue;
+    if (one == 0.f || (far && c != 6)) continue;
+    const float round = k.round[c] * (a.N % 4 ? k.off : 1.f);
     const long tiles = (long)((a.M + g.bm - 1) / g.bm) *
                        ((width + g.bn - 1) / g.bn);
     for (int sk = 1; sk <= 8; sk++) {
@@ -960,7 +979,7 @@ static GpPick gp_pick(const GpArgs& a, long part_floats, int ncnt) {
         t += one + (full - one) * (k.second + (1.f - k.second) * (rest - 1.f));
       else if (rest > 0.f)
         t += one * (k.first + (1.f - k.first) * rest);
-      t = t * ((slabs + sk - 1) / sk) + (rounds + (rest > 0.f)) * k.round[c];
+      t = t * ((slabs + sk - 1) / sk) + (rounds + (rest > 0.f)) * round;
       // parts written and read, and a trip for each
       if (sk > 1) t += k.split + (float)(parts * k.part);
       if (best < 0 || t < best_t) {
@@ -1058,6 +1077,40 @@ extern "C" float gemm_prompt_time(int fp4, int M, int N, int K, int act,
   a.act = act;
   return fp4 ? gp_pick<GP_MXFP4>(a, part_floats, ncnt).time
              : gp_pick<GP_BF16>(a, part_floats, ncnt).time;
+}
+
+// What a product runs by, on the host alone: rows and outputs of a tile, parts of
+// K, whether by k_gemm_wide, whether W goes past the caches, waves of a block.
+// kind: GP_BF16 ..; all 0: by launch_mid_gemm.
+template <int T>
+static void gp_plan(GpArgs& a, long part_floats, int ncnt, int* out) {
+  const GpPick p = gp_pick<T>(a, part_floats, ncnt);
+  const GpTile& g = gp_tiles[p.tile];
+  const bool far = T != GP_MXFP4 && a.K > GP_FAR;
+  gp_tiling(a, g.bm, a.act >= 0 ? g.bn / 2 : g.bn);
+  out[0] = g.bm;
+  out[1] = g.bn;
+  out[3] = T != GP_MXFP4 && p.tile < 2 && !(T == GP_E4M3 && a.K % 128);
+  out[2] = out[3] ? gw_parts<T>(a.K, p.sk) : p.sk;
+  out[4] = T != GP_MXFP4 && !far && p.tile > 0 && gp_once<T>(a);
+  out[5] = p.tile == 2 || p.tile == 7 || (T == GP_MXFP4 && p.tile > 3) ? 4 : 8;
+}
+
+extern "C" int gemm_prompt_plan(int kind, int M, int N, int K, int act,
+                                long part_floats, int ncnt, int* out) {
+  if (M < 1 || N < 1 || K < 64 || K % 64 || kind < GP_BF16 || kind > GP_MXFP4)
+    return 1;
+  GpArgs a = {};
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.act = act;
+  for (int i = 0; i < 6; i++) out[i] = 0;
+  if (kind == GP_MXFP4) gp_plan<GP_MXFP4>(a, part_floats, ncnt, out);
+  else if (mid_takes(kind == GP_E4M3, M, N, K, act >= 0)) return 0;
+  else if (kind == GP_E4M3) gp_plan<GP_E4M3>(a, part_floats, ncnt, out);
+  else gp_plan<GP_BF16>(a, part_floats, ncnt, out);
+  return 0;
 }
 
 // ---- routed experts --------------------------------------------------------

@@ -60,6 +60,8 @@ _SIGS = {
                       ctypes.c_void_p],
     "launch_gemm_prompt": [ctypes.c_void_p] * 9 + [ctypes.c_long] +
                           [ctypes.c_int] * 5 + [ctypes.c_void_p],
+    "gemm_prompt_plan": [ctypes.c_int] * 5 + [ctypes.c_long, ctypes.c_int,
+                                              ctypes.c_void_p],
     "launch_row_gemm": [ctypes.c_void_p] * 11 + [ctypes.c_long] +
                        [ctypes.c_int] * 11 +
                        [ctypes.c_float, ctypes.c_float, ctypes.c_void_p],
@@ -450,6 +452,23 @@ def gemm(X: torch.Tensor, W: torch.Tensor, Y: torch.Tensor,
     M, K = X.shape
     _gemm_prompt("gemm", X, W, None, None, Y, M, K, res, bias, act, accbuf,
                  cnt)
+
+
+def gemm_prompt_plan(kind: str, M: int, N: int, K: int, act: int = -1,
+                     part: int = 1 << 62, cnt: int = 1024) -> dict | None:
+    """How gemm ("bf16"), gemm_fp8 and gemm_fp4w go about a product with so
+    many floats of accbuf and counters: rows and outputs of a tile, parts of K,
+    whether by the two groups of waves that take turns (wide), whether W is read
+    past the caches (once), waves of a block; None: by mid_gemm.  Host arithmetic
+    only."""
+    out = (ctypes.c_int * 6)()
+    _check(lib().gemm_prompt_plan(
+        ("bf16", "fp8", "fp4").index(kind), M, N, K, act, ctypes.c_long(part),
+        cnt, ctypes.cast(out, ctypes.c_void_p)), "gemm_prompt_plan")
+    if not out[0]:
+        return None
+    return dict(rows=out[0], outputs=out[1], parts=out[2], wide=bool(out[3]),
+                once=bool(out[4]), waves=out[5])
 
 
 FEW_ROWS = 16        # rows that row_gemm takes
