@@ -877,56 +877,46 @@ static const GpTile gp_tiles[8] = {
 // no multiple of four and leave one by one.  0: not for that type (e4m3 in
 // 128x128 by four waves: no product of the fits chose it).
 // The numbers are about us, but fitted to what they choose: the times of every
-// likely tile and split (1 to 8 parts), W from memory, for 17 to 2000 rows of
-// 126 shapes and for 14 numbers of rows each of 30 shapes of models, so that
-// few products take longer than by the numbers before, or than by whole rounds
-// and splits of 1, 2, 4 and 8.  Of 1804 products, and 880 with a gate, above
-// the best, and how many took 4% longer than by the latter, before -> now:
-//   bf16 2.8% -> 1.5%, 51 -> 13; with a gate 2.8% -> 1.9%, 50 -> 7
-//   e4m3 2.0% -> 1.4%, 51 -> 1; with a gate 2.9% -> 1.8%, 29 -> 1
-// (us: 64x256x3584 15.3 -> 10.6; 128x6144x3584 e4m3 19.1 -> 16.6; before, they
-// were fitted to 27 shapes of models, with and without gates alike).  Beside
-// e4m3 rounding sums in another order are other values: K is split as it was
-// but for 2% of the products.  MXFP4 is fitted to 64, 130, 600 and 2048 rows of
+// likely tile and split (1 to 8 parts), W from memory, of 26250 products of 17
+// to 2048 rows, 29 and 12 (with a gate) shapes of models and others of 64 to
+// 24000 outputs and K of 128 to 19200, so that few take longer than by the
+// numbers and kernels before k_gemm_wide and tiles of eight waves.  Above the
+// best of the times, and how many took 4% longer than by those kernels, by
+// numbers fitted to K from 2048 on -> now, half of the products, which were not
+// fitted (outputs a multiple of four):
+//   bf16 2.4% -> 1.6%, 53 -> 27 of 1959; with a gate 2.0% -> 1.0%, 17 -> 2 of 1026
+//   e4m3 2.4%, 21 of 1240, as it was: beside e4m3 rounding parts of K elsewhere
+//       are other values; with a gate 1.4% -> 1.0%, 21 -> 7 of 678
+//   e4m3 rows of half a slab, which k_gemm_wide does not take, by numbers of
+//       their own 3.2% -> 1.7%, 57 -> 30 of 1647; with a gate 2.0% -> 0.9%,
+//       61 -> 14 of 1067
+// (us: 1883x1152x896 17.2 -> 13.8; 789x1536x576 with a gate 12.6 -> 9.2; e4m3
+// 1792x4786x704 63.5 -> 41.9.)  MXFP4 is fitted to 64, 130, 600 and 2048 rows of
 // five shapes (2.2%).
-// The numbers of the 256-wide tiles (and of bf16 128x128 of eight waves) were
-// fitted again when k_gemm_wide took them over, to 432 products of 100 to 2048
-// rows of 27 shapes.  Above the best, and how many by more than 4%, by the
-// numbers that were -> now: bf16 1.0% -> 0.8%, 14 -> 9; with a gate 0.2%, 1;
-// e4m3 1.9% -> 0.3%, 14 -> 3; with a gate 9.4% -> 0.2%, 29 -> 1.  And, to 648
-// of 20 to 2048 rows, those of the others when 64x64, 64x128 and 128x64 went
-// from four waves to eight (64 rows of 16384x2048 18.5 -> 17.4, 100 of
-// 8192x2048 21.4 to 24.4 -> 12.8 to 21.4; over all 4% in bf16, 5% in e4m3):
-// bf16 2.0% -> 1.3%, with a gate 1.2% -> 0.8%, e4m3 as it was 1.5%, with a gate
-// 1.1% -> 0.5%.
-// e4m3 rows with half a slab at their end, which k_gemm_wide does not take, have
-// numbers of their own, fitted to half of 8474 products: above the best of the
-// others' 3.2% -> 1.7%, 4% longer than before k_gemm_wide 57 -> 30 of 1647; with a
-// gate 2.0% -> 0.9%, 61 -> 14 of 1067 (1792x4786x704 63.5 us, so 41.9).
 struct GpCost {
   float one[8], full[8], round[8], second, first, split, part, off;
 };
 static const GpCost gp_cost[7] = {
     {// bf16
-     {1.29f, 0.665f, 0.62f, 0.51f, 1.24f, 0.443f, 0.261f, 0.257f},
-     {1.29f, 0.665f, 1.09f, 0.51f, 1.37f, 1.07f, 0.501f, 0.438f},
-     {7.85f, 3.82f, 2.87f, 4.5f, 2.1f, 1.21f, 1.54f, 1.24f},
-     0.7f, 1.f, 2.22f, 4.94e-6f, 1.f},
+     {1.4f, 0.864f, 0.807f, 0.608f, 2.27f, 0.463f, 0.305f, 0.26f},
+     {1.4f, 0.864f, 1.66f, 0.608f, 4.51f, 0.729f, 0.536f, 0.518f},
+     {13.9f, 6.96f, 4.85f, 4.27f, 2.55f, 3.19f, 2.01f, 1.77f},
+     0.904f, 0.846f, 1.43f, 4.03e-6f, 2.92f},
     {// bf16 with a gate
-     {1.46f, 0.87f, 0.592f, 0.518f, 0.854f, 0.481f, 0.261f, 0.234f},
-     {1.46f, 0.87f, 1.22f, 0.518f, 0.854f, 0.822f, 0.576f, 0.312f},
-     {4.86f, 3.2f, 2.36f, 3.37f, 2.56f, 2.98f, 1.09f, 1.56f},
-     0.616f, 0.96f, 1.77f, 4.79e-6f, 1.f},
+     {1.17f, 0.775f, 1.85f, 0.523f, 0.556f, 0.507f, 0.317f, 0.262f},
+     {1.17f, 0.775f, 4.01f, 0.523f, 0.914f, 0.66f, 0.556f, 0.576f},
+     {20.f, 11.9f, 4.6f, 8.12f, 4.74f, 5.17f, 3.97f, 3.58f},
+     1.f, 0.854f, 2.25f, 3.92e-6f, 1.f},
     {// e4m3
      {1.76f, 0.954f, 0.f, 0.752f, 0.633f, 0.892f, 0.405f, 0.286f},
      {1.76f, 0.954f, 0.f, 0.752f, 0.817f, 0.892f, 0.556f, 0.449f},
      {6.f, 3.81f, 0.f, 2.16f, 2.07f, 2.84f, 1.14f, 1.21f},
      0.626f, 0.952f, 0.273f, 5.43e-6f, 1.f},
     {// e4m3 with a gate
-     {1.87f, 1.17f, 0.f, 0.745f, 0.651f, 0.78f, 0.45f, 0.286f},
-     {1.87f, 1.17f, 0.f, 0.745f, 0.878f, 0.78f, 0.45f, 0.474f},
-     {6.f, 3.98f, 0.f, 2.18f, 1.8f, 1.28f, 1.68f, 1.85f},
-     0.632f, 1.f, 0.778f, 4.63e-6f, 1.f},
+     {2.43f, 1.66f, 0.f, 1.04f, 0.897f, 0.775f, 0.439f, 0.299f},
+     {2.43f, 1.66f, 0.f, 1.04f, 1.36f, 1.15f, 0.717f, 0.505f},
+     {6.56f, 3.27f, 0.f, 2.88f, 0.546f, 0.677f, 0.926f, 1.05f},
+     0.656f, 1.f, 1.06f, 3.35e-6f, 1.f},
     {// e4m3, half a slab at the end of a row
      {0.f, 1.84f, 0.f, 1.03f, 0.903f, 0.842f, 0.589f, 0.374f},
      {0.f, 1.84f, 0.f, 1.03f, 1.29f, 1.22f, 0.836f, 0.618f},

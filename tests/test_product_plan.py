@@ -34,3 +34,21 @@ def test_only_whole_slabs_go_by_two_groups_of_waves(M, N, K, act):
     assert not plan("fp8", M, N, K + 64, act)["wide"]
     assert plan("bf16", M, N, K, act)["wide"]
     assert not plan("fp4", M, N, K, act)["wide"]
+
+
+# few slabs: what a tile takes before its first product and behind its last
+# weighs more than a slab, by 128x128 tiles of four waves above all
+@pytest.mark.parametrize("kind,M,N,K,act", [
+    ("bf16", 789, 1536, 576, 0), ("bf16", 1159, 1536, 576, 0),
+    ("bf16", 746, 1748, 768, 0), ("bf16", 1883, 1152, 896, -1),
+    ("bf16", 1024, 2344, 384, -1), ("bf16", 226, 10756, 832, -1)])
+def test_few_slabs_are_not_for_four_waves(kind, M, N, K, act):
+    assert plan(kind, M, N, K, act)["waves"] == 8
+
+
+# outputs that are no multiple of four leave one by one: a large tile has most
+@pytest.mark.parametrize("M,N,K", [(144, 16890, 384), (397, 8358, 512),
+                                   (388, 8605, 832), (816, 4690, 128)])
+def test_outputs_that_leave_one_by_one(M, N, K):
+    p = plan("bf16", M, N, K)
+    assert p["rows"] * p["outputs"] < 128 * 128
