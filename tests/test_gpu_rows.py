@@ -388,59 +388,150 @@ def test_many_rows(M, N, K, kind, act):
     assert (Y[M] == 7.0).all() and not cnt.any()
 
 
-# each tile by itself and with K split over blocks, where the sizes above leave
-# it out: 256x256 (bf16), 128x256, 128x128 of eight waves, 64x128, 128x64;
-# parts of 128x128, 64x128, 64x64 and 32x64
-@pytest.mark.parametrize("M,N,K,kind,act", [
-    (1037, 10902, 192, "bf16", -1), (525, 11405, 704, "bf16", -1),
-    (513, 3878, 512, "bf16", -1), (1601, 598, 5632, "bf16", -1),
-    (132, 16809, 64, "bf16", -1), (429, 376, 2112, "bf16", -1),
-    (66, 58, 896, "bf16", -1), (517, 1812, 448, "bf16", 0),
-    (589, 418, 7552, "bf16", 0), (130, 8243, 128, "bf16", 0),
-    (33, 8564, 6720, "bf16", 0), (582, 1621, 1152, "bf16", 0),
-    (43, 65, 960, "bf16", 0), (26, 129, 2112, "bf16", 0),
-    (584, 5294, 192, "fp8", -1), (871, 4614, 448, "fp8", -1),
-    (425, 340, 6400, "fp8", -1), (67, 70, 960, "fp8", -1),
-    (137, 7852, 448, "fp8", 0), (596, 845, 7680, "fp8", 0),
-    (19, 16845, 64, "fp8", 0), (378, 193, 5056, "fp8", 0)])
-def test_many_rows_of_each_tile(M, N, K, kind, act):
+# each tile (rows and outputs, parts of K, waves, whether by two groups of them) by
+# itself and with K split over blocks, where the sizes above leave it out; 128x256
+# of e4m3 rows with half a slab too, 128x128 of four waves and of eight
+@pytest.mark.parametrize("M,N,K,kind,act,tile", [
+    (1037, 10902, 192, "bf16", -1, (128, 128, 1, 4, False)),
+    (525, 11405, 704, "bf16", -1, (128, 256, 1, 8, True)),
+    (513, 3878, 512, "bf16", -1, (128, 64, 1, 8, False)),
+    (1601, 598, 5632, "bf16", -1, (128, 128, 3, 8, False)),
+    (132, 16809, 64, "bf16", -1, (64, 128, 1, 8, False)),
+    (429, 376, 2112, "bf16", -1, (64, 64, 3, 8, False)),
+    (66, 58, 896, "bf16", -1, (32, 64, 3, 4, False)),
+    (517, 1812, 448, "bf16", 0, (128, 64, 1, 8, False)),
+    (589, 418, 7552, "bf16", 0, (128, 128, 5, 8, False)),
+    (130, 8243, 128, "bf16", 0, (64, 128, 1, 8, False)),
+    (33, 8564, 6720, "bf16", 0, (64, 128, 3, 8, False)),
+    (582, 1621, 1152, "bf16", 0, (64, 64, 1, 8, False)),
+    (43, 65, 960, "bf16", 0, (32, 64, 1, 4, False)),
+    (26, 129, 2112, "bf16", 0, (32, 64, 7, 4, False)),
+    (584, 5294, 192, "fp8", -1, (128, 64, 1, 8, False)),
+    (871, 4614, 448, "fp8", -1, (128, 64, 1, 8, False)),
+    (425, 340, 6400, "fp8", -1, (64, 64, 5, 8, False)),
+    (67, 70, 960, "fp8", -1, (32, 64, 1, 4, False)),
+    (137, 7852, 448, "fp8", 0, (128, 64, 1, 8, False)),
+    (596, 845, 7680, "fp8", 0, (128, 64, 3, 8, False)),
+    (19, 16845, 64, "fp8", 0, (64, 128, 1, 8, False)),
+    (378, 193, 5056, "fp8", 0, (32, 64, 2, 4, False)),
+    (145, 16724, 448, "fp8", -1, (64, 128, 1, 8, False)),
+    (174, 5488, 6464, "fp8", -1, (64, 128, 3, 8, False)),
+    (98, 8286, 6464, "fp8", -1, (128, 64, 3, 8, False)),
+    (68, 16752, 3264, "fp8", -1, (128, 128, 1, 8, False)),
+    (99, 8213, 9600, "fp8", -1, (128, 128, 3, 8, False)),
+    (200, 16680, 448, "fp8", -1, (128, 256, 1, 8, False)),
+    (330, 3640, 19264, "fp8", -1, (128, 256, 5, 8, False)),
+    (214, 2487, 9600, "fp8", 0, (128, 128, 3, 8, False)),
+    (130, 6977, 4096, "fp8", 0, (128, 128, 1, 8, False)),
+    (133, 12433, 448, "fp8", 0, (128, 256, 1, 8, False)),
+    (335, 2003, 19264, "fp8", 0, (128, 256, 5, 8, False)),
+    (166, 2812, 9600, "fp8", 0, (64, 128, 3, 8, False)),
+    (66, 2853, 9600, "fp8", 0, (128, 64, 5, 8, False)),
+    (67, 2744, 9600, "bf16", -1, (128, 64, 5, 8, False)),
+    (66, 1512, 9600, "bf16", 0, (128, 64, 5, 8, False)),
+    (69, 8808, 2112, "bf16", 0, (128, 128, 1, 8, False)),
+    (35, 1835, 3264, "bf16", 0, (64, 64, 4, 8, False)),
+    (905, 8494, 384, "bf16", -1, (64, 64, 1, 8, False)),
+    (391, 10822, 192, "bf16", -1, (128, 128, 1, 4, False)),
+    (1045, 11186, 192, "bf16", -1, (128, 128, 1, 4, False)),
+    (675, 10949, 320, "bf16", -1, (64, 64, 1, 8, False)),
+    (199, 8994, 8192, "bf16", -1, (128, 128, 1, 8, False)),
+    (385, 8380, 64, "bf16", 0, (64, 128, 1, 8, False)),
+    (1188, 9848, 64, "bf16", 0, (128, 128, 1, 4, False)),
+    (1159, 9732, 128, "bf16", 0, (128, 128, 1, 4, False)),
+    (1052, 10895, 192, "bf16", 0, (128, 64, 1, 8, False)),
+    (259, 8593, 128, "bf16", 0, (64, 128, 1, 8, False)),
+    (566, 10887, 128, "bf16", 0, (128, 128, 1, 4, False)),
+    (555, 11005, 192, "bf16", 0, (128, 64, 1, 8, False)),
+    (1167, 9842, 128, "fp8", 0, (64, 128, 1, 8, False)),
+    (1164, 9823, 256, "fp8", 0, (128, 64, 1, 8, False)),
+    (1156, 10068, 384, "fp8", 0, (64, 128, 1, 8, False)),
+    (547, 11509, 128, "fp8", 0, (64, 128, 1, 8, False)),
+    (542, 11246, 256, "fp8", 0, (128, 64, 1, 8, False)),
+    (521, 11510, 384, "fp8", 0, (128, 64, 1, 8, False))])
+def test_many_rows_of_each_tile(M, N, K, kind, act, tile):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    p = ho.gemm_prompt_plan(kind, M, N, K, act, 1 << 24, 1024)
+    assert (p["rows"], p["outputs"], p["parts"], p["waves"],
+            p["wide"]) == tile
     test_many_rows(M, N, K, kind, act)
 
 
-# tiles 256 wide: slabs fewer than the ring holds, one, two and three, and
-# several tiles a block (more than 256), so that one's slabs are asked for
-# while another is multiplied; 256 and 128 rows, with a rest both ways; parts
-# of K, also with a short last one
-@pytest.mark.parametrize("M,N,K,kind,act", [
-    (905, 8494, 384, "bf16", -1), (391, 10822, 192, "bf16", -1),
-    (1045, 11186, 192, "bf16", -1), (675, 10949, 320, "bf16", -1),
-    (153, 11205, 12864, "bf16", -1), (199, 8994, 8192, "bf16", -1),
-    (223, 2589, 17600, "bf16", 0),
-    (385, 8380, 64, "bf16", 0), (1188, 9848, 64, "bf16", 0),
-    (1159, 9732, 128, "bf16", 0), (1052, 10895, 192, "bf16", 0),
-    (1025, 10942, 256, "bf16", 0), (259, 8593, 128, "bf16", 0),
-    (566, 10887, 128, "bf16", 0), (555, 11005, 192, "bf16", 0),
-    (793, 10086, 128, "fp8", -1), (840, 9423, 384, "fp8", -1),
-    (332, 11127, 128, "fp8", -1), (330, 10970, 256, "fp8", -1),
-    (340, 11179, 384, "fp8", -1), (1167, 9842, 128, "fp8", 0),
-    (1164, 9823, 256, "fp8", 0), (1156, 10068, 384, "fp8", 0),
-    (547, 11509, 128, "fp8", 0), (542, 11246, 256, "fp8", 0),
-    (521, 11510, 384, "fp8", 0)])
-def test_many_rows_of_wide_tiles(M, N, K, kind, act):
+# tiles 256 wide by two groups of waves: slabs fewer than the ring holds, one,
+# two and three, and several tiles a block (more than 256), so that one's slabs
+# are asked for while another is multiplied; 256 and 128 rows, with a rest both
+# ways; parts of K, also with a short last one
+@pytest.mark.parametrize("M,N,K,kind,act,rows,parts", [
+    (153, 11205, 12864, "bf16", -1, 128, 2),
+    (223, 2589, 17600, "bf16", 0, 128, 5),
+    (1025, 10942, 256, "bf16", 0, 256, 1),
+    (793, 10086, 128, "fp8", -1, 256, 1), (840, 9423, 384, "fp8", -1, 256, 1),
+    (332, 11127, 128, "fp8", -1, 128, 1), (330, 10970, 256, "fp8", -1, 128, 1),
+    (340, 11179, 384, "fp8", -1, 128, 1),
+    (195, 16680, 192, "bf16", -1, 128, 1),
+    (790, 16468, 192, "bf16", -1, 128, 1),
+    (1290, 10764, 320, "bf16", -1, 128, 1),
+    (788, 16657, 512, "bf16", -1, 128, 1),
+    (131, 16672, 768, "bf16", -1, 128, 1),
+    (131, 8688, 9600, "bf16", -1, 128, 3),
+    (652, 16604, 192, "bf16", -1, 256, 1),
+    (1807, 13164, 192, "bf16", -1, 256, 1),
+    (1409, 16516, 320, "bf16", -1, 256, 1),
+    (401, 16808, 640, "bf16", -1, 256, 1),
+    (196, 12624, 192, "bf16", 0, 128, 1), (341, 16438, 256, "bf16", 0, 128, 1),
+    (258, 16470, 512, "bf16", 0, 128, 1), (137, 11036, 576, "bf16", 0, 128, 1),
+    (130, 4100, 9600, "bf16", 0, 128, 3), (390, 14161, 128, "bf16", 0, 256, 1),
+    (709, 16463, 128, "bf16", 0, 256, 1), (654, 16797, 256, "bf16", 0, 256, 1),
+    (195, 16406, 576, "bf16", 0, 256, 1), (661, 16536, 576, "bf16", 0, 256, 1),
+    (194, 16525, 128, "fp8", -1, 128, 1), (784, 16783, 128, "fp8", -1, 128, 1),
+    (815, 16762, 512, "fp8", -1, 128, 1),
+    (194, 16444, 1152, "fp8", -1, 128, 1),
+    (327, 3782, 19200, "fp8", -1, 128, 4),
+    (1562, 15116, 128, "fp8", -1, 256, 1),
+    (1539, 15149, 512, "fp8", -1, 256, 1),
+    (449, 16753, 1152, "fp8", -1, 256, 1), (261, 10856, 384, "fp8", 0, 128, 1),
+    (321, 16544, 640, "fp8", 0, 128, 1), (262, 16482, 1152, "fp8", 0, 128, 1),
+    (201, 2728, 12800, "fp8", 0, 128, 5), (196, 4232, 8192, "fp8", 0, 128, 3),
+    (1094, 1808, 12800, "fp8", 0, 128, 3), (400, 15116, 256, "fp8", 0, 256, 1),
+    (780, 15087, 384, "fp8", 0, 256, 1), (264, 13676, 896, "fp8", 0, 256, 1),
+    (641, 16697, 1152, "fp8", 0, 256, 1)])
+def test_many_rows_of_wide_tiles(M, N, K, kind, act, rows, parts):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    p = ho.gemm_prompt_plan(kind, M, N, K, act, 1 << 24, 1024)
+    assert p["wide"] and (p["rows"], p["parts"]) == (rows, parts)
     test_many_rows(M, N, K, kind, act)
 
 
 # one row of tiles beside 32 MB of W or just less of it: read past the caches
-# by each tile of up to 128 rows, with a rest both ways and parts of K
-@pytest.mark.parametrize("M,N,K,kind,act", [
-    (37, 8203, 2048, "bf16", 0), (61, 2050, 8256, "bf16", -1),
-    (65, 16850, 1088, "bf16", -1), (99, 9001, 2048, "bf16", -1),
-    (128, 14300, 2048, "bf16", 0), (128, 28690, 640, "bf16", -1),
-    (128, 8190, 2048, "bf16", -1), (70, 4110, 8192, "bf16", -1),
-    (33, 8203, 4096, "fp8", 0), (57, 16500, 2176, "fp8", -1),
-    (128, 8400, 2176, "fp8", 0), (121, 17010, 2112, "fp8", -1),
-    (128, 34000, 1024, "fp8", -1), (128, 4099, 8320, "fp8", -1)])
-def test_many_rows_beside_large_weights(M, N, K, kind, act):
+# (once) by each tile of up to 128 rows, with a rest both ways and parts of K
+@pytest.mark.parametrize("M,N,K,kind,act,tile,once", [
+    (37, 8203, 2048, "bf16", 0, (64, 128, 1), True),
+    (61, 2050, 8256, "bf16", -1, (64, 64, 6), True),
+    (65, 16850, 1088, "bf16", -1, (128, 64, 1), True),
+    (99, 9001, 2048, "bf16", -1, (64, 64, 1), False),
+    (128, 14300, 2048, "bf16", 0, (128, 128, 1), True),
+    (128, 28690, 640, "bf16", -1, (128, 64, 1), True),
+    (128, 8190, 2048, "bf16", -1, (64, 64, 1), False),
+    (70, 4110, 8192, "bf16", -1, (64, 64, 3), False),
+    (33, 8203, 4096, "fp8", 0, (64, 64, 1), True),
+    (57, 16500, 2176, "fp8", -1, (64, 64, 1), True),
+    (128, 8400, 2176, "fp8", 0, (128, 64, 1), True),
+    (121, 17010, 2112, "fp8", -1, (128, 64, 1), True),
+    (128, 34000, 1024, "fp8", -1, (128, 256, 1), True),
+    (128, 4099, 8320, "fp8", -1, (64, 64, 3), False),
+    (67, 16613, 512, "bf16", 0, (128, 256, 1), True),
+    (65, 16690, 576, "bf16", 0, (128, 256, 1), True),
+    (66, 16396, 1152, "fp8", 0, (128, 256, 1), True),
+    (40, 16400, 2048, "fp8", 0, (64, 128, 1), True),
+    (20, 70000, 256, "bf16", -1, (32, 64, 1), True),
+    (64, 8200, 4096, "bf16", -1, (64, 64, 1), True)])
+def test_many_rows_beside_large_weights(M, N, K, kind, act, tile, once):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
+    p = ho.gemm_prompt_plan(kind, M, N, K, act, 1 << 24, 1024)
+    assert (p["rows"], p["outputs"], p["parts"]) == tile and p["once"] == once
     test_many_rows(M, N, K, kind, act)
 
 
@@ -794,6 +885,24 @@ def test_experts_of_many_rows(M, E, top, kind, H=192, I=320):
     (2200, 1, 1, 2112, 1088), (520, 8, 2, 384, 1536), (300, 3, 1, 640, 5504)])
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
 def test_experts_of_wide_tiles(M, E, top, H, I, kind):
+    test_experts_of_many_rows(M, E, top, kind, H, I)
+
+
+# more tiles than blocks: one expert's slabs are asked for while another's are
+# multiplied.  Both products, the first alone; one slab, two, three, many; an
+# expert with hardly a row.  The shares of experts are as above.
+@pytest.mark.parametrize("M,E,top,H,I,both", [
+    (1500, 4, 2, 2944, 1792, True), (1100, 8, 2, 3584, 2176, True),
+    (2100, 8, 1, 128, 4224, False), (1100, 8, 2, 256, 4096, False),
+    (1300, 12, 2, 384, 3328, False), (900, 3, 1, 640, 5504, False)])
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+def test_experts_of_several_tiles_a_block(M, E, top, H, I, both, kind):
+    r = torch.rand(M, E, generator=torch.Generator().manual_seed(5))
+    r[:, E - 1] *= 0.01
+    rows = torch.bincount(r.topk(top, 1).indices.reshape(-1), minlength=E)
+    tiles = (-(-rows // 128)).sum().item()
+    assert M * top >= 96 * E and tiles * -(-2 * I // 256) > 256 + 32
+    assert (tiles * -(-H // 256) > 256 + 32) == both
     test_experts_of_many_rows(M, E, top, kind, H, I)
 
 
