@@ -236,7 +236,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) k_gemm_prompt(GpArgs a) {
   const int tiles = a.tm * a.tn, chunk = (tiles + 7) / 8;
   const int tile = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= chunk || tile >= tiles) return;
-  const GpAt at = gp_at(a, tile);
+  const GpAt at = MOE ? GpAt{tile % a.tm, tile / a.tm} : gp_at(a, tile);
   const int bm = MOE ? 0 : at.row * BM;
   const int bn = at.col * (GLU ? BN / 2 : BN);
   // the rows of a tile that are there
