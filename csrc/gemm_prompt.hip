@@ -1218,6 +1218,34 @@ static hipError_t gp_experts(GpArgs a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Whether routed experts go by k_gemm_wide: 128x256 tiles in turns with more than
+// a 128x128 tile a CU to do (8 experts, 1100 rows, 2 each, 2048->2x4096 143 us, so
+// 107, e4m3 101, 69; 4096->2048 80, 64; 700 rows 4096->2x14336 594, 478; 16 experts
+// of 1024 30, 21).  With a tile a CU or less the small ones end sooner: 700 rows
+// 4096->2048 46, 60.  Row offsets have 32 bits.
+//
+// The host does not know what the router chose.  It counts on half a row tile an
+// expert for the last of its rows, but on no more than if all had as many: eight
+// of 212 rows each have 16 tiles, not 17 (848 rows, 2 each, 4096->2048 47 us by
+// small tiles, 64 by wide ones).  Of 17900 products 4% slower than by small tiles
+// as they were 461 without that bound, 248 with it.
+static bool expert_wide(bool f8, int pairs, int E, int N, int K, int act) {
+  const int glu = act >= 0 ? 2 : 1, even = E * ((pairs / E + 127) / 128);
+  const float tiles = fminf(pairs / 128.f + E / 2.f, even);
+  return expert_bm(pairs, E) == 128 && !(f8 && K % 128) &&
+         (size_t)pairs * K * (f8 ? 1 : 2) <= UINT32_MAX &&
+         tiles * ((N * glu + 127) / 128) > 256.f;
+}
+
+// Rows of a tile and whether by k_gemm_wide, on the host alone
+extern "C" int expert_gemm_plan(int f8, int pairs, int E, int N, int K, int act,
+                                int* out) {
+  if (pairs < 1 || E < 1 || E > 64 || N < 1 || K < 64 || K % 64) return 1;
+  out[0] = expert_bm(pairs, E);
+  out[1] = expert_wide(f8, pairs, E, N, K, act);
+  return 0;
+}
+
 // y = x W^T of each pair's expert.  sorted: of launch_expert_sort.  gather: x
 // by token, y in the sorted order; else x in that order, y by pair.
 extern "C" hipError_t launch_expert_gemm(
@@ -1233,17 +1261,8 @@ extern "C" hipError_t launch_expert_gemm(
               nullptr, (u16*)y, nullptr, nullptr, pairs, N, K, act, tiles, 0, tiles,
               p, p + pairs, p + pairs + tiles, p + pairs + 2 * tiles, top,
               gather};
-  // 128x256 tiles in turns with more than a 128x128 tile a CU to do, half a
-  // row tile an expert counted on for the last of its rows: 8 experts, 1100
-  // rows, 2 each, 2048->2x4096 143 us, so 107 (e4m3 101, 69), 4096->2048 80,
-  // 64; 700 rows 4096->2x14336 594, 478; 16 experts of 1024 30, 21.  With a
-  // tile a CU or less the small ones end sooner: 700 rows 4096->2048 46,
-  // 60.  Row offsets have 32 bits.
-  const int glu = act >= 0 ? 2 : 1;
-  if (bm == 128 && (!sx || K % 128 == 0) &&
-      (size_t)pairs * K * (sx ? 1 : 2) <= UINT32_MAX &&
-      (pairs / 128 + E / 2) * ((N * glu + 127L) / 128) > 256) {
-    a.tn = (N * glu + 255) / 256;
+  if (expert_wide(sx, pairs, E, N, K, act)) {
+    a.tn = (N * (act >= 0 ? 2 : 1) + 255) / 256;
     const int share = (tiles * a.tn + 7) / 8;
     const dim3 grid(8 * (share < 32 ? share : 32)), nt(512);
 #define WIDE(F8, GLU)                                                        \

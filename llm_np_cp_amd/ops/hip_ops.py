@@ -100,6 +100,7 @@ _SIGS = {
                           [ctypes.c_long, ctypes.c_void_p],
     "launch_expert_gemm": [ctypes.c_void_p] * 6 + [ctypes.c_int] * 7 +
                           [ctypes.c_void_p],
+    "expert_gemm_plan": [ctypes.c_int] * 6 + [ctypes.c_void_p],
     "launch_expert_sum": [ctypes.c_void_p] * 4 + [ctypes.c_int] * 3 +
                          [ctypes.c_void_p],
     "launch_moe_scale_add": [ctypes.c_void_p] * 3 +
@@ -1007,6 +1008,17 @@ def expert_gemm(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor,
     _check(lib().launch_expert_gemm(
         _ptr(x), _ptr(w), _ptr(sx), _ptr(sw), _ptr(y), _ptr(order), pairs, E,
         top, int(gather), N, K, act, _stream()), "expert_gemm")
+
+
+def expert_gemm_plan(kind: str, pairs: int, E: int, N: int, K: int,
+                     act: int = -1) -> dict:
+    """Rows of expert_gemm's tiles and whether two groups of waves take turns at
+    them (wide).  Host arithmetic only."""
+    out = (ctypes.c_int * 2)()
+    _check(lib().expert_gemm_plan(
+        ("bf16", "fp8").index(kind), pairs, E, N, K, act,
+        ctypes.cast(out, ctypes.c_void_p)), "expert_gemm_plan")
+    return dict(rows=out[0], wide=bool(out[1]))
 
 
 def expert_sum(y: torch.Tensor, w: torch.Tensor, idx: torch.Tensor,

@@ -22,7 +22,7 @@ from torch.utils._python_dispatch import TorchDispatchMode
 INTS, FLOATS = 32, 8
 # native functions that enqueue nothing
 ASKS = frozenset(("row_gemm_plan", "chain_slots", "stack_chunk_rows",
-                  "attn_prefill_plan", "gemm_prompt_plan"))
+                  "attn_prefill_plan", "gemm_prompt_plan", "expert_gemm_plan"))
 _local = threading.local()
 
 

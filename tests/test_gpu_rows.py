@@ -894,15 +894,20 @@ def test_experts_of_wide_tiles(M, E, top, H, I, kind):
 @pytest.mark.parametrize("M,E,top,H,I,both", [
     (1500, 4, 2, 2944, 1792, True), (1100, 8, 2, 3584, 2176, True),
     (2100, 8, 1, 128, 4224, False), (1100, 8, 2, 256, 4096, False),
-    (1300, 12, 2, 384, 3328, False), (900, 3, 1, 640, 5504, False)])
+    (1300, 12, 2, 384, 3328, False), (900, 3, 1, 640, 5504, False),
+    (1000, 64, 8, 128, 640, False)])
 @pytest.mark.parametrize("kind", ["bf16", "fp8"])
 def test_experts_of_several_tiles_a_block(M, E, top, H, I, both, kind):
+    from llm_np_cp_amd.ops import hip_ops as ho
+
     r = torch.rand(M, E, generator=torch.Generator().manual_seed(5))
     r[:, E - 1] *= 0.01
     rows = torch.bincount(r.topk(top, 1).indices.reshape(-1), minlength=E)
     tiles = (-(-rows // 128)).sum().item()
-    assert M * top >= 96 * E and tiles * -(-2 * I // 256) > 256 + 32
+    assert tiles * -(-2 * I // 256) > 256 + 32
     assert (tiles * -(-H // 256) > 256 + 32) == both
+    assert ho.expert_gemm_plan(kind, M * top, E, I, H, 0)["wide"]
+    assert ho.expert_gemm_plan(kind, M * top, E, H, I)["wide"] == both
     test_experts_of_many_rows(M, E, top, kind, H, I)
 
 

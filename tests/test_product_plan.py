@@ -52,3 +52,18 @@ def test_few_slabs_are_not_for_four_waves(kind, M, N, K, act):
 def test_outputs_that_leave_one_by_one(M, N, K):
     p = plan("bf16", M, N, K)
     assert p["rows"] * p["outputs"] < 128 * 128
+
+
+# no more row tiles are counted on than experts of as many rows each have: those
+# leave small tiles one a CU, which end before half as many wide ones
+@pytest.mark.parametrize("M,E,top,N,K,act,wide", [
+    (848, 8, 2, 2048, 4096, -1, False), (456, 4, 2, 4096, 14336, -1, False),
+    (192, 4, 4, 2048, 4096, 0, False), (1100, 8, 2, 2048, 4096, -1, True),
+    (1100, 8, 2, 4096, 2048, 0, True), (700, 8, 2, 14336, 4096, 0, True),
+    (700, 8, 2, 2048, 4096, -1, False), (300, 8, 2, 14336, 4096, 0, False)])
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+def test_wide_tiles_of_experts(M, E, top, N, K, act, wide, kind):
+    p = ho.expert_gemm_plan(kind, M * top, E, N, K, act)
+    assert p["wide"] == wide and (p["rows"] == 128 or not wide)
+    if kind == "fp8":
+        assert not ho.expert_gemm_plan(kind, M * top, E, N, K + 64, act)["wide"]
