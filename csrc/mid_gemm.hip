@@ -343,20 +343,24 @@ static bool mid_takes_few(bool f8, int M, int N, int K) {
   return K % 8192 || N <= (M > 12 ? 3584 : 2560);
 }
 
-// More rows and gates: us, the best tile / here, W from memory, 17 to 64 rows
-// of 126 shapes:
-//   bf16  rows of up to 4.5 KB  2304x2048 17 rows 10.2/7.5, 64 11.7/10.3;
-//       6144x2048 48 1.07 of the time here, 64 1.03
-//     up to 8 KB  17x3584x3584 12.8/10.5, 48 15.2/14.5; the more rows of X, the
-//       more columns it takes to be worth their way (48x1024x4096 0.85,
-//       48x3072x4096 1.04, 64x3072x4096 0.94 of the time here), and 4608 make
-//       144 blocks of 32, too few (33x4608x3584 0.96)
-//     longer  3072x8192 24 rows 17.4/17.1, 48 19.9/20.4; 3584x14336 17
-//       25.6/24.4, 32 26.2/27.7; 17x4608x14336 0.78
-//   e4m3  4096x4096 17 12.1/8.0, 64 13.0/11.1; 3584x14336 17 18.8/16.4, 64
-//       22.5/22.4; 512x8192 64 12.1/15.5
-//   gate  8192x2048 17 19.2/15.4, 32 19.2/17.1; 17x8192x3584 24.4/25.5; e4m3
-//       8192x2048 17 12.5/10.2, 6144x1024 32 8.5/9.7
+// More rows and gates: us, the best tile / here, W from memory:
+//   bf16  rows of up to 4.5 KB  2304x2048 17 rows 8.5/6.0, 64 8.8/7.7; 6144x2048
+//       48 11.7/10.6, 64 12.3/11.5
+//     up to 8 KB  17x3584x3584 12.0/9.2, 48 13.2/12.1; the more rows of X, the
+//       more columns it takes to be worth their way (48x1024x4096 9.2/10.0,
+//       48x3072x4096 12.4/11.9, 64x3072x4096 12.9/13.4), and 4608 make 144
+//       blocks of 32, too few (33x4608x3584 13.9/14.9)
+//     longer  3072x8192 24 rows 15.5/15.9, 48 17.3/19.6; 3584x14336 17
+//       22.7/23.5, 32 23.8/26.7; 17x4608x14336 27.0/38.1
+//   e4m3  4096x4096 17 10.6/6.7, 64 11.0/8.6; 3584x14336 17 16.5/15.7, 64
+//       20.0/20.6; 512x8192 64 9.6/11.4
+//   gate  8192x2048 17 16.7/14.7, 32 16.6/16.5; 17x8192x3584 21.7/25.0; e4m3
+//       8192x2048 17 10.8/9.6, 6144x1024 32 6.4/8.7
+// The lines lie where they did beside tiles of four waves, to which most of
+// this was further ahead.  By times of 5200 products without a gate and 1060
+// with one: of the 4119 and 352 that are taken a tile is 4 and 5% faster for 309
+// and 121 (bf16 of more than 8 KB a row, 32 rows with a gate), of those left 191
+// and 92 are slower by tiles.
 bool mid_takes(bool f8, int M, int N, int K, bool glu) {
   if (glu)
     return M > 16 && M <= 32 && N <= 8192 && K <= 2048 &&
