@@ -248,13 +248,13 @@ extern "C" hipError_t stack_forward(const StackPlan* plan, int M, int keys,
 // of 128 where as many chunks take less so by the numbers that choose the
 // products' tiles.  2048 rows of 2304 outputs are 288 tiles, one round of 256
 // CUs and a rest; 1792 are 252.  ms, chunks of 2048 -> as here, four layers 2304
-// wide: 2100 rows 2.46 -> 2.28, 3000 3.27 -> 2.93, 5003 5.34 -> 4.74.  Where 2048
-// rows are whole rounds they stay: two layers 4096 wide, 5003 rows 4.86, in
-// chunks of 1792 5.18.  A chunk more costs what it saves (2048 rows 2304 wide
-// 2.11, as 1792 and 256 2.27).  A rest of 64 rows and fewer goes by other
+// wide: 2100 rows 2.29 -> 2.11, 3000 3.04 -> 2.80, 5003 5.02 -> 4.49.  Where 2048
+// rows are whole rounds they stay: two layers 4096 wide, 5003 rows 4.47, in
+// chunks of 1792 4.78.  A chunk more costs what it saves (2048 rows 2304 wide
+// 1.91, as 1792 and 256 2.08).  A rest of 64 rows and fewer goes by other
 // kernels than the numbers are of, and attention is in them by 3% alone: over
-// 105 lengths up to 8300 rows of six widths where chunks are smaller for it,
-// none took longer (0.99 to 1.16 times as fast).  Beside e4m3 rows sums in another order are other
+// 24 lengths up to 8000 rows of six widths none took longer (0.995 to 1.12 times
+// as fast).  Beside e4m3 rows sums in another order are other
 // values, and routed experts' rows are where the router sends them: these stay.
 extern "C" int stack_chunk_rows(const StackPlan* plan, int n, int most) {
   const StackPlan& p = *plan;
