@@ -1035,13 +1035,16 @@ def test_rotated_rows(hd, nh, kvh, M, pos0, kv8):
 
 
 # prompts of one batch: one wave a tile and four, a sequence that goes on
-# behind earlier keys, windows, keys split over blocks, pools out of order
+# behind earlier keys, windows, keys split over blocks, pools out of order; parts
+# of the keys row by row and in lines, of which short sequences have none
 @pytest.mark.parametrize("hd,nh,kvh", [(64, 8, 2), (128, 3, 1), (256, 2, 2)])
 @pytest.mark.parametrize("segs,window,cap", [
     ([(0, 0, 1), (2, 0, 4)], 0, 0.0),
     ([(1, 700, 3), (0, 0, 2), (2, 31, 8)], 40, 50.0),
     ([(2, 0, 33), (0, 130, 1), (1, 0, 129)], 0, 0.0),
-    ([(0, 2000, 9), (1, 0, 43), (2, 3, 300)], 64, 0.0)])
+    ([(0, 2000, 9), (1, 0, 43), (2, 3, 300)], 64, 0.0),
+    ([(2, 1500, 30), (0, 0, 12), (1, 700, 5)], 0, 0.0),
+    ([(2, 2500, 40), (0, 0, 150), (1, 700, 5)], 0, 50.0)])
 @pytest.mark.parametrize("kv8", [False, True])
 def test_prompts_of_one_batch(hd, nh, kvh, segs, window, cap, kv8):
     from llm_np_cp_amd.ops import hip_ops as ho
