@@ -776,6 +776,13 @@ static hipError_t ap_run(ApArgs a, int kv8, const ApPlan& plan,
   return hipGetLastError();
 }
 
+// Counts that a call can have; heads, rows and their parts are divided by.
+static bool ap_takes(int M, int nh, int kvh, bool several, int most,
+                     int ntiles) {
+  return M > 0 && nh > 0 && kvh > 0 && nh % kvh == 0 &&
+         (!several || (ntiles > 0 && most > 0));
+}
+
 // keys: number of keys that the last row sees, as far as the host knows
 // (a hint for the split; the kernel goes by *len_ptr).  tiles: M rows of
 // several sequences, the longest of `most` rows; a tile has 32 rows times
@@ -787,8 +794,7 @@ extern "C" hipError_t launch_attn_prefill_mfma(
     long part_floats, int kv8, int M, int nh, int kvh, int hd, int ldq,
     int S, int keys, int most, int ntiles, float scale, float softcap,
     int window, hipStream_t stream) {
-  if (M < 1 || kvh < 1 || nh % kvh || ldq < nh * hd || ldq % 8 ||
-      (tiles && (ntiles < 1 || most < 1)))
+  if (!ap_takes(M, nh, kvh, tiles, most, ntiles) || ldq < nh * hd || ldq % 8)
     return hipErrorInvalidValue;
   if (!tiles) {
     most = M;
@@ -814,11 +820,14 @@ extern "C" hipError_t launch_attn_prefill_mfma(
 }
 
 // How such a call runs, on the host alone: ranges of keys, whether two groups of
-// waves share a block's, whether parts lie row by row.  1: a head dim that is
-// none of the kernels'.
+// waves share a block's, whether parts lie row by row.  1: counts or a head dim
+// that the launch refuses.
 extern "C" int attn_prefill_plan(int kv8, int M, int nh, int kvh, int hd,
                                  int keys, int most, int ntiles, int window,
                                  long part_floats, int* out) {
+  if (!ap_takes(M, nh, kvh, ntiles, most, ntiles) ||
+      (hd != 64 && hd != 128 && hd != 256))
+    return 1;
   ApArgs a = {};
   a.M = M;
   a.nh = nh;
@@ -826,7 +835,6 @@ extern "C" int attn_prefill_plan(int kv8, int M, int nh, int kvh, int hd,
   a.window = window;
   a.part = part_floats > 0 ? (float*)out : nullptr;      // is there or not
   if (!ntiles) most = M;
-  if (hd != 64 && hd != 128 && hd != 256) return 1;
   const ApPlan p =
       hd == 64 ? ap_plan<64, 64>(a, kv8, keys, part_floats, most, ntiles)
       : hd == 128 ? ap_plan<128, 64>(a, kv8, keys, part_floats, most, ntiles)

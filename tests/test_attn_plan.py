@@ -81,3 +81,30 @@ def test_two_groups_of_waves_have_two_halves_at_most():
     assert not plan(256, 16, 8, [(0, 1999)])["two"]
     assert not plan(64, 32, 8, [(0, 1999)], kv8=True)["two"]
     assert not plan(64, 32, 8, [(0, 2048)] * 2)["two"]    # 1024 blocks
+
+
+# what the launch refuses the plan refuses too: no rows, no heads, heads that are
+# no multiple of the kv heads, several sequences without their longest (these
+# counts are divided by, on the host), another head dim
+REFUSED = [dict(M=0), dict(nh=0), dict(nh=-4), dict(kvh=0), dict(kvh=-2),
+           dict(nh=5), dict(ntiles=3), dict(ntiles=-1, most=2), dict(hd=96)]
+
+
+@pytest.mark.parametrize("bad", REFUSED)
+def test_plan_refuses_what_the_launch_does(bad):
+    kw = dict(M=4, nh=4, kvh=2, hd=64, keys=100, part=1 << 20)
+    assert ho.attn_prefill_plan(**kw)["ranges"] > 0
+    with pytest.raises(RuntimeError):
+        ho.attn_prefill_plan(**{**kw, **bad})
+
+
+# refused by its counts, before any pointer or the device is looked at
+@pytest.mark.parametrize("bad", REFUSED)
+def test_launch_refuses_bad_counts(bad):
+    c = dict(dict(M=4, nh=4, kvh=2, hd=64, most=0, ntiles=0), **bad)
+    at = 1 << 12                       # there or not is all that is asked
+    rc = ho.lib().launch_attn_prefill_mfma(
+        0, 0, 0, 0, 0, at if c["ntiles"] else 0, 0, 0, at, 1 << 20, 0, c["M"],
+        c["nh"], c["kvh"], c["hd"], 512, 128, 100, c["most"], c["ntiles"], 0.1,
+        0.0, 0, 0)
+    assert rc == 1                     # hipErrorInvalidValue
