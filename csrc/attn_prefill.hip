@@ -23,8 +23,9 @@
 // 5 rows of 24/8 heads over 906 keys, split: 11 us, unsplit per-head waves
 // 74 us.  Head dim 256 at two waves a SIMD just fits the registers where LDS
 // addresses are made again for each tile (2048 rows of 16/8 heads behind 2048
-// keys with a soft cap 181 us, so 177); beside an e4m3 pool it spills 27 (6
-// where one wave has all rows).  One wave a SIMD without spills was slower.
+// keys with a soft cap 181 us, so 177); beside an e4m3 pool it spills 28, with a
+// cap 29 (6 where one wave has all rows).  One wave a SIMD without spills was
+// slower.  Of the others 64 dims by two groups of waves without a cap spills one.
 //
 // Where a block's own keys are what takes long (the last rows of a prompt see
 // all of them, and a block goes through its tiles one after the other), two

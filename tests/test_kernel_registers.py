@@ -1,6 +1,7 @@
 """Registers of built kernels, from the notes of their code objects: as many
-blocks fit a CU as a kernel's comments and the rules that choose it count on, and
-nothing that was asked for early is spilled."""
+blocks fit a CU as a kernel's comments and the rules that choose it count on,
+nothing that was asked for early is spilled, and where a kernel spills it is no
+more than its comment says."""
 
 import os
 import re
@@ -74,3 +75,28 @@ def test_product_tiles(built):
                for n in found)                          # beside MXFP4
     for n, (registers, spilled) in found.items():
         assert spilled == 0 and waves(registers) >= 2, n
+
+
+# dims, keys a tile, waves that share the rows, groups of them, e4m3 pool, cap:
+# registers that are spilled
+ROWS_SPILL = {(64, 64, 4, 2, 0, 0): 1,
+              (256, 32, 1, 1, 1, 0): 6, (256, 32, 1, 1, 1, 1): 6,
+              (256, 32, 4, 1, 1, 0): 28, (256, 32, 4, 1, 1, 1): 29}
+
+
+def test_prompt_attention(built):
+    """Four waves or two groups of four: two blocks a CU, of 128 dims by two
+    groups one; blocks of one wave have what LDS leaves of the registers."""
+    found = {}
+    for n, v in built["llmops"].items():
+        m = re.search(r"k_attn_rowsILi(\d+)ELi(\d+)ELi(\d)ELi(\d)ELb(\d)ELb(\d)E",
+                      n)
+        if m:
+            found[tuple(map(int, m.groups()))] = v
+    assert set(ROWS_SPILL) <= set(found)
+    assert {k[0] for k in found} == {64, 128, 256}
+    for k, (registers, spilled) in found.items():
+        hd, _, nw, groups = k[:4]
+        least = 1 if nw == 1 else 4 if groups == 2 and hd == 64 else 2
+        assert waves(registers) >= least, k
+        assert spilled <= ROWS_SPILL.get(k, 0), k
