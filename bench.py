@@ -1,16 +1,16 @@
 #!/usr/bin/env python3
-"""Flagship decode benchmark (driver contract).
+"""Flagship decode benchmark: one JSON line.
 
 Measures decode tokens/sec, batch 1, synthetic prompt, random-init
 weights, bf16.  Default model is Llama-3.2-1B at
-EVERY N (TP=N) so the driver's 1/2/4/8-GPU curve compares like with
+EVERY N (TP=N) so that a curve over 1, 2, 4 and 8 GPUs compares like with
 like; the metric's second config (Gemma-2-9B TP=8, fp8) runs via
 ``--model gemma-2-9b --dtype fp8``.  A "step" is one decoded token; the
 timed region is K replayed decode steps (full forward incl.
 lm_head + sampling).
 
 Usage: python bench.py [--gpus N] [--steps K] [--warmup W] [--model M]
-Launched by the driver for N>1 via torch.distributed.run (one rank/GPU).
+For N>1 launch it by torch.distributed.run (one rank/GPU).
 """
 
 import argparse
@@ -168,7 +168,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=20)
     ap.add_argument("--model", type=str, default="llama-3.2-1b",
                     help="model preset (default llama-3.2-1b at every N "
-                         "so the driver's 1/2/4/8-GPU scaling curve "
+                         "so that a curve over 1, 2, 4 and 8 GPUs "
                          "compares like with like; gemma-2-9b etc. via "
                          "this flag; synthetic random-init weights)")
     ap.add_argument("--prompt-len", type=int, default=64)

@@ -8,7 +8,7 @@ The kernels are validated three ways without needing an 8-GPU node:
      run XgmiComm.create()'s hardware self-check against gloo;
   3. a full TP=2 engine decode (two processes, one GPU) captures the
      one-shot collectives inside a hipGraph and replays it.
-Cross-DEVICE coherence still needs a multi-GPU node (driver round-end);
+Cross-DEVICE coherence still needs a node of several GPUs;
 XgmiComm.create() re-runs the same self-check there at engine init.
 """
 

@@ -121,7 +121,7 @@ def test_timing_and_tracing_utils():
 
 def test_gpu_model_fails_loudly_without_gpu():
     """The HIP engine must never silently fall back on CPU-only hosts
-    (driver requirement: no eager/CPU fallback masquerading as the
+    (no eager/CPU fallback masquerading as the
     native path)."""
     import torch
     if torch.cuda.is_available():

@@ -1,6 +1,6 @@
 #!/bin/sh
-# Developer gate: CPU test tier + gfx950 cross-compile (mirrors what
-# the CI driver runs on a GPU-less host).
+# Developer gate: CPU test tier + gfx950 cross-compile, on a host
+# without a GPU.
 set -e
 cd "$(dirname "$0")/.."
 python -m pytest tests/ -x -q -m "not gpu"
